@@ -6,12 +6,10 @@
 // at the end: per term four v_mad_u64_u32 and a carry chain instead of a full modular
 // multiply-add.  Results are the same canonical residues.
 //
-// k_matmul is built for the shape the prover uses it in: few rows of A (1 for the
-// projection seam `chi^T W`, layergkr/projection.py:150-167, and for combine_t,
-// layergkr/gpu.py:301-308) against a tall B that is streamed once per row of A.  Lanes
-// run along the columns of B (coalesced), the inner dimension is split across
-// workgroups so that even a single output row fills the GPU, and a second small
-// kernel adds the partial sums.
+// k_matmul is built for few rows of A (1 for the projection seam `chi^T W`, layergkr/projection.py:150-167, and for
+// combine_t, layergkr/gpu.py:301-308) against a tall B that is streamed once per eight rows of A.  Lanes run along the
+// columns of B (coalesced), the inner dimension is split across wavefronts and workgroups so that even a single output
+// row fills the GPU, and a second small kernel adds the partial sums of the workgroups.
 #include "common.hpp"
 #include "gl_field.hpp"
 
@@ -43,43 +41,92 @@ struct WideAcc {
     }
 };
 
+// sum of a[l] b[l] with a[l] the same for the whole wavefront, as three 64-bit sums of 32 x 32-bit products (weights 1,
+// 2^32, 2^64) and the counts of their wrap-arounds: the multiply-add leaves its carry in a scalar pair and one
+// instruction counts it, 8 instructions per term where a 160-bit accumulator takes 13 (the carry has to ripple).  The
+// carries are read four instructions after they were written (two wait states are needed).
+struct UniformDot {
+    u64 lo = 0, mid = 0, hi = 0;
+    u32 n_lo = 0, n_mid = 0, n_hi = 0;
+    __device__ __forceinline__ void fma(u64 a, u64 b) {
+        u64 c0, c1, c2, c3;
+        asm("v_mad_u64_u32 %[lo], %[c0], %[a0], %[b0], %[lo]\n\t"
+            "v_mad_u64_u32 %[mid], %[c1], %[a0], %[b1], %[mid]\n\t"
+            "v_mad_u64_u32 %[hi], %[c2], %[a1], %[b1], %[hi]\n\t"
+            "v_mad_u64_u32 %[mid], %[c3], %[a1], %[b0], %[mid]\n\t"
+            "v_addc_co_u32 %[n0], %[c0], 0, %[n0], %[c0]\n\t"
+            "v_addc_co_u32 %[n1], %[c1], 0, %[n1], %[c1]\n\t"
+            "v_addc_co_u32 %[n2], %[c2], 0, %[n2], %[c2]\n\t"
+            "v_addc_co_u32 %[n1], %[c3], 0, %[n1], %[c3]"
+            : [lo] "+v"(lo), [mid] "+v"(mid), [hi] "+v"(hi), [n0] "+v"(n_lo), [n1] "+v"(n_mid), [n2] "+v"(n_hi), [c0] "=&s"(c0),
+              [c1] "=&s"(c1), [c2] "=&s"(c2), [c3] "=&s"(c3)
+            : [a0] "s"((u32)a), [a1] "s"((u32)(a >> 32)), [b0] "v"((u32)b), [b1] "v"((u32)(b >> 32)));
+    }
+    // 2^64 = 2^32 - 1, 2^96 = -1, 2^128 = -2^32 (mod p)
+    __device__ __forceinline__ u64 reduce() const {
+        u64 r = gl::add(gl::canon(lo), gl::mul(mid, (u64)1 << 32));                  // lo + 2^32 mid
+        r = gl::add(r, gl::mul(gl::add(gl::canon(hi), n_lo), gl::EPS));             // + 2^64 (hi + n_lo)
+        r = gl::sub(r, n_mid);                                                      // - n_mid
+        return gl::sub(r, gl::canon((u64)n_hi << 32));                              // - 2^32 n_hi
+    }
+};
+
 // partial[s][i][j] = sum over the s-th slice of the inner dimension of A[i][l] * B[l][j]
-// A thread owns column j for MB consecutive rows of A, so B is streamed once per MB rows, and requests UN
-// elements of its column before it uses the first (one row of A against a 4096 x 65536 B: 5.5 TB/s with eight
-// loads in flight, 4.9 TB/s with the loop left to the compiler).  B is read once and with the streaming hint: the
-// projections of a layer's weight codewords 4.19-4.31 -> 3.87 ms, 6.3 TB/s, what a kernel that only reads reaches.
-template <int MB, int UN>
-__global__ __launch_bounds__(BLOCK) void k_matmul(const u64 *__restrict__ A, const u64 *__restrict__ B, u64 *__restrict__ out,
-                                                  i64 m, i64 k, i64 n, i64 k_per_split) {
-    const i64 j = (i64)blockIdx.x * BLOCK + threadIdx.x;
+// A lane owns column j for MB consecutive rows of A, so B is streamed once per MB rows, and requests UN elements of its
+// column before it uses the first (one row of A against a 4096 x 65536 B: 5.5 TB/s with eight loads in flight, 4.9 TB/s
+// with the loop left to the compiler; with the streaming hint 6.3 TB/s, what a kernel that only reads reaches).
+// The slice is divided again over the KS wavefronts of a workgroup, which add up through LDS: a product of few columns
+// fills the chip in one launch.
+template <int MB, int UN, int KS>
+__global__ __launch_bounds__(64 * KS) void k_matmul(const u64 *__restrict__ A, const u64 *__restrict__ B, u64 *__restrict__ out, i64 m, i64 k,
+                                                    i64 n, i64 k_per_split) {
+    __shared__ u64 part[KS > 1 ? KS : 1][MB][64];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const i64 j = (i64)blockIdx.x * 64 + lane;
     const i64 i0 = (i64)blockIdx.y * MB, s = blockIdx.z;
-    if (j >= n) return;
-    const i64 l0 = s * k_per_split, l1 = (l0 + k_per_split < k) ? l0 + k_per_split : k;
+    const i64 s0 = s * k_per_split, s1 = (s0 + k_per_split < k) ? s0 + k_per_split : k;
+    const i64 per = (s1 - s0 + KS - 1) / KS;
+    const i64 l0 = s0 + w * per, l1 = (l0 + per < s1) ? l0 + per : s1;
     const int rows = (m - i0 < MB) ? (int)(m - i0) : MB;
-    WideAcc acc[MB];
-    i64 l = l0;
-    for (; l + UN <= l1; l += UN) {
-        u64 b[UN];
+    UniformDot acc[MB];
+    if (j < n) {
+        const u64 *b_col = B + j;
+        i64 l = l0;
+        for (; l + UN <= l1; l += UN) {
+            u64 b[UN];
 #pragma unroll
-        for (int u = 0; u < UN; ++u) b[u] = __builtin_nontemporal_load(&B[(l + u) * n + j]);
+            for (int u = 0; u < UN; ++u) b[u] = __builtin_nontemporal_load(&b_col[(l + u) * n]);
 #pragma unroll
-        for (int r = 0; r < MB; ++r) {
-            if (r < rows) {
-                const u64 *a = A + (i0 + r) * k + l;
+            for (int r = 0; r < MB; ++r) {
+                const u64 *a = A + (i0 + (r < rows ? r : 0)) * k + l;
 #pragma unroll
                 for (int u = 0; u < UN; ++u) acc[r].fma(a[u], b[u]);
             }
         }
-    }
-    for (; l < l1; ++l) {
-        const u64 b = B[l * n + j];
+        for (; l < l1; ++l) {
+            const u64 b = b_col[l * n];
 #pragma unroll
-        for (int r = 0; r < MB; ++r)
-            if (r < rows) acc[r].fma(A[(i0 + r) * k + l], b);
+            for (int r = 0; r < MB; ++r) acc[r].fma(A[(i0 + (r < rows ? r : 0)) * k + l], b);
+        }
+    }
+    if (KS == 1) {
+        if (j < n) {
+#pragma unroll
+            for (int r = 0; r < MB; ++r)
+                if (r < rows) out[(s * m + i0 + r) * n + j] = acc[r].reduce();
+        }
+        return;
     }
 #pragma unroll
-    for (int r = 0; r < MB; ++r)
-        if (r < rows) out[(s * m + i0 + r) * n + j] = acc[r].reduce();
+    for (int r = 0; r < MB; ++r) part[w][r][lane] = acc[r].reduce();
+    __syncthreads();
+    // row r of the tile is added up by wavefront r mod KS
+    for (int r = w; r < rows; r += KS) {
+        u64 v = part[0][r][lane];
+#pragma unroll
+        for (int q = 1; q < KS; ++q) v = gl::add(v, part[q][r][lane]);
+        if (j < n) out[(s * m + i0 + r) * n + j] = v;
+    }
 }
 
 // an empty inner dimension gives the zero matrix (a kernel, not a memset: the call may be under stream capture)
@@ -148,17 +195,36 @@ __global__ __launch_bounds__(BLOCK) void k_poly_eval(const u64 *__restrict__ coe
     out[r * kp + p] = acc;
 }
 
-// rows of A a thread takes together
-inline int pick_mb(i64 m) { return m >= 4 ? 4 : (m >= 2 ? 2 : 1); }
+// How a product on the VALU is cut up: rows of A a lane takes together (mb), wavefronts of a workgroup along the inner
+// dimension (ks), and slices of it over workgroups (splits), whose partial sums a second launch adds up.  About 8192
+// wavefronts in all, eight to a SIMD, with at least 16 terms each (4096 and 16384 measured within 10 % of it from one row
+// to 32, 32768 up to 25 % slower); fewer rows to a lane while even so there would be less than two wavefronts to a SIMD
+// (24 x 760 x 1070: 21 -> 18 us).  One row against 32768 columns or more streams fastest with one wavefront to a workgroup
+// (1 x 4096 x 65536: 312 us, 6.9 TB/s; 360 us with four along the inner dimension); everything else takes four (12 x 4096
+// x 4096: 90 us, 103 with sixteen, which saves the second launch now and then but leaves CUs idle).
+struct DirectPlan {
+    int mb, ks, splits;
+};
+DirectPlan plan_direct(i64 m, i64 k, i64 n) {
+    DirectPlan D;
+    const i64 cols = (n + 63) / 64, most = k / 16 > 1 ? k / 16 : 1;
+    D.mb = m >= 8 ? 8 : (m >= 4 ? 4 : (m >= 2 ? 2 : 1));
+    while (D.mb > 1 && cols * ((m + D.mb - 1) / D.mb) * most < 4096) D.mb >>= 1;
+    i64 want = 8192 / (cols * ((m + D.mb - 1) / D.mb));
+    if (want > most) want = most;
+    D.ks = (m == 1 && cols >= 512) || want < 3 ? 1 : 4;
+    const i64 splits = want / D.ks;
+    D.splits = (int)(splits < 1 ? 1 : (splits > 64 ? 64 : splits));
+    if (D.ks > 1 && D.splits == 2) D.splits = 1;           // a second launch for twice the wavefronts does not pay
+    return D;
+}
 
-int pick_splits(i64 m, i64 k, i64 n) {
-    i64 col_blocks = (n + BLOCK - 1) / BLOCK;
-    i64 row_blocks = (m + pick_mb(m) - 1) / pick_mb(m);
-    i64 want = 4096 / (col_blocks * row_blocks > 0 ? col_blocks * row_blocks : 1);      // aim at a few thousand workgroups
-    i64 cap = k / 32;                                                  // at least 32 terms per slice
-    if (want > cap) want = cap;
-    if (want > 64) want = 64;
-    return (int)(want < 1 ? 1 : want);
+template <int MB, int UN>
+void launch_direct(const DirectPlan &D, const u64 *A, const u64 *B, u64 *dst, i64 m, i64 k, i64 n, hipStream_t s) {
+    const i64 per = (k + D.splits - 1) / D.splits;
+    dim3 grid((unsigned)((n + 63) / 64), (unsigned)((m + MB - 1) / MB), (unsigned)D.splits);
+    if (D.ks == 4) hipLaunchKernelGGL((k_matmul<MB, UN, 4>), grid, dim3(256), 0, s, A, B, dst, m, k, n, per);
+    else hipLaunchKernelGGL((k_matmul<MB, UN, 1>), grid, dim3(64), 0, s, A, B, dst, m, k, n, per);
 }
 
 }  // namespace
@@ -167,7 +233,7 @@ extern "C" {
 
 size_t vi_gl_matmul_workspace_bytes(int64_t m, int64_t k, int64_t n) {
     if (m <= 0 || k <= 0 || n <= 0) return 0;
-    int s = pick_splits(m, k, n);
+    const int s = plan_direct(m, k, n).splits;
     return s > 1 ? (size_t)s * (size_t)m * (size_t)n * sizeof(u64) : 0;
 }
 
@@ -184,16 +250,15 @@ int vi_gl_matmul(const uint64_t *A, const uint64_t *B, uint64_t *C, int64_t m, i
         VI_LAUNCH_CHECK("k_zero");
         return VI_OK;
     }
-    const int splits = pick_splits(m, k, n);
+    const DirectPlan D = plan_direct(m, k, n);
+    const int splits = D.splits;
     if (splits > 1 && (!ws || ws_bytes < vi_gl_matmul_workspace_bytes(m, k, n)))
         return vi::fail(VI_ENOMEM, "vi_gl_matmul: workspace below %zu bytes", vi_gl_matmul_workspace_bytes(m, k, n));
-    const i64 per = (k + splits - 1) / splits;
-    const int mb = pick_mb(m);
-    dim3 grid((unsigned)((n + BLOCK - 1) / BLOCK), (unsigned)((m + mb - 1) / mb), (unsigned)splits);
     u64 *dst = splits > 1 ? (u64 *)ws : C;
-    if (mb == 1) hipLaunchKernelGGL((k_matmul<1, 8>), grid, dim3(BLOCK), 0, s, A, B, dst, (i64)m, (i64)k, (i64)n, per);
-    if (mb == 2) hipLaunchKernelGGL((k_matmul<2, 4>), grid, dim3(BLOCK), 0, s, A, B, dst, (i64)m, (i64)k, (i64)n, per);
-    if (mb == 4) hipLaunchKernelGGL((k_matmul<4, 4>), grid, dim3(BLOCK), 0, s, A, B, dst, (i64)m, (i64)k, (i64)n, per);
+    if (D.mb == 1) launch_direct<1, 8>(D, A, B, dst, m, k, n, s);
+    if (D.mb == 2) launch_direct<2, 8>(D, A, B, dst, m, k, n, s);
+    if (D.mb == 4) launch_direct<4, 8>(D, A, B, dst, m, k, n, s);
+    if (D.mb == 8) launch_direct<8, 8>(D, A, B, dst, m, k, n, s);
     VI_LAUNCH_CHECK("k_matmul");
     if (splits > 1) {
         const i64 mn = m * n;
