@@ -1,0 +1,37 @@
+"""GPU parity: gl_matmul at the edges of its tiles, blocks and slices, on the VALU (few rows) and on the matrix cores
+(many rows), against Python big-int sums (bit-exact); larger results by sampled rows and columns."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+from tests.gpu_util import P, rand_field, to_dev, to_np  # noqa: E402
+
+
+@pytest.mark.parametrize("m,k,n,fill", [
+    # VALU: row remainders of a lane's tile, slices over wavefronts and over workgroups, one row streamed
+    (9, 33, 65, None), (17, 500, 129, None), (13, 16, 64, None), (1, 20, 40000, None), (8, 3000, 40, "top"), (1, 2048, 33000, "any"),
+    # matrix cores: 64 x 64, 128 x 128 and 128 x 256 tiles with remainders, inner dimensions around a step and a slice,
+    # the largest sums, words at and above p, columns in several blocks
+    (64, 1000, 3000, None), (65, 1023, 2999, "any"), (129, 700, 4097, None), (700, 257, 2100, "any"), (1025, 65, 4300, None),
+    (130, 8192, 130, "top"), (131, 8193, 129, "half"), (200, 16400, 70, "any"), (100, 40, 250001, None)])
+def test_matmul_edges(m, k, n, fill):
+    from verinf_amd.prover import cuda_primitives as cp
+    A, B = rand_field((m, k), 1 + m), rand_field((k, n), 2 + n)
+    if fill == "top":
+        A[:], B[:] = P - 1, P - 1
+    elif fill == "half":                                        # the word of largest size as a signed number, both signs
+        A[:], B[:] = 0x8080808080808080, 0x7F7F7F7F7F7F7F7F
+        B[::2] += 1
+    elif fill == "any":                                         # words that are not canonical
+        A[:, ::3] = np.uint64((1 << 64) - 1) - A[:, ::3] % np.uint64(1 << 20)
+        B[::2] = np.uint64((1 << 64) - 1) - B[::2] % np.uint64(1 << 33)
+    print(m, k, n, fill, flush=True)
+    got = to_np(cp.gl_matmul(to_dev(A), to_dev(B)))
+    assert got.shape == (m, n)
+    budget = 4_000_000 // k                                     # entries checked
+    rows = sorted({0, m // 2, m - 1, min(m - 1, 63)})
+    cols = np.unique(np.linspace(0, n - 1, max(2, budget // len(rows))).astype(int)) if n * len(rows) > budget else np.arange(n)
+    want = (A[rows].astype(object).dot(B[:, cols].astype(object)) % P).astype(np.uint64)
+    assert np.array_equal(got[np.ix_(rows, cols)], want)

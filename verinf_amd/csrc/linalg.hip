@@ -9,9 +9,11 @@
 // k_matmul is built for few rows of A (1 for the projection seam `chi^T W`, layergkr/projection.py:150-167, and for
 // combine_t, layergkr/gpu.py:301-308) against a tall B that is streamed once per eight rows of A.  Lanes run along the
 // columns of B (coalesced), the inner dimension is split across wavefronts and workgroups so that even a single output
-// row fills the GPU, and a second small kernel adds the partial sums of the workgroups.
+// row fills the GPU, and a second small kernel adds the partial sums of the workgroups.  Products of many rows go to
+// the matrix cores (matmul_rns.hip).
 #include "common.hpp"
 #include "gl_field.hpp"
+#include "matmul_rns.hpp"
 
 namespace {
 
@@ -233,6 +235,7 @@ extern "C" {
 
 size_t vi_gl_matmul_workspace_bytes(int64_t m, int64_t k, int64_t n) {
     if (m <= 0 || k <= 0 || n <= 0) return 0;
+    if (vi::rns_matmul_pays(m, k, n)) return vi::rns_matmul_workspace_bytes(m, k, n);
     const int s = plan_direct(m, k, n).splits;
     return s > 1 ? (size_t)s * (size_t)m * (size_t)n * sizeof(u64) : 0;
 }
@@ -249,6 +252,11 @@ int vi_gl_matmul(const uint64_t *A, const uint64_t *B, uint64_t *C, int64_t m, i
         hipLaunchKernelGGL(k_zero, dim3((unsigned)((mn + BLOCK - 1) / BLOCK)), dim3(BLOCK), 0, s, C, mn);
         VI_LAUNCH_CHECK("k_zero");
         return VI_OK;
+    }
+    if (vi::rns_matmul_pays(m, k, n)) {
+        const size_t need = vi::rns_matmul_workspace_bytes(m, k, n);
+        if (!ws || ws_bytes < need) return vi::fail(VI_ENOMEM, "vi_gl_matmul: workspace below %zu bytes", need);
+        return vi::rns_matmul(A, B, C, m, k, n, ws, s);
     }
     const DirectPlan D = plan_direct(m, k, n);
     const int splits = D.splits;

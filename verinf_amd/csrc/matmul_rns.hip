@@ -1,0 +1,423 @@
+// Dense products over the field on the int8 matrix cores.
+//
+// A 64 x 64-bit multiply-accumulate is 13 or more VALU instructions, so a product of many rows of A is bound by VALU
+// issue at about 2 T multiply-adds per second whatever its tiling.  Here the exact integer product is computed modulo 18
+// pairwise coprime numbers m_i <= 256 instead and put together by the Chinese remainder theorem (the residue-number
+// form of integer matrix products; Ozaki, Uchino, Imamura 2024 use it for floating point).  Modulo one m_i an operand
+// is a signed byte, so each residue is ONE int8 matrix product on v_mfma_i32_32x32x32_i8: 18 byte multiply-adds per
+// field multiply-add, where splitting both operands into bytes would take 64.
+//
+// What bounds it at 1000 x 4096 x 4096 (8240 us on the VALU, 450 here): the int8 products 340 us, 1.8 POP/s with the
+// operands crossing the LDS once per 32 (columns: 64) rows of a wavefront's tile; the residues 85 us, 0.44 GB at the rate
+// of a copy; the reconstruction 20 us.
+//
+//   k_residues        words -> 18 planes of signed bytes
+//   k_residue_gemm    per plane an int8 product; the 32-bit sums are reduced mod m_i to one byte
+//   k_from_residues   18 bytes -> the integer mod p
+//
+// Range.  A word is taken as the integer D = w or w - p with eight balanced digits (bytes in [-128, 127]), |D| <=
+// 2^63.006, so a sum of K products is below 2^126.012 K in size; the product M of the moduli is 2^140.45, and for K <=
+// MAX_K = 8192 the sum stays within 0.37 M of zero: the multiple of M to take off is the nearest integer to
+// sum_i y_i / m_i and a sum of 20-bit fractions finds it (error below 0.003, room 0.13).  A longer inner dimension is
+// cut into slices whose results are added mod p.  The 32-bit sums stay below 2^14 K = 2^27.
+//
+// Layout.  A plane holds units of 16 consecutive inner indices: [unit][row of A or column of B][16 bytes].  A unit is
+// what one lane of the MFMA takes (16 of the 32 inner indices of a step), the global loads, the LDS tile and the
+// operand reads are all contiguous 16-byte accesses in this order, and B is transposed on the way without a pass.
+#include "matmul_rns.hpp"
+
+#include <utility>
+
+#include "common.hpp"
+#include "gl_field.hpp"
+
+namespace {
+
+constexpr int BLOCK = 256;
+constexpr int NMOD = 18;
+constexpr int MODS[NMOD] = {256, 255, 253, 251, 247, 241, 239, 233, 229, 227, 223, 217, 211, 199, 197, 193, 191, 181};
+constexpr int MAX_K = 8192;                    // inner indices of one slice
+constexpr int UNIT = 16;                       // inner indices of a unit
+
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v16i __attribute__((ext_vector_type(16)));
+
+// ---- constants of the residues, all at compile time -------------------------------------------------------------
+constexpr u64 mulmod(u64 a, u64 b) { return (u64)((unsigned __int128)a * b % gl::P); }
+
+// prod of the moduli other than i, mod q (q < 2^16)
+constexpr int others_mod(int i, int q) {
+    int r = 1 % q;
+    for (int j = 0; j < NMOD; ++j)
+        if (j != i) r = r * (MODS[j] % q) % q;
+    return r;
+}
+// (M / m_i)^-1 mod m_i
+constexpr int crt_factor(int i) {
+    const int m = MODS[i], c = others_mod(i, m);
+    for (int x = 1; x < m; ++x)
+        if (c * x % m == 1) return x;
+    return 0;
+}
+// M / m_i mod p (i = NMOD: M mod p)
+constexpr u64 others_mod_p(int i) {
+    u64 r = 1;
+    for (int j = 0; j < NMOD; ++j)
+        if (j != i) r = mulmod(r, (u64)MODS[j]);
+    return r;
+}
+constexpr int balanced(int v, int m) { return v > m / 2 || (v == m / 2 && m == 256) ? v - m : v; }
+
+// the weights 256^j f mod m_i of four digits j = first .. first + 3, as signed bytes
+constexpr u32 digit_weights(int i, int first, int f) {
+    const int m = MODS[i];
+    int pw = 1 % m;
+    for (int j = 0; j < first; ++j) pw = pw * 256 % m;
+    u32 w = 0;
+    for (int j = 0; j < 4; ++j) {
+        w |= (u32)(balanced(pw * f % m, m) & 0xFF) << (8 * j);
+        pw = pw * 256 % m;
+    }
+    return w;
+}
+
+// ---- words to residues ------------------------------------------------------------------------------------------
+// the eight balanced digits of D(w) as signed bytes: w, or w - p = w + 2^32 - 1 - 2^64 for the upper half, plus 128 per
+// digit with carries, minus 128 per digit without
+__device__ __forceinline__ void balanced_digits(u64 w, int &lo, int &hi) {
+    constexpr u64 BIAS = 0x8080808080808080ull;
+    u64 t = w > ~BIAS ? w + gl::EPS : w;
+    t = (t + BIAS) ^ BIAS;
+    lo = (int)(u32)t;
+    hi = (int)(u32)(t >> 32);
+}
+
+// a word whose low byte is the residue mod MODS[I] (signed, of f D): two byte dot products with the digits' weights give
+// |x| <= 2^17, and x - m round(x / m) needs only the low bits of the quotient, which the addition of 1.5 * 2^23 leaves
+// in the low mantissa bits
+template <int I, bool CRT>
+__device__ __forceinline__ u32 residue(int lo, int hi) {
+    constexpr int m = MODS[I], f = CRT ? crt_factor(I) : 1;
+    constexpr u32 wl = digit_weights(I, 0, f), wh = digit_weights(I, 4, f);
+    const int x = __builtin_amdgcn_sdot4(hi, (int)wh, __builtin_amdgcn_sdot4(lo, (int)wl, 0, false), false);
+    const u32 q = __float_as_uint(__builtin_fmaf((float)x, 1.0f / (float)m, 12582912.0f));
+    return (u32)x + __umul24(q, (1u << 24) - (u32)m);
+}
+
+__device__ __forceinline__ u32 pack_bytes(u32 a, u32 b, u32 c, u32 d) {
+    return __builtin_amdgcn_perm(b, a, 0x0c0c0400u) | __builtin_amdgcn_perm(d, c, 0x04000c0cu);
+}
+
+template <int I, bool CRT>
+__device__ __forceinline__ void store_residues(const int (&lo)[UNIT], const int (&hi)[UNIT], v4i *planes, i64 plane, i64 at) {
+    v4i v;
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+        v[g] = (int)pack_bytes(residue<I, CRT>(lo[4 * g], hi[4 * g]), residue<I, CRT>(lo[4 * g + 1], hi[4 * g + 1]),
+                               residue<I, CRT>(lo[4 * g + 2], hi[4 * g + 2]), residue<I, CRT>(lo[4 * g + 3], hi[4 * g + 3]));
+    planes[I * plane + at] = v;
+}
+template <bool CRT, int... I>
+__device__ __forceinline__ void store_all(const int (&lo)[UNIT], const int (&hi)[UNIT], v4i *planes, i64 plane, i64 at,
+                                          std::integer_sequence<int, I...>) {
+    (store_residues<I, CRT>(lo, hi, planes, plane, at), ...);
+}
+
+// Both operands in one launch; units of 16 inner indices from l0, zero beyond k.
+//
+// B: a workgroup takes 256 columns of one unit, lanes along the columns, so that the sixteen reads and the eighteen
+// 16-byte stores of a wavefront are contiguous.
+//
+// A: a workgroup takes 64 rows of four units.  Rows are read along the inner dimension (contiguous) into LDS and picked
+// up unit by unit with the lanes along the rows (an odd pitch in words: no bank conflicts), so that the stores are
+// contiguous here too; read by each lane from its own row, the launch took 37 us for 1000 x 4096 words, 15 this way.
+// The residues carry the factor of the remainder theorem, so that the sums of the products come out as its y_i.
+constexpr int A_ROWS = 64, A_UNITS = 4, A_PITCH = A_UNITS * UNIT + 1;
+
+struct Operand {
+    const u64 *src;                            // first word of the slice
+    i64 ld, count, pitch;                      // row length in memory; rows of A or columns of B; the same padded
+    v4i *planes;
+    unsigned groups;                           // workgroups along rows or columns
+};
+
+__global__ __launch_bounds__(BLOCK) void k_residues(const Operand A, const Operand B, i64 k, int units, unsigned a_blocks) {
+    __shared__ u64 tile[A_ROWS * A_PITCH];
+    u64 w[UNIT];
+    const int tid = threadIdx.x;
+    const bool is_a = blockIdx.x < a_blocks;
+    i64 unit, at;
+    if (is_a) {
+        const i64 r0 = (i64)(blockIdx.x % A.groups) * A_ROWS, l0 = (i64)(blockIdx.x / A.groups) * (A_UNITS * UNIT);
+#pragma unroll
+        for (int i = 0; i < A_ROWS * A_UNITS * UNIT / BLOCK; ++i) {
+            const int r = (tid >> 6) + i * (BLOCK / 64), l = tid & 63;
+            tile[r * A_PITCH + l] = (r0 + r < A.count && l0 + l < k) ? A.src[(r0 + r) * A.ld + l0 + l] : 0;
+        }
+        __syncthreads();
+        unit = (l0 / UNIT) + (tid >> 6);
+        at = r0 + (tid & 63);
+#pragma unroll
+        for (int u = 0; u < UNIT; ++u) w[u] = tile[(tid & 63) * A_PITCH + (tid >> 6) * UNIT + u];
+        if (at >= A.count) return;
+    } else {
+        const unsigned id = blockIdx.x - a_blocks;
+        unit = id / B.groups;
+        at = (i64)(id % B.groups) * BLOCK + tid;
+        if (at >= B.count) return;
+        const u64 *src = B.src + unit * UNIT * B.ld + at;
+#pragma unroll
+        for (int u = 0; u < UNIT; ++u) w[u] = unit * UNIT + u < k ? __builtin_nontemporal_load(&src[u * B.ld]) : 0;
+    }
+    int lo[UNIT], hi[UNIT];
+#pragma unroll
+    for (int u = 0; u < UNIT; ++u) balanced_digits(w[u], lo[u], hi[u]);
+    constexpr auto all = std::make_integer_sequence<int, NMOD>();
+    if (is_a) store_all<true>(lo, hi, A.planes, (i64)units * A.pitch, unit * A.pitch + at, all);
+    else store_all<false>(lo, hi, B.planes, (i64)units * B.pitch, unit * B.pitch + at, all);
+}
+
+// ---- the int8 products ------------------------------------------------------------------------------------------
+// per modulus: m, floor(2^32 / m), a multiple of m above 2^28
+struct ModConst {
+    u32 m[NMOD], inv[NMOD], off[NMOD];
+};
+
+// One 64 WM x 64 WN tile of one plane per workgroup: four wavefronts in a 2 x 2 square, each WM x WN MFMA tiles of
+// 32 x 32.  BKU units of the inner dimension per step through two LDS buffers, the next step's global loads in
+// registers while the current one is multiplied.
+template <int WM, int WN, int BKU, int OCC>
+__global__ __launch_bounds__(BLOCK, OCC) void k_residue_gemm(const v4i *__restrict__ Ap, const v4i *__restrict__ Bp, u32 *__restrict__ Cp,
+                                                             int units, i64 mpad, i64 npad, int mt, int nt, ModConst K) {
+    constexpr int TM = 64 * WM, TN = 64 * WN;
+    constexpr int LA = BKU * TM / BLOCK, LB = BKU * TN / BLOCK;
+    __shared__ v4i As[2][BKU * TM];
+    __shared__ v4i Bs[2][BKU * TN];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    // consecutive ids of one XCD take tiles that share their columns of B
+    u32 id = blockIdx.x;
+    const u32 total = gridDim.x;
+    if ((total & 7) == 0) id = (id & 7) * (total >> 3) + (id >> 3);
+    const int mod = id / (mt * nt), rest = id - mod * (mt * nt);
+    const int tn = rest / mt, tm = rest - tn * mt;
+    const v4i *a_src = Ap + (i64)mod * units * mpad + (i64)tm * TM;
+    const v4i *b_src = Bp + (i64)mod * units * npad + (i64)tn * TN;
+
+    v4i ra[LA], rb[LB];
+    auto fetch = [&](int u0) {
+#pragma unroll
+        for (int i = 0; i < LA; ++i) {
+            const int c = tid + i * BLOCK;
+            ra[i] = a_src[(i64)(u0 + c / TM) * mpad + c % TM];
+        }
+#pragma unroll
+        for (int i = 0; i < LB; ++i) {
+            const int c = tid + i * BLOCK;
+            rb[i] = b_src[(i64)(u0 + c / TN) * npad + c % TN];
+        }
+    };
+    auto put = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < LA; ++i) As[buf][tid + i * BLOCK] = ra[i];
+#pragma unroll
+        for (int i = 0; i < LB; ++i) Bs[buf][tid + i * BLOCK] = rb[i];
+    };
+
+    v16i acc[WM][WN];
+#pragma unroll
+    for (int i = 0; i < WM; ++i)
+#pragma unroll
+        for (int j = 0; j < WN; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
+    const int row0 = (wave >> 1) * (32 * WM) + (lane & 31), col0 = (wave & 1) * (32 * WN) + (lane & 31), half = lane >> 5;
+
+    fetch(0);
+    put(0);
+    __syncthreads();
+    int buf = 0;
+    for (int u0 = 0; u0 < units; u0 += BKU, buf ^= 1) {
+        const bool more = u0 + BKU < units;
+        if (more) fetch(u0 + BKU);
+#pragma unroll
+        for (int s = 0; s < BKU / 2; ++s) {
+            v4i a[WM], b[WN];
+#pragma unroll
+            for (int i = 0; i < WM; ++i) a[i] = As[buf][(2 * s + half) * TM + row0 + 32 * i];
+#pragma unroll
+            for (int j = 0; j < WN; ++j) b[j] = Bs[buf][(2 * s + half) * TN + col0 + 32 * j];
+#pragma unroll
+            for (int i = 0; i < WM; ++i)
+#pragma unroll
+                for (int j = 0; j < WN; ++j) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[i], b[j], acc[i][j], 0, 0, 0);
+        }
+        if (more) put(buf ^ 1);
+        __syncthreads();
+    }
+
+    // y = sum mod m in [0, m); register r of a tile is row 8 (r / 4) + 4 half + r % 4: four rows make a word of C's plane
+    const u32 m = K.m[mod], inv = K.inv[mod], off = K.off[mod];
+    u32 *dst = Cp + (i64)mod * (mpad / 4) * npad + (i64)tn * TN + col0;
+    const i64 q0 = ((i64)tm * TM + (wave >> 1) * (32 * WM)) / 4 + half;
+#pragma unroll
+    for (int i = 0; i < WM; ++i)
+#pragma unroll
+        for (int j = 0; j < WN; ++j)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                u32 y[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const u32 u = (u32)acc[i][j][4 * g + r] + off;
+                    const u32 v = u - __umulhi(u, inv) * m;
+                    y[r] = min(v, v - m);
+                }
+                dst[(q0 + 8 * i + 2 * g) * npad + 32 * j] = pack_bytes(y[0], y[1], y[2], y[3]);
+            }
+}
+
+// ---- residues to words ------------------------------------------------------------------------------------------
+struct CrtSum {
+    u64 lo, hi;                                // sum of y_i (M / m_i mod p), by halves of the constant
+    u32 q;                                     // sum of y_i / m_i in 2^-20
+};
+template <int I>
+__device__ __forceinline__ void crt_add(CrtSum &S, u32 y) {
+    constexpr u64 c = others_mod_p(I);
+    constexpr u32 fr = (u32)(((1 << 21) / MODS[I] + 1) / 2);       // round(2^20 / m)
+    S.lo += (u64)y * (u32)c;
+    S.hi += (u64)y * (u32)(c >> 32);
+    S.q += __umul24(y, fr);
+}
+template <int... I>
+__device__ __forceinline__ void crt_all(CrtSum (&S)[4], const u32 (&w)[NMOD], std::integer_sequence<int, I...>) {
+    ((crt_add<I>(S[0], w[I] & 0xFF), crt_add<I>(S[1], (w[I] >> 8) & 0xFF), crt_add<I>(S[2], (w[I] >> 16) & 0xFF), crt_add<I>(S[3], w[I] >> 24)), ...);
+}
+
+// Four rows of one column per thread: eighteen words in, four words of C out (added to what is there when `accumulate`).
+__global__ __launch_bounds__(BLOCK) void k_from_residues(const u32 *__restrict__ Cp, i64 plane, i64 npad, u64 *C, i64 ld, i64 m, i64 width, int accumulate) {
+    const i64 j = (i64)blockIdx.x * BLOCK + threadIdx.x, r4 = blockIdx.y;
+    if (j >= width) return;
+    u32 w[NMOD];
+#pragma unroll
+    for (int i = 0; i < NMOD; ++i) w[i] = __builtin_nontemporal_load(&Cp[i * plane + r4 * npad + j]);
+    CrtSum S[4] = {};
+    crt_all(S, w, std::make_integer_sequence<int, NMOD>());
+    constexpr u64 neg_m = gl::P - others_mod_p(NMOD);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const i64 row = 4 * r4 + r;
+        if (row >= m) break;
+        const u32 q = (S[r].q + (1u << 19)) >> 20;                  // the multiple of M to take off
+        const u64 lo = S[r].lo + (u64)q * (u32)neg_m, hi = S[r].hi + (u64)q * (u32)(neg_m >> 32);
+        const u64 low = lo + (hi << 32);
+        u64 v = gl::reduce128(low, (hi >> 32) + (low < lo ? 1 : 0));
+        u64 *out = C + row * ld + j;
+        if (accumulate) v = gl::add(v, *out);
+        *out = v;
+    }
+}
+
+// ---- the host side ----------------------------------------------------------------------------------------------
+inline i64 round_up(i64 v, i64 to) { return (v + to - 1) / to * to; }
+
+struct Plan {
+    int wm, wn;                                // MFMA tiles per wavefront
+    i64 kc, mb, nb;                            // slice of the inner dimension, block of rows, block of columns
+    size_t a_bytes, b_bytes, c_bytes;
+};
+
+constexpr int STEP_UNITS = 4;
+
+// The tile is the largest that still gives the 256 CUs a few workgroups each: 128 x 256 (its operands cross the LDS
+// least; 1000 x 4096 x 4096: 448 us, 495 with 128 x 128, 665 with 64 x 64; 256 x 256 leaves one wavefront to a SIMD,
+// 475 us), then 128 x 128 (128 x 4096 x 4096: 165 us, 200 with 64 x 64), and 64 x 64 for up to 64 rows or few tiles
+// (300 x 9000 x 500: 118 us, 130 and 148 with the larger two).
+Plan make_plan(i64 m, i64 k, i64 n) {
+    Plan L;
+    auto tiles = [&](int wm, int wn) { return (m + 64 * wm - 1) / (64 * wm) * ((n + 64 * wn - 1) / (64 * wn)) * NMOD; };
+    L.wm = m <= 64 || tiles(2, 2) < 400 ? 1 : 2;
+    L.wn = L.wm == 1 ? 1 : (tiles(2, 4) < 2048 ? 2 : 4);
+    const i64 tm = 64 * L.wm, tn = 64 * L.wn;
+    const i64 slices = (k + MAX_K - 1) / MAX_K;
+    L.kc = round_up((k + slices - 1) / slices, STEP_UNITS * UNIT);
+    // bytes of the planes of one operand, and of the result: smaller blocks mean more, shorter launches (64 MiB: twice the
+    // time at 1000 x 4096 x 4096, 160 MiB: 3 % more)
+    constexpr i64 CAP = (i64)384 << 20;
+    L.mb = CAP / (NMOD * L.kc) / tm * tm;
+    if (L.mb > 8192) L.mb = 8192;
+    if (L.mb < tm) L.mb = tm;
+    if (L.mb > m) L.mb = m;
+    const i64 mpad = round_up(L.mb, tm);
+    L.nb = CAP / (NMOD * (L.kc > mpad ? L.kc : mpad)) / tn * tn;
+    if (L.nb < tn) L.nb = tn;
+    L.nb = round_up((n + (n + L.nb - 1) / L.nb - 1) / ((n + L.nb - 1) / L.nb), tn);      // blocks of about the same width
+    if (L.nb > n) L.nb = n;
+    const i64 npad = round_up(L.nb, tn);
+    L.a_bytes = (size_t)NMOD * L.kc * mpad;
+    L.b_bytes = (size_t)NMOD * L.kc * npad;
+    L.c_bytes = (size_t)NMOD * mpad * npad;
+    return L;
+}
+
+template <int WM, int WN, int OCC>
+void launch_gemm(const v4i *A, const v4i *B, u32 *C, int units, i64 mpad, i64 npad, const ModConst &K, hipStream_t s) {
+    const int mt = (int)(mpad / (64 * WM)), nt = (int)(npad / (64 * WN));
+    hipLaunchKernelGGL((k_residue_gemm<WM, WN, STEP_UNITS, OCC>), dim3((unsigned)(mt * nt * NMOD)), dim3(BLOCK), 0, s, A, B, C, units, mpad, npad, mt, nt, K);
+}
+
+}  // namespace
+
+namespace vi {
+
+// Estimates in us fitted to measurements of both paths from 1 x 64 x 64 to 2048 x 4096 x 2048 (within a third of the
+// times): here three launches, 36 bytes through memory per word of A, B and C, and 52 T multiply-adds per second; on the
+// VALU 2.6 T.  They meet at 32 rows for a 4096 x 4096 matrix (155 us each) and at 45 rows for 760 x 1070 (27 us).
+bool rns_matmul_pays(int64_t m, int64_t k, int64_t n) {
+    const double macs = (double)m * (double)k * (double)n;
+    const double words = (double)m * (double)k + (double)k * (double)n + (double)m * (double)n;
+    return 18.0 + words / 112e3 + macs / 52e6 < 8.0 + macs / 2.6e6;
+}
+
+size_t rns_matmul_workspace_bytes(int64_t m, int64_t k, int64_t n) {
+    const Plan L = make_plan(m, k, n);
+    return L.a_bytes + L.b_bytes + L.c_bytes;
+}
+
+int rns_matmul(const uint64_t *A, const uint64_t *B, uint64_t *C, int64_t m, int64_t k, int64_t n, void *ws, hipStream_t s) {
+    const Plan L = make_plan(m, k, n);
+    v4i *Ap = (v4i *)ws, *Bp = (v4i *)((char *)ws + L.a_bytes);
+    u32 *Cp = (u32 *)((char *)ws + L.a_bytes + L.b_bytes);
+    ModConst K;
+    for (int i = 0; i < NMOD; ++i) {
+        K.m[i] = (u32)MODS[i];
+        K.inv[i] = (u32)((1ull << 32) / (u32)MODS[i]);
+        K.off[i] = (u32)MODS[i] * ((1u << 28) / (u32)MODS[i] + 1);
+    }
+    for (i64 l0 = 0; l0 < k; l0 += L.kc) {
+        const i64 kc = k - l0 < L.kc ? k - l0 : L.kc;
+        const i64 units = round_up(kc, STEP_UNITS * UNIT) / UNIT;
+        for (i64 i0 = 0; i0 < m; i0 += L.mb) {
+            const i64 mb = m - i0 < L.mb ? m - i0 : L.mb, mpad = round_up(mb, 64 * L.wm);
+            Operand OA = {A + i0 * k + l0, (i64)k, mb, mpad, Ap, (unsigned)((mb + A_ROWS - 1) / A_ROWS)};
+            for (i64 j0 = 0; j0 < n; j0 += L.nb) {
+                const i64 nb = n - j0 < L.nb ? n - j0 : L.nb, npad = round_up(nb, 64 * L.wn);
+                const Operand OB = {B + l0 * n + j0, (i64)n, nb, npad, Bp, (unsigned)((nb + BLOCK - 1) / BLOCK)};
+                const unsigned a_blocks = j0 == 0 ? OA.groups * (unsigned)(units / A_UNITS) : 0;
+                hipLaunchKernelGGL(k_residues, dim3(a_blocks + OB.groups * (unsigned)units), dim3(BLOCK), 0, s, OA, OB, kc, (int)units, a_blocks);
+                VI_LAUNCH_CHECK("k_residues");
+                const int u = (int)units;
+                if (L.wn == 4) launch_gemm<2, 4, 2>(Ap, Bp, Cp, u, mpad, npad, K, s);
+                else if (L.wn == 2) launch_gemm<2, 2, 3>(Ap, Bp, Cp, u, mpad, npad, K, s);
+                else launch_gemm<1, 1, 4>(Ap, Bp, Cp, u, mpad, npad, K, s);
+                VI_LAUNCH_CHECK("k_residue_gemm");
+                hipLaunchKernelGGL(k_from_residues, dim3((unsigned)((nb + BLOCK - 1) / BLOCK), (unsigned)((mb + 3) / 4)), dim3(BLOCK), 0, s, (const u32 *)Cp,
+                                   mpad / 4 * npad, npad, C + i0 * n + j0, (i64)n, mb, nb, l0 > 0 ? 1 : 0);
+                VI_LAUNCH_CHECK("k_from_residues");
+            }
+        }
+    }
+    return VI_OK;
+}
+
+}  // namespace vi
