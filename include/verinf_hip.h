@@ -37,6 +37,16 @@ const char *vi_last_error(void);
 /* Library version, "major.minor". */
 const char *vi_version(void);
 
+/* `bytes` (a multiple of 4) from device memory to `host`, pinned host memory (hipHostMalloc) of host_bytes >= bytes rounded
+ * up to 8, plus 8: the word behind the data is the arrival tag.  Waits until the stream has come to this point and the
+ * data is there (the tag is polled; the stream is queried from time to time, so a failed launch ends the wait). */
+int vi_read_back(const void *src, int64_t bytes, void *host, size_t host_bytes, void *stream);
+
+/* n <= VI_UPLOAD_WORDS words of ordinary host memory to device memory, inside the arguments of a kernel: they are taken
+ * before the call returns, and nothing waits for the stream. */
+#define VI_UPLOAD_WORDS 448
+int vi_upload_words(const uint64_t *host, int64_t n, uint64_t *dst, void *stream);
+
 /* ---- elementwise field ops --------------------------------------------------
  * Replaces gl_mul / gl_add / gl_sub (prover/cuda_primitives.py:208-271, 1086-1088):
  * out[i] = a[i] op b[i].  op: 0 add, 1 sub, 2 mul.  out may alias a or b. */

@@ -5,10 +5,14 @@ loudly if it is missing.  torch is imported first on purpose: its bundled HIP
 runtime must be the one the library binds to, so that tensor pointers and stream
 handles mean the same thing on both sides.
 """
+import array
+import contextlib
 import ctypes
 import os
+import threading
 from ctypes import POINTER, c_char_p, c_double, c_int, c_int64, c_size_t, c_uint64, c_void_p
 
+import numpy as np
 import torch  # noqa: F401  (must precede the CDLL below)
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -18,6 +22,7 @@ LIB_PATH = os.environ.get("VERINF_HIP_LIB") or os.path.join(_HERE, "libverinf_hi
 
 EXPORTS = [
     "vi_last_error", "vi_version",
+    "vi_read_back", "vi_upload_words",
     "vi_gl_binop", "vi_gl_binop_bcast", "vi_gl_unop", "vi_gl_axpy", "vi_gl_probe",
     "vi_gl_sum_workspace_bytes", "vi_gl_sum",
     "vi_gl_matmul_workspace_bytes", "vi_gl_matmul", "vi_gl_matvec", "vi_poly_eval",
@@ -112,6 +117,10 @@ def lib():
     L.vi_challenge.argtypes = [vp, vp, c_int, vp, i64, vp, vp]
     L.vi_gl_spmv.argtypes = [vp, vp, vp, i64, i64, vp, vp, vp, c_int, vp, vp]
     L.vi_lookup_multiplicities.argtypes = [vp, i64, vp, i64, c_int, vp, vp]
+    L.vi_read_back.argtypes = [vp, i64, vp, sz, vp]
+    L.vi_read_back.restype = c_int
+    L.vi_upload_words.argtypes = [vp, i64, vp, vp]
+    L.vi_upload_words.restype = c_int
     L.vi_eq_vector.argtypes = [POINTER(u64), c_int, c_int, vp, vp]
     L.vi_mle_eval_workspace_bytes.restype = sz
     L.vi_mle_eval_workspace_bytes.argtypes = [i64]
@@ -139,9 +148,24 @@ def check(rc: int) -> None:
         raise VerinfHipError(f"libverinf_hip error {rc}: {msg}")
 
 
+# The handle of torch's current stream and the current device as plain integers, straight from torch's bindings: the
+# Stream object of torch.cuda.current_stream() costs 2.8 us and a torch.cuda.device() block 1.3 us per call, more than
+# the kernels of a small call take (0.08 and 0.13 us this way).
+_raw_stream = torch._C._cuda_getCurrentRawStream
+_get_device = torch._C._cuda_getDevice
+
+
 def stream_ptr() -> int:
     """hipStream_t of torch's current stream (kernels are queued behind torch's own work)."""
-    return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(_get_device())
+
+
+_NO_GUARD = contextlib.nullcontext()
+
+
+def on_device(dev):
+    """Context that makes `dev` current; nothing to do (and nothing paid) when it already is."""
+    return _NO_GUARD if dev.index is None or dev.index == _get_device() else torch.cuda.device(dev)
 
 
 _ws_cache = {}
@@ -154,15 +178,77 @@ def workspace(nbytes: int, device=None, tag: str = "ws", stream_ptr=None):
     (or two host threads on their own streams) never share scratch, and a buffer is only ever used on the
     stream it was allocated on -- when it is outgrown and dropped, the caching allocator may reuse its memory
     in stream order without further bookkeeping.  Buffers grow and are kept; release_workspaces() drops them."""
-    device = torch.device("cuda", torch.cuda.current_device()) if device is None else device
+    index = _get_device() if device is None or device.index is None else device.index
     # stream_ptr: the current stream's handle when the caller has looked it up already
-    key = (tag, device.index, torch.cuda.current_stream(device).cuda_stream if stream_ptr is None else stream_ptr)
+    key = (tag, index, _raw_stream(index) if stream_ptr is None else stream_ptr)
     buf = _ws_cache.get(key)
     if buf is None or buf.numel() < nbytes:
-        with torch.cuda.device(device):
-            buf = torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=device)
+        with torch.cuda.device(index):
+            buf = torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=torch.device("cuda", index))
         _ws_cache[key] = buf
     return buf
+
+
+_pinned = threading.local()
+
+
+def pinned_words(words: int, stream_ptr: int):
+    """Pinned host words that kernels of a call write results into and the call reads them from, with a numpy view of
+    the same memory.  One buffer per host thread and stream: a call has read its results before the next one on that
+    stream starts, and two threads (or two streams) never see each other's.  Buffers grow and are kept for the life
+    of the thread (a few KiB each)."""
+    bufs = getattr(_pinned, "bufs", None)
+    if bufs is None:
+        bufs = _pinned.bufs = {}
+    key = (_get_device(), stream_ptr)
+    buf = bufs.get(key)
+    if buf is None or buf[0].numel() < words:
+        t = torch.zeros(max(words, 512), dtype=torch.uint64).pin_memory()
+        buf = bufs[key] = (t, t.numpy())
+    return buf
+
+
+def read_back_ptr(src: int, nbytes: int, sp: int) -> bytes:
+    """`nbytes` (a multiple of 4) at device address `src`, once the stream `sp` has reached this point.
+
+    A kernel writes the bytes and then a tag into pinned memory and the host polls the tag: 6 us less than a copy
+    and a stream synchronisation."""
+    words = (nbytes + 7) // 8
+    host, view = pinned_words(words + 1, sp)
+    check(lib().vi_read_back(src, nbytes, host.data_ptr(), host.numel() * 8, sp))
+    return view[:words].tobytes()[:nbytes]
+
+
+def read_back(t, nbytes: int) -> bytes:
+    """The first `nbytes` of a contiguous device tensor, through the current stream."""
+    with on_device(t.device):
+        return read_back_ptr(t.data_ptr(), nbytes, stream_ptr())
+
+
+_UPLOAD_WORDS = 448         # VI_UPLOAD_WORDS
+_P = (1 << 64) - (1 << 32) + 1
+
+
+def field_words(values):
+    """Python integers as an array('Q') of residues mod p."""
+    try:
+        words = array.array("Q", values)         # 20 ns per entry, ten times less than int(v) % p one by one
+    except (OverflowError, TypeError):
+        return array.array("Q", [int(v) % _P for v in values])
+    if len(words) and (max(words) if len(words) < 64 else int(np.frombuffer(words, dtype=np.uint64).max())) >= _P:
+        return array.array("Q", [v % _P for v in words])
+    return words
+
+
+def upload_words(words):
+    """An array('Q') as a (1, n) uint64 tensor on the current device.  Short ones travel in a kernel's arguments (one
+    launch); a copy from pageable memory waits for the stream first (15 us with nothing to wait for)."""
+    n = len(words)
+    if n > _UPLOAD_WORDS or n == 0:
+        return torch.from_numpy(np.frombuffer(words, dtype=np.uint64).reshape(1, n).copy()).cuda()
+    out = torch.empty((1, n), dtype=torch.uint64, device="cuda")
+    check(lib().vi_upload_words(words.buffer_info()[0], n, out.data_ptr(), stream_ptr()))
+    return out
 
 
 def release_workspaces() -> None:

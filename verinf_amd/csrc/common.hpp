@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdarg>
 #include <cstdio>
 
@@ -27,6 +28,35 @@ inline int ilog2(long long x) {
     int l = 0;
     while ((1ll << l) < x) ++l;
     return l;
+}
+
+// Waits until the kernel that finishes a result has stored `seq` behind it in pinned host memory.  The word is polled (a
+// stream synchronisation costs several microseconds more); every 2^16 polls the stream is queried, so a failed launch or
+// a stream that drained without the store ends the wait with an error instead of spinning.
+inline int wait_for_tag(const char *who, const volatile uint64_t *flag, uint64_t seq, hipStream_t s) {
+    for (unsigned spins = 1;; ++spins) {
+        if (*flag == seq) break;
+        __builtin_ia32_pause();
+        if ((spins & 0xFFFF) == 0) {
+            hipError_t e = hipStreamQuery(s);
+            if (e == hipErrorNotReady) {
+                (void)hipGetLastError();                 // "not ready" is no error for the launch checks that follow
+                continue;
+            }
+            if (e != hipSuccess) return fail(VI_EHIP, "%s: %s while waiting for a result", who, hipGetErrorString(e));
+            // drained: host memory that is not coherent while a kernel runs shows the store now
+            if (*flag == seq) break;
+            return fail(VI_EHIP, "%s: the stream drained without the result", who);
+        }
+    }
+    std::atomic_thread_fence(std::memory_order_acquire);
+    return VI_OK;
+}
+
+// a tag no earlier call has used, so that nothing such a call may have left in flight can pass for this one's result
+inline uint64_t new_tag() {
+    static std::atomic<uint64_t> calls{0};
+    return (calls.fetch_add(1) + 1) << 32;
 }
 
 }  // namespace vi

@@ -207,6 +207,22 @@ __global__ __launch_bounds__(BLOCK) void k_sum_final(const u64 *partial, int nb,
     if (threadIdx.x == 0) out[0] = r;
 }
 
+// words of a small result to pinned host memory, then the tag the host polls (one workgroup, so that one barrier and one
+// fence order the data before the tag)
+__global__ __launch_bounds__(BLOCK) void k_read_back(const u32 *src, int words, u32 *host, u64 *flag, u64 tag) {
+    for (int i = threadIdx.x; i < words; i += BLOCK) host[i] = src[i];
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(flag, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+struct Words {
+    u64 w[VI_UPLOAD_WORDS];
+};
+__global__ __launch_bounds__(BLOCK) void k_upload(const Words W, int n, u64 *dst) {
+    for (int i = threadIdx.x; i < n; i += BLOCK) dst[i] = W.w[i];
+}
+
 inline bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 
 }  // namespace
@@ -215,6 +231,31 @@ extern "C" {
 
 const char *vi_last_error(void) { return vi::err_buf(); }
 const char *vi_version(void) { return "0.2"; }
+
+int vi_read_back(const void *src, int64_t bytes, void *host, size_t host_bytes, void *stream) {
+    if (bytes <= 0 || bytes > (1 << 20) || (bytes & 3)) return vi::fail(VI_EINVAL, "vi_read_back: %lld bytes (a multiple of 4 up to 2^20)", (long long)bytes);
+    const size_t data = ((size_t)bytes + 7) & ~(size_t)7;
+    if (!src || !host || ((uintptr_t)src & 3) || ((uintptr_t)host & 7)) return vi::fail(VI_EINVAL, "vi_read_back: null or unaligned pointer");
+    if (host_bytes < data + 8) return vi::fail(VI_ENOMEM, "vi_read_back: host buffer below %zu bytes", data + 8);
+    u64 *flag = (u64 *)((char *)host + data);
+    const u64 tag = vi::new_tag();
+    *(volatile u64 *)flag = 0;
+    std::atomic_thread_fence(std::memory_order_seq_cst);
+    hipLaunchKernelGGL(k_read_back, dim3(1), dim3(BLOCK), 0, (hipStream_t)stream, (const u32 *)src, (int)(bytes / 4), (u32 *)host, flag, tag);
+    VI_LAUNCH_CHECK("k_read_back");
+    return vi::wait_for_tag("vi_read_back", flag, tag, (hipStream_t)stream);
+}
+
+int vi_upload_words(const uint64_t *host, int64_t n, uint64_t *dst, void *stream) {
+    if (n < 0 || n > VI_UPLOAD_WORDS) return vi::fail(VI_EINVAL, "vi_upload_words: n = %lld (0 .. %d)", (long long)n, VI_UPLOAD_WORDS);
+    if (n == 0) return VI_OK;
+    if (!host || !dst) return vi::fail(VI_EINVAL, "vi_upload_words: null pointer");
+    Words W;
+    for (i64 i = 0; i < VI_UPLOAD_WORDS; ++i) W.w[i] = i < n ? host[i] : 0;
+    hipLaunchKernelGGL(k_upload, dim3(1), dim3(BLOCK), 0, (hipStream_t)stream, W, (int)n, dst);
+    VI_LAUNCH_CHECK("k_upload");
+    return VI_OK;
+}
 
 int vi_gl_binop(int op, const uint64_t *a, const uint64_t *b, uint64_t *out, int64_t n, void *stream) {
     if (op < 0 || op > 2) return vi::fail(VI_EINVAL, "vi_gl_binop: op %d", op);

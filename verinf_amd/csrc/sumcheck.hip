@@ -1194,28 +1194,6 @@ u64 interpolate_at(const u64 *y, const u64 *winv, int n, u64 x) {
     return total;
 }
 
-// Waits until the kernel that finishes a round's samples has stored `seq` behind them.  The word is polled (a stream
-// synchronisation costs several microseconds more per round); every 2^16 polls the stream is queried, so a failed
-// launch or a stream that drained without the store ends the wait with an error instead of spinning.
-int wait_for_samples(const volatile u64 *flag, u64 seq, hipStream_t s) {
-    for (unsigned spins = 1;; ++spins) {
-        if (*flag == seq) break;
-        __builtin_ia32_pause();
-        if ((spins & 0xFFFF) == 0) {
-            hipError_t e = hipStreamQuery(s);
-            if (e == hipErrorNotReady) {
-                (void)hipGetLastError();                 // "not ready" is no error for the launch checks that follow
-                continue;
-            }
-            if (e != hipSuccess) return vi::fail(VI_EHIP, "vi_sumcheck_prove: %s while waiting for a round", hipGetErrorString(e));
-            // drained: host memory that is not coherent while a kernel runs shows the store now
-            if (*flag == seq) break;
-            return vi::fail(VI_EHIP, "vi_sumcheck_prove: the stream drained without the round's samples");
-        }
-    }
-    std::atomic_thread_fence(std::memory_order_acquire);
-    return VI_OK;
-}
 }  // namespace
 
 int vi_sumcheck_prove(const uint64_t *const *tables, uint64_t *const *work, int n_tables, int64_t size,
@@ -1242,8 +1220,7 @@ int vi_sumcheck_prove(const uint64_t *const *tables, uint64_t *const *work, int 
     int64_t half = size / 2;
     // host_samples[NSAMP] is the arrival word: round k's kernel stores (call number << 32) + k + 1 there behind its
     // samples, so that nothing an earlier call may have left in flight on this buffer can pass for a round of this one
-    static std::atomic<u64> calls{0};
-    const u64 tag = (calls.fetch_add(1) + 1) << 32;
+    const u64 tag = vi::new_tag();
     volatile u64 *arrived = host_samples + NSAMP;
     *arrived = 0;
     std::atomic_thread_fence(std::memory_order_seq_cst);
@@ -1255,7 +1232,7 @@ int vi_sumcheck_prove(const uint64_t *const *tables, uint64_t *const *work, int 
     const uint64_t *const *src = tables;
     int round = 0;
     for (;;) {
-        rc = wait_for_samples(arrived, tag + (u64)round + 1, s);
+        rc = vi::wait_for_tag("vi_sumcheck_prove", arrived, tag + (u64)round + 1, s);
         if (rc) break;
         u64 y[NSAMP];
         for (int x = 0; x < ns; ++x) y[x] = out_samples[(size_t)round * ns + x] = ((const volatile u64 *)host_samples)[x];

@@ -21,9 +21,8 @@ mle_eval work on Python lists).  The dense Lagrange-matrix encoders
 (`encode_batch[_t]`) of the reference module are not provided: the NTT encoder is
 the one encoder here.
 """
-import contextlib
 import ctypes
-import threading
+import struct
 from typing import Optional, Sequence
 
 import torch
@@ -96,8 +95,10 @@ def encode_batch_ntt(cfg: Config, messages):
             raise ValueError(f"message {width} > K_DEG {cfg.K_DEG}")
         msgs = _to_device_rows(messages, max(width, 1))
     rows = int(msgs.shape[0])
-    out = torch.empty((rows, cfg.N_LIG), dtype=torch.uint64, device=msgs.device)
     step = _chunk_rows(cfg, rows) if rows else 1
+    if step >= rows:
+        return cp.coset_lde(msgs, cfg.K_DEG, cfg.N_LIG, GLOBAL_G)
+    out = torch.empty((rows, cfg.N_LIG), dtype=torch.uint64, device=msgs.device)
     for lo in range(0, rows, step):
         hi = min(lo + step, rows)
         cp.coset_lde(msgs[lo:hi], cfg.K_DEG, cfg.N_LIG, GLOBAL_G, out=out[lo:hi])
@@ -141,8 +142,7 @@ def selftest_ntt_spot(cfg: Config, n_cols: int = 24, seed: int = 5) -> Optional[
 
 
 def _u64_row(values):
-    import numpy as np
-    return torch.from_numpy(np.array([[int(v) % P for v in values]], dtype=np.uint64)).cuda()
+    return _lib.upload_words(_lib.field_words(values))
 
 
 def linear_combination(cfg: Config, codewords, coeffs: Sequence[int]):
@@ -167,9 +167,8 @@ def hash_and_tree(cfg: Config, mat):
     """Column digests and the Merkle tree of a device codeword matrix, both computed on the
     device (gpu.py:274-288): returns (root bytes, list of (k_i, 32) uint8 level tensors)."""
     _require_gpu()
-    dig = cp.hash_columns_streamed(mat)
-    root_t, levels_t = cp.merkle_build_blake3(dig)
-    return bytes(root_t.cpu().tolist()), levels_t
+    levels_t = cp.merkle_levels(cp.hash_columns_streamed(mat))
+    return _lib.read_back(levels_t[-1], 32), levels_t
 
 
 def levels_to_host(levels_t):
@@ -189,8 +188,7 @@ def column(mat, col: int):
 
 # ---- multilinear helpers ---------------------------------------------------------------
 def _point(z):
-    arr = (ctypes.c_uint64 * max(len(z), 1))(*[int(v) % P for v in z])
-    return arr
+    return (ctypes.c_uint64 * max(len(z), 1))(*[int(v) % P for v in z])
 
 
 def eq_vector_t(z: Sequence[int], msb_first: bool = False):
@@ -219,12 +217,14 @@ def mle_eval_t(tables, point: Sequence[int]):
     if mat.dim() != 2 or int(mat.shape[1]) != (1 << n):
         raise RuntimeError(f"mle_eval_t: tables of length {tuple(tables.shape)} do not match {n} variables")
     k = int(mat.shape[0])
-    out = torch.empty(max(k, 1), dtype=torch.uint64, device=tables.device)
+    if k == 0:
+        return []
     L = _lib.lib()
-    ws = _lib.workspace(L.vi_mle_eval_workspace_bytes(k), tables.device, "mle")
-    _lib.check(L.vi_mle_eval(mat.data_ptr(), k, 1 << n, _point(point), n, out.data_ptr(), ws.data_ptr(), ws.numel(),
-                             _lib.stream_ptr()))
-    vals = [int(v) for v in out[:k].cpu().tolist()]
+    sp = _lib.stream_ptr()
+    ws_bytes = L.vi_mle_eval_workspace_bytes(k)
+    ws = _lib.workspace(ws_bytes + 8 * k, tables.device, "mle", sp).data_ptr()
+    _lib.check(L.vi_mle_eval(mat.data_ptr(), k, 1 << n, _point(point), n, ws + ws_bytes, ws, ws_bytes, sp))
+    vals = list(struct.unpack(f"<{k}Q", _lib.read_back_ptr(ws + ws_bytes, 8 * k, sp)))
     return vals[0] if one else vals
 
 
@@ -238,7 +238,7 @@ def gl_sum(t):
     v = v.contiguous()
     out = torch.empty(1, dtype=torch.uint64, device=v.device)
     L = _lib.lib()
-    with torch.cuda.device(v.device):
+    with _lib.on_device(v.device):
         ws = _lib.workspace(L.vi_gl_sum_workspace_bytes(v.numel()), v.device, "sum")
         _lib.check(L.vi_gl_sum(v.data_ptr(), v.numel(), out.data_ptr(), ws.data_ptr(), ws.numel(),
                                _lib.stream_ptr()))
@@ -267,7 +267,7 @@ class _Problem:
 
 def _fold_tables(src, dst, half: int, r: int):
     L = _lib.lib()
-    with torch.cuda.device(src[0].device):
+    with _lib.on_device(src[0].device):
         _lib.check(L.vi_sumcheck_fold_eval(_Problem.ptrs(src), _Problem.ptrs(dst), len(src), half, r % P,
                                            None, None, None, 0, None, None, None, 0, _lib.stream_ptr()))
 
@@ -370,7 +370,7 @@ def prove_terms_gpu(terms, coin, field_p: int, mask=None, mu0: int = 0):
             mu = _poly_eval(h, r, field_p)
     L = _lib.lib()
     dev = tables[0].device
-    with _on_device(dev):
+    with _lib.on_device(dev):
         stream = torch.cuda.current_stream()
         sp = stream.cuda_stream
         ws = _lib.workspace(L.vi_sumcheck_prove_coins_workspace_bytes(size), dev, "sumcheck_coins", sp)
@@ -379,7 +379,7 @@ def prove_terms_gpu(terms, coin, field_p: int, mask=None, mu0: int = 0):
         half_bytes = (size // 2) * 8
         work = _lib.workspace(max(prob.n_tables * half_bytes, 256), dev, "sumcheck_work", sp)
         work_p = (ctypes.c_void_p * prob.n_tables)(*[work.data_ptr() + t * half_bytes for t in range(prob.n_tables)])
-        samples_host, samples_np = _pinned_samples(8 * n_rounds, sp)
+        samples_host, samples_np = _lib.pinned_words(8 * n_rounds, sp)
         chal = (ctypes.c_uint64 * n_rounds)(*challenges)
         _lib.check(L.vi_sumcheck_prove_coins(_Problem.ptrs(tables), work_p, prob.n_tables, size,
                                              prob.term_off, prob.factor_idx, prob.coeffs, prob.n_terms, chal,
@@ -411,12 +411,12 @@ def prove_terms_gpu_interactive(terms, coin, field_p: int, mask=None, mu0: int =
     dev = tables[0].device
     mu = mu0 % field_p
 
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         ws = _lib.workspace(L.vi_sumcheck_workspace_bytes(), dev, "sumcheck")
         # The round loop runs inside the library: per round one fused launch, a wait on a word of pinned host
         # memory that the kernel stores behind its samples, and this callback -- the only Python left in the
         # loop -- which applies the optional scalar mask and asks the verifier coin for the challenge.
-        samples_host, _ = _pinned_samples(16, torch.cuda.current_stream().cuda_stream)
+        samples_host, _ = _lib.pinned_words(16, _lib.stream_ptr())
         work = _work_tables(tables, size, dev)
         round_polys, challenges = [], []
         state = {"mu": mu, "error": None}
@@ -444,7 +444,7 @@ def prove_terms_gpu_interactive(terms, coin, field_p: int, mask=None, mu0: int =
         rc = L.vi_sumcheck_prove(_Problem.ptrs(tables), _Problem.ptrs(work), prob.n_tables, size, prob.term_off,
                                  prob.factor_idx, prob.coeffs, prob.n_terms, cb, None, samples_host.data_ptr(),
                                  samples_host.numel(), out_samples, out_chals, ws.data_ptr(), ws.numel(),
-                                 torch.cuda.current_stream().cuda_stream)
+                                 _lib.stream_ptr())
         if state["error"] is not None:
             raise state["error"]
         _lib.check(rc)
@@ -459,31 +459,6 @@ def _work_tables(tables, size, dev):
     if size < 4:
         return tables                        # one round: nothing is folded
     return [torch.empty(size // 2, dtype=torch.uint64, device=dev) for _ in tables]
-
-
-_PINNED = threading.local()
-_NO_GUARD = contextlib.nullcontext()
-
-
-def _on_device(dev):
-    """Context that makes `dev` current; nothing to do (and nothing paid) when it already is."""
-    return _NO_GUARD if dev.index is None or dev.index == torch.cuda.current_device() else torch.cuda.device(dev)
-
-
-def _pinned_samples(words: int, stream_ptr: int):
-    """Pinned host words the sumcheck kernels write their samples into (and, for the interactive loop, the tag of
-    the round that has arrived), with a numpy view of the same memory.  One buffer per host thread and stream: a
-    proof is read back before the next one on that stream starts, and two threads (or two streams) never see each
-    other's samples."""
-    bufs = getattr(_PINNED, "bufs", None)
-    if bufs is None:
-        bufs = _PINNED.bufs = {}
-    key = (torch.cuda.current_device(), stream_ptr)
-    buf = bufs.get(key)
-    if buf is None or buf[0].numel() < words:
-        t = torch.zeros(max(words, 512), dtype=torch.uint64).pin_memory()
-        buf = bufs[key] = (t, t.numpy())
-    return buf
 
 
 def _poly_eval(coeffs: Sequence[int], x: int, p: int) -> int:

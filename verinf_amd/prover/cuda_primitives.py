@@ -47,7 +47,7 @@ def _binop(op, a, b, who):
     if a.shape != b.shape:
         raise RuntimeError(f"{who}: shape mismatch")
     out = torch.empty_like(a)
-    with torch.cuda.device(a.device):
+    with _lib.on_device(a.device):
         _lib.check(_lib.lib().vi_gl_binop(_OPS[op], a.data_ptr(), b.data_ptr(), out.data_ptr(),
                                           a.numel(), _lib.stream_ptr()))
     return out
@@ -73,7 +73,7 @@ def gl_mul_bcast(a, b_row):
     if b_row.dim() != 1 or a.shape[-1] != b_row.numel():
         raise RuntimeError("gl_mul_bcast: last dimension mismatch")
     out = torch.empty_like(a)
-    with torch.cuda.device(a.device):
+    with _lib.on_device(a.device):
         _lib.check(_lib.lib().vi_gl_binop_bcast(2, a.data_ptr(), b_row.data_ptr(), b_row.numel(),
                                                 out.data_ptr(), a.numel(), _lib.stream_ptr()))
     return out
@@ -82,7 +82,7 @@ def gl_mul_bcast(a, b_row):
 def _unop(op, a, arg):
     _check_u64(a, "a")
     out = torch.empty_like(a)
-    with torch.cuda.device(a.device):
+    with _lib.on_device(a.device):
         _lib.check(_lib.lib().vi_gl_unop(op, a.data_ptr(), int(arg) & ((1 << 64) - 1), out.data_ptr(),
                                          a.numel(), _lib.stream_ptr()))
     return out
@@ -120,7 +120,7 @@ def gl_axpy(y, alpha, x):
     _check_u64(x, "x")
     if y.shape != x.shape:
         raise RuntimeError("gl_axpy: shape mismatch")
-    with torch.cuda.device(y.device):
+    with _lib.on_device(y.device):
         _lib.check(_lib.lib().vi_gl_axpy(y.data_ptr(), int(alpha) % P, x.data_ptr(), y.numel(),
                                          _lib.stream_ptr()))
 
@@ -135,14 +135,15 @@ _NTT_WS_CAP = 1 << 30
 
 def _ntt(rows, m, n, inverse):
     L = _lib.lib()
-    with torch.cuda.device(rows.device):
+    with _lib.on_device(rows.device):
         # the library transforms the rows in chunks that fit the workspace it is given: one row is the minimum,
         # 1 GiB is enough to fill the GPU, and a large batch does not double its footprint for the process's life
         need = min(L.vi_ntt_workspace_bytes(m, n), max(_NTT_WS_CAP, n * 8))
-        ws = _lib.workspace(need, rows.device, "ntt") if need else None
-        _lib.check(L.vi_ntt_batched(rows.data_ptr(), m, n, int(inverse),
-                                    ws.data_ptr() if ws is not None else None,
-                                    ws.numel() if ws is not None else 0, _lib.stream_ptr()))
+        ws, ws_bytes = None, 0
+        if need:
+            buf = _lib.workspace(need, rows.device, "ntt")
+            ws, ws_bytes = buf.data_ptr(), buf.numel()
+        _lib.check(L.vi_ntt_batched(rows.data_ptr(), m, n, int(inverse), ws, ws_bytes, _lib.stream_ptr()))
 
 
 def _ntt_1d(a, inverse):
@@ -228,7 +229,7 @@ def coset_lde(messages, k_deg, n_lig, shift=GLOBAL_G, out=None):
     if w == 0:                      # an empty message is the zero polynomial
         return out.view(torch.int64).zero_().view(torch.uint64)
     L = _lib.lib()
-    with torch.cuda.device(messages.device):
+    with _lib.on_device(messages.device):
         ws = _lib.workspace(L.vi_coset_lde_workspace_bytes(m, k_deg, n_lig), messages.device, "lde")
         _lib.check(L.vi_coset_lde(messages.data_ptr(), m, w, in_stride, k_deg, n_lig, int(shift) % P,
                                   out.data_ptr(), n_lig, ws.data_ptr(), ws.numel(), _lib.stream_ptr()))
@@ -258,7 +259,7 @@ def coset_lde_with_coeffs(messages, k_deg, n_lig, shift=GLOBAL_G, need_codewords
             out.view(torch.int64).zero_()
         return coeffs, out
     L = _lib.lib()
-    with torch.cuda.device(messages.device):
+    with _lib.on_device(messages.device):
         ws = _lib.workspace(L.vi_coset_lde_workspace_bytes(m, k_deg, n_lig), messages.device, "lde")
         _lib.check(L.vi_coset_lde_coeffs(messages.data_ptr(), m, w, in_stride, k_deg, n_lig, int(shift) % P,
                                          coeffs.data_ptr(), k_deg, out.data_ptr() if out is not None else None, n_lig,
@@ -277,7 +278,7 @@ def coset_extend(coeffs, k_deg, n_lig, shift=GLOBAL_G, out=None):
     if w == 0:
         return out.view(torch.int64).zero_().view(torch.uint64)
     L = _lib.lib()
-    with torch.cuda.device(coeffs.device):
+    with _lib.on_device(coeffs.device):
         ws = _lib.workspace(L.vi_coset_lde_workspace_bytes(m, k_deg, n_lig), coeffs.device, "lde")
         _lib.check(L.vi_coset_extend(coeffs.data_ptr(), m, w, in_stride, k_deg, n_lig, int(shift) % P,
                                      out.data_ptr(), n_lig, ws.data_ptr(), ws.numel(), _lib.stream_ptr()))
@@ -307,14 +308,14 @@ def gl_matmul(A, B):
         raise RuntimeError("gl_matmul: inner dim mismatch")
     C = torch.empty((m, n), dtype=torch.uint64, device=A.device)
     L = _lib.lib()
-    with torch.cuda.device(A.device):
+    a_ptr, c_ptr = A.data_ptr(), C.data_ptr()
+    with _lib.on_device(A.device):
         for lo in range(0, m, 65535):
-            hi = min(lo + 65535, m)
-            need = L.vi_gl_matmul_workspace_bytes(hi - lo, k, n)
-            ws = _lib.workspace(need, A.device, "matmul") if need else None
-            _lib.check(L.vi_gl_matmul(A[lo:hi].data_ptr() if m else None, B.data_ptr(), C[lo:hi].data_ptr() if m else None,
-                                      hi - lo, k, n, ws.data_ptr() if ws is not None else None,
-                                      ws.numel() if ws is not None else 0, _lib.stream_ptr()))
+            rows = min(65535, m - lo)
+            need = L.vi_gl_matmul_workspace_bytes(rows, k, n)
+            ws = _lib.workspace(need, A.device, "matmul").data_ptr() if need else None
+            _lib.check(L.vi_gl_matmul(a_ptr + lo * k * 8, B.data_ptr(), c_ptr + lo * n * 8, rows, k, n, ws, need,
+                                      _lib.stream_ptr()))
     return C
 
 
@@ -328,7 +329,7 @@ def gl_matvec(M, v):
     if int(v.shape[0]) != n:
         raise RuntimeError("gl_matvec: dim mismatch")
     out = torch.empty((m,), dtype=torch.uint64, device=M.device)
-    with torch.cuda.device(M.device):
+    with _lib.on_device(M.device):
         _lib.check(_lib.lib().vi_gl_matvec(M.data_ptr(), v.data_ptr(), out.data_ptr(), m, n, _lib.stream_ptr()))
     return out
 
@@ -348,7 +349,7 @@ def poly_eval(coeffs, points):
     k = int(points.shape[0])
     out = torch.empty((m, k), dtype=torch.uint64, device=coeffs.device)
     L = _lib.lib()
-    with torch.cuda.device(coeffs.device):
+    with _lib.on_device(coeffs.device):
         for lo in range(0, m, 65535):
             hi = min(lo + 65535, m)
             src = coeffs if one_d else coeffs[lo:hi]
@@ -586,23 +587,27 @@ def merkle_build_blake3(leaves):
     levels[0] = leaves, levels[-1] = (1, 32) holding the root
     (prover/cuda_primitives.py:1388-1402).  All levels above the leaves are built by one library
     call (up to nine levels per launch) into one buffer; the list holds views of it."""
+    levels = merkle_levels(leaves)
+    root = levels[-1].view(-1)[:32].clone()
+    return root, levels
+
+
+def merkle_levels(leaves):
+    """The levels of merkle_build_blake3 without a copy of the root: it is the one row of the last level."""
     assert leaves.dim() == 2 and leaves.size(1) == 32
     assert leaves.dtype == torch.uint8 and leaves.is_cuda
     cur = leaves.contiguous()
-    levels = [leaves]
     k = int(cur.size(0))
-    if k > 1:
-        L = _lib.lib()
-        buf = torch.empty((int(L.vi_merkle_tree_nodes(k)), 32), dtype=torch.uint8, device=cur.device)
-        with torch.cuda.device(cur.device):
-            _lib.check(L.vi_merkle_tree(cur.data_ptr(), k, buf.data_ptr(), _lib.stream_ptr()))
-        off = 0
-        while k > 1:
-            k = (k + 1) // 2
-            levels.append(buf[off:off + k])
-            off += k
-    root = levels[-1].view(-1)[:32].clone()
-    return root, levels
+    if k <= 1:
+        return [leaves]
+    sizes = []
+    while k > 1:
+        k = (k + 1) // 2
+        sizes.append(k)
+    buf = torch.empty((sum(sizes), 32), dtype=torch.uint8, device=cur.device)
+    with _lib.on_device(cur.device):
+        _lib.check(_lib.lib().vi_merkle_tree(cur.data_ptr(), int(cur.size(0)), buf.data_ptr(), _lib.stream_ptr()))
+    return [leaves, *buf.split(sizes)]
 
 
 # ---- combiner challenges, CSR matvec, LogUp multiplicities (prover/cuda_primitives.py:512-592, 1008-1052) ----

@@ -19,7 +19,7 @@ _QTYPE_ID = {"Q4_K": 4, "Q5_K": 5, "Q6_K": 6}
 def kquant_to_field(raw_u8_cuda: torch.Tensor, qtype: str, S: int) -> torch.Tensor:
     """raw K-quant bytes -> flat uint64 field tensor of n_blocks*256 integers."""
     assert qtype in _QTYPE_ID, f"kquant_to_field: unsupported type {qtype}"
-    raw = raw_u8_cuda.reshape(-1)
+    raw = raw_u8_cuda if raw_u8_cuda.is_contiguous() else raw_u8_cuda.reshape(-1)
     if not (raw.is_cuda and raw.dtype == torch.uint8 and raw.is_contiguous()):
         raise RuntimeError("kquant_to_field: raw must be a contiguous CUDA uint8 tensor")
     bb = BLOCK_BYTES[qtype]
@@ -28,7 +28,7 @@ def kquant_to_field(raw_u8_cuda: torch.Tensor, qtype: str, S: int) -> torch.Tens
         raise RuntimeError(f"kquant_to_field: {raw.numel()} bytes is not a multiple of the {bb}-byte {qtype} block")
     out = torch.empty(n_blocks * QK_K, dtype=torch.uint64, device=raw.device)
     if n_blocks:
-        with torch.cuda.device(raw.device):
+        with _lib.on_device(raw.device):
             _lib.check(_lib.lib().vi_kquant_to_field(_QTYPE_ID[qtype], raw.data_ptr(), n_blocks, float(S),
                                                      out.data_ptr(), _lib.stream_ptr()))
     return out
@@ -40,7 +40,7 @@ def kquant_to_field_transposed(raw_u8_cuda: torch.Tensor, qtype: str, S: int, d_
     .view(uint64).reshape(-1)` -- the (k_in, n_out) order in which the loader commits an expert
     matrix (prover/loader.py:427-436) -- in one pass, without the intermediate decoded matrix."""
     assert qtype in _QTYPE_ID, f"kquant_to_field_transposed: unsupported type {qtype}"
-    raw = raw_u8_cuda.reshape(-1)
+    raw = raw_u8_cuda if raw_u8_cuda.is_contiguous() else raw_u8_cuda.reshape(-1)
     if not (raw.is_cuda and raw.dtype == torch.uint8 and raw.is_contiguous()):
         raise RuntimeError("kquant_to_field_transposed: raw must be a contiguous CUDA uint8 tensor")
     bb = BLOCK_BYTES[qtype]
@@ -51,7 +51,7 @@ def kquant_to_field_transposed(raw_u8_cuda: torch.Tensor, qtype: str, S: int, d_
     d_in = n_blocks // d_out * QK_K
     out = torch.empty(n_blocks * QK_K, dtype=torch.uint64, device=raw.device)
     if n_blocks:
-        with torch.cuda.device(raw.device):
+        with _lib.on_device(raw.device):
             _lib.check(_lib.lib().vi_kquant_to_field_transposed(_QTYPE_ID[qtype], raw.data_ptr(), d_out, d_in, float(S),
                                                                 out.data_ptr(), _lib.stream_ptr()))
     return out
