@@ -343,6 +343,13 @@ int vi_gl_spmv(const uint64_t *values, const uint64_t *col_idx, const uint64_t *
 int vi_lookup_multiplicities(const uint64_t *x, int64_t n_x, const uint64_t *table, int64_t n_table, int table_is_range,
                              uint64_t *mult, void *stream);
 
+/* The same counts through per-workgroup histograms in LDS and, for a table that is not a range, a hash table (of up to
+ * 2^30 entries): mult[j] = (accumulate: mult[j] +) #{i : j is the first index with table[j] == x[i]}.
+ * ws: vi_lookup_histogram_workspace_bytes() bytes of device scratch. */
+size_t vi_lookup_histogram_workspace_bytes(int64_t n_x, int64_t n_table, int table_is_range);
+int vi_lookup_histogram(const uint64_t *x, int64_t n_x, const uint64_t *table, int64_t n_table, int table_is_range, int accumulate,
+                        uint64_t *mult, void *ws, size_t ws_bytes, void *stream);
+
 /* ---------------------------------------------------------------------------------------------
  * Measurement hook (no counterpart in the reference): the issue rate of the integer VALU instructions the field
  * arithmetic and the hashing consist of, which is the bound their kernels are put against.

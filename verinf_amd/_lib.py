@@ -37,6 +37,7 @@ EXPORTS = [
     "vi_merkle_level", "vi_merkle_tree_nodes", "vi_merkle_tree", "vi_row_prg",
     "vi_eq_vector", "vi_mle_eval_workspace_bytes", "vi_mle_eval",
     "vi_challenge", "vi_gl_spmv", "vi_lookup_multiplicities",
+    "vi_lookup_histogram_workspace_bytes", "vi_lookup_histogram",
     "vi_valu_probe_count", "vi_valu_probe_name", "vi_wall_clock_khz", "vi_valu_probe",
 ]
 
@@ -117,6 +118,10 @@ def lib():
     L.vi_challenge.argtypes = [vp, vp, c_int, vp, i64, vp, vp]
     L.vi_gl_spmv.argtypes = [vp, vp, vp, i64, i64, vp, vp, vp, c_int, vp, vp]
     L.vi_lookup_multiplicities.argtypes = [vp, i64, vp, i64, c_int, vp, vp]
+    L.vi_lookup_histogram_workspace_bytes.restype = sz
+    L.vi_lookup_histogram_workspace_bytes.argtypes = [i64, i64, c_int]
+    L.vi_lookup_histogram.argtypes = [vp, i64, vp, i64, c_int, c_int, vp, vp, sz, vp]
+    L.vi_lookup_histogram.restype = c_int
     L.vi_read_back.argtypes = [vp, i64, vp, sz, vp]
     L.vi_read_back.restype = c_int
     L.vi_upload_words.argtypes = [vp, i64, vp, vp]

@@ -310,27 +310,6 @@ __global__ __launch_bounds__(BLOCK) void k_spmv(const u64 *__restrict__ values, 
     }
 }
 
-// LogUp multiplicities (prover/kernels/gl_extras.cuh:118-150): mult[j] += 1 for the first j with
-// table[j] == x[i]; values that are not in the table count nowhere.  t_len_range > 0 says the
-// table is literally 0 .. t_len_range-1, so x[i] is its own index.
-__global__ __launch_bounds__(BLOCK) void k_lookup_mult(const u64 *__restrict__ x, i64 n_x, const u64 *__restrict__ table, i64 n_table,
-                                                       i64 t_len_range, unsigned long long *__restrict__ mult) {
-    const i64 stride = (i64)gridDim.x * BLOCK;
-    for (i64 i = (i64)blockIdx.x * BLOCK + threadIdx.x; i < n_x; i += stride) {
-        const u64 xi = x[i];
-        if (t_len_range > 0) {
-            if (xi < (u64)t_len_range) atomicAdd(&mult[xi], 1ULL);
-            continue;
-        }
-        for (i64 j = 0; j < n_table; ++j) {
-            if (table[j] == xi) {
-                atomicAdd(&mult[j], 1ULL);
-                break;
-            }
-        }
-    }
-}
-
 inline i64 chunks_of(i64 m) { return m <= 0 ? 1 : (m + ROWS_PER_CHUNK - 1) / ROWS_PER_CHUNK; }
 
 }  // namespace
@@ -510,17 +489,6 @@ int vi_gl_spmv(const uint64_t *values, const uint64_t *col_idx, const uint64_t *
                            label, label_len, (i64)n_rows, y);
     }
     VI_LAUNCH_CHECK("k_spmv");
-    return VI_OK;
-}
-
-int vi_lookup_multiplicities(const uint64_t *x, int64_t n_x, const uint64_t *table, int64_t n_table, int table_is_range,
-                             uint64_t *mult, void *stream) {
-    if (n_x < 0 || n_table < 0) return vi::fail(VI_EINVAL, "vi_lookup_multiplicities: n_x = %lld, n_table = %lld", (long long)n_x, (long long)n_table);
-    if (n_x == 0 || n_table == 0) return VI_OK;
-    if (!x || !mult || (!table_is_range && !table)) return vi::fail(VI_EINVAL, "vi_lookup_multiplicities: null pointer");
-    hipLaunchKernelGGL(k_lookup_mult, dim3(capped_grid(n_x)), dim3(BLOCK), 0, (hipStream_t)stream, x, (i64)n_x, table, (i64)n_table,
-                       (i64)(table_is_range ? n_table : 0), (unsigned long long *)mult);
-    VI_LAUNCH_CHECK("k_lookup_mult");
     return VI_OK;
 }
 

@@ -714,16 +714,26 @@ def lookup_multiplicities_into(x, table, mult, label=""):
         raise RuntimeError("mult length must match table")
     if x.numel() == 0 or table.numel() == 0:
         return
-    _lib.check(_lib.lib().vi_lookup_multiplicities(x.data_ptr(), int(x.numel()), table.data_ptr(), int(table.numel()),
-                                                   1 if _is_range_table(table) else 0, mult.data_ptr(), _lib.stream_ptr()))
+    _histogram(x, table, mult, 1)
+
+
+def _histogram(x, table, mult, accumulate):
+    L = _lib.lib()
+    n_x, n_t, is_range = int(x.numel()), int(table.numel()), 1 if _is_range_table(table) else 0
+    need = L.vi_lookup_histogram_workspace_bytes(n_x, n_t, is_range)
+    ws = _lib.workspace(need, x.device, "lookup").data_ptr() if need else None
+    _lib.check(L.vi_lookup_histogram(x.data_ptr(), n_x, table.data_ptr(), n_t, is_range, accumulate, mult.data_ptr(), ws, need,
+                                     _lib.stream_ptr()))
 
 
 def lookup_multiplicities(x, table):
     """Per-table-entry multiplicity histogram (prover/cuda_primitives.py:1426-1428)."""
     _check_u64(x, "x")
     _check_u64(table, "table")
-    mult = torch.zeros(int(table.numel()), dtype=torch.int64, device=table.device).view(torch.uint64)
     if x.dim() != 1 or table.dim() != 1:
         raise RuntimeError("x and table must be 1-D")
-    lookup_multiplicities_into(x, table, mult)
+    if x.numel() == 0 or table.numel() == 0:
+        return torch.zeros(int(table.numel()), dtype=torch.int64, device=table.device).view(torch.uint64)
+    mult = torch.empty_like(table)
+    _histogram(x, table, mult, 0)
     return mult
