@@ -1,0 +1,82 @@
+"""GPU parity of the single-launch transforms and extensions of short rows: every row length and direction, ragged batches,
+narrow and strided sources, coefficients beside, in place and alone, one to many cosets -- against the oracle, and against
+the multi-pass kernels by running the same rows inside a batch too large for the single launch."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+from oracle import oracle as O  # noqa: E402
+from tests.gpu_util import P, rand_field, to_dev, to_np  # noqa: E402
+
+
+@pytest.fixture(scope="module")
+def cp():
+    from verinf_amd.prover import cuda_primitives
+    return cuda_primitives
+
+
+@pytest.mark.parametrize("logn", range(3, 12))
+@pytest.mark.parametrize("m", [1, 3, 129])
+def test_transforms(cp, logn, m):
+    n = 1 << logn
+    a = rand_field((m, n), 10 * logn + m)
+    a[0, :3] = [P - 1, 0, P - 1]
+    raw = a.copy()
+    raw[-1, -2:] = [np.uint64((1 << 64) - 1), np.uint64(P + 1)]                        # words that are not canonical
+    a[-1, -2:] = [np.uint64(((1 << 64) - 1) % P), 1]
+    d = to_dev(raw)
+    cp.ntt_forward_batched(d)
+    fwd = to_np(d)
+    assert np.array_equal(fwd, O.ntt_rows(a))
+    big = to_dev(np.concatenate([a] * ((1 << 20) // a.size + 1)))                      # the multi-pass kernels
+    cp.ntt_forward_batched(big)
+    assert np.array_equal(to_np(big)[-m:], fwd)
+    cp.ntt_inverse_batched(d)
+    assert np.array_equal(to_np(d), a)
+    inv = to_dev(a)
+    cp.ntt_inverse_batched(inv)
+    assert np.array_equal(to_np(inv), O.ntt_rows(a, inverse=True))
+
+
+@pytest.mark.parametrize("logk", range(3, 13))
+@pytest.mark.parametrize("log_rho", [0, 1, 2, 3, 5])
+@pytest.mark.parametrize("m", [1, 5])
+def test_extensions(cp, logk, log_rho, m):
+    K, N = 1 << logk, 1 << (logk + log_rho)
+    for w in (K, K - 3, 1):
+        a = rand_field((m, w), 100 * logk + 10 * log_rho + w)
+        wide = torch.empty((m, w + 5), dtype=torch.int64, device="cuda").view(torch.uint64)
+        wide.view(torch.int64)[:, :w] = to_dev(a).view(torch.int64)
+        src = wide[:, :w]                                                              # strided rows
+        want = O.coset_lde_rows(a, K, N, 7)
+        assert np.array_equal(to_np(cp.coset_lde(src, K, N)), want)
+        coeffs, code = cp.coset_lde_with_coeffs(src, K, N)
+        assert np.array_equal(to_np(code), want)
+        only, none = cp.coset_lde_with_coeffs(src, K, N, need_codewords=False)
+        assert none is None and torch.equal(only, coeffs)
+        assert np.array_equal(to_np(cp.coset_extend(coeffs, K, N)), want)
+        back = coeffs.clone()
+        cp.ntt_forward_batched(back)
+        assert np.array_equal(to_np(back)[:, :w], a)
+    full = rand_field((m, K), 9 + logk)
+    own = to_dev(full)
+    coeffs, code = cp.coset_lde_with_coeffs(own, K, N, in_place=True)
+    assert coeffs.data_ptr() == own.data_ptr()
+    assert np.array_equal(to_np(code), O.coset_lde_rows(full, K, N, 7))
+    back = coeffs.clone()
+    cp.ntt_forward_batched(back)
+    assert np.array_equal(to_np(back), full)
+
+
+@pytest.mark.parametrize("logk,log_rho,m", [(5, 1, 70000), (6, 2, 9000), (10, 1, 1100), (8, 2, 1025), (12, 2, 300), (9, 3, 300)])
+def test_larger_batches(cp, logk, log_rho, m):
+    """All cosets in one workgroup, and the first batches beyond the single launch."""
+    K, N = 1 << logk, 1 << (logk + log_rho)
+    a = rand_field((m, K), logk)
+    got = to_np(cp.coset_lde(to_dev(a), K, N))
+    rows = sorted({0, 1, m // 3, m // 2, m - 2, m - 1})
+    assert np.array_equal(got[rows], O.coset_lde_rows(np.ascontiguousarray(a[rows]), K, N, 7))
+    coeffs, code = cp.coset_lde_with_coeffs(to_dev(a), K, N, in_place=True)
+    assert np.array_equal(to_np(code), got)

@@ -234,7 +234,7 @@ struct DeviceTables {
 
 std::mutex g_mu;
 std::map<std::tuple<int, int, int>, DeviceTables *> g_tables;        // (device, logn, inverse + 2 * row split)
-std::map<std::pair<int, int>, u64 *> g_twl;                          // (device, inverse)
+std::map<std::pair<int, int>, u64 *> g_twl;                          // (device, inverse + 2 * all 4096 powers)
 std::map<std::tuple<int, int, int, u64>, u64 *> g_pre;               // (device, logK, logN, shift)
 
 int upload(const std::vector<u64> &h, u64 **out) {
@@ -249,12 +249,13 @@ int upload(const std::vector<u64> &h, u64 **out) {
     return VI_OK;
 }
 
-int get_twl(int dev, int inv, const u64 **out) {
-    auto key = std::make_pair(dev, inv);
+// full: all 4096 powers (small transforms)
+int get_twl(int dev, int inv, const u64 **out, bool full = false) {
+    auto key = std::make_pair(dev, inv + (full ? 2 : 0));
     auto it = g_twl.find(key);
     if (it == g_twl.end()) {
         u64 *d = nullptr;
-        int rc = upload(make_twl(inv), &d);
+        int rc = upload(full ? make_twf(inv) : make_twl(inv), &d);
         if (rc) return rc;
         it = g_twl.emplace(key, d).first;
     }
@@ -486,6 +487,53 @@ i64 max_lde_chunk(int logK, int logN) {
 
 }  // namespace
 
+#include "ntt_small.hpp"
+
+namespace {
+
+// Where the single launch of ntt_small.hpp is the faster one; sweep over row lengths and batch sizes, us per call, the
+// passes of k_ntt_fast against it.
+//
+// Transforms of 8 and 16 points: always (2^26 points 465 against 241; the passes have no register kernel below 32).  32 to
+// 2048 points: up to 2^20 points in the batch (2^16 points 6.5 to 11.0 against 4.3 to 7.1; 2^20 points 7.4 to 11.8 against
+// 6.1 to 11.6; beyond that the sixteen points a thread of the passes holds need fewer instructions).  A row of 4096 fills a
+// CU's issue slots either way (11.2 against 11.0).
+bool small_ntt_pays(i64 m, int logn) {
+    if (logn < SMALL_MIN_LOG || logn >= SMALL_MAX_LOG) return false;
+    return logn <= 4 || (m << logn) <= ((i64)1 << 20);
+}
+
+// Extensions by the number of cosets and the points written: with two cosets always up to K = 2^7 and at 2^10 (the passes
+// store a column of such a row pair by pair, 2^26 points 2613 against 272 at K = 2^5, 670 against 528 at 2^10), with four up
+// to K = 2^6 and at 2^10; otherwise while the batch leaves SIMDs idle (2^16 points 17 to 50 against 5 to 23; the limits are
+// where the two meet).  More cosets spread a thread's stores over more lines, so the limits fall.
+bool small_lde_pays(i64 m, int logK, int logN, bool in_place) {
+    if (logK < SMALL_MIN_LOG || logK > SMALL_MAX_LOG) return false;
+    const int log_rho = logN - logK;
+    if (log_rho > 8) return false;
+    int log_most;
+    if (log_rho <= 1) log_most = logK <= 7 || logK == 10 ? 62 : (logK == 11 ? 24 : 21);
+    else if (log_rho == 2) log_most = logK <= 6 || logK == 10 ? 62 : (logK <= 9 ? 21 : (logK == 11 ? 23 : 22));
+    else {
+        // in place one workgroup has to run through the cosets of its rows: eight or more of them are the longer chain
+        if (in_place && logK > 4) return false;
+        log_most = logK <= 4 ? 22 : (logK <= 9 ? 19 : 20);
+    }
+    return m <= (((i64)1 << log_most) >> logN);
+}
+
+// the tables of the small transforms on the current device
+int get_small_tables(const u64 **inv, const u64 **fwd) {
+    int dev = 0;
+    VI_HIP(hipGetDevice(&dev));
+    std::lock_guard<std::mutex> lock(g_mu);
+    int rc = inv ? get_twl(dev, 1, inv, true) : VI_OK;
+    if (!rc && fwd) rc = get_twl(dev, 0, fwd, true);
+    return rc;
+}
+
+}  // namespace
+
 extern "C" {
 
 size_t vi_ntt_workspace_bytes(int64_t m, int64_t n) {
@@ -502,6 +550,15 @@ int vi_ntt_batched(uint64_t *rows, int64_t m, int64_t n, int inverse, void *ws, 
     if (m == 0) return VI_OK;
     if (!rows) return vi::fail(VI_EINVAL, "vi_ntt_batched: null rows");
     const int logn = vi::ilog2(n);
+    if (small_ntt_pays(m, logn)) {
+        const u64 *tab = nullptr;
+        int rc = inverse ? get_small_tables(&tab, nullptr) : get_small_tables(nullptr, &tab);
+        if (rc) return rc;
+        const u64 scale = inverse ? ntt::inverse((u64)n % gl::P) : 1;
+        small_dispatch(logn, [&](auto l) { launch_small_ntt<decltype(l)::value>(rows, m, tab, scale, inverse != 0, (hipStream_t)stream); });
+        VI_LAUNCH_CHECK("k_small_ntt");
+        return VI_OK;
+    }
     const Tables *T = nullptr;
     if (row_launch_on() && row_single_ok(logn)) {
         int rc = get_tables(logn, inverse ? 1 : 0, &T, true);
@@ -558,6 +615,7 @@ int64_t vi_coset_lde_launches(int64_t m, int64_t K, int64_t N, size_t ws_bytes) 
     size_t one = vi_coset_lde_min_workspace_bytes(K, N);
     if (!one || m <= 0 || ws_bytes < one) return 0;
     i64 chunk = (i64)(ws_bytes / one);
+    if (small_lde_pays(m, vi::ilog2(K), vi::ilog2(N), false)) return 1;
     if (chunk > m) chunk = m;
     if (chunk > max_lde_chunk(vi::ilog2(K), vi::ilog2(N))) chunk = max_lde_chunk(vi::ilog2(K), vi::ilog2(N));
     const i64 n_chunks = (m + chunk - 1) / chunk;         // balancing keeps the chunk count
@@ -628,6 +686,29 @@ int coset_lde_impl(const char *who, const uint64_t *in, int64_t m, int64_t width
     chunk = (m + ((m + chunk - 1) / chunk) - 1) / ((m + chunk - 1) / chunk);   // same chunk count, even sizes
     const Tables *Ti = nullptr, *Tf = nullptr;
     const u64 *pre = nullptr;
+    if (small_lde_pays(m, logK, logN, coeffs == in)) {
+        SmallLde S{};
+        int rc = get_small_tables(&S.tab_inv, &S.tab_fwd);
+        if (!rc && out) rc = get_pre(logK, logN, shift, &S.pre);
+        if (rc) return rc;
+        S.in = in;
+        S.m = m;
+        S.width = width;
+        S.in_stride = in_stride;
+        S.coeffs = in_is_coeffs ? nullptr : coeffs;
+        S.coeffs_stride = coeffs_stride;
+        S.out = out;
+        S.out_stride = out_stride;
+        S.scale = ntt::inverse((u64)K % gl::P);
+        S.log_rho = logN - logK;
+        // one workgroup per coset while that fills idle SIMDs; a batch with a wavefront or more per SIMD saves the repeated
+        // inverse transforms instead (512 rows of 2^9 -> 2^11: 21 us, 24 with one coset each; 256 rows: 20 and 15)
+        const int log_full = logK <= 10 ? 18 : (logK == 11 ? 19 : 20);
+        S.cosets = !out || coeffs == in || (m << logK) >= ((i64)1 << log_full) ? 1 << S.log_rho : 1;
+        small_dispatch(logK, [&](auto l) { launch_small_lde<decltype(l)::value>(S, in_is_coeffs, (hipStream_t)stream); });
+        VI_LAUNCH_CHECK("k_small_lde");
+        return VI_OK;
+    }
     int rc = get_tables(logK, 1, &Ti);
     if (!rc) rc = get_tables(logK, 0, &Tf);
     if (!rc) rc = get_pre(logK, logN, shift, &pre);

@@ -102,6 +102,16 @@ inline std::vector<u64> make_twl(int inv) {
     return t;
 }
 
+// w_4096^j (or inverse), all of them: the twiddles of the single-launch small transforms
+inline std::vector<u64> make_twf(int inv) {
+    std::vector<u64> t((size_t)1 << TWL_LOG);
+    u64 w = root_of_unity(TWL_LOG);
+    if (inv) w = inverse(w);
+    u64 c = 1;
+    for (auto &x : t) { x = c; c = gl::mul(c, w); }
+    return t;
+}
+
 // pre[t][i] = (shift * w_N^t)^i, t < rho, i < K: the coefficient twist that moves the
 // evaluation domain of coset t onto shift * w_N^t * <w_K>
 // (layergkr/gpu.py:128-138 for t = 0; prover/core.py:702-718 for the rho cosets)
