@@ -302,6 +302,11 @@ int vi_merkle_tree(const uint8_t *leaves, int64_t count, uint8_t *levels_out, vo
 int vi_row_prg(const uint8_t *seed, const uint64_t *row_indices, int64_t row_offset, int64_t n_rows, int64_t slack,
                uint64_t *out, int64_t out_stride, void *stream);
 
+/* Padded rows: out (n_rows x width, contiguous) = [messages row r (ell words, pitch in_stride) | pad of width - ell words as
+ * vi_row_prg gives for row_offset + r].  One launch for the copy and the pad of prover/core.py:783-794. */
+int vi_pad_rows(const uint8_t *seed, int64_t row_offset, const uint64_t *messages, int64_t n_rows, int64_t ell, int64_t in_stride,
+                int64_t width, uint64_t *out, void *stream);
+
 /* ---------------------------------------------------------------------------------------------
  * Multilinear helpers around the sumchecks.  A point z is a HOST array of n_vars <= 32 words (reduced
  * mod p by the callee).

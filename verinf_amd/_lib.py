@@ -34,7 +34,7 @@ EXPORTS = [
     "vi_sumcheck_workspace_bytes", "vi_sumcheck_eval", "vi_sumcheck_eval_static", "vi_sumcheck_fold_eval",
     "vi_sumcheck_prove", "vi_sumcheck_prove_coins_workspace_bytes", "vi_sumcheck_prove_coins",
     "vi_hash_columns_workspace_bytes", "vi_hash_columns", "vi_hash_columns_update", "vi_hash_columns_finalize",
-    "vi_merkle_level", "vi_merkle_tree_nodes", "vi_merkle_tree", "vi_row_prg",
+    "vi_merkle_level", "vi_merkle_tree_nodes", "vi_merkle_tree", "vi_row_prg", "vi_pad_rows",
     "vi_eq_vector", "vi_mle_eval_workspace_bytes", "vi_mle_eval",
     "vi_challenge", "vi_gl_spmv", "vi_lookup_multiplicities",
     "vi_lookup_histogram_workspace_bytes", "vi_lookup_histogram",
@@ -115,6 +115,8 @@ def lib():
     L.vi_merkle_tree_nodes.argtypes = [i64]
     L.vi_merkle_tree.argtypes = [vp, i64, vp, vp]
     L.vi_row_prg.argtypes = [vp, vp, i64, i64, i64, vp, i64, vp]
+    L.vi_pad_rows.argtypes = [vp, i64, vp, i64, i64, i64, i64, vp, vp]
+    L.vi_pad_rows.restype = c_int
     L.vi_challenge.argtypes = [vp, vp, c_int, vp, i64, vp, vp]
     L.vi_gl_spmv.argtypes = [vp, vp, vp, i64, i64, vp, vp, vp, c_int, vp, vp]
     L.vi_lookup_multiplicities.argtypes = [vp, i64, vp, i64, c_int, vp, vp]

@@ -76,6 +76,114 @@ __device__ __forceinline__ void compress(u32 (&cv)[8], const u32 (&m)[16], u64 c
     for (int i = 0; i < 8; ++i) cv[i] = s[i] ^ s[i + 8];
 }
 
+// ---- one compression on four lanes ------------------------------------------------------------------------------
+// A compression is 681 instructions in a row, 1.3 us for the wavefront that runs it alone; the upper levels of a tree and
+// short messages of few columns are such chains.  Lane q of four holds column q of the state, so the four G functions of a
+// half round are one, and the rows turn by lane permutes for the diagonal half: 330 instructions, at 1.9 times the issue
+// slots altogether, so only where the chip has them to spare.
+struct QuadSchedule {
+    int at[7][4];                            // message words of this lane: two of each half round, per round
+};
+
+__device__ __forceinline__ int quad_pick(int q, int a, int b, int c, int d) { return q < 2 ? (q == 0 ? a : b) : (q == 2 ? c : d); }
+
+template <int R>
+__device__ __forceinline__ void quad_schedule_round(QuadSchedule &S, int q) {
+    S.at[R][0] = quad_pick(q, sched(R, 0), sched(R, 2), sched(R, 4), sched(R, 6));
+    S.at[R][1] = quad_pick(q, sched(R, 1), sched(R, 3), sched(R, 5), sched(R, 7));
+    S.at[R][2] = quad_pick(q, sched(R, 8), sched(R, 10), sched(R, 12), sched(R, 14));
+    S.at[R][3] = quad_pick(q, sched(R, 9), sched(R, 11), sched(R, 13), sched(R, 15));
+    if constexpr (R < 6) quad_schedule_round<R + 1>(S, q);
+}
+
+// the value of lane (q + N) mod 4 of the quad
+template <int N>
+__device__ __forceinline__ u32 quad_turn(u32 v) {
+    constexpr int perm = ((0 + N) & 3) | (((1 + N) & 3) << 2) | (((2 + N) & 3) << 4) | (((3 + N) & 3) << 6);
+    return (u32)__builtin_amdgcn_mov_dpp((int)v, perm, 0xF, 0xF, true);
+}
+
+// lo, hi: words q and 4 + q of the chaining value, in and out.  msg: the sixteen message words of the quad in LDS.  All four
+// lanes of a quad take part.
+__device__ __forceinline__ void quad_compress(u32 &lo, u32 &hi, const u32 *msg, const QuadSchedule &S, int q, u64 counter, u32 block_len, u32 flags) {
+    u32 m[7][4];
+#pragma unroll
+    for (int r = 0; r < 7; ++r)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) m[r][j] = msg[S.at[r][j]];
+    u32 a = lo, b = hi, c = IV[q], d = q == 0 ? (u32)counter : (q == 1 ? (u32)(counter >> 32) : (q == 2 ? block_len : flags));
+#pragma unroll
+    for (int r = 0; r < 7; ++r) {
+        B3_G(a, b, c, d, m[r][0], m[r][1])
+        b = quad_turn<1>(b);
+        c = quad_turn<2>(c);
+        d = quad_turn<3>(d);
+        B3_G(a, b, c, d, m[r][2], m[r][3])
+        b = quad_turn<3>(b);
+        c = quad_turn<2>(c);
+        d = quad_turn<1>(d);
+    }
+    lo = a ^ c;
+    hi = b ^ d;
+}
+
+// LDS written by lanes of this wavefront, to be read by others of it
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// k_chunk_cvs with four lanes per column (up to QUAD_MAX chunk-columns, see vi_hash_columns_update): 64 columns per workgroup
+constexpr int QUAD_COLS = BLOCK / 4, QUAD_PITCH = 17;
+
+__global__ __launch_bounds__(BLOCK) void k_chunk_cvs_quad(const u64 *__restrict__ rows, i64 slab_rows, i64 n, i64 stride, i64 chunk0,
+                                                          int single_root, u32 *__restrict__ cvs) {
+    __shared__ u32 msg[QUAD_COLS * QUAD_PITCH];
+    const int q = threadIdx.x & 3, local = threadIdx.x >> 2;
+    const i64 col = (i64)blockIdx.x * QUAD_COLS + local;
+    const bool there = col < n;
+    const i64 c = blockIdx.y;
+    const i64 r0 = c * ROWS_PER_CHUNK;
+    const i64 nrows = (slab_rows - r0 < ROWS_PER_CHUNK) ? (slab_rows - r0) : ROWS_PER_CHUNK;   // >= 0
+    const int n_blocks = nrows == 0 ? 1 : (int)((nrows + ROWS_PER_BLOCK - 1) / ROWS_PER_BLOCK);
+    const u64 *p = rows + r0 * stride + (there ? col : 0);
+    QuadSchedule S;
+    quad_schedule_round<0>(S, q);
+    u32 *mine = msg + local * QUAD_PITCH;
+    u32 lo = IV[q], hi = IV[4 + q];
+    // rows q and 4 + q of a block are this lane's to fetch, a block ahead
+    u64 v[2];
+    auto fetch = [&](int b) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const i64 r = (i64)b * ROWS_PER_BLOCK + q + 4 * i;
+            v[i] = r < nrows ? p[r * stride] : 0;
+        }
+    };
+    fetch(0);
+    for (int b = 0; b < n_blocks; ++b) {
+        wave_lds_sync();                     // the block before has been read
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            mine[2 * (q + 4 * i)] = (u32)v[i];
+            mine[2 * (q + 4 * i) + 1] = (u32)(v[i] >> 32);
+        }
+        wave_lds_sync();
+        if (b + 1 < n_blocks) fetch(b + 1);
+        const i64 left = nrows - (i64)b * ROWS_PER_BLOCK;
+        const int here = left >= ROWS_PER_BLOCK ? ROWS_PER_BLOCK : (int)left;
+        u32 flags = 0;
+        if (b == 0) flags |= CHUNK_START;
+        if (b == n_blocks - 1) flags |= CHUNK_END | (single_root ? ROOT : 0u);
+        quad_compress(lo, hi, mine, S, q, (u64)(chunk0 + c), (u32)(here * 8), flags);
+    }
+    if (there) {
+        u32 *o = cvs + ((chunk0 + c) * n + col) * 8;
+        o[q] = lo;
+        o[4 + q] = hi;
+    }
+}
+
 // Chaining value of chunk (chunk0 + blockIdx.y) of every column.
 //   rows          first row of the slab (row pitch `stride` words), slab_rows rows in it
 //   single_root   the whole message is this one chunk: its last block carries ROOT
@@ -175,9 +283,12 @@ __global__ __launch_bounds__(BLOCK) void k_merkle_level(const u32 *__restrict__ 
 // level j (1-based) of this launch starts at out + 8 * (c_1 + ... + c_{j-1}) words, c_j = ceil(c_{j-1} / 2),
 // c_0 = count.  The odd last node of a level is paired with itself, as in k_merkle_level.
 constexpr int SUB_LEVELS = 9;
+constexpr int QUAD_LEVEL = 3;                                  // first level of a launch with four lanes per parent (2^(9-3) * 4 = BLOCK)
 
 __global__ __launch_bounds__(BLOCK) void k_merkle_subtree(const u32 *__restrict__ nodes, i64 count, int levels, u32 *__restrict__ out) {
     __shared__ u32 buf[2][BLOCK * 8];
+    QuadSchedule S;
+    quad_schedule_round<0>(S, threadIdx.x & 3);
     const i64 base = (i64)blockIdx.x << SUB_LEVELS;            // first input node of the block
     i64 c_prev = count, off = 0;                               // nodes of the level below, word offset of this level in out
     for (int j = 1; j <= levels; ++j) {
@@ -185,7 +296,24 @@ __global__ __launch_bounds__(BLOCK) void k_merkle_subtree(const u32 *__restrict_
         const i64 first = base >> j;                           // first node of level j in the block
         const int in_block = 1 << (SUB_LEVELS - j);
         const i64 i = first + threadIdx.x;
-        if ((int)threadIdx.x < in_block && i < c) {
+        if (j >= QUAD_LEVEL) {
+            // at most 64 parents: four lanes each (all levels but the first find their children in LDS)
+            const int local = threadIdx.x >> 2, q = threadIdx.x & 3;
+            const i64 ip = first + local;
+            if (local < in_block && ip < c) {                  // the same for the four lanes of a parent
+                u32 *pair = buf[j & 1] + (2 * local) * 8;
+                if (2 * ip + 1 >= c_prev) {                    // no right child: the left one twice
+                    pair[8 + q] = pair[q];
+                    pair[12 + q] = pair[4 + q];
+                    wave_lds_sync();
+                }
+                u32 lo = IV[q], hi = IV[4 + q];
+                quad_compress(lo, hi, pair, S, q, 0, 64, CHUNK_START | CHUNK_END | ROOT);
+                u32 *o = out + off + ip * 8, *keep = buf[(j + 1) & 1] + local * 8;
+                o[q] = keep[q] = lo;
+                o[4 + q] = keep[4 + q] = hi;
+            }
+        } else if ((int)threadIdx.x < in_block && i < c) {
             u32 m[16], cv[8];
             const bool has_right = 2 * i + 1 < c_prev;
             if (j == 1) {
@@ -220,12 +348,7 @@ __global__ __launch_bounds__(BLOCK) void k_merkle_subtree(const u32 *__restrict_
 // that stores are coalesced; the reference gives a whole row to one thread.
 // row = row_indices[r] when row_indices is given, else the 32-bit sum row_offset + r (the
 // reference's contiguous variant computes the row number in uint32).
-__global__ __launch_bounds__(BLOCK) void k_row_prg(const u32 *__restrict__ seed, const u64 *__restrict__ row_indices, u32 row_offset,
-                                                   i64 n_rows, i64 slack, u64 *__restrict__ out, i64 out_stride) {
-    const i64 g = (i64)blockIdx.x * BLOCK + threadIdx.x;
-    if (g >= n_rows * slack) return;
-    const i64 r = g / slack, k = g - r * slack;
-    const u64 row = row_indices ? row_indices[r] : (u64)(u32)(row_offset + (u32)r);
+__device__ __forceinline__ u64 prg_word(const u32 *__restrict__ seed, u64 row, i64 k) {
     u32 m[16], cv[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) { m[i] = seed[i]; cv[i] = IV[i]; }
@@ -234,7 +357,26 @@ __global__ __launch_bounds__(BLOCK) void k_row_prg(const u32 *__restrict__ seed,
     m[12] = m[13] = m[14] = m[15] = 0;
     compress(cv, m, 0, 48, CHUNK_START | CHUNK_END | ROOT);
     const u64 raw = ((u64)cv[1] << 32) | cv[0];
-    out[r * out_stride + k] = raw >= 0xFFFFFFFF00000001ull ? raw - 0xFFFFFFFF00000001ull : raw;
+    return raw >= 0xFFFFFFFF00000001ull ? raw - 0xFFFFFFFF00000001ull : raw;
+}
+
+__global__ __launch_bounds__(BLOCK) void k_row_prg(const u32 *__restrict__ seed, const u64 *__restrict__ row_indices, u32 row_offset,
+                                                   i64 n_rows, i64 slack, u64 *__restrict__ out, i64 out_stride) {
+    const i64 g = (i64)blockIdx.x * BLOCK + threadIdx.x;
+    if (g >= n_rows * slack) return;
+    const i64 r = g / slack, k = g - r * slack;
+    out[r * out_stride + k] = prg_word(seed, row_indices ? row_indices[r] : (u64)(u32)(row_offset + (u32)r), k);
+}
+
+// Message and pad of a padded row in one launch: out[r][k] = messages[r][k] for k < ell, and the value of k_row_prg at
+// k - ell behind it.  The hashing is bound by VALU issue, so the copy rides along (333 rows of 8192 + 8192: 9 us as a launch
+// of its own).
+__global__ __launch_bounds__(BLOCK) void k_pad_rows(const u32 *__restrict__ seed, u32 row_offset, const u64 *__restrict__ messages, i64 in_stride,
+                                                    i64 ell, i64 n_rows, i64 width, u64 *__restrict__ out) {
+    const i64 g = (i64)blockIdx.x * BLOCK + threadIdx.x;
+    if (g >= n_rows * width) return;
+    const i64 r = g / width, k = g - r * width;
+    out[g] = k < ell ? messages[r * in_stride + k] : prg_word(seed, (u64)(u32)(row_offset + (u32)r), k - ell);
 }
 
 // The test-combiner challenge of the protocol (prover/protocol.py:127-135, device twin
@@ -316,6 +458,28 @@ inline i64 chunks_of(i64 m) { return m <= 0 ? 1 : (m + ROWS_PER_CHUNK - 1) / ROW
 
 extern "C" {
 
+}  // extern "C"
+
+namespace {
+// Up to this many chunk-columns -- a wavefront per SIMD with four lanes each -- the chain of a chunk's sixteen compressions is
+// what the launch takes, and four lanes halve it.
+constexpr i64 QUAD_MAX = 1 << 14;
+
+int launch_chunks(const u64 *rows, i64 slab_rows, i64 n, i64 row_stride, i64 chunk0, i64 slab_chunks, bool single_root, u32 *cvs, hipStream_t s) {
+    if (n * slab_chunks <= QUAD_MAX) {
+        dim3 grid((unsigned)((n + QUAD_COLS - 1) / QUAD_COLS), (unsigned)slab_chunks);
+        hipLaunchKernelGGL(k_chunk_cvs_quad, grid, dim3(BLOCK), 0, s, rows, slab_rows, n, row_stride, chunk0, single_root ? 1 : 0, cvs);
+    } else {
+        dim3 grid((unsigned)((n + BLOCK - 1) / BLOCK), (unsigned)slab_chunks);
+        hipLaunchKernelGGL(k_chunk_cvs, grid, dim3(BLOCK), 0, s, rows, slab_rows, n, row_stride, chunk0, single_root ? 1 : 0, cvs);
+    }
+    VI_LAUNCH_CHECK("k_chunk_cvs");
+    return VI_OK;
+}
+}  // namespace
+
+extern "C" {
+
 size_t vi_hash_columns_workspace_bytes(int64_t m, int64_t n) {
     if (m < 0 || n <= 0) return 0;
     // chunk chaining values + one ping-pong level
@@ -336,11 +500,7 @@ int vi_hash_columns_update(const uint64_t *rows, int64_t slab_rows, int64_t n, i
     if (!ws || ws_bytes < (size_t)(n_chunks_total + (n_chunks_total + 1) / 2) * (size_t)n * 32)
         return vi::fail(VI_ENOMEM, "vi_hash_columns_update: workspace too small");
     if (slab_chunks > 65535) return vi::fail(VI_EINVAL, "vi_hash_columns_update: at most 65535 chunks (8,388,480 rows) per call");
-    dim3 grid((unsigned)((n + BLOCK - 1) / BLOCK), (unsigned)slab_chunks);
-    hipLaunchKernelGGL(k_chunk_cvs, grid, dim3(BLOCK), 0, (hipStream_t)stream, rows, (i64)slab_rows, (i64)n, (i64)row_stride,
-                       (i64)chunk0, n_chunks_total == 1 ? 1 : 0, (u32 *)ws);
-    VI_LAUNCH_CHECK("k_chunk_cvs");
-    return VI_OK;
+    return launch_chunks(rows, slab_rows, n, row_stride, chunk0, slab_chunks, n_chunks_total == 1, (u32 *)ws, (hipStream_t)stream);
 }
 
 int vi_hash_columns_finalize(int64_t n, int64_t n_chunks_total, void *ws, size_t ws_bytes, uint8_t *digests, void *stream) {
@@ -382,6 +542,8 @@ int vi_hash_columns(const uint64_t *mat, int64_t m, int64_t n, int64_t row_strid
                     size_t ws_bytes, void *stream) {
     if (m < 0) return vi::fail(VI_EINVAL, "vi_hash_columns: m = %lld", (long long)m);
     const i64 total = chunks_of(m);
+    if (total == 1 && n > 0 && row_stride >= n && (m == 0 || mat) && digests && ((uintptr_t)digests & 3) == 0)      // the one chunk is the root
+        return launch_chunks(mat, m, n, row_stride, 0, 1, true, (u32 *)digests, (hipStream_t)stream);
     for (i64 c0 = 0; c0 < total; c0 += 65535) {
         const i64 cc = total - c0 < 65535 ? total - c0 : 65535;
         const i64 r0 = c0 * ROWS_PER_CHUNK;
@@ -443,6 +605,21 @@ int vi_row_prg(const uint8_t *seed, const uint64_t *row_indices, int64_t row_off
     hipLaunchKernelGGL(k_row_prg, dim3((unsigned)blocks), dim3(BLOCK), 0, (hipStream_t)stream, (const u32 *)seed, row_indices,
                        (u32)row_offset, (i64)n_rows, (i64)slack, out, (i64)out_stride);
     VI_LAUNCH_CHECK("k_row_prg");
+    return VI_OK;
+}
+
+int vi_pad_rows(const uint8_t *seed, int64_t row_offset, const uint64_t *messages, int64_t n_rows, int64_t ell, int64_t in_stride,
+                int64_t width, uint64_t *out, void *stream) {
+    if (n_rows < 0 || ell < 0 || width < ell || in_stride < ell)
+        return vi::fail(VI_EINVAL, "vi_pad_rows: bad shape n_rows=%lld ell=%lld in_stride=%lld width=%lld", (long long)n_rows, (long long)ell, (long long)in_stride, (long long)width);
+    if (n_rows == 0 || width == 0) return VI_OK;
+    if (!out || (ell > 0 && !messages) || (width > ell && !seed)) return vi::fail(VI_EINVAL, "vi_pad_rows: null pointer");
+    if ((uintptr_t)seed & 3) return vi::fail(VI_EINVAL, "vi_pad_rows: seed must be 4-byte aligned");
+    const i64 blocks = (n_rows * width + BLOCK - 1) / BLOCK;
+    if (blocks > 0x7FFFFFFF) return vi::fail(VI_EINVAL, "vi_pad_rows: %lld words exceed one launch", (long long)(n_rows * width));
+    hipLaunchKernelGGL(k_pad_rows, dim3((unsigned)blocks), dim3(BLOCK), 0, (hipStream_t)stream, (const u32 *)seed, (u32)row_offset, messages,
+                       (i64)in_stride, (i64)ell, (i64)n_rows, (i64)width, out);
+    VI_LAUNCH_CHECK("k_pad_rows");
     return VI_OK;
 }
 

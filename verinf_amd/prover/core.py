@@ -17,8 +17,8 @@ from typing import Optional, Tuple
 import torch
 
 from .cuda_primitives import (  # noqa: F401  (re-exported like the reference)
-    MerkleColumnAccumulator, coset_extend, coset_lde_with_coeffs, hash_columns_streamed, merkle_build_blake3, row_prg,
-    row_prg_indexed)
+    MerkleColumnAccumulator, coset_extend, coset_lde_with_coeffs, hash_columns_streamed, merkle_build_blake3, pad_rows,
+    row_prg, row_prg_indexed)
 from .protocol import GLOBAL_G, P
 
 
@@ -90,9 +90,14 @@ def encode_messages(messages: torch.Tensor, cfg: LigeroConfig, *, master_seed: t
                 f"Proof is sound but not zero-knowledge under this config.",
                 UserWarning, stacklevel=2)
         padded = torch.empty((m, cfg.K_DEG), dtype=torch.uint64, device=messages.device)
-        padded.view(torch.int64)[:, :cfg.ELL] = messages.view(torch.int64)
-        row_prg(master_seed, row_offset, m, slack, out=padded[:, cfg.ELL:])
-        # `padded` is ours: the row polynomials take its place
+        if messages.is_cuda and messages.dtype in (torch.uint64, torch.int64) and (cfg.ELL == 1 or messages.stride(1) == 1) \
+                and (m == 1 or messages.stride(0) >= cfg.ELL):
+            pad_rows(master_seed, row_offset, messages, padded)
+        else:
+            padded.view(torch.int64)[:, :cfg.ELL] = messages.view(torch.int64)
+            row_prg(master_seed, row_offset, m, slack, out=padded[:, cfg.ELL:])
+        # `padded` is ours: the row polynomials take its place, unless the batch is so small that the cosets of a row run in
+        # workgroups of their own, which must not overwrite what the others still read
         return coset_lde_with_coeffs(padded, cfg.K_DEG, cfg.N_LIG, cfg.coset_shift, need_codewords=need_codewords,
-                                     in_place=True)
+                                     in_place=m * cfg.N_LIG > (1 << 21))
     return coset_lde_with_coeffs(messages, cfg.K_DEG, cfg.N_LIG, cfg.coset_shift, need_codewords=need_codewords)

@@ -19,6 +19,8 @@ Additions over the reference surface:
   coset_extend(coeffs, k_deg, n_lig, shift)  coefficients -> coset evaluations
   gl_mul_bcast(a, b_row)                     a * (b_row broadcast over rows) without materialising it
   row_prg(..., out=)                         the pad written straight into a column slice
+  pad_rows(seed, row_offset, messages, out)  messages and their pad into padded rows, in one launch
+  merkle_levels(leaves)                      the levels of merkle_build_blake3 without a copy of the root
 """
 import torch
 
@@ -555,6 +557,18 @@ def row_prg(master_seed, row_offset, n_rows, slack_per_row, out=None):
         if n_rows and slack and (out.stride(1) != 1 or (n_rows > 1 and out.stride(0) < slack)):
             raise RuntimeError("out must have unit column stride and non-overlapping rows")
     return _row_prg(master_seed, None, row_offset, n_rows, slack, out)
+
+
+def pad_rows(master_seed, row_offset, messages, padded):
+    """padded[r] = messages[r] followed by row_prg(master_seed, row_offset + r), in one launch: `padded` is a contiguous
+    (rows, K) tensor, `messages` (rows, ELL <= K) with unit column stride."""
+    _check_seed(master_seed)
+    _check_u64(padded, "padded")
+    m, ell = int(messages.shape[0]), int(messages.shape[1])
+    stride = int(messages.stride(0)) if m > 1 else max(ell, 1)
+    with _lib.on_device(padded.device):
+        _lib.check(_lib.lib().vi_pad_rows(master_seed.data_ptr(), int(row_offset) & 0xFFFFFFFF, messages.data_ptr(), m, ell, stride,
+                                          int(padded.shape[1]), padded.data_ptr(), _lib.stream_ptr()))
 
 
 def row_prg_indexed(master_seed, row_indices, slack_per_row):
