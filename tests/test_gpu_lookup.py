@@ -38,10 +38,14 @@ def test_range_tables(n_x, n_table):
     _check(x, np.arange(n_table, dtype=np.uint64))
 
 
-def test_range_table_of_more_slices_than_groups():
+@pytest.mark.parametrize("n", [1 << 21, (1 << 21) + 1, (1 << 23) + 5])                 # 64 slices of 32768 entries, and more
+@pytest.mark.parametrize("n_x", [50000, 200001])
+def test_tables_of_many_slices(n_x, n):
     rng = np.random.default_rng(3)
-    n = (1 << 23) + 5
-    _check(rng.integers(0, n, 50000).astype(np.uint64), np.arange(n, dtype=np.uint64))
+    x = rng.integers(0, n + 1000, n_x).astype(np.uint64)
+    x[:100] = n - 1
+    _check(x, np.arange(n, dtype=np.uint64))
+    _check(x * np.uint64(3), np.arange(n, dtype=np.uint64)[::-1] * np.uint64(3))
 
 
 @pytest.mark.parametrize("n_x,n_table", [(1, 1), (1000, 3), (50001, 300), (200000, 4097), (100000, 40000)])

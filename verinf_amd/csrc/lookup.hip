@@ -146,7 +146,18 @@ __global__ __launch_bounds__(BLOCK) void k_add_rows(const u32 *__restrict__ rows
     }
 }
 
-// one global atomic per look-up, the table searched from the front: no workspace
+// one global atomic per look-up, through the hash table where there is one
+template <bool RANGE>
+__global__ __launch_bounds__(BLOCK) void k_count_global(const u64 *__restrict__ x, i64 n_x, const Slot *__restrict__ slots, int bits, i64 n_table,
+                                                        unsigned long long *__restrict__ mult) {
+    const i64 stride = (i64)gridDim.x * BLOCK;
+    for (i64 i = (i64)blockIdx.x * BLOCK + threadIdx.x; i < n_x; i += stride) {
+        const u64 at = index_of<RANGE>(x[i], slots, bits);
+        if (at < (u64)n_table) atomicAdd(&mult[at], 1ULL);
+    }
+}
+
+// the same without a hash table, the table searched from the front: no workspace
 __global__ __launch_bounds__(BLOCK) void k_lookup_mult(const u64 *__restrict__ x, i64 n_x, const u64 *__restrict__ table, i64 n_table,
                                                        i64 t_len_range, unsigned long long *__restrict__ mult) {
     const i64 stride = (i64)gridDim.x * BLOCK;
@@ -179,21 +190,22 @@ struct Plan {
 
 Plan make_plan(i64 n_x, i64 n_table, bool range) {
     Plan L = {};
-    // few look-ups, spread over many entries: 30000 in a 2^16 table take 3.6 us and 2.5 us for clearing the counts, 11 us
-    // through the histogram
-    L.direct = range && n_table >= 8192 && n_x <= 131072;
-    if (L.direct) return L;
+    L.bits = 1;
+    while (((i64)1 << L.bits) < 2 * n_table) ++L.bits;
+    L.slot_bytes = range ? 0 : sizeof(Slot) << L.bits;
     L.slices = (n_table + SLICE - 1) / SLICE;
+    // Few look-ups, spread over many entries: 30000 in a 2^16 table take 3.6 us and 2.5 us for clearing the counts, 11 us
+    // through the histogram.  And a table of many slices: all of them read all look-ups, 10 us a slice for 2^24 of them
+    // against 711 us of atomics in all.
+    L.direct = (range && n_table >= 8192 && n_x <= 131072) || L.slices > 64;
+    if (L.direct) return L;
     // a workgroup per CU, but no more rows than look-ups are worth: clearing and storing a slice's counters takes as long
     // as some eight thousand look-ups
     L.groups = (n_x + 8191) / 8192;
     if (L.groups * L.slices > MAX_GROUPS) L.groups = MAX_GROUPS / L.slices;
-    if (L.groups < 1) L.groups = 1;
+    if (L.groups < (n_x >> 31) + 1) L.groups = (n_x >> 31) + 1;        // a group's counters have 32 bits
     L.copies = 1;
     while (L.copies < MAX_COPIES && n_table * L.copies * 2 <= SLICE) L.copies *= 2;
-    L.bits = 1;
-    while (((i64)1 << L.bits) < 2 * n_table) ++L.bits;
-    L.slot_bytes = range ? 0 : sizeof(Slot) << L.bits;
     L.row_bytes = L.groups > 1 ? (size_t)L.groups * n_table * sizeof(u32) : 0;
     return L;
 }
@@ -229,13 +241,6 @@ int vi_lookup_histogram(const uint64_t *x, int64_t n_x, const uint64_t *table, i
     const size_t need = L.slot_bytes + L.row_bytes;
     if (need && (!ws || ws_bytes < need)) return vi::fail(VI_ENOMEM, "vi_lookup_histogram: workspace below %zu bytes", need);
     hipStream_t s = (hipStream_t)stream;
-    if (L.direct) {
-        if (!accumulate) {
-            hipLaunchKernelGGL(k_clear_counts, dim3(capped_grid(n_table)), dim3(BLOCK), 0, s, mult, (i64)n_table);
-            VI_LAUNCH_CHECK("k_clear_counts");
-        }
-        return vi_lookup_multiplicities(x, n_x, table, n_table, table_is_range, mult, stream);
-    }
     Slot *slots = (Slot *)ws;
     u32 *rows = L.row_bytes ? (u32 *)((char *)ws + L.slot_bytes) : nullptr;
     if (!table_is_range) {
@@ -243,6 +248,19 @@ int vi_lookup_histogram(const uint64_t *x, int64_t n_x, const uint64_t *table, i
         VI_LAUNCH_CHECK("k_clear_slots");
         hipLaunchKernelGGL(k_insert, dim3(capped_grid(n_table)), dim3(BLOCK), 0, s, table, (i64)n_table, slots, L.bits);
         VI_LAUNCH_CHECK("k_insert");
+    }
+    if (L.direct) {
+        if (!accumulate) {
+            hipLaunchKernelGGL(k_clear_counts, dim3(capped_grid(n_table)), dim3(BLOCK), 0, s, mult, (i64)n_table);
+            VI_LAUNCH_CHECK("k_clear_counts");
+        }
+        if (n_x == 0) return VI_OK;
+        if (table_is_range)
+            hipLaunchKernelGGL(k_count_global<true>, dim3(capped_grid(n_x)), dim3(BLOCK), 0, s, x, (i64)n_x, (const Slot *)slots, L.bits, (i64)n_table, (unsigned long long *)mult);
+        else
+            hipLaunchKernelGGL(k_count_global<false>, dim3(capped_grid(n_x)), dim3(BLOCK), 0, s, x, (i64)n_x, (const Slot *)slots, L.bits, (i64)n_table, (unsigned long long *)mult);
+        VI_LAUNCH_CHECK("k_count_global");
+        return VI_OK;
     }
     const i64 per = (n_x + L.groups - 1) / L.groups;
     const i64 in_slice = n_table < SLICE ? n_table : SLICE;

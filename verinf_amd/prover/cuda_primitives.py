@@ -565,6 +565,10 @@ def pad_rows(master_seed, row_offset, messages, padded):
     _check_seed(master_seed)
     _check_u64(padded, "padded")
     m, ell = int(messages.shape[0]), int(messages.shape[1])
+    if padded.dim() != 2 or int(padded.shape[0]) != m or int(padded.shape[1]) < ell:
+        raise RuntimeError("pad_rows: padded does not hold the rows of messages")
+    if not messages.is_cuda or messages.dtype not in (torch.uint64, torch.int64) or (ell > 1 and messages.stride(1) != 1):
+        raise RuntimeError("pad_rows: messages must be cuda uint64 rows with unit column stride")
     stride = int(messages.stride(0)) if m > 1 else max(ell, 1)
     with _lib.on_device(padded.device):
         _lib.check(_lib.lib().vi_pad_rows(master_seed.data_ptr(), int(row_offset) & 0xFFFFFFFF, messages.data_ptr(), m, ell, stride,
@@ -734,6 +738,11 @@ def lookup_multiplicities_into(x, table, mult, label=""):
 def _histogram(x, table, mult, accumulate):
     L = _lib.lib()
     n_x, n_t, is_range = int(x.numel()), int(table.numel()), 1 if _is_range_table(table) else 0
+    if n_t > 1 << 30:                # beyond the 32-bit indices of the hash table
+        if not accumulate:
+            mult.view(torch.int64).zero_()
+        _lib.check(L.vi_lookup_multiplicities(x.data_ptr(), n_x, table.data_ptr(), n_t, is_range, mult.data_ptr(), _lib.stream_ptr()))
+        return
     need = L.vi_lookup_histogram_workspace_bytes(n_x, n_t, is_range)
     ws = _lib.workspace(need, x.device, "lookup").data_ptr() if need else None
     _lib.check(L.vi_lookup_histogram(x.data_ptr(), n_x, table.data_ptr(), n_t, is_range, accumulate, mult.data_ptr(), ws, need,
