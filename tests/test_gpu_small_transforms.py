@@ -1,6 +1,10 @@
 """GPU parity of the single-launch transforms and extensions of short rows: every row length and direction, ragged batches,
 narrow and strided sources, coefficients beside, in place and alone, one to many cosets -- against the oracle, and against
 the multi-pass kernels by running the same rows inside a batch too large for the single launch."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -80,3 +84,34 @@ def test_larger_batches(cp, logk, log_rho, m):
     assert np.array_equal(got[rows], O.coset_lde_rows(np.ascontiguousarray(a[rows]), K, N, 7))
     coeffs, code = cp.coset_lde_with_coeffs(to_dev(a), K, N, in_place=True)
     assert np.array_equal(to_np(code), got)
+
+
+_CAPTURE = """
+import torch
+from tests.gpu_util import rand_field, to_dev
+from verinf_amd.prover import cuda_primitives as cp
+for logn, first, then in ((5, 3, 1 << 16), (6, 1 << 15, 3), (8, 3, 1 << 13), (10, 1 << 11, 2), (11, 2, 1 << 10)):
+    n = 1 << logn
+    cp.ntt_forward_batched(to_dev(rand_field((first, n), 1)))
+    src = [to_dev(rand_field((then, n), 2 + i)) for i in range(3)]
+    buf = src[0].clone()
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        cp.ntt_forward_batched(buf)
+    for s in src:
+        buf.copy_(s)
+        g.replay()
+        torch.cuda.synchronize()
+        cp.ntt_forward_batched(s)
+        assert torch.equal(buf.view(torch.int64), s.view(torch.int64)), logn
+print("captured")
+"""
+
+
+def test_a_captured_call_finds_the_tables_of_another_batch_size():
+    """A call of one batch size prepares its row length for all of them: the other kernels capture with nothing left to
+    upload.  In a process of its own, where no other test has prepared anything."""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", _CAPTURE], cwd=root, capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and r.stdout.endswith("captured\n"), r.stderr[-2000:]

@@ -225,6 +225,8 @@ __global__ __launch_bounds__(NTHREADS, VI_MID_MIN_WG) void k_lde_mid(const PassA
     }
 }
 
+#include "ntt_small.hpp"
+
 namespace {
 
 struct DeviceTables {
@@ -296,6 +298,9 @@ int get_tables(int logn, int inv, const Tables **out, bool row = false) {
             if (!rc) { D->T.tw[q] = d; D->owned.push_back(d); }
         }
         if (!rc) rc = get_twl(dev, inv, &D->T.twl);
+        // with the tables of the passes, whichever batch comes first: a call of another size finds all it needs
+        D->T.full = nullptr;
+        if (!rc && logn >= SMALL_MIN_LOG && logn <= SMALL_MAX_LOG) rc = get_twl(dev, inv, &D->T.full, true);
         if (rc) {                                          // give back what was uploaded before the failure
             for (void *p : D->owned) (void)hipFree(p);
             delete D;
@@ -485,12 +490,6 @@ i64 max_lde_chunk(int logK, int logN) {
     return cap;
 }
 
-}  // namespace
-
-#include "ntt_small.hpp"
-
-namespace {
-
 // Where the single launch of ntt_small.hpp is the faster one; sweep over row lengths and batch sizes, us per call, the
 // passes of k_ntt_fast against it.
 //
@@ -522,16 +521,6 @@ bool small_lde_pays(i64 m, int logK, int logN, bool in_place) {
     return m <= (((i64)1 << log_most) >> logN);
 }
 
-// the tables of the small transforms on the current device
-int get_small_tables(const u64 **inv, const u64 **fwd) {
-    int dev = 0;
-    VI_HIP(hipGetDevice(&dev));
-    std::lock_guard<std::mutex> lock(g_mu);
-    int rc = inv ? get_twl(dev, 1, inv, true) : VI_OK;
-    if (!rc && fwd) rc = get_twl(dev, 0, fwd, true);
-    return rc;
-}
-
 }  // namespace
 
 extern "C" {
@@ -550,19 +539,17 @@ int vi_ntt_batched(uint64_t *rows, int64_t m, int64_t n, int inverse, void *ws, 
     if (m == 0) return VI_OK;
     if (!rows) return vi::fail(VI_EINVAL, "vi_ntt_batched: null rows");
     const int logn = vi::ilog2(n);
+    const Tables *T = nullptr;
+    const bool row = row_launch_on() && row_single_ok(logn);
+    int rc = get_tables(logn, inverse ? 1 : 0, &T, row);
+    if (rc) return rc;
     if (small_ntt_pays(m, logn)) {
-        const u64 *tab = nullptr;
-        int rc = inverse ? get_small_tables(&tab, nullptr) : get_small_tables(nullptr, &tab);
-        if (rc) return rc;
         const u64 scale = inverse ? ntt::inverse((u64)n % gl::P) : 1;
-        small_dispatch(logn, [&](auto l) { launch_small_ntt<decltype(l)::value>(rows, m, tab, scale, inverse != 0, (hipStream_t)stream); });
+        small_dispatch(logn, [&](auto l) { launch_small_ntt<decltype(l)::value>(rows, m, T->full, scale, inverse != 0, (hipStream_t)stream); });
         VI_LAUNCH_CHECK("k_small_ntt");
         return VI_OK;
     }
-    const Tables *T = nullptr;
-    if (row_launch_on() && row_single_ok(logn)) {
-        int rc = get_tables(logn, inverse ? 1 : 0, &T, true);
-        if (rc) return rc;
+    if (row) {
         const i64 cap = max_rows_per_launch(logn);
         for (i64 lo = 0; lo < m; lo += cap) {
             PassArgs P0, P1;
@@ -572,8 +559,6 @@ int vi_ntt_batched(uint64_t *rows, int64_t m, int64_t n, int inverse, void *ws, 
         }
         return VI_OK;
     }
-    int rc = get_tables(logn, inverse ? 1 : 0, &T);
-    if (rc) return rc;
     i64 chunk = m;
     if (T->sp.p > 1) {
         i64 fit = (i64)(ws_bytes / ((size_t)n * sizeof(u64)));
@@ -686,11 +671,15 @@ int coset_lde_impl(const char *who, const uint64_t *in, int64_t m, int64_t width
     chunk = (m + ((m + chunk - 1) / chunk) - 1) / ((m + chunk - 1) / chunk);   // same chunk count, even sizes
     const Tables *Ti = nullptr, *Tf = nullptr;
     const u64 *pre = nullptr;
+    int rc = get_tables(logK, 1, &Ti);
+    if (!rc) rc = get_tables(logK, 0, &Tf);
+    if (!rc) rc = get_pre(logK, logN, shift, &pre);
+    if (rc) return rc;
     if (small_lde_pays(m, logK, logN, coeffs == in)) {
         SmallLde S{};
-        int rc = get_small_tables(&S.tab_inv, &S.tab_fwd);
-        if (!rc && out) rc = get_pre(logK, logN, shift, &S.pre);
-        if (rc) return rc;
+        S.tab_inv = Ti->full;
+        S.tab_fwd = Tf->full;
+        S.pre = pre;
         S.in = in;
         S.m = m;
         S.width = width;
@@ -709,10 +698,6 @@ int coset_lde_impl(const char *who, const uint64_t *in, int64_t m, int64_t width
         VI_LAUNCH_CHECK("k_small_lde");
         return VI_OK;
     }
-    int rc = get_tables(logK, 1, &Ti);
-    if (!rc) rc = get_tables(logK, 0, &Tf);
-    if (!rc) rc = get_pre(logK, logN, shift, &pre);
-    if (rc) return rc;
     // the split form of the coset factors: its tables lie behind the N words of pre
     static const bool use_merged = []() { const char *e = getenv("VI_LDE_MERGED"); return !e || e[0] != '0'; }();
     const u64 *merged = (use_merged && coset_mergeable(logK, logN)) ? pre + N : nullptr;

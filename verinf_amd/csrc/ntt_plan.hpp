@@ -171,6 +171,7 @@ struct Tables {
     const u64 *tw[3];
     const u64 *twi[4];
     const u64 *twl;
+    const u64 *full;                           // w_4096^j, all 4096 of them, where ntt_small.hpp has a kernel for the length
     u64 scale;
     int inverse;
 };
