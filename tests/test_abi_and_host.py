@@ -281,3 +281,12 @@ int main(void) {
                            "-Wl,-rpath," + os.path.dirname(lib), "-Wl,-rpath," + hip_lib_dir, "-L" + hip_lib_dir, "-lamdhip64"])
     res = subprocess.run([str(exe)], capture_output=True, text=True)
     assert res.returncode == 0, (res.returncode, res.stdout, res.stderr)
+
+
+def test_field_words_takes_what_a_sequence_of_integers_may_be():
+    from verinf_amd import _lib
+    P = _lib._P
+    for values in ([], [0, 1, P - 1], [P, P + 1, (1 << 64) - 1], [-1, 1 << 70], (3, 4), range(5), bytes(range(16)), bytearray(b"12345678"),
+                   [True, False], [2.0, 3]):
+        assert list(_lib.field_words(values)) == [int(v) % P for v in values]
+    assert list(_lib.field_words(v for v in (1, -1, 2))) == [1, P - 1, 2]

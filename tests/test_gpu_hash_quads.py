@@ -49,3 +49,13 @@ def test_padded_rows(m, ell, width, stride):
     cp.pad_rows(torch.tensor(list(seed), dtype=torch.uint8, device="cuda"), 4_000_000_000, to_dev(wide)[:, :ell], padded)
     want = np.concatenate([wide[:, :ell], O.row_prg(seed, 4_000_000_000, m, width - ell)], axis=1) if width > ell else wide[:, :ell]
     assert np.array_equal(to_np(padded), want)
+
+
+def test_a_message_of_one_chunk_without_workspace_is_refused():
+    from verinf_amd import _lib
+    mat = to_dev(rand_field((8, 64), 1))
+    out = torch.zeros(64 * 32, dtype=torch.uint8, device="cuda")
+    ws = torch.empty(64, dtype=torch.uint8, device="cuda")
+    for ptr, size in ((None, 0), (ws.data_ptr(), 64)):
+        assert _lib.lib().vi_hash_columns(mat.data_ptr(), 8, 64, 64, out.data_ptr(), ptr, size, _lib.stream_ptr()) != 0
+    assert not out.any()

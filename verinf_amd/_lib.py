@@ -238,6 +238,8 @@ _P = (1 << 64) - (1 << 32) + 1
 
 def field_words(values):
     """Python integers as an array('Q') of residues mod p."""
+    if not isinstance(values, (list, tuple)):    # array() takes the bytes of a bytes object for memory, and a generator runs once
+        return array.array("Q", [int(v) % _P for v in values])
     try:
         words = array.array("Q", values)         # 20 ns per entry, ten times less than int(v) % p one by one
     except (OverflowError, TypeError):

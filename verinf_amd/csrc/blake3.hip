@@ -456,10 +456,6 @@ inline i64 chunks_of(i64 m) { return m <= 0 ? 1 : (m + ROWS_PER_CHUNK - 1) / ROW
 
 }  // namespace
 
-extern "C" {
-
-}  // extern "C"
-
 namespace {
 // Up to this many chunk-columns -- a wavefront per SIMD with four lanes each -- the chain of a chunk's sixteen compressions is
 // what the launch takes, and four lanes halve it.
@@ -542,7 +538,9 @@ int vi_hash_columns(const uint64_t *mat, int64_t m, int64_t n, int64_t row_strid
                     size_t ws_bytes, void *stream) {
     if (m < 0) return vi::fail(VI_EINVAL, "vi_hash_columns: m = %lld", (long long)m);
     const i64 total = chunks_of(m);
-    if (total == 1 && n > 0 && row_stride >= n && (m == 0 || mat) && digests && ((uintptr_t)digests & 3) == 0)      // the one chunk is the root
+    // the one chunk is the root; what the general path refuses is left to it
+    if (total == 1 && n > 0 && row_stride >= n && (m == 0 || mat) && digests && ((uintptr_t)digests & 3) == 0 && ws &&
+        ws_bytes >= vi_hash_columns_workspace_bytes(m, n))
         return launch_chunks(mat, m, n, row_stride, 0, 1, true, (u32 *)digests, (hipStream_t)stream);
     for (i64 c0 = 0; c0 < total; c0 += 65535) {
         const i64 cc = total - c0 < 65535 ? total - c0 : 65535;

@@ -220,11 +220,12 @@ def mle_eval_t(tables, point: Sequence[int]):
     if k == 0:
         return []
     L = _lib.lib()
-    sp = _lib.stream_ptr()
-    ws_bytes = L.vi_mle_eval_workspace_bytes(k)
-    ws = _lib.workspace(ws_bytes + 8 * k, tables.device, "mle", sp).data_ptr()
-    _lib.check(L.vi_mle_eval(mat.data_ptr(), k, 1 << n, _point(point), n, ws + ws_bytes, ws, ws_bytes, sp))
-    vals = list(struct.unpack(f"<{k}Q", _lib.read_back_ptr(ws + ws_bytes, 8 * k, sp)))
+    with _lib.on_device(tables.device):
+        sp = _lib.stream_ptr()
+        ws_bytes = L.vi_mle_eval_workspace_bytes(k)
+        ws = _lib.workspace(ws_bytes + 8 * k, tables.device, "mle", sp).data_ptr()
+        _lib.check(L.vi_mle_eval(mat.data_ptr(), k, 1 << n, _point(point), n, ws + ws_bytes, ws, ws_bytes, sp))
+        vals = list(struct.unpack(f"<{k}Q", _lib.read_back_ptr(ws + ws_bytes, 8 * k, sp)))
     return vals[0] if one else vals
 
 
