@@ -109,6 +109,8 @@ int vi_poly_eval(const uint64_t *coeffs, int64_t m, int64_t d, const uint64_t *p
  * Environment: VI_NTT_ROW=0 (read once per process) runs rows of 1024 .. 4096 elements as two
  * passes through the workspace instead; vi_ntt_workspace_bytes then reports what that needs. */
 size_t vi_ntt_workspace_bytes(int64_t m, int64_t n);
+/* What the call can make use of: few rows of 2^12 points are faster in two launches, through a workspace of this size. */
+size_t vi_ntt_best_workspace_bytes(int64_t m, int64_t n);
 int vi_ntt_batched(uint64_t *rows, int64_t m, int64_t n, int inverse, void *ws, size_t ws_bytes,
                    void *stream);
 

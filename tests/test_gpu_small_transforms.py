@@ -86,11 +86,73 @@ def test_larger_batches(cp, logk, log_rho, m):
     assert np.array_equal(to_np(code), got)
 
 
+@pytest.mark.parametrize("logn", range(12, 21))
+def test_transforms_of_longer_rows(cp, logn):
+    """Few rows (two or three launches of four points per thread) against the oracle and against a batch beyond them."""
+    n = 1 << logn
+    m = 1 if logn > 18 else 3
+    a = rand_field((m, n), logn)
+    raw = a.copy()
+    raw[-1, -2:] = [np.uint64((1 << 64) - 1), np.uint64(P + 1)]                        # words that are not canonical
+    a[-1, -2:] = [np.uint64(((1 << 64) - 1) % P), 1]
+    d = to_dev(raw)
+    cp.ntt_forward_batched(d)
+    fwd = to_np(d)
+    assert np.array_equal(fwd, O.ntt_rows(a))
+    big = to_dev(np.concatenate([a] * ((1 << (22 if logn == 17 else 20)) // a.size + 1)))
+    cp.ntt_forward_batched(big)
+    assert np.array_equal(to_np(big)[-m:], fwd)
+    cp.ntt_inverse_batched(d)
+    assert np.array_equal(to_np(d), a)
+    inv = to_dev(a)
+    cp.ntt_inverse_batched(inv)
+    assert np.array_equal(to_np(inv), O.ntt_rows(a, inverse=True))
+
+
+@pytest.mark.parametrize("logk", range(10, 19))
+@pytest.mark.parametrize("log_rho", [0, 1, 2, 3, 5])
+def test_extensions_of_longer_rows(cp, logk, log_rho):
+    K, N = 1 << logk, 1 << (logk + log_rho)
+    if logk in (10, 11) and log_rho < 3 or N > 1 << 21:
+        pytest.skip("another kernel's sizes")
+    m = max(1, min(3, (1 << 20) // N)) if logk > 11 else (1 << 20) // N + 1
+    for w in (K, K // 2 + 3, 1):
+        a = rand_field((m, w), 100 * logk + 10 * log_rho + w)
+        wide = torch.empty((m, w + 5), dtype=torch.int64, device="cuda").view(torch.uint64)
+        wide.view(torch.int64)[:, :w] = to_dev(a).view(torch.int64)
+        src = wide[:, :w]                                                              # strided rows
+        code = cp.coset_lde(src, K, N)
+        rows = sorted({0, m - 1})
+        assert np.array_equal(to_np(code)[rows], O.coset_lde_rows(np.ascontiguousarray(a[rows]), K, N, 7))
+        coeffs, again = cp.coset_lde_with_coeffs(src, K, N)
+        assert torch.equal(again.view(torch.int64), code.view(torch.int64))
+        only, none = cp.coset_lde_with_coeffs(src, K, N, need_codewords=False)
+        assert none is None and torch.equal(only.view(torch.int64), coeffs.view(torch.int64))
+        assert torch.equal(cp.coset_extend(coeffs, K, N).view(torch.int64), code.view(torch.int64))
+        back = coeffs.clone()
+        cp.ntt_forward_batched(back)
+        assert np.array_equal(to_np(back)[:, :w], a)
+        own = torch.zeros((m, K), dtype=torch.int64, device="cuda").view(torch.uint64)
+        own.view(torch.int64)[:, :w] = to_dev(a).view(torch.int64)
+        held, again = cp.coset_lde_with_coeffs(own, K, N, in_place=True)
+        assert held.data_ptr() == own.data_ptr()
+        assert torch.equal(held.view(torch.int64), coeffs.view(torch.int64)) and torch.equal(again.view(torch.int64), code.view(torch.int64))
+
+
+@pytest.mark.parametrize("logk,log_rho,log_most", [(12, 1, 19), (13, 2, 21), (14, 2, 22), (16, 1, 20), (16, 2, 21)])
+def test_extensions_on_both_sides_of_the_switch(cp, logk, log_rho, log_most):
+    K, N = 1 << logk, 1 << (logk + log_rho)
+    m = (1 << log_most) // N
+    a = to_dev(rand_field((m + 1, K), logk))
+    assert torch.equal(cp.coset_lde(a[:m], K, N).view(torch.int64), cp.coset_lde(a, K, N)[:m].view(torch.int64))
+
+
 _CAPTURE = """
 import torch
 from tests.gpu_util import rand_field, to_dev
 from verinf_amd.prover import cuda_primitives as cp
-for logn, first, then in ((5, 3, 1 << 16), (6, 1 << 15, 3), (8, 3, 1 << 13), (10, 1 << 11, 2), (11, 2, 1 << 10)):
+for logn, first, then in ((5, 3, 1 << 16), (6, 1 << 15, 3), (8, 3, 1 << 13), (10, 1 << 11, 2), (11, 2, 1 << 10),
+                          (12, 4, 1 << 9), (13, 1 << 8, 4)):
     n = 1 << logn
     cp.ntt_forward_batched(to_dev(rand_field((first, n), 1)))
     src = [to_dev(rand_field((then, n), 2 + i)) for i in range(3)]

@@ -26,7 +26,7 @@ EXPORTS = [
     "vi_gl_binop", "vi_gl_binop_bcast", "vi_gl_unop", "vi_gl_axpy", "vi_gl_probe",
     "vi_gl_sum_workspace_bytes", "vi_gl_sum",
     "vi_gl_matmul_workspace_bytes", "vi_gl_matmul", "vi_gl_matvec", "vi_poly_eval",
-    "vi_ntt_workspace_bytes", "vi_ntt_batched",
+    "vi_ntt_workspace_bytes", "vi_ntt_best_workspace_bytes", "vi_ntt_batched",
     "vi_coset_lde_workspace_bytes", "vi_coset_lde_min_workspace_bytes", "vi_coset_lde_launches",
     "vi_coset_lde", "vi_coset_lde_coeffs", "vi_coset_extend",
     "vi_kquant_to_field",
@@ -79,6 +79,8 @@ def lib():
     L.vi_poly_eval.argtypes = [vp, i64, i64, vp, i64, vp, vp]
     L.vi_ntt_workspace_bytes.restype = sz
     L.vi_ntt_workspace_bytes.argtypes = [i64, i64]
+    L.vi_ntt_best_workspace_bytes.restype = sz
+    L.vi_ntt_best_workspace_bytes.argtypes = [i64, i64]
     L.vi_ntt_batched.argtypes = [vp, i64, i64, c_int, vp, sz, vp]
     L.vi_coset_lde_workspace_bytes.restype = sz
     L.vi_coset_lde_workspace_bytes.argtypes = [i64, i64, i64]

@@ -300,7 +300,7 @@ int get_tables(int logn, int inv, const Tables **out, bool row = false) {
         if (!rc) rc = get_twl(dev, inv, &D->T.twl);
         // with the tables of the passes, whichever batch comes first: a call of another size finds all it needs
         D->T.full = nullptr;
-        if (!rc && logn >= SMALL_MIN_LOG && logn <= SMALL_MAX_LOG) rc = get_twl(dev, inv, &D->T.full, true);
+        if (!rc && logn >= SMALL_MIN_LOG) rc = get_twl(dev, inv, &D->T.full, true);
         if (rc) {                                          // give back what was uploaded before the failure
             for (void *p : D->owned) (void)hipFree(p);
             delete D;
@@ -496,7 +496,7 @@ i64 max_lde_chunk(int logK, int logN) {
 // Transforms of 8 and 16 points: always (2^26 points 465 against 241; the passes have no register kernel below 32).  32 to
 // 2048 points: up to 2^20 points in the batch (2^16 points 6.5 to 11.0 against 4.3 to 7.1; 2^20 points 7.4 to 11.8 against
 // 6.1 to 11.6; beyond that the sixteen points a thread of the passes holds need fewer instructions).  A row of 4096 fills a
-// CU's issue slots either way (11.2 against 11.0).
+// CU's issue slots either way (11.2 against 11.0; spread over the chip in two launches 8.6, small_ntt_passes_pay).
 bool small_ntt_pays(i64 m, int logn) {
     if (logn < SMALL_MIN_LOG || logn >= SMALL_MAX_LOG) return false;
     return logn <= 4 || (m << logn) <= ((i64)1 << 20);
@@ -516,9 +516,61 @@ bool small_lde_pays(i64 m, int logK, int logN, bool in_place) {
     else {
         // in place one workgroup has to run through the cosets of its rows: eight or more of them are the longer chain
         if (in_place && logK > 4) return false;
-        log_most = logK <= 4 ? 22 : (logK <= 9 ? 19 : 20);
+        log_most = logK <= 4 ? 22 : 19;
     }
     return m <= (((i64)1 << log_most) >> logN);
+}
+
+// Where the passes of ntt_small.hpp are the faster ones for rows of several passes (us per call, the passes of k_ntt_fast, or
+// k_ntt_row for rows of 2^12, against them).  Every digit has a kernel.
+bool small_digits(const Split &sp) {
+    for (int q = 0; q < sp.p; ++q)
+        if (sp.a[q] < 5 || sp.a[q] > 8) return false;
+    return sp.p >= 2;
+}
+
+// Transforms, by the points in the batch, which is where the two meet: 2^12 points 11.6 against 8.6, 2^14 16 to 18 against 9 to
+// 14, rows of 2^17 to 2^20 25 to 30 against 12 to 29.  A last digit of 2^8 has four columns a workgroup (2^18 points in rows
+// of 2^16: 18.5 and 13.2, 2^19: 18.8 both), one of 2^5 suits k_ntt_fast badly (2^22 points in rows of 2^17: 53 and 49).
+bool small_ntt_passes_pay(i64 m, int logn, const Split &sp) {
+    if (logn < 12 || !small_digits(sp)) return false;
+    const int log_most = sp.p == 2 ? (sp.a[1] == 8 ? 18 : 19) : (sp.a[2] == 5 ? 22 : 20);
+    return m <= (((i64)1 << log_most) >> logn);
+}
+
+// Extensions, by log2 of the points written, for K = 2^10 .. 2^18 and 1, 2, 4, 8 or more cosets: where the two meet in a sweep
+// over both (rows of 2^13 to 2^16, few of them: 33 to 58 against 16 to 20 at four cosets, up to 154 against 34 at sixteen, where
+// k_ntt_fast takes the cosets one after the other).  Rows of 2^10 and 2^11 with fewer cosets have the single launch.
+bool small_lde_passes_pay(i64 m, int logK, int logN, const Split &sp) {
+    static constexpr int log_most[9][4] = {{0, 0, 0, 24},    {0, 0, 0, 24},    {19, 19, 22, 23}, {19, 21, 21, 22}, {19, 21, 22, 23},
+                                           {19, 20, 20, 21}, {19, 20, 21, 22}, {23, 23, 23, 23}, {21, 21, 21, 23}};
+    if (logK < 10 || logK > 18 || !small_digits(sp)) return false;
+    const int log_rho = logN - logK;
+    return m <= (((i64)1 << log_most[logK - 10][log_rho < 3 ? log_rho : 3]) >> logN);
+}
+
+// Which launches an extension takes
+enum LdeRoute { LDE_PASSES, LDE_SINGLE, LDE_SMALL_PASSES };
+LdeRoute lde_route(i64 m, int logK, int logN, bool in_place, const Split &sp) {
+    const bool passes = small_lde_passes_pay(m, logK, logN, sp);
+    // a row of 2^12 fills a CU: 22.6 us in one launch, 14.8 in four
+    if (!(passes && logK == 12) && small_lde_pays(m, logK, logN, in_place)) return LDE_SINGLE;
+    return passes ? LDE_SMALL_PASSES : LDE_PASSES;
+}
+
+// full[inverse]: w_4096^j of either direction
+int launch_small_passes(const std::vector<PassArgs> &passes, const u64 *const (&full)[2], hipStream_t s) {
+    for (const PassArgs &P : passes) {
+        const u64 *tab = full[P.inverse ? 1 : 0];
+        switch (P.a) {
+            case 5: launch_small_pass<5>(P, tab, s); break;
+            case 6: launch_small_pass<6>(P, tab, s); break;
+            case 7: launch_small_pass<7>(P, tab, s); break;
+            default: launch_small_pass<8>(P, tab, s); break;
+        }
+        VI_LAUNCH_CHECK("k_small_pass");
+    }
+    return VI_OK;
 }
 
 }  // namespace
@@ -531,6 +583,11 @@ size_t vi_ntt_workspace_bytes(int64_t m, int64_t n) {
     return split_digits(vi::ilog2(n)).p > 1 ? (size_t)m * (size_t)n * sizeof(u64) : 0;
 }
 
+size_t vi_ntt_best_workspace_bytes(int64_t m, int64_t n) {
+    if (m > 0 && n == TILE && small_ntt_passes_pay(m, TILE_LOG, split_digits(TILE_LOG))) return (size_t)m * (size_t)n * sizeof(u64);
+    return vi_ntt_workspace_bytes(m, n);
+}
+
 int vi_ntt_batched(uint64_t *rows, int64_t m, int64_t n, int inverse, void *ws, size_t ws_bytes,
                    void *stream) {
     if (m < 0) return vi::fail(VI_EINVAL, "vi_ntt_batched: m = %lld", (long long)m);
@@ -539,10 +596,15 @@ int vi_ntt_batched(uint64_t *rows, int64_t m, int64_t n, int inverse, void *ws, 
     if (m == 0) return VI_OK;
     if (!rows) return vi::fail(VI_EINVAL, "vi_ntt_batched: null rows");
     const int logn = vi::ilog2(n);
-    const Tables *T = nullptr;
-    const bool row = row_launch_on() && row_single_ok(logn);
+    const Tables *T = nullptr, *T2 = nullptr;
+    bool row = row_launch_on() && row_single_ok(logn);
     int rc = get_tables(logn, inverse ? 1 : 0, &T, row);
+    if (!rc && row && logn == TILE_LOG) rc = get_tables(logn, inverse ? 1 : 0, &T2);
     if (rc) return rc;
+    if (T2 && ws && ws_bytes >= (size_t)m * (size_t)n * sizeof(u64) && small_ntt_passes_pay(m, logn, T2->sp)) {
+        T = T2;
+        row = false;
+    }
     if (small_ntt_pays(m, logn)) {
         const u64 scale = inverse ? ntt::inverse((u64)n % gl::P) : 1;
         small_dispatch(logn, [&](auto l) { launch_small_ntt<decltype(l)::value>(rows, m, T->full, scale, inverse != 0, (hipStream_t)stream); });
@@ -568,11 +630,12 @@ int vi_ntt_batched(uint64_t *rows, int64_t m, int64_t n, int inverse, void *ws, 
         if (fit < chunk) chunk = fit;
     }
     if (chunk > max_rows_per_launch(logn)) chunk = max_rows_per_launch(logn);
+    const bool small = small_ntt_passes_pay(m, logn, T->sp);
     for (i64 lo = 0; lo < m; lo += chunk) {
         i64 cnt = (m - lo < chunk) ? (m - lo) : chunk;
         std::vector<PassArgs> passes;
         build_ntt_passes(*T, rows + lo * n, (u64 *)ws, cnt, passes);
-        rc = launch_passes(passes, (hipStream_t)stream);
+        rc = small ? launch_small_passes(passes, {T->full, T->full}, (hipStream_t)stream) : launch_passes(passes, (hipStream_t)stream);
         if (rc) return rc;
     }
     return VI_OK;
@@ -600,7 +663,8 @@ int64_t vi_coset_lde_launches(int64_t m, int64_t K, int64_t N, size_t ws_bytes) 
     size_t one = vi_coset_lde_min_workspace_bytes(K, N);
     if (!one || m <= 0 || ws_bytes < one) return 0;
     i64 chunk = (i64)(ws_bytes / one);
-    if (small_lde_pays(m, vi::ilog2(K), vi::ilog2(N), false)) return 1;
+    const LdeRoute route = lde_route(m, vi::ilog2(K), vi::ilog2(N), false, split_digits(vi::ilog2(K)));
+    if (route == LDE_SINGLE) return 1;
     if (chunk > m) chunk = m;
     if (chunk > max_lde_chunk(vi::ilog2(K), vi::ilog2(N))) chunk = max_lde_chunk(vi::ilog2(K), vi::ilog2(N));
     const i64 n_chunks = (m + chunk - 1) / chunk;         // balancing keeps the chunk count
@@ -614,7 +678,8 @@ int64_t vi_coset_lde_launches(int64_t m, int64_t K, int64_t N, size_t ws_bytes) 
     Ti.scale = Tf.scale = 1;
     u64 *dummy = (u64 *)(uintptr_t)4096;
     std::vector<PassArgs> passes;
-    build_lde_passes(Ti, Tf, dummy, logN, dummy, K, K, dummy, N, dummy, chunk, passes);
+    build_lde_passes(Ti, Tf, dummy, logN, dummy, K, K, dummy, N, dummy, chunk, passes, nullptr, 0, false,
+                     route != LDE_SMALL_PASSES);
     i64 per_chunk = 0;
     for (size_t q = 0; q < passes.size(); ++q) {
         if (passes[q].fuse_next && q + 1 < passes.size() && passes_fusable(passes[q], passes[q + 1])) ++q;
@@ -675,7 +740,8 @@ int coset_lde_impl(const char *who, const uint64_t *in, int64_t m, int64_t width
     if (!rc) rc = get_tables(logK, 0, &Tf);
     if (!rc) rc = get_pre(logK, logN, shift, &pre);
     if (rc) return rc;
-    if (small_lde_pays(m, logK, logN, coeffs == in)) {
+    const LdeRoute route = lde_route(m, logK, logN, coeffs == in, Ti->sp);
+    if (route == LDE_SINGLE) {
         SmallLde S{};
         S.tab_inv = Ti->full;
         S.tab_fwd = Tf->full;
@@ -701,13 +767,14 @@ int coset_lde_impl(const char *who, const uint64_t *in, int64_t m, int64_t width
     // the split form of the coset factors: its tables lie behind the N words of pre
     static const bool use_merged = []() { const char *e = getenv("VI_LDE_MERGED"); return !e || e[0] != '0'; }();
     const u64 *merged = (use_merged && coset_mergeable(logK, logN)) ? pre + N : nullptr;
+    const bool small = route == LDE_SMALL_PASSES;
     for (i64 lo = 0; lo < m; lo += chunk) {
         i64 cnt = (m - lo < chunk) ? (m - lo) : chunk;
         std::vector<PassArgs> passes;
         build_lde_passes(*Ti, *Tf, pre, logN, in + lo * in_stride, width, in_stride, out ? out + lo * out_stride : nullptr,
                          out_stride, (u64 *)ws, cnt, passes, coeffs ? coeffs + lo * coeffs_stride : nullptr, coeffs_stride,
-                         in_is_coeffs, true, merged);
-        rc = launch_passes(passes, (hipStream_t)stream);
+                         in_is_coeffs, !small, small ? nullptr : merged);
+        rc = small ? launch_small_passes(passes, {Tf->full, Ti->full}, (hipStream_t)stream) : launch_passes(passes, (hipStream_t)stream);
         if (rc) return rc;
     }
     return VI_OK;

@@ -7,6 +7,10 @@
 // every twiddle of the thread requested together with the data.  An extension keeps its coefficients in registers
 // between the inverse and the forward transform: decimation in frequency leaves a thread the four consecutive slots
 // (bit-reversed coefficients) that decimation in time starts from, so there is no reordering in between.
+//
+// Rows of more points take the passes of ntt_plan.hpp, digit by digit, with the same four points per thread (k_small_pass): a
+// launch takes 4.3 us where one of k_ntt_fast takes 8, and the cosets of an extension run side by side.  One row of 2^16
+// extended to 2^18: 57 -> 21 us; 16 rows of 2^12 transformed: 11.6 -> 8.6 us.
 #pragma once
 
 namespace {
@@ -26,10 +30,10 @@ struct SmallShape {
 __device__ __forceinline__ int small_pad(int s) { return s + (s >> 4); }
 
 // every thread's LDS writes before any later read; rows of up to 256 points live inside one wavefront, whose LDS accesses
-// are in order
-template <int LOGN>
+// are in order, unless their threads are dealt over the workgroup (SPREAD)
+template <int LOGN, bool SPREAD = false>
 __device__ __forceinline__ void small_sync() {
-    if (SmallShape<LOGN>::TR > 64) __syncthreads();
+    if (SPREAD || SmallShape<LOGN>::TR > 64) __syncthreads();
     else {
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -72,7 +76,7 @@ __device__ __forceinline__ int small_slot(int t, int c) {
 }
 
 // Decimation in frequency over a row: x[c] = point t + c N / 4 on entry, slot 4 t + c of the bit-reversed result on return.
-template <int LOGN, bool INV>
+template <int LOGN, bool INV, bool SPREAD = false>
 __device__ __forceinline__ void small_dif(u64 (&x)[4], const SmallTwiddles<LOGN> &W, int t, u64 *row) {
     constexpr int LEVELS = SmallShape<LOGN>::LEVELS, N = SmallShape<LOGN>::N;
     static_for<0, LEVELS>([&](auto l_) {
@@ -108,7 +112,7 @@ __device__ __forceinline__ void small_dif(u64 (&x)[4], const SmallTwiddles<LOGN>
             constexpr int LW = (LOGN & 1) && l == 0 ? N : L, LR = small_span<LOGN>(l + 1);
 #pragma unroll
             for (int c = 0; c < 4; ++c) row[small_pad(small_slot<LW>(t, c))] = x[c];
-            small_sync<LOGN>();
+            small_sync<LOGN, SPREAD>();
 #pragma unroll
             for (int c = 0; c < 4; ++c) x[c] = row[small_pad(small_slot<LR>(t, c))];
         }
@@ -250,6 +254,90 @@ __global__ __launch_bounds__(SmallShape<LOGN>::WG) void k_small_lde(const SmallL
 #pragma unroll
             for (int c = 0; c < 4; ++c) o[(i64)(t + c * S::TR) << A.log_rho] = x[c];
         }
+    }
+}
+
+// One pass (digit of 2^A points, PassArgs of ntt_pass.hpp) of a transform whose rows are too long for the single launch, in
+// batches that leave the chip idle: the same four points per thread, 1024 points and so many columns per workgroup.  A
+// non-final pass deals the threads of a sub-transform over the workgroup, so that neighbouring lanes read neighbouring
+// columns; a final pass reads its contiguous digits row by row.  Both store along the columns, through LDS.  The cosets of a
+// first forward pass are workgroups of their own.
+template <int A>
+struct SmallPassShape {
+    static constexpr int N = 1 << A, TR = N / 4, COLS = 256 / TR, PITCH = N + N / 16 + 1;
+};
+
+template <int A, bool INV, bool FINAL>
+__global__ __launch_bounds__(256) void k_small_pass(const PassArgs P, const u64 *__restrict__ full) {
+    using S = SmallPassShape<A>;
+    __shared__ u64 lds[S::COLS * S::PITCH];
+    const int tid = threadIdx.x;
+    const int t = FINAL ? tid & (S::TR - 1) : tid / S::COLS, c = FINAL ? tid / S::TR : tid & (S::COLS - 1);
+    const i64 g0 = (i64)blockIdx.x * S::COLS, coset = blockIdx.y;
+    const int lc = P.B + (FINAL ? P.log_rho : P.logR);                 // columns per row, log2
+    u64 *mine = lds + c * S::PITCH;
+
+    // gather: element l of the column at src[base + idx0 + l * step]
+    const i64 g = g0 + c, row = g >> lc, col = g & (((i64)1 << lc) - 1);
+    i64 base = row * P.src_row_stride, idx0, step;
+    if (FINAL) {
+        base += (col & (((i64)1 << P.log_rho) - 1)) * P.src_coset_stride;
+        idx0 = storage_prefix(P, col >> P.log_rho) << A;
+        step = 1;
+    } else {
+        idx0 = ((col >> P.logR) << (A + P.logR)) + (col & (((i64)1 << P.logR) - 1));
+        step = (i64)1 << P.logR;
+    }
+    u64 x[4], f[4], w[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const i64 idx = idx0 + (t + i * S::TR) * step;
+        x[i] = row < P.n_rows && idx < P.src_width ? P.src[base + idx] : 0;
+        if (!FINAL) f[i] = P.pre ? P.pre[(coset << P.logn) + idx] : 1;
+    }
+    // scatter: column oc of the workgroup, outputs k0 + i * 256 / COLS; the inter-pass twiddles are requested here
+    const int oc = tid & (S::COLS - 1), k0 = tid / S::COLS;
+    const i64 og = g0 + oc, orow = og >> lc, ocol = og & (((i64)1 << lc) - 1);
+    const i64 r = ocol & (((i64)1 << P.logR) - 1);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w[i] = FINAL ? P.scale : P.tw[((i64)(k0 + i * S::TR) << P.logR) + r];
+    SmallTwiddles<A> W;
+    W.load(full, t);
+
+    if (P.canon_src) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[i] = gl::canon(x[i]);
+    }
+    if (!FINAL && P.pre) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[i] = gl::mul(x[i], f[i]);
+    }
+    small_dif<A, INV, !FINAL>(x, W, t, mine);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) mine[small_pad(4 * t + i)] = x[i];      // the slots this thread read last
+    __syncthreads();
+    if (orow >= P.n_rows) return;
+    u64 *o = P.dst + orow * P.dst_row_stride;
+    if (!FINAL) o += coset * P.dst_coset_stride + ((ocol >> P.logR) << (A + P.logR)) + r;
+    else o += ocol;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int k = k0 + i * S::TR;
+        u64 v = lds[oc * S::PITCH + small_pad(small_brev(k, A))];
+        if (!FINAL || P.scale != 1) v = gl::mul(v, w[i]);
+        o[(i64)k << (FINAL ? lc : P.logR)] = v;
+    }
+}
+
+template <int A>
+void launch_small_pass(const PassArgs &P, const u64 *full, hipStream_t s) {
+    const i64 cols = P.n_rows << (P.is_final ? P.B + P.log_rho : P.B + P.logR);
+    const dim3 grid((unsigned)((cols + SmallPassShape<A>::COLS - 1) / SmallPassShape<A>::COLS), !P.is_final && P.loop_cosets ? 1u << P.log_rho : 1u);
+    switch ((P.inverse ? 2 : 0) + (P.is_final ? 1 : 0)) {
+        case 0: hipLaunchKernelGGL((k_small_pass<A, false, false>), grid, dim3(256), 0, s, P, full); break;
+        case 1: hipLaunchKernelGGL((k_small_pass<A, false, true>), grid, dim3(256), 0, s, P, full); break;
+        case 2: hipLaunchKernelGGL((k_small_pass<A, true, false>), grid, dim3(256), 0, s, P, full); break;
+        default: hipLaunchKernelGGL((k_small_pass<A, true, true>), grid, dim3(256), 0, s, P, full); break;
     }
 }
 

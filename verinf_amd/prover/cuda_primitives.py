@@ -140,7 +140,7 @@ def _ntt(rows, m, n, inverse):
     with _lib.on_device(rows.device):
         # the library transforms the rows in chunks that fit the workspace it is given: one row is the minimum,
         # 1 GiB is enough to fill the GPU, and a large batch does not double its footprint for the process's life
-        need = min(L.vi_ntt_workspace_bytes(m, n), max(_NTT_WS_CAP, n * 8))
+        need = min(L.vi_ntt_best_workspace_bytes(m, n), max(_NTT_WS_CAP, n * 8))
         ws, ws_bytes = None, 0
         if need:
             buf = _lib.workspace(need, rows.device, "ntt")
