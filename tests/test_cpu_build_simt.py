@@ -1,0 +1,23 @@
+"""Whole kernels on the CPU: translation units of the library compiled with g++ against cpu_build/simt (workgroups as fibers) and
+run through their own entry points under AddressSanitizer and UBSan, results against the oracle.  An index outside a buffer, a
+barrier that not every thread reaches or a wrong launch shape fails here and not on the GPU."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+DIR = os.path.join(HERE, "cpu_build")
+
+
+@pytest.mark.parametrize("what", ["lookup"])
+def test_kernels_on_the_cpu(what):
+    so = os.path.join(DIR, f"simt_{what}.so")
+    subprocess.check_call(["g++", "-O1", "-g", "-std=c++17", "-fPIC", "-shared", "-fno-extern-tls-init", "-fsanitize=address,undefined",
+                           "-fno-sanitize-recover=undefined", "-I", os.path.join(DIR, "simt"), "-o", so, os.path.join(DIR, f"simt_{what}.cpp")])
+    asan = subprocess.check_output(["g++", "-print-file-name=libasan.so"], text=True).strip()
+    env = dict(os.environ, LD_PRELOAD=asan, ASAN_OPTIONS="detect_leaks=0,verify_asan_link_order=0", OPENBLAS_NUM_THREADS="1")
+    res = subprocess.run([sys.executable, os.path.join(DIR, "simt_checks.py"), what, so], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True,
+                         env=env, timeout=600)
+    assert res.returncode == 0 and res.stdout.strip().endswith("OK"), res.stdout[-4000:]

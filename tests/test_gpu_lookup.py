@@ -19,7 +19,6 @@ def _counts(x, table):
 
 def _check(x, table):
     from verinf_amd.prover import cuda_primitives as cp
-    cp._range_table_cache.clear()                              # tables of this test come and go at the same addresses
     dx, dt = to_dev(x), to_dev(table)
     want = _counts(x, table)
     assert np.array_equal(to_np(cp.lookup_multiplicities(dx, dt)), want)
@@ -57,3 +56,81 @@ def test_other_tables(n_x, n_table):
     x = table[rng.integers(0, n_table, n_x)]
     x[::7] = rand_field((len(x[::7]),), 9)
     _check(x, table)
+
+
+@pytest.mark.parametrize("n_table", [512, 4096, 4097, 65536, 1 << 20])
+def test_a_table_changed_in_place_is_looked_at_again(n_table):
+    """The same storage holds a range, then one entry that is not its index (at either end and inside), then a range again."""
+    from verinf_amd.prover import cuda_primitives as cp
+    dt = to_dev(np.arange(n_table, dtype=np.uint64))
+    rng = np.random.default_rng(n_table)
+    x = np.concatenate([rng.integers(0, n_table, 200000).astype(np.uint64), [n_table + 5] * 9]).astype(np.uint64)
+    x[:50] = 0
+    x[50:90] = n_table - 1
+    x[90:120] = n_table // 2
+    dx = to_dev(x)
+    for at in (None, 0, n_table - 1, n_table // 2, None):
+        table = np.arange(n_table, dtype=np.uint64)
+        if at is not None:
+            table[at] = n_table + 5
+        dt.copy_(to_dev(table))
+        assert np.array_equal(to_np(cp.lookup_multiplicities(dx, dt)), _counts(x, table)), at
+
+
+@pytest.mark.parametrize("n_x,n_table", [(100, 3000), (300001, 3000), (100000, 8192), (131073, 8192), (5000, 70000), (300001, 70000)])
+def test_a_promised_range_needs_no_table(n_x, n_table):
+    """table_is_range = 1 through the C ABI: no table is read."""
+    from verinf_amd import _lib
+    L = _lib.lib()
+    x = np.random.default_rng(n_x).integers(0, n_table + 100, n_x).astype(np.uint64)
+    dx, want = to_dev(x), _counts(x, np.arange(n_table, dtype=np.uint64))
+    need = L.vi_lookup_histogram_workspace_bytes(n_x, n_table, 1)
+    ws = torch.empty(max(need, 16), dtype=torch.uint8, device="cuda")
+    mult = to_dev(np.full(n_table, 7, dtype=np.uint64))
+    for accumulate, plus in ((1, 7), (0, 0)):
+        _lib.check(L.vi_lookup_histogram(dx.data_ptr(), n_x, None, n_table, 1, accumulate, mult.data_ptr(), ws.data_ptr(), need, _lib.stream_ptr()))
+        assert np.array_equal(to_np(mult), want + np.uint64(plus))
+
+
+def test_captured_calls_of_both_kinds_of_table():
+    """The launches of a call do not depend on what the table holds: a graph captured over a range counts right after its
+    table has become another one."""
+    from verinf_amd.prover import cuda_primitives as cp
+    n_x, n_table = 200000, 5000
+    dx = to_dev(np.random.default_rng(1).integers(0, n_table, n_x).astype(np.uint64))
+    dt = to_dev(np.arange(n_table, dtype=np.uint64))
+    mult = torch.zeros(n_table, dtype=torch.int64, device="cuda").view(torch.uint64)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        cp.lookup_multiplicities_into(dx, dt, mult)
+        mult.view(torch.int64).zero_()
+    side.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=side):
+        cp.lookup_multiplicities_into(dx, dt, mult)
+    tables = [np.arange(n_table, dtype=np.uint64), rand_field((n_table,), 3), np.arange(n_table, dtype=np.uint64)[::-1].copy()]
+    want = np.zeros(n_table, dtype=np.uint64)
+    for i, table in enumerate(tables):
+        dt.copy_(to_dev(table))
+        x = table[np.random.default_rng(i).integers(0, n_table, n_x)]
+        dx.copy_(to_dev(x))
+        g.replay()
+        torch.cuda.synchronize()
+        want += _counts(x, table)
+        assert np.array_equal(to_np(mult), want), i
+
+
+def test_a_table_beyond_the_hash():
+    """More than 2^30 entries: a range is indexed, another table searched from the front."""
+    from verinf_amd.prover import cuda_primitives as cp
+    n_table = (1 << 30) + 7
+    table = torch.arange(n_table, dtype=torch.int64, device="cuda")
+    x = np.array([0, n_table - 1, n_table - 1, n_table, 12345] + [5] * 30, dtype=np.uint64)
+    got = cp.lookup_multiplicities(to_dev(x), table.view(torch.uint64)).view(torch.int64)
+    assert got[[0, 5, 12345, n_table - 1]].tolist() == [1, 30, 1, 2] and int(got.sum()) == 34
+    table[n_table - 1] = 3                                     # entries near the front only: a search walks up to them
+    got = cp.lookup_multiplicities(to_dev(x[4:]), table.view(torch.uint64)).view(torch.int64)
+    assert got[[5, 12345]].tolist() == [30, 1] and int(got.sum()) == 31
+    del got, table
+    torch.cuda.empty_cache()

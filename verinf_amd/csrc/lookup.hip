@@ -1,14 +1,16 @@
 // LogUp multiplicities: how often each table entry was looked up (prover/kernels/gl_extras.cuh:118-150).
 //
-// Counting with one global atomic per look-up runs at 20 G per second whatever the table (1.5 M look-ups in a 2^16 table:
-// 77 us) and slower the more look-ups share an entry.  Here a workgroup counts its share of the look-ups in LDS, for a
-// slice of up to 32768 entries, leaves its counts as one row of a workspace, and a second launch adds up the rows: 13 us
-// for the same call.  A table of up to 1024 entries is kept several times over, one copy per group of lanes, so that
-// look-ups of one entry do not queue up.
+// Counting with one global atomic per look-up runs at about 22 G per second whatever the table (1.5 M look-ups in a 2^16
+// table: 65 us) and slower the more look-ups share an entry.  Here a workgroup counts its share of the look-ups in LDS, for a
+// slice of up to 32768 entries, leaves its counts as one row of a workspace, and a second launch adds up the rows.  Small
+// tables are kept several times over, one copy per group of lanes, so that look-ups of one entry do not queue up.
 //
-// A table that is not literally 0 .. T-1 is first turned into a hash table (linear probing, at most half full) of
-// entry -> first index that holds it; a look-up then costs a probe or two where the search from the front costs half the
-// table.
+// A table that is literally 0 .. T-1 is indexed; any other one is first turned into a hash table (linear probing, at most
+// half full) of entry -> first index that holds it, and a look-up then costs a probe or two where the search from the
+// front costs half the table.  Which of the two a table is, is looked at in every call, on the device: up to 4096 entries
+// by every workgroup for itself (k_count_small: table and hash in LDS), beyond by a launch over the table (k_survey), whose
+// findings the later launches read.  us per call in a queue of them, 1.5 M look-ups: 9.7 in 2^6 entries, 12.0 in 2^12, 23.8
+// in 2^16, 55 in 2^20 (19.0 and 48 for the last two when the caller promises a range); 10^6 look-ups in 3003 values 12.6.
 #include "common.hpp"
 #include "gl_field.hpp"
 
@@ -20,41 +22,72 @@ constexpr int SLICE = 32768;                   // counters of a workgroup: 128 K
 constexpr int MAX_COPIES = 32;
 constexpr i64 MAX_GROUPS = 256;                // rows of the workspace per slice
 constexpr u32 EMPTY = 0xFFFFFFFFu;
-
-struct Slot {                                  // one entry of the hash table
-    u64 key;
-    u32 index, unused;
-};
+constexpr i64 MAX_HASHED = (i64)1 << 30;       // entries of a hash table
+constexpr int SMALL_TABLE = 4096;              // entries of a table that every workgroup takes into its LDS
+constexpr int SMALL_COUNTERS = 16384;          // counters beside it
+constexpr int SURVEYORS = 256;                 // workgroups of k_survey at most
 
 // Fibonacci hashing into 2^bits slots
 __device__ __forceinline__ u32 slot_of(u64 key, int bits) { return (u32)((key * 0x9E3779B97F4A7C15ull) >> (64 - bits)); }
 
-__global__ __launch_bounds__(BLOCK) void k_clear_slots(Slot *slots, i64 n) {
-    const i64 stride = (i64)gridDim.x * BLOCK;
-    for (i64 i = (i64)blockIdx.x * BLOCK + threadIdx.x; i < n; i += stride) slots[i].index = EMPTY;
+// How a look-up finds its entry.
+struct Finder {
+    const u64 *table;
+    i64 n_table;
+    u64 *keys;                                 // the hash table: entry and index of each slot (EMPTY: unused)
+    u32 *index;
+    int bits;                                  // log2 of the slots, 0: no hash table
+    const u32 *odd;                            // what each workgroup of the survey found: 1 when an entry is not its index
+    int n_odd;                                 // 0: the caller promises a range
+};
+
+// Workgroup w looks at its share of the table and notes in odd[w] whether table[j] == j throughout, empties its share of the
+// slots and, when the counts are not added to what is there, zeroes its share of them.  It and the launch of k_insert that
+// finds nothing to do cost a call over a range 3 us at 2^13 entries, 5 at 2^16 and 7 at 2^20 (8 bytes read and 8 to 24 written
+// per entry).
+__global__ __launch_bounds__(COUNT_THREADS) void k_survey(const Finder F, u32 *odd, u64 *clear) {
+    const i64 first = (i64)blockIdx.x * COUNT_THREADS + threadIdx.x, stride = (i64)gridDim.x * COUNT_THREADS;
+    int differs = 0;
+    for (i64 j = first; j < F.n_table; j += stride) {
+        differs |= F.table[j] != (u64)j;
+        if (clear) clear[j] = 0;
+    }
+    const i64 n_slots = F.bits ? (i64)1 << F.bits : 0;
+    for (i64 j = first; j < n_slots; j += stride) F.index[j] = EMPTY;
+    differs = __syncthreads_or(differs);
+    if (threadIdx.x == 0) odd[blockIdx.x] = differs ? 1 : 0;
+}
+
+// the survey's result, the same for every thread of a workgroup (which all call this)
+__device__ __forceinline__ bool is_range(const Finder &F) {
+    return !__syncthreads_or((int)threadIdx.x < F.n_odd && F.odd[threadIdx.x] != 0);
 }
 
 // A slot belongs to the first index that claims it; later indices of the same entry lower it to the smallest.  The entry
 // of a claimed slot is read from the table (every index it ever holds has the same one).  Ends after at most 2^bits
 // probes, and half of the slots stay empty.
-__global__ __launch_bounds__(BLOCK) void k_insert(const u64 *__restrict__ table, i64 n_table, Slot *slots, int bits) {
-    const i64 stride = (i64)gridDim.x * BLOCK;
+__device__ __forceinline__ void insert(const u64 *table, u32 j, u64 key, u64 *keys, u32 *index, int bits) {
     const u32 mask = (1u << bits) - 1;
-    for (i64 j = (i64)blockIdx.x * BLOCK + threadIdx.x; j < n_table; j += stride) {
-        const u64 key = table[j];
-        u32 h = slot_of(key, bits);
-        for (u32 probes = 0; probes <= mask; ++probes, h = (h + 1) & mask) {
-            const u32 was = atomicCAS(&slots[h].index, EMPTY, (u32)j);
-            if (was == EMPTY) {
-                slots[h].key = key;
-                break;
-            }
-            if (table[was] == key) {
-                atomicMin(&slots[h].index, (u32)j);
-                break;
-            }
+    u32 h = slot_of(key, bits);
+    for (u32 probes = 0; probes <= mask; ++probes, h = (h + 1) & mask) {
+        const u32 was = atomicCAS(&index[h], EMPTY, j);
+        if (was == EMPTY) {
+            if (keys) keys[h] = key;
+            return;
+        }
+        if (table[was] == key) {
+            atomicMin(&index[h], j);
+            return;
         }
     }
+}
+
+// nothing to do for a range
+__global__ __launch_bounds__(BLOCK) void k_insert(const Finder F) {
+    if (is_range(F)) return;
+    const i64 stride = (i64)gridDim.x * BLOCK;
+    for (i64 j = (i64)blockIdx.x * BLOCK + threadIdx.x; j < F.n_table; j += stride)
+        insert(F.table, (u32)j, F.table[j], F.keys, F.index, F.bits);
 }
 
 __global__ __launch_bounds__(BLOCK) void k_clear_counts(u64 *mult, i64 n) {
@@ -64,59 +97,115 @@ __global__ __launch_bounds__(BLOCK) void k_clear_counts(u64 *mult, i64 n) {
 
 // the index a value counts for, or at least n_table for none
 template <bool RANGE>
-__device__ __forceinline__ u64 index_of(u64 x, const Slot *__restrict__ slots, int bits) {
+__device__ __forceinline__ u64 index_of(u64 x, const Finder &F) {
     if (RANGE) return x;
-    const u32 mask = (1u << bits) - 1;
-    u32 h = slot_of(x, bits);
+    if (F.bits == 0) {                         // a table beyond the indices of a slot: searched from the front
+        i64 j = 0;
+        while (j < F.n_table && F.table[j] != x) ++j;
+        return (u64)j;
+    }
+    const u32 mask = (1u << F.bits) - 1;
+    u32 h = slot_of(x, F.bits);
     for (u32 probes = 0; probes <= mask; ++probes, h = (h + 1) & mask) {
-        const ulonglong2 s = *reinterpret_cast<const ulonglong2 *>(slots + h);
-        if ((u32)s.y == EMPTY) break;
-        if (s.x == x) return (u32)s.y;
+        const u32 at = F.index[h];
+        const u64 key = F.keys[h];             // beside the index, not behind it (an unused slot holds anything)
+        if (at == EMPTY) break;
+        if (key == x) return at;
     }
     return ~0ull;
 }
 
-// Workgroup (slice, group): counts of the entries slice * SLICE .. of the group's share of x.  `copies` (a power of two)
-// interleaved counters per entry.  rows: the group's row of n_table counts, or null when there is one group: the counts go
-// straight to mult.
-template <bool RANGE>
-__global__ __launch_bounds__(COUNT_THREADS) void k_count(const u64 *__restrict__ x, i64 n_x, i64 per_group, const Slot *__restrict__ slots, int bits,
-                                                         i64 n_table, int copies, u32 *rows, u64 *mult, int accumulate) {
-    extern __shared__ u32 counts[];
-    const int tid = threadIdx.x;
-    const i64 base = (i64)blockIdx.x * SLICE, group = blockIdx.y;
-    const int mine = n_table - base < SLICE ? (int)(n_table - base) : SLICE;
-    const int n_counts = mine * copies;
-    // the launch's LDS is a whole number of 16-byte words
-    for (int i = tid; i < (n_counts + 3) / 4; i += COUNT_THREADS) reinterpret_cast<uint4 *>(counts)[i] = make_uint4(0, 0, 0, 0);
-    __syncthreads();
-    const i64 lo = group * per_group, hi = lo + per_group < n_x ? lo + per_group : n_x;
-    const int copy = tid & (copies - 1);
+// counts of the entries base .. base + mine - 1 among x[lo .. hi - 1], each at(value) an index of the table; `copies` (a power
+// of two) interleaved counters per entry
+template <class F>
+__device__ __forceinline__ void count(const u64 *__restrict__ x, i64 lo, i64 hi, u64 base, int mine, int copies, u32 *counts, F at) {
+    const int copy = threadIdx.x & (copies - 1);
     constexpr int UN = 4;                      // look-ups of a thread in flight
-    for (i64 i0 = lo + tid; i0 < hi; i0 += UN * COUNT_THREADS) {
+    for (i64 i0 = lo + threadIdx.x; i0 < hi; i0 += UN * COUNT_THREADS) {
         u64 v[UN];
 #pragma unroll
         for (int u = 0; u < UN; ++u) v[u] = i0 + u * COUNT_THREADS < hi ? x[i0 + u * COUNT_THREADS] : 0;
 #pragma unroll
         for (int u = 0; u < UN; ++u) {
             if (i0 + u * COUNT_THREADS < hi) {
-                const u64 at = index_of<RANGE>(v[u], slots, bits) - (u64)base;
-                if (at < (u64)mine) atomicAdd(&counts[(int)at * copies + copy], 1u);
+                const u64 j = at(v[u]) - base;
+                if (j < (u64)mine) atomicAdd(&counts[(int)j * copies + copy], 1u);
             }
         }
     }
-    __syncthreads();
-    if (rows && copies == 1 && (mine & 3) == 0 && (n_table & 3) == 0) {        // 16-byte aligned rows
-        uint4 *to = reinterpret_cast<uint4 *>(rows + group * n_table + base);
+}
+
+// a workgroup's counts to its row, or straight to the result where there are no rows
+__device__ __forceinline__ void put_counts(const u32 *counts, int mine, int copies, u32 *row, bool aligned, u64 *mult, int accumulate) {
+    const int tid = threadIdx.x;
+    if (row && copies == 1 && aligned && (mine & 3) == 0) {
+        uint4 *to = reinterpret_cast<uint4 *>(row);
         for (int i = tid; i < mine / 4; i += COUNT_THREADS) to[i] = reinterpret_cast<const uint4 *>(counts)[i];
         return;
     }
     for (int i = tid; i < mine; i += COUNT_THREADS) {
         u32 c = 0;
         for (int k = 0; k < copies; ++k) c += counts[i * copies + ((k + tid) & (copies - 1))];
-        if (rows) rows[group * n_table + base + i] = c;
-        else mult[base + i] = accumulate ? mult[base + i] + c : (u64)c;
+        if (row) row[i] = c;
+        else mult[i] = accumulate ? mult[i] + c : (u64)c;
     }
+}
+
+// Workgroup (slice, group): counts of the entries slice * SLICE .. of the group's share of x.  rows: the group's row of n_table
+// counts, or null when there is one group: the counts go straight to mult.
+__global__ __launch_bounds__(COUNT_THREADS) void k_count(const u64 *__restrict__ x, i64 n_x, i64 per_group, const Finder F, int copies, u32 *rows,
+                                                         u64 *mult, int accumulate) {
+    extern __shared__ uint4 lds_counts[];
+    u32 *counts = reinterpret_cast<u32 *>(lds_counts);
+    const i64 base = (i64)blockIdx.x * SLICE, group = blockIdx.y;
+    const int mine = F.n_table - base < SLICE ? (int)(F.n_table - base) : SLICE;
+    // the launch's LDS is a whole number of 16-byte words
+    for (int i = threadIdx.x; i < (mine * copies + 3) / 4; i += COUNT_THREADS) lds_counts[i] = make_uint4(0, 0, 0, 0);
+    const bool range = is_range(F);            // a barrier as well
+    const i64 lo = group * per_group, hi = lo + per_group < n_x ? lo + per_group : n_x;
+    if (range) count(x, lo, hi, (u64)base, mine, copies, counts, [&](u64 v) { return index_of<true>(v, F); });
+    else count(x, lo, hi, (u64)base, mine, copies, counts, [&](u64 v) { return index_of<false>(v, F); });
+    __syncthreads();
+    put_counts(counts, mine, copies, rows ? rows + group * F.n_table + base : nullptr, (F.n_table & 3) == 0, mult + base, accumulate);
+}
+
+// The same for a table of up to SMALL_TABLE entries that nothing is known of: every workgroup takes it into its LDS, sees
+// whether it is a range and, if not, makes its own hash table beside it.  One launch where the survey of a longer table takes
+// two more (1.5 M look-ups in 2^12 entries 12.0 us, in 2^13 through the survey 18.4); 32 KiB of table per workgroup come
+// from the L2.
+__global__ __launch_bounds__(COUNT_THREADS) void k_count_small(const u64 *__restrict__ x, i64 n_x, i64 per_group, const u64 *__restrict__ table,
+                                                               int n_table, int bits, int copies, u32 *rows, u64 *mult, int accumulate) {
+    extern __shared__ uint4 lds_counts[];
+    const int tid = threadIdx.x, words = (n_table * copies + 3) / 4, n_slots = 1 << bits;
+    u32 *counts = reinterpret_cast<u32 *>(lds_counts);
+    u64 *keys = reinterpret_cast<u64 *>(lds_counts + words);
+    u32 *index = reinterpret_cast<u32 *>(keys + n_table);
+    int odd = 0;
+    for (int j = tid; j < n_table; j += COUNT_THREADS) {
+        const u64 key = table[j];
+        keys[j] = key;
+        odd |= key != (u64)j;
+    }
+    for (int i = tid; i < words; i += COUNT_THREADS) lds_counts[i] = make_uint4(0, 0, 0, 0);
+    for (int i = tid; i < n_slots; i += COUNT_THREADS) index[i] = EMPTY;
+    odd = __syncthreads_or(odd);
+    const i64 group = blockIdx.x, lo = group * per_group, hi = lo + per_group < n_x ? lo + per_group : n_x;
+    if (!odd) count(x, lo, hi, 0, n_table, copies, counts, [](u64 v) { return v; });
+    else {
+        for (int j = tid; j < n_table; j += COUNT_THREADS) insert(keys, (u32)j, keys[j], nullptr, index, bits);
+        __syncthreads();
+        count(x, lo, hi, 0, n_table, copies, counts, [&](u64 v) -> u64 {
+            u32 h = slot_of(v, bits);
+            for (int probes = 0; probes < n_slots; ++probes, h = (h + 1) & (n_slots - 1)) {
+                const u32 at = index[h];
+                if (at == EMPTY) break;
+                if (keys[at] == v) return at;
+            }
+            return ~0ull;
+        });
+    }
+    __syncthreads();
+    put_counts(counts, n_table, copies, rows ? rows + group * n_table : nullptr, (n_table & 3) == 0, mult, accumulate);
 }
 
 // mult[j] (+)= sum over the rows: 64 entries per workgroup, the rows dealt over its four wavefronts, eight in flight
@@ -146,18 +235,23 @@ __global__ __launch_bounds__(BLOCK) void k_add_rows(const u32 *__restrict__ rows
     }
 }
 
-// one global atomic per look-up, through the hash table where there is one
-template <bool RANGE>
-__global__ __launch_bounds__(BLOCK) void k_count_global(const u64 *__restrict__ x, i64 n_x, const Slot *__restrict__ slots, int bits, i64 n_table,
-                                                        unsigned long long *__restrict__ mult) {
-    const i64 stride = (i64)gridDim.x * BLOCK;
-    for (i64 i = (i64)blockIdx.x * BLOCK + threadIdx.x; i < n_x; i += stride) {
-        const u64 at = index_of<RANGE>(x[i], slots, bits);
-        if (at < (u64)n_table) atomicAdd(&mult[at], 1ULL);
+// one global atomic per look-up
+__global__ __launch_bounds__(BLOCK) void k_count_global(const u64 *__restrict__ x, i64 n_x, const Finder F, unsigned long long *__restrict__ mult) {
+    const i64 stride = (i64)gridDim.x * BLOCK, first = (i64)blockIdx.x * BLOCK + threadIdx.x;
+    if (is_range(F)) {
+        for (i64 i = first; i < n_x; i += stride) {
+            const u64 at = index_of<true>(x[i], F);
+            if (at < (u64)F.n_table) atomicAdd(&mult[at], 1ULL);
+        }
+    } else {
+        for (i64 i = first; i < n_x; i += stride) {
+            const u64 at = index_of<false>(x[i], F);
+            if (at < (u64)F.n_table) atomicAdd(&mult[at], 1ULL);
+        }
     }
 }
 
-// the same without a hash table, the table searched from the front: no workspace
+// the same without a workspace, a table that is not promised to be a range searched from the front
 __global__ __launch_bounds__(BLOCK) void k_lookup_mult(const u64 *__restrict__ x, i64 n_x, const u64 *__restrict__ table, i64 n_table,
                                                        i64 t_len_range, unsigned long long *__restrict__ mult) {
     const i64 stride = (i64)gridDim.x * BLOCK;
@@ -182,32 +276,63 @@ inline unsigned capped_grid(i64 work_items) {
 }
 
 struct Plan {
-    bool direct;                               // one global atomic per look-up
+    bool small, direct;                        // k_count_small; one global atomic per look-up
     i64 slices, groups;
-    int copies, bits;
-    size_t slot_bytes, row_bytes;
+    int copies, bits, surveyors;
+    size_t key_bytes, index_bytes, odd_bytes, row_bytes;
+    size_t bytes() const { return key_bytes + index_bytes + odd_bytes + row_bytes; }
 };
 
-Plan make_plan(i64 n_x, i64 n_table, bool range) {
+// promised: the caller says that the table is a range
+Plan make_plan(i64 n_x, i64 n_table, bool promised) {
     Plan L = {};
-    L.bits = 1;
-    while (((i64)1 << L.bits) < 2 * n_table) ++L.bits;
-    L.slot_bytes = range ? 0 : sizeof(Slot) << L.bits;
+    L.small = !promised && n_table <= SMALL_TABLE;
+    if (!promised) {
+        // slots have 32-bit indices: a longer table is searched
+        if (n_table <= MAX_HASHED) {
+            L.bits = 1;
+            while (((i64)1 << L.bits) < 2 * n_table) ++L.bits;
+        }
+        if (!L.small) {
+            const i64 shares = (n_table + 4 * COUNT_THREADS - 1) / (4 * COUNT_THREADS);
+            L.surveyors = (int)(shares < SURVEYORS ? shares : SURVEYORS);
+            if (L.bits) {
+                L.key_bytes = sizeof(u64) << L.bits;
+                L.index_bytes = sizeof(u32) << L.bits;
+            }
+            L.odd_bytes = SURVEYORS * sizeof(u32);
+        }
+    }
     L.slices = (n_table + SLICE - 1) / SLICE;
     // Few look-ups, spread over many entries: 30000 in a 2^16 table take 3.6 us and 2.5 us for clearing the counts, 11 us
     // through the histogram.  And a table of many slices: all of them read all look-ups, 10 us a slice for 2^24 of them
     // against 711 us of atomics in all.
-    L.direct = (range && n_table >= 8192 && n_x <= 131072) || L.slices > 64;
+    L.direct = (n_table >= 8192 && n_x <= 131072) || L.slices > 64;
     if (L.direct) return L;
     // a workgroup per CU, but no more rows than look-ups are worth: clearing and storing a slice's counters takes as long
     // as some eight thousand look-ups
     L.groups = (n_x + 8191) / 8192;
     if (L.groups * L.slices > MAX_GROUPS) L.groups = MAX_GROUPS / L.slices;
     if (L.groups < (n_x >> 31) + 1) L.groups = (n_x >> 31) + 1;        // a group's counters have 32 bits
+    const i64 counters = L.small ? SMALL_COUNTERS : SLICE;
     L.copies = 1;
-    while (L.copies < MAX_COPIES && n_table * L.copies * 2 <= SLICE) L.copies *= 2;
+    while (L.copies < MAX_COPIES && n_table * L.copies * 2 <= counters) L.copies *= 2;
     L.row_bytes = L.groups > 1 ? (size_t)L.groups * n_table * sizeof(u32) : 0;
     return L;
+}
+
+// more than 64 KiB of dynamic LDS has to be asked for, once per device and kernel
+int ask_for_lds() {
+    static std::atomic<unsigned long long> asked{0};
+    int dev = 0;
+    VI_HIP(hipGetDevice(&dev));
+    const unsigned long long bit = 1ull << (dev & 63);
+    if (asked.load(std::memory_order_acquire) & bit) return VI_OK;
+    VI_HIP(hipFuncSetAttribute((const void *)k_count, hipFuncAttributeMaxDynamicSharedMemorySize, SLICE * (int)sizeof(u32)));
+    VI_HIP(hipFuncSetAttribute((const void *)k_count_small, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               SMALL_COUNTERS * (int)sizeof(u32) + SMALL_TABLE * (int)(sizeof(u64) + 2 * sizeof(u32))));
+    asked.fetch_or(bit, std::memory_order_release);
+    return VI_OK;
 }
 
 }  // namespace
@@ -227,60 +352,62 @@ int vi_lookup_multiplicities(const uint64_t *x, int64_t n_x, const uint64_t *tab
 
 size_t vi_lookup_histogram_workspace_bytes(int64_t n_x, int64_t n_table, int table_is_range) {
     if (n_x <= 0 || n_table <= 0) return 0;
-    const Plan L = make_plan(n_x, n_table, table_is_range != 0);
-    return L.slot_bytes + L.row_bytes;
+    return make_plan(n_x, n_table, table_is_range != 0).bytes();
 }
 
 int vi_lookup_histogram(const uint64_t *x, int64_t n_x, const uint64_t *table, int64_t n_table, int table_is_range, int accumulate,
                         uint64_t *mult, void *ws, size_t ws_bytes, void *stream) {
-    if (n_x < 0 || n_table < 0 || n_table > ((int64_t)1 << 30))
-        return vi::fail(VI_EINVAL, "vi_lookup_histogram: n_x = %lld, n_table = %lld", (long long)n_x, (long long)n_table);
+    if (n_x < 0 || n_table < 0) return vi::fail(VI_EINVAL, "vi_lookup_histogram: n_x = %lld, n_table = %lld", (long long)n_x, (long long)n_table);
     if (n_table == 0 || (n_x == 0 && accumulate)) return VI_OK;
     if ((n_x > 0 && !x) || !mult || (!table_is_range && !table)) return vi::fail(VI_EINVAL, "vi_lookup_histogram: null pointer");
-    const Plan L = make_plan(n_x, n_table, table_is_range != 0);
-    const size_t need = L.slot_bytes + L.row_bytes;
-    if (need && (!ws || ws_bytes < need)) return vi::fail(VI_ENOMEM, "vi_lookup_histogram: workspace below %zu bytes", need);
     hipStream_t s = (hipStream_t)stream;
-    Slot *slots = (Slot *)ws;
-    u32 *rows = L.row_bytes ? (u32 *)((char *)ws + L.slot_bytes) : nullptr;
-    if (!table_is_range) {
-        hipLaunchKernelGGL(k_clear_slots, dim3(capped_grid((i64)1 << L.bits)), dim3(BLOCK), 0, s, slots, (i64)1 << L.bits);
-        VI_LAUNCH_CHECK("k_clear_slots");
-        hipLaunchKernelGGL(k_insert, dim3(capped_grid(n_table)), dim3(BLOCK), 0, s, table, (i64)n_table, slots, L.bits);
-        VI_LAUNCH_CHECK("k_insert");
+    if (n_x == 0) {
+        hipLaunchKernelGGL(k_clear_counts, dim3(capped_grid(n_table)), dim3(BLOCK), 0, s, mult, (i64)n_table);
+        VI_LAUNCH_CHECK("k_clear_counts");
+        return VI_OK;
+    }
+    const Plan L = make_plan(n_x, n_table, table_is_range != 0);
+    if (L.bytes() && (!ws || ws_bytes < L.bytes())) return vi::fail(VI_ENOMEM, "vi_lookup_histogram: workspace below %zu bytes", L.bytes());
+    if (int rc = ask_for_lds()) return rc;
+    Finder F = {};
+    F.table = table;
+    F.n_table = n_table;
+    F.bits = L.bits;
+    F.keys = (u64 *)ws;
+    F.index = (u32 *)((char *)ws + L.key_bytes);
+    u32 *odd = (u32 *)((char *)ws + L.key_bytes + L.index_bytes);
+    u32 *rows = L.row_bytes ? (u32 *)((char *)ws + L.key_bytes + L.index_bytes + L.odd_bytes) : nullptr;
+    F.odd = odd;
+    F.n_odd = L.surveyors;
+    if (L.surveyors) {
+        hipLaunchKernelGGL(k_survey, dim3((unsigned)L.surveyors), dim3(COUNT_THREADS), 0, s, F, odd, L.direct && !accumulate ? mult : nullptr);
+        VI_LAUNCH_CHECK("k_survey");
+        if (L.bits) {
+            hipLaunchKernelGGL(k_insert, dim3(capped_grid(n_table)), dim3(BLOCK), 0, s, F);
+            VI_LAUNCH_CHECK("k_insert");
+        }
+    } else if (L.direct && !accumulate) {
+        hipLaunchKernelGGL(k_clear_counts, dim3(capped_grid(n_table)), dim3(BLOCK), 0, s, mult, (i64)n_table);
+        VI_LAUNCH_CHECK("k_clear_counts");
     }
     if (L.direct) {
-        if (!accumulate) {
-            hipLaunchKernelGGL(k_clear_counts, dim3(capped_grid(n_table)), dim3(BLOCK), 0, s, mult, (i64)n_table);
-            VI_LAUNCH_CHECK("k_clear_counts");
-        }
-        if (n_x == 0) return VI_OK;
-        if (table_is_range)
-            hipLaunchKernelGGL(k_count_global<true>, dim3(capped_grid(n_x)), dim3(BLOCK), 0, s, x, (i64)n_x, (const Slot *)slots, L.bits, (i64)n_table, (unsigned long long *)mult);
-        else
-            hipLaunchKernelGGL(k_count_global<false>, dim3(capped_grid(n_x)), dim3(BLOCK), 0, s, x, (i64)n_x, (const Slot *)slots, L.bits, (i64)n_table, (unsigned long long *)mult);
+        hipLaunchKernelGGL(k_count_global, dim3(capped_grid(n_x)), dim3(BLOCK), 0, s, x, (i64)n_x, F, (unsigned long long *)mult);
         VI_LAUNCH_CHECK("k_count_global");
         return VI_OK;
     }
     const i64 per = (n_x + L.groups - 1) / L.groups;
     const i64 in_slice = n_table < SLICE ? n_table : SLICE;
-    const size_t lds = ((size_t)in_slice * L.copies * sizeof(u32) + 15) & ~(size_t)15;
-    const dim3 grid((unsigned)L.slices, (unsigned)L.groups);
-    // more than 64 KiB of dynamic LDS has to be asked for, once per device and kernel
-    static std::atomic<unsigned long long> asked{0};
-    int dev = 0;
-    VI_HIP(hipGetDevice(&dev));
-    const unsigned long long bit = 1ull << (dev & 63);
-    if (!(asked.load(std::memory_order_acquire) & bit)) {
-        VI_HIP(hipFuncSetAttribute((const void *)k_count<true>, hipFuncAttributeMaxDynamicSharedMemorySize, SLICE * (int)sizeof(u32)));
-        VI_HIP(hipFuncSetAttribute((const void *)k_count<false>, hipFuncAttributeMaxDynamicSharedMemorySize, SLICE * (int)sizeof(u32)));
-        asked.fetch_or(bit, std::memory_order_release);
+    size_t lds = ((size_t)in_slice * L.copies * sizeof(u32) + 15) & ~(size_t)15;
+    if (L.small) {
+        lds += (size_t)n_table * sizeof(u64) + (sizeof(u32) << L.bits);
+        hipLaunchKernelGGL(k_count_small, dim3((unsigned)L.groups), dim3(COUNT_THREADS), lds, s, x, (i64)n_x, per, table, (int)n_table, L.bits, L.copies,
+                           rows, mult, accumulate);
+        VI_LAUNCH_CHECK("k_count_small");
+    } else {
+        hipLaunchKernelGGL(k_count, dim3((unsigned)L.slices, (unsigned)L.groups), dim3(COUNT_THREADS), lds, s, x, (i64)n_x, per, F, L.copies, rows, mult,
+                           accumulate);
+        VI_LAUNCH_CHECK("k_count");
     }
-    if (table_is_range)
-        hipLaunchKernelGGL(k_count<true>, grid, dim3(COUNT_THREADS), lds, s, x, (i64)n_x, per, (const Slot *)slots, L.bits, (i64)n_table, L.copies, rows, mult, accumulate);
-    else
-        hipLaunchKernelGGL(k_count<false>, grid, dim3(COUNT_THREADS), lds, s, x, (i64)n_x, per, (const Slot *)slots, L.bits, (i64)n_table, L.copies, rows, mult, accumulate);
-    VI_LAUNCH_CHECK("k_count");
     if (rows) {
         hipLaunchKernelGGL(k_add_rows, dim3((unsigned)((n_table + 63) / 64)), dim3(BLOCK), 0, s, (const u32 *)rows, (int)L.groups, (i64)n_table, mult, accumulate);
         VI_LAUNCH_CHECK("k_add_rows");

@@ -707,19 +707,6 @@ def gl_spmv_challenged(values, col_idx, row_ptr, seed, label, n_rows):
     return _spmv(values, col_idx, row_ptr, n_rows, None, seed, label)
 
 
-_range_table_cache: dict = {}
-
-
-def _is_range_table(table):
-    """One probe per table tensor: is table[i] == i for all i?  Cached by storage address and
-    length, as the reference does (tables are immutable once built, cuda_primitives.py:1411-1423)."""
-    key = (table.data_ptr(), table.numel())
-    if key not in _range_table_cache:
-        ref = torch.arange(table.numel(), dtype=torch.int64, device=table.device).view(torch.uint64)
-        _range_table_cache[key] = bool(torch.equal(table, ref))
-    return _range_table_cache[key]
-
-
 def lookup_multiplicities_into(x, table, mult, label=""):
     """In-place mult[j] += #{i : x[i] == table[j]}; values outside the table count nowhere
     (prover/cuda_primitives.py:1431-1446).  A table that is literally 0 .. T-1 is indexed directly."""
@@ -736,16 +723,12 @@ def lookup_multiplicities_into(x, table, mult, label=""):
 
 
 def _histogram(x, table, mult, accumulate):
+    # whether the table is a range is looked at on the device, in every call: nothing is kept of a table
     L = _lib.lib()
-    n_x, n_t, is_range = int(x.numel()), int(table.numel()), 1 if _is_range_table(table) else 0
-    if n_t > 1 << 30:                # beyond the 32-bit indices of the hash table
-        if not accumulate:
-            mult.view(torch.int64).zero_()
-        _lib.check(L.vi_lookup_multiplicities(x.data_ptr(), n_x, table.data_ptr(), n_t, is_range, mult.data_ptr(), _lib.stream_ptr()))
-        return
-    need = L.vi_lookup_histogram_workspace_bytes(n_x, n_t, is_range)
+    n_x, n_t = int(x.numel()), int(table.numel())
+    need = L.vi_lookup_histogram_workspace_bytes(n_x, n_t, 0)
     ws = _lib.workspace(need, x.device, "lookup").data_ptr() if need else None
-    _lib.check(L.vi_lookup_histogram(x.data_ptr(), n_x, table.data_ptr(), n_t, is_range, accumulate, mult.data_ptr(), ws, need,
+    _lib.check(L.vi_lookup_histogram(x.data_ptr(), n_x, table.data_ptr(), n_t, 0, accumulate, mult.data_ptr(), ws, need,
                                      _lib.stream_ptr()))
 
 
