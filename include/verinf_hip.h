@@ -354,6 +354,7 @@ int vi_lookup_multiplicities(const uint64_t *x, int64_t n_x, const uint64_t *tab
  * with table[j] == x[i]}.  table_is_range != 0 promises table[j] == j (table may then be NULL); with 0 every call looks at
  * the table on the device and goes through a hash table when it is not a range (a table of more than 2^30 entries that is
  * not one is searched from the front, entry by entry).
+ * With `accumulate` the counts are added atomically: calls on several streams may add into one mult.
  * ws: vi_lookup_histogram_workspace_bytes() bytes of device scratch. */
 size_t vi_lookup_histogram_workspace_bytes(int64_t n_x, int64_t n_table, int table_is_range);
 int vi_lookup_histogram(const uint64_t *x, int64_t n_x, const uint64_t *table, int64_t n_table, int table_is_range, int accumulate,

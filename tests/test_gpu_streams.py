@@ -65,3 +65,24 @@ def test_wrappers_from_two_threads_on_their_own_streams():
     assert len({k[2] for k in keys}) >= 2
     _lib.release_workspaces()
     assert not _lib._ws_cache
+
+
+@pytest.mark.parametrize("n_table", [100, 5000, 40000])
+def test_look_ups_on_two_streams_add_into_one_table(n_table):
+    """lookup_multiplicities_into adds: calls on streams without an order between them lose no counts."""
+    from verinf_amd.prover import cuda_primitives as cp
+    rng = np.random.default_rng(n_table)
+    table = to_dev(np.arange(n_table, dtype=np.uint64))
+    for n_x in (5000, 300000):                                   # one workgroup per slice, and rows added up by a second launch
+        xs = [rng.integers(0, n_table, n_x).astype(np.uint64) for _ in range(2)]
+        dev = [to_dev(x) for x in xs]
+        mult = torch.zeros(n_table, dtype=torch.int64, device="cuda").view(torch.uint64)
+        torch.cuda.synchronize()
+        streams, rounds = [torch.cuda.Stream(), torch.cuda.Stream()], 40
+        for _ in range(rounds):
+            for s, x in zip(streams, dev):
+                with torch.cuda.stream(s):
+                    cp.lookup_multiplicities_into(x, table, mult)
+        torch.cuda.synchronize()
+        want = sum(np.bincount(x.astype(np.int64), minlength=n_table) for x in xs) * rounds
+        assert np.array_equal(to_np(mult), want.astype(np.uint64))

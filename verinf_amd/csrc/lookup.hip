@@ -135,6 +135,12 @@ __device__ __forceinline__ void count(const u64 *__restrict__ x, i64 lo, i64 hi,
     }
 }
 
+// mult = c, or mult += c: an atomic one, as calls on other streams may be adding to the same counts
+__device__ __forceinline__ void put(u64 *mult, u64 c, int accumulate) {
+    if (!accumulate) *mult = c;
+    else if (c) atomicAdd((unsigned long long *)mult, (unsigned long long)c);
+}
+
 // a workgroup's counts to its row, or straight to the result where there are no rows
 __device__ __forceinline__ void put_counts(const u32 *counts, int mine, int copies, u32 *row, bool aligned, u64 *mult, int accumulate) {
     const int tid = threadIdx.x;
@@ -147,7 +153,7 @@ __device__ __forceinline__ void put_counts(const u32 *counts, int mine, int copi
         u32 c = 0;
         for (int k = 0; k < copies; ++k) c += counts[i * copies + ((k + tid) & (copies - 1))];
         if (row) row[i] = c;
-        else mult[i] = accumulate ? mult[i] + c : (u64)c;
+        else put(&mult[i], c, accumulate);
     }
 }
 
@@ -231,7 +237,7 @@ __global__ __launch_bounds__(BLOCK) void k_add_rows(const u32 *__restrict__ rows
     __syncthreads();
     if (w == 0 && j < n_table) {
         sum = part[0][lane] + part[1][lane] + part[2][lane] + part[3][lane];
-        mult[j] = accumulate ? mult[j] + sum : sum;
+        put(&mult[j], sum, accumulate);
     }
 }
 
