@@ -86,3 +86,93 @@ def test_look_ups_on_two_streams_add_into_one_table(n_table):
         torch.cuda.synchronize()
         want = sum(np.bincount(x.astype(np.int64), minlength=n_table) for x in xs) * rounds
         assert np.array_equal(to_np(mult), want.astype(np.uint64))
+
+
+def _two_threads(job, count=2):
+    """job(i) on `count` threads that switch as often as the interpreter can, all on the default stream."""
+    import sys
+    errors, gate = [], threading.Barrier(count)
+
+    def work(i):
+        try:
+            gate.wait()
+            job(i)
+        except BaseException as exc:                             # surfaced by the main thread
+            errors.append(exc)
+
+    before = sys.getswitchinterval()
+    sys.setswitchinterval(1e-6)
+    try:
+        threads = [threading.Thread(target=work, args=(i,)) for i in range(count)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+    finally:
+        sys.setswitchinterval(before)
+    assert not errors, errors
+
+
+def test_threads_that_share_a_stream_do_not_share_a_call():
+    """Calls of several launches through scratch: the launches of two threads' calls on one stream do not mix, also while the
+    scratch grows."""
+    from verinf_amd import _lib
+    from verinf_amd.layergkr import gpu
+    from verinf_amd.prover import cuda_primitives as cp
+    _lib.release_workspaces()
+
+    def inputs(i):
+        tabs = [rand_field(1 << (10 + i), 70 + 10 * i + j) for j in range(3)]
+        table = np.arange(5000 + 3000 * i, dtype=np.uint64)
+        return {"lde": rand_field((5 + 40 * i, 1 << 13), 61 + i), "ntt": rand_field((3 + 9 * i, 1 << 14), 63 + i),
+                "a": rand_field((70 + 60 * i, 300), 65 + i), "b": rand_field((300, 500 + 300 * i), 67 + i),
+                "x": np.random.default_rng(i).integers(0, len(table), 200000 + 100000 * i).astype(np.uint64), "table": table,
+                "hash": rand_field((300 + 100 * i, 64), 69 + i), "sum": rand_field(70000 + i, 80 + i), "tabs": tabs,
+                "mat": np.stack(tabs), "coins": [random.Random(i + 7 * j).randrange(P) for j in range(10 + i)]}
+
+    data = [inputs(i) for i in range(2)]
+    dev = [{k: [to_dev(t) for t in v] if k == "tabs" else (v if k == "coins" else to_dev(v)) for k, v in d.items()} for d in data]
+
+    def calls(d):
+        rows = d["ntt"].clone()
+        cp.ntt_forward_batched(rows)
+        claim, polys, _, _ = gpu.prove_terms_gpu([(1, d["tabs"])], lambda r: d["coins"][r], P)
+        return [cp.coset_lde(d["lde"], 1 << 13, 1 << 15), rows, cp.gl_matmul(d["a"], d["b"]), cp.lookup_multiplicities(d["x"], d["table"]),
+                cp.hash_columns_streamed(d["hash"]), gpu.gl_sum(d["sum"])], claim, polys, gpu.mle_eval_t(d["mat"], d["coins"])
+
+    out = {0: [], 1: []}
+    _two_threads(lambda i: out[i].extend(calls(dev[i]) for _ in range(25)))
+    torch.cuda.synchronize()
+    for i in range(2):
+        d = data[i]
+        want = [O.coset_lde_rows(d["lde"], 1 << 13, 1 << 15, 7), O.ntt_rows(d["ntt"]), None,
+                np.bincount(d["x"].astype(np.int64), minlength=len(d["table"])).astype(np.uint64), O.hash_columns(d["hash"]), None]
+        want[2] = (d["a"].astype(object).dot(d["b"].astype(object)) % P).astype(np.uint64)
+        want[5] = np.array([sum(int(v) for v in d["sum"]) % P], dtype=np.uint64)
+        want_claim, want_samples, _ = O.sumcheck_prove(d["tabs"], [(1, [0, 1, 2])], d["coins"])
+        want_ends = [O.mle_eval(t, d["coins"]) for t in d["tabs"]]
+        for tensors, claim, polys, ends in out[i]:
+            for k, (got, w) in enumerate(zip(tensors, want)):
+                assert np.array_equal(to_np(got), w), k
+            assert claim == want_claim and [[y for _, y in s] for s in polys] == want_samples and ends == want_ends
+
+
+def test_interactive_proofs_on_one_stream_in_step():
+    """Two provers whose coins wait for each other in every round: neither holds what the other one needs."""
+    from verinf_amd.layergkr import gpu
+    n_rounds, gate = 9, threading.Barrier(2, timeout=60)
+    tabs = [[rand_field(1 << n_rounds, 90 + 10 * i + j) for j in range(3)] for i in range(2)]
+    dev = [[to_dev(t) for t in ts] for ts in tabs]
+    coins = [random.Random(5).randrange(P) for _ in range(n_rounds)]
+    out = [None, None]
+
+    def job(i):
+        def coin(rnd, samples):
+            gate.wait()
+            return coins[rnd]
+        out[i] = gpu.prove_terms_gpu_interactive([(1, dev[i]), (3, dev[i][:2])], coin, P)
+
+    _two_threads(job)
+    for i in range(2):
+        want_claim, want_samples, _ = O.sumcheck_prove(tabs[i], [(1, [0, 1, 2]), (3, [0, 1])], coins)
+        assert out[i][0] == want_claim and [[y for _, y in s] for s in out[i][1]] == want_samples

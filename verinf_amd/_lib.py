@@ -178,23 +178,33 @@ def on_device(dev):
 
 
 _ws_cache = {}
+_stream_locks = {}
 
 
-def workspace(nbytes: int, device=None, tag: str = "ws", stream_ptr=None):
-    """A cached uint8 device buffer of at least nbytes for the CURRENT stream of `device`.
+def stream_lock(stream_ptr: int):
+    """The lock of the current device's stream with this handle, which a call that uses workspace() holds from there to its
+    last launch.
+
+    Host threads that share a stream share its scratch buffers: what one call leaves in them for its next launch has to
+    stay there until that launch is queued, and a buffer that another thread outgrows must not be dropped before.  The
+    lock is held while work is queued, not while the host waits for a result or runs a caller's code."""
+    key = (_get_device(), stream_ptr)
+    lock = _stream_locks.get(key)
+    return lock if lock is not None else _stream_locks.setdefault(key, threading.RLock())
+
+
+def workspace(nbytes: int, tag: str, stream_ptr: int):
+    """A cached uint8 device buffer of at least nbytes for a stream of the current device; the caller holds stream_lock().
 
     One buffer per (purpose, device, stream): the wrappers launch on torch's current stream, so two streams
     (or two host threads on their own streams) never share scratch, and a buffer is only ever used on the
     stream it was allocated on -- when it is outgrown and dropped, the caching allocator may reuse its memory
     in stream order without further bookkeeping.  Buffers grow and are kept; release_workspaces() drops them."""
-    index = _get_device() if device is None or device.index is None else device.index
-    # stream_ptr: the current stream's handle when the caller has looked it up already
-    key = (tag, index, _raw_stream(index) if stream_ptr is None else stream_ptr)
+    index = _get_device()
+    key = (tag, index, stream_ptr)
     buf = _ws_cache.get(key)
     if buf is None or buf.numel() < nbytes:
-        with torch.cuda.device(index):
-            buf = torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=torch.device("cuda", index))
-        _ws_cache[key] = buf
+        buf = _ws_cache[key] = torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=torch.device("cuda", index))
     return buf
 
 
@@ -214,6 +224,22 @@ def pinned_words(words: int, stream_ptr: int):
     if buf is None or buf[0].numel() < words:
         t = torch.zeros(max(words, 512), dtype=torch.uint64).pin_memory()
         buf = bufs[key] = (t, t.numpy())
+    return buf
+
+
+_results = threading.local()
+
+
+def result_words(words: int, stream_ptr: int):
+    """Device words for a result that the host waits for: one buffer per host thread and stream like pinned_words(), so that
+    another thread's call cannot write over it while this one waits."""
+    bufs = getattr(_results, "bufs", None)
+    if bufs is None:
+        bufs = _results.bufs = {}
+    key = (_get_device(), stream_ptr)
+    buf = bufs.get(key)
+    if buf is None or buf.numel() < words:
+        buf = bufs[key] = torch.empty(max(words, 512), dtype=torch.uint64, device=torch.device("cuda", key[0]))
     return buf
 
 
@@ -265,4 +291,6 @@ def upload_words(words):
 def release_workspaces() -> None:
     """Drop every cached scratch buffer (they come back on demand).  Call it with the device idle: a buffer
     still in use by queued kernels must not be handed back to the allocator from another stream."""
-    _ws_cache.clear()
+    for key in list(_ws_cache):
+        with _stream_locks.get(key[1:], _NO_GUARD):          # not between a call's look-up and its launches
+            _ws_cache.pop(key, None)

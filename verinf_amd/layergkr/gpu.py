@@ -223,9 +223,11 @@ def mle_eval_t(tables, point: Sequence[int]):
     with _lib.on_device(tables.device):
         sp = _lib.stream_ptr()
         ws_bytes = L.vi_mle_eval_workspace_bytes(k)
-        ws = _lib.workspace(ws_bytes + 8 * k, tables.device, "mle", sp).data_ptr()
-        _lib.check(L.vi_mle_eval(mat.data_ptr(), k, 1 << n, _point(point), n, ws + ws_bytes, ws, ws_bytes, sp))
-        vals = list(struct.unpack(f"<{k}Q", _lib.read_back_ptr(ws + ws_bytes, 8 * k, sp)))
+        out = _lib.result_words(k, sp)
+        with _lib.stream_lock(sp):
+            ws = _lib.workspace(ws_bytes, "mle", sp)
+            _lib.check(L.vi_mle_eval(mat.data_ptr(), k, 1 << n, _point(point), n, out.data_ptr(), ws.data_ptr(), ws_bytes, sp))
+        vals = list(struct.unpack(f"<{k}Q", _lib.read_back_ptr(out.data_ptr(), 8 * k, sp)))
     return vals[0] if one else vals
 
 
@@ -240,9 +242,10 @@ def gl_sum(t):
     out = torch.empty(1, dtype=torch.uint64, device=v.device)
     L = _lib.lib()
     with _lib.on_device(v.device):
-        ws = _lib.workspace(L.vi_gl_sum_workspace_bytes(v.numel()), v.device, "sum")
-        _lib.check(L.vi_gl_sum(v.data_ptr(), v.numel(), out.data_ptr(), ws.data_ptr(), ws.numel(),
-                               _lib.stream_ptr()))
+        sp = _lib.stream_ptr()
+        with _lib.stream_lock(sp):
+            ws = _lib.workspace(L.vi_gl_sum_workspace_bytes(v.numel()), "sum", sp)
+            _lib.check(L.vi_gl_sum(v.data_ptr(), v.numel(), out.data_ptr(), ws.data_ptr(), ws.numel(), sp))
     return out
 
 
@@ -374,17 +377,18 @@ def prove_terms_gpu(terms, coin, field_p: int, mask=None, mu0: int = 0):
     with _lib.on_device(dev):
         stream = torch.cuda.current_stream()
         sp = stream.cuda_stream
-        ws = _lib.workspace(L.vi_sumcheck_prove_coins_workspace_bytes(size), dev, "sumcheck_coins", sp)
-        # the folded tables live in one cached scratch buffer, a half-length slice per table (the caller's
-        # tensors are never written)
-        half_bytes = (size // 2) * 8
-        work = _lib.workspace(max(prob.n_tables * half_bytes, 256), dev, "sumcheck_work", sp)
-        work_p = (ctypes.c_void_p * prob.n_tables)(*[work.data_ptr() + t * half_bytes for t in range(prob.n_tables)])
         samples_host, samples_np = _lib.pinned_words(8 * n_rounds, sp)
         chal = (ctypes.c_uint64 * n_rounds)(*challenges)
-        _lib.check(L.vi_sumcheck_prove_coins(_Problem.ptrs(tables), work_p, prob.n_tables, size,
-                                             prob.term_off, prob.factor_idx, prob.coeffs, prob.n_terms, chal,
-                                             samples_host.data_ptr(), ws.data_ptr(), ws.numel(), sp))
+        with _lib.stream_lock(sp):
+            ws = _lib.workspace(L.vi_sumcheck_prove_coins_workspace_bytes(size), "sumcheck_coins", sp)
+            # the folded tables live in one cached scratch buffer, a half-length slice per table (the caller's
+            # tensors are never written)
+            half_bytes = (size // 2) * 8
+            work = _lib.workspace(max(prob.n_tables * half_bytes, 256), "sumcheck_work", sp)
+            work_p = (ctypes.c_void_p * prob.n_tables)(*[work.data_ptr() + t * half_bytes for t in range(prob.n_tables)])
+            _lib.check(L.vi_sumcheck_prove_coins(_Problem.ptrs(tables), work_p, prob.n_tables, size,
+                                                 prob.term_off, prob.factor_idx, prob.coeffs, prob.n_terms, chal,
+                                                 samples_host.data_ptr(), ws.data_ptr(), ws.numel(), sp))
         stream.synchronize()
         rows = samples_np[:8 * n_rounds].reshape(n_rounds, 8)[:, :deg + 1].tolist()
     if mask is None:
@@ -413,7 +417,8 @@ def prove_terms_gpu_interactive(terms, coin, field_p: int, mask=None, mu0: int =
     mu = mu0 % field_p
 
     with _lib.on_device(dev):
-        ws = _lib.workspace(L.vi_sumcheck_workspace_bytes(), dev, "sumcheck")
+        # scratch of this proof alone: it is in use from round to round, and the coin's code runs in between
+        ws = torch.empty(L.vi_sumcheck_workspace_bytes(), dtype=torch.uint8, device=dev)
         # The round loop runs inside the library: per round one fused launch, a wait on a word of pinned host
         # memory that the kernel stores behind its samples, and this callback -- the only Python left in the
         # loop -- which applies the optional scalar mask and asks the verifier coin for the challenge.

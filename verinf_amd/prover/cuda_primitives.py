@@ -141,11 +141,13 @@ def _ntt(rows, m, n, inverse):
         # the library transforms the rows in chunks that fit the workspace it is given: one row is the minimum,
         # 1 GiB is enough to fill the GPU, and a large batch does not double its footprint for the process's life
         need = min(L.vi_ntt_best_workspace_bytes(m, n), max(_NTT_WS_CAP, n * 8))
-        ws, ws_bytes = None, 0
-        if need:
-            buf = _lib.workspace(need, rows.device, "ntt")
-            ws, ws_bytes = buf.data_ptr(), buf.numel()
-        _lib.check(L.vi_ntt_batched(rows.data_ptr(), m, n, int(inverse), ws, ws_bytes, _lib.stream_ptr()))
+        sp = _lib.stream_ptr()
+        if not need:
+            _lib.check(L.vi_ntt_batched(rows.data_ptr(), m, n, int(inverse), None, 0, sp))
+            return
+        with _lib.stream_lock(sp):
+            ws = _lib.workspace(need, "ntt", sp)
+            _lib.check(L.vi_ntt_batched(rows.data_ptr(), m, n, int(inverse), ws.data_ptr(), ws.numel(), sp))
 
 
 def _ntt_1d(a, inverse):
@@ -232,9 +234,11 @@ def coset_lde(messages, k_deg, n_lig, shift=GLOBAL_G, out=None):
         return out.view(torch.int64).zero_().view(torch.uint64)
     L = _lib.lib()
     with _lib.on_device(messages.device):
-        ws = _lib.workspace(L.vi_coset_lde_workspace_bytes(m, k_deg, n_lig), messages.device, "lde")
-        _lib.check(L.vi_coset_lde(messages.data_ptr(), m, w, in_stride, k_deg, n_lig, int(shift) % P,
-                                  out.data_ptr(), n_lig, ws.data_ptr(), ws.numel(), _lib.stream_ptr()))
+        sp = _lib.stream_ptr()
+        with _lib.stream_lock(sp):
+            ws = _lib.workspace(L.vi_coset_lde_workspace_bytes(m, k_deg, n_lig), "lde", sp)
+            _lib.check(L.vi_coset_lde(messages.data_ptr(), m, w, in_stride, k_deg, n_lig, int(shift) % P,
+                                      out.data_ptr(), n_lig, ws.data_ptr(), ws.numel(), sp))
     return out
 
 
@@ -262,10 +266,12 @@ def coset_lde_with_coeffs(messages, k_deg, n_lig, shift=GLOBAL_G, need_codewords
         return coeffs, out
     L = _lib.lib()
     with _lib.on_device(messages.device):
-        ws = _lib.workspace(L.vi_coset_lde_workspace_bytes(m, k_deg, n_lig), messages.device, "lde")
-        _lib.check(L.vi_coset_lde_coeffs(messages.data_ptr(), m, w, in_stride, k_deg, n_lig, int(shift) % P,
-                                         coeffs.data_ptr(), k_deg, out.data_ptr() if out is not None else None, n_lig,
-                                         ws.data_ptr(), ws.numel(), _lib.stream_ptr()))
+        sp = _lib.stream_ptr()
+        with _lib.stream_lock(sp):
+            ws = _lib.workspace(L.vi_coset_lde_workspace_bytes(m, k_deg, n_lig), "lde", sp)
+            _lib.check(L.vi_coset_lde_coeffs(messages.data_ptr(), m, w, in_stride, k_deg, n_lig, int(shift) % P,
+                                             coeffs.data_ptr(), k_deg, out.data_ptr() if out is not None else None, n_lig,
+                                             ws.data_ptr(), ws.numel(), sp))
     return coeffs, out
 
 
@@ -281,9 +287,11 @@ def coset_extend(coeffs, k_deg, n_lig, shift=GLOBAL_G, out=None):
         return out.view(torch.int64).zero_().view(torch.uint64)
     L = _lib.lib()
     with _lib.on_device(coeffs.device):
-        ws = _lib.workspace(L.vi_coset_lde_workspace_bytes(m, k_deg, n_lig), coeffs.device, "lde")
-        _lib.check(L.vi_coset_extend(coeffs.data_ptr(), m, w, in_stride, k_deg, n_lig, int(shift) % P,
-                                     out.data_ptr(), n_lig, ws.data_ptr(), ws.numel(), _lib.stream_ptr()))
+        sp = _lib.stream_ptr()
+        with _lib.stream_lock(sp):
+            ws = _lib.workspace(L.vi_coset_lde_workspace_bytes(m, k_deg, n_lig), "lde", sp)
+            _lib.check(L.vi_coset_extend(coeffs.data_ptr(), m, w, in_stride, k_deg, n_lig, int(shift) % P,
+                                         out.data_ptr(), n_lig, ws.data_ptr(), ws.numel(), sp))
     return out
 
 
@@ -312,12 +320,16 @@ def gl_matmul(A, B):
     L = _lib.lib()
     a_ptr, c_ptr = A.data_ptr(), C.data_ptr()
     with _lib.on_device(A.device):
+        sp = _lib.stream_ptr()
         for lo in range(0, m, 65535):
             rows = min(65535, m - lo)
             need = L.vi_gl_matmul_workspace_bytes(rows, k, n)
-            ws = _lib.workspace(need, A.device, "matmul").data_ptr() if need else None
-            _lib.check(L.vi_gl_matmul(a_ptr + lo * k * 8, B.data_ptr(), c_ptr + lo * n * 8, rows, k, n, ws, need,
-                                      _lib.stream_ptr()))
+            if not need:
+                _lib.check(L.vi_gl_matmul(a_ptr + lo * k * 8, B.data_ptr(), c_ptr + lo * n * 8, rows, k, n, None, 0, sp))
+                continue
+            with _lib.stream_lock(sp):
+                ws = _lib.workspace(need, "matmul", sp)
+                _lib.check(L.vi_gl_matmul(a_ptr + lo * k * 8, B.data_ptr(), c_ptr + lo * n * 8, rows, k, n, ws.data_ptr(), need, sp))
     return C
 
 
@@ -444,9 +456,11 @@ def hash_columns_streamed(matrix):
     L = _lib.lib()
     out = torch.empty((n, 32), dtype=torch.uint8, device=matrix.device)
     nbytes = L.vi_hash_columns_workspace_bytes(m, n)
-    ws = _lib.workspace(nbytes, matrix.device, "hash")
-    _lib.check(L.vi_hash_columns(matrix.data_ptr(), m, n, stride, out.data_ptr(), ws.data_ptr(), ws.numel(),
-                                 _lib.stream_ptr()))
+    with _lib.on_device(matrix.device):
+        sp = _lib.stream_ptr()
+        with _lib.stream_lock(sp):
+            ws = _lib.workspace(nbytes, "hash", sp)
+            _lib.check(L.vi_hash_columns(matrix.data_ptr(), m, n, stride, out.data_ptr(), ws.data_ptr(), ws.numel(), sp))
     return out
 
 
@@ -727,9 +741,15 @@ def _histogram(x, table, mult, accumulate):
     L = _lib.lib()
     n_x, n_t = int(x.numel()), int(table.numel())
     need = L.vi_lookup_histogram_workspace_bytes(n_x, n_t, 0)
-    ws = _lib.workspace(need, x.device, "lookup").data_ptr() if need else None
-    _lib.check(L.vi_lookup_histogram(x.data_ptr(), n_x, table.data_ptr(), n_t, 0, accumulate, mult.data_ptr(), ws, need,
-                                     _lib.stream_ptr()))
+    args = (x.data_ptr(), n_x, table.data_ptr(), n_t, 0, accumulate, mult.data_ptr())
+    with _lib.on_device(x.device):
+        sp = _lib.stream_ptr()
+        if not need:
+            _lib.check(L.vi_lookup_histogram(*args, None, 0, sp))
+            return
+        with _lib.stream_lock(sp):
+            ws = _lib.workspace(need, "lookup", sp)
+            _lib.check(L.vi_lookup_histogram(*args, ws.data_ptr(), need, sp))
 
 
 def lookup_multiplicities(x, table):
