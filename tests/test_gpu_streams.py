@@ -176,3 +176,48 @@ def test_interactive_proofs_on_one_stream_in_step():
     for i in range(2):
         want_claim, want_samples, _ = O.sumcheck_prove(tabs[i], [(1, [0, 1, 2]), (3, [0, 1])], coins)
         assert out[i][0] == want_claim and [[y for _, y in s] for s in out[i][1]] == want_samples
+
+
+def test_a_graph_keeps_its_scratch_when_later_calls_outgrow_it():
+    """Captured calls that use scratch, replayed after larger calls on the same stream took bigger buffers and other tensors
+    took the memory that the smaller ones had."""
+    from verinf_amd import _lib
+    from verinf_amd.layergkr import gpu
+    from verinf_amd.prover import cuda_primitives as cp
+    _lib.release_workspaces()
+    side = torch.cuda.Stream()
+
+    def calls(lde, rows, a, b, x, table, mat, vec):
+        rows = rows.clone()
+        cp.ntt_forward_batched(rows)
+        return [cp.coset_lde(lde, 1 << 13, 1 << 15), rows, cp.gl_matmul(a, b), cp.lookup_multiplicities(x, table), cp.hash_columns_streamed(mat),
+                gpu.gl_sum(vec)]
+
+    def inputs(scale, seed):
+        shapes = ((2 * scale, 1 << 13), (2 * scale, 1 << 14), (80 * scale, 200), (200, 400 * scale))
+        table = np.arange(6000 * scale, dtype=np.uint64)
+        x = np.random.default_rng(seed).integers(0, len(table), 150000).astype(np.uint64)
+        return [*(to_dev(rand_field(s, seed + i)) for i, s in enumerate(shapes)), to_dev(x), to_dev(table), to_dev(rand_field((300 * scale, 64), seed + 9)),
+                to_dev(rand_field(5000 * scale, seed + 10))]
+
+    args, side_args = inputs(1, 1), inputs(8, 50)
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        calls(*args)                                             # tables are uploaded here, and small scratch is cached
+    side.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=side):
+        outs = calls(*args)
+    with torch.cuda.stream(side):
+        calls(*side_args)
+    side.synchronize()
+    others = [torch.full((1 << s,), 0x5A, dtype=torch.uint8, device="cuda") for s in range(10, 24) for _ in range(2)]
+    for seed in (1, 20, 40):
+        for old, new in zip(args, inputs(1, seed)):
+            old.copy_(new)
+        want = calls(*args)
+        g.replay()
+        torch.cuda.synchronize()
+        for k, (got, w) in enumerate(zip(outs, want)):
+            assert np.array_equal(to_np(got), to_np(w)), (seed, k)
+        assert all(bool((o == 0x5A).all()) for o in others)

@@ -162,6 +162,7 @@ def check(rc: int) -> None:
 # the kernels of a small call take (0.08 and 0.13 us this way).
 _raw_stream = torch._C._cuda_getCurrentRawStream
 _get_device = torch._C._cuda_getDevice
+_capturing = torch._C._cuda_isCurrentStreamCapturing
 
 
 def stream_ptr() -> int:
@@ -199,8 +200,12 @@ def workspace(nbytes: int, tag: str, stream_ptr: int):
     One buffer per (purpose, device, stream): the wrappers launch on torch's current stream, so two streams
     (or two host threads on their own streams) never share scratch, and a buffer is only ever used on the
     stream it was allocated on -- when it is outgrown and dropped, the caching allocator may reuse its memory
-    in stream order without further bookkeeping.  Buffers grow and are kept; release_workspaces() drops them."""
+    in stream order without further bookkeeping.  Buffers grow and are kept; release_workspaces() drops them.
+    A call under stream capture gets a buffer of its own from the graph's memory: the graph keeps its address, and a
+    cached one may be outgrown and given back while the graph lives."""
     index = _get_device()
+    if stream_ptr and _capturing():              # the default stream (0) cannot be captured; asking costs 0.35 us
+        return torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=torch.device("cuda", index))
     key = (tag, index, stream_ptr)
     buf = _ws_cache.get(key)
     if buf is None or buf.numel() < nbytes:
