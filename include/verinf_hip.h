@@ -87,8 +87,9 @@ int vi_gl_sum(const uint64_t *a, int64_t n, uint64_t *out, void *ws, size_t ws_b
  * Replace gl_matmul / gl_matvec (prover/cuda_primitives.py:485-510,
  * prover/kernels/gl_matmul.cuh:29-59) and poly_eval (cuda_primitives.py:462-479,
  * prover/kernels/gl_extras.cuh:93-108).  All matrices row-major and dense.
- *   vi_gl_matmul   C (m x n) = A (m x k) B (k x n); at most 65535 rows of A; the shape it is
- *                  tuned for is a few rows of A against a tall B (projection seam, combine).
+ *   vi_gl_matmul   C (m x n) = A (m x k) B (k x n); at most 65535 rows of A.  A few rows of A stream a
+ *                  tall B (projection seam, combine); products of many rows go to the matrix cores, through
+ *                  planes of residues in the workspace (up to about 1.1 GiB; 8-byte aligned, as for every entry).
  *   vi_gl_matvec   w (m) = M (m x n) v (n)
  *   vi_poly_eval   out[r][p] = sum_i coeffs[r][i] points[p]^i, coeffs (m x d), out (m x k) */
 size_t vi_gl_matmul_workspace_bytes(int64_t m, int64_t k, int64_t n);
@@ -355,7 +356,7 @@ int vi_lookup_multiplicities(const uint64_t *x, int64_t n_x, const uint64_t *tab
  * the table on the device and goes through a hash table when it is not a range (a table of more than 2^30 entries that is
  * not one is searched from the front, entry by entry).
  * With `accumulate` the counts are added atomically: calls on several streams may add into one mult.
- * ws: vi_lookup_histogram_workspace_bytes() bytes of device scratch. */
+ * ws: vi_lookup_histogram_workspace_bytes() bytes of device scratch, 8-byte aligned as for every entry. */
 size_t vi_lookup_histogram_workspace_bytes(int64_t n_x, int64_t n_table, int table_is_range);
 int vi_lookup_histogram(const uint64_t *x, int64_t n_x, const uint64_t *table, int64_t n_table, int table_is_range, int accumulate,
                         uint64_t *mult, void *ws, size_t ws_bytes, void *stream);

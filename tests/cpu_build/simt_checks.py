@@ -25,11 +25,10 @@ def ptr(a):
 
 
 def scratch(nbytes):
-    """nbytes of garbage, 16-byte aligned, nothing behind them."""
-    a = np.empty(nbytes, dtype=np.uint8)
+    """nbytes of garbage from an address that is a multiple of 8 only, nothing behind them."""
+    a = np.full(nbytes + 8, 0xA5, dtype=np.uint8)
     assert a.ctypes.data % 16 == 0
-    a[:] = 0xA5
-    return a
+    return a[8:]
 
 
 def lookup(so):
@@ -57,7 +56,7 @@ def lookup(so):
 
     # one and several groups, copies per entry, both sides of the small table, slices, one atomic per look-up
     for n_x, n_t in ((0, 5), (1, 1), (9000, 3), (500, 1024), (9001, 1025), (300, 4096), (9001, 4096), (9001, 4097), (700, 8191), (900, 8192),
-                     (131073, 8192), (9001, 32771), (140001, 32771)):
+                     (131073, 8192), (9001, 32771), (140001, 32772)):
         rng = np.random.default_rng(n_x + n_t)
         span = np.arange(n_t, dtype=np.uint64)
         x = rng.integers(0, n_t + n_t // 8 + 1, n_x).astype(np.uint64)

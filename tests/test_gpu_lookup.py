@@ -134,3 +134,19 @@ def test_a_table_beyond_the_hash():
     assert got[[5, 12345]].tolist() == [30, 1] and int(got.sum()) == 31
     del got, table
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("n_table", [3000, 40000])
+@pytest.mark.parametrize("skip", [0, 4, 8])
+def test_scratch_of_any_alignment(n_table, skip):
+    from verinf_amd import _lib
+    L = _lib.lib()
+    table = rand_field((n_table,), 4)
+    x = table[np.random.default_rng(2).integers(0, n_table, 300000)]
+    dx, dt = to_dev(x), to_dev(table)
+    need = L.vi_lookup_histogram_workspace_bytes(len(x), n_table, 0)
+    ws = torch.full((need + skip + 64,), 0x5A, dtype=torch.uint8, device="cuda")
+    mult = torch.empty(n_table, dtype=torch.uint64, device="cuda")
+    _lib.check(L.vi_lookup_histogram(dx.data_ptr(), len(x), dt.data_ptr(), n_table, 0, 0, mult.data_ptr(), ws.data_ptr() + skip, need, _lib.stream_ptr()))
+    assert np.array_equal(to_np(mult), _counts(x, table))
+    assert bool((ws[:skip] == 0x5A).all()) and bool((ws[need + skip:] == 0x5A).all())

@@ -35,3 +35,20 @@ def test_matmul_edges(m, k, n, fill):
     cols = np.unique(np.linspace(0, n - 1, max(2, budget // len(rows))).astype(int)) if n * len(rows) > budget else np.arange(n)
     want = (A[rows].astype(object).dot(B[:, cols].astype(object)) % P).astype(np.uint64)
     assert np.array_equal(got[np.ix_(rows, cols)], want)
+
+
+@pytest.mark.parametrize("skip", [0, 8])
+def test_scratch_of_any_alignment(skip):
+    from verinf_amd import _lib
+    L = _lib.lib()
+    m, k, n = 130, 70, 150
+    A, B = rand_field((m, k), 1), rand_field((k, n), 2)
+    dA, dB, C = to_dev(A), to_dev(B), torch.empty((m, n), dtype=torch.uint64, device="cuda")
+    while (need := L.vi_gl_matmul_workspace_bytes(m, k, n)) < 18 * 128 * 128:           # a size of the matrix cores
+        m *= 2
+        A = rand_field((m, k), 1)
+        dA, C = to_dev(A), torch.empty((m, n), dtype=torch.uint64, device="cuda")
+    ws = torch.full((need + skip + 64,), 0x5A, dtype=torch.uint8, device="cuda")
+    _lib.check(L.vi_gl_matmul(dA.data_ptr(), dB.data_ptr(), C.data_ptr(), m, k, n, ws.data_ptr() + skip, need, _lib.stream_ptr()))
+    assert np.array_equal(to_np(C), (A.astype(object).dot(B.astype(object)) % P).astype(np.uint64))
+    assert bool((ws[:skip] == 0x5A).all()) and bool((ws[need + skip:] == 0x5A).all())

@@ -30,6 +30,11 @@ inline int ilog2(long long x) {
     return l;
 }
 
+// A workspace whose kernels use 16-byte accesses: the first such address at or behind ws.  Its *_workspace_bytes() includes
+// the WS_SLACK bytes this may skip.
+constexpr size_t WS_SLACK = 16;
+inline void *align16(void *ws) { return (void *)(((uintptr_t)ws + 15) & ~(uintptr_t)15); }
+
 // Waits until the kernel that finishes a result has stored `seq` behind it in pinned host memory.  The word is polled (a
 // stream synchronisation costs several microseconds more); every 2^16 polls the stream is queried, so a failed launch or
 // a stream that drained without the store ends the wait with an error instead of spinning.

@@ -286,7 +286,10 @@ struct Plan {
     i64 slices, groups;
     int copies, bits, surveyors;
     size_t key_bytes, index_bytes, odd_bytes, row_bytes;
-    size_t bytes() const { return key_bytes + index_bytes + odd_bytes + row_bytes; }
+    size_t bytes() const {
+        const size_t used = key_bytes + index_bytes + odd_bytes + row_bytes;
+        return used ? used + vi::WS_SLACK : 0;
+    }
 };
 
 // promised: the caller says that the table is a range
@@ -375,6 +378,7 @@ int vi_lookup_histogram(const uint64_t *x, int64_t n_x, const uint64_t *table, i
     const Plan L = make_plan(n_x, n_table, table_is_range != 0);
     if (L.bytes() && (!ws || ws_bytes < L.bytes())) return vi::fail(VI_ENOMEM, "vi_lookup_histogram: workspace below %zu bytes", L.bytes());
     if (int rc = ask_for_lds()) return rc;
+    ws = vi::align16(ws);
     Finder F = {};
     F.table = table;
     F.n_table = n_table;

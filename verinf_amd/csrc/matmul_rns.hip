@@ -381,11 +381,12 @@ bool rns_matmul_pays(int64_t m, int64_t k, int64_t n) {
 
 size_t rns_matmul_workspace_bytes(int64_t m, int64_t k, int64_t n) {
     const Plan L = make_plan(m, k, n);
-    return L.a_bytes + L.b_bytes + L.c_bytes;
+    return L.a_bytes + L.b_bytes + L.c_bytes + WS_SLACK;
 }
 
 int rns_matmul(const uint64_t *A, const uint64_t *B, uint64_t *C, int64_t m, int64_t k, int64_t n, void *ws, hipStream_t s) {
     const Plan L = make_plan(m, k, n);
+    ws = align16(ws);
     v4i *Ap = (v4i *)ws, *Bp = (v4i *)((char *)ws + L.a_bytes);
     u32 *Cp = (u32 *)((char *)ws + L.a_bytes + L.b_bytes);
     ModConst K;
