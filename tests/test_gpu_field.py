@@ -184,3 +184,24 @@ def test_device_field_primitives_one_by_one():
         assert run(300 + e, canon, canon) == [(x << e) % P for x in canon], e
     with pytest.raises(RuntimeError):
         _lib.check(L.vi_gl_probe(99, 0, 0, 0, 1, None))
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, (1 << 17) - 1, 1 << 17, (1 << 17) + 1])
+def test_inverses_around_the_switch_to_shared_inversions(cp, n):
+    """One inversion per element up to 2^17 elements, shared ones beyond: zeros, words at and above p, and the result over the
+    input through the C ABI."""
+    from verinf_amd import _lib
+    raw = rand_field((n,), n)
+    raw[::5] = 0
+    raw[n // 2:] = np.where(raw[n // 2:] < 2**32 - 1, raw[n // 2:] + np.uint64(P), raw[n // 2:])      # a few non-canonical words
+    raw[-1] = P
+    raw[n // 3] = (1 << 64) - 1
+    d = to_dev(raw)
+    got = to_np(cp.gl_inv_batched(d))
+    a = raw % np.uint64(P)
+    zero = a == 0
+    assert not got[zero].any() and (got < np.uint64(P)).all()
+    prod = to_np(cp.gl_mul(to_dev(a), to_dev(got)))
+    assert (prod[~zero] == 1).all()
+    _lib.check(_lib.lib().vi_gl_unop(2, d.data_ptr(), 0, d.data_ptr(), n, _lib.stream_ptr()))
+    assert np.array_equal(to_np(d), got)

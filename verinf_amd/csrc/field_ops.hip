@@ -122,10 +122,20 @@ __global__ __launch_bounds__(BLOCK) void k_probe(int op, const u64 *a, const u64
 // accesses stay contiguous, and multiplies them up; the first wavefront does the same with the products of all threads
 // and inverts ONE product per lane (74 multiplications in a chain); the single inverses are peeled off in turn.  A
 // wavefront that inverts costs the same however many of its lanes do, so the chain is paid once per 4096 elements and
-// not once per 512: 35 instead of 98 multiplications per wavefront and 512 elements (1.5 M elements: 21 -> 9 us).
+// not once per 512: 35 instead of 98 multiplications per wavefront and 512 elements (1.5 M elements: 16.9 -> 13.8 us).
 // Zeros are taken out of the product and map to zero, so every output equals the Fermat power a^(p-2) of the reference
 // kernel (prover/cuda_primitives.py:289-303).
 constexpr int INV_E = 8, INV_THREADS = 512;
+
+// Few elements: an inversion each.  A launch lasts as long as one thread's chain while a SIMD has a wavefront or two, and
+// without products before and after it the chain is the shortest (us per call in a queue: 1000 elements 9.5 -> 6.3, 2^16 10.5
+// -> 6.4, 2^17 10.6 -> 7.4, 200000 with a third wavefront 10.6 -> 11.5).
+constexpr i64 INV_FEW = (i64)1 << 17;
+
+__global__ __launch_bounds__(64) void k_inv_each(const u64 *a, u64 *out, i64 n) {
+    const i64 i = (i64)blockIdx.x * 64 + threadIdx.x;
+    if (i < n) out[i] = gl::inv(gl::canon(a[i]));
+}
 
 __global__ __launch_bounds__(INV_THREADS) void k_inv_batched(const u64 *a, u64 *out, i64 n, i64 groups) {
     __shared__ u64 prod[INV_THREADS];
@@ -322,6 +332,11 @@ int vi_gl_unop(int op, const uint64_t *a, uint64_t arg, uint64_t *out, int64_t n
     if (n == 0) return VI_OK;
     if (!a || !out) return vi::fail(VI_EINVAL, "vi_gl_unop: null pointer");
     if (op == 2) {
+        if (n <= INV_FEW) {
+            hipLaunchKernelGGL(k_inv_each, dim3((unsigned)((n + 63) / 64)), dim3(64), 0, (hipStream_t)stream, a, out, (i64)n);
+            VI_LAUNCH_CHECK("k_inv_each");
+            return VI_OK;
+        }
         const i64 groups = (n + INV_E - 1) / INV_E;
         const i64 blocks = (groups + INV_THREADS - 1) / INV_THREADS;
         if (blocks > 0x7FFFFFFF) return vi::fail(VI_EINVAL, "vi_gl_unop: n = %lld", (long long)n);
