@@ -197,9 +197,13 @@ C simt_mfma_i32_32x32x32_i8(const A &a, const A &b, C c) {
 
 typedef void *hipStream_t;
 typedef int hipError_t;
-enum { hipSuccess = 0, hipErrorNotReady = 1, hipFuncAttributeMaxDynamicSharedMemorySize = 0 };
+enum { hipSuccess = 0, hipErrorNotReady = 1, hipFuncAttributeMaxDynamicSharedMemorySize = 0, hipMemcpyHostToDevice = 1 };
 inline hipError_t hipGetLastError() { return hipSuccess; }
 inline const char *hipGetErrorString(hipError_t) { return ""; }
 inline hipError_t hipStreamQuery(hipStream_t) { return hipSuccess; }
 inline hipError_t hipGetDevice(int *d) { *d = 0; return hipSuccess; }
 inline hipError_t hipFuncSetAttribute(const void *, int, int) { return hipSuccess; }
+inline hipError_t hipSetDevice(int) { return hipSuccess; }
+inline hipError_t hipMalloc(void **p, size_t n) { *p = malloc(n); return hipSuccess; }
+inline hipError_t hipFree(void *p) { free(p); return hipSuccess; }
+inline hipError_t hipMemcpy(void *to, const void *from, size_t n, int) { memcpy(to, from, n); return hipSuccess; }

@@ -78,6 +78,108 @@ def lookup(so):
     print("lookup", flush=True)
 
 
+def _ntt_lib(so):
+    L = ctypes.CDLL(so)
+    for name in ("vi_ntt_workspace_bytes", "vi_ntt_best_workspace_bytes"):
+        getattr(L, name).restype, getattr(L, name).argtypes = SZ, [I64, I64]
+    L.vi_ntt_batched.argtypes = [VP, I64, I64, ctypes.c_int, VP, SZ, VP]
+    L.vi_coset_lde_workspace_bytes.restype, L.vi_coset_lde_workspace_bytes.argtypes = SZ, [I64, I64, I64]
+    L.vi_coset_lde_min_workspace_bytes.restype, L.vi_coset_lde_min_workspace_bytes.argtypes = SZ, [I64, I64]
+    L.vi_coset_lde_launches.restype, L.vi_coset_lde_launches.argtypes = I64, [I64, I64, I64, SZ]
+    L.vi_coset_lde.argtypes = [VP, I64, I64, I64, I64, I64, ctypes.c_uint64, VP, I64, VP, SZ, VP]
+    L.vi_coset_lde_coeffs.argtypes = [VP, I64, I64, I64, I64, I64, ctypes.c_uint64, VP, I64, VP, I64, VP, SZ, VP]
+    L.vi_coset_extend.argtypes = [VP, I64, I64, I64, I64, I64, ctypes.c_uint64, VP, I64, VP, SZ, VP]
+    L.simt_launches.restype = ctypes.c_long
+    return L
+
+
+def ntt(so):
+    """Transforms through vi_ntt_batched: every length class, at the batch sizes that take few-row kernels."""
+    L = _ntt_lib(so)
+    row_switch = os.environ.get("VI_NTT_ROW") != "0"
+
+    def run(rows, inverse, ws_bytes=None):
+        m, n = rows.shape
+        ws = scratch(L.vi_ntt_best_workspace_bytes(m, n) if ws_bytes is None else ws_bytes)
+        before = L.simt_launches()
+        rc = L.vi_ntt_batched(ptr(rows), m, n, inverse, ptr(ws) if len(ws) else None, len(ws), None)
+        return rc, L.simt_launches() - before
+
+    for logn, m in [(1, 3), (2, 5), (3, 1), (3, 130), (4, 70), (5, 33), (6, 1), (7, 9), (8, 5), (9, 3), (10, 2), (11, 1), (11, 3), (12, 1), (12, 3), (13, 2),
+                    (14, 1), (15, 1), (16, 1), (17, 1)]:
+        n = 1 << logn
+        raw = field((m, n), logn + m)
+        raw[-1, -2:] = [(1 << 64) - 1, P + 1]
+        want = raw % np.uint64(P)
+        a = raw.copy()
+        rc, launches = run(a, 0)
+        assert rc == 0 and np.array_equal(a, O.ntt_rows(want)), (logn, m)
+        if 3 <= logn <= 11:                                    # the single launch, or the passes the switch asks for
+            assert launches == (1 if row_switch or logn < 10 else 2), (logn, launches)
+        rc, _ = run(a, 1)
+        assert rc == 0 and np.array_equal(a, want), (logn, m)
+        if logn >= 12:                                         # one row of scratch: the rows one after the other
+            a = raw.copy()
+            rc, _ = run(a, 0, 8 * n)
+            assert rc == 0 and np.array_equal(a, O.ntt_rows(want)), (logn, m)
+        # without scratch: rows of up to 2^12 points need none, unless the switch asks for their two passes
+        a = raw.copy()
+        rc, _ = run(a, 0, 0)
+        assert (rc == 0) == (logn <= (12 if row_switch else 9)), (logn, rc)
+        if rc == 0:
+            assert np.array_equal(a, O.ntt_rows(want))
+    print("ntt", flush=True)
+
+
+def lde(so):
+    """Extensions through the three entry points: values, coefficients beside and in place, from coefficients; strided sources of
+    any width, one to 32 cosets, scratch for all rows and for one."""
+    L = _ntt_lib(so)
+
+    def check(logK, log_rho, m, w, shift):
+        K, N = 1 << logK, 1 << (logK + log_rho)
+        stride = w + 3
+        flat = field((m - 1) * stride + w, logK + w)           # the last row ends with its last word
+        src = np.lib.stride_tricks.as_strided(flat, (m, w), (8 * stride, 8))
+        rows = np.ascontiguousarray(src)
+        want = O.coset_lde_rows(rows, K, N, shift)
+        padded = np.zeros((m, K), dtype=np.uint64)
+        padded[:, :w] = rows
+        want_c = O.ntt_rows(padded, inverse=True)
+        for nbytes in (L.vi_coset_lde_workspace_bytes(m, K, N), L.vi_coset_lde_min_workspace_bytes(K, N)):
+            ws = scratch(nbytes)
+            what = (logK, log_rho, m, w, nbytes)
+            out = np.empty((m, N), dtype=np.uint64)
+            before = L.simt_launches()
+            assert L.vi_coset_lde(ptr(flat), m, w, stride, K, N, shift, ptr(out), N, ptr(ws), nbytes, None) == 0
+            assert np.array_equal(out, want), what
+            assert L.simt_launches() - before == L.vi_coset_lde_launches(m, K, N, nbytes), what
+            out = np.empty((m, N), dtype=np.uint64)
+            co = np.empty((m, K), dtype=np.uint64)
+            assert L.vi_coset_lde_coeffs(ptr(flat), m, w, stride, K, N, shift, ptr(co), K, ptr(out), N, ptr(ws), nbytes, None) == 0
+            assert np.array_equal(out, want) and np.array_equal(co, want_c), what
+            co = np.empty((m, K), dtype=np.uint64)
+            assert L.vi_coset_lde_coeffs(ptr(flat), m, w, stride, K, N, shift, ptr(co), K, None, N, ptr(ws), nbytes, None) == 0
+            assert np.array_equal(co, want_c), what
+            out = np.empty((m, N), dtype=np.uint64)
+            assert L.vi_coset_extend(ptr(co), m, K, K, K, N, shift, ptr(out), N, ptr(ws), nbytes, None) == 0
+            assert np.array_equal(out, want), what
+            own, out = padded.copy(), np.empty((m, N), dtype=np.uint64)
+            assert L.vi_coset_lde_coeffs(ptr(own), m, K, K, K, N, shift, ptr(own), K, ptr(out), N, ptr(ws), nbytes, None) == 0
+            assert np.array_equal(out, want) and np.array_equal(own, want_c), what
+
+    for logK in range(1, 13):
+        for log_rho in (0, 1, 2, 3, 5):
+            if logK + log_rho > 14:
+                continue
+            K = 1 << logK
+            check(logK, log_rho, 3 if logK < 10 else 1, [1, K - 1, K][(logK + log_rho) % 3] or 1, 7)
+    for logK, log_rho, m, w in ((3, 1, 300, 5), (6, 2, 70, 64), (10, 3, 2, 600), (11, 3, 1, 2048), (13, 1, 2, 5000), (13, 2, 1, 8192), (14, 0, 1, 100),
+                                (14, 2, 1, 9000)):
+        check(logK, log_rho, m, w, 11)
+    print("lde", flush=True)
+
+
 if __name__ == "__main__":
     globals()[sys.argv[1]](sys.argv[2])
     print("OK")

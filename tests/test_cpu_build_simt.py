@@ -11,13 +11,24 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 DIR = os.path.join(HERE, "cpu_build")
 
 
-@pytest.mark.parametrize("what", ["lookup"])
-def test_kernels_on_the_cpu(what):
-    so = os.path.join(DIR, f"simt_{what}.so")
-    subprocess.check_call(["g++", "-O1", "-g", "-std=c++17", "-fPIC", "-shared", "-fno-extern-tls-init", "-fsanitize=address,undefined",
-                           "-fno-sanitize-recover=undefined", "-I", os.path.join(DIR, "simt"), "-o", so, os.path.join(DIR, f"simt_{what}.cpp")])
+def _build(unit, folder):
+    so = os.path.join(folder, f"simt_{unit}.so")
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-fPIC", "-shared", "-fno-extern-tls-init", "-fsanitize=address,undefined",
+                           "-fno-sanitize-recover=undefined", "-I", os.path.join(DIR, "simt"), "-o", so, os.path.join(DIR, f"simt_{unit}.cpp")])
+    return so
+
+
+@pytest.fixture(scope="module")
+def built(tmp_path_factory):
+    """One build per translation unit, made when a test first asks for it."""
+    made, folder = {}, str(tmp_path_factory.mktemp("simt"))
+    return lambda unit: made[unit] if unit in made else made.setdefault(unit, _build(unit, folder))
+
+
+@pytest.mark.parametrize("unit,what,switches", [("lookup", "lookup", {}), ("ntt", "ntt", {}), ("ntt", "ntt", {"VI_NTT_ROW": "0"}), ("ntt", "lde", {})])
+def test_kernels_on_the_cpu(built, unit, what, switches):
     asan = subprocess.check_output(["g++", "-print-file-name=libasan.so"], text=True).strip()
-    env = dict(os.environ, LD_PRELOAD=asan, ASAN_OPTIONS="detect_leaks=0,verify_asan_link_order=0", OPENBLAS_NUM_THREADS="1")
-    res = subprocess.run([sys.executable, os.path.join(DIR, "simt_checks.py"), what, so], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True,
-                         env=env, timeout=600)
+    env = dict(os.environ, LD_PRELOAD=asan, ASAN_OPTIONS="detect_leaks=0,verify_asan_link_order=0", OPENBLAS_NUM_THREADS="1", **switches)
+    res = subprocess.run([sys.executable, os.path.join(DIR, "simt_checks.py"), what, built(unit)], stdout=subprocess.PIPE, stderr=subprocess.STDOUT,
+                         text=True, env=env, timeout=600)
     assert res.returncode == 0 and res.stdout.strip().endswith("OK"), res.stdout[-4000:]

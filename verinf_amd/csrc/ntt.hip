@@ -443,7 +443,8 @@ int launch_passes(const std::vector<PassArgs> &passes, hipStream_t s) {
     return VI_OK;
 }
 
-// VI_NTT_ROW=0 (read once per process): rows of 2^10 .. 2^12 points as two launches through a workspace, like longer rows
+// VI_NTT_ROW=0 (read once per process): rows of 2^10 .. 2^12 points as two launches through a workspace, like longer rows,
+// whatever the batch
 bool row_launch_on() {
     static const bool on = []() { const char *e = getenv("VI_NTT_ROW"); return !(e && e[0] == '0'); }();
     return on;
@@ -605,7 +606,7 @@ int vi_ntt_batched(uint64_t *rows, int64_t m, int64_t n, int inverse, void *ws, 
         T = T2;
         row = false;
     }
-    if (small_ntt_pays(m, logn)) {
+    if (small_ntt_pays(m, logn) && (row || !row_single_ok(logn))) {
         const u64 scale = inverse ? ntt::inverse((u64)n % gl::P) : 1;
         small_dispatch(logn, [&](auto l) { launch_small_ntt<decltype(l)::value>(rows, m, T->full, scale, inverse != 0, (hipStream_t)stream); });
         VI_LAUNCH_CHECK("k_small_ntt");
