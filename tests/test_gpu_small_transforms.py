@@ -109,12 +109,10 @@ def test_transforms_of_longer_rows(cp, logn):
     assert np.array_equal(to_np(inv), O.ntt_rows(a, inverse=True))
 
 
-@pytest.mark.parametrize("logk", range(10, 19))
-@pytest.mark.parametrize("log_rho", [0, 1, 2, 3, 5])
+# rows of 2^10 and 2^11 with up to four cosets have the single launch
+@pytest.mark.parametrize("logk,log_rho", [(k, r) for r in (0, 1, 2, 3, 5) for k in range(10, 19) if (k > 11 or r >= 3) and k + r <= 21])
 def test_extensions_of_longer_rows(cp, logk, log_rho):
     K, N = 1 << logk, 1 << (logk + log_rho)
-    if logk in (10, 11) and log_rho < 3 or N > 1 << 21:
-        pytest.skip("another kernel's sizes")
     m = max(1, min(3, (1 << 20) // N)) if logk > 11 else (1 << 20) // N + 1
     for w in (K, K // 2 + 3, 1):
         a = rand_field((m, w), 100 * logk + 10 * log_rho + w)

@@ -608,7 +608,10 @@ int vi_ntt_batched(uint64_t *rows, int64_t m, int64_t n, int inverse, void *ws, 
     }
     if (small_ntt_pays(m, logn) && (row || !row_single_ok(logn))) {
         const u64 scale = inverse ? ntt::inverse((u64)n % gl::P) : 1;
-        small_dispatch(logn, [&](auto l) { launch_small_ntt<decltype(l)::value>(rows, m, T->full, scale, inverse != 0, (hipStream_t)stream); });
+        small_dispatch(logn, [&](auto l) {
+            constexpr int LOGN = decltype(l)::value;
+            if constexpr (LOGN < SMALL_MAX_LOG) launch_small_ntt<LOGN>(rows, m, T->full, scale, inverse != 0, (hipStream_t)stream);
+        });
         VI_LAUNCH_CHECK("k_small_ntt");
         return VI_OK;
     }
