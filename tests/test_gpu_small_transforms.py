@@ -137,12 +137,16 @@ def test_extensions_of_longer_rows(cp, logk, log_rho):
         assert torch.equal(held.view(torch.int64), coeffs.view(torch.int64)) and torch.equal(again.view(torch.int64), code.view(torch.int64))
 
 
-@pytest.mark.parametrize("logk,log_rho,log_most", [(12, 1, 19), (13, 2, 21), (14, 2, 22), (16, 1, 20), (16, 2, 21)])
-def test_extensions_on_both_sides_of_the_switch(cp, logk, log_rho, log_most):
+# m rows take one set of launches, m + 1 another
+@pytest.mark.parametrize("logk,log_rho,m", [(6, 2, 8192), (7, 2, 4096), (10, 3, 64), (10, 3, 3559), (11, 1, 4096), (12, 0, 128), (12, 0, 256), (12, 0, 485),
+                                            (12, 1, 64), (12, 1, 128), (12, 2, 502), (13, 2, 151), (14, 2, 65), (16, 1, 8), (16, 2, 8), (18, 2, 11)])
+def test_extensions_on_both_sides_of_the_switch(cp, logk, log_rho, m):
     K, N = 1 << logk, 1 << (logk + log_rho)
-    m = (1 << log_most) // N
     a = to_dev(rand_field((m + 1, K), logk))
-    assert torch.equal(cp.coset_lde(a[:m], K, N).view(torch.int64), cp.coset_lde(a, K, N)[:m].view(torch.int64))
+    few, more = cp.coset_lde(a[:m], K, N).view(torch.int64), cp.coset_lde(a, K, N).view(torch.int64)
+    assert torch.equal(few, more[:m])
+    for row in (0, m - 1):
+        assert np.array_equal(to_np(more[row].view(torch.uint64)), O.coset_lde_rows(to_np(a[row:row + 1]), K, N, 7)[0])
 
 
 _CAPTURE = """

@@ -503,23 +503,35 @@ bool small_ntt_pays(i64 m, int logn) {
     return logn <= 4 || (m << logn) <= ((i64)1 << 20);
 }
 
-// Extensions by the number of cosets and the points written: with two cosets always up to K = 2^7 and at 2^10 (the passes
-// store a column of such a row pair by pair, 2^26 points 2613 against 272 at K = 2^5, 670 against 528 at 2^10), with four up
-// to K = 2^6 and at 2^10; otherwise while the batch leaves SIMDs idle (2^16 points 17 to 50 against 5 to 23; the limits are
-// where the two meet).  More cosets spread a thread's stores over more lines, so the limits fall.
+// Extensions of K < 2^12 in one launch, by log2 of the points written.  While a batch leaves SIMDs idle the single launch is the
+// shorter chain (2^16 points 16 to 36 against 5 to 16): up to 2^21, or 2^19 from eight cosets on (2^22 at K <= 2^4), as its
+// stores are single words rho apart.  Beyond that it stays ahead where the passes are slow themselves (us for 2^26 points):
+// below 32 points they have no register kernel (K = 2^3, two cosets 709 against 266); short rows they store a column at a time,
+// rho words in a piece (one or two cosets up to K = 2^7: 1356 and 289 at 2^5, 506 and 409 at 2^7; four at 2^6: 312 and 471);
+// and at K = 2^10 they go twice through memory in each direction (four cosets 580 and 513).  At K = 2^11, and at 2^5 with four
+// cosets, the two meet at 2^24 points.
 bool small_lde_pays(i64 m, int logK, int logN, bool in_place) {
-    if (logK < SMALL_MIN_LOG || logK > SMALL_MAX_LOG) return false;
+    if (logK < SMALL_MIN_LOG || logK >= SMALL_MAX_LOG) return false;
     const int log_rho = logN - logK;
     if (log_rho > 8) return false;
     int log_most;
-    if (log_rho <= 1) log_most = logK <= 7 || logK == 10 ? 62 : (logK == 11 ? 24 : 21);
-    else if (log_rho == 2) log_most = logK <= 6 || logK == 10 ? 62 : (logK <= 9 ? 21 : (logK == 11 ? 23 : 22));
-    else {
+    if (log_rho <= 2) {
+        const int short_rows = log_rho <= 1 ? 7 : 4;
+        log_most = logK <= short_rows || logK == 10 ? 62 : (logK == 11 || logK == 5 ? 24 : 21);
+    } else {
         // in place one workgroup has to run through the cosets of its rows: eight or more of them are the longer chain
         if (in_place && logK > 4) return false;
         log_most = logK <= 4 ? 22 : 19;
     }
     return m <= (((i64)1 << log_most) >> logN);
+}
+
+// A row of 2^12 fills a CU, so the single launch takes 23 us per round of 256 workgroups (34 with two cosets in each): ahead of
+// both kinds of passes only when there is one round, and that about full (2^20 points written, one coset: 24, passes 32 and
+// 33; two: 27, 39 and 29; half of it 24 against 22 in passes).
+bool single_round_of_rows(i64 m, int log_rho, bool in_place) {
+    const i64 workgroups = in_place || m >= 256 ? m : m << log_rho;
+    return log_rho <= 1 && workgroups > 128 && workgroups <= 256;
 }
 
 // Where the passes of ntt_small.hpp are the faster ones for rows of several passes (us per call, the passes of k_ntt_fast, or
@@ -539,24 +551,42 @@ bool small_ntt_passes_pay(i64 m, int logn, const Split &sp) {
     return m <= (((i64)1 << log_most) >> logn);
 }
 
-// Extensions, by log2 of the points written, for K = 2^10 .. 2^18 and 1, 2, 4, 8 or more cosets: where the two meet in a sweep
-// over both (rows of 2^13 to 2^16, few of them: 33 to 58 against 16 to 20 at four cosets, up to 154 against 34 at sixteen, where
-// k_ntt_fast takes the cosets one after the other).  Rows of 2^10 and 2^11 with fewer cosets have the single launch.
+// Extensions of K = 2^10 .. 2^18 in passes: the time of either kind in us, and the shorter one is taken.  `million`: points that
+// go through each pass, in millions (m K on the way to the coefficients, m N on the way back).
+//
+// k_small_pass: 3.7 us a launch and so many us per million points, more for long digits, of which a workgroup holds fewer
+// columns (digits of 2^5 .. 2^8: 32 .. 4, runs of 256 .. 32 bytes).
+//
+// k_ntt_fast: 7.8 us a launch, one wavefront's chain, and 2.95 per million.  With K = L L the middle two are one launch whose
+// workgroups go through the cosets one after the other: 21 + 7 per coset for all three, and 1.84 per million (memory hides
+// behind the chain).
+//
+// Fitted to a sweep over K, 1 to 32 cosets and batches of 1 .. 2^24 points written, where the choice loses 0.2 % on average and
+// 16 % at most (k_small_pass, k_ntt_fast: 2^14 -> 2^16 one row 18, 53; 64 rows 63, 69; 256 rows 209, 141; 1 x 2^16 -> 2^21 48,
+// 309).
+double small_passes_us(const Split &sp, double million) {
+    static constexpr double per_million[4] = {3.2, 3.5, 5.05, 7.7};
+    double us = 0;
+    for (int q = 0; q < sp.p; ++q) us += 2 * 3.7 + per_million[sp.a[q] - 5] * million;
+    return us;
+}
+double fast_passes_us(const Split &sp, int log_rho, double million) {
+    if (sp.p == 2 && sp.a[0] == sp.a[1] && sp.a[0] >= 6) return 21 + 7.0 * (double)(1 << log_rho) + 2 * 1.84 * million;
+    return sp.p * (2 * 7.8 + 2.95 * million);
+}
 bool small_lde_passes_pay(i64 m, int logK, int logN, const Split &sp) {
-    static constexpr int log_most[9][4] = {{0, 0, 0, 24},    {0, 0, 0, 24},    {19, 19, 22, 23}, {19, 21, 21, 22}, {19, 21, 22, 23},
-                                           {19, 20, 20, 21}, {19, 20, 21, 22}, {23, 23, 23, 23}, {21, 21, 21, 23}};
-    if (logK < 10 || logK > 18 || !small_digits(sp)) return false;
     const int log_rho = logN - logK;
-    return m <= (((i64)1 << log_most[logK - 10][log_rho < 3 ? log_rho : 3]) >> logN);
+    if (logK < 10 || logK > 18 || log_rho > 15 || !small_digits(sp)) return false;      // cosets: the grid's second dimension
+    const double million = (double)m * (double)(((i64)1 << logK) + ((i64)1 << logN)) * 1e-6;
+    return small_passes_us(sp, million) < fast_passes_us(sp, log_rho, million);
 }
 
 // Which launches an extension takes
 enum LdeRoute { LDE_PASSES, LDE_SINGLE, LDE_SMALL_PASSES };
 LdeRoute lde_route(i64 m, int logK, int logN, bool in_place, const Split &sp) {
-    const bool passes = small_lde_passes_pay(m, logK, logN, sp);
-    // a row of 2^12 fills a CU: 22.6 us in one launch, 14.8 in four
-    if (!(passes && logK == 12) && small_lde_pays(m, logK, logN, in_place)) return LDE_SINGLE;
-    return passes ? LDE_SMALL_PASSES : LDE_PASSES;
+    if (small_lde_pays(m, logK, logN, in_place)) return LDE_SINGLE;
+    if (logK == SMALL_MAX_LOG && single_round_of_rows(m, logN - logK, in_place)) return LDE_SINGLE;
+    return small_lde_passes_pay(m, logK, logN, sp) ? LDE_SMALL_PASSES : LDE_PASSES;
 }
 
 // full[inverse]: w_4096^j of either direction
