@@ -120,7 +120,7 @@ inline void launch(dim3 grid, dim3 block, const std::function<void()> &f) {
 }
 
 inline int any_true;
-inline int32_t wave_a[64][4], wave_b[64][4];                          // operands of a matrix instruction, by lane
+inline int32_t wave_a[16][64][4], wave_b[16][64][4];                  // operands of a matrix instruction, by wavefront and lane
 
 }  // namespace simt
 
@@ -176,24 +176,25 @@ inline uint32_t __builtin_amdgcn_perm(uint32_t a, uint32_t b, uint32_t sel) {
 // 32 x 32 x 32 on signed bytes: lane l holds row (column) l % 32 of A (B), the sixteen inner indices from 16 (l / 32); register r of
 // the result is row 8 (r / 4) + 4 (l / 32) + r % 4 of column l % 32
 template <class A, class C>
-C simt_mfma_i32_32x32x32_i8(const A &a, const A &b, C c) {
-    const int lane = threadIdx.x & 63;
+void simt_mfma_i32_32x32x32_i8(const A &a, const A &b, C &c) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     for (int i = 0; i < 4; ++i) {
-        simt::wave_a[lane][i] = a[i];
-        simt::wave_b[lane][i] = b[i];
+        simt::wave_a[wave][lane][i] = a[i];
+        simt::wave_b[wave][lane][i] = b[i];
     }
     __builtin_amdgcn_wave_barrier();
     for (int r = 0; r < 16; ++r) {
         const int row = 8 * (r / 4) + 4 * (lane / 32) + r % 4, col = lane % 32;
         int sum = 0;
         for (int half = 0; half < 2; ++half)
-            for (int i = 0; i < 4; ++i) sum = __builtin_amdgcn_sdot4(simt::wave_a[row + 32 * half][i], simt::wave_b[col + 32 * half][i], sum, false);
+            for (int i = 0; i < 4; ++i)
+                sum = __builtin_amdgcn_sdot4(simt::wave_a[wave][row + 32 * half][i], simt::wave_b[wave][col + 32 * half][i], sum, false);
         c[r] += sum;
     }
     __builtin_amdgcn_wave_barrier();
-    return c;
 }
-#define __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, x, y, z) simt_mfma_i32_32x32x32_i8(a, b, c)
+// the accumulator is updated where it lies, as the kernels do
+#define __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, x, y, z) (simt_mfma_i32_32x32x32_i8(a, b, c), c)
 
 typedef void *hipStream_t;
 typedef int hipError_t;

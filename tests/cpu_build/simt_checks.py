@@ -180,6 +180,38 @@ def lde(so):
     print("lde", flush=True)
 
 
+def matmul(so):
+    """Products through residues: every tile shape with remainders, one unit of the inner dimension and several, the largest sums of
+    either sign, words at and above p, slices of the inner dimension."""
+    L = ctypes.CDLL(so)
+    L.simt_matmul_workspace.restype, L.simt_matmul_workspace.argtypes = SZ, [I64] * 3
+    L.simt_matmul.argtypes = [VP, VP, VP, I64, I64, I64, VP]
+    L.simt_tile_workspace.restype, L.simt_tile_workspace.argtypes = SZ, [I64, ctypes.c_int]
+    L.simt_tile.restype, L.simt_tile.argtypes = None, [VP, VP, VP, I64, I64, I64, ctypes.c_int, VP]
+    for m, k, n, fill in ((1, 1, 1, None), (3, 17, 70, "any"), (64, 64, 64, "top"), (65, 100, 65, "half"), (130, 33, 130, None), (5, 8193, 3, "top"),
+                          (120, 70, 250, 4), (128, 64, 256, 4), (128, 130, 128, 2), (67, 5, 100, 2)):
+        print("matmul", m, k, n, fill, flush=True)
+        A, B = field((m, k), m), field((k, n), n)
+        if fill == "top":
+            A[:], B[:] = P - 1, P - 1
+        elif fill == "half":                                   # the words of largest size as signed numbers
+            A[:], B[:] = 0x8080808080808080, 0x7F7F7F7F7F7F7F7F
+            B[::2] += np.uint64(1)
+        elif fill == "any":
+            A[:, ::3] = np.uint64((1 << 64) - 1) - A[:, ::3] % np.uint64(1 << 20)
+            B[::2] = np.uint64((1 << 64) - 1) - B[::2] % np.uint64(1 << 33)
+        C = np.empty((m, n), dtype=np.uint64)
+        if fill in (2, 4):                                     # one tile of 128 x 64 fill
+            ws = scratch(L.simt_tile_workspace(k, fill))
+            L.simt_tile(ptr(A), ptr(B), ptr(C), m, k, n, fill, ptr(ws))
+        else:
+            ws = scratch(L.simt_matmul_workspace(m, k, n))
+            assert L.simt_matmul(ptr(A), ptr(B), ptr(C), m, k, n, ptr(ws)) == 0
+        rows = sorted({0, m // 2, m - 1})
+        want = (A[rows].astype(object).dot(B.astype(object)) % P).astype(np.uint64)
+        assert np.array_equal(C[rows], want), (m, k, n, fill)
+
+
 if __name__ == "__main__":
     globals()[sys.argv[1]](sys.argv[2])
     print("OK")
