@@ -103,7 +103,14 @@ inline void run_group(unsigned n) {
     }
 }
 
+inline std::function<void()> before_launch;                           // once, in front of the next launch: another thread's call
+
 inline void launch(dim3 grid, dim3 block, const std::function<void()> &f) {
+    if (before_launch) {
+        const std::function<void()> other = std::move(before_launch);
+        before_launch = nullptr;
+        other();
+    }
     if (block.x * block.y > 1024 || grid.x == 0 || grid.y == 0 || grid.x > 0x7FFFFFFFu || grid.y > 65535) {
         fprintf(stderr, "launch outside the limits\n");
         abort();

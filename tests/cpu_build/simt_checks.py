@@ -212,6 +212,18 @@ def matmul(so):
         assert np.array_equal(C[rows], want), (m, k, n, fill)
 
 
+def tables(so):
+    """The tables of a call stay until its launches are queued, whatever other threads' calls evict in between."""
+    L = _ntt_lib(so)
+    for K, N in ((64, 128), (1 << 13, 1 << 14)):               # the single launch, and passes
+        a, out = field((2, K), 1), np.empty((2, N), dtype=np.uint64)
+        ws = scratch(L.vi_coset_lde_workspace_bytes(2, K, N))
+        L.simt_other_shifts(40)
+        assert L.vi_coset_lde(ptr(a), 2, K, K, K, N, 7, ptr(out), N, ptr(ws), len(ws), None) == 0
+        assert np.array_equal(out, O.coset_lde_rows(a, K, N, 7))
+    print("tables", flush=True)
+
+
 if __name__ == "__main__":
     globals()[sys.argv[1]](sys.argv[2])
     print("OK")

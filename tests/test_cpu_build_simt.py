@@ -25,7 +25,7 @@ def built(tmp_path_factory):
     return lambda unit: made[unit] if unit in made else made.setdefault(unit, _build(unit, folder))
 
 
-@pytest.mark.parametrize("unit,what,switches", [("lookup", "lookup", {}), ("ntt", "ntt", {}), ("ntt", "ntt", {"VI_NTT_ROW": "0"}), ("ntt", "lde", {}),
+@pytest.mark.parametrize("unit,what,switches", [("lookup", "lookup", {}), ("ntt", "ntt", {}), ("ntt", "ntt", {"VI_NTT_ROW": "0"}), ("ntt", "lde", {}), ("ntt", "tables", {}),
                                                 ("matmul", "matmul", {})])
 def test_kernels_on_the_cpu(built, unit, what, switches):
     asan = subprocess.check_output(["g++", "-print-file-name=libasan.so"], text=True).strip()

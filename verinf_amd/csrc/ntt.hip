@@ -237,7 +237,12 @@ struct DeviceTables {
 std::mutex g_mu;
 std::map<std::tuple<int, int, int>, DeviceTables *> g_tables;        // (device, logn, inverse + 2 * row split)
 std::map<std::pair<int, int>, u64 *> g_twl;                          // (device, inverse + 2 * all 4096 powers)
-std::map<std::tuple<int, int, int, u64>, u64 *> g_pre;               // (device, logK, logN, shift)
+struct CosetTable {
+    u64 *words = nullptr;
+    u64 used = 0;                              // time of last use
+    int calls = 0;                             // calls between their look-up and their last launch
+};
+std::map<std::tuple<int, int, int, u64>, CosetTable> g_pre;          // (device, logK, logN, shift)
 
 int upload(const std::vector<u64> &h, u64 **out) {
     void *d = nullptr;
@@ -314,40 +319,57 @@ int get_tables(int logn, int inv, const Tables **out, bool row = false) {
 
 // Coset multiplier tables are N words each and depend on the shift: the most recently used MAX_PRE per process are
 // kept, the least recently used one is freed when a new one is needed (hipFree waits for the kernels that may still
-// read it).
+// read it; a table whose kernels are not all queued yet is left alone, beyond MAX_PRE if need be).
 constexpr size_t MAX_PRE = 16;
 u64 g_pre_clock = 0;
-std::map<std::tuple<int, int, int, u64>, u64> g_pre_used;            // key -> time of last use
 
-int get_pre(int logK, int logN, u64 shift, const u64 **out) {
+// Holds a table while a call queues the launches that read it.
+struct CosetPin {
+    CosetTable *table = nullptr;
+    CosetPin() = default;
+    CosetPin(const CosetPin &) = delete;
+    CosetPin &operator=(const CosetPin &) = delete;
+    ~CosetPin() {
+        if (!table) return;
+        std::lock_guard<std::mutex> lock(g_mu);
+        --table->calls;
+    }
+};
+
+int free_oldest_pre(int dev) {
+    auto victim = g_pre.end();
+    for (auto it = g_pre.begin(); it != g_pre.end(); ++it)
+        if (it->second.calls == 0 && (victim == g_pre.end() || it->second.used < victim->second.used)) victim = it;
+    if (victim == g_pre.end()) return VI_OK;
+    const int vdev = std::get<0>(victim->first);
+    if (vdev != dev) VI_HIP(hipSetDevice(vdev));
+    const hipError_t e = hipFree(victim->second.words);
+    if (vdev != dev) VI_HIP(hipSetDevice(dev));
+    if (e != hipSuccess) return vi::fail(VI_EHIP, "hipFree of a coset table: %s", hipGetErrorString(e));
+    g_pre.erase(victim);
+    return VI_OK;
+}
+
+int get_pre(int logK, int logN, u64 shift, const u64 **out, CosetPin &pin) {
     int dev = 0;
     VI_HIP(hipGetDevice(&dev));
     std::lock_guard<std::mutex> lock(g_mu);
     auto key = std::make_tuple(dev, logK, logN, shift);
     auto it = g_pre.find(key);
     if (it == g_pre.end()) {
-        if (g_pre.size() >= MAX_PRE) {
-            auto oldest = g_pre_used.begin();
-            for (auto u = g_pre_used.begin(); u != g_pre_used.end(); ++u)
-                if (u->second < oldest->second) oldest = u;
-            auto victim = g_pre.find(oldest->first);
-            int vdev = std::get<0>(victim->first);
-            if (vdev != dev) VI_HIP(hipSetDevice(vdev));
-            hipError_t e = hipFree(victim->second);
-            if (vdev != dev) VI_HIP(hipSetDevice(dev));
-            if (e != hipSuccess) return vi::fail(VI_EHIP, "hipFree of a coset table: %s", hipGetErrorString(e));
-            g_pre.erase(victim);
-            g_pre_used.erase(oldest);
-        }
-        u64 *d = nullptr;
+        for (size_t over = g_pre.size(); over >= MAX_PRE; --over)
+            if (int rc = free_oldest_pre(dev)) return rc;
+        CosetTable T;
         std::vector<u64> h = make_coset_pre(logK, logN, shift);
         if (coset_mergeable(logK, logN)) append_coset_merged(logK, logN, h);
-        int rc = upload(h, &d);
+        int rc = upload(h, &T.words);
         if (rc) return rc;
-        it = g_pre.emplace(key, d).first;
+        it = g_pre.emplace(key, T).first;
     }
-    g_pre_used[key] = ++g_pre_clock;
-    *out = it->second;
+    it->second.used = ++g_pre_clock;
+    ++it->second.calls;
+    pin.table = &it->second;                   // nodes of a map stay where they are
+    *out = it->second.words;
     return VI_OK;
 }
 
@@ -770,9 +792,10 @@ int coset_lde_impl(const char *who, const uint64_t *in, int64_t m, int64_t width
     chunk = (m + ((m + chunk - 1) / chunk) - 1) / ((m + chunk - 1) / chunk);   // same chunk count, even sizes
     const Tables *Ti = nullptr, *Tf = nullptr;
     const u64 *pre = nullptr;
+    CosetPin pin;
     int rc = get_tables(logK, 1, &Ti);
     if (!rc) rc = get_tables(logK, 0, &Tf);
-    if (!rc) rc = get_pre(logK, logN, shift, &pre);
+    if (!rc) rc = get_pre(logK, logN, shift, &pre, pin);
     if (rc) return rc;
     const LdeRoute route = lde_route(m, logK, logN, coeffs == in, Ti->sp);
     if (route == LDE_SINGLE) {
