@@ -9,7 +9,7 @@
 // half full) of entry -> first index that holds it, and a look-up then costs a probe or two where the search from the
 // front costs half the table.  Which of the two a table is, is looked at in every call, on the device: up to 4096 entries
 // by every workgroup for itself (k_count_small: table and hash in LDS), beyond by a launch over the table (k_survey), whose
-// findings the later launches read.  us per call in a queue of them, 1.5 M look-ups: 9.7 in 2^6 entries, 12.0 in 2^12, 23.8
+// findings the later launches read.  us per call in a queue of them, 1.5 M look-ups: 9.7 in 2^6 entries, 12.0 in 2^12, 23.0
 // in 2^16, 55 in 2^20 (19.0 and 48 for the last two when the caller promises a range); 10^6 look-ups in 3003 values 12.6.
 #include "common.hpp"
 #include "gl_field.hpp"
@@ -43,7 +43,7 @@ struct Finder {
 
 // Workgroup w looks at its share of the table and notes in odd[w] whether table[j] == j throughout, empties its share of the
 // slots and, when the counts are not added to what is there, zeroes its share of them.  It and the launch of k_insert that
-// finds nothing to do cost a call over a range 3 us at 2^13 entries, 5 at 2^16 and 7 at 2^20 (8 bytes read and 8 to 24 written
+// finds nothing to do cost a call over a range 4 us at 2^13 entries and 2^16 and 7 at 2^20 (8 bytes read and 8 to 24 written
 // per entry).
 __global__ __launch_bounds__(COUNT_THREADS) void k_survey(const Finder F, u32 *odd, u64 *clear) {
     const i64 first = (i64)blockIdx.x * COUNT_THREADS + threadIdx.x, stride = (i64)gridDim.x * COUNT_THREADS;
@@ -58,10 +58,10 @@ __global__ __launch_bounds__(COUNT_THREADS) void k_survey(const Finder F, u32 *o
     if (threadIdx.x == 0) odd[blockIdx.x] = differs ? 1 : 0;
 }
 
-// the survey's result, the same for every thread of a workgroup (which all call this)
-__device__ __forceinline__ bool is_range(const Finder &F) {
-    return !__syncthreads_or((int)threadIdx.x < F.n_odd && F.odd[threadIdx.x] != 0);
-}
+// the survey's result: a thread's part of it, which may be asked for early, and the whole, the same for every thread of a
+// workgroup (which all call this)
+__device__ __forceinline__ u32 odd_part(const Finder &F) { return (int)threadIdx.x < F.n_odd ? F.odd[threadIdx.x] : 0; }
+__device__ __forceinline__ bool is_range(u32 part) { return !__syncthreads_or((int)part); }
 
 // A slot belongs to the first index that claims it; later indices of the same entry lower it to the smallest.  The entry
 // of a claimed slot is read from the table (every index it ever holds has the same one).  Ends after at most 2^bits
@@ -84,7 +84,7 @@ __device__ __forceinline__ void insert(const u64 *table, u32 j, u64 key, u64 *ke
 
 // nothing to do for a range
 __global__ __launch_bounds__(BLOCK) void k_insert(const Finder F) {
-    if (is_range(F)) return;
+    if (is_range(odd_part(F))) return;
     const i64 stride = (i64)gridDim.x * BLOCK;
     for (i64 j = (i64)blockIdx.x * BLOCK + threadIdx.x; j < F.n_table; j += stride)
         insert(F.table, (u32)j, F.table[j], F.keys, F.index, F.bits);
@@ -165,9 +165,10 @@ __global__ __launch_bounds__(COUNT_THREADS) void k_count(const u64 *__restrict__
     u32 *counts = reinterpret_cast<u32 *>(lds_counts);
     const i64 base = (i64)blockIdx.x * SLICE, group = blockIdx.y;
     const int mine = F.n_table - base < SLICE ? (int)(F.n_table - base) : SLICE;
+    const u32 part = odd_part(F);
     // the launch's LDS is a whole number of 16-byte words
     for (int i = threadIdx.x; i < (mine * copies + 3) / 4; i += COUNT_THREADS) lds_counts[i] = make_uint4(0, 0, 0, 0);
-    const bool range = is_range(F);            // a barrier as well
+    const bool range = is_range(part);         // a barrier as well
     const i64 lo = group * per_group, hi = lo + per_group < n_x ? lo + per_group : n_x;
     if (range) count(x, lo, hi, (u64)base, mine, copies, counts, [&](u64 v) { return index_of<true>(v, F); });
     else count(x, lo, hi, (u64)base, mine, copies, counts, [&](u64 v) { return index_of<false>(v, F); });
@@ -244,7 +245,7 @@ __global__ __launch_bounds__(BLOCK) void k_add_rows(const u32 *__restrict__ rows
 // one global atomic per look-up
 __global__ __launch_bounds__(BLOCK) void k_count_global(const u64 *__restrict__ x, i64 n_x, const Finder F, unsigned long long *__restrict__ mult) {
     const i64 stride = (i64)gridDim.x * BLOCK, first = (i64)blockIdx.x * BLOCK + threadIdx.x;
-    if (is_range(F)) {
+    if (is_range(odd_part(F))) {
         for (i64 i = first; i < n_x; i += stride) {
             const u64 at = index_of<true>(x[i], F);
             if (at < (u64)F.n_table) atomicAdd(&mult[at], 1ULL);
@@ -303,7 +304,7 @@ Plan make_plan(i64 n_x, i64 n_table, bool promised) {
             while (((i64)1 << L.bits) < 2 * n_table) ++L.bits;
         }
         if (!L.small) {
-            const i64 shares = (n_table + 4 * COUNT_THREADS - 1) / (4 * COUNT_THREADS);
+            const i64 shares = (n_table + COUNT_THREADS - 1) / COUNT_THREADS;
             L.surveyors = (int)(shares < SURVEYORS ? shares : SURVEYORS);
             if (L.bits) {
                 L.key_bytes = sizeof(u64) << L.bits;

@@ -739,7 +739,7 @@ def lookup_multiplicities_into(x, table, mult, label=""):
 def _histogram(x, table, mult, accumulate):
     # whether the table is a range is looked at on the device, in every call: nothing is kept of a table
     L = _lib.lib()
-    n_x, n_t = int(x.numel()), int(table.numel())
+    n_x, n_t = x.numel(), table.numel()
     need = L.vi_lookup_histogram_workspace_bytes(n_x, n_t, 0)
     args = (x.data_ptr(), n_x, table.data_ptr(), n_t, 0, accumulate, mult.data_ptr())
     with _lib.on_device(x.device):
@@ -759,7 +759,7 @@ def lookup_multiplicities(x, table):
     if x.dim() != 1 or table.dim() != 1:
         raise RuntimeError("x and table must be 1-D")
     if x.numel() == 0 or table.numel() == 0:
-        return torch.zeros(int(table.numel()), dtype=torch.int64, device=table.device).view(torch.uint64)
+        return torch.zeros(table.numel(), dtype=torch.int64, device=table.device).view(torch.uint64)
     mult = torch.empty_like(table)
     _histogram(x, table, mult, 0)
     return mult
