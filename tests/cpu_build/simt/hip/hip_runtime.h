@@ -28,6 +28,7 @@ struct dim3 {
     unsigned x, y, z;
     dim3(unsigned x_ = 1, unsigned y_ = 1, unsigned z_ = 1) : x(x_), y(y_), z(z_) {}
 };
+struct alignas(16) ulonglong2 { unsigned long long x, y; };
 struct alignas(16) uint4 { uint32_t x, y, z, w; };
 inline uint4 make_uint4(uint32_t x, uint32_t y, uint32_t z, uint32_t w) { return uint4{x, y, z, w}; }
 
@@ -147,14 +148,16 @@ inline void __threadfence_system() {}
 #define __builtin_amdgcn_fence(...) ((void)0)
 #define __builtin_amdgcn_wave_barrier() simt::wait_at(simt::AT_WAVE)
 #define __builtin_nontemporal_load(p) (*(p))
+#define __hip_atomic_load(p, order, scope) (*(p))
+#define __hip_atomic_store(p, v, order, scope) (*(p) = (v))
 #define __builtin_nontemporal_store(v, p) (*(p) = (v))
 
 template <class T, class V>
 T atomicAdd(T *p, V v) { T was = *p; *p += (T)v; return was; }
-template <class T>
-T atomicMin(T *p, T v) { T was = *p; if (v < was) *p = v; return was; }
-template <class T>
-T atomicCAS(T *p, T expect, T v) { T was = *p; if (was == expect) *p = v; return was; }
+template <class T, class V>
+T atomicMin(T *p, V v) { T was = *p; if ((T)v < was) *p = (T)v; return was; }
+template <class T, class E, class V>
+T atomicCAS(T *p, E expect, V v) { T was = *p; if (was == (T)expect) *p = (T)v; return was; }
 
 inline uint32_t __brev(uint32_t v) {
     uint32_t r = 0;
@@ -209,6 +212,8 @@ enum { hipSuccess = 0, hipErrorNotReady = 1, hipFuncAttributeMaxDynamicSharedMem
 inline hipError_t hipGetLastError() { return hipSuccess; }
 inline const char *hipGetErrorString(hipError_t) { return ""; }
 inline hipError_t hipStreamQuery(hipStream_t) { return hipSuccess; }
+enum hipStreamCaptureStatus { hipStreamCaptureStatusNone = 0 };
+inline hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus *s) { *s = hipStreamCaptureStatusNone; return hipSuccess; }
 inline hipError_t hipGetDevice(int *d) { *d = 0; return hipSuccess; }
 inline hipError_t hipFuncSetAttribute(const void *, int, int) { return hipSuccess; }
 inline hipError_t hipSetDevice(int) { return hipSuccess; }

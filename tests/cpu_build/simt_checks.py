@@ -38,12 +38,34 @@ def lookup(so):
     L.vi_lookup_histogram.argtypes = [VP, I64, VP, I64, ctypes.c_int, ctypes.c_int, VP, VP, SZ, VP]
     L.vi_lookup_multiplicities.argtypes = [VP, I64, VP, I64, ctypes.c_int, VP, VP]
 
-    def check(x, table, promised=0):
-        n_x, n_t = len(x), len(table)
+    def counts(x, table):
         keys, first = np.unique(table, return_index=True)
         at = np.minimum(np.searchsorted(keys, x), len(keys) - 1)
-        hit = keys[at] == x if n_x else np.zeros(0, bool)
-        want = np.bincount(first[at[hit]], minlength=n_t).astype(np.uint64)
+        hit = keys[at] == x if len(x) else np.zeros(0, bool)
+        return np.bincount(first[at[hit]], minlength=len(table)).astype(np.uint64)
+
+    # the first call of the library, whose tag is 1: scratch that holds slots of that very tag, naming any index or none
+    rng = np.random.default_rng(0)
+    n_t = 5000
+    table = field(n_t, 1)
+    table[::4] = np.arange(0, n_t, 4)                          # some entries are their own index
+    table[1::4] = table[rng.integers(0, n_t, len(table[1::4]))]
+    x = np.concatenate([table[rng.integers(0, n_t, 9001)], np.arange(0, 600, dtype=np.uint64)])
+    ws = scratch(L.vi_lookup_histogram_workspace_bytes(len(x), n_t, 0))
+    slots = ws[(-ws.ctypes.data) % 16:][:8 << 14].view(np.uint64)
+    taken = rng.random(len(slots)) < 0.4
+    slots[taken] = (np.uint64(1 << 30) | rng.integers(0, 2 * n_t, len(slots)).astype(np.uint64))[taken]
+    mult = np.empty(n_t, dtype=np.uint64)
+    assert L.vi_lookup_histogram(ptr(x), len(x), ptr(table), n_t, 0, 0, ptr(mult), ptr(ws), len(ws), None) == 0
+    assert np.array_equal(mult, counts(x, table))
+    for seed in (2, 3):                                        # the same scratch again, with slots of the calls before
+        table = np.random.default_rng(seed).permutation(table)
+        assert L.vi_lookup_histogram(ptr(x), len(x), ptr(table), n_t, 0, 0, ptr(mult), ptr(ws), len(ws), None) == 0
+        assert np.array_equal(mult, counts(x, table))
+
+    def check(x, table, promised=0):
+        n_x, n_t = len(x), len(table)
+        want = counts(x, table)
         need = L.vi_lookup_histogram_workspace_bytes(n_x, n_t, promised)
         for accumulate, before in ((1, 7), (0, 12345)):
             mult, ws = np.full(n_t, before, dtype=np.uint64), scratch(need)
@@ -63,11 +85,11 @@ def lookup(so):
         x[-1:] = (1 << 64) - 1
         check(x, span)
         check(x, span, promised=1)
-        if n_x > 100000:                                       # long runs, less often
-            continue
         odd = span.copy()                                      # all but a range: the last entry, then the first
         odd[-1] = n_t + 1
         check(x, odd)
+        if n_t > 4097:                                         # long runs, less often
+            continue
         odd[0] = 5 % n_t
         check(x, odd)
         table = field(n_t, n_x)

@@ -58,6 +58,17 @@ inline int wait_for_tag(const char *who, const volatile uint64_t *flag, uint64_t
     return VI_OK;
 }
 
+// whether the stream is being captured; the default stream cannot be, and may not be asked while another one is
+inline int capturing(hipStream_t s, bool *is) {
+    *is = false;
+    if (!s) return VI_OK;
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    const hipError_t e = hipStreamIsCapturing(s, &status);
+    if (e != hipSuccess) return fail(VI_EHIP, "hipStreamIsCapturing: %s", hipGetErrorString(e));
+    *is = status != hipStreamCaptureStatusNone;
+    return VI_OK;
+}
+
 // a tag no earlier call has used, so that nothing such a call may have left in flight can pass for this one's result
 inline uint64_t new_tag() {
     static std::atomic<uint64_t> calls{0};

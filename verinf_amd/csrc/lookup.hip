@@ -5,12 +5,13 @@
 // slice of up to 32768 entries, leaves its counts as one row of a workspace, and a second launch adds up the rows.  Small
 // tables are kept several times over, one copy per group of lanes, so that look-ups of one entry do not queue up.
 //
-// A table that is literally 0 .. T-1 is indexed; any other one is first turned into a hash table (linear probing, at most
-// half full) of entry -> first index that holds it, and a look-up then costs a probe or two where the search from the
-// front costs half the table.  Which of the two a table is, is looked at in every call, on the device: up to 4096 entries
-// by every workgroup for itself (k_count_small: table and hash in LDS), beyond by a launch over the table (k_survey), whose
-// findings the later launches read.  us per call in a queue of them, 1.5 M look-ups: 9.7 in 2^6 entries, 12.0 in 2^12, 23.0
-// in 2^16, 55 in 2^20 (19.0 and 48 for the last two when the caller promises a range); 10^6 look-ups in 3003 values 12.6.
+// A table that is literally 0 .. T-1 is indexed; of any other one the entries that are not their own index go into a hash
+// table (linear probing, at most half full) of entry -> first index that holds it, and a look-up costs a probe or two where
+// the search from the front costs half the table.  Which of the two a table is, is looked at in every call, on the device: up
+// to 4096 entries by every workgroup for itself (k_count_small: table and hash in LDS), beyond by a launch over the table
+// (k_survey), whose findings the counting workgroups read.  us per call in a queue of them, 1.5 M look-ups: 10 in 2^6 entries,
+// 12.0 in 2^12, 21.4 in 2^16, 52 in 2^20 (19.0 and 48 for the last two when the caller promises a range); 10^6 look-ups in 3003
+// values 12.6, in 40000 36.
 #include "common.hpp"
 #include "gl_field.hpp"
 
@@ -23,6 +24,7 @@ constexpr int MAX_COPIES = 32;
 constexpr i64 MAX_GROUPS = 256;                // rows of the workspace per slice
 constexpr u32 EMPTY = 0xFFFFFFFFu;
 constexpr i64 MAX_HASHED = (i64)1 << 30;       // entries of a hash table
+constexpr u64 INDEX_BITS = MAX_HASHED - 1;
 constexpr int SMALL_TABLE = 4096;              // entries of a table that every workgroup takes into its LDS
 constexpr int SMALL_COUNTERS = 16384;          // counters beside it
 constexpr int SURVEYORS = 256;                 // workgroups of k_survey at most
@@ -30,64 +32,72 @@ constexpr int SURVEYORS = 256;                 // workgroups of k_survey at most
 // Fibonacci hashing into 2^bits slots
 __device__ __forceinline__ u32 slot_of(u64 key, int bits) { return (u32)((key * 0x9E3779B97F4A7C15ull) >> (64 - bits)); }
 
+// One slot of the hash table in memory: an index of the table under the tag of the call (any other tag: unused).
+typedef unsigned long long Slot;
+
 // How a look-up finds its entry.
 struct Finder {
     const u64 *table;
     i64 n_table;
-    u64 *keys;                                 // the hash table: entry and index of each slot (EMPTY: unused)
-    u32 *index;
+    Slot *slots;
     int bits;                                  // log2 of the slots, 0: no hash table
-    const u32 *odd;                            // what each workgroup of the survey found: 1 when an entry is not its index
-    int n_odd;                                 // 0: the caller promises a range
+    u64 tag;                                   // of this call, in the bits above an index
+    u32 *found;                                // what each workgroup of the survey saw: OFF, DIAGONAL or both
+    int n_found;                               // 0: the caller promises a range
 };
+constexpr u32 OFF = 1, DIAGONAL = 2;           // entries that are not, and that are, their own index
 
-// Workgroup w looks at its share of the table and notes in odd[w] whether table[j] == j throughout, empties its share of the
-// slots and, when the counts are not added to what is there, zeroes its share of them.  It and the launch of k_insert that
-// finds nothing to do cost a call over a range 4 us at 2^13 entries and 2^16 and 7 at 2^20 (8 bytes read and 8 to 24 written
-// per entry).
-__global__ __launch_bounds__(COUNT_THREADS) void k_survey(const Finder F, u32 *odd, u64 *clear) {
-    const i64 first = (i64)blockIdx.x * COUNT_THREADS + threadIdx.x, stride = (i64)gridDim.x * COUNT_THREADS;
-    int differs = 0;
-    for (i64 j = first; j < F.n_table; j += stride) {
-        differs |= F.table[j] != (u64)j;
-        if (clear) clear[j] = 0;
+// A slot belongs to the first index that claims it; later indices of the same entry lower it to the smallest (every index it
+// ever holds has the same entry, which is read from the table).  Slots need no emptying: what lies there from before has
+// another tag.  Where it has this one all the same (one tag in 2^34) it is met like a claim: the index it names is compared
+// with the table here and by the look-ups, so it can stand in the way but not be taken for another entry.
+// Ends after at most 2^bits probes; half of the slots stay unused.
+__device__ __forceinline__ void insert(const Finder &F, u64 j, u64 key) {
+    const u32 mask = (1u << F.bits) - 1;
+    u32 h = slot_of(key, F.bits);
+    for (u32 probes = 0; probes <= mask; ++probes, h = (h + 1) & mask) {
+        Slot was = __hip_atomic_load(&F.slots[h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if ((was & ~INDEX_BITS) != F.tag) {
+            const Slot now = atomicCAS(&F.slots[h], was, (Slot)(F.tag | j));
+            if (now == was) return;
+            was = now;                         // another thread of this call was faster
+        }
+        const u64 other = was & INDEX_BITS;
+        if (other < (u64)F.n_table && F.table[other] == key) {
+            atomicMin(&F.slots[h], (Slot)(F.tag | j));
+            return;
+        }
     }
-    const i64 n_slots = F.bits ? (i64)1 << F.bits : 0;
-    for (i64 j = first; j < n_slots; j += stride) F.index[j] = EMPTY;
-    differs = __syncthreads_or(differs);
-    if (threadIdx.x == 0) odd[blockIdx.x] = differs ? 1 : 0;
+}
+
+// Goes over the table: notes in found[workgroup] whether there are entries that are, and that are not, their own index, and puts
+// the latter into the hash table; a range puts nothing.  When single look-ups are going to be added to the result it is zeroed
+// here (the launch that would do this is saved).  Costs a call over a range 2 to 3 us up to 2^18 entries, 4 at 2^20.
+__global__ __launch_bounds__(COUNT_THREADS) void k_survey(const Finder F, u64 *clear) {
+    const i64 first = (i64)blockIdx.x * COUNT_THREADS + threadIdx.x, stride = (i64)gridDim.x * COUNT_THREADS;
+    bool off = false, diagonal = false;
+    for (i64 j = first; j < F.n_table; j += stride) {
+        const u64 key = F.table[j];
+        if (clear) clear[j] = 0;
+        if (key == (u64)j) diagonal = true;
+        else {
+            off = true;
+            if (F.bits) insert(F, (u64)j, key);
+        }
+    }
+    off = __syncthreads_or(off);
+    diagonal = __syncthreads_or(diagonal);
+    if (threadIdx.x == 0) F.found[blockIdx.x] = (off ? OFF : 0) | (diagonal ? DIAGONAL : 0);
 }
 
 // the survey's result: a thread's part of it, which may be asked for early, and the whole, the same for every thread of a
 // workgroup (which all call this)
-__device__ __forceinline__ u32 odd_part(const Finder &F) { return (int)threadIdx.x < F.n_odd ? F.odd[threadIdx.x] : 0; }
-__device__ __forceinline__ bool is_range(u32 part) { return !__syncthreads_or((int)part); }
+__device__ __forceinline__ u32 found_part(const Finder &F) { return (int)threadIdx.x < F.n_found ? F.found[threadIdx.x] : 0; }
+__device__ __forceinline__ bool found_any(u32 part, u32 what) { return __syncthreads_or((part & what) != 0); }
 
-// A slot belongs to the first index that claims it; later indices of the same entry lower it to the smallest.  The entry
-// of a claimed slot is read from the table (every index it ever holds has the same one).  Ends after at most 2^bits
-// probes, and half of the slots stay empty.
-__device__ __forceinline__ void insert(const u64 *table, u32 j, u64 key, u64 *keys, u32 *index, int bits) {
-    const u32 mask = (1u << bits) - 1;
-    u32 h = slot_of(key, bits);
-    for (u32 probes = 0; probes <= mask; ++probes, h = (h + 1) & mask) {
-        const u32 was = atomicCAS(&index[h], EMPTY, j);
-        if (was == EMPTY) {
-            if (keys) keys[h] = key;
-            return;
-        }
-        if (table[was] == key) {
-            atomicMin(&index[h], j);
-            return;
-        }
-    }
-}
-
-// nothing to do for a range
-__global__ __launch_bounds__(BLOCK) void k_insert(const Finder F) {
-    if (is_range(odd_part(F))) return;
+__global__ __launch_bounds__(BLOCK) void k_clear_slots(Slot *slots, i64 n) {
     const i64 stride = (i64)gridDim.x * BLOCK;
-    for (i64 j = (i64)blockIdx.x * BLOCK + threadIdx.x; j < F.n_table; j += stride)
-        insert(F.table, (u32)j, F.table[j], F.keys, F.index, F.bits);
+    for (i64 i = (i64)blockIdx.x * BLOCK + threadIdx.x; i < n; i += stride) slots[i] = 0;
 }
 
 __global__ __launch_bounds__(BLOCK) void k_clear_counts(u64 *mult, i64 n) {
@@ -95,24 +105,25 @@ __global__ __launch_bounds__(BLOCK) void k_clear_counts(u64 *mult, i64 n) {
     for (i64 i = (i64)blockIdx.x * BLOCK + threadIdx.x; i < n; i += stride) mult[i] = 0;
 }
 
-// the index a value counts for, or at least n_table for none
-template <bool RANGE>
-__device__ __forceinline__ u64 index_of(u64 x, const Finder &F) {
-    if (RANGE) return x;
+// The index a value counts for, or at least n_table for none: the smaller one of its own, where the table holds it there, and of
+// the one in the hash table.
+__device__ __forceinline__ u64 index_of(u64 x, const Finder &F, bool diagonal) {
     if (F.bits == 0) {                         // a table beyond the indices of a slot: searched from the front
         i64 j = 0;
         while (j < F.n_table && F.table[j] != x) ++j;
         return (u64)j;
     }
+    u64 own = ~0ull;
+    if (diagonal && x < (u64)F.n_table && F.table[x] == x) own = x;
     const u32 mask = (1u << F.bits) - 1;
     u32 h = slot_of(x, F.bits);
     for (u32 probes = 0; probes <= mask; ++probes, h = (h + 1) & mask) {
-        const u32 at = F.index[h];
-        const u64 key = F.keys[h];             // beside the index, not behind it (an unused slot holds anything)
-        if (at == EMPTY) break;
-        if (key == x) return at;
+        const Slot slot = F.slots[h];
+        if ((slot & ~INDEX_BITS) != F.tag) break;
+        const u64 at = slot & INDEX_BITS;
+        if (at < (u64)F.n_table && F.table[at] == x) return at < own ? at : own;
     }
-    return ~0ull;
+    return own;
 }
 
 // counts of the entries base .. base + mine - 1 among x[lo .. hi - 1], each at(value) an index of the table; `copies` (a power
@@ -165,20 +176,23 @@ __global__ __launch_bounds__(COUNT_THREADS) void k_count(const u64 *__restrict__
     u32 *counts = reinterpret_cast<u32 *>(lds_counts);
     const i64 base = (i64)blockIdx.x * SLICE, group = blockIdx.y;
     const int mine = F.n_table - base < SLICE ? (int)(F.n_table - base) : SLICE;
-    const u32 part = odd_part(F);
+    const u32 part = found_part(F);
     // the launch's LDS is a whole number of 16-byte words
     for (int i = threadIdx.x; i < (mine * copies + 3) / 4; i += COUNT_THREADS) lds_counts[i] = make_uint4(0, 0, 0, 0);
-    const bool range = is_range(part);         // a barrier as well
+    const bool range = !found_any(part, OFF);  // a barrier as well
     const i64 lo = group * per_group, hi = lo + per_group < n_x ? lo + per_group : n_x;
-    if (range) count(x, lo, hi, (u64)base, mine, copies, counts, [&](u64 v) { return index_of<true>(v, F); });
-    else count(x, lo, hi, (u64)base, mine, copies, counts, [&](u64 v) { return index_of<false>(v, F); });
+    if (range) count(x, lo, hi, (u64)base, mine, copies, counts, [](u64 v) { return v; });
+    else {
+        const bool diagonal = found_any(part, DIAGONAL);
+        count(x, lo, hi, (u64)base, mine, copies, counts, [&](u64 v) { return index_of(v, F, diagonal); });
+    }
     __syncthreads();
     put_counts(counts, mine, copies, rows ? rows + group * F.n_table + base : nullptr, (F.n_table & 3) == 0, mult + base, accumulate);
 }
 
 // The same for a table of up to SMALL_TABLE entries that nothing is known of: every workgroup takes it into its LDS, sees
 // whether it is a range and, if not, makes its own hash table beside it.  One launch where the survey of a longer table takes
-// two more (1.5 M look-ups in 2^12 entries 12.0 us, in 2^13 through the survey 18.4); 32 KiB of table per workgroup come
+// one more (1.5 M look-ups in 2^12 entries 12.0 us, in 2^13 through the survey 17.2); 32 KiB of table per workgroup come
 // from the L2.
 __global__ __launch_bounds__(COUNT_THREADS) void k_count_small(const u64 *__restrict__ x, i64 n_x, i64 per_group, const u64 *__restrict__ table,
                                                                int n_table, int bits, int copies, u32 *rows, u64 *mult, int accumulate) {
@@ -199,7 +213,18 @@ __global__ __launch_bounds__(COUNT_THREADS) void k_count_small(const u64 *__rest
     const i64 group = blockIdx.x, lo = group * per_group, hi = lo + per_group < n_x ? lo + per_group : n_x;
     if (!odd) count(x, lo, hi, 0, n_table, copies, counts, [](u64 v) { return v; });
     else {
-        for (int j = tid; j < n_table; j += COUNT_THREADS) insert(keys, (u32)j, keys[j], nullptr, index, bits);
+        for (int j = tid; j < n_table; j += COUNT_THREADS) {
+            const u64 key = keys[j];
+            u32 h = slot_of(key, bits);
+            for (int probes = 0; probes < n_slots; ++probes, h = (h + 1) & (n_slots - 1)) {
+                const u32 was = atomicCAS(&index[h], EMPTY, (u32)j);
+                if (was == EMPTY) break;
+                if (keys[was] == key) {
+                    atomicMin(&index[h], (u32)j);
+                    break;
+                }
+            }
+        }
         __syncthreads();
         count(x, lo, hi, 0, n_table, copies, counts, [&](u64 v) -> u64 {
             u32 h = slot_of(v, bits);
@@ -245,14 +270,16 @@ __global__ __launch_bounds__(BLOCK) void k_add_rows(const u32 *__restrict__ rows
 // one global atomic per look-up
 __global__ __launch_bounds__(BLOCK) void k_count_global(const u64 *__restrict__ x, i64 n_x, const Finder F, unsigned long long *__restrict__ mult) {
     const i64 stride = (i64)gridDim.x * BLOCK, first = (i64)blockIdx.x * BLOCK + threadIdx.x;
-    if (is_range(odd_part(F))) {
+    const u32 part = found_part(F);
+    if (!found_any(part, OFF)) {
         for (i64 i = first; i < n_x; i += stride) {
-            const u64 at = index_of<true>(x[i], F);
+            const u64 at = x[i];
             if (at < (u64)F.n_table) atomicAdd(&mult[at], 1ULL);
         }
     } else {
+        const bool diagonal = found_any(part, DIAGONAL);
         for (i64 i = first; i < n_x; i += stride) {
-            const u64 at = index_of<false>(x[i], F);
+            const u64 at = index_of(x[i], F, diagonal);
             if (at < (u64)F.n_table) atomicAdd(&mult[at], 1ULL);
         }
     }
@@ -286,9 +313,9 @@ struct Plan {
     bool small, direct;                        // k_count_small; one global atomic per look-up
     i64 slices, groups;
     int copies, bits, surveyors;
-    size_t key_bytes, index_bytes, odd_bytes, row_bytes;
+    size_t slot_bytes, found_bytes, row_bytes;
     size_t bytes() const {
-        const size_t used = key_bytes + index_bytes + odd_bytes + row_bytes;
+        const size_t used = slot_bytes + found_bytes + row_bytes;
         return used ? used + vi::WS_SLACK : 0;
     }
 };
@@ -306,11 +333,8 @@ Plan make_plan(i64 n_x, i64 n_table, bool promised) {
         if (!L.small) {
             const i64 shares = (n_table + COUNT_THREADS - 1) / COUNT_THREADS;
             L.surveyors = (int)(shares < SURVEYORS ? shares : SURVEYORS);
-            if (L.bits) {
-                L.key_bytes = sizeof(u64) << L.bits;
-                L.index_bytes = sizeof(u32) << L.bits;
-            }
-            L.odd_bytes = SURVEYORS * sizeof(u32);
+            if (L.bits) L.slot_bytes = sizeof(Slot) << L.bits;
+            L.found_bytes = SURVEYORS * sizeof(u32);
         }
     }
     L.slices = (n_table + SLICE - 1) / SLICE;
@@ -329,6 +353,12 @@ Plan make_plan(i64 n_x, i64 n_table, bool promised) {
     while (L.copies < MAX_COPIES && n_table * L.copies * 2 <= counters) L.copies *= 2;
     L.row_bytes = L.groups > 1 ? (size_t)L.groups * n_table * sizeof(u32) : 0;
     return L;
+}
+
+// 1 .. 2^34 - 1 in the bits above an index; 0 is what an emptied slot holds
+u64 next_tag() {
+    static std::atomic<u64> calls{0};
+    return (calls.fetch_add(1, std::memory_order_relaxed) % (((u64)1 << 34) - 1) + 1) << 30;
 }
 
 // more than 64 KiB of dynamic LDS has to be asked for, once per device and kernel
@@ -383,20 +413,22 @@ int vi_lookup_histogram(const uint64_t *x, int64_t n_x, const uint64_t *table, i
     Finder F = {};
     F.table = table;
     F.n_table = n_table;
+    F.slots = (Slot *)ws;
     F.bits = L.bits;
-    F.keys = (u64 *)ws;
-    F.index = (u32 *)((char *)ws + L.key_bytes);
-    u32 *odd = (u32 *)((char *)ws + L.key_bytes + L.index_bytes);
-    u32 *rows = L.row_bytes ? (u32 *)((char *)ws + L.key_bytes + L.index_bytes + L.odd_bytes) : nullptr;
-    F.odd = odd;
-    F.n_odd = L.surveyors;
+    F.found = (u32 *)((char *)ws + L.slot_bytes);
+    F.n_found = L.surveyors;
+    u32 *rows = L.row_bytes ? (u32 *)((char *)ws + L.slot_bytes + L.found_bytes) : nullptr;
     if (L.surveyors) {
-        hipLaunchKernelGGL(k_survey, dim3((unsigned)L.surveyors), dim3(COUNT_THREADS), 0, s, F, odd, L.direct && !accumulate ? mult : nullptr);
-        VI_LAUNCH_CHECK("k_survey");
-        if (L.bits) {
-            hipLaunchKernelGGL(k_insert, dim3(capped_grid(n_table)), dim3(BLOCK), 0, s, F);
-            VI_LAUNCH_CHECK("k_insert");
+        // a replay has the tag of the capture, so a captured call empties the slots
+        F.tag = next_tag();
+        bool captured = false;
+        if (int rc = vi::capturing(s, &captured)) return rc;
+        if (captured && L.bits) {
+            hipLaunchKernelGGL(k_clear_slots, dim3(capped_grid((i64)1 << L.bits)), dim3(BLOCK), 0, s, F.slots, (i64)1 << L.bits);
+            VI_LAUNCH_CHECK("k_clear_slots");
         }
+        hipLaunchKernelGGL(k_survey, dim3((unsigned)L.surveyors), dim3(COUNT_THREADS), 0, s, F, L.direct && !accumulate ? mult : nullptr);
+        VI_LAUNCH_CHECK("k_survey");
     } else if (L.direct && !accumulate) {
         hipLaunchKernelGGL(k_clear_counts, dim3(capped_grid(n_table)), dim3(BLOCK), 0, s, mult, (i64)n_table);
         VI_LAUNCH_CHECK("k_clear_counts");

@@ -1,15 +1,16 @@
 // Dense products over the field on the int8 matrix cores.
 //
-// A 64 x 64-bit multiply-accumulate is 13 or more VALU instructions, so a product of many rows of A is bound by VALU
-// issue at about 2 T multiply-adds per second whatever its tiling.  Here the exact integer product is computed modulo 18
+// A 64 x 64-bit multiply-accumulate is at least 8 VALU instructions, so a product of many rows of A is bound by VALU
+// issue at 2 to 2.6 T multiply-adds per second whatever its tiling.  Here the exact integer product is computed modulo 18
 // pairwise coprime numbers m_i <= 256 instead and put together by the Chinese remainder theorem (the residue-number
 // form of integer matrix products; Ozaki, Uchino, Imamura 2024 use it for floating point).  Modulo one m_i an operand
 // is a signed byte, so each residue is ONE int8 matrix product on v_mfma_i32_32x32x32_i8: 18 byte multiply-adds per
 // field multiply-add, where splitting both operands into bytes would take 64.
 //
-// What bounds it at 1000 x 4096 x 4096 (8240 us on the VALU, 450 here): the int8 products 340 us, 1.8 POP/s with the
-// operands crossing the LDS once per 32 (columns: 64) rows of a wavefront's tile; the residues 85 us, 0.44 GB at the rate
-// of a copy; the reconstruction 20 us.
+// What bounds it at 1000 x 4096 x 4096 (8240 us on the VALU, 470 here): the int8 products 346 us, 1.8 POP/s -- the matrix
+// cores are busy 43 % of the cycles and the LDS a third, neither at its limit: with two wavefronts to a SIMD (registers) the
+// barrier and the operand reads of a step are not covered by the other one's products; the residues 104 us, 0.44 GB at the
+// rate of a copy; the reconstruction 21 us.
 //
 //   k_residues        words -> 18 planes of signed bytes
 //   k_residue_gemm    per plane an int8 product; the 32-bit sums are reduced mod m_i to one byte

@@ -10,7 +10,8 @@
 //
 // Rows of more points take the passes of ntt_plan.hpp, digit by digit, with the same four points per thread (k_small_pass): a
 // launch takes 4.3 us where one of k_ntt_fast takes 8, and the cosets of an extension run side by side.  One row of 2^16
-// extended to 2^18: 57 -> 21 us; 16 rows of 2^12 transformed: 11.6 -> 8.6 us.
+// extended to 2^18: 57 -> 21 us; 16 rows of 2^12 transformed, calls in a queue: 11.6 -> 8.6 us (two launches where k_ntt_row is
+// one: a program that transforms them there and back with a copy in between takes 25 us either way).
 #pragma once
 
 namespace {
