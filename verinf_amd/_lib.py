@@ -8,6 +8,7 @@ handles mean the same thing on both sides.
 import array
 import contextlib
 import ctypes
+import functools
 import os
 import threading
 from ctypes import POINTER, c_char_p, c_double, c_int, c_int64, c_size_t, c_uint64, c_void_p
@@ -176,6 +177,12 @@ _NO_GUARD = contextlib.nullcontext()
 def on_device(dev):
     """Context that makes `dev` current; nothing to do (and nothing paid) when it already is."""
     return _NO_GUARD if dev.index is None or dev.index == _get_device() else torch.cuda.device(dev)
+
+
+@functools.lru_cache(maxsize=1024)
+def workspace_bytes(entry: str, *sizes: int) -> int:
+    """vi_<entry>_workspace_bytes(*sizes), which depends on nothing else (0.1 us where the call through ctypes takes 0.5)."""
+    return getattr(lib(), f"vi_{entry}_workspace_bytes")(*sizes)
 
 
 _ws_cache = {}

@@ -222,7 +222,7 @@ def mle_eval_t(tables, point: Sequence[int]):
     L = _lib.lib()
     with _lib.on_device(tables.device):
         sp = _lib.stream_ptr()
-        ws_bytes = L.vi_mle_eval_workspace_bytes(k)
+        ws_bytes = _lib.workspace_bytes("mle_eval", k)
         out = _lib.result_words(k, sp)
         with _lib.stream_lock(sp):
             ws = _lib.workspace(ws_bytes, "mle", sp)
@@ -244,7 +244,7 @@ def gl_sum(t):
     with _lib.on_device(v.device):
         sp = _lib.stream_ptr()
         with _lib.stream_lock(sp):
-            ws = _lib.workspace(L.vi_gl_sum_workspace_bytes(v.numel()), "sum", sp)
+            ws = _lib.workspace(_lib.workspace_bytes("gl_sum", v.numel()), "sum", sp)
             _lib.check(L.vi_gl_sum(v.data_ptr(), v.numel(), out.data_ptr(), ws.data_ptr(), ws.numel(), sp))
     return out
 
@@ -380,7 +380,7 @@ def prove_terms_gpu(terms, coin, field_p: int, mask=None, mu0: int = 0):
         samples_host, samples_np = _lib.pinned_words(8 * n_rounds, sp)
         chal = (ctypes.c_uint64 * n_rounds)(*challenges)
         with _lib.stream_lock(sp):
-            ws = _lib.workspace(L.vi_sumcheck_prove_coins_workspace_bytes(size), "sumcheck_coins", sp)
+            ws = _lib.workspace(_lib.workspace_bytes("sumcheck_prove_coins", size), "sumcheck_coins", sp)
             # the folded tables live in one cached scratch buffer, a half-length slice per table (the caller's
             # tensors are never written)
             half_bytes = (size // 2) * 8

@@ -140,7 +140,7 @@ def _ntt(rows, m, n, inverse):
     with _lib.on_device(rows.device):
         # the library transforms the rows in chunks that fit the workspace it is given: one row is the minimum,
         # 1 GiB is enough to fill the GPU, and a large batch does not double its footprint for the process's life
-        need = min(L.vi_ntt_best_workspace_bytes(m, n), max(_NTT_WS_CAP, n * 8))
+        need = min(_lib.workspace_bytes("ntt_best", m, n), max(_NTT_WS_CAP, n * 8))
         sp = _lib.stream_ptr()
         if not need:
             _lib.check(L.vi_ntt_batched(rows.data_ptr(), m, n, int(inverse), None, 0, sp))
@@ -236,7 +236,7 @@ def coset_lde(messages, k_deg, n_lig, shift=GLOBAL_G, out=None):
     with _lib.on_device(messages.device):
         sp = _lib.stream_ptr()
         with _lib.stream_lock(sp):
-            ws = _lib.workspace(L.vi_coset_lde_workspace_bytes(m, k_deg, n_lig), "lde", sp)
+            ws = _lib.workspace(_lib.workspace_bytes("coset_lde", m, k_deg, n_lig), "lde", sp)
             _lib.check(L.vi_coset_lde(messages.data_ptr(), m, w, in_stride, k_deg, n_lig, int(shift) % P,
                                       out.data_ptr(), n_lig, ws.data_ptr(), ws.numel(), sp))
     return out
@@ -268,7 +268,7 @@ def coset_lde_with_coeffs(messages, k_deg, n_lig, shift=GLOBAL_G, need_codewords
     with _lib.on_device(messages.device):
         sp = _lib.stream_ptr()
         with _lib.stream_lock(sp):
-            ws = _lib.workspace(L.vi_coset_lde_workspace_bytes(m, k_deg, n_lig), "lde", sp)
+            ws = _lib.workspace(_lib.workspace_bytes("coset_lde", m, k_deg, n_lig), "lde", sp)
             _lib.check(L.vi_coset_lde_coeffs(messages.data_ptr(), m, w, in_stride, k_deg, n_lig, int(shift) % P,
                                              coeffs.data_ptr(), k_deg, out.data_ptr() if out is not None else None, n_lig,
                                              ws.data_ptr(), ws.numel(), sp))
@@ -289,7 +289,7 @@ def coset_extend(coeffs, k_deg, n_lig, shift=GLOBAL_G, out=None):
     with _lib.on_device(coeffs.device):
         sp = _lib.stream_ptr()
         with _lib.stream_lock(sp):
-            ws = _lib.workspace(L.vi_coset_lde_workspace_bytes(m, k_deg, n_lig), "lde", sp)
+            ws = _lib.workspace(_lib.workspace_bytes("coset_lde", m, k_deg, n_lig), "lde", sp)
             _lib.check(L.vi_coset_extend(coeffs.data_ptr(), m, w, in_stride, k_deg, n_lig, int(shift) % P,
                                          out.data_ptr(), n_lig, ws.data_ptr(), ws.numel(), sp))
     return out
@@ -323,7 +323,7 @@ def gl_matmul(A, B):
         sp = _lib.stream_ptr()
         for lo in range(0, m, 65535):
             rows = min(65535, m - lo)
-            need = L.vi_gl_matmul_workspace_bytes(rows, k, n)
+            need = _lib.workspace_bytes("gl_matmul", rows, k, n)
             if not need:
                 _lib.check(L.vi_gl_matmul(a_ptr + lo * k * 8, B.data_ptr(), c_ptr + lo * n * 8, rows, k, n, None, 0, sp))
                 continue
@@ -455,7 +455,7 @@ def hash_columns_streamed(matrix):
         raise RuntimeError("matrix must be contiguous")
     L = _lib.lib()
     out = torch.empty((n, 32), dtype=torch.uint8, device=matrix.device)
-    nbytes = L.vi_hash_columns_workspace_bytes(m, n)
+    nbytes = _lib.workspace_bytes("hash_columns", m, n)
     with _lib.on_device(matrix.device):
         sp = _lib.stream_ptr()
         with _lib.stream_lock(sp):
@@ -483,7 +483,7 @@ class MerkleColumnAccumulator:
         self.n_total_rows = int(n_total_rows)
         self.n_chunks_total = _n_chunks(n_total_rows)
         L = _lib.lib()
-        nbytes = L.vi_hash_columns_workspace_bytes(self.n_total_rows, self.n_cols)
+        nbytes = _lib.workspace_bytes("hash_columns", self.n_total_rows, self.n_cols)
         self._states = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
         self._chunks_seen = 0
         self._rows_seen = 0
@@ -740,7 +740,7 @@ def _histogram(x, table, mult, accumulate):
     # whether the table is a range is looked at on the device, in every call: nothing is kept of a table
     L = _lib.lib()
     n_x, n_t = x.numel(), table.numel()
-    need = L.vi_lookup_histogram_workspace_bytes(n_x, n_t, 0)
+    need = _lib.workspace_bytes("lookup_histogram", n_x, n_t, 0)
     args = (x.data_ptr(), n_x, table.data_ptr(), n_t, 0, accumulate, mult.data_ptr())
     with _lib.on_device(x.device):
         sp = _lib.stream_ptr()
