@@ -127,7 +127,7 @@ inline void launch(dim3 grid, dim3 block, const std::function<void()> &f) {
         }
 }
 
-inline int any_true;
+inline int any_true, wave_any[16];
 inline int32_t wave_a[16][64][4], wave_b[16][64][4];                  // operands of a matrix instruction, by wavefront and lane
 
 }  // namespace simt
@@ -144,6 +144,16 @@ inline int __syncthreads_or(int v) {
     __syncthreads();
     return r;
 }
+inline int __any(int v) {                                             // over the threads of a wavefront that are still there
+    int &any = simt::wave_any[threadIdx.x >> 6];
+    any = 0;
+    simt::wait_at(simt::AT_WAVE);
+    any |= v != 0;
+    simt::wait_at(simt::AT_WAVE);
+    const int r = any;
+    simt::wait_at(simt::AT_WAVE);
+    return r;
+}
 inline void __threadfence_system() {}
 #define __builtin_amdgcn_fence(...) ((void)0)
 #define __builtin_amdgcn_wave_barrier() simt::wait_at(simt::AT_WAVE)
@@ -154,6 +164,8 @@ inline void __threadfence_system() {}
 
 template <class T, class V>
 T atomicAdd(T *p, V v) { T was = *p; *p += (T)v; return was; }
+template <class T, class V>
+T atomicOr(T *p, V v) { T was = *p; *p |= (T)v; return was; }
 template <class T, class V>
 T atomicMin(T *p, V v) { T was = *p; if ((T)v < was) *p = (T)v; return was; }
 template <class T, class E, class V>

@@ -44,7 +44,9 @@ def lookup(so):
         hit = keys[at] == x if len(x) else np.zeros(0, bool)
         return np.bincount(first[at[hit]], minlength=len(table)).astype(np.uint64)
 
-    # the first call of the library, whose tag is 1: scratch that holds slots of that very tag, naming any index or none
+    # the first calls of the library, whose tags are known: scratch that holds slots of that very tag, naming any index or none, in
+    # some of the slots and in all of them
+    tags = [1 << 63 | (n * 0x9E3779B97F4A7C15 & (1 << 33) - 1) << 30 for n in range(2)]
     rng = np.random.default_rng(0)
     n_t = 5000
     table = field(n_t, 1)
@@ -53,11 +55,12 @@ def lookup(so):
     x = np.concatenate([table[rng.integers(0, n_t, 9001)], np.arange(0, 600, dtype=np.uint64)])
     ws = scratch(L.vi_lookup_histogram_workspace_bytes(len(x), n_t, 0))
     slots = ws[(-ws.ctypes.data) % 16:][:8 << 14].view(np.uint64)
-    taken = rng.random(len(slots)) < 0.4
-    slots[taken] = (np.uint64(1 << 30) | rng.integers(0, 2 * n_t, len(slots)).astype(np.uint64))[taken]
     mult = np.empty(n_t, dtype=np.uint64)
-    assert L.vi_lookup_histogram(ptr(x), len(x), ptr(table), n_t, 0, 0, ptr(mult), ptr(ws), len(ws), None) == 0
-    assert np.array_equal(mult, counts(x, table))
+    for tag, share in zip(tags, (0.4, 1.0)):
+        taken = rng.random(len(slots)) < share
+        slots[taken] = (np.uint64(tag) | rng.integers(0, 2 * n_t, len(slots)).astype(np.uint64))[taken]
+        assert L.vi_lookup_histogram(ptr(x), len(x), ptr(table), n_t, 0, 0, ptr(mult), ptr(ws), len(ws), None) == 0
+        assert np.array_equal(mult, counts(x, table)), share
     for seed in (2, 3):                                        # the same scratch again, with slots of the calls before
         table = np.random.default_rng(seed).permutation(table)
         assert L.vi_lookup_histogram(ptr(x), len(x), ptr(table), n_t, 0, 0, ptr(mult), ptr(ws), len(ws), None) == 0

@@ -10,7 +10,7 @@
 // the search from the front costs half the table.  Which of the two a table is, is looked at in every call, on the device: up
 // to 4096 entries by every workgroup for itself (k_count_small: table and hash in LDS), beyond by a launch over the table
 // (k_survey), whose findings the counting workgroups read.  us per call in a queue of them, 1.5 M look-ups: 10 in 2^6 entries,
-// 12.0 in 2^12, 21.4 in 2^16, 52 in 2^20 (19.0 and 48 for the last two when the caller promises a range); 10^6 look-ups in 3003
+// 12.0 in 2^12, 21.0 in 2^16, 51 in 2^20 (19.0 and 48 for the last two when the caller promises a range); 10^6 look-ups in 3003
 // values 12.6, in 40000 36.
 #include "common.hpp"
 #include "gl_field.hpp"
@@ -42,52 +42,59 @@ struct Finder {
     Slot *slots;
     int bits;                                  // log2 of the slots, 0: no hash table
     u64 tag;                                   // of this call, in the bits above an index
-    u32 *found;                                // what each workgroup of the survey saw: OFF, DIAGONAL or both
+    u32 *found;                                // what each workgroup of the survey saw
     int n_found;                               // 0: the caller promises a range
 };
 constexpr u32 OFF = 1, DIAGONAL = 2;           // entries that are not, and that are, their own index
+constexpr u32 LOST = 4;                        // an entry that found no slot: the table is searched from the front
+constexpr u32 MAX_PROBES = 1 << 14;
 
 // A slot belongs to the first index that claims it; later indices of the same entry lower it to the smallest (every index it
 // ever holds has the same entry, which is read from the table).  Slots need no emptying: what lies there from before has
-// another tag.  Where it has this one all the same (one tag in 2^34) it is met like a claim: the index it names is compared
-// with the table here and by the look-ups, so it can stand in the way but not be taken for another entry.
-// Ends after at most 2^bits probes; half of the slots stay unused.
-__device__ __forceinline__ void insert(const Finder &F, u64 j, u64 key) {
+// another tag, unless by an accident of one in 2^33.  Even then it is met like a claim: the index it names is compared with the
+// table, here and by the look-ups, so it can stand in the way but not be taken for another entry, and an entry that finds no
+// slot within MAX_PROBES is reported.  Half of the slots and more stay unused.
+__device__ __forceinline__ bool insert(const Finder &F, u64 j, u64 key) {
     const u32 mask = (1u << F.bits) - 1;
     u32 h = slot_of(key, F.bits);
-    for (u32 probes = 0; probes <= mask; ++probes, h = (h + 1) & mask) {
+    for (u32 probes = 0; probes <= mask && probes < MAX_PROBES; ++probes, h = (h + 1) & mask) {
         Slot was = __hip_atomic_load(&F.slots[h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if ((was & ~INDEX_BITS) != F.tag) {
             const Slot now = atomicCAS(&F.slots[h], was, (Slot)(F.tag | j));
-            if (now == was) return;
+            if (now == was) return true;
             was = now;                         // another thread of this call was faster
         }
         const u64 other = was & INDEX_BITS;
         if (other < (u64)F.n_table && F.table[other] == key) {
             atomicMin(&F.slots[h], (Slot)(F.tag | j));
-            return;
+            return true;
         }
     }
+    return false;
 }
 
 // Goes over the table: notes in found[workgroup] whether there are entries that are, and that are not, their own index, and puts
 // the latter into the hash table; a range puts nothing.  When single look-ups are going to be added to the result it is zeroed
-// here (the launch that would do this is saved).  Costs a call over a range 2 to 3 us up to 2^18 entries, 4 at 2^20.
+// here (the launch that would do this is saved).  Costs a call over a range 2 us up to 2^18 entries, 3 at 2^20.
 __global__ __launch_bounds__(COUNT_THREADS) void k_survey(const Finder F, u64 *clear) {
     const i64 first = (i64)blockIdx.x * COUNT_THREADS + threadIdx.x, stride = (i64)gridDim.x * COUNT_THREADS;
-    bool off = false, diagonal = false;
+    __shared__ u32 seen;
+    if (threadIdx.x == 0) seen = 0;
+    __syncthreads();
+    bool off = false, diagonal = false, lost = false;
     for (i64 j = first; j < F.n_table; j += stride) {
         const u64 key = F.table[j];
         if (clear) clear[j] = 0;
         if (key == (u64)j) diagonal = true;
         else {
             off = true;
-            if (F.bits) insert(F, (u64)j, key);
+            if (F.bits && !insert(F, (u64)j, key)) lost = true;
         }
     }
-    off = __syncthreads_or(off);
-    diagonal = __syncthreads_or(diagonal);
-    if (threadIdx.x == 0) F.found[blockIdx.x] = (off ? OFF : 0) | (diagonal ? DIAGONAL : 0);
+    const u32 mine = (__any(off) ? OFF : 0) | (__any(diagonal) ? DIAGONAL : 0) | (__any(lost) ? LOST : 0);
+    if ((threadIdx.x & 63) == 0) atomicOr(&seen, mine);
+    __syncthreads();
+    if (threadIdx.x == 0) F.found[blockIdx.x] = seen;
 }
 
 // the survey's result: a thread's part of it, which may be asked for early, and the whole, the same for every thread of a
@@ -107,8 +114,8 @@ __global__ __launch_bounds__(BLOCK) void k_clear_counts(u64 *mult, i64 n) {
 
 // The index a value counts for, or at least n_table for none: the smaller one of its own, where the table holds it there, and of
 // the one in the hash table.
-__device__ __forceinline__ u64 index_of(u64 x, const Finder &F, bool diagonal) {
-    if (F.bits == 0) {                         // a table beyond the indices of a slot: searched from the front
+__device__ __forceinline__ u64 index_of(u64 x, const Finder &F, bool diagonal, bool search) {
+    if (search) {                              // from the front
         i64 j = 0;
         while (j < F.n_table && F.table[j] != x) ++j;
         return (u64)j;
@@ -117,7 +124,7 @@ __device__ __forceinline__ u64 index_of(u64 x, const Finder &F, bool diagonal) {
     if (diagonal && x < (u64)F.n_table && F.table[x] == x) own = x;
     const u32 mask = (1u << F.bits) - 1;
     u32 h = slot_of(x, F.bits);
-    for (u32 probes = 0; probes <= mask; ++probes, h = (h + 1) & mask) {
+    for (u32 probes = 0; probes <= mask && probes < MAX_PROBES; ++probes, h = (h + 1) & mask) {
         const Slot slot = F.slots[h];
         if ((slot & ~INDEX_BITS) != F.tag) break;
         const u64 at = slot & INDEX_BITS;
@@ -183,8 +190,8 @@ __global__ __launch_bounds__(COUNT_THREADS) void k_count(const u64 *__restrict__
     const i64 lo = group * per_group, hi = lo + per_group < n_x ? lo + per_group : n_x;
     if (range) count(x, lo, hi, (u64)base, mine, copies, counts, [](u64 v) { return v; });
     else {
-        const bool diagonal = found_any(part, DIAGONAL);
-        count(x, lo, hi, (u64)base, mine, copies, counts, [&](u64 v) { return index_of(v, F, diagonal); });
+        const bool diagonal = found_any(part, DIAGONAL), search = found_any(part, LOST) || F.bits == 0;
+        count(x, lo, hi, (u64)base, mine, copies, counts, [&](u64 v) { return index_of(v, F, diagonal, search); });
     }
     __syncthreads();
     put_counts(counts, mine, copies, rows ? rows + group * F.n_table + base : nullptr, (F.n_table & 3) == 0, mult + base, accumulate);
@@ -192,7 +199,7 @@ __global__ __launch_bounds__(COUNT_THREADS) void k_count(const u64 *__restrict__
 
 // The same for a table of up to SMALL_TABLE entries that nothing is known of: every workgroup takes it into its LDS, sees
 // whether it is a range and, if not, makes its own hash table beside it.  One launch where the survey of a longer table takes
-// one more (1.5 M look-ups in 2^12 entries 12.0 us, in 2^13 through the survey 17.2); 32 KiB of table per workgroup come
+// one more (1.5 M look-ups in 2^12 entries 12.0 us, in 2^13 through the survey 16.6); 32 KiB of table per workgroup come
 // from the L2.
 __global__ __launch_bounds__(COUNT_THREADS) void k_count_small(const u64 *__restrict__ x, i64 n_x, i64 per_group, const u64 *__restrict__ table,
                                                                int n_table, int bits, int copies, u32 *rows, u64 *mult, int accumulate) {
@@ -277,9 +284,9 @@ __global__ __launch_bounds__(BLOCK) void k_count_global(const u64 *__restrict__ 
             if (at < (u64)F.n_table) atomicAdd(&mult[at], 1ULL);
         }
     } else {
-        const bool diagonal = found_any(part, DIAGONAL);
+        const bool diagonal = found_any(part, DIAGONAL), search = found_any(part, LOST) || F.bits == 0;
         for (i64 i = first; i < n_x; i += stride) {
-            const u64 at = index_of(x[i], F, diagonal);
+            const u64 at = index_of(x[i], F, diagonal, search);
             if (at < (u64)F.n_table) atomicAdd(&mult[at], 1ULL);
         }
     }
@@ -355,10 +362,12 @@ Plan make_plan(i64 n_x, i64 n_table, bool promised) {
     return L;
 }
 
-// 1 .. 2^34 - 1 in the bits above an index; 0 is what an emptied slot holds
+// The tag of a call, in the 34 bits above an index.  The top bit is set, as it is in no emptied slot, count or other small number
+// that scratch may hold; the others take all values in turn, scattered so that no run of calls meets a common pattern.
 u64 next_tag() {
     static std::atomic<u64> calls{0};
-    return (calls.fetch_add(1, std::memory_order_relaxed) % (((u64)1 << 34) - 1) + 1) << 30;
+    const u64 n = calls.fetch_add(1, std::memory_order_relaxed) * 0x9E3779B97F4A7C15ull & (((u64)1 << 33) - 1);
+    return ((u64)1 << 63) | n << 30;
 }
 
 // more than 64 KiB of dynamic LDS has to be asked for, once per device and kernel
