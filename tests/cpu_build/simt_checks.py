@@ -61,6 +61,8 @@ def lookup(so):
         slots[taken] = (np.uint64(tag) | rng.integers(0, 2 * n_t, len(slots)).astype(np.uint64))[taken]
         assert L.vi_lookup_histogram(ptr(x), len(x), ptr(table), n_t, 0, 0, ptr(mult), ptr(ws), len(ws), None) == 0
         assert np.array_equal(mult, counts(x, table)), share
+        found = int(ws[(-ws.ctypes.data) % 16:][8 << 14:][:4].view(np.uint32)[0])
+        assert found == (7 if share == 1.0 else 3)             # off and on the diagonal, and entries without a slot
     for seed in (2, 3):                                        # the same scratch again, with slots of the calls before
         table = np.random.default_rng(seed).permutation(table)
         assert L.vi_lookup_histogram(ptr(x), len(x), ptr(table), n_t, 0, 0, ptr(mult), ptr(ws), len(ws), None) == 0
