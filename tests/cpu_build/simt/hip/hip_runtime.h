@@ -171,6 +171,7 @@ T atomicMin(T *p, V v) { T was = *p; if ((T)v < was) *p = (T)v; return was; }
 template <class T, class E, class V>
 T atomicCAS(T *p, E expect, V v) { T was = *p; if (was == (T)expect) *p = (T)v; return was; }
 
+inline uint32_t __builtin_amdgcn_readfirstlane(uint32_t v) { return v; }   // of values that are the same for the wavefront
 inline uint32_t __brev(uint32_t v) {
     uint32_t r = 0;
     for (int b = 0; b < 32; ++b) r |= ((v >> b) & 1) << (31 - b);

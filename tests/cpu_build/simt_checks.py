@@ -207,6 +207,13 @@ def lde(so):
     print("lde", flush=True)
 
 
+def small(shape, seed, fill):
+    """Signed 16-bit numbers mod p: any, the largest, the lowest."""
+    x = np.random.default_rng(seed).integers(-(1 << 15), 1 << 15, shape)
+    x[:] = {"top": (1 << 15) - 1, "low": -(1 << 15)}.get(fill.split()[-1], x)
+    return np.where(x < 0, x.astype(np.uint64) + np.uint64(P), x.astype(np.uint64))
+
+
 def matmul(so):
     """Products through residues: every tile shape with remainders, one unit of the inner dimension and several, the largest sums of
     either sign, words at and above p, slices of the inner dimension."""
@@ -216,7 +223,8 @@ def matmul(so):
     L.simt_tile_workspace.restype, L.simt_tile_workspace.argtypes = SZ, [I64, ctypes.c_int]
     L.simt_tile.restype, L.simt_tile.argtypes = None, [VP, VP, VP, I64, I64, I64, ctypes.c_int, VP]
     for m, k, n, fill in ((1, 1, 1, None), (3, 17, 70, "any"), (64, 64, 64, "top"), (65, 100, 65, "half"), (130, 33, 130, None), (5, 8193, 3, "top"),
-                          (120, 70, 250, 4), (128, 64, 256, 4), (128, 130, 128, 2), (67, 5, 100, 2)):
+                          (120, 70, 250, 4), (128, 64, 256, 4), (128, 130, 128, 2), (67, 5, 100, 2),
+                          (3, 17, 70, "i16"), (64, 64, 128, "i16 top"), (65, 129, 130, "i16"), (5, 1030, 3, "i16 low"), (70, 65, 40, "over a"), (40, 130, 300, "over b")):
         print("matmul", m, k, n, fill, flush=True)
         A, B = field((m, k), m), field((k, n), n)
         if fill == "top":
@@ -224,6 +232,11 @@ def matmul(so):
         elif fill == "half":                                   # the words of largest size as signed numbers
             A[:], B[:] = 0x8080808080808080, 0x7F7F7F7F7F7F7F7F
             B[::2] += np.uint64(1)
+        elif isinstance(fill, str) and fill != "any":          # 16-bit signed numbers, the last word of A or B one beyond them
+            A[:] = small((m, k), 1, fill)
+            B[:] = small((k, n), 2, fill)
+            if fill.startswith("over"):
+                (A if fill == "over a" else B)[-1, -1] = (1 << 15) if fill == "over a" else P - (1 << 15) - 1
         elif fill == "any":
             A[:, ::3] = np.uint64((1 << 64) - 1) - A[:, ::3] % np.uint64(1 << 20)
             B[::2] = np.uint64((1 << 64) - 1) - B[::2] % np.uint64(1 << 33)

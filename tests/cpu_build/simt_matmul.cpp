@@ -1,4 +1,4 @@
-// Field products through residues (verinf_amd/csrc/matmul_rns.hip) on the CPU, launches and all.
+// Field products through residues (verinf_amd/csrc/matmul_rns.hip) and of small numbers (matmul_i16.hpp) on the CPU, launches and all.
 #include <hip/hip_runtime.h>
 #include "../../verinf_amd/csrc/matmul_rns.hip"
 
@@ -20,12 +20,13 @@ static void one_tile(const u64 *A, const u64 *B, u64 *C, i64 m, i64 k, i64 n, vo
         K.inv[i] = (u32)((1ull << 32) / (u32)MODS[i]);
         K.off[i] = (u32)MODS[i] * ((1u << 28) / (u32)MODS[i] + 1);
     }
-    const Operand OA = {A, k, m, mpad, Ap, (unsigned)((m + A_ROWS - 1) / A_ROWS)}, OB = {B, n, n, npad, Bp, (unsigned)((n + BLOCK - 1) / BLOCK)};
-    const unsigned a_blocks = OA.groups * (unsigned)(units / A_UNITS);
-    hipLaunchKernelGGL(k_residues, dim3(a_blocks + OB.groups * (unsigned)units), dim3(BLOCK), 0, nullptr, OA, OB, k, (int)units, a_blocks);
-    launch_gemm<2, WN, OCC>(Ap, Bp, Cp, (int)units, mpad, npad, K, nullptr);
+    const Operand OA = {A, k, m, mpad, Ap, (unsigned)((m + LINES - 1) / LINES)}, OB = {B, n, n, npad, Bp, (unsigned)((n + LINES - 1) / LINES)};
+    const unsigned chunks = (unsigned)(units / ITEM_UNITS), b_items = OB.groups * chunks;
+    const Cut D = {OA, OB, k, (int)units, b_items, b_items + OA.groups * chunks};
+    hipLaunchKernelGGL(k_residues, dim3(D.items), dim3(BLOCK), 0, nullptr, D, (const u32 *)nullptr);
+    launch_gemm<2, WN, OCC>(Ap, Bp, Cp, (int)units, mpad, npad, K, nullptr, nullptr);
     hipLaunchKernelGGL(k_from_residues, dim3((unsigned)((n + BLOCK - 1) / BLOCK), (unsigned)((m + 3) / 4)), dim3(BLOCK), 0, nullptr, (const u32 *)Cp,
-                       mpad / 4 * npad, npad, C, n, m, n, 0);
+                       mpad / 4 * npad, npad, C, n, m, n, 0, i16::Job{});
 }
 extern "C" size_t simt_tile_workspace(int64_t k, int wn) {
     return NMOD * (size_t)(round_up(k, STEP_UNITS * UNIT) * (128 + 64 * wn) + 128 * 64 * wn) + vi::WS_SLACK;

@@ -52,3 +52,28 @@ def test_scratch_of_any_alignment(skip):
     _lib.check(L.vi_gl_matmul(dA.data_ptr(), dB.data_ptr(), C.data_ptr(), m, k, n, ws.data_ptr() + skip, need, _lib.stream_ptr()))
     assert np.array_equal(to_np(C), (A.astype(object).dot(B.astype(object)) % P).astype(np.uint64))
     assert bool((ws[:skip] == 0x5A).all()) and bool((ws[need + skip:] == 0x5A).all())
+
+
+# 16-bit signed numbers: tiles of 64 x 128 and 128 x 128 with remainders, steps and slices of the inner dimension with remainders,
+# the largest sums, one word of A or B a step beyond the range (then the residues do the product)
+@pytest.mark.parametrize("m,k,n", [(40, 64, 3000), (64, 1000, 3001), (65, 1023, 2999), (129, 700, 4097), (1025, 65, 4300), (300, 9000, 500),
+                                   (128, 8192, 128), (100, 32768, 70), (100, 32769, 70)])
+@pytest.mark.parametrize("fill", ["any", "top", "low", "over a", "over b"])
+def test_matmul_of_small_numbers(m, k, n, fill):
+    from verinf_amd.prover import cuda_primitives as cp
+    rng = np.random.default_rng(m)
+    lo, hi = {"top": ((1 << 15) - 1, 1 << 15), "low": (-(1 << 15), 1 - (1 << 15))}.get(fill, (-(1 << 15), 1 << 15))
+    A, B = rng.integers(lo, hi, (m, k)), rng.integers(lo, hi, (k, n))
+    if fill == "over a":
+        A[-1, -1] = 1 << 15
+    if fill == "over b":
+        B[-1, -1] = -(1 << 15) - 1
+    dA, dB = (to_dev(np.where(x < 0, x.astype(np.uint64) + np.uint64(P), x.astype(np.uint64))) for x in (A, B))
+    print(m, k, n, fill, flush=True)
+    got = to_np(cp.gl_matmul(dA, dB))
+    rows = sorted({0, m // 2, m - 1, min(m - 1, 63)})
+    want = A[rows] @ B                                          # below 2^45
+    assert np.array_equal(got[rows], np.where(want < 0, want.astype(np.uint64) + np.uint64(P), want.astype(np.uint64)))
+    ones = to_np(cp.gl_matmul(dA, to_dev(np.ones((k, 300), dtype=np.uint64))))[:, 299]        # every row
+    want = A.sum(axis=1)
+    assert np.array_equal(ones, np.where(want < 0, want.astype(np.uint64) + np.uint64(P), want.astype(np.uint64)))

@@ -7,12 +7,15 @@
 // is a signed byte, so each residue is ONE int8 matrix product on v_mfma_i32_32x32x32_i8: 18 byte multiply-adds per
 // field multiply-add, where splitting both operands into bytes would take 64.
 //
-// What bounds it at 1000 x 4096 x 4096 (8240 us on the VALU, 470 here): the int8 products 346 us, 1.8 POP/s -- the matrix
-// cores are busy 43 % of the cycles and the LDS a third, neither at its limit: with two wavefronts to a SIMD (registers) the
-// barrier and the operand reads of a step are not covered by the other one's products; the residues 104 us, 0.44 GB at the
-// rate of a copy; the reconstruction 21 us.
+// What bounds it at 1000 x 4096 x 4096 (8240 us on the VALU, 440 here): the int8 products 334 us, 1.8 POP/s of the 2.9 to 3.5 that a
+// loop of nothing else holds on random bytes -- the matrix cores are busy 43 % of the cycles and the LDS a third, neither at its limit: with
+// two wavefronts to a SIMD (registers) the barrier and the operand reads of a step are not covered by the other one's products; the
+// residues 104 us, 0.44 GB at the rate of a copy; the reconstruction 21 us.
 //
-//   k_residues        words -> 18 planes of signed bytes
+// Operands that are 16-bit signed numbers take fewer byte products (matmul_i16.hpp): k_cut looks at them, k_product does their
+// product, and the kernels behind it leave at once when it is done.
+//
+//   k_cut, k_residues words -> 18 planes of signed bytes
 //   k_residue_gemm    per plane an int8 product; the 32-bit sums are reduced mod m_i to one byte
 //   k_from_residues   18 bytes -> the integer mod p
 //
@@ -31,6 +34,7 @@
 
 #include "common.hpp"
 #include "gl_field.hpp"
+#include "matmul_i16.hpp"
 
 namespace {
 
@@ -39,6 +43,7 @@ constexpr int NMOD = 18;
 constexpr int MODS[NMOD] = {256, 255, 253, 251, 247, 241, 239, 233, 229, 227, 223, 217, 211, 199, 197, 193, 191, 181};
 constexpr int MAX_K = 8192;                    // inner indices of one slice
 constexpr int UNIT = 16;                       // inner indices of a unit
+constexpr unsigned RESIDUE_BLOCKS = 768;       // workgroups of k_product where it makes residues: what is resident at once
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
@@ -124,58 +129,158 @@ __device__ __forceinline__ void store_all(const int (&lo)[UNIT], const int (&hi)
     (store_residues<I, CRT>(lo, hi, planes, plane, at), ...);
 }
 
-// Both operands in one launch; units of 16 inner indices from l0, zero beyond k.
-//
-// B: a workgroup takes 256 columns of one unit, lanes along the columns, so that the sixteen reads and the eighteen
-// 16-byte stores of a wavefront are contiguous.
-//
-// A: a workgroup takes 64 rows of four units.  Rows are read along the inner dimension (contiguous) into LDS and picked
-// up unit by unit with the lanes along the rows (an odd pitch in words: no bank conflicts), so that the stores are
-// contiguous here too; read by each lane from its own row, the launch took 37 us for 1000 x 4096 words, 15 this way.
-// The residues carry the factor of the remainder theorem, so that the sums of the products come out as its y_i.
-constexpr int A_ROWS = 64, A_UNITS = 4, A_PITCH = A_UNITS * UNIT + 1;
+// ---- cutting up the operands --------------------------------------------------------------------------------------
+// An item is four units (64 inner indices) of 64 rows of A or columns of B; a wavefront takes one unit, its lanes along the rows or
+// columns, so that the sixteen words that a lane reads of B and all stores are contiguous over the wavefront.  A is read along the
+// inner dimension into LDS for that and picked up with the lanes along the rows (an odd pitch in words: no bank conflicts); read by
+// each lane from its own row, 1000 x 4096 words took 37 us, 15 this way.  Inner indices from k to the padded length count as zeros.
+// The residues of A carry the factor of the remainder theorem, so that the sums of the products come out as its y_i.
+constexpr int ITEM_UNITS = 4, LINES = 64, TILE_PITCH = ITEM_UNITS * UNIT + 1;
 
 struct Operand {
     const u64 *src;                            // first word of the slice
     i64 ld, count, pitch;                      // row length in memory; rows of A or columns of B; the same padded
     v4i *planes;
-    unsigned groups;                           // workgroups along rows or columns
+    unsigned groups;                           // items along rows or columns
+};
+struct Cut {
+    Operand A, B;
+    i64 k;                                     // inner indices of the slice
+    int units;
+    unsigned b_items, items;                   // items of B (first), of both
 };
 
-__global__ __launch_bounds__(BLOCK) void k_residues(const Operand A, const Operand B, i64 k, int units, unsigned a_blocks) {
-    __shared__ u64 tile[A_ROWS * A_PITCH];
-    u64 w[UNIT];
-    const int tid = threadIdx.x;
-    const bool is_a = blockIdx.x < a_blocks;
-    i64 unit, at;
-    if (is_a) {
-        const i64 r0 = (i64)(blockIdx.x % A.groups) * A_ROWS, l0 = (i64)(blockIdx.x / A.groups) * (A_UNITS * UNIT);
+// the sixteen words that a thread holds of an item: of its own column of B, or of A in the order of memory
+__device__ __forceinline__ void load_item(const Cut &D, unsigned it, u64 (&w)[UNIT]) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const bool is_b = it < D.b_items;
+    const unsigned id = is_b ? it : it - D.b_items, groups = is_b ? D.B.groups : D.A.groups;
+    const i64 l0 = (i64)(id / groups) * (ITEM_UNITS * UNIT), first = (i64)(id % groups) * LINES;
+    if (is_b) {
+        const i64 l = l0 + wave * UNIT, at = first + lane;
+        const u64 *src = D.B.src + l * D.B.ld + at;
 #pragma unroll
-        for (int i = 0; i < A_ROWS * A_UNITS * UNIT / BLOCK; ++i) {
-            const int r = (tid >> 6) + i * (BLOCK / 64), l = tid & 63;
-            tile[r * A_PITCH + l] = (r0 + r < A.count && l0 + l < k) ? A.src[(r0 + r) * A.ld + l0 + l] : 0;
-        }
-        __syncthreads();
-        unit = (l0 / UNIT) + (tid >> 6);
-        at = r0 + (tid & 63);
-#pragma unroll
-        for (int u = 0; u < UNIT; ++u) w[u] = tile[(tid & 63) * A_PITCH + (tid >> 6) * UNIT + u];
-        if (at >= A.count) return;
+        for (int u = 0; u < UNIT; ++u) w[u] = at < D.B.count && l + u < D.k ? __builtin_nontemporal_load(&src[u * D.B.ld]) : 0;
     } else {
-        const unsigned id = blockIdx.x - a_blocks;
-        unit = id / B.groups;
-        at = (i64)(id % B.groups) * BLOCK + tid;
-        if (at >= B.count) return;
-        const u64 *src = B.src + unit * UNIT * B.ld + at;
+        const i64 l = l0 + lane;
+        const u64 *src = D.A.src + (first + wave) * D.A.ld + l;
 #pragma unroll
-        for (int u = 0; u < UNIT; ++u) w[u] = unit * UNIT + u < k ? __builtin_nontemporal_load(&src[u * B.ld]) : 0;
+        for (int i = 0; i < UNIT; ++i) w[i] = first + wave + 4 * i < D.A.count && l < D.k ? src[4 * i * D.A.ld] : 0;
     }
+}
+// words of an item of A -> those of the thread's own row
+__device__ __forceinline__ void turn_item(u64 (&w)[UNIT], u64 *tile) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    __syncthreads();                                       // the tile of the item before has been read
+#pragma unroll
+    for (int i = 0; i < UNIT; ++i) tile[(wave + 4 * i) * TILE_PITCH + lane] = w[i];
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < UNIT; ++u) w[u] = tile[lane * TILE_PITCH + wave * UNIT + u];
+}
+__device__ __forceinline__ void store_residues_of(const Cut &D, unsigned it, const u64 (&w)[UNIT]) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const bool is_b = it < D.b_items;
+    const Operand &S = is_b ? D.B : D.A;
+    const unsigned id = is_b ? it : it - D.b_items;
+    const i64 unit = (i64)(id / S.groups) * ITEM_UNITS + wave, at = (i64)(id % S.groups) * LINES + lane;
+    if (at >= S.count) return;
     int lo[UNIT], hi[UNIT];
 #pragma unroll
     for (int u = 0; u < UNIT; ++u) balanced_digits(w[u], lo[u], hi[u]);
     constexpr auto all = std::make_integer_sequence<int, NMOD>();
-    if (is_a) store_all<true>(lo, hi, A.planes, (i64)units * A.pitch, unit * A.pitch + at, all);
-    else store_all<false>(lo, hi, B.planes, (i64)units * B.pitch, unit * B.pitch + at, all);
+    if (is_b) store_all<false>(lo, hi, S.planes, (i64)D.units * S.pitch, unit * S.pitch + at, all);
+    else store_all<true>(lo, hi, S.planes, (i64)D.units * S.pitch, unit * S.pitch + at, all);
+}
+
+// residues of all items of a block, by a launch of any size
+__device__ __forceinline__ void residues(const Cut &D, u64 *tile) {
+    for (unsigned it = blockIdx.x; it < D.items; it += gridDim.x) {
+        u64 w[UNIT];
+        load_item(D, it, w);
+        if (it >= D.b_items) turn_item(w, tile);
+        store_residues_of(D, it, w);
+    }
+}
+// done: whether matmul_i16.hpp has finished the product (NULL: it was not tried)
+__global__ __launch_bounds__(BLOCK) void k_residues(const Cut D, const u32 *done) {
+    __shared__ u64 tile[LINES * TILE_PITCH];
+    if (done && *done) return;
+    residues(D, tile);
+}
+
+// The first launch of a product that matmul_i16.hpp may be able to do, as many workgroups as are resident at once: 31 us for the bytes of
+// 128 x 4096 x 4096 (a workgroup per item 39), 94 for its residues (84).  Products of arbitrary words pay that and k_product, which
+// then finds nothing to do: 128 x 4096 x 4096 167 -> 183 us, 100 x 760 x 1070 29 -> 33; from some 500 rows on the faster products outweigh it
+// (1000 x 4096 x 4096 470 -> 435).  256 words of either operand, the same for every workgroup,
+// decide whether to try (all words of 1000 x 4096 x 4096 read and cut up for nothing would be 37 us); the first item's words are on
+// their way behind them, and the next item's while this one's are cut up.  flags: 0 where all words of a workgroup's items fitted, 1
+// where one did not (the workgroup leaves), 2 if the sample says residues, which the launch then makes.
+// one_block: the product is one block of one slice, so that the items are those of the residues too; otherwise the sample's answer
+// is 1, and the next launch makes the residues of the first block.
+enum { FITS = 0, TOO_LARGE = 1, CUT_TO_RESIDUES = 2 };
+
+__global__ __launch_bounds__(BLOCK, 4) void k_cut(const Cut D, const i16::Job J, int one_block) {
+    __shared__ u64 tile[LINES * TILE_PITCH];
+    __shared__ int part[BLOCK];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    u64 w[UNIT];
+    u32 beyond = 0;
+    {
+        const i64 na = D.A.count * D.k, nb = D.k * D.B.count;
+        const i64 ea = tid * (na / BLOCK) + (na < BLOCK ? tid : 0), eb = tid * (nb / BLOCK) + (nb < BLOCK ? tid : 0);
+        const u64 wa = ea < na ? D.A.src[ea] : 0, wb = eb < nb ? D.B.src[eb] : 0;
+        load_item(D, blockIdx.x, w);
+        i16::signed_low(wa, beyond);
+        i16::signed_low(wb, beyond);
+    }
+    const bool small = !__syncthreads_or((int)beyond);
+    if (!small && !one_block) {
+        if (tid == 0) J.flags[blockIdx.x] = TOO_LARGE;
+        return;
+    }
+    for (unsigned it = blockIdx.x; it < D.items; it += gridDim.x) {
+        if (it >= D.b_items) turn_item(w, tile);
+        u64 now[UNIT];
+#pragma unroll
+        for (int u = 0; u < UNIT; ++u) now[u] = w[u];
+        if (it + gridDim.x < D.items) load_item(D, it + gridDim.x, w);
+        if (!small) {
+            store_residues_of(D, it, now);
+            continue;
+        }
+        const bool is_b = it < D.b_items;
+        const i16::Side &S = is_b ? J.B : J.A;
+        const unsigned id = is_b ? it : it - D.b_items, groups = is_b ? D.B.groups : D.A.groups;
+        const i64 chunk = id / groups, at = (i64)(id % groups) * LINES + lane;          // pitch: a multiple of LINES
+        part[tid] = i16::store_digits(now, S.planes + (chunk * ITEM_UNITS + wave) * S.pitch + at, (i64)D.units * S.pitch, beyond);
+        if (__syncthreads_or((int)beyond)) {
+            if (tid == 0) J.flags[blockIdx.x] = TOO_LARGE;
+            return;
+        }
+        if (tid < LINES) S.sums[chunk * S.pitch + at] = part[tid] + part[tid + 64] + part[tid + 128] + part[tid + 192];
+        __syncthreads();
+    }
+    if (tid == 0) J.flags[blockIdx.x] = small ? FITS : CUT_TO_RESIDUES;
+}
+
+// The launch behind k_cut: the product of 16-bit numbers; or the residues of the first block, where a word has turned out not to fit
+// after the sample did; or nothing.
+template <int MT, int NT>
+__global__ __launch_bounds__(BLOCK, 3) void k_product(const Cut D, const i16::Job J) {
+    __shared__ union {
+        i16::Lds<MT, NT> product;
+        u64 tile[LINES * TILE_PITCH];
+    } lds;
+    u32 seen = FITS;
+    for (int i = threadIdx.x; i < J.n_flags; i += BLOCK) seen |= J.flags[i];
+    const bool fits = !__syncthreads_or((int)seen), cut = __syncthreads_or((int)(seen & CUT_TO_RESIDUES));
+    if (blockIdx.x == 0 && threadIdx.x == 0) *J.done = fits;
+    if (!fits) {
+        if (!cut) residues(D, lds.tile);
+    } else if (blockIdx.x < (unsigned)(J.tiles * J.slices)) {
+        i16::product<MT, NT>(J, lds.product);
+    }
 }
 
 // ---- the int8 products ------------------------------------------------------------------------------------------
@@ -185,16 +290,17 @@ struct ModConst {
 };
 
 // One 64 WM x 64 WN tile of one plane per workgroup: four wavefronts in a 2 x 2 square, each WM x WN MFMA tiles of
-// 32 x 32.  BKU units of the inner dimension per step through two LDS buffers, the next step's global loads in
-// registers while the current one is multiplied.
+// 32 x 32.  BKU units of the inner dimension per step through two LDS buffers, the next step's loads going straight into the one
+// while the other is multiplied (through registers: 346 us at 1000 x 4096 x 4096, 334 this way; three buffers 375).
 template <int WM, int WN, int BKU, int OCC>
 __global__ __launch_bounds__(BLOCK, OCC) void k_residue_gemm(const v4i *__restrict__ Ap, const v4i *__restrict__ Bp, u32 *__restrict__ Cp,
-                                                             int units, i64 mpad, i64 npad, int mt, int nt, ModConst K) {
+                                                             int units, i64 mpad, i64 npad, int mt, int nt, ModConst K, const u32 *done) {
     constexpr int TM = 64 * WM, TN = 64 * WN;
-    constexpr int LA = BKU * TM / BLOCK, LB = BKU * TN / BLOCK;
+    constexpr int LOADS = BKU * (TM + TN) / BLOCK;                     // loads of 64 16-byte words of a step per wavefront
     __shared__ v4i As[2][BKU * TM];
     __shared__ v4i Bs[2][BKU * TN];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (done && *done) return;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // consecutive ids of one XCD take tiles that share their columns of B
     u32 id = blockIdx.x;
     const u32 total = gridDim.x;
@@ -204,24 +310,14 @@ __global__ __launch_bounds__(BLOCK, OCC) void k_residue_gemm(const v4i *__restri
     const v4i *a_src = Ap + (i64)mod * units * mpad + (i64)tm * TM;
     const v4i *b_src = Bp + (i64)mod * units * npad + (i64)tn * TN;
 
-    v4i ra[LA], rb[LB];
-    auto fetch = [&](int u0) {
+    // load j of the wavefront is chunk wave LOADS + j of a step: [A or B][unit][64 rows]
+    auto fetch = [&](int u0, int buf) {
 #pragma unroll
-        for (int i = 0; i < LA; ++i) {
-            const int c = tid + i * BLOCK;
-            ra[i] = a_src[(i64)(u0 + c / TM) * mpad + c % TM];
+        for (int j = 0; j < LOADS; ++j) {
+            const int c = wave * LOADS + j, ca = BKU * TM / 64, cb = c - ca;
+            if (c < ca) i16::fetch_to_lds(a_src + (i64)(u0 + c / (TM / 64)) * mpad + c % (TM / 64) * 64, &As[buf][c * 64], lane);
+            else i16::fetch_to_lds(b_src + (i64)(u0 + cb / (TN / 64)) * npad + cb % (TN / 64) * 64, &Bs[buf][cb * 64], lane);
         }
-#pragma unroll
-        for (int i = 0; i < LB; ++i) {
-            const int c = tid + i * BLOCK;
-            rb[i] = b_src[(i64)(u0 + c / TN) * npad + c % TN];
-        }
-    };
-    auto put = [&](int buf) {
-#pragma unroll
-        for (int i = 0; i < LA; ++i) As[buf][tid + i * BLOCK] = ra[i];
-#pragma unroll
-        for (int i = 0; i < LB; ++i) Bs[buf][tid + i * BLOCK] = rb[i];
     };
 
     v16i acc[WM][WN];
@@ -233,13 +329,11 @@ __global__ __launch_bounds__(BLOCK, OCC) void k_residue_gemm(const v4i *__restri
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
     const int row0 = (wave >> 1) * (32 * WM) + (lane & 31), col0 = (wave & 1) * (32 * WN) + (lane & 31), half = lane >> 5;
 
-    fetch(0);
-    put(0);
-    __syncthreads();
+    fetch(0, 0);
     int buf = 0;
     for (int u0 = 0; u0 < units; u0 += BKU, buf ^= 1) {
-        const bool more = u0 + BKU < units;
-        if (more) fetch(u0 + BKU);
+        i16::wait_and_meet();
+        if (u0 + BKU < units) fetch(u0 + BKU, buf ^ 1);
 #pragma unroll
         for (int s = 0; s < BKU / 2; ++s) {
             v4i a[WM], b[WN];
@@ -252,8 +346,6 @@ __global__ __launch_bounds__(BLOCK, OCC) void k_residue_gemm(const v4i *__restri
 #pragma unroll
                 for (int j = 0; j < WN; ++j) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[i], b[j], acc[i][j], 0, 0, 0);
         }
-        if (more) put(buf ^ 1);
-        __syncthreads();
     }
 
     // y = sum mod m in [0, m); register r of a tile is row 8 (r / 4) + 4 half + r % 4: four rows make a word of C's plane
@@ -295,8 +387,13 @@ __device__ __forceinline__ void crt_all(CrtSum (&S)[4], const u32 (&w)[NMOD], st
     ((crt_add<I>(S[0], w[I] & 0xFF), crt_add<I>(S[1], (w[I] >> 8) & 0xFF), crt_add<I>(S[2], (w[I] >> 16) & 0xFF), crt_add<I>(S[3], w[I] >> 24)), ...);
 }
 
-// Four rows of one column per thread: eighteen words in, four words of C out (added to what is there when `accumulate`).
-__global__ __launch_bounds__(BLOCK) void k_from_residues(const u32 *__restrict__ Cp, i64 plane, i64 npad, u64 *C, i64 ld, i64 m, i64 width, int accumulate) {
+// Four rows of one column per thread: eighteen words in, four words of C out (added to what is there when `accumulate`).  After a
+// product of 16-bit numbers in slices, J.slices > 1, the launch adds up the slices.
+__global__ __launch_bounds__(BLOCK) void k_from_residues(const u32 *__restrict__ Cp, i64 plane, i64 npad, u64 *C, i64 ld, i64 m, i64 width, int accumulate, const i16::Job J) {
+    if (J.done && *J.done) {
+        if (J.slices > 1) i16::add_slices(J, ((i64)blockIdx.y * gridDim.x + blockIdx.x) * BLOCK + threadIdx.x, (i64)gridDim.x * gridDim.y * BLOCK);
+        return;
+    }
     const i64 j = (i64)blockIdx.x * BLOCK + threadIdx.x, r4 = blockIdx.y;
     if (j >= width) return;
     u32 w[NMOD];
@@ -362,9 +459,9 @@ Plan make_plan(i64 m, i64 k, i64 n) {
 }
 
 template <int WM, int WN, int OCC>
-void launch_gemm(const v4i *A, const v4i *B, u32 *C, int units, i64 mpad, i64 npad, const ModConst &K, hipStream_t s) {
+void launch_gemm(const v4i *A, const v4i *B, u32 *C, int units, i64 mpad, i64 npad, const ModConst &K, const u32 *done, hipStream_t s) {
     const int mt = (int)(mpad / (64 * WM)), nt = (int)(npad / (64 * WN));
-    hipLaunchKernelGGL((k_residue_gemm<WM, WN, STEP_UNITS, OCC>), dim3((unsigned)(mt * nt * NMOD)), dim3(BLOCK), 0, s, A, B, C, units, mpad, npad, mt, nt, K);
+    hipLaunchKernelGGL((k_residue_gemm<WM, WN, STEP_UNITS, OCC>), dim3((unsigned)(mt * nt * NMOD)), dim3(BLOCK), 0, s, A, B, C, units, mpad, npad, mt, nt, K, done);
 }
 
 }  // namespace
@@ -382,40 +479,67 @@ bool rns_matmul_pays(int64_t m, int64_t k, int64_t n) {
 
 size_t rns_matmul_workspace_bytes(int64_t m, int64_t k, int64_t n) {
     const Plan L = make_plan(m, k, n);
-    return L.a_bytes + L.b_bytes + L.c_bytes + WS_SLACK;
+    const size_t own = L.a_bytes + L.b_bytes + L.c_bytes + i16::GATE_BYTES, small = i16::takes(m, k, n) ? i16::workspace_bytes(m, k, n) : 0;
+    return (own > small ? own : small) + WS_SLACK;
 }
 
 int rns_matmul(const uint64_t *A, const uint64_t *B, uint64_t *C, int64_t m, int64_t k, int64_t n, void *ws, hipStream_t s) {
     const Plan L = make_plan(m, k, n);
     ws = align16(ws);
-    v4i *Ap = (v4i *)ws, *Bp = (v4i *)((char *)ws + L.a_bytes);
-    u32 *Cp = (u32 *)((char *)ws + L.a_bytes + L.b_bytes);
+    // the planes of the residues lie over the bytes of k_cut: they are written when those are of no use
+    v4i *Ap = (v4i *)((char *)ws + i16::GATE_BYTES), *Bp = (v4i *)((char *)Ap + L.a_bytes);
+    u32 *Cp = (u32 *)((char *)Bp + L.b_bytes);
     ModConst K;
     for (int i = 0; i < NMOD; ++i) {
         K.m[i] = (u32)MODS[i];
         K.inv[i] = (u32)((1ull << 32) / (u32)MODS[i]);
         K.off[i] = (u32)MODS[i] * ((1u << 28) / (u32)MODS[i] + 1);
     }
+    auto cut = [&](i64 i0, i64 mb, i64 l0, i64 kc, i64 j0, i64 nb, bool with_a) {
+        Cut D;
+        D.A = {A + i0 * k + l0, (i64)k, mb, round_up(mb, 64 * L.wm), Ap, (unsigned)((mb + LINES - 1) / LINES)};
+        D.B = {B + l0 * n + j0, (i64)n, nb, round_up(nb, 64 * L.wn), Bp, (unsigned)((nb + LINES - 1) / LINES)};
+        D.k = kc;
+        D.units = (int)(round_up(kc, STEP_UNITS * UNIT) / UNIT);
+        const unsigned chunks = (unsigned)(D.units / ITEM_UNITS);
+        D.b_items = D.B.groups * chunks;
+        D.items = D.b_items + (with_a ? D.A.groups * chunks : 0);
+        return D;
+    };
+    i16::Job J = {};
+    const bool small = i16::takes(m, k, n);
+    if (small) {
+        J = i16::make_job(C, m, k, n, ws);
+        const Cut D = cut(0, m, 0, k, 0, n, true);
+        J.n_flags = (int)(D.items < i16::MAX_CUT_BLOCKS ? D.items : i16::MAX_CUT_BLOCKS);
+        hipLaunchKernelGGL(k_cut, dim3((unsigned)J.n_flags), dim3(BLOCK), 0, s, D, J, m == L.mb && k <= L.kc && n == L.nb ? 1 : 0);
+        VI_LAUNCH_CHECK("k_cut");
+    }
     for (i64 l0 = 0; l0 < k; l0 += L.kc) {
         const i64 kc = k - l0 < L.kc ? k - l0 : L.kc;
-        const i64 units = round_up(kc, STEP_UNITS * UNIT) / UNIT;
         for (i64 i0 = 0; i0 < m; i0 += L.mb) {
             const i64 mb = m - i0 < L.mb ? m - i0 : L.mb, mpad = round_up(mb, 64 * L.wm);
-            Operand OA = {A + i0 * k + l0, (i64)k, mb, mpad, Ap, (unsigned)((mb + A_ROWS - 1) / A_ROWS)};
             for (i64 j0 = 0; j0 < n; j0 += L.nb) {
                 const i64 nb = n - j0 < L.nb ? n - j0 : L.nb, npad = round_up(nb, 64 * L.wn);
-                const Operand OB = {B + l0 * n + j0, (i64)n, nb, npad, Bp, (unsigned)((nb + BLOCK - 1) / BLOCK)};
-                const unsigned a_blocks = j0 == 0 ? OA.groups * (unsigned)(units / A_UNITS) : 0;
-                hipLaunchKernelGGL(k_residues, dim3(a_blocks + OB.groups * (unsigned)units), dim3(BLOCK), 0, s, OA, OB, kc, (int)units, a_blocks);
-                VI_LAUNCH_CHECK("k_residues");
-                const int u = (int)units;
-                if (L.wn == 4) launch_gemm<2, 4, 2>(Ap, Bp, Cp, u, mpad, npad, K, s);
-                else if (L.wn == 2) launch_gemm<2, 2, 3>(Ap, Bp, Cp, u, mpad, npad, K, s);
-                else launch_gemm<1, 1, 4>(Ap, Bp, Cp, u, mpad, npad, K, s);
+                const Cut D = cut(i0, mb, l0, kc, j0, nb, j0 == 0);
+                if (small && l0 == 0 && i0 == 0 && j0 == 0) {
+                    const unsigned tiles = (unsigned)(J.tiles * J.slices), most = D.items < RESIDUE_BLOCKS ? D.items : RESIDUE_BLOCKS;
+                    const dim3 grid(tiles > most ? tiles : most);
+                    if (m <= 64) hipLaunchKernelGGL((k_product<1, 2>), grid, dim3(BLOCK), 0, s, D, J);
+                    else hipLaunchKernelGGL((k_product<2, 1>), grid, dim3(BLOCK), 0, s, D, J);
+                    VI_LAUNCH_CHECK("k_product");
+                } else {
+                    hipLaunchKernelGGL(k_residues, dim3(D.items), dim3(BLOCK), 0, s, D, (const u32 *)J.done);
+                    VI_LAUNCH_CHECK("k_residues");
+                }
+                if (L.wn == 4) launch_gemm<2, 4, 2>(Ap, Bp, Cp, D.units, mpad, npad, K, J.done, s);
+                else if (L.wn == 2) launch_gemm<2, 2, 3>(Ap, Bp, Cp, D.units, mpad, npad, K, J.done, s);
+                else launch_gemm<1, 1, 4>(Ap, Bp, Cp, D.units, mpad, npad, K, J.done, s);
                 VI_LAUNCH_CHECK("k_residue_gemm");
                 hipLaunchKernelGGL(k_from_residues, dim3((unsigned)((nb + BLOCK - 1) / BLOCK), (unsigned)((mb + 3) / 4)), dim3(BLOCK), 0, s, (const u32 *)Cp,
-                                   mpad / 4 * npad, npad, C + i0 * n + j0, (i64)n, mb, nb, l0 > 0 ? 1 : 0);
+                                   mpad / 4 * npad, npad, C + i0 * n + j0, (i64)n, mb, nb, l0 > 0 ? 1 : 0, J);
                 VI_LAUNCH_CHECK("k_from_residues");
+                J.slices = 1;                              // added up by the first of these launches
             }
         }
     }
