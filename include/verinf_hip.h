@@ -247,9 +247,9 @@ int vi_sumcheck_prove(const uint64_t *const *tables, uint64_t *const *work, int 
  * calls `coin(rnd)` with the round number only (layergkr/gpu.py:403, layergkr/sumcheck.py:217) and its callers draw
  * the coins before the proof starts (layergkr/full_layer.py:222-224, layergkr/relations.py:122-123,
  * layergkr/layer.py:123-125).  All rounds are queued on the stream without a host round trip, and the call returns
- * without waiting.  A single product of up to four distinct tables and the hadamard gate batch eq * (a * b + c' * c)
- * run three rounds per pass over the tables and every round of the last few thousand entries in one workgroup; other
- * sums keep one launch per round.
+ * without waiting.  A single product of up to four distinct tables, the hadamard gate batch eq * (a * b + c' * c) and
+ * sums of products of two tables and single tables under a common factor run three rounds per pass over the tables;
+ * other sums keep one launch per round.
  *   challenges    host, v = log2(size) words (reduced mod p by the callee)
  *   samples       v rows of 8 words the GPU can write (device memory or pinned host memory): S_round(x) at
  *                 samples[8 * round + x], x = 0..deg, complete once the stream has reached the end of the call's work

@@ -674,3 +674,41 @@ def _lagrange_at(ys, r):
 def cp_mul(x, y):
     from verinf_amd.prover import cuda_primitives as cp
     return cp.gl_mul(x, y)
+
+
+# Sums under a common factor, table 0: products alone, single tables alone (degree 2), both; a constant (the common factor by itself);
+# a table in several products, in a product and by itself, squared; the common factor inside a product and by itself squared; more
+# single tables than the rows of a pass take at four each; coefficients 0.  Sizes: fewer entries than lanes, one to eight to a lane, one
+# to three passes with every remainder.
+_SUM_FORMS = {
+    "products": [(3, [0, 1, 2]), (5, [0, 3, 4])],
+    "singles": [(3, [0, 1]), (P - 7, [2, 0]), (11, [0, 3])],
+    "constant": [(3, [0, 1]), (P - 2, [0])],
+    "mixed": [(3, [0, 1, 2]), (P - 3, [0, 3]), (9, [4, 0]), (P - 9, [5, 0]), (6, [0, 6, 6]), (P - 6, [0, 6]), (4, [0])],
+    "shared": [(3, [0, 1, 2]), (5, [1, 0, 3]), (7, [2, 3, 0]), (8, [0, 1]), (0, [0, 4]), (0, [0, 1, 4])],
+    "common twice": [(3, [0, 0, 1]), (5, [0, 0]), (2, [1, 2, 0])],
+    "many": [(k + 1, [0, k % 37 + 1]) for k in range(90)] + [(k + 2, [0, k + 1, k + 38]) for k in range(20)],
+}
+
+
+@pytest.mark.parametrize("form", list(_SUM_FORMS))
+@pytest.mark.parametrize("v", [1, 2, 5, 6, 7, 8, 9, 10, 11, 12, 13, 16])
+def test_sums_under_a_common_factor(mods, form, v):
+    gpu, _ = mods
+    terms = _SUM_FORMS[form]
+    n = 1 + max(max(fs) for _, fs in terms)
+    if v == 16 and n > 30:
+        v = 14                                                 # the oracle's time
+    tabs = [rand_field(1 << v, 3000 + 100 * v + t) for t in range(n)]
+    tabs[1][-1], tabs[-1][0] = P - 1, 0
+    raw = [t.copy() for t in tabs]
+    raw[0][0], raw[1][0] = np.uint64(2**64 - 1), np.uint64(P + 1)              # caller words at and above p
+    tabs[0][0], tabs[1][0] = (2**64 - 1) % P, 1
+    coins, _ = _coins(v, 70 + v)
+    print(form, v, flush=True)
+    dev = [to_dev(t) for t in raw]
+    claim, polys, _, _ = gpu.prove_terms_gpu([(c, [dev[i] for i in fs]) for c, fs in terms], lambda i: coins[i], P)
+    want_claim, want_samples, _ = O.sumcheck_prove(tabs, terms, coins)
+    assert claim == want_claim and [[y for _, y in s] for s in polys] == want_samples
+    for t, d in zip(raw, dev):
+        assert np.array_equal(to_np(d), t), "caller's table was modified"

@@ -1263,6 +1263,7 @@ int vi_sumcheck_prove(const uint64_t *const *tables, uint64_t *const *work, int 
 }  // extern "C"
 
 #include "sumcheck_fast.hpp"
+#include "sumcheck_sum.hpp"
 
 namespace {
 
@@ -1583,6 +1584,14 @@ int prove_coins_impl(const char *who, const uint64_t *const *tables, uint64_t *c
     C.n_prior = v;
     C.deg = deg;
 
+    // products of two tables and single tables under a common factor: three rounds per pass (the hadamard gate batch of four tables
+    // has kernels of its own)
+    {
+        SumShape S;
+        if (sum_shape(n_tables, term_off, factor_idx, coeffs, n_terms, S) &&
+            !(n_tables == 4 && S.products.size() == 1 && S.singles.size() == 1 && S.c0 == 0))
+            return prove_sum(S, tables, work, size, C, part, samples, s);
+    }
     // many terms that are a single table under the common factor: from round 1 on they are one table (needs a round
     // to fold into, so at least two rounds)
     if (may_reduce && v >= 2) {

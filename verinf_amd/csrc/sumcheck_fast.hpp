@@ -18,8 +18,9 @@
 //
 // Shapes with their own unrolled evaluation (the ones the layer proof consists of): a single product of up to
 // four distinct tables (a matmul contraction, eq * a * b, the three-factor benchmark instance) and the hadamard
-// gate batch eq * (a * b + c' * c).  Other sums keep one launch per round (k_round / k_eval_mem) but are queued
-// back to back in the same way and finished by k_finish.
+// gate batch eq * (a * b + c' * c).  Sums of products of two tables and single tables under a common factor have passes of three rounds
+// too (sumcheck_sum.hpp).  Other sums keep one launch per round (k_round / k_eval_mem) but are queued back to back in the same way
+// and finished by k_finish.
 #pragma once
 
 namespace {
@@ -53,21 +54,44 @@ struct FinishShared {
     u64 claim[MAX_ROUNDS + 1];
 };
 
-// Lagrange basis at the challenges (one thread per round) and the sums of the partials the earlier launches left
+// The sums over the wavefront of N values per lane: a step adds the halves of the lanes and halves the values, each half of the
+// lanes going on with its own (N / 2 + N / 4 + ... shuffles instead of 6 N; a pass over few entries 14.9 -> 11.2 us).  Returns one total per lane; slot: whose, -1 for none.
+template <int N>
+__device__ __forceinline__ u64 wave_totals(u64 (&v)[N], int off, int &slot) {
+    const int lane = threadIdx.x & 63;
+    if constexpr (N == 1) {
+        u64 s = v[0];
+        for (; off > 0; off >>= 1) s = gl::addc(s, __shfl_xor(s, off, 64));
+        slot = 0;
+        return s;
+    } else {
+        constexpr int H = (N + 1) / 2;
+        const bool upper = (lane & off) != 0;
+        u64 half[H];
+#pragma unroll
+        for (int i = 0; i < H; ++i) {
+            const u64 lo = v[i], hi = i + H < N ? v[i + H] : 0;
+            const u64 keep = upper ? hi : lo, give = upper ? lo : hi;
+            half[i] = gl::addc(keep, __shfl_xor(give, off, 64));
+        }
+        const u64 s = wave_totals<H>(half, off >> 1, slot);
+        if (slot >= 0 && upper) slot = slot + H < N ? slot + H : -1;
+        return s;
+    }
+}
+
+// Lagrange basis at the challenges (one thread per round and point) and the sums of the partials the earlier launches left
 // (one wavefront per round).  The caller synchronises the workgroup before finish_samples().
 __device__ __forceinline__ void finish_begin(const ChainDesc &C, const u64 *part, FinishShared &sh) {
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, nw = blockDim.x >> 6;
-    if (tid < C.n_rounds) {
-        const u64 r = C.r[tid];
-#pragma unroll
-        for (int x = 0; x < NSAMP; ++x) {
-            if (x <= C.deg) {
-                u64 num = C.winv[x];
-#pragma unroll
-                for (int j = 0; j < NSAMP; ++j)
-                    if (j <= C.deg && j != x) num = gl::mul(num, gl::sub(r, (u64)j));
-                sh.lag[tid][x] = num;
-            }
+    for (int e = tid; e < C.n_rounds * NSAMP; e += blockDim.x) {
+        const int k = e / NSAMP, x = e % NSAMP;
+        if (x <= C.deg) {
+            const u64 r = C.r[k];
+            u64 num = C.winv[x];
+            for (int j = 0; j <= C.deg; ++j)
+                if (j != x) num = gl::mul(num, gl::sub(r, (u64)j));
+            sh.lag[k][x] = num;
         }
     }
     for (int k = w; k < C.n_prior; k += nw) {
@@ -91,13 +115,9 @@ __device__ __forceinline__ void finish_begin(const ChainDesc &C, const u64 *part
                 for (int x = 0; x < NSAMP; ++x)
                     if (x <= C.deg) v[x] = gl::addc(v[x], t[u][x]);
         }
-#pragma unroll
-        for (int x = 0; x < NSAMP; ++x) {
-            if (x <= C.deg) {
-                const u64 sum = wave_sum(v[x]);
-                if (lane == 0) sh.raw[k][x] = sum;
-            }
-        }
+        int slot;
+        const u64 sum = wave_totals<NSAMP>(v, 32, slot);
+        if (slot >= 0 && slot <= C.deg) sh.raw[k][slot] = sum;
     }
 }
 
@@ -194,9 +214,10 @@ struct FastDesc {
     u64 lin_coeff;
 };
 
+// SHAPE 3: the product of two tables as part of a sum of degree 3: S(2) is taken as well, the leading coefficient is 0.
 template <int NT, int SHAPE>
 struct FastShape {
-    static constexpr int NS = SHAPE == 2 ? 4 : NT + 1;
+    static constexpr int NS = SHAPE >= 2 ? 4 : NT + 1;
     // degree >= 2: the last slot takes the leading coefficient instead of S(deg) (ChainDesc::inf_node)
     static constexpr bool INF = NS >= 3;
 };
@@ -242,6 +263,8 @@ __device__ __forceinline__ void eval_pair(const u64 (&lo)[NT], const u64 (&hi)[N
                 // eq (a b + c): the c term has degree 2 and does not reach the leading coefficient
                 if (at_inf) acc[x].add_product(gl::mul_lazy(dif[1], dif[2]), dif[0]);
                 else acc[x].add_product(gl::mul_add_lazy(cur[1], cur[2], cur[3]), cur[0]);
+            } else if constexpr (SHAPE == 3) {
+                if (!at_inf) acc[x].add_product(cur[0], cur[1]);
             } else if constexpr (NT == 1) {
                 acc[x].add_product(cur[0], 1);
             } else {
@@ -301,6 +324,64 @@ __device__ __forceinline__ void block_sum_rows(const u64 *rows, int n_rows, u64 
     __syncthreads();
 }
 
+// a pass's sums of its three rounds over the workgroup, times scale -> row at `row`, region_words apart
+template <int NS>
+__device__ __forceinline__ void pass_sums(const SampleAcc<true> (&acc0)[NS], const SampleAcc<true> (&acc1)[NS], const SampleAcc<true> (&acc2)[NS],
+                                          u64 (*red)[3 * NS], u64 *row, i64 region_words, u64 scale) {
+    u64 v[3 * NS];
+#pragma unroll
+    for (int x = 0; x < NS; ++x) {
+        v[x] = acc0[x].value();
+        v[NS + x] = acc1[x].value();
+        v[2 * NS + x] = acc2[x].value();
+    }
+    int slot;
+    const u64 sum = wave_totals<3 * NS>(v, 32, slot);
+    if (slot >= 0) red[threadIdx.x >> 6][slot] = sum;
+    __syncthreads();
+    if (threadIdx.x < 3 * NS) {
+        u64 s = red[0][threadIdx.x];
+#pragma unroll
+        for (int w = 1; w < BLOCK / 64; ++w) s = gl::addc(s, red[w][threadIdx.x]);
+        if (scale != 1) s = gl::mul(s, scale);
+        row[threadIdx.x / NS * region_words + threadIdx.x % NS] = s;
+    }
+}
+
+// Three rounds on eight entries of every table, v[t][c] = entry i + c cols (canonical): the samples of the seven pairs into the rounds'
+// accumulators, the entry folded three times into `folded`.  FIRST: the first round sums S(1) too.
+template <int NT, int SHAPE, bool FIRST>
+__device__ __forceinline__ void three_rounds(u64 (&v)[NT][8], u64 r0, u64 r1, u64 r2, SampleAcc<true> (&acc0)[FastShape<NT, SHAPE>::NS],
+                                             SampleAcc<true> (&acc1)[FastShape<NT, SHAPE>::NS], SampleAcc<true> (&acc2)[FastShape<NT, SHAPE>::NS],
+                                             u64 (&folded)[NT]) {
+    // the scheduler is kept from interleaving the pairs: each one's temporaries die before the next starts
+    u64 lo[NT], hi[NT], dif[NT];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        VI_SCHED_FENCE();
+#pragma unroll
+        for (int t = 0; t < NT; ++t) { lo[t] = v[t][c]; hi[t] = v[t][c + 4]; }
+        eval_pair<NT, SHAPE, !FIRST, true>(lo, hi, dif, acc0);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) v[t][c] = gl::mul_add(r0, dif[t], lo[t]);
+    }
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        VI_SCHED_FENCE();
+#pragma unroll
+        for (int t = 0; t < NT; ++t) { lo[t] = v[t][c]; hi[t] = v[t][c + 2]; }
+        eval_pair<NT, SHAPE, true, true>(lo, hi, dif, acc1);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) v[t][c] = gl::mul_add(r1, dif[t], lo[t]);
+    }
+    VI_SCHED_FENCE();
+#pragma unroll
+    for (int t = 0; t < NT; ++t) { lo[t] = v[t][0]; hi[t] = v[t][1]; }
+    eval_pair<NT, SHAPE, true, true>(lo, hi, dif, acc2);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) folded[t] = gl::mul_add(r2, dif[t], lo[t]);
+}
+
 // Three rounds in one pass.  cols = n / 8 for tables of n words; thread i < cols owns entries i + c cols.
 // FIRST: the tables are the caller's (words reduced on load, round 0 sums every sample).
 // part: three regions of gridDim.x rows of NSAMP words, one per round.
@@ -311,7 +392,7 @@ template <int NT, int SHAPE, bool FIRST>
 __global__ __launch_bounds__(BLOCK) void k_pass3(const FastDesc D, i64 cols, u64 r0, u64 r1, u64 r2, u64 *part,
                                                  const u64 *prev_part, int prev_rows, u64 *prev_sums) {
     constexpr int NS = FastShape<NT, SHAPE>::NS;
-    __shared__ u64 red[BLOCK / 64][3][NS];
+    __shared__ u64 red[BLOCK / 64][3 * NS];
     __shared__ u64 red_prev[BLOCK / 64][NSAMP];
     if (prev_rows > 0 && blockIdx.x < 3)
         block_sum_rows<NS>(prev_part + (i64)blockIdx.x * prev_rows * NSAMP, prev_rows, prev_sums + blockIdx.x * NSAMP, red_prev);
@@ -337,46 +418,12 @@ __global__ __launch_bounds__(BLOCK) void k_pass3(const FastDesc D, i64 cols, u64
                     }
                 }
         }
-        // the scheduler is kept from interleaving the pairs: each one's temporaries die before the next starts
-        u64 lo[NT], hi[NT], dif[NT];
+        u64 folded[NT];
+        three_rounds<NT, SHAPE, FIRST>(v, r0, r1, r2, acc0, acc1, acc2, folded);
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            VI_SCHED_FENCE();
-#pragma unroll
-            for (int t = 0; t < NT; ++t) { lo[t] = v[t][c]; hi[t] = v[t][c + 4]; }
-            eval_pair<NT, SHAPE, !FIRST, true>(lo, hi, dif, acc0);
-#pragma unroll
-            for (int t = 0; t < NT; ++t) v[t][c] = gl::mul_add(r0, dif[t], lo[t]);
-        }
-#pragma unroll
-        for (int c = 0; c < 2; ++c) {
-            VI_SCHED_FENCE();
-#pragma unroll
-            for (int t = 0; t < NT; ++t) { lo[t] = v[t][c]; hi[t] = v[t][c + 2]; }
-            eval_pair<NT, SHAPE, true, true>(lo, hi, dif, acc1);
-#pragma unroll
-            for (int t = 0; t < NT; ++t) v[t][c] = gl::mul_add(r1, dif[t], lo[t]);
-        }
-        VI_SCHED_FENCE();
-#pragma unroll
-        for (int t = 0; t < NT; ++t) { lo[t] = v[t][0]; hi[t] = v[t][1]; }
-        eval_pair<NT, SHAPE, true, true>(lo, hi, dif, acc2);
-#pragma unroll
-        for (int t = 0; t < NT; ++t) D.dst[t][i] = gl::mul_add(r2, dif[t], lo[t]);
+        for (int t = 0; t < NT; ++t) D.dst[t][i] = folded[t];
     }
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-#pragma unroll
-    for (int x = 0; x < NS; ++x) {
-        const u64 s0 = wave_sum(acc0[x].value()), s1 = wave_sum(acc1[x].value()), s2 = wave_sum(acc2[x].value());
-        if (lane == 0) { red[w][0][x] = s0; red[w][1][x] = s1; red[w][2][x] = s2; }
-    }
-    __syncthreads();
-    if (threadIdx.x < 3 * NS) {
-        const int j = threadIdx.x / NS, x = threadIdx.x % NS;
-        u64 s = red[0][j][x];
-        for (int i = 1; i < BLOCK / 64; ++i) s = gl::addc(s, red[i][j][x]);
-        part[((i64)j * gridDim.x + blockIdx.x) * NSAMP + x] = s;
-    }
+    pass_sums<NS>(acc0, acc1, acc2, red, part + (i64)blockIdx.x * NSAMP, (i64)gridDim.x * NSAMP, 1);
 }
 
 // pairs per table a tail workgroup holds after its first fold
