@@ -150,3 +150,21 @@ def test_scratch_of_any_alignment(n_table, skip):
     _lib.check(L.vi_lookup_histogram(dx.data_ptr(), len(x), dt.data_ptr(), n_table, 0, 0, mult.data_ptr(), ws.data_ptr() + skip, need, _lib.stream_ptr()))
     assert np.array_equal(to_np(mult), _counts(x, table))
     assert bool((ws[:skip] == 0x5A).all()) and bool((ws[need + skip:] == 0x5A).all())
+
+
+@pytest.mark.parametrize("n_x,n_table", [(131073, 8192), (140001, 8193), (300001, 65535), (1500001, 65536), (140001, 65537), (400000, 131073),
+                                         (256 * 65535, 65536), (256 * 65535 + 1, 65536)])
+@pytest.mark.parametrize("kind", ["range", "one entry", "other"])
+def test_counters_of_16_bits(n_x, n_table, kind):
+    """Tables from 8192 entries on: one and two slices, odd lengths, up to as many look-ups of one entry as such a counter holds."""
+    from verinf_amd.prover import cuda_primitives as cp
+    rng = np.random.default_rng(n_x + n_table)
+    at = rng.integers(0, n_table, n_x)
+    at[:n_x if kind == "one entry" else n_x // 3] = n_table - 1
+    table = np.arange(n_table, dtype=np.uint64)
+    if kind == "other":
+        table = table * np.uint64(0x9E3779B97F4A7C15)          # different, as the factor is odd
+    print(n_x, n_table, kind, flush=True)
+    x = table[at]
+    got = to_np(cp.lookup_multiplicities(to_dev(x), to_dev(table)))
+    assert np.array_equal(got, np.bincount(at, minlength=n_table).astype(np.uint64))

@@ -12,6 +12,8 @@
 // (k_survey), whose findings the counting workgroups read.  us per call in a queue of them, 1.5 M look-ups: 10 in 2^6 entries,
 // 12.0 in 2^12, 21.0 in 2^16, 51 in 2^20 (19.0 and 48 for the last two when the caller promises a range); 10^6 look-ups in 3003
 // values 12.6, in 40000 36.
+#include <algorithm>
+
 #include "common.hpp"
 #include "gl_field.hpp"
 
@@ -21,6 +23,7 @@ constexpr int BLOCK = 256;
 constexpr int COUNT_THREADS = 1024;
 constexpr int SLICE = 32768;                   // counters of a workgroup: 128 KiB of LDS
 constexpr int MAX_COPIES = 32;
+constexpr i64 MAX_HALF = 0xFFFF;               // look-ups of a group that counts in 16 bits
 constexpr i64 MAX_GROUPS = 256;                // rows of the workspace per slice
 constexpr u32 EMPTY = 0xFFFFFFFFu;
 constexpr i64 MAX_HASHED = (i64)1 << 30;       // entries of a hash table
@@ -134,20 +137,35 @@ __device__ __forceinline__ u64 index_of(u64 x, const Finder &F, bool diagonal, b
 }
 
 // counts of the entries base .. base + mine - 1 among x[lo .. hi - 1], each at(value) an index of the table; `copies` (a power
-// of two) interleaved counters per entry
-template <class F>
+// of two) interleaved counters per entry.  HALF: counters of 16 bits, two to a word, one copy.
+template <bool HALF, class F>
 __device__ __forceinline__ void count(const u64 *__restrict__ x, i64 lo, i64 hi, u64 base, int mine, int copies, u32 *counts, F at) {
     const int copy = threadIdx.x & (copies - 1);
-    constexpr int UN = 4;                      // look-ups of a thread in flight
+    constexpr int UN = HALF ? 8 : 4;           // look-ups of a thread in flight
     for (i64 i0 = lo + threadIdx.x; i0 < hi; i0 += UN * COUNT_THREADS) {
         u64 v[UN];
 #pragma unroll
         for (int u = 0; u < UN; ++u) v[u] = i0 + u * COUNT_THREADS < hi ? x[i0 + u * COUNT_THREADS] : 0;
+        u32 times[UN];
+#pragma unroll
+        for (int u = 0; u < UN; ++u) times[u] = i0 + u * COUNT_THREADS < hi ? 1 : 0;
+        if (HALF) {
+            // without copies a value that many look-ups share would queue up: those of the thread that equal its first go as one
+            // (1.5 M look-ups of one entry of 2^16: 34.5 us without this, 17.1 with it, 27.1 with 32-bit counters)
+#pragma unroll
+            for (int u = 1; u < UN; ++u) {
+                const bool same = v[u] == v[0];
+                times[0] += same ? times[u] : 0;
+                times[u] = same ? 0 : times[u];
+            }
+        }
 #pragma unroll
         for (int u = 0; u < UN; ++u) {
-            if (i0 + u * COUNT_THREADS < hi) {
+            if (times[u]) {
                 const u64 j = at(v[u]) - base;
-                if (j < (u64)mine) atomicAdd(&counts[(int)j * copies + copy], 1u);
+                if (j >= (u64)mine) continue;
+                if (HALF) atomicAdd(&counts[(int)j >> 1], times[u] << (16 * ((int)j & 1)));
+                else atomicAdd(&counts[(int)j * copies + copy], 1u);
             }
         }
     }
@@ -176,24 +194,37 @@ __device__ __forceinline__ void put_counts(const u32 *counts, int mine, int copi
 }
 
 // Workgroup (slice, group): counts of the entries slice * SLICE .. of the group's share of x.  rows: the group's row of n_table
-// counts, or null when there is one group: the counts go straight to mult.
+// counts, or null when there is one group: the counts go straight to mult.  HALF: slices of 2 SLICE entries and rows of 16-bit counts, an
+// even number of them; there is more than one group, and none has more than MAX_HALF look-ups.
+// Over a range only the first range_groups groups count, with a larger share each.
+template <bool HALF>
 __global__ __launch_bounds__(COUNT_THREADS) void k_count(const u64 *__restrict__ x, i64 n_x, i64 per_group, const Finder F, int copies, u32 *rows,
-                                                         u64 *mult, int accumulate) {
+                                                         u64 *mult, int accumulate, int range_groups) {
     extern __shared__ uint4 lds_counts[];
     u32 *counts = reinterpret_cast<u32 *>(lds_counts);
-    const i64 base = (i64)blockIdx.x * SLICE, group = blockIdx.y;
-    const int mine = F.n_table - base < SLICE ? (int)(F.n_table - base) : SLICE;
+    constexpr int MOST = HALF ? 2 * SLICE : SLICE;
+    const i64 base = (i64)blockIdx.x * MOST, group = blockIdx.y;
+    const int mine = F.n_table - base < MOST ? (int)(F.n_table - base) : MOST, words = HALF ? (mine + 1) / 2 : mine * copies;
     const u32 part = found_part(F);
     // the launch's LDS is a whole number of 16-byte words
-    for (int i = threadIdx.x; i < (mine * copies + 3) / 4; i += COUNT_THREADS) lds_counts[i] = make_uint4(0, 0, 0, 0);
+    for (int i = threadIdx.x; i < (words + 3) / 4; i += COUNT_THREADS) lds_counts[i] = make_uint4(0, 0, 0, 0);
     const bool range = !found_any(part, OFF);  // a barrier as well
+    if (HALF && range) {
+        if (group >= range_groups) return;
+        per_group = (n_x + range_groups - 1) / range_groups;
+    }
     const i64 lo = group * per_group, hi = lo + per_group < n_x ? lo + per_group : n_x;
-    if (range) count(x, lo, hi, (u64)base, mine, copies, counts, [](u64 v) { return v; });
+    if (range) count<HALF>(x, lo, hi, (u64)base, mine, copies, counts, [](u64 v) { return v; });
     else {
         const bool diagonal = found_any(part, DIAGONAL), search = found_any(part, LOST) || F.bits == 0;
-        count(x, lo, hi, (u64)base, mine, copies, counts, [&](u64 v) { return index_of(v, F, diagonal, search); });
+        count<HALF>(x, lo, hi, (u64)base, mine, copies, counts, [&](u64 v) { return index_of(v, F, diagonal, search); });
     }
     __syncthreads();
+    if (HALF) {
+        const i64 row_words = (F.n_table + 1) / 2;
+        put_counts(counts, words, 1, rows + group * row_words + base / 2, (row_words & 3) == 0, nullptr, 0);
+        return;
+    }
     put_counts(counts, mine, copies, rows ? rows + group * F.n_table + base : nullptr, (F.n_table & 3) == 0, mult + base, accumulate);
 }
 
@@ -218,7 +249,7 @@ __global__ __launch_bounds__(COUNT_THREADS) void k_count_small(const u64 *__rest
     for (int i = tid; i < n_slots; i += COUNT_THREADS) index[i] = EMPTY;
     odd = __syncthreads_or(odd);
     const i64 group = blockIdx.x, lo = group * per_group, hi = lo + per_group < n_x ? lo + per_group : n_x;
-    if (!odd) count(x, lo, hi, 0, n_table, copies, counts, [](u64 v) { return v; });
+    if (!odd) count<false>(x, lo, hi, 0, n_table, copies, counts, [](u64 v) { return v; });
     else {
         for (int j = tid; j < n_table; j += COUNT_THREADS) {
             const u64 key = keys[j];
@@ -233,7 +264,7 @@ __global__ __launch_bounds__(COUNT_THREADS) void k_count_small(const u64 *__rest
             }
         }
         __syncthreads();
-        count(x, lo, hi, 0, n_table, copies, counts, [&](u64 v) -> u64 {
+        count<false>(x, lo, hi, 0, n_table, copies, counts, [&](u64 v) -> u64 {
             u32 h = slot_of(v, bits);
             for (int probes = 0; probes < n_slots; ++probes, h = (h + 1) & (n_slots - 1)) {
                 const u32 at = index[h];
@@ -247,30 +278,41 @@ __global__ __launch_bounds__(COUNT_THREADS) void k_count_small(const u64 *__rest
     put_counts(counts, n_table, copies, rows ? rows + group * n_table : nullptr, (n_table & 3) == 0, mult, accumulate);
 }
 
-// mult[j] (+)= sum over the rows: 64 entries per workgroup, the rows dealt over its four wavefronts, eight in flight
-__global__ __launch_bounds__(BLOCK) void k_add_rows(const u32 *__restrict__ rows, int groups, i64 n_table, u64 *mult, int accumulate) {
-    __shared__ u64 part[BLOCK / 64][64];
+// mult[j] (+)= sum over the rows: 64 words of the rows per workgroup, the rows dealt over its four wavefronts, eight in flight.
+// HALF: two 16-bit counts to a word, fewer rows over a range (k_count).
+template <bool HALF>
+__global__ __launch_bounds__(BLOCK) void k_add_rows(const u32 *__restrict__ rows, int groups, i64 n_table, u64 *mult, int accumulate, const u32 *found,
+                                                    int n_found, int range_groups) {
+    constexpr int PER = HALF ? 2 : 1;
+    __shared__ u64 part[PER][BLOCK / 64][64];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const i64 j = (i64)blockIdx.x * 64 + lane;
-    u64 sum = 0;
-    if (j < n_table) {
+    const i64 at = (i64)blockIdx.x * 64 + lane, row_words = (n_table + PER - 1) / PER;
+    u64 sum[PER] = {};
+    if (HALF && !found_any((int)threadIdx.x < n_found ? found[threadIdx.x] : 0, OFF)) groups = range_groups;
+    if (at < row_words) {
         constexpr int UN = 8;
         for (int g0 = w; g0 < groups; g0 += UN * (BLOCK / 64)) {
             u32 c[UN];
 #pragma unroll
             for (int u = 0; u < UN; ++u) {
                 const int g = g0 + u * (BLOCK / 64);
-                c[u] = g < groups ? rows[(i64)g * n_table + j] : 0;
+                c[u] = g < groups ? rows[(i64)g * row_words + at] : 0;
             }
 #pragma unroll
-            for (int u = 0; u < UN; ++u) sum += c[u];
+            for (int u = 0; u < UN; ++u) {
+                sum[0] += HALF ? c[u] & 0xFFFF : c[u];
+                if (HALF) sum[PER - 1] += c[u] >> 16;
+            }
         }
     }
-    part[w][lane] = sum;
+#pragma unroll
+    for (int q = 0; q < PER; ++q) part[q][w][lane] = sum[q];
     __syncthreads();
-    if (w == 0 && j < n_table) {
-        sum = part[0][lane] + part[1][lane] + part[2][lane] + part[3][lane];
-        put(&mult[j], sum, accumulate);
+    // the workgroup's 64 PER counts in the order of the table
+    const i64 j = (i64)blockIdx.x * 64 * PER + threadIdx.x;
+    if (threadIdx.x < 64 * PER && j < n_table) {
+        const int q = threadIdx.x % PER, word = threadIdx.x / PER;
+        put(&mult[j], part[q][0][word] + part[q][1][word] + part[q][2][word] + part[q][3][word], accumulate);
     }
 }
 
@@ -317,8 +359,8 @@ inline unsigned capped_grid(i64 work_items) {
 }
 
 struct Plan {
-    bool small, direct;                        // k_count_small; one global atomic per look-up
-    i64 slices, groups;
+    bool small, direct, half;                  // k_count_small; one global atomic per look-up; 16-bit counters
+    i64 slices, groups, range_groups;          // groups: with 16-bit counters of another table, range_groups of a range
     int copies, bits, surveyors;
     size_t slot_bytes, found_bytes, row_bytes;
     size_t bytes() const {
@@ -355,6 +397,23 @@ Plan make_plan(i64 n_x, i64 n_table, bool promised) {
     L.groups = (n_x + 8191) / 8192;
     if (L.groups * L.slices > MAX_GROUPS) L.groups = MAX_GROUPS / L.slices;
     if (L.groups < (n_x >> 31) + 1) L.groups = (n_x >> 31) + 1;        // a group's counters have 32 bits
+    // From 8192 entries on 16-bit counters: half the bytes go through the rows, and half the slices read the look-ups, as long as no group
+    // has more look-ups than such a counter holds.  Over a range a group's look-ups cost less than its row: from 64 groups on they are
+    // larger (1.5 M in a range of 2^16: 21.0 us with 32-bit counters, 21.6 with 184 groups, 17.9 with 62; 10^6 in 40000 other entries
+    // 35.6, 49 with 41 groups, 30.7 with 123; 1.5 M in 2^14 20.1 -> 14.4).
+    if (n_table >= 8192) {
+        const i64 slices = (n_table + 2 * SLICE - 1) / (2 * SLICE), most = MAX_GROUPS / slices;
+        const i64 groups = std::min((n_x + 8191) / 8192, most), range_groups = std::min(std::max(std::min(groups, (i64)64), (n_x + 24575) / 24576), most);
+        if (range_groups > 1 && (n_x + range_groups - 1) / range_groups <= MAX_HALF) {
+            L.half = true;
+            L.slices = slices;
+            L.groups = groups;
+            L.range_groups = range_groups;
+            L.copies = 1;
+            L.row_bytes = (size_t)groups * ((n_table + 1) / 2) * sizeof(u32);
+            return L;
+        }
+    }
     const i64 counters = L.small ? SMALL_COUNTERS : SLICE;
     L.copies = 1;
     while (L.copies < MAX_COPIES && n_table * L.copies * 2 <= counters) L.copies *= 2;
@@ -377,7 +436,8 @@ int ask_for_lds() {
     VI_HIP(hipGetDevice(&dev));
     const unsigned long long bit = 1ull << (dev & 63);
     if (asked.load(std::memory_order_acquire) & bit) return VI_OK;
-    VI_HIP(hipFuncSetAttribute((const void *)k_count, hipFuncAttributeMaxDynamicSharedMemorySize, SLICE * (int)sizeof(u32)));
+    VI_HIP(hipFuncSetAttribute((const void *)k_count<true>, hipFuncAttributeMaxDynamicSharedMemorySize, SLICE * (int)sizeof(u32)));
+    VI_HIP(hipFuncSetAttribute((const void *)k_count<false>, hipFuncAttributeMaxDynamicSharedMemorySize, SLICE * (int)sizeof(u32)));
     VI_HIP(hipFuncSetAttribute((const void *)k_count_small, hipFuncAttributeMaxDynamicSharedMemorySize,
                                SMALL_COUNTERS * (int)sizeof(u32) + SMALL_TABLE * (int)(sizeof(u64) + 2 * sizeof(u32))));
     asked.fetch_or(bit, std::memory_order_release);
@@ -456,12 +516,20 @@ int vi_lookup_histogram(const uint64_t *x, int64_t n_x, const uint64_t *table, i
                            rows, mult, accumulate);
         VI_LAUNCH_CHECK("k_count_small");
     } else {
-        hipLaunchKernelGGL(k_count, dim3((unsigned)L.slices, (unsigned)L.groups), dim3(COUNT_THREADS), lds, s, x, (i64)n_x, per, F, L.copies, rows, mult,
-                           accumulate);
+        const dim3 grid((unsigned)L.slices, (unsigned)L.groups);
+        if (L.half) lds = (size_t)SLICE * sizeof(u32);
+        if (L.half) hipLaunchKernelGGL(k_count<true>, grid, dim3(COUNT_THREADS), lds, s, x, (i64)n_x, per, F, L.copies, rows, mult, accumulate, (int)L.range_groups);
+        else hipLaunchKernelGGL(k_count<false>, grid, dim3(COUNT_THREADS), lds, s, x, (i64)n_x, per, F, L.copies, rows, mult, accumulate, 0);
         VI_LAUNCH_CHECK("k_count");
     }
     if (rows) {
-        hipLaunchKernelGGL(k_add_rows, dim3((unsigned)((n_table + 63) / 64)), dim3(BLOCK), 0, s, (const u32 *)rows, (int)L.groups, (i64)n_table, mult, accumulate);
+        const unsigned adders = (unsigned)((n_table + (L.half ? 127 : 63)) / (L.half ? 128 : 64));
+        if (L.half)
+            hipLaunchKernelGGL(k_add_rows<true>, dim3(adders), dim3(BLOCK), 0, s, (const u32 *)rows, (int)L.groups, (i64)n_table, mult, accumulate,
+                               (const u32 *)F.found, F.n_found, (int)L.range_groups);
+        else
+            hipLaunchKernelGGL(k_add_rows<false>, dim3(adders), dim3(BLOCK), 0, s, (const u32 *)rows, (int)L.groups, (i64)n_table, mult, accumulate,
+                               (const u32 *)nullptr, 0, 0);
         VI_LAUNCH_CHECK("k_add_rows");
     }
     return VI_OK;
