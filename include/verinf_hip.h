@@ -42,6 +42,12 @@ const char *vi_version(void);
  * data is there (the tag is polled; the stream is queried from time to time, so a failed launch ends the wait). */
 int vi_read_back(const void *src, int64_t bytes, void *host, size_t host_bytes, void *stream);
 
+/* Waits for results that the kernels queued on the stream write into pinned host memory themselves: until the first n words
+ * of each of `rows` rows of row_words words are field elements.  The caller has set them to VI_NO_WORD before the launch.  The
+ * words are polled, the stream is queried from time to time, so that a failed launch ends the wait. */
+#define VI_NO_WORD 0xFFFFFFFFFFFFFFFFull
+int vi_wait_words(const uint64_t *words, int64_t rows, int64_t row_words, int64_t n, void *stream);
+
 /* n <= VI_UPLOAD_WORDS words of ordinary host memory to device memory, inside the arguments of a kernel: they are taken
  * before the call returns, and nothing waits for the stream. */
 #define VI_UPLOAD_WORDS 448

@@ -30,3 +30,18 @@ def test_upload_of_python_integers(n):
         assert tuple(t.shape) == (1, n) and t.dtype == torch.uint64
         assert to_np(t)[0].tolist() == [v % P for v in values]
     assert to_np(_lib.upload_words(_lib.field_words(np.arange(3, dtype=np.uint64))))[0].tolist() == [0, 1, 2]
+
+
+def test_waiting_for_words():
+    """Results that are there already, arguments that make no sense, and a stream that has nothing more to write."""
+    from verinf_amd import _lib
+    L = _lib.lib()
+    host, view = _lib.pinned_words(64, _lib.stream_ptr())
+    view[:24] = _lib.NO_WORD
+    view.reshape(-1)[:24].reshape(3, 8)[:, :5] = 7
+    assert L.vi_wait_words(host.data_ptr(), 3, 8, 5, _lib.stream_ptr()) == 0
+    assert L.vi_wait_words(host.data_ptr(), 0, 8, 5, _lib.stream_ptr()) == 0
+    torch.cuda.synchronize()
+    assert L.vi_wait_words(host.data_ptr(), 3, 8, 6, _lib.stream_ptr()) == -2 and b"drained" in L.vi_last_error()
+    assert L.vi_wait_words(host.data_ptr(), 3, 4, 5, None) == -1 and L.vi_wait_words(host.data_ptr() + 4, 1, 1, 1, None) == -1
+    assert L.vi_wait_words(None, 1, 1, 1, None) == -1

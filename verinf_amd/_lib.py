@@ -23,7 +23,7 @@ LIB_PATH = os.environ.get("VERINF_HIP_LIB") or os.path.join(_HERE, "libverinf_hi
 
 EXPORTS = [
     "vi_last_error", "vi_version",
-    "vi_read_back", "vi_upload_words",
+    "vi_read_back", "vi_wait_words", "vi_upload_words",
     "vi_gl_binop", "vi_gl_binop_bcast", "vi_gl_unop", "vi_gl_axpy", "vi_gl_probe",
     "vi_gl_sum_workspace_bytes", "vi_gl_sum",
     "vi_gl_matmul_workspace_bytes", "vi_gl_matmul", "vi_gl_matvec", "vi_poly_eval",
@@ -129,6 +129,8 @@ def lib():
     L.vi_lookup_histogram.restype = c_int
     L.vi_read_back.argtypes = [vp, i64, vp, sz, vp]
     L.vi_read_back.restype = c_int
+    L.vi_wait_words.argtypes = [vp, i64, i64, i64, vp]
+    L.vi_wait_words.restype = c_int
     L.vi_upload_words.argtypes = [vp, i64, vp, vp]
     L.vi_upload_words.restype = c_int
     L.vi_eq_vector.argtypes = [POINTER(u64), c_int, c_int, vp, vp]
@@ -239,20 +241,7 @@ def pinned_words(words: int, stream_ptr: int):
     return buf
 
 
-_results = threading.local()
-
-
-def result_words(words: int, stream_ptr: int):
-    """Device words for a result that the host waits for: one buffer per host thread and stream like pinned_words(), so that
-    another thread's call cannot write over it while this one waits."""
-    bufs = getattr(_results, "bufs", None)
-    if bufs is None:
-        bufs = _results.bufs = {}
-    key = (_get_device(), stream_ptr)
-    buf = bufs.get(key)
-    if buf is None or buf.numel() < words:
-        buf = bufs[key] = torch.empty(max(words, 512), dtype=torch.uint64, device=torch.device("cuda", key[0]))
-    return buf
+NO_WORD = 0xFFFFFFFFFFFFFFFF    # VI_NO_WORD: no field element
 
 
 def read_back_ptr(src: int, nbytes: int, sp: int) -> bytes:

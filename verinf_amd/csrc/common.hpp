@@ -35,12 +35,13 @@ inline int ilog2(long long x) {
 constexpr size_t WS_SLACK = 16;
 inline void *align16(void *ws) { return (void *)(((uintptr_t)ws + 15) & ~(uintptr_t)15); }
 
-// Waits until the kernel that finishes a result has stored `seq` behind it in pinned host memory.  The word is polled (a
-// stream synchronisation costs several microseconds more); every 2^16 polls the stream is queried, so a failed launch or
-// a stream that drained without the store ends the wait with an error instead of spinning.
-inline int wait_for_tag(const char *who, const volatile uint64_t *flag, uint64_t seq, hipStream_t s) {
+// Waits until arrived() is true of pinned host memory that a kernel on the stream writes.  It is asked again and again (a stream
+// synchronisation costs several microseconds more); every 2^16 times the stream is queried, so a failed launch or a stream that
+// drained without the result ends the wait with an error instead of spinning.
+template <class Arrived>
+inline int wait_until(const char *who, Arrived arrived, hipStream_t s) {
     for (unsigned spins = 1;; ++spins) {
-        if (*flag == seq) break;
+        if (arrived()) break;
         __builtin_ia32_pause();
         if ((spins & 0xFFFF) == 0) {
             hipError_t e = hipStreamQuery(s);
@@ -50,12 +51,16 @@ inline int wait_for_tag(const char *who, const volatile uint64_t *flag, uint64_t
             }
             if (e != hipSuccess) return fail(VI_EHIP, "%s: %s while waiting for a result", who, hipGetErrorString(e));
             // drained: host memory that is not coherent while a kernel runs shows the store now
-            if (*flag == seq) break;
+            if (arrived()) break;
             return fail(VI_EHIP, "%s: the stream drained without the result", who);
         }
     }
     std::atomic_thread_fence(std::memory_order_acquire);
     return VI_OK;
+}
+// the same for a result behind which the kernel stores `seq`
+inline int wait_for_tag(const char *who, const volatile uint64_t *flag, uint64_t seq, hipStream_t s) {
+    return wait_until(who, [=] { return *flag == seq; }, s);
 }
 
 // whether the stream is being captured; the default stream cannot be, and may not be asked while another one is

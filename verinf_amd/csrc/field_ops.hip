@@ -279,6 +279,20 @@ int vi_read_back(const void *src, int64_t bytes, void *host, size_t host_bytes, 
     return vi::wait_for_tag("vi_read_back", flag, tag, (hipStream_t)stream);
 }
 
+int vi_wait_words(const uint64_t *words, int64_t rows, int64_t row_words, int64_t n, void *stream) {
+    if (rows < 0 || n < 0 || row_words < n) return vi::fail(VI_EINVAL, "vi_wait_words: %lld of %lld words in %lld rows", (long long)n, (long long)row_words, (long long)rows);
+    if (rows == 0 || n == 0) return VI_OK;
+    if (!words || ((uintptr_t)words & 7)) return vi::fail(VI_EINVAL, "vi_wait_words: null or unaligned pointer");
+    const volatile uint64_t *w = words;
+    int64_t r = 0, i = 0;
+    return vi::wait_until("vi_wait_words", [&] {
+        for (; r < rows; ++r, i = 0)
+            for (; i < n; ++i)
+                if (w[r * row_words + i] == VI_NO_WORD) return false;
+        return true;
+    }, (hipStream_t)stream);
+}
+
 int vi_upload_words(const uint64_t *host, int64_t n, uint64_t *dst, void *stream) {
     if (n < 0 || n > VI_UPLOAD_WORDS) return vi::fail(VI_EINVAL, "vi_upload_words: n = %lld (0 .. %d)", (long long)n, VI_UPLOAD_WORDS);
     if (n == 0) return VI_OK;

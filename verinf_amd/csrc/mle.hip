@@ -142,7 +142,8 @@ __global__ __launch_bounds__(BLOCK) void k_mle_final(const u64 *__restrict__ par
     u64 acc = 0;
     for (int i = threadIdx.x; i < nb; i += BLOCK) acc = gl::add(acc, partial[(i64)blockIdx.x * nb + i]);
     const u64 r = block_sum(acc, lds4);
-    if (threadIdx.x == 0) out[blockIdx.x] = r;
+    // straight through to memory: `out` may be host memory that is being polled
+    if (threadIdx.x == 0) __hip_atomic_store(&out[blockIdx.x], r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 int load_point(const char *who, const uint64_t *z, int n, bool msb_first, Point &pt) {

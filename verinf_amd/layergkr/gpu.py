@@ -22,7 +22,6 @@ mle_eval work on Python lists).  The dense Lagrange-matrix encoders
 the one encoder here.
 """
 import ctypes
-import struct
 from typing import Optional, Sequence
 
 import torch
@@ -223,11 +222,14 @@ def mle_eval_t(tables, point: Sequence[int]):
     with _lib.on_device(tables.device):
         sp = _lib.stream_ptr()
         ws_bytes = _lib.workspace_bytes("mle_eval", k)
-        out = _lib.result_words(k, sp)
+        # the last kernel writes the values into pinned memory, which is polled until all are there
+        host, view = _lib.pinned_words(k, sp)
+        view[:k] = _lib.NO_WORD
         with _lib.stream_lock(sp):
             ws = _lib.workspace(ws_bytes, "mle", sp)
-            _lib.check(L.vi_mle_eval(mat.data_ptr(), k, 1 << n, _point(point), n, out.data_ptr(), ws.data_ptr(), ws_bytes, sp))
-        vals = list(struct.unpack(f"<{k}Q", _lib.read_back_ptr(out.data_ptr(), 8 * k, sp)))
+            _lib.check(L.vi_mle_eval(mat.data_ptr(), k, 1 << n, _point(point), n, host.data_ptr(), ws.data_ptr(), ws_bytes, sp))
+        _lib.check(L.vi_wait_words(host.data_ptr(), 1, k, k, sp))
+        vals = view[:k].tolist()
     return vals[0] if one else vals
 
 
@@ -249,30 +251,56 @@ def gl_sum(t):
     return out
 
 
-class _Problem:
-    """Host-side descriptor of a sum-of-products problem in the C ABI's shape."""
+def _pointers(tensors):
+    return (ctypes.c_void_p * len(tensors))(*[t.data_ptr() for t in tensors])
 
-    def __init__(self, tables, terms):
-        self.n_tables = len(tables)
-        off, idx = [0], []
-        for _, fs in terms:
-            idx.extend(fs)
-            off.append(len(idx))
-        self.n_terms = len(terms)
-        self.deg = max(len(fs) for _, fs in terms)
+
+class _Problem:
+    """A sum of products in the C ABI's shape: distinct factor objects as device tables, the terms over their indices."""
+
+    def __init__(self, terms, field_p, who):
+        if field_p != P:
+            raise ValueError(f"{who}: only the Goldilocks field is supported")
+        if not terms:
+            raise ValueError("no terms")
+        seen, tables, off, idx, coeffs, deg = {}, [], [0], [], [], 0
+        for c, fs in terms:
+            for f in fs:
+                k = id(f)
+                i = seen.get(k)
+                if i is None:
+                    i = seen[k] = len(tables)
+                    tables.append(_as_table(f, field_p))
+                idx.append(i)
+            n = len(idx)
+            deg = max(deg, n - off[-1])
+            off.append(n)
+            coeffs.append(int(c) % field_p)
+        size = tables[0].numel()
+        for t in tables:
+            if t.numel() != size:
+                raise ValueError(f"{who}: factors of different lengths")
+        if size < 1 or size & (size - 1):
+            raise ValueError(f"{who}: table length must be a power of two")
+        self.tables, self.size, self.deg = tables, size, deg
+        self.n_tables, self.n_terms = len(tables), len(coeffs)
+        self._lists = off, idx, coeffs
         self.term_off = (ctypes.c_int * len(off))(*off)
         self.factor_idx = (ctypes.c_int * max(len(idx), 1))(*idx)
-        self.coeffs = (ctypes.c_uint64 * len(terms))(*[c % P for c, _ in terms])
+        self.coeffs = (ctypes.c_uint64 * len(coeffs))(*coeffs)
 
-    @staticmethod
-    def ptrs(tensors):
-        return (ctypes.c_void_p * len(tensors))(*[t.data_ptr() for t in tensors])
+    def pointers(self):
+        return _pointers(self.tables)
+
+    def terms(self):
+        off, idx, coeffs = self._lists
+        return [(c, idx[off[k]:off[k + 1]]) for k, c in enumerate(coeffs)]
 
 
 def _fold_tables(src, dst, half: int, r: int):
     L = _lib.lib()
     with _lib.on_device(src[0].device):
-        _lib.check(L.vi_sumcheck_fold_eval(_Problem.ptrs(src), _Problem.ptrs(dst), len(src), half, r % P,
+        _lib.check(L.vi_sumcheck_fold_eval(_pointers(src), _pointers(dst), len(src), half, r % P,
                                            None, None, None, 0, None, None, None, 0, _lib.stream_ptr()))
 
 
@@ -298,30 +326,6 @@ def _as_table(v, field_p):
         return v if v.dim() == 1 and v.is_contiguous() else v.reshape(-1).contiguous()
     import numpy as np
     return torch.from_numpy(np.array([int(x) % field_p for x in v], dtype=np.uint64)).cuda()
-
-
-def _sumcheck_problem(terms, field_p, who):
-    """Distinct factor objects as device tables + the terms over their indices."""
-    if field_p != P:
-        raise ValueError(f"{who}: only the Goldilocks field is supported")
-    if not terms:
-        raise ValueError("no terms")
-    uniq, tables, tterms = {}, [], []
-    for c, fs in terms:
-        ids = []
-        for f in fs:
-            k = id(f)
-            if k not in uniq:
-                uniq[k] = len(tables)
-                tables.append(_as_table(f, field_p))
-            ids.append(uniq[k])
-        tterms.append((int(c) % field_p, ids))
-    size = int(tables[0].numel())
-    if any(int(t.numel()) != size for t in tables):
-        raise ValueError(f"{who}: factors of different lengths")
-    if size < 1 or size & (size - 1):
-        raise ValueError(f"{who}: table length must be a power of two")
-    return tables, tterms, size
 
 
 def _single_point(tables, tterms, mu0, field_p):
@@ -357,48 +361,51 @@ def prove_terms_gpu(terms, coin, field_p: int, mask=None, mu0: int = 0):
     (vi_sumcheck_prove_coins).  prove_terms_gpu_interactive is the variant for a coin that
     does need the samples."""
     _require_gpu()
-    tables, tterms, size = _sumcheck_problem(terms, field_p, "prove_terms_gpu")
+    prob = _Problem(terms, field_p, "prove_terms_gpu")
+    tables, size = prob.tables, prob.size
     n_rounds = size.bit_length() - 1
     if n_rounds == 0:
-        return _single_point(tables, tterms, mu0, field_p)
-    prob = _Problem(tables, tterms)
+        return _single_point(tables, prob.terms(), mu0, field_p)
     deg = prob.deg
     mu = mu0 % field_p
     challenges, masks = [], []
-    for rnd in range(n_rounds):
-        h = mask(deg, mu) if mask is not None else None
-        r = coin(rnd) % field_p
-        challenges.append(r)
-        masks.append(h)
-        if h is not None:
+    if mask is None:
+        challenges = [coin(rnd) % field_p for rnd in range(n_rounds)]
+    else:
+        for rnd in range(n_rounds):
+            h = mask(deg, mu)
+            r = coin(rnd) % field_p
+            challenges.append(r)
+            masks.append(h)
             mu = _poly_eval(h, r, field_p)
     L = _lib.lib()
     dev = tables[0].device
     with _lib.on_device(dev):
-        stream = torch.cuda.current_stream()
-        sp = stream.cuda_stream
-        samples_host, samples_np = _lib.pinned_words(8 * n_rounds, sp)
+        sp = _lib.stream_ptr()
+        host, view = _lib.pinned_words(8 * n_rounds, sp)
+        view[:8 * n_rounds] = _lib.NO_WORD
+        samples_p = host.data_ptr()
         chal = (ctypes.c_uint64 * n_rounds)(*challenges)
+        tables_p = prob.pointers()
         with _lib.stream_lock(sp):
             ws = _lib.workspace(_lib.workspace_bytes("sumcheck_prove_coins", size), "sumcheck_coins", sp)
             # the folded tables live in one cached scratch buffer, a half-length slice per table (the caller's
             # tensors are never written)
             half_bytes = (size // 2) * 8
             work = _lib.workspace(max(prob.n_tables * half_bytes, 256), "sumcheck_work", sp)
-            work_p = (ctypes.c_void_p * prob.n_tables)(*[work.data_ptr() + t * half_bytes for t in range(prob.n_tables)])
-            _lib.check(L.vi_sumcheck_prove_coins(_Problem.ptrs(tables), work_p, prob.n_tables, size,
-                                                 prob.term_off, prob.factor_idx, prob.coeffs, prob.n_terms, chal,
-                                                 samples_host.data_ptr(), ws.data_ptr(), ws.numel(), sp))
-        stream.synchronize()
-        rows = samples_np[:8 * n_rounds].reshape(n_rounds, 8)[:, :deg + 1].tolist()
-    if mask is None:
-        round_polys = [list(enumerate(ys)) for ys in rows]
-    else:
-        round_polys = [[(x, (y + _poly_eval(h, x, field_p)) % field_p) for x, y in enumerate(ys)]
-                       for ys, h in zip(rows, masks)]
+            first = work.data_ptr()
+            work_p = (ctypes.c_void_p * prob.n_tables)(*range(first, first + prob.n_tables * half_bytes, half_bytes))
+            _lib.check(L.vi_sumcheck_prove_coins(tables_p, work_p, prob.n_tables, size, prob.term_off, prob.factor_idx,
+                                                 prob.coeffs, prob.n_terms, chal, samples_p, ws.data_ptr(), ws.numel(), sp))
+        # while the kernels run: what the masks add to the samples
+        added = [[_poly_eval(h, x, field_p) for x in range(deg + 1)] for h in masks]
+        _lib.check(L.vi_wait_words(samples_p, n_rounds, 8, deg + 1, sp))
+        rows = view[:8 * n_rounds].reshape(n_rounds, 8)[:, :deg + 1].tolist()
     # S(0) + S(1) of the first round is the sum over the cube
     claim = (rows[0][0] + rows[0][1] + mu0) % field_p
-    return claim, round_polys, challenges, mu
+    if mask is not None:
+        rows = [[(y + a) % field_p for y, a in zip(ys, hs)] for ys, hs in zip(rows, added)]
+    return claim, [list(enumerate(ys)) for ys in rows], challenges, mu
 
 
 def prove_terms_gpu_interactive(terms, coin, field_p: int, mask=None, mu0: int = 0):
@@ -406,11 +413,11 @@ def prove_terms_gpu_interactive(terms, coin, field_p: int, mask=None, mu0: int =
     samples = [(x, S(x))] of that round (mask applied) -> challenge.  One launch and one host
     wait per round (vi_sumcheck_prove); same return value."""
     _require_gpu()
-    tables, tterms, size = _sumcheck_problem(terms, field_p, "prove_terms_gpu_interactive")
+    prob = _Problem(terms, field_p, "prove_terms_gpu_interactive")
+    tables, size = prob.tables, prob.size
     n_rounds = size.bit_length() - 1
     if n_rounds == 0:
-        return _single_point(tables, tterms, mu0, field_p)
-    prob = _Problem(tables, tterms)
+        return _single_point(tables, prob.terms(), mu0, field_p)
     deg = prob.deg
     L = _lib.lib()
     dev = tables[0].device
@@ -447,7 +454,7 @@ def prove_terms_gpu_interactive(terms, coin, field_p: int, mask=None, mu0: int =
         cb = _lib.COIN_FN(on_round)
         out_samples = (ctypes.c_uint64 * (n_rounds * (deg + 1)))()
         out_chals = (ctypes.c_uint64 * n_rounds)()
-        rc = L.vi_sumcheck_prove(_Problem.ptrs(tables), _Problem.ptrs(work), prob.n_tables, size, prob.term_off,
+        rc = L.vi_sumcheck_prove(_pointers(tables), _pointers(work), prob.n_tables, size, prob.term_off,
                                  prob.factor_idx, prob.coeffs, prob.n_terms, cb, None, samples_host.data_ptr(),
                                  samples_host.numel(), out_samples, out_chals, ws.data_ptr(), ws.numel(),
                                  _lib.stream_ptr())
