@@ -712,3 +712,20 @@ def test_sums_under_a_common_factor(mods, form, v):
     assert claim == want_claim and [[y for _, y in s] for s in polys] == want_samples
     for t, d in zip(raw, dev):
         assert np.array_equal(to_np(d), t), "caller's table was modified"
+
+
+@pytest.mark.parametrize("coins", [[0, 5], [2, 7], [9, 2, 3], [9, 8, 0], [1, 1, 1], [P - 1, P - 2, 1], [3, 4, 5, 0, 2, 1, 0]])
+@pytest.mark.parametrize("terms,v", [([(5, [0])], 14), ([(1, [0, 1])], 13), ([(7, [0, 1])], 16), ([(1, [0, 1, 2])], 13), ([(1, [0, 1, 2])], 16),
+                                     ([(3, [0, 1, 2, 3])], 13), ([(3, [0, 1, 2]), (P - 3, [0, 3])], 13), ([(3, [0, 1]), (4, [0, 2])], 10),
+                                     ([(3, [0, 1, 2]), (4, [0, 2]), (6, [0, 3])], 10), ([(3, [0, 1, 2]), (4, [0, 2]), (6, [0, 3])], 13)])
+def test_first_sample_at_one_from_a_later_round(mods, terms, v, coins):
+    """A proof whose first launch does three rounds sums S(1) in round 3 instead of 0 and goes back from there, unless one of the first
+    challenges is a zero of the way back (0 and 2; 0 alone in degree 1)."""
+    gpu, _ = mods
+    coins = coins + _coins(v, 31)[0][len(coins):]
+    tabs = [rand_field(1 << v, 4000 + t) for t in range(1 + max(max(fs) for _, fs in terms))]
+    dev = [to_dev(t) for t in tabs]
+    print(terms, v, coins[:4], flush=True)
+    claim, polys, _, _ = gpu.prove_terms_gpu([(c, [dev[i] for i in fs]) for c, fs in terms], lambda i: coins[i], P)
+    want_claim, want_samples, _ = O.sumcheck_prove(tabs, terms, coins)
+    assert claim == want_claim and [[y for _, y in s] for s in polys] == want_samples

@@ -1578,6 +1578,8 @@ int prove_coins_impl(const char *who, const uint64_t *const *tables, uint64_t *c
     C.scale = 1;
     C.skip_mask = 0;
     C.inf_node = 0;
+    C.late = 0;
+    C.late_inv = 0;
     C.dfact = 1;
     for (int x = 0; x < NSAMP; ++x) C.cinf[x] = 0;
     C.n_rounds = v;

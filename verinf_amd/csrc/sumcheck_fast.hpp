@@ -42,6 +42,10 @@ struct ChainDesc {
     u64 cinf[NSAMP];
     u64 dfact;
     int inf_node;
+    // late: the round that sums S(1) where round 0 does not (0 = round 0 does): it has an eighth of the pairs.  The claims before it are
+    // affine in the first, claim_late = A claim_0 + B, and late_inv = 1 / A
+    int late;
+    u64 late_inv;
     unsigned off[MAX_ROUNDS];               // word offset of round k's per-workgroup partial sums in the workspace
     unsigned short nb[MAX_ROUNDS];          // rows of NSAMP words round k left there
     int n_rounds, n_prior, deg;             // rounds of the proof; rounds whose partial sums are in the workspace
@@ -52,6 +56,7 @@ struct FinishShared {
     u64 lag[MAX_ROUNDS][NSAMP];             // Lagrange basis of the points 0..deg at r_k
     u64 a[MAX_ROUNDS], b[MAX_ROUNDS];       // claim_(k+1) = a_k claim_k + b_k
     u64 claim[MAX_ROUNDS + 1];
+    u64 late_claim;
 };
 
 // The sums over the wavefront of N values per lane: a step adds the halves of the lanes and halves the values, each half of the
@@ -172,10 +177,15 @@ __device__ __forceinline__ void finish_samples(const ChainDesc &C, FinishShared 
         }
         sh.a[k] = a;
         sh.b[k] = b;
+        if (k == C.late) sh.late_claim = gl::addc(y[0], y[1]);
     }
     __syncthreads();
     if (threadIdx.x == 0) {
         u64 claim = 0;                       // a round that summed every sample does not read it
+        if (C.late > 0) {
+            for (int j = 0; j < C.late; ++j) claim = gl::addc(gl::mul(sh.a[j], claim), sh.b[j]);
+            claim = gl::mul(gl::sub(sh.late_claim, claim), C.late_inv);
+        }
         for (int j = 0; j < C.n_rounds; ++j) {
             sh.claim[j] = claim;
             claim = gl::addc(gl::mul(sh.a[j], claim), sh.b[j]);
@@ -283,6 +293,19 @@ __device__ __forceinline__ void eval_pair(const u64 (&lo)[NT], const u64 (&hi)[N
     }
 }
 
+// Caller data, any 64-bit word is taken as its residue.  Words at or above p have all of the upper half set, as few others have:
+// where no lane of the wavefront holds such a word, one maximum per two words is all that this costs.
+template <int N>
+__device__ __forceinline__ void canon_all(u64 (&v)[N]) {
+    u32 top = 0;
+#pragma unroll
+    for (int i = 0; i < N; ++i) top = max(top, (u32)(v[i] >> 32));
+    if (__any(top == 0xFFFFFFFFu)) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) v[i] = gl::canon(v[i]);
+    }
+}
+
 template <int NT, int SHAPE, bool FIRST>
 __device__ __forceinline__ u64 fast_load(const FastDesc &D, int t, i64 idx) {
     u64 v = D.src[t][idx];
@@ -350,8 +373,8 @@ __device__ __forceinline__ void pass_sums(const SampleAcc<true> (&acc0)[NS], con
 }
 
 // Three rounds on eight entries of every table, v[t][c] = entry i + c cols (canonical): the samples of the seven pairs into the rounds'
-// accumulators, the entry folded three times into `folded`.  FIRST: the first round sums S(1) too.
-template <int NT, int SHAPE, bool FIRST>
+// accumulators, the entry folded three times into `folded`.  ONE: the first round sums S(1) too.
+template <int NT, int SHAPE, bool ONE>
 __device__ __forceinline__ void three_rounds(u64 (&v)[NT][8], u64 r0, u64 r1, u64 r2, SampleAcc<true> (&acc0)[FastShape<NT, SHAPE>::NS],
                                              SampleAcc<true> (&acc1)[FastShape<NT, SHAPE>::NS], SampleAcc<true> (&acc2)[FastShape<NT, SHAPE>::NS],
                                              u64 (&folded)[NT]) {
@@ -362,7 +385,7 @@ __device__ __forceinline__ void three_rounds(u64 (&v)[NT][8], u64 r0, u64 r1, u6
         VI_SCHED_FENCE();
 #pragma unroll
         for (int t = 0; t < NT; ++t) { lo[t] = v[t][c]; hi[t] = v[t][c + 4]; }
-        eval_pair<NT, SHAPE, !FIRST, true>(lo, hi, dif, acc0);
+        eval_pair<NT, SHAPE, !ONE, true>(lo, hi, dif, acc0);
 #pragma unroll
         for (int t = 0; t < NT; ++t) v[t][c] = gl::mul_add(r0, dif[t], lo[t]);
     }
@@ -384,12 +407,12 @@ __device__ __forceinline__ void three_rounds(u64 (&v)[NT][8], u64 r0, u64 r1, u6
 }
 
 // Three rounds in one pass.  cols = n / 8 for tables of n words; thread i < cols owns entries i + c cols.
-// FIRST: the tables are the caller's (words reduced on load, round 0 sums every sample).
+// FIRST: the tables are the caller's (words reduced on load).  ONE: the first of the rounds sums every sample.
 // part: three regions of gridDim.x rows of NSAMP words, one per round.
 // prev_part / prev_rows / prev_sums: the previous pass's three regions of prev_rows rows each; workgroup j < 3 adds
 // region j up into row j of prev_sums before it starts on its own columns, so that the kernel that finishes the
 // proof finds one row per round instead of a thousand (prev_rows = 0: nothing to add up).
-template <int NT, int SHAPE, bool FIRST>
+template <int NT, int SHAPE, bool FIRST, bool ONE>
 __global__ __launch_bounds__(BLOCK) void k_pass3(const FastDesc D, i64 cols, u64 r0, u64 r1, u64 r2, u64 *part,
                                                  const u64 *prev_part, int prev_rows, u64 *prev_sums) {
     constexpr int NS = FastShape<NT, SHAPE>::NS;
@@ -409,18 +432,20 @@ __global__ __launch_bounds__(BLOCK) void k_pass3(const FastDesc D, i64 cols, u64
             for (int c = 0; c < 8; ++c) v[t][c] = D.src[t][i + c * cols];
         if (FIRST) {
 #pragma unroll
-            for (int t = 0; t < NT; ++t)
+            for (int t = 0; t < NT; ++t) {
+                if (SHAPE == 2 && t == 3) {
 #pragma unroll
-                for (int c = 0; c < 8; ++c) {
-                    v[t][c] = gl::canon(v[t][c]);
-                    if (SHAPE == 2 && t == 3) {
+                    for (int c = 0; c < 8; ++c) {
                         v[t][c] = gl::mul(v[t][c], D.lin_coeff);
                         VI_SCHED_FENCE();
                     }
+                } else {
+                    canon_all(v[t]);
                 }
+            }
         }
         u64 folded[NT];
-        three_rounds<NT, SHAPE, FIRST>(v, r0, r1, r2, acc0, acc1, acc2, folded);
+        three_rounds<NT, SHAPE, ONE>(v, r0, r1, r2, acc0, acc1, acc2, folded);
 #pragma unroll
         for (int t = 0; t < NT; ++t) D.dst[t][i] = folded[t];
     }
@@ -457,7 +482,7 @@ __device__ __forceinline__ void tail_round_total(u64 (*red_par)[NSAMP], int acti
 }
 
 // Every remaining round in one workgroup: tables of `size` <= 2 TailCap<NT>::HALF words; rounds C.n_prior .. C.n_rounds - 1.
-// FIRST: the proof starts here (the tables are the caller's).  The folded tables live in LDS and are not written back.
+// FIRST: the proof starts here (the tables are the caller's).  ONE: the launch's first round sums S(1).  The folded tables live in LDS and are not written back.
 // A round costs its longest thread, so what a round does besides its one pair per thread is kept off that path:
 //  - rounds of more than TAIL_DEFER pairs add their sums up across the workgroup as they go (every wavefront is busy);
 //  - smaller rounds leave each thread's sums in LDS -- the round of h pairs in lane_sums[.][h .. 2h) -- and nine
@@ -466,7 +491,7 @@ __device__ __forceinline__ void tail_round_total(u64 (*red_par)[NSAMP], int acti
 //    lane and partners fetched by lane shuffles: no LDS traffic for the tables, no workgroup barrier per round.
 constexpr int TAIL_DEFER = 256;
 
-template <int NT, int SHAPE, bool FIRST>
+template <int NT, int SHAPE, bool FIRST, bool ONE>
 __global__ __launch_bounds__(TAIL_THREADS) void k_tail(const FastDesc D, i64 size, const ChainDesc C, const u64 *part, u64 *out) {
     constexpr int NS = FastShape<NT, SHAPE>::NS;
     constexpr int HALF = TailCap<NT>::HALF;
@@ -493,7 +518,7 @@ __global__ __launch_bounds__(TAIL_THREADS) void k_tail(const FastDesc D, i64 siz
                 lo[t] = fast_load<NT, SHAPE, FIRST>(D, t, i);
                 hi[t] = fast_load<NT, SHAPE, FIRST>(D, t, (i64)h + i);
             }
-            eval_pair<NT, SHAPE, !FIRST, false>(lo, hi, dif, acc);
+            eval_pair<NT, SHAPE, !ONE, false>(lo, hi, dif, acc);
             if (h > 1) {
 #pragma unroll
                 for (int t = 0; t < NT; ++t) tab[t][i] = gl::mul_add(r, dif[t], lo[t]);
@@ -588,7 +613,7 @@ __global__ __launch_bounds__(TAIL_THREADS) void k_tail(const FastDesc D, i64 siz
     finish_samples(C, sh, out);
 }
 
-template <int NT, int SHAPE, bool FIRST>
+template <int NT, int SHAPE, bool FIRST, bool ONE>
 int launch_pass3(const FastDesc &F, i64 cols, const u64 *r, u64 *part, const u64 *prev_part, int prev_rows,
                  u64 *prev_sums, hipStream_t s) {
     static std::mutex mu;
@@ -598,13 +623,13 @@ int launch_pass3(const FastDesc &F, i64 cols, const u64 *r, u64 *part, const u64
     int cap;
     {
         std::lock_guard<std::mutex> lock(mu);
-        if (!caps[dev]) caps[dev] = resident_blocks(k_pass3<NT, SHAPE, FIRST>, 64);
+        if (!caps[dev]) caps[dev] = resident_blocks(k_pass3<NT, SHAPE, FIRST, ONE>, 64);
         cap = caps[dev];
     }
     int nb = blocks_for(cols);
     if (nb > cap) nb = cap;
     if (nb < 3 && prev_rows > 0) nb = 3;     // the first three workgroups add up the previous pass's sums
-    hipLaunchKernelGGL((k_pass3<NT, SHAPE, FIRST>), dim3(nb), dim3(BLOCK), 0, s, F, cols, r[0], r[1], r[2], part,
+    hipLaunchKernelGGL((k_pass3<NT, SHAPE, FIRST, ONE>), dim3(nb), dim3(BLOCK), 0, s, F, cols, r[0], r[1], r[2], part,
                        prev_part, prev_rows, prev_sums);
     return nb;
 }
@@ -627,6 +652,35 @@ void fill_inf_node(ChainDesc &C, int d) {
     }
 }
 
+// Round 3 sums S(1) in the place of round 0, for a proof whose first launch does three rounds: C.late, C.late_inv, C.skip_mask.  A
+// challenge at which S(1) does not enter the next claim (0, and 2 in degree 2 and 3) leaves round 0 as it is.  Called with r, winv
+// and the constants of inf_node set.
+void fill_late(ChainDesc &C, bool passes) {
+    C.late = 0;
+    C.late_inv = 0;
+    if (passes) {
+        u64 product = 1;
+        for (int k = 0; k < 3; ++k) {
+            auto basis = [&](int x) {
+                u64 l = C.winv[x];
+                for (int j = 0; j <= C.deg; ++j)
+                    if (j != x) l = gl::mul(l, gl::sub(C.r[k], (u64)j));
+                return l;
+            };
+            u64 a = basis(1);
+            if (C.inf_node) a = C.deg == 1 ? 0 : gl::add(a, gl::mul(basis(C.deg), C.cinf[1]));
+            product = gl::mul(product, a);
+        }
+        if (product != 0) {
+            C.late = 3;
+            C.late_inv = gl::inv(product);
+        }
+    }
+    C.skip_mask = 0;
+    for (int j = 0; j < C.n_rounds; ++j)
+        if (j != C.late) C.skip_mask |= 1ull << j;
+}
+
 // The whole proof of a fixed shape: passes of three rounds while the tables exceed a tail workgroup, then the tail.
 // part: workspace of at least (n_rounds + 1) * MAX_BLOCKS * NSAMP words; C arrives with r, winv, scale, deg, n_rounds set.
 template <int NT, int SHAPE>
@@ -635,9 +689,8 @@ int prove_fast_shape(FastDesc F, i64 size, ChainDesc &C, u64 *part, u64 *out, hi
     int k = 0;
     unsigned off = 0;
     bool first = true;
-    C.skip_mask = 0;
-    for (int j = 1; j < C.n_rounds; ++j) C.skip_mask |= 1ull << j;
     if (FastShape<NT, SHAPE>::INF) fill_inf_node(C, C.deg);
+    fill_late(C, size > TAIL_MAX);
     // one row per round for the sums that a pass adds up for the pass before it: the last MAX_ROUNDS rows of the workspace
     const unsigned sums_off = (unsigned)C.n_rounds * MAX_BLOCKS * NSAMP;
     const u64 *prev_part = nullptr;
@@ -645,8 +698,10 @@ int prove_fast_shape(FastDesc F, i64 size, ChainDesc &C, u64 *part, u64 *out, hi
     while (size > TAIL_MAX) {
         const i64 cols = size >> 3;
         u64 *prev_sums = part + sums_off + (unsigned)prev_k * NSAMP;
-        const int nb = first ? launch_pass3<NT, SHAPE, true>(F, cols, C.r + k, part + off, prev_part, prev_rows, prev_sums, s)
-                             : launch_pass3<NT, SHAPE, false>(F, cols, C.r + k, part + off, prev_part, prev_rows, prev_sums, s);
+        const bool one = k == C.late;
+        auto launch = [&](auto kernel_of) { return kernel_of(F, cols, C.r + k, part + off, prev_part, prev_rows, prev_sums, s); };
+        const int nb = first ? (one ? launch(launch_pass3<NT, SHAPE, true, true>) : launch(launch_pass3<NT, SHAPE, true, false>))
+                             : (one ? launch(launch_pass3<NT, SHAPE, false, true>) : launch(launch_pass3<NT, SHAPE, false, false>));
         VI_LAUNCH_CHECK("sumcheck pass (three rounds)");
         if (prev_rows > 0) {
             for (int j = 0; j < 3; ++j) {    // this launch has left the previous pass's rounds as one row each
@@ -670,8 +725,10 @@ int prove_fast_shape(FastDesc F, i64 size, ChainDesc &C, u64 *part, u64 *out, hi
         }
     }
     C.n_prior = k;
-    if (first) hipLaunchKernelGGL((k_tail<NT, SHAPE, true>), dim3(1), dim3(TAIL_THREADS), 0, s, F, size, C, (const u64 *)part, out);
-    else hipLaunchKernelGGL((k_tail<NT, SHAPE, false>), dim3(1), dim3(TAIL_THREADS), 0, s, F, size, C, (const u64 *)part, out);
+    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(1), dim3(TAIL_THREADS), 0, s, F, size, C, (const u64 *)part, out); };
+    if (first) launch(k_tail<NT, SHAPE, true, true>);
+    else if (k == C.late) launch(k_tail<NT, SHAPE, false, true>);
+    else launch(k_tail<NT, SHAPE, false, false>);
     VI_LAUNCH_CHECK("sumcheck tail");
     return VI_OK;
 }

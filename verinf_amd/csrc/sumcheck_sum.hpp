@@ -49,10 +49,7 @@ template <bool FIRST>
 __device__ __forceinline__ void load_table(const u64 *f, i64 i, i64 cols, int entries, u64 (&v)[8]) {
 #pragma unroll
     for (int c = 0; c < 8; ++c) v[c] = c < entries ? f[i + c * cols] : 0;
-    if (FIRST) {
-#pragma unroll
-        for (int c = 0; c < 8; ++c) v[c] = gl::canon(v[c]);
-    }
+    if (FIRST) canon_all(v);
 }
 // the same of the sum of a row's single tables: plain integers of five words, reduced once
 __device__ __forceinline__ void load_singles(const SumDesc &D, int row, i64 i, i64 cols, int entries, u64 (&v)[8]) {
@@ -82,7 +79,7 @@ __device__ __forceinline__ void load_singles(const SumDesc &D, int row, i64 i, i
 
 // part: three regions of gridDim.x * n_rows rows of NSAMP words, one per round.  A row of workgroups behind those of the terms adds up
 // the regions of the pass before.
-template <bool FIRST>
+template <bool FIRST, bool ONE>
 __global__ __launch_bounds__(BLOCK) void k_sum3(const SumDesc D, i64 cols, u64 r0, u64 r1, u64 r2, u64 *part, const u64 *prev_part, int prev_rows,
                                                 u64 *prev_sums) {
     constexpr int NS = 4;
@@ -104,7 +101,7 @@ __global__ __launch_bounds__(BLOCK) void k_sum3(const SumDesc D, i64 cols, u64 r
             u64 v[2][8], folded[2];
             load_table<FIRST>(D.common, i, cols, 8, v[0]);
             load_singles(D, row, i, cols, 8, v[1]);
-            three_rounds<2, 3, FIRST>(v, r0, r1, r2, acc0, acc1, acc2, folded);
+            three_rounds<2, 3, ONE>(v, r0, r1, r2, acc0, acc1, acc2, folded);
             D.single_dst[row][i] = folded[1];
             common = folded[0];
         } else {
@@ -112,7 +109,7 @@ __global__ __launch_bounds__(BLOCK) void k_sum3(const SumDesc D, i64 cols, u64 r
             load_table<FIRST>(D.common, i, cols, 8, v[0]);
             load_table<FIRST>(D.a[k], i, cols, 8, v[1]);
             load_table<FIRST>(D.b[k], i, cols, 8, v[2]);
-            three_rounds<3, 1, FIRST>(v, r0, r1, r2, acc0, acc1, acc2, folded);
+            three_rounds<3, 1, ONE>(v, r0, r1, r2, acc0, acc1, acc2, folded);
             if (D.a_dst[k]) D.a_dst[k][i] = folded[1];
             if (D.b_dst[k]) D.b_dst[k][i] = folded[2];
             common = folded[0];
@@ -129,7 +126,7 @@ struct TailCoins {
 };
 
 // a round on P pairs of every lane: their samples, and the entries folded
-template <int P, bool FIRST>
+template <int P, bool ONE>
 __device__ __forceinline__ void lane_round(u64 (&v)[3][8], u64 r, u64 (&total)[4]) {
     SampleAcc<false> acc[4];
 #pragma unroll
@@ -139,7 +136,7 @@ __device__ __forceinline__ void lane_round(u64 (&v)[3][8], u64 r, u64 (&total)[4
     for (int c = 0; c < P; ++c) {
 #pragma unroll
         for (int t = 0; t < 3; ++t) { lo[t] = v[t][c]; hi[t] = v[t][c + P]; }
-        eval_pair<3, 1, !FIRST, false>(lo, hi, dif, acc);
+        eval_pair<3, 1, !ONE, false>(lo, hi, dif, acc);
 #pragma unroll
         for (int t = 0; t < 3; ++t) v[t][c] = gl::mul_add(r, dif[t], lo[t]);
     }
@@ -149,8 +146,8 @@ __device__ __forceinline__ void lane_round(u64 (&v)[3][8], u64 r, u64 (&total)[4
 
 // size: entries per table, a power of two up to SUM_TAIL.  part: a region of n_rows rows of NSAMP words per round, in the order of
 // the rounds.  Workgroups behind those of the rows add up the three regions of the pass before.
-// FIRST: every round sums S(1) (the proof's first is the one that it is used of).
-template <bool FIRST>
+// FIRST: the tables are the caller's.  ONE: every round sums S(1) (the first of the launch is the one that it is used of).
+template <bool FIRST, bool ONE>
 __global__ __launch_bounds__(BLOCK) void k_sum_tail(const SumDesc D, int size, const TailCoins C, u64 *part, const u64 *prev_part, int prev_rows, u64 *prev_sums) {
     __shared__ u64 red_prev[BLOCK / 64][NSAMP];
     const int lane = threadIdx.x & 63, n_rows = D.n_rows, groups = (n_rows + BLOCK / 64 - 1) / (BLOCK / 64);
@@ -184,9 +181,9 @@ __global__ __launch_bounds__(BLOCK) void k_sum_tail(const SumDesc D, int size, c
     for (int q = 0; q < 9; ++q)
 #pragma unroll
         for (int x = 0; x < 4; ++x) total[q][x] = 0;
-    if (entries >= 8) lane_round<4, FIRST>(v, C.r[8], total[0]);
-    if (entries >= 4) lane_round<2, FIRST>(v, C.r[7], total[1]);
-    if (entries >= 2) lane_round<1, FIRST>(v, C.r[6], total[2]);
+    if (entries >= 8) lane_round<4, ONE>(v, C.r[8], total[0]);
+    if (entries >= 4) lane_round<2, ONE>(v, C.r[7], total[1]);
+    if (entries >= 2) lane_round<1, ONE>(v, C.r[6], total[2]);
 #pragma unroll
     for (int level = 5; level >= 0; --level) {
         const int h = 1 << level;
@@ -200,7 +197,7 @@ __global__ __launch_bounds__(BLOCK) void k_sum_tail(const SumDesc D, int size, c
                 lo[t] = v[t][0];
                 hi[t] = __shfl_down(v[t][0], (unsigned)h, 64);         // lanes past the pairs compute on what they get and drop it
             }
-            eval_pair<3, 1, !FIRST, false>(lo, hi, dif, acc);
+            eval_pair<3, 1, !ONE, false>(lo, hi, dif, acc);
 #pragma unroll
             for (int t = 0; t < 3; ++t) v[t][0] = gl::mul_add(C.r[level], dif[t], lo[t]);
 #pragma unroll
@@ -273,14 +270,14 @@ bool sum_shape(int n_tables, const int *term_off, const int *factor_idx, const u
     return S.products.size() <= (size_t)SUM_PRODUCTS && S.singles.size() <= (size_t)SUM_SINGLES && S.products.size() + S.singles.size() > 0;
 }
 
-template <bool FIRST>
+template <bool FIRST, bool ONE>
 int sum_resident() {
     static std::mutex mu;
     static int caps[64] = {0};
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
     std::lock_guard<std::mutex> lock(mu);
-    if (!caps[dev]) caps[dev] = resident_blocks(k_sum3<FIRST>, 64);
+    if (!caps[dev]) caps[dev] = resident_blocks(k_sum3<FIRST, ONE>, 64);
     return caps[dev];
 }
 
@@ -312,7 +309,7 @@ int prove_sum(const SumShape &S, const uint64_t *const *tables, uint64_t *const 
     };
     deal_singles();
     if (C.deg == 3) fill_inf_node(C, 3);
-    for (int j = 1; j < C.n_rounds; ++j) C.skip_mask |= 1ull << j;
+    fill_late(C, size > SUM_TAIL);
     const unsigned sums_off = (unsigned)C.n_rounds * MAX_BLOCKS * NSAMP;
     const i64 upper = size >> 2;
     const u64 *prev_part = nullptr;
@@ -347,13 +344,20 @@ int prove_sum(const SumShape &S, const uint64_t *const *tables, uint64_t *const 
             D.b_dst[q] = own(S.products[q].b);
         }
         for (int q = 0; q < D.n_single_rows; ++q) D.single_dst[q] = work[q] + upper + written;
-        const int rows = D.n_rows, cap = first ? sum_resident<true>() : sum_resident<false>();
+        const bool one = k == C.late;
+        const int rows = D.n_rows, cap = first ? (one ? sum_resident<true, true>() : sum_resident<true, false>())
+                                               : (one ? sum_resident<false, true>() : sum_resident<false, false>());
         int gx = blocks_for(cols);
         if (gx * rows > cap) gx = std::max(1, cap / rows);
         u64 *prev_sums = part + sums_off + (unsigned)std::max(k - 3, 0) * NSAMP;
         const dim3 grid((unsigned)gx, (unsigned)(rows + (prev_rows > 0 ? 1 : 0)));
-        if (first) hipLaunchKernelGGL(k_sum3<true>, grid, dim3(BLOCK), 0, s, D, cols, C.r[k], C.r[k + 1], C.r[k + 2], part + off, prev_part, prev_rows, prev_sums);
-        else hipLaunchKernelGGL(k_sum3<false>, grid, dim3(BLOCK), 0, s, D, cols, C.r[k], C.r[k + 1], C.r[k + 2], part + off, prev_part, prev_rows, prev_sums);
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, grid, dim3(BLOCK), 0, s, D, cols, C.r[k], C.r[k + 1], C.r[k + 2], part + off, prev_part, prev_rows, prev_sums);
+        };
+        if (first && one) launch(k_sum3<true, true>);
+        else if (first) launch(k_sum3<true, false>);
+        else if (one) launch(k_sum3<false, true>);
+        else launch(k_sum3<false, false>);
         VI_LAUNCH_CHECK("sumcheck pass (sum under a common factor)");
         note(3, gx * rows);
         prev_part = part + off;
@@ -382,8 +386,12 @@ int prove_sum(const SumShape &S, const uint64_t *const *tables, uint64_t *const 
     for (int level = 0; level < 9; ++level) T.r[level] = level < rounds ? C.r[C.n_rounds - 1 - level] : 0;
     u64 *prev_sums = part + sums_off + (unsigned)std::max(k - 3, 0) * NSAMP;
     const dim3 grid((unsigned)((rows + BLOCK / 64 - 1) / (BLOCK / 64) + (prev_rows > 0 ? 3 : 0)));
-    if (first) hipLaunchKernelGGL(k_sum_tail<true>, grid, dim3(BLOCK), 0, s, D, (int)size, T, part + off, prev_part, prev_rows, prev_sums);
-    else hipLaunchKernelGGL(k_sum_tail<false>, grid, dim3(BLOCK), 0, s, D, (int)size, T, part + off, prev_part, prev_rows, prev_sums);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(BLOCK), 0, s, D, (int)size, T, part + off, prev_part, prev_rows, prev_sums);
+    };
+    if (first) launch(k_sum_tail<true, true>);
+    else if (k == C.late) launch(k_sum_tail<false, true>);
+    else launch(k_sum_tail<false, false>);
     VI_LAUNCH_CHECK("sumcheck tail (sum under a common factor)");
     note(rounds, rows);
     C.n_prior = C.n_rounds;
