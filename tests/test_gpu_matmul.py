@@ -77,3 +77,15 @@ def test_matmul_of_small_numbers(m, k, n, fill):
     ones = to_np(cp.gl_matmul(dA, to_dev(np.ones((k, 300), dtype=np.uint64))))[:, 299]        # every row
     want = A.sum(axis=1)
     assert np.array_equal(ones, np.where(want < 0, want.astype(np.uint64) + np.uint64(P), want.astype(np.uint64)))
+
+
+@pytest.mark.parametrize("m", list(range(1, 11)) + [13, 17, 21, 24])
+@pytest.mark.parametrize("k,n", [(9, 65), (1300, 129), (3000, 64), (700, 4097)])
+def test_few_rows(m, k, n):
+    """Every number of rows to a lane, one and several blocks of rows, one to 64 slices of the inner dimension."""
+    from verinf_amd.prover import cuda_primitives as cp
+    A, B = rand_field((m, k), m), rand_field((k, n), n)
+    A[0, :], B[:, -1] = P - 1, P - 1
+    got = to_np(cp.gl_matmul(to_dev(A), to_dev(B)))
+    cols = np.unique(np.linspace(0, n - 1, min(n, 3_000_000 // (m * k) + 2)).astype(int))
+    assert np.array_equal(got[:, cols], (A.astype(object).dot(B[:, cols].astype(object)) % P).astype(np.uint64))

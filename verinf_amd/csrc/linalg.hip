@@ -137,12 +137,29 @@ __global__ __launch_bounds__(BLOCK) void k_zero(u64 *__restrict__ out, i64 n) {
     if (e < n) out[e] = 0;
 }
 
+// The sums of the slices: 64 entries per workgroup, the slices dealt over its four wavefronts, eight of them in flight (one thread
+// per entry going through all of them: 13 us for 46 slices of 2804 entries, 18 for 64 of 1000; 4 this way).
 __global__ __launch_bounds__(BLOCK) void k_add_partials(const u64 *__restrict__ partial, u64 *__restrict__ out, i64 mn, int splits) {
-    const i64 e = (i64)blockIdx.x * BLOCK + threadIdx.x;
-    if (e >= mn) return;
-    u64 acc = partial[e];
-    for (int s = 1; s < splits; ++s) acc = gl::add(acc, partial[(i64)s * mn + e]);
-    out[e] = acc;
+    __shared__ u64 part[BLOCK / 64][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const i64 e = (i64)blockIdx.x * 64 + lane;
+    u64 acc = 0;
+    if (e < mn) {
+        constexpr int UN = 8;
+        for (int s0 = w; s0 < splits; s0 += UN * (BLOCK / 64)) {
+            u64 v[UN];
+#pragma unroll
+            for (int u = 0; u < UN; ++u) {
+                const int s = s0 + u * (BLOCK / 64);
+                v[u] = s < splits ? partial[(i64)s * mn + e] : 0;
+            }
+#pragma unroll
+            for (int u = 0; u < UN; ++u) acc = gl::add(acc, v[u]);
+        }
+    }
+    part[w][lane] = acc;
+    __syncthreads();
+    if (w == 0 && e < mn) out[e] = gl::add(gl::add(part[0][lane], part[1][lane]), gl::add(part[2][lane], part[3][lane]));
 }
 
 // TPR threads per row of M (a wavefront, or the whole workgroup when there are too few rows for a wavefront
@@ -198,9 +215,14 @@ __global__ __launch_bounds__(BLOCK) void k_poly_eval(const u64 *__restrict__ coe
 }
 
 // How a product on the VALU is cut up: rows of A a lane takes together (mb), wavefronts of a workgroup along the inner
-// dimension (ks), and slices of it over workgroups (splits), whose partial sums a second launch adds up.  About 8192
+// dimension (ks), and slices of it over workgroups (splits), whose partial sums a second launch adds up.  The rows are dealt
+// evenly over as few blocks of at most eight as there have to be, so that B is read no more often than that and no row is computed
+// twice (3 x 4096 x 16384: 161 -> 91 us, which two rows to a lane read twice; 5 rows 179 -> 109; 9 x 12000 x 12000, two blocks of 8,
+// 643 -> 427; seven rows to a lane are slower than
+// eight, 20 x 12000 x 12000 1205 against 945, and seven rows alone fastest as four and three).  About 8192
 // wavefronts in all, eight to a SIMD, with at least 16 terms each (4096 and 16384 measured within 10 % of it from one row
-// to 32, 32768 up to 25 % slower); fewer rows to a lane while even so there would be less than two wavefronts to a SIMD
+// to 32, 32768 up to 25 % slower; 4096 is up to 15 % faster at 10 M entries of B and 40 % slower at 288 M); fewer rows to a
+// lane while even so there would be less than two wavefronts to a SIMD
 // (24 x 760 x 1070: 21 -> 18 us).  One row against 32768 columns or more streams fastest with one wavefront to a workgroup
 // (1 x 4096 x 65536: 312 us, 6.9 TB/s; 360 us with four along the inner dimension); everything else takes four (12 x 4096
 // x 4096: 90 us, 103 with sixteen, which saves the second launch now and then but leaves CUs idle).
@@ -210,8 +232,10 @@ struct DirectPlan {
 DirectPlan plan_direct(i64 m, i64 k, i64 n) {
     DirectPlan D;
     const i64 cols = (n + 63) / 64, most = k / 16 > 1 ? k / 16 : 1;
-    D.mb = m >= 8 ? 8 : (m >= 4 ? 4 : (m >= 2 ? 2 : 1));
-    while (D.mb > 1 && cols * ((m + D.mb - 1) / D.mb) * most < 4096) D.mb >>= 1;
+    const i64 blocks = (m + 7) / 8;
+    D.mb = (int)((m + blocks - 1) / blocks);
+    if (D.mb == 7) D.mb = m == 7 ? 4 : 8;
+    while (D.mb > 1 && cols * ((m + D.mb - 1) / D.mb) * most < 4096) D.mb = (D.mb + 1) / 2;
     i64 want = 8192 / (cols * ((m + D.mb - 1) / D.mb));
     if (want > most) want = most;
     D.ks = (m == 1 && cols >= 512) || want < 3 ? 1 : 4;
@@ -263,14 +287,19 @@ int vi_gl_matmul(const uint64_t *A, const uint64_t *B, uint64_t *C, int64_t m, i
     if (splits > 1 && (!ws || ws_bytes < vi_gl_matmul_workspace_bytes(m, k, n)))
         return vi::fail(VI_ENOMEM, "vi_gl_matmul: workspace below %zu bytes", vi_gl_matmul_workspace_bytes(m, k, n));
     u64 *dst = splits > 1 ? (u64 *)ws : C;
-    if (D.mb == 1) launch_direct<1, 8>(D, A, B, dst, m, k, n, s);
-    if (D.mb == 2) launch_direct<2, 8>(D, A, B, dst, m, k, n, s);
-    if (D.mb == 4) launch_direct<4, 8>(D, A, B, dst, m, k, n, s);
-    if (D.mb == 8) launch_direct<8, 8>(D, A, B, dst, m, k, n, s);
+    switch (D.mb) {
+        case 1: launch_direct<1, 8>(D, A, B, dst, m, k, n, s); break;
+        case 2: launch_direct<2, 8>(D, A, B, dst, m, k, n, s); break;
+        case 3: launch_direct<3, 8>(D, A, B, dst, m, k, n, s); break;
+        case 4: launch_direct<4, 8>(D, A, B, dst, m, k, n, s); break;
+        case 5: launch_direct<5, 8>(D, A, B, dst, m, k, n, s); break;
+        case 6: launch_direct<6, 8>(D, A, B, dst, m, k, n, s); break;
+        default: launch_direct<8, 8>(D, A, B, dst, m, k, n, s); break;
+    }
     VI_LAUNCH_CHECK("k_matmul");
     if (splits > 1) {
         const i64 mn = m * n;
-        hipLaunchKernelGGL(k_add_partials, dim3((unsigned)((mn + BLOCK - 1) / BLOCK)), dim3(BLOCK), 0, s, (const u64 *)ws, C, mn, splits);
+        hipLaunchKernelGGL(k_add_partials, dim3((unsigned)((mn + 63) / 64)), dim3(BLOCK), 0, s, (const u64 *)ws, C, mn, splits);
         VI_LAUNCH_CHECK("k_add_partials");
     }
     return VI_OK;
