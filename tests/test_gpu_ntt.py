@@ -197,6 +197,30 @@ def test_lde_strided_rows_other_shift_and_legacy_encoder(cp):
     assert tuple(empty.shape) == (0, 32)
 
 
+@pytest.mark.parametrize("logK,log_rho", [(12, 1), (12, 2), (12, 3), (14, 2), (14, 4), (16, 3)])
+def test_lde_with_cosets_dealt_to_several_workgroups(cp, logK, log_rho):
+    """Tiles around the counts where the share of the cosets that a workgroup takes changes, and around full rounds of workgroups;
+    codewords beside and without the coefficients, which overwrite their messages."""
+    from verinf_amd import _lib
+    L = _lib.lib()
+    K, N, per_row = 1 << logK, 1 << (logK + log_rho), 1 << (logK - 12)
+    counts = [96, 97, 192, 193, 384, 385, 640, 641] + ([1023, 1024, 1025, 1409] if log_rho < 4 and logK < 16 else [])
+    for m in sorted({-(-tiles // per_row) for tiles in counts}):
+        d = rand_field_dev((m, K), m)
+        keep = d.clone()
+        out = cp.coset_lde(d, K, N, 7)
+        rows = sorted({0, m // 2, m - 1})
+        host, got = (np.ascontiguousarray(np.stack([to_np(t[r]) for r in rows])) for t in (keep, out))
+        assert np.array_equal(got, O.coset_lde_rows(host, K, N, 7)), m
+        ws = torch.empty(L.vi_coset_lde_workspace_bytes(m, K, N), dtype=torch.uint8, device="cuda")
+        again = torch.empty((m, N), dtype=torch.uint64, device="cuda")
+        _lib.check(L.vi_coset_lde_coeffs(d.data_ptr(), m, K, K, K, N, 7, d.data_ptr(), K, again.data_ptr(), N, ws.data_ptr(), ws.numel(),
+                                         _lib.stream_ptr()))
+        assert torch.equal(out, again), m
+        cp.ntt_forward_batched(d)
+        assert torch.equal(d, keep), m
+
+
 def test_lde_small_workspace_chunks_are_bit_identical(cp):
     """Forcing the library to process the rows in several chunks changes nothing."""
     from verinf_amd import _lib

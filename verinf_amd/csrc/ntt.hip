@@ -177,7 +177,7 @@ __global__ __launch_bounds__(NTHREADS, 4) void k_ntt_row(const PassArgs P0, cons
 // MRG: the coset factors split into shift^i (once), a power of two per input, and factors carried by the twiddle
 // tables of each coset (ntt_plan.hpp, append_coset_merged).
 template <int A2, bool MRG>
-__global__ __launch_bounds__(NTHREADS, VI_MID_MIN_WG) void k_lde_mid(const PassArgs Ai_in, const PassArgs Af_in) {
+__global__ __launch_bounds__(NTHREADS, VI_MID_MIN_WG) void k_lde_mid(const PassArgs Ai_in, const PassArgs Af_in, u32 whole, int log_parts) {
     PassArgs Ai = Ai_in, Af = Af_in;
     Ai.is_final = 1;
     Af.is_final = 0;
@@ -185,9 +185,13 @@ __global__ __launch_bounds__(NTHREADS, VI_MID_MIN_WG) void k_lde_mid(const PassA
     __shared__ u64 twi_i[16 << A2];
     __shared__ u64 twi_f[16 << A2];                        // MRG: the inner twiddles of the coset in hand
     const int tid = threadIdx.x;
-    const i64 tile = blockIdx.x;
+    // tiles from `whole` on: a workgroup per part of their cosets
+    const u32 extra = blockIdx.x < whole ? 0 : blockIdx.x - whole, part = extra & ((1u << log_parts) - 1);
+    const i64 tile = blockIdx.x < whole ? blockIdx.x : whole + (extra >> log_parts);
+    const int cosets = (1 << Af.log_rho) >> (blockIdx.x < whole ? 0 : log_parts), t0 = (int)part * cosets;
+    if (part) Ai.dst = nullptr;                            // the coefficients are written once
     constexpr int PER = (16 << A2) / NTHREADS > 0 ? (16 << A2) / NTHREADS : 1;
-    const u64 *src_f = MRG ? Af.twim : Af.twi;
+    const u64 *src_f = MRG ? Af.twim + ((size_t)t0 << Af.a) : Af.twi;
     u64 ti[PER], tf[PER];
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
@@ -209,18 +213,17 @@ __global__ __launch_bounds__(NTHREADS, VI_MID_MIN_WG) void k_lde_mid(const PassA
     __syncthreads();
     fused_stage2_inv<A2>(Ai, tile, tid, lds, coef);
     if (MRG) fused_twist<A2>(Af, tile, tid, coef);
-    const int rho = 1 << Af.log_rho;
-    for (int t = 0; t < rho; ++t) {
+    for (int t = t0; t < t0 + cosets; ++t) {
         __syncthreads();                                   // every thread is done reading the tile of the step before
         fused_stage1_fwd<A2, MRG>(Af, tile, tid, t, coef, twi_f, lds);
         __syncthreads();
         fused_stage2_fwd<A2, MRG>(Af, tile, tid, t, lds);
         // stage 1 of this coset is over everywhere, so its inner twiddles make way for the next coset's (fetched and
         // stored in one place: held in registers across either stage they cost the kernel its fourth workgroup per CU)
-        if (MRG && t + 1 < rho) {
+        if (MRG && t + 1 < t0 + cosets) {
 #pragma unroll
             for (int i = 0; i < PER; ++i)
-                if (tid + i * NTHREADS < (16 << A2)) twi_f[tid + i * NTHREADS] = src_f[((size_t)(t + 1) << Af.a) + tid + i * NTHREADS];
+                if (tid + i * NTHREADS < (16 << A2)) twi_f[tid + i * NTHREADS] = src_f[((size_t)(t + 1 - t0) << Af.a) + tid + i * NTHREADS];
         }
     }
 }
@@ -405,26 +408,41 @@ void launch_fast(const PassArgs &A, dim3 grid, dim3 block, hipStream_t s) {
     }
 }
 
+// The fused launch holds MID_RESIDENT workgroups at once, each going through the cosets of a tile one by one.  The tiles of its last,
+// partial round (or of all, where they are few) are dealt to several workgroups, a part of the cosets each, which repeat the inverse
+// half: as many parts as leave room for one more workgroup on every CU; half the cosets of up to 640 tiles where there are
+// eight or more of them.  us per extension, whole -> parts: 64 rows of 2^14 -> 2^16 70 -> 59, -> 2^17 123 -> 98; 275 rows 180 -> 167, 311 -> 287;
+// beyond those limits whole tiles are faster (128 rows -> 2^16 97 and 98, 192 rows 124 and 131).
+constexpr u32 MID_RESIDENT = 256 * VI_MID_MIN_WG;
+
+int mid_log_parts(u32 tiles, int log_rho) {
+    int log_parts = 0;
+    while (log_parts < log_rho && (tiles << (log_parts + 1)) <= MID_RESIDENT - 256) ++log_parts;
+    return log_parts == 0 && log_rho >= 3 && tiles <= 640 ? 1 : log_parts;
+}
+
 int launch_fused(const PassArgs &Ai_in, const PassArgs &Af_in, hipStream_t s) {
     PassArgs Ai = Ai_in, Af = Af_in;
     Ai.uniform = Af.uniform = 1;
     Ai.n1_valid = Af.n1_valid = 16;
     const i64 tiles = pass_tiles(Ai);
     if (tiles > 0x7FFFFFFF) return vi::fail(VI_EINVAL, "ntt pass: %lld tiles exceed the grid limit", (long long)tiles);
-    dim3 grid((unsigned)tiles), block(NTHREADS);
+    const u32 rest = (u32)tiles % MID_RESIDENT, whole = (u32)tiles - rest;
+    const int log_parts = mid_log_parts(rest, Af.log_rho);
+    dim3 grid((unsigned)(whole + (rest << log_parts))), block(NTHREADS);
     if (Af.twm && Af.twim && Af.merge_unit > 0) {
         switch (Ai.a - FAST_A1) {
-            case 1: hipLaunchKernelGGL((k_lde_mid<1, true>), grid, block, 0, s, Ai, Af); break;
-            case 2: hipLaunchKernelGGL((k_lde_mid<2, true>), grid, block, 0, s, Ai, Af); break;
-            case 3: hipLaunchKernelGGL((k_lde_mid<3, true>), grid, block, 0, s, Ai, Af); break;
-            default: hipLaunchKernelGGL((k_lde_mid<4, true>), grid, block, 0, s, Ai, Af); break;
+            case 1: hipLaunchKernelGGL((k_lde_mid<1, true>), grid, block, 0, s, Ai, Af, whole, log_parts); break;
+            case 2: hipLaunchKernelGGL((k_lde_mid<2, true>), grid, block, 0, s, Ai, Af, whole, log_parts); break;
+            case 3: hipLaunchKernelGGL((k_lde_mid<3, true>), grid, block, 0, s, Ai, Af, whole, log_parts); break;
+            default: hipLaunchKernelGGL((k_lde_mid<4, true>), grid, block, 0, s, Ai, Af, whole, log_parts); break;
         }
     } else {
         switch (Ai.a - FAST_A1) {
-            case 1: hipLaunchKernelGGL((k_lde_mid<1, false>), grid, block, 0, s, Ai, Af); break;
-            case 2: hipLaunchKernelGGL((k_lde_mid<2, false>), grid, block, 0, s, Ai, Af); break;
-            case 3: hipLaunchKernelGGL((k_lde_mid<3, false>), grid, block, 0, s, Ai, Af); break;
-            default: hipLaunchKernelGGL((k_lde_mid<4, false>), grid, block, 0, s, Ai, Af); break;
+            case 1: hipLaunchKernelGGL((k_lde_mid<1, false>), grid, block, 0, s, Ai, Af, whole, log_parts); break;
+            case 2: hipLaunchKernelGGL((k_lde_mid<2, false>), grid, block, 0, s, Ai, Af, whole, log_parts); break;
+            case 3: hipLaunchKernelGGL((k_lde_mid<3, false>), grid, block, 0, s, Ai, Af, whole, log_parts); break;
+            default: hipLaunchKernelGGL((k_lde_mid<4, false>), grid, block, 0, s, Ai, Af, whole, log_parts); break;
         }
     }
     VI_LAUNCH_CHECK("k_lde_mid");
@@ -580,27 +598,29 @@ bool small_ntt_passes_pay(i64 m, int logn, const Split &sp) {
 // columns (digits of 2^5 .. 2^8: 32 .. 4, runs of 256 .. 32 bytes).
 //
 // k_ntt_fast: 7.8 us a launch, one wavefront's chain, and 2.95 per million.  With K = L L the middle two are one launch whose
-// workgroups go through the cosets one after the other: 21 + 7 per coset for all three, and 1.84 per million (memory hides
-// behind the chain).
+// workgroups go through the cosets of their part one after the other: 21 + 7 per coset of a part for all three, and 1.84 per million
+// (memory hides behind the chain), 3.0 where tiles are dealt out in parts.
 //
-// Fitted to a sweep over K, 1 to 32 cosets and batches of 1 .. 2^24 points written, where the choice loses 0.2 % on average and
-// 16 % at most (k_small_pass, k_ntt_fast: 2^14 -> 2^16 one row 18, 53; 64 rows 63, 69; 256 rows 209, 141; 1 x 2^16 -> 2^21 48,
-// 309).
+// Fitted to a sweep over K, 1 to 32 cosets and batches of 1 .. 2^24 points written (k_small_pass, k_ntt_fast: 2^14 -> 2^16 one row
+// 18, 40; 32 rows 44, 48; 64 rows 66, 59; 256 rows 209, 141).
 double small_passes_us(const Split &sp, double million) {
     static constexpr double per_million[4] = {3.2, 3.5, 5.05, 7.7};
     double us = 0;
     for (int q = 0; q < sp.p; ++q) us += 2 * 3.7 + per_million[sp.a[q] - 5] * million;
     return us;
 }
-double fast_passes_us(const Split &sp, int log_rho, double million) {
-    if (sp.p == 2 && sp.a[0] == sp.a[1] && sp.a[0] >= 6) return 21 + 7.0 * (double)(1 << log_rho) + 2 * 1.84 * million;
+double fast_passes_us(const Split &sp, int log_rho, double tiles, double million) {
+    if (sp.p == 2 && sp.a[0] == sp.a[1] && sp.a[0] >= 6) {
+        const int log_parts = tiles < MID_RESIDENT ? mid_log_parts((u32)tiles, log_rho) : 0;
+        return 21 + 7.0 * (double)((1 << log_rho) >> log_parts) + 2 * (log_parts ? 3.0 : 1.84) * million;
+    }
     return sp.p * (2 * 7.8 + 2.95 * million);
 }
 bool small_lde_passes_pay(i64 m, int logK, int logN, const Split &sp) {
     const int log_rho = logN - logK;
     if (logK < 10 || logK > 18 || log_rho > 15 || !small_digits(sp)) return false;      // cosets: the grid's second dimension
     const double million = (double)m * (double)(((i64)1 << logK) + ((i64)1 << logN)) * 1e-6;
-    return small_passes_us(sp, million) < fast_passes_us(sp, log_rho, million);
+    return small_passes_us(sp, million) < fast_passes_us(sp, log_rho, (double)m * (double)((i64)1 << logK) / TILE, million);
 }
 
 // Which launches an extension takes
