@@ -51,6 +51,19 @@ def test_padded_rows(m, ell, width, stride):
     assert np.array_equal(to_np(padded), want)
 
 
+@pytest.mark.parametrize("m,ell,width", [(1023, 300, 512), (1025, 511, 512), (8200, 40, 64), (30000, 7, 19), (200000, 1, 3), (37, 9001, 16383), (150, 40000, 65536)])
+def test_padded_rows_in_larger_batches(m, ell, width):
+    """One, four and eight words a thread; rows whose words do not divide over the lanes."""
+    from verinf_amd.prover import cuda_primitives as cp
+    seed = bytes(range(7, 39))
+    messages = torch.randint(0, 1 << 62, (m, ell), dtype=torch.int64, device="cuda").view(torch.uint64)
+    padded = torch.empty((m, width), dtype=torch.uint64, device="cuda")
+    cp.pad_rows(torch.tensor(list(seed), dtype=torch.uint8, device="cuda"), 11, messages, padded)
+    assert torch.equal(padded[:, :ell], messages)
+    for r in {0, 1, m // 2, m - 1}:
+        assert np.array_equal(to_np(padded[r, ell:]), O.row_prg(seed, 11 + r, 1, width - ell)[0]), r
+
+
 def test_a_message_of_one_chunk_without_workspace_is_refused():
     from verinf_amd import _lib
     mat = to_dev(rand_field((8, 64), 1))

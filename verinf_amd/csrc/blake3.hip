@@ -41,10 +41,21 @@ __host__ __device__ constexpr int sched(int r, int i) {
 
 __device__ __forceinline__ u32 rotr(u32 x, int n) { return __builtin_amdgcn_alignbit(x, x, n); }
 
+// a + b + m in one instruction, out of the optimiser's reach
+__device__ __forceinline__ u32 add3(u32 a, u32 b, u32 m) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    u32 r;
+    asm("v_add3_u32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(m));
+    return r;
+#else
+    return a + b + m;
+#endif
+}
+
 #define B3_G(a, b, c, d, mx, my)            \
-    a = a + b + (mx); d = rotr(d ^ a, 16);  \
+    a = add3(a, b, mx); d = rotr(d ^ a, 16);  \
     c = c + d;        b = rotr(b ^ c, 12);  \
-    a = a + b + (my); d = rotr(d ^ a, 8);   \
+    a = add3(a, b, my); d = rotr(d ^ a, 8);   \
     c = c + d;        b = rotr(b ^ c, 7);
 
 template <int R>
@@ -348,15 +359,43 @@ __global__ __launch_bounds__(BLOCK) void k_merkle_subtree(const u32 *__restrict_
 // that stores are coalesced; the reference gives a whole row to one thread.
 // row = row_indices[r] when row_indices is given, else the 32-bit sum row_offset + r (the
 // reference's contiguous variant computes the row number in uint32).
-__device__ __forceinline__ u64 prg_word(const u32 *__restrict__ seed, u64 row, i64 k) {
-    u32 m[16], cv[8];
+//
+// Seven of the eight G of the first round see neither k nor anything that came of it: they are the row's (PrgRow), and a thread
+// that hashes several values of a row runs them once.
+struct PrgRow {
+    u32 m[16], s[16];                          // message words but for k; the state, the second G of its diagonals left out
+};
+
+__device__ __forceinline__ PrgRow prg_row(const u32 *__restrict__ seed, u64 row) {
+    PrgRow R;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) { m[i] = seed[i]; cv[i] = IV[i]; }
-    m[8] = (u32)row; m[9] = (u32)(row >> 32);
-    m[10] = (u32)k;  m[11] = (u32)((u64)k >> 32);
-    m[12] = m[13] = m[14] = m[15] = 0;
-    compress(cv, m, 0, 48, CHUNK_START | CHUNK_END | ROOT);
-    const u64 raw = ((u64)cv[1] << 32) | cv[0];
+    for (int i = 0; i < 8; ++i) { R.m[i] = seed[i]; R.s[i] = IV[i]; }
+    R.m[8] = (u32)row; R.m[9] = (u32)(row >> 32);
+    R.m[10] = R.m[11] = R.m[12] = R.m[13] = R.m[14] = R.m[15] = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) R.s[8 + i] = IV[i];
+    R.s[12] = R.s[13] = 0;
+    R.s[14] = 48;
+    R.s[15] = CHUNK_START | CHUNK_END | ROOT;
+    B3_G(R.s[0], R.s[4], R.s[8], R.s[12], R.m[0], R.m[1])
+    B3_G(R.s[1], R.s[5], R.s[9], R.s[13], R.m[2], R.m[3])
+    B3_G(R.s[2], R.s[6], R.s[10], R.s[14], R.m[4], R.m[5])
+    B3_G(R.s[3], R.s[7], R.s[11], R.s[15], R.m[6], R.m[7])
+    B3_G(R.s[0], R.s[5], R.s[10], R.s[15], R.m[8], R.m[9])
+    B3_G(R.s[2], R.s[7], R.s[8], R.s[13], 0, 0)
+    B3_G(R.s[3], R.s[4], R.s[9], R.s[14], 0, 0)
+    return R;
+}
+
+__device__ __forceinline__ u64 prg_word(const PrgRow &R, i64 k) {
+    u32 m[16], s[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) { m[i] = R.m[i]; s[i] = R.s[i]; }
+    m[10] = (u32)k; m[11] = (u32)((u64)k >> 32);
+    B3_G(s[1], s[6], s[11], s[12], m[10], m[11])
+    b3_round<1>(s, m); b3_round<2>(s, m); b3_round<3>(s, m);
+    b3_round<4>(s, m); b3_round<5>(s, m); b3_round<6>(s, m);
+    const u64 raw = ((u64)(s[1] ^ s[9]) << 32) | (s[0] ^ s[8]);
     return raw >= 0xFFFFFFFF00000001ull ? raw - 0xFFFFFFFF00000001ull : raw;
 }
 
@@ -365,18 +404,25 @@ __global__ __launch_bounds__(BLOCK) void k_row_prg(const u32 *__restrict__ seed,
     const i64 g = (i64)blockIdx.x * BLOCK + threadIdx.x;
     if (g >= n_rows * slack) return;
     const i64 r = g / slack, k = g - r * slack;
-    out[r * out_stride + k] = prg_word(seed, row_indices ? row_indices[r] : (u64)(u32)(row_offset + (u32)r), k);
+    out[r * out_stride + k] = prg_word(prg_row(seed, row_indices ? row_indices[r] : (u64)(u32)(row_offset + (u32)r)), k);
 }
 
 // Message and pad of a padded row in one launch: out[r][k] = messages[r][k] for k < ell, and the value of k_row_prg at
-// k - ell behind it.  The hashing is bound by VALU issue, so the copy rides along (333 rows of 8192 + 8192: 9 us as a launch
-// of its own).
+// k - ell behind it.  The hashing is bound by VALU issue (600 instructions a value), so the copy rides along (333 rows of
+// 8192 + 8192: 9 us as a launch of its own).  2^log_lanes threads of a workgroup take words first, first + step, ... of a row,
+// spread over the whole row so that every workgroup copies and hashes its share; the values of a thread have one PrgRow.
 __global__ __launch_bounds__(BLOCK) void k_pad_rows(const u32 *__restrict__ seed, u32 row_offset, const u64 *__restrict__ messages, i64 in_stride,
-                                                    i64 ell, i64 n_rows, i64 width, u64 *__restrict__ out) {
-    const i64 g = (i64)blockIdx.x * BLOCK + threadIdx.x;
-    if (g >= n_rows * width) return;
-    const i64 r = g / width, k = g - r * width;
-    out[g] = k < ell ? messages[r * in_stride + k] : prg_word(seed, (u64)(u32)(row_offset + (u32)r), k - ell);
+                                                    i64 ell, i64 n_rows, u32 segments, int log_lanes, i64 width, u64 *__restrict__ out) {
+    const u32 group = blockIdx.x / segments;
+    const i64 r = ((i64)group * BLOCK + threadIdx.x) >> log_lanes, step = (i64)segments << log_lanes;
+    if (r >= n_rows) return;
+    const u64 *from = messages + r * in_stride;
+    u64 *to = out + r * width;
+    i64 k = ((i64)(blockIdx.x - group * segments) << log_lanes) + (threadIdx.x & ((1 << log_lanes) - 1));
+    for (; k < ell; k += step) to[k] = from[k];
+    if (k >= width) return;
+    const PrgRow R = prg_row(seed, (u64)(u32)(row_offset + (u32)r));
+    for (; k < width; k += step) to[k] = prg_word(R, k - ell);
 }
 
 // The test-combiner challenge of the protocol (prover/protocol.py:127-135, device twin
@@ -613,10 +659,19 @@ int vi_pad_rows(const uint8_t *seed, int64_t row_offset, const uint64_t *message
     if (n_rows == 0 || width == 0) return VI_OK;
     if (!out || (ell > 0 && !messages) || (width > ell && !seed)) return vi::fail(VI_EINVAL, "vi_pad_rows: null pointer");
     if ((uintptr_t)seed & 3) return vi::fail(VI_EINVAL, "vi_pad_rows: seed must be 4-byte aligned");
-    const i64 blocks = (n_rows * width + BLOCK - 1) / BLOCK;
-    if (blocks > 0x7FFFFFFF) return vi::fail(VI_EINVAL, "vi_pad_rows: %lld words exceed one launch", (long long)(n_rows * width));
-    hipLaunchKernelGGL(k_pad_rows, dim3((unsigned)blocks), dim3(BLOCK), 0, (hipStream_t)stream, (const u32 *)seed, (u32)row_offset, messages,
-                       (i64)in_stride, (i64)ell, (i64)n_rows, (i64)width, out);
+    // Eight or four words a thread, in batches that fill the chip with them (us with 1, 4, 8: 1000 rows of 30000 + 35536 764, 678, 650; 333 of
+    // 8192 + 8192 64.7, 56.6, 57.2; 40 of 5000 + 11384 15.0, 13.0, 16.1; 3000 of 300 + 212 31.8, 18.0, 18.0, where the lanes of a wavefront
+    // also copy or hash together), one in smaller ones, which wait for a thread's chain (400 of 300 + 212 7.5, 7.8).  A row has up to
+    // 256 lanes, sixteen (a run of 128 bytes) before a lane takes a second word.
+    const i64 words = n_rows * width;
+    const int log_per = words >= ((i64)1 << 23) ? 3 : words >= ((i64)1 << 19) ? 2 : 0;
+    int log_lanes = 0;
+    while ((1 << log_lanes) < BLOCK && ((i64)1 << (log_lanes + (log_lanes >= 4 ? log_per : 0))) < width) ++log_lanes;
+    const i64 units = (width + ((i64)1 << log_lanes) - 1) >> log_lanes, segments = log_lanes < 8 ? 1 : (units + (1 << log_per) - 1) >> log_per;
+    const i64 groups = (n_rows + (BLOCK >> log_lanes) - 1) / (BLOCK >> log_lanes);
+    if (groups > 0x7FFFFFFF / segments) return vi::fail(VI_EINVAL, "vi_pad_rows: %lld words exceed one launch", (long long)(n_rows * width));
+    hipLaunchKernelGGL(k_pad_rows, dim3((unsigned)(groups * segments)), dim3(BLOCK), 0, (hipStream_t)stream, (const u32 *)seed, (u32)row_offset, messages,
+                       (i64)in_stride, (i64)ell, (i64)n_rows, (u32)segments, log_lanes, (i64)width, out);
     VI_LAUNCH_CHECK("k_pad_rows");
     return VI_OK;
 }
