@@ -204,6 +204,7 @@ def lde(so):
     for logK, log_rho, m, w in ((3, 1, 300, 5), (6, 2, 70, 64), (10, 3, 2, 600), (11, 3, 1, 2048), (13, 1, 2, 5000), (13, 2, 1, 8192), (14, 0, 1, 100),
                                 (14, 2, 1, 9000)):
         check(logK, log_rho, m, w, 11)
+    check(10, 2, 257, 1000, 11)                                # rows in one launch
     print("lde", flush=True)
 
 

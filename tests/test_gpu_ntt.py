@@ -197,6 +197,43 @@ def test_lde_strided_rows_other_shift_and_legacy_encoder(cp):
     assert tuple(empty.shape) == (0, 32)
 
 
+@pytest.mark.parametrize("logK,log_rho", [(10, 1), (10, 2), (10, 3), (11, 1), (11, 2), (11, 3), (12, 1), (12, 2)])
+def test_lde_of_rows_in_one_launch(cp, logK, log_rho):
+    """Batches at the limit where they begin and with partly filled tiles; strided sources of any width, strided coefficients and
+    codewords, coefficients in place, from coefficients, and rows in chunks."""
+    from verinf_amd import _lib
+    L = _lib.lib()
+    K, N = 1 << logK, 1 << (logK + log_rho)
+    limit = (1 << 22) // N
+    for m, width in ((limit, K), (limit + 1, K - 1), (limit + 7, K // 2 + 3), (limit // 4, 1), (limit // 4 - 1, K)):
+        src = rand_field_dev((m, K + 3), m + width)[:, :width]
+        rows = sorted({0, 1, m // 2, m - 1})
+        host = np.ascontiguousarray(np.stack([to_np(src[r].contiguous()) for r in rows]))
+        padded = np.zeros((len(rows), K), dtype=np.uint64)
+        padded[:, :width] = host
+        want, want_c = O.coset_lde_rows(host, K, N, 11), O.ntt_rows(padded, inverse=True)
+        one = L.vi_coset_lde_min_workspace_bytes(K, N)
+        ws = torch.empty(one * (m // 3 + 1), dtype=torch.uint8, device="cuda")
+        out = torch.full((m, N + 5), 7, dtype=torch.int64, device="cuda").view(torch.uint64)
+        co = torch.full((m, K + 2), 9, dtype=torch.int64, device="cuda").view(torch.uint64)
+        pick = lambda t, n: np.stack([to_np(t[r, :n].contiguous()) for r in rows])  # noqa: E731
+        _lib.check(L.vi_coset_lde_coeffs(src.data_ptr(), m, width, K + 3, K, N, 11, co.data_ptr(), K + 2, out.data_ptr(), N + 5,
+                                         ws.data_ptr(), ws.numel(), _lib.stream_ptr()))
+        assert np.array_equal(pick(out, N), want) and np.array_equal(pick(co, K), want_c), (m, width)
+        assert bool((out.view(torch.int64)[:, N:] == 7).all()) and bool((co.view(torch.int64)[:, K:] == 9).all())
+        again = torch.empty((m, N), dtype=torch.uint64, device="cuda")
+        _lib.check(L.vi_coset_lde(src.data_ptr(), m, width, K + 3, K, N, 11, again.data_ptr(), N, ws.data_ptr(), ws.numel(), _lib.stream_ptr()))
+        assert torch.equal(again, out[:, :N])
+        again.zero_()
+        _lib.check(L.vi_coset_extend(co.data_ptr(), m, K, K + 2, K, N, 11, again.data_ptr(), N, ws.data_ptr(), ws.numel(), _lib.stream_ptr()))
+        assert torch.equal(again, out[:, :N])
+        own = torch.zeros((m, K), dtype=torch.uint64, device="cuda")
+        own[:, :width] = src
+        _lib.check(L.vi_coset_lde_coeffs(own.data_ptr(), m, K, K, K, N, 11, own.data_ptr(), K, again.data_ptr(), N, ws.data_ptr(), ws.numel(),
+                                         _lib.stream_ptr()))
+        assert torch.equal(again, out[:, :N]) and torch.equal(own, co[:, :K])
+
+
 @pytest.mark.parametrize("logK,log_rho", [(12, 1), (12, 2), (12, 3), (14, 2), (14, 4), (16, 3)])
 def test_lde_with_cosets_dealt_to_several_workgroups(cp, logK, log_rho):
     """Tiles around the counts where the share of the cosets that a workgroup takes changes, and around full rounds of workgroups;

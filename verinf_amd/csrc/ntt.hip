@@ -167,6 +167,44 @@ __global__ __launch_bounds__(NTHREADS, 4) void k_ntt_row(const PassArgs P0, cons
     fast_stage2<4, INV, UNI>(P1, tile, tid, 0, lds);
 }
 
+// Codewords of rows of 2^10 .. 2^12 coefficients in one launch: one read of the coefficients, one write of the codewords, where
+// passes write and read all cosets once more.  Bound by VALU issue: 130 instructions a word at K = 2^10, four cosets, 272 us for
+// 2^26 words of a floor of 255 (and 68 for the coefficients); whole extensions of 2^26 words, before and after: 2^10 -> 2^12 494 and 340 us, 2^11 -> 2^13
+// 562 and 355, 2^12 -> 2^14 485 and 424.  A workgroup has all cosets of a row where they fit its tile; else their workgroups
+// follow each other on one XCD, whose L2 puts the lines together (written 1.13 times at 2^12 -> 2^14).
+template <int A0, int LR>
+__global__ __launch_bounds__(NTHREADS, 4) void k_lde_row(const LdeRow A) {
+    using S = LdeRowShape<A0, LR>;
+    __shared__ u64 lds[TILE + 256];
+    __shared__ u64 twi[256];
+    const int tid = threadIdx.x;
+    u32 group = blockIdx.x / S::PARTS, part = blockIdx.x % S::PARTS;
+    if (S::PARTS > 1 && (gridDim.x & (8 * S::PARTS - 1)) == 0) {
+        // the tiles of a row, whose words alternate in the codeword, one after the other on one XCD
+        const u32 xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+        part = slot % S::PARTS;
+        group = (slot / S::PARTS) * 8 + xcd;
+    }
+    const u64 tw_mine = A.twi[tid];
+    u64 coef[S::ROWS << A0];
+    lde_row_load<A0, LR>(A, group, tid, coef);
+    static_for<0, S::PARTS>([&](auto p_) {
+        constexpr int p = decltype(p_)::value;
+        if (S::PARTS == 1 || part == p) lde_row_stage0<A0, LR, p * S::COSETS>(A, tid, coef, lds);
+    });
+    twi[twi_slot<4, true>(tid >> 4, tid & 15)] = tw_mine;
+    __syncthreads();
+    u64 reg[16];
+    row_gather(lds, tid, reg);
+    __syncthreads();
+    PassArgs P{};
+    P.a = 8;
+    P.is_final = 1;
+    fast_stage1<4, false, false, true>(P, 0, tid, 0, 0xFFFFu, reg, reg, twi, lds);
+    __syncthreads();
+    lde_row_store<A0, LR>(A, group, (int)part * S::COSETS, tid, lds);
+}
+
 // The last inverse pass and the first forward pass of a coset extension in one launch (fused_stage2_inv): the
 // coefficients stay in registers between the two, so they are neither written to nor read back from HBM (unless the
 // caller wants them), and the rho cosets are expanded by a loop inside the workgroup.
@@ -364,6 +402,7 @@ int get_pre(int logK, int logN, u64 shift, const u64 **out, CosetPin &pin) {
             if (int rc = free_oldest_pre(dev)) return rc;
         CosetTable T;
         std::vector<u64> h = make_coset_pre(logK, logN, shift);
+        if (coset_rows_ok(logK, logN)) append_coset_rows(logK, logN, h);
         if (coset_mergeable(logK, logN)) append_coset_merged(logK, logN, h);
         int rc = upload(h, &T.words);
         if (rc) return rc;
@@ -515,6 +554,20 @@ int launch_row(const PassArgs &P0, const PassArgs &P1, hipStream_t s) {
     return VI_OK;
 }
 
+template <int A0>
+void launch_lde_row(const LdeRow &A, int log_rho, hipStream_t s) {
+    const i64 pairs = A.n_rows << log_rho;
+    constexpr int per = 16 >> A0;
+    const dim3 grid((unsigned)((pairs + per - 1) / per)), block(NTHREADS);
+    switch (log_rho) {
+        case 1: hipLaunchKernelGGL((k_lde_row<A0, 1>), grid, block, 0, s, A); break;
+        case 2: hipLaunchKernelGGL((k_lde_row<A0, 2>), grid, block, 0, s, A); break;
+        default:
+            if constexpr (A0 <= 3) hipLaunchKernelGGL((k_lde_row<A0, 3>), grid, block, 0, s, A);
+            break;
+    }
+}
+
 // rows per launch so that grids stay below 2^31 tiles
 i64 max_rows_per_launch(int logn) { return ((i64)1 << 40) >> logn; }
 
@@ -623,9 +676,20 @@ bool small_lde_passes_pay(i64 m, int logK, int logN, const Split &sp) {
     return small_passes_us(sp, million) < fast_passes_us(sp, log_rho, (double)m * (double)((i64)1 << logK) / TILE, million);
 }
 
+// Extensions of K = 2^10 .. 2^12 by two, four or eight as one launch to the coefficients (k_ntt_row) and one to the codewords
+// (k_lde_row), from 2^20 .. 2^22 points written, where the shorter chains of ntt_small.hpp meet it.  us, the better of the other
+// routes and this one: 2^20 points 2^10 -> 2^12 22 and 23, -> 2^13 26 and 23, -> 2^11 18 and 24; 2^21 27 and 27, 37 and 27, 27 and 29;
+// 2^12 -> 2^14 28 and 29, with 2^21 40 and 33; 2^24 points 2^10 -> 2^12 137 and 88, 2^11 -> 2^13 153 and 99, 2^12 -> 2^14 136 and 118.
+bool row_lde_pays(i64 m, int logK, int logN) {
+    if (!row_launch_on() || !coset_rows_ok(logK, logN)) return false;
+    const int log_least = logK == TILE_LOG ? 21 : (logN - logK >= 2 ? 20 : 22);
+    return m >= (((i64)1 << log_least) >> logN);
+}
+
 // Which launches an extension takes
-enum LdeRoute { LDE_PASSES, LDE_SINGLE, LDE_SMALL_PASSES };
+enum LdeRoute { LDE_PASSES, LDE_SINGLE, LDE_SMALL_PASSES, LDE_ROWS };
 LdeRoute lde_route(i64 m, int logK, int logN, bool in_place, const Split &sp) {
+    if (row_lde_pays(m, logK, logN)) return LDE_ROWS;
     if (small_lde_pays(m, logK, logN, in_place)) return LDE_SINGLE;
     if (logK == SMALL_MAX_LOG && single_round_of_rows(m, logN - logK, in_place)) return LDE_SINGLE;
     return small_lde_passes_pay(m, logK, logN, sp) ? LDE_SMALL_PASSES : LDE_PASSES;
@@ -745,6 +809,7 @@ int64_t vi_coset_lde_launches(int64_t m, int64_t K, int64_t N, size_t ws_bytes) 
     if (chunk > max_lde_chunk(vi::ilog2(K), vi::ilog2(N))) chunk = max_lde_chunk(vi::ilog2(K), vi::ilog2(N));
     const i64 n_chunks = (m + chunk - 1) / chunk;         // balancing keeps the chunk count
     chunk = (m + n_chunks - 1) / n_chunks;
+    if (route == LDE_ROWS) return 2 * n_chunks;
     // the pass list of one chunk, planned with placeholder addresses (only their being null or not matters)
     const int logK = vi::ilog2(K), logN = vi::ilog2(N);
     Tables Ti{}, Tf{};
@@ -778,6 +843,33 @@ int zero_rows(u64 *dst, i64 m, i64 cols, i64 stride, hipStream_t s) {
     if (blocks > 65536) blocks = 65536;
     hipLaunchKernelGGL(k_zero_rows, dim3((unsigned)blocks), dim3(NTHREADS), 0, s, dst, m, cols, stride);
     VI_LAUNCH_CHECK("k_zero_rows");
+    return VI_OK;
+}
+
+// LDE_ROWS over a chunk: the values in R to coefficients at `coeffs` (Ti: their tables; null when R has coefficients), and on to R.out
+int row_extension(LdeRow R, const Tables *Ti, u64 *coeffs, i64 coeffs_stride, int logK, int log_rho, hipStream_t s) {
+    if (Ti) {
+        PassArgs P0 = base_pass(*Ti, 0, R.n_rows), P1 = base_pass(*Ti, 1, R.n_rows);
+        P0.src = R.src;
+        P0.src_width = R.width;
+        P0.src_row_stride = R.src_stride;
+        P0.canon_src = 1;
+        P1.dst = coeffs;
+        P1.src_row_stride = (i64)1 << logK;
+        P1.dst_row_stride = coeffs_stride;
+        if (int rc = launch_row(P0, P1, s)) return rc;
+        R.src = coeffs;
+        R.width = (i64)1 << logK;
+        R.src_stride = coeffs_stride;
+        R.canon_src = 0;
+    }
+    if (!R.out) return VI_OK;
+    switch (logK) {
+        case 10: launch_lde_row<2>(R, log_rho, s); break;
+        case 11: launch_lde_row<3>(R, log_rho, s); break;
+        default: launch_lde_row<4>(R, log_rho, s); break;
+    }
+    VI_LAUNCH_CHECK("k_lde_row");
     return VI_OK;
 }
 
@@ -818,6 +910,12 @@ int coset_lde_impl(const char *who, const uint64_t *in, int64_t m, int64_t width
     if (!rc) rc = get_pre(logK, logN, shift, &pre, pin);
     if (rc) return rc;
     const LdeRoute route = lde_route(m, logK, logN, coeffs == in, Ti->sp);
+    const Tables *TiRow = nullptr, *TfRow = nullptr;
+    if (route == LDE_ROWS) {
+        rc = get_tables(logK, 1, &TiRow, true);
+        if (!rc) rc = get_tables(logK, 0, &TfRow, true);
+        if (rc) return rc;
+    }
     if (route == LDE_SINGLE) {
         SmallLde S{};
         S.tab_inv = Ti->full;
@@ -843,10 +941,17 @@ int coset_lde_impl(const char *who, const uint64_t *in, int64_t m, int64_t width
     }
     // the split form of the coset factors: its tables lie behind the N words of pre
     static const bool use_merged = []() { const char *e = getenv("VI_LDE_MERGED"); return !e || e[0] != '0'; }();
-    const u64 *merged = (use_merged && coset_mergeable(logK, logN)) ? pre + N : nullptr;
+    const u64 *merged = (use_merged && coset_mergeable(logK, logN)) ? pre + (coset_rows_ok(logK, logN) ? 2 * N : N) : nullptr;
     const bool small = route == LDE_SMALL_PASSES;
     for (i64 lo = 0; lo < m; lo += chunk) {
         i64 cnt = (m - lo < chunk) ? (m - lo) : chunk;
+        if (route == LDE_ROWS) {
+            const LdeRow R{in + lo * in_stride, cnt, width, in_stride, 1, out ? out + lo * out_stride : nullptr, out_stride, pre, pre + N, TfRow->twi[1]};
+            rc = row_extension(R, in_is_coeffs ? nullptr : TiRow, coeffs ? coeffs + lo * coeffs_stride : (u64 *)ws,
+                               coeffs ? coeffs_stride : K, logK, logN - logK, (hipStream_t)stream);
+            if (rc) return rc;
+            continue;
+        }
         std::vector<PassArgs> passes;
         build_lde_passes(*Ti, *Tf, pre, logN, in + lo * in_stride, width, in_stride, out ? out + lo * out_stride : nullptr,
                          out_stride, (u64 *)ws, cnt, passes, coeffs ? coeffs + lo * coeffs_stride : nullptr, coeffs_stride,

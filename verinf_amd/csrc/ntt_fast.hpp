@@ -800,6 +800,106 @@ VI_HD void row_gather(const u64 *lds, int tid, u64 (&reg)[16]) {
     for (int n1 = 0; n1 < 16; ++n1) reg[n1] = lds[c * ROW_ST + (n1 << 4) + n2];
 }
 
+// The forward half of a coset extension of rows of 2^(A0 + 8) coefficients, codewords in one launch (row_stage0 and its last
+// digit with the cosets beside the rows).  A tile is 16 >> A0 pairs (row, coset) of PARTS tiles per row or ROWS rows per tile.
+struct LdeRow {
+    const u64 *src;                            // coefficients, or what vi_coset_extend was given
+    i64 n_rows, width, src_stride;
+    int canon_src;
+    u64 *out;
+    i64 out_stride;
+    const u64 *pre, *tw, *twi;                 // shift^i; w_K^(k r) w_N^(t r) at [t][k][r]; w_256^(n2 k1) at [n2][k1]
+};
+template <int A0, int LR>
+struct LdeRowShape {
+    static constexpr int E0 = 1 << A0, NSUB = 16 / E0, RHO = 1 << LR;
+    static constexpr int COSETS = RHO < NSUB ? RHO : NSUB, ROWS = NSUB / COSETS, PARTS = RHO / COSETS;
+    static_assert(A0 + LR <= 6, "w_N^(256 t) is a power of two");
+};
+
+// coefficients r, r + 256, ... of each row of the tile, times shift^i
+template <int A0, int LR>
+VI_HD void lde_row_load(const LdeRow &A, i64 group, int tid, u64 (&coef)[LdeRowShape<A0, LR>::ROWS << A0]) {
+    using S = LdeRowShape<A0, LR>;
+    u64 pw[S::E0];
+    u32 ok = 0;
+#pragma unroll
+    for (int i = 0; i < S::ROWS; ++i) {
+        const i64 row = group * S::ROWS + i;
+#pragma unroll
+        for (int n1 = 0; n1 < S::E0; ++n1) {
+            const i64 idx = (n1 << 8) + tid;
+            const bool there = row < A.n_rows && idx < A.width;
+            ok |= there ? 1u << (i * S::E0 + n1) : 0u;
+            coef[i * S::E0 + n1] = A.src[there ? row * A.src_stride + idx : 0];
+        }
+    }
+#pragma unroll
+    for (int n1 = 0; n1 < S::E0; ++n1) pw[n1] = A.pre[(n1 << 8) + tid];
+    VI_SCHED_FENCE();
+#pragma unroll
+    for (int e = 0; e < S::ROWS * S::E0; ++e) {
+        u64 v = (ok >> e) & 1 ? coef[e] : 0;
+        if (A.canon_src) v = gl::canon(v);
+        coef[e] = gl::mul(v, pw[e & (S::E0 - 1)]);
+    }
+}
+
+// the first digit of the tile's pairs, cosets T0 .. T0 + COSETS - 1, into the columns that row_gather reads
+template <int A0, int LR, int T0>
+VI_HD void lde_row_stage0(const LdeRow &A, int tid, const u64 (&coef)[LdeRowShape<A0, LR>::ROWS << A0], u64 *lds) {
+    using S = LdeRowShape<A0, LR>;
+    static_for<0, S::COSETS>([&](auto t_) {
+        constexpr int t = T0 + decltype(t_)::value;
+        u64 tw[S::E0];
+#pragma unroll
+        for (int k = 0; k < S::E0; ++k) tw[k] = t > 0 || k > 0 ? A.tw[((t << A0) + k) * 256 + tid] : 1;
+#pragma unroll
+        for (int i = 0; i < S::ROWS; ++i) {
+            u64 x[S::E0];
+            static_for<0, S::E0>([&](auto n_) {
+                constexpr int n1 = decltype(n_)::value, e = (39 * (64 >> (A0 + LR)) * t * n1) % 192;
+                if constexpr (e == 0) x[n1] = coef[i * S::E0 + n1];
+                else x[n1] = gl::mul_pow2c_pinned<e>(coef[i * S::E0 + n1]);
+            });
+            VI_SCHED_FENCE();
+            dft_reg<A0, false>(x);
+#pragma unroll
+            for (int k = 0; k < S::E0; ++k) {
+                u64 v = x[k];
+                if (t > 0 || k > 0) v = gl::mul(v, tw[k]);
+                lds[(((i * S::COSETS + decltype(t_)::value) << A0) + k) * ROW_ST + tid] = v;
+            }
+            VI_SCHED_FENCE();
+        }
+    });
+}
+
+// second half of the last digit; cosets of a row interleaved
+template <int A0, int LR>
+VI_HD void lde_row_store(const LdeRow &A, i64 group, int t0, int tid, const u64 *lds) {
+    using S = LdeRowShape<A0, LR>;
+    const int c = tid & 15, k1 = tid >> 4, j = c >> A0;
+    const i64 row = group * S::ROWS + j / S::COSETS;
+    u64 x[16];
+#pragma unroll
+    for (int n2 = 0; n2 < 16; ++n2) x[n2] = lds[((k1 << 4) + n2) * 17 + c];
+    VI_SCHED_FENCE();
+    dft_reg<4, false>(x);
+    VI_SCHED_FENCE();
+    if (row >= A.n_rows) return;
+    const u32 off = (u32)(((c & (S::E0 - 1)) + (k1 << A0)) << LR) + (u32)(t0 + j % S::COSETS);
+    if constexpr (S::ROWS == 1) {
+        const URun dst = urun(A.out + group * A.out_stride);
+#pragma unroll
+        for (int k2 = 0; k2 < 16; ++k2) ustore(dst, (u32)k2 << (A0 + 4 + LR), off, x[k2]);
+    } else {
+        u64 *o = A.out + row * A.out_stride + off;
+#pragma unroll
+        for (int k2 = 0; k2 < 16; ++k2) o[k2 << (A0 + 4 + LR)] = x[k2];
+    }
+}
+
 // can passes Ai (last inverse) and Af (first forward, expanding into cosets) run as one fused launch?
 inline bool passes_fusable(const PassArgs &Ai_in, const PassArgs &Af_in) {
     PassArgs Ai = Ai_in, Af = Af_in;

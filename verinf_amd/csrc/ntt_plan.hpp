@@ -164,6 +164,29 @@ inline void append_coset_merged(int logK, int logN, std::vector<u64> &t) {
     }
 }
 
+// The same split for rows of 2^10 .. 2^12 points whose codewords come from one launch (lde_row_stage0): i = n1 256 + r, the
+// factor w_N^(256 t n1) a power of two when K rho / 256 <= 64.  Appended: w_K^(k r) w_N^(t r) at [t][k][r] (N words).
+inline bool coset_rows_ok(int logK, int logN) {
+    const int log_rho = logN - logK;
+    return row_single_ok(logK) && log_rho >= 1 && log_rho <= 3 && logN <= 14;
+}
+inline void append_coset_rows(int logK, int logN, std::vector<u64> &t) {
+    const Split rs = row_split(logK);
+    const HostTables H = make_tables(logK, 0, &rs);
+    const u64 wN = root_of_unity(logN);
+    const size_t K = (size_t)1 << logK, base = t.size();
+    t.resize(base + (K << (logN - logK)));
+    u64 wc = 1;                                            // w_N^t
+    for (size_t c = 0; c < (size_t)1 << (logN - logK); ++c) {
+        u64 cur = 1;
+        for (size_t r = 0; r < 256; ++r) {
+            for (size_t k = 0; k < K / 256; ++k) t[base + c * K + k * 256 + r] = gl::mul(H.tw[0][k * 256 + r], cur);
+            cur = gl::mul(cur, wc);
+        }
+        wc = gl::mul(wc, wN);
+    }
+}
+
 // device (or host) addresses of the tables of one (logn, direction)
 struct Tables {
     Split sp;
