@@ -729,3 +729,16 @@ def test_first_sample_at_one_from_a_later_round(mods, terms, v, coins):
     claim, polys, _, _ = gpu.prove_terms_gpu([(c, [dev[i] for i in fs]) for c, fs in terms], lambda i: coins[i], P)
     want_claim, want_samples, _ = O.sumcheck_prove(tabs, terms, coins)
     assert claim == want_claim and [[y for _, y in s] for s in polys] == want_samples
+
+
+@pytest.mark.parametrize("v", range(1, 16))
+@pytest.mark.parametrize("terms", [[(5, [0])], [(7, [0, 1])], [(1, [0, 1, 2])], [(3, [0, 1, 2, 3])], [(3, [0, 1, 2]), (P - 3, [0, 3])]])
+def test_every_length_of_the_last_launch(mods, terms, v):
+    """Tables of 2 .. 2^15 entries: rounds left to the first wavefront, to the workgroup, and to passes before it."""
+    gpu, _ = mods
+    coins = _coins(v, 77 + v)[0]
+    tabs = [rand_field(1 << v, 60 * v + t) for t in range(1 + max(max(fs) for _, fs in terms))]
+    dev = [to_dev(t) for t in tabs]
+    claim, polys, _, _ = gpu.prove_terms_gpu([(c, [dev[i] for i in fs]) for c, fs in terms], lambda i: coins[i], P)
+    want_claim, want_samples, _ = O.sumcheck_prove(tabs, terms, coins)
+    assert claim == want_claim and [[y for _, y in s] for s in polys] == want_samples

@@ -54,9 +54,6 @@ struct ChainDesc {
 struct FinishShared {
     u64 raw[MAX_ROUNDS][NSAMP];             // summed samples per round, before scale and chain
     u64 lag[MAX_ROUNDS][NSAMP];             // Lagrange basis of the points 0..deg at r_k
-    u64 a[MAX_ROUNDS], b[MAX_ROUNDS];       // claim_(k+1) = a_k claim_k + b_k
-    u64 claim[MAX_ROUNDS + 1];
-    u64 late_claim;
 };
 
 // The sums over the wavefront of N values per lane: a step adds the halves of the lanes and halves the values, each half of the
@@ -135,13 +132,14 @@ __device__ __forceinline__ void finish_samples(const ChainDesc &C, FinishShared 
     const bool inf = C.inf_node != 0;
     u64 y[NSAMP];
     u64 top_a = 0, top_b = 0;                // S_k(deg) = top_a claim_k + top_b when it is not summed itself
+    u64 a = 0, b = 0;                        // claim_(k+1) = a claim_k + b
+#pragma unroll
+    for (int x = 0; x < NSAMP; ++x) y[x] = 0;
     if (mine) {
         // every sample is a + b claim_k for known a, b: S(1) = claim - S(0) where it was skipped, S(deg) from
-        // the leading coefficient; so claim_(k+1) = sum_x L_x(r_k) S_k(x) = a_k claim_k + b_k
-        u64 a = 0, b = 0;
+        // the leading coefficient; so claim_(k+1) = sum_x L_x(r_k) S_k(x) = a claim_k + b
 #pragma unroll
         for (int x = 0; x < NSAMP; ++x) {
-            y[x] = 0;
             if (x <= C.deg && !(skip && x == 1)) {
                 y[x] = sh.raw[k][x];
                 if (C.scale != 1) y[x] = gl::mul(y[x], C.scale);
@@ -175,25 +173,22 @@ __device__ __forceinline__ void finish_samples(const ChainDesc &C, FinishShared 
                 }
             }
         }
-        sh.a[k] = a;
-        sh.b[k] = b;
-        if (k == C.late) sh.late_claim = gl::addc(y[0], y[1]);
     }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        u64 claim = 0;                       // a round that summed every sample does not read it
-        if (C.late > 0) {
-            for (int j = 0; j < C.late; ++j) claim = gl::addc(gl::mul(sh.a[j], claim), sh.b[j]);
-            claim = gl::mul(gl::sub(sh.late_claim, claim), C.late_inv);
-        }
-        for (int j = 0; j < C.n_rounds; ++j) {
-            sh.claim[j] = claim;
-            claim = gl::addc(gl::mul(sh.a[j], claim), sh.b[j]);
+    // claim_(k+1) in terms of claim_0, a prefix product of affine maps in the first wavefront (one after the other, 18 rounds
+    // took 3 us)
+    if (k >= 64) return;
+    for (int d = 1; d < C.n_rounds; d <<= 1) {
+        const u64 pa = __shfl_up(a, (unsigned)d, 64), pb = __shfl_up(b, (unsigned)d, 64);
+        if (k >= d) {
+            b = gl::mul_add(a, pb, b);
+            a = gl::mul(a, pa);
         }
     }
-    __syncthreads();
+    u64 first = 0;                           // a round that summed every sample does not read it
+    if (C.late > 0) first = gl::mul(gl::sub(__shfl(gl::addc(y[0], y[1]), C.late, 64), __shfl(b, C.late - 1, 64)), C.late_inv);
+    const u64 prev_a = __shfl_up(a, 1, 64), prev_b = __shfl_up(b, 1, 64);
     if (mine) {
-        const u64 claim = sh.claim[k];
+        const u64 claim = k == 0 ? first : gl::mul_add(prev_a, first, prev_b);
         if (skip) y[1] = gl::sub(claim, y[0]);
 #pragma unroll
         for (int x = 0; x < NSAMP; ++x) {
@@ -459,54 +454,44 @@ struct TailCap {
     static_assert(NT * HALF <= TAIL_WORDS, "tail tables exceed their LDS share");
 };
 
-// sums of one round over the workgroup: every wavefront that had pairs leaves its sums in red_par, the caller
-// synchronises, and threads x < NS add them up into raw_k
-template <int NS>
-__device__ __forceinline__ void tail_wave_sums(const SampleAcc<false> (&acc)[NS], u64 (*red_par)[NSAMP], int active_waves) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    if (w < active_waves) {
-#pragma unroll
-        for (int x = 0; x < NS; ++x) {
-            const u64 s = wave_sum(acc[x].v);
-            if (lane == 0) red_par[w][x] = s;
-        }
-    }
-}
-template <int NS>
-__device__ __forceinline__ void tail_round_total(u64 (*red_par)[NSAMP], int active_waves, u64 *raw_k) {
-    if (threadIdx.x < NS) {
-        u64 s = red_par[0][threadIdx.x];
-        for (int i = 1; i < active_waves; ++i) s = gl::addc(s, red_par[i][threadIdx.x]);
-        raw_k[threadIdx.x] = s;
-    }
-}
-
 // Every remaining round in one workgroup: tables of `size` <= 2 TailCap<NT>::HALF words; rounds C.n_prior .. C.n_rounds - 1.
 // FIRST: the proof starts here (the tables are the caller's).  ONE: the launch's first round sums S(1).  The folded tables live in LDS and are not written back.
-// A round costs its longest thread, so what a round does besides its one pair per thread is kept off that path:
-//  - rounds of more than TAIL_DEFER pairs add their sums up across the workgroup as they go (every wavefront is busy);
-//  - smaller rounds leave each thread's sums in LDS -- the round of h pairs in lane_sums[.][h .. 2h) -- and nine
-//    wavefronts add the nine of them up at the end, all at once;
-//  - once a table fits the lanes of one wavefront (64 entries) the first wavefront goes on alone, a table entry per
-//    lane and partners fetched by lane shuffles: no LDS traffic for the tables, no workgroup barrier per round.
-constexpr int TAIL_DEFER = 256;
+// A round costs its longest thread and a barrier, so what can wait is kept off that path:
+//  - every round leaves its threads' sums in LDS, and a wavefront per round adds them up at the end, all at once (summed across
+//    the workgroup as they went, the rounds of more than 256 pairs took 1 us longer each);
+//  - once a table fits the lanes of one wavefront (64 entries) the first wavefront goes on alone, a table entry per lane and
+//    partners fetched by lane shuffles, and only folds: it leaves the tables of those rounds behind, and a wavefront per round
+//    takes the samples from them at the end.
+// 12 rounds over two tables 21.0 -> 15.2 us, the last 11 of 26 over three 35.4 -> 24.4.
+constexpr int TAIL_SMALL = 6;                // rounds of 32, 16, .. 1 pairs
 
 template <int NT, int SHAPE, bool FIRST, bool ONE>
 __global__ __launch_bounds__(TAIL_THREADS) void k_tail(const FastDesc D, i64 size, const ChainDesc C, const u64 *part, u64 *out) {
     constexpr int NS = FastShape<NT, SHAPE>::NS;
     constexpr int HALF = TailCap<NT>::HALF;
+    // sums of the round of h pairs: min(h, TAIL_THREADS) words at [h, 2 h), or one after the other beyond 2 TAIL_THREADS
+    constexpr int SUMS = HALF <= TAIL_THREADS ? 2 * TAIL_THREADS : (HALF == 2 * TAIL_THREADS ? 3 : 4) * TAIL_THREADS;
+    auto sums_at = [](int h) { return h <= 2 * TAIL_THREADS ? h : 3 * TAIL_THREADS; };
+    static_assert(HALF <= 4 * TAIL_THREADS, "rounds of more pairs need more room for their sums");
     __shared__ u64 tab[NT][HALF];
-    __shared__ u64 red[2][TAIL_THREADS / 64][NSAMP];
-    __shared__ u64 lane_sums[NS][2 * TAIL_DEFER];
+    __shared__ u64 lane_sums[NS][SUMS];
+    __shared__ u64 small[NT][128];           // the table of s <= 64 entries at [s, 2 s)
     __shared__ FinishShared sh;
     finish_begin(C, part, sh);
 
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    int k = C.n_prior, par = 0;
+    int k = C.n_prior;
     int h = (int)(size >> 1);
     const int h_first = h;
     SampleAcc<false> acc[NS];
     u64 lo[NT], hi[NT], dif[NT];
+    auto leave_sums = [&]() {
+        if (tid < h) {
+#pragma unroll
+            for (int x = 0; x < NS; ++x) lane_sums[x][sums_at(h) + tid] = acc[x].v;
+        }
+        __syncthreads();
+    };
     {
         // first round of this launch: pairs from memory, folded values into LDS
 #pragma unroll
@@ -524,19 +509,7 @@ __global__ __launch_bounds__(TAIL_THREADS) void k_tail(const FastDesc D, i64 siz
                 for (int t = 0; t < NT; ++t) tab[t][i] = gl::mul_add(r, dif[t], lo[t]);
             }
         }
-        if (h > TAIL_DEFER) {
-            const int aw = h >= TAIL_THREADS ? TAIL_THREADS / 64 : (h + 63) >> 6;
-            tail_wave_sums<NS>(acc, red[par], aw);
-            __syncthreads();
-            tail_round_total<NS>(red[par], aw, sh.raw[k]);
-            par ^= 1;
-        } else {
-            if (tid < h) {
-#pragma unroll
-                for (int x = 0; x < NS; ++x) lane_sums[x][h + tid] = acc[x].v;
-            }
-            __syncthreads();
-        }
+        leave_sums();
     }
     // rounds on tables of more than 64 entries: pairs from LDS, a workgroup barrier per round
     for (h >>= 1; h >= 64; h >>= 1) {
@@ -551,62 +524,57 @@ __global__ __launch_bounds__(TAIL_THREADS) void k_tail(const FastDesc D, i64 siz
 #pragma unroll
             for (int t = 0; t < NT; ++t) tab[t][i] = gl::mul_add(r, dif[t], lo[t]);
         }
-        if (h > TAIL_DEFER) {
-            const int aw = h >= TAIL_THREADS ? TAIL_THREADS / 64 : (h + 63) >> 6;
-            tail_wave_sums<NS>(acc, red[par], aw);
-            __syncthreads();
-            tail_round_total<NS>(red[par], aw, sh.raw[k]);
-            par ^= 1;
-        } else {
-            if (tid < h) {
-#pragma unroll
-                for (int x = 0; x < NS; ++x) lane_sums[x][h + tid] = acc[x].v;
-            }
-            __syncthreads();
-        }
+        leave_sums();
     }
     // tables of at most 64 entries: the first wavefront alone, lane i holding entry i of every table
-    if (w == 0 && h >= 1) {
+    const int h_small = h;
+    if (w == 0) {
         u64 val[NT];
 #pragma unroll
         for (int t = 0; t < NT; ++t) val[t] = (lane < 2 * h) ? tab[t][lane] : 0;
         for (; h >= 1; h >>= 1) {
-            ++k;
-#pragma unroll
-            for (int x = 0; x < NS; ++x) acc[x].zero();
-            const u64 r = C.r[k];
+            const u64 r = C.r[++k];
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
-                lo[t] = val[t];
-                hi[t] = __shfl_down(val[t], (unsigned)h, 64);      // lanes past the pairs compute on what they get and drop it
-            }
-            eval_pair<NT, SHAPE, true, false>(lo, hi, dif, acc);
-#pragma unroll
-            for (int t = 0; t < NT; ++t) val[t] = gl::mul_add(r, dif[t], lo[t]);
-            if (lane < h) {
-#pragma unroll
-                for (int x = 0; x < NS; ++x) lane_sums[x][h + lane] = acc[x].v;
+                if (lane < 2 * h) small[t][2 * h + lane] = val[t];
+                const u64 up = __shfl_down(val[t], (unsigned)h, 64);       // lanes past the pairs compute on what they get and drop it
+                val[t] = gl::mul_add(r, gl::sub(up, val[t]), val[t]);
             }
         }
     }
     __syncthreads();
-    // the deferred rounds: wavefront j adds up the round of TAIL_DEFER >> j pairs, the (log2 of that + 1)-th from last
-    {
-        const int hd = TAIL_DEFER >> w;
-        if (w < 9 && hd <= h_first) {
-            int lg = 0;
-            while ((1 << lg) < hd) ++lg;
-            const int kd = C.n_rounds - 1 - lg;
-            const bool skip1 = (C.skip_mask >> kd) & 1;
+    // wavefront w < TAIL_SMALL: the round of 32 >> w pairs; the others a round of h_small < 2^j <= h_first pairs
+    auto keep = [&](u64 (&v)[NS], int pairs) {
+        int slot;
+        const u64 sum = wave_totals<NS>(v, 32, slot);
+        const int kd = C.n_rounds - 1 - (31 - __builtin_clz((unsigned)pairs));
+        if (slot >= 0) sh.raw[kd][slot] = sum;
+    };
+    u64 v[NS];
+    if (w < TAIL_SMALL) {
+        const int pairs = 32 >> w;
+        if (pairs <= h_small) {
 #pragma unroll
-            for (int x = 0; x < NS; ++x) {
-                if (!(skip1 && x == 1)) {
-                    u64 v = 0;
-                    for (int i = lane; i < hd; i += 64) v = gl::addc(v, lane_sums[x][hd + i]);
-                    v = wave_sum(v);
-                    if (lane == 0) sh.raw[kd][x] = v;
-                }
+            for (int x = 0; x < NS; ++x) acc[x].zero();
+            if (lane < pairs) {
+#pragma unroll
+                for (int t = 0; t < NT; ++t) { lo[t] = small[t][2 * pairs + lane]; hi[t] = small[t][3 * pairs + lane]; }
+                eval_pair<NT, SHAPE, true, false>(lo, hi, dif, acc);
             }
+#pragma unroll
+            for (int x = 0; x < NS; ++x) v[x] = acc[x].v;
+            keep(v, pairs);
+        }
+    } else {
+        const int pairs = h_first >> (w - TAIL_SMALL);
+        if (pairs > h_small) {
+            const int words = pairs < TAIL_THREADS ? pairs : TAIL_THREADS, at = sums_at(pairs);
+#pragma unroll
+            for (int x = 0; x < NS; ++x) v[x] = 0;
+            for (int i = lane; i < words; i += 64)
+#pragma unroll
+                for (int x = 0; x < NS; ++x) v[x] = gl::addc(v[x], lane_sums[x][at + i]);
+            keep(v, pairs);
         }
     }
     __syncthreads();
