@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 
 torch = pytest.importorskip("torch")
 from oracle import oracle as O  # noqa: E402
-from tests.gpu_util import P, rand_field, to_dev, to_np, unhex  # noqa: E402
+from tests.gpu_util import P, rand_field, rand_field_dev, to_dev, to_np, unhex  # noqa: E402
 
 
 @pytest.fixture(scope="module")
@@ -205,3 +205,31 @@ def test_inverses_around_the_switch_to_shared_inversions(cp, n):
     assert (prod[~zero] == 1).all()
     _lib.check(_lib.lib().vi_gl_unop(2, d.data_ptr(), 0, d.data_ptr(), n, _lib.stream_ptr()))
     assert np.array_equal(to_np(d), got)
+
+
+@pytest.mark.parametrize("n", [(1 << 20) - 1, 1 << 20, (1 << 20) + 1, (1 << 21) - 1, 1 << 21, (1 << 21) + 1, 12 * 256 * 900 - 1, 12 * 256 * 900 + 1])
+def test_inverses_of_four_eight_and_twelve_elements_a_thread(cp, n):
+    d = rand_field_dev((n,), n)
+    d.view(torch.int64)[::100003] = 0
+    got = cp.gl_inv_batched(d)
+    want = torch.ones_like(d)
+    want.view(torch.int64)[::100003] = 0
+    assert torch.equal(cp.gl_mul(d, got), want)
+    assert int(got.view(torch.int64)[::100003].abs().sum()) == 0
+    own = d.clone()
+    from verinf_amd import _lib
+    _lib.check(_lib.lib().vi_gl_unop(2, own.data_ptr(), 0, own.data_ptr(), n, _lib.stream_ptr()))
+    assert torch.equal(own, got)
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 511, 513, 4097, (1 << 21) + 1])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_sums_and_products_of_odd_lengths(cp, n, shift):
+    """Pairs of elements and the last one of an odd number; operands that do not start on 16 bytes go one by one."""
+    a, b = rand_field_dev((n + shift,), 1)[shift:], rand_field_dev((n + shift,), 2)[shift:]
+    sums, differences, products = cp.gl_add(a, b), cp.gl_sub(a, b), cp.gl_mul(a, b)
+    assert torch.equal(cp.gl_sub(sums, b), a) and torch.equal(cp.gl_add(differences, b), a)
+    picks = sorted({0, n // 2, max(n - 2, 0), n - 1})
+    for i in picks:
+        x, y = int(a[i].item()), int(b[i].item())
+        assert [int(t[i].item()) for t in (sums, differences, products)] == [(x + y) % P, (x - y) % P, x * y % P]

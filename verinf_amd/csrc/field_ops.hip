@@ -29,10 +29,14 @@ __global__ __launch_bounds__(BLOCK) void k_binop(const u64 *a, const u64 *b, u64
         __builtin_nontemporal_store(apply<OP>(__builtin_nontemporal_load(a + i), __builtin_nontemporal_load(b + i)), out + i);
 }
 
-// two elements per lane through 16-byte accesses (operands 16-byte aligned, n even)
+// two elements per lane through 16-byte accesses (operands 16-byte aligned); the last of an odd number by itself
 template <int OP>
-__global__ __launch_bounds__(BLOCK) void k_binop_v2(const ulonglong2 *a, const ulonglong2 *b, ulonglong2 *out, i64 n2) {
-    i64 stride = (i64)gridDim.x * BLOCK;
+__global__ __launch_bounds__(BLOCK) void k_binop_v2(const ulonglong2 *a, const ulonglong2 *b, ulonglong2 *out, i64 n) {
+    const i64 stride = (i64)gridDim.x * BLOCK, n2 = n >> 1;
+    if ((n & 1) && blockIdx.x == gridDim.x - 1 && threadIdx.x == BLOCK - 1) {
+        const u64 *x = (const u64 *)a, *y = (const u64 *)b;
+        ((u64 *)out)[n - 1] = apply<OP>(x[n - 1], y[n - 1]);
+    }
     for (i64 i = (i64)blockIdx.x * BLOCK + threadIdx.x; i < n2; i += stride) {
         // operands read once, result not read back by this launch: streaming hints (2^24 elements 5.1 -> 5.9 TB/s,
         // 2^27 4.40 -> 4.50 TB/s)
@@ -121,11 +125,14 @@ __global__ __launch_bounds__(BLOCK) void k_probe(int op, const u64 *a, const u64
 // workgroup): a thread takes INV_E elements, one from each of INV_E equal slabs of the array so that a wavefront's
 // accesses stay contiguous, and multiplies them up; the first wavefront does the same with the products of all threads
 // and inverts ONE product per lane (74 multiplications in a chain); the single inverses are peeled off in turn.  A
-// wavefront that inverts costs the same however many of its lanes do, so the chain is paid once per 4096 elements and
-// not once per 512: 35 instead of 98 multiplications per wavefront and 512 elements (1.5 M elements: 16.9 -> 13.8 us).
-// Zeros are taken out of the product and map to zero, so every output equals the Fermat power a^(p-2) of the reference
-// kernel (prover/cuda_primitives.py:289-303).
-constexpr int INV_E = 8, INV_THREADS = 512;
+// wavefront that inverts costs the same however many of its lanes do, so the chain is paid once per
+// workgroup and not once per wavefront.  Workgroups of 256 rather than 512 have the shorter chain and fill the SIMDs while one wavefront of each
+// inverts (1.5 M elements 13.6 -> 12.4 us, 16 M 89 -> 71).  Zeros are taken out of the product and map to zero, so every output
+// equals the Fermat power a^(p-2) of the reference kernel (prover/cuda_primitives.py:289-303).
+//
+// Elements of a thread: four while the chip has SIMDs to spare, then eight, then twelve, which share an inversion (us with 4, 8 and 12:
+// 300000 8.7, 9.7, 10.7; 700001 9.6, 10.9, 11.3; 1.5 M 13.3, 12.4, 13.3; 3 M 21.8, 22.0, 17.5; 6 M 33.6, 32.4, 29.4; 16 M 78.6, 70.8, 68.0).
+constexpr int INV_THREADS = 256;
 
 // Few elements: an inversion each.  A launch lasts as long as one thread's chain while a SIMD has a wavefront or two, and
 // without products before and after it the chain is the shortest (us per call in a queue: 1000 elements 9.5 -> 6.3, 2^16 10.5
@@ -137,6 +144,7 @@ __global__ __launch_bounds__(64) void k_inv_each(const u64 *a, u64 *out, i64 n) 
     if (i < n) out[i] = gl::inv(gl::canon(a[i]));
 }
 
+template <int INV_E>
 __global__ __launch_bounds__(INV_THREADS) void k_inv_batched(const u64 *a, u64 *out, i64 n, i64 groups) {
     __shared__ u64 prod[INV_THREADS];
     const int tid = threadIdx.x;
@@ -310,13 +318,13 @@ int vi_gl_binop(int op, const uint64_t *a, const uint64_t *b, uint64_t *out, int
     if (n == 0) return VI_OK;
     if (!a || !b || !out) return vi::fail(VI_EINVAL, "vi_gl_binop: null pointer");
     hipStream_t s = (hipStream_t)stream;
-    if ((n & 1) == 0 && aligned16(a) && aligned16(b) && aligned16(out)) {
-        i64 n2 = n / 2;
+    if (aligned16(a) && aligned16(b) && aligned16(out)) {
+        const i64 n2 = (n + 1) / 2;
         auto A = (const ulonglong2 *)a, B = (const ulonglong2 *)b;
         auto O = (ulonglong2 *)out;
-        if (op == 0) hipLaunchKernelGGL(k_binop_v2<0>, dim3(grid_for(n2)), dim3(BLOCK), 0, s, A, B, O, n2);
-        if (op == 1) hipLaunchKernelGGL(k_binop_v2<1>, dim3(grid_for(n2)), dim3(BLOCK), 0, s, A, B, O, n2);
-        if (op == 2) hipLaunchKernelGGL(k_binop_v2<2>, dim3(grid_for(n2)), dim3(BLOCK), 0, s, A, B, O, n2);
+        if (op == 0) hipLaunchKernelGGL(k_binop_v2<0>, dim3(grid_for(n2)), dim3(BLOCK), 0, s, A, B, O, (i64)n);
+        if (op == 1) hipLaunchKernelGGL(k_binop_v2<1>, dim3(grid_for(n2)), dim3(BLOCK), 0, s, A, B, O, (i64)n);
+        if (op == 2) hipLaunchKernelGGL(k_binop_v2<2>, dim3(grid_for(n2)), dim3(BLOCK), 0, s, A, B, O, (i64)n);
     } else {
         if (op == 0) hipLaunchKernelGGL(k_binop<0>, dim3(grid_for(n)), dim3(BLOCK), 0, s, a, b, out, (i64)n);
         if (op == 1) hipLaunchKernelGGL(k_binop<1>, dim3(grid_for(n)), dim3(BLOCK), 0, s, a, b, out, (i64)n);
@@ -351,10 +359,14 @@ int vi_gl_unop(int op, const uint64_t *a, uint64_t arg, uint64_t *out, int64_t n
             VI_LAUNCH_CHECK("k_inv_each");
             return VI_OK;
         }
-        const i64 groups = (n + INV_E - 1) / INV_E;
+        const int each = n <= ((i64)1 << 20) ? 4 : n <= ((i64)1 << 21) ? 8 : 12;
+        const i64 groups = (n + each - 1) / each;
         const i64 blocks = (groups + INV_THREADS - 1) / INV_THREADS;
         if (blocks > 0x7FFFFFFF) return vi::fail(VI_EINVAL, "vi_gl_unop: n = %lld", (long long)n);
-        hipLaunchKernelGGL(k_inv_batched, dim3((unsigned)blocks), dim3(INV_THREADS), 0, (hipStream_t)stream, a, out, (i64)n, groups);
+        const dim3 grid((unsigned)blocks), block(INV_THREADS);
+        if (each == 4) hipLaunchKernelGGL(k_inv_batched<4>, grid, block, 0, (hipStream_t)stream, a, out, (i64)n, groups);
+        else if (each == 8) hipLaunchKernelGGL(k_inv_batched<8>, grid, block, 0, (hipStream_t)stream, a, out, (i64)n, groups);
+        else hipLaunchKernelGGL(k_inv_batched<12>, grid, block, 0, (hipStream_t)stream, a, out, (i64)n, groups);
         VI_LAUNCH_CHECK("k_inv_batched");
         return VI_OK;
     }
