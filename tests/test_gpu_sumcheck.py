@@ -714,6 +714,15 @@ def test_sums_under_a_common_factor(mods, form, v):
         assert np.array_equal(to_np(d), t), "caller's table was modified"
 
 
+@pytest.mark.parametrize("v", [2, 10, 11, 12])
+@pytest.mark.parametrize("singles", [128, 129, 140])
+def test_single_tables_around_what_a_descriptor_holds(mods, singles, v):
+    """Beyond 128 single tables under the common factor the sum is rewritten after its first round, from where on it is folded in place."""
+    gpu, _ = mods
+    terms = [(3, [0, 1, 2]), (5, [0, 3, 4])] + [(k + 2, [0, 5 + k]) for k in range(singles)]
+    _check(gpu, [rand_field(1 << v, 5000 + t) for t in range(5 + singles)], terms, 90 + v, True)
+
+
 @pytest.mark.parametrize("coins", [[0, 5], [2, 7], [9, 2, 3], [9, 8, 0], [1, 1, 1], [P - 1, P - 2, 1], [3, 4, 5, 0, 2, 1, 0]])
 @pytest.mark.parametrize("terms,v", [([(5, [0])], 14), ([(1, [0, 1])], 13), ([(7, [0, 1])], 16), ([(1, [0, 1, 2])], 13), ([(1, [0, 1, 2])], 16),
                                      ([(3, [0, 1, 2, 3])], 13), ([(3, [0, 1, 2]), (P - 3, [0, 3])], 13), ([(3, [0, 1]), (4, [0, 2])], 10),

@@ -1587,8 +1587,9 @@ int prove_coins_impl(const char *who, const uint64_t *const *tables, uint64_t *c
     C.deg = deg;
 
     // products of two tables and single tables under a common factor: three rounds per pass (the hadamard gate batch of four tables
-    // has kernels of its own)
-    {
+    // has kernels of its own).  Not the rewritten problem of prove_coins_reduced, which has more single tables than a descriptor and whose
+    // tables are the work buffers: a row of workgroups would write over entries of the common factor that others still have to read
+    if (may_reduce) {
         SumShape S;
         if (sum_shape(n_tables, term_off, factor_idx, coeffs, n_terms, S) &&
             !(n_tables == 4 && S.products.size() == 1 && S.singles.size() == 1 && S.c0 == 0))

@@ -281,7 +281,7 @@ int sum_resident() {
     return caps[dev];
 }
 
-// The whole proof.  part: workspace of (n_rounds + 1) * MAX_BLOCKS * NSAMP words; C arrives with r, winv, deg, n_rounds set.
+// The whole proof.  tables and work are different buffers.  part: workspace of (n_rounds + 1) * MAX_BLOCKS * NSAMP words; C arrives with r, winv, deg, n_rounds set.
 // A pass writes behind what the pass before it wrote in the tables' buffers (size / 2 words each: an eighth, a 64th, ... of the
 // size), as other rows may still be reading that; the sums of single tables have the upper halves of the buffers.
 int prove_sum(const SumShape &S, const uint64_t *const *tables, uint64_t *const *work, i64 size, ChainDesc &C, u64 *part, u64 *out, hipStream_t s) {
