@@ -173,9 +173,32 @@ print("captured")
 """
 
 
-def test_a_captured_call_finds_the_tables_of_another_batch_size():
+_CAPTURE_EXTENSIONS = """
+import torch
+from tests.gpu_util import rand_field, to_dev
+from verinf_amd.prover import cuda_primitives as cp
+for logk, log_rate, first, then in ((9, 2, 3, 1 << 12), (10, 2, 3, 1 << 10), (11, 1, 1 << 11, 2), (12, 2, 2, 1 << 8), (12, 1, 1 << 10, 2), (14, 2, 64, 2)):
+    k, n = 1 << logk, 1 << (logk + log_rate)
+    cp.coset_lde(to_dev(rand_field((first, k), 1)), k, n, 7)
+    src = [to_dev(rand_field((then, k), 2 + i)) for i in range(3)]
+    buf = src[0].clone()
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        out = cp.coset_lde(buf, k, n, 7)
+    for s in src:
+        buf.copy_(s)
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int64), cp.coset_lde(s, k, n, 7).view(torch.int64)), (logk, then)
+print("captured")
+"""
+
+
+@pytest.mark.parametrize("calls", [_CAPTURE, _CAPTURE_EXTENSIONS], ids=["transforms", "extensions"])
+def test_a_captured_call_finds_the_tables_of_another_batch_size(calls):
     """A call of one batch size prepares its row length for all of them: the other kernels capture with nothing left to
     upload.  In a process of its own, where no other test has prepared anything."""
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-    r = subprocess.run([sys.executable, "-c", _CAPTURE], cwd=root, capture_output=True, text=True, timeout=100)
+    r = subprocess.run([sys.executable, "-c", calls], cwd=root, capture_output=True, text=True, timeout=100)
     assert r.returncode == 0 and r.stdout.endswith("captured\n"), r.stderr[-2000:]

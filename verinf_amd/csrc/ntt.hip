@@ -911,7 +911,7 @@ int coset_lde_impl(const char *who, const uint64_t *in, int64_t m, int64_t width
     if (rc) return rc;
     const LdeRoute route = lde_route(m, logK, logN, coeffs == in, Ti->sp);
     const Tables *TiRow = nullptr, *TfRow = nullptr;
-    if (route == LDE_ROWS) {
+    if (coset_rows_ok(logK, logN)) {                       // whatever the batch: one of another size may be captured
         rc = get_tables(logK, 1, &TiRow, true);
         if (!rc) rc = get_tables(logK, 0, &TfRow, true);
         if (rc) return rc;
