@@ -10,8 +10,8 @@
 // the search from the front costs half the table.  Which of the two a table is, is looked at in every call, on the device: up
 // to 4096 entries by every workgroup for itself (k_count_small: table and hash in LDS), beyond by a launch over the table
 // (k_survey), whose findings the counting workgroups read.  us per call in a queue of them, 1.5 M look-ups: 10 in 2^6 entries,
-// 12.0 in 2^12, 21.0 in 2^16, 51 in 2^20 (19.0 and 48 for the last two when the caller promises a range); 10^6 look-ups in 3003
-// values 12.6, in 40000 36.
+// 12.0 in 2^12, 17.9 in 2^16, 51 in 2^20 (48 for the last when the caller promises a range); 10^6 look-ups in 3003
+// values 12.6, in 40000 31.
 #include <algorithm>
 
 #include "common.hpp"
