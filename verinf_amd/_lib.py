@@ -223,25 +223,61 @@ def workspace(nbytes: int, tag: str, stream_ptr: int):
 
 
 _pinned = threading.local()
+NO_WORD = 0xFFFFFFFFFFFFFFFF    # VI_NO_WORD: no field element
 
 
-def pinned_words(words: int, stream_ptr: int):
-    """Pinned host words that kernels of a call write results into and the call reads them from, with a numpy view of
-    the same memory.  One buffer per host thread and stream: a call has read its results before the next one on that
-    stream starts, and two threads (or two streams) never see each other's.  Buffers grow and are kept for the life
-    of the thread (a few KiB each)."""
+class _Words:
+    """Pinned host words and a numpy view of the same memory.  As a context: a call's kernels write the words and the call
+    polls them.  Left by an exception, those kernels may still be on their way, and words they write later would pass for the
+    results of the next call, so the stream is waited for."""
+    __slots__ = ("host", "view", "polled")
+
+    def __init__(self, words):
+        self.host = torch.zeros(words, dtype=torch.uint64).pin_memory()
+        self.view = self.host.numpy()
+        self.polled = False
+
+    def __enter__(self):
+        self.polled = True
+        return self
+
+    def __exit__(self, kind, value, trace):
+        if kind is not None:
+            torch.cuda.current_stream().synchronize()
+        self.polled = False
+
+
+def _words(words: int, stream_ptr: int):
     bufs = getattr(_pinned, "bufs", None)
     if bufs is None:
         bufs = _pinned.bufs = {}
     key = (_get_device(), stream_ptr)
     buf = bufs.get(key)
-    if buf is None or buf[0].numel() < words:
-        t = torch.zeros(max(words, 512), dtype=torch.uint64).pin_memory()
-        buf = bufs[key] = (t, t.numpy())
+    if buf is not None and buf.polled:
+        # the context was left without its wait (a second interrupt), or a call runs inside another one's: what is queued is
+        # waited for before the buffer may go, and its words are left to whoever still reads them
+        torch.cuda.current_stream().synchronize()
+        buf = None
+    if buf is None or buf.host.numel() < words:
+        buf = bufs[key] = _Words(max(words, 512))
     return buf
 
 
-NO_WORD = 0xFFFFFFFFFFFFFFFF    # VI_NO_WORD: no field element
+def pinned_words(words: int, stream_ptr: int):
+    """Pinned host words that kernels of a call write results into and the call reads them from, with a numpy view of
+    the same memory; stream_ptr is torch's current stream.  One buffer per host thread and stream: a call has read its
+    results before the next one on that stream starts, and two threads (or two streams) never see each other's.  Buffers
+    grow and are kept for the life of the thread (a few KiB each)."""
+    buf = _words(words, stream_ptr)
+    return buf.host, buf.view
+
+
+def polled_words(words: int, stream_ptr: int):
+    """The same buffer for results that vi_wait_words() waits for: a context around launches and wait, with `words` words
+    set to NO_WORD."""
+    buf = _words(words, stream_ptr)
+    buf.view[:words] = NO_WORD
+    return buf
 
 
 def read_back_ptr(src: int, nbytes: int, sp: int) -> bytes:

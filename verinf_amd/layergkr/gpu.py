@@ -223,13 +223,12 @@ def mle_eval_t(tables, point: Sequence[int]):
         sp = _lib.stream_ptr()
         ws_bytes = _lib.workspace_bytes("mle_eval", k)
         # the last kernel writes the values into pinned memory, which is polled until all are there
-        host, view = _lib.pinned_words(k, sp)
-        view[:k] = _lib.NO_WORD
-        with _lib.stream_lock(sp):
-            ws = _lib.workspace(ws_bytes, "mle", sp)
-            _lib.check(L.vi_mle_eval(mat.data_ptr(), k, 1 << n, _point(point), n, host.data_ptr(), ws.data_ptr(), ws_bytes, sp))
-        _lib.check(L.vi_wait_words(host.data_ptr(), 1, k, k, sp))
-        vals = view[:k].tolist()
+        with _lib.polled_words(k, sp) as out:
+            with _lib.stream_lock(sp):
+                ws = _lib.workspace(ws_bytes, "mle", sp)
+                _lib.check(L.vi_mle_eval(mat.data_ptr(), k, 1 << n, _point(point), n, out.host.data_ptr(), ws.data_ptr(), ws_bytes, sp))
+            _lib.check(L.vi_wait_words(out.host.data_ptr(), 1, k, k, sp))
+            vals = out.view[:k].tolist()
     return vals[0] if one else vals
 
 
@@ -382,25 +381,24 @@ def prove_terms_gpu(terms, coin, field_p: int, mask=None, mu0: int = 0):
     dev = tables[0].device
     with _lib.on_device(dev):
         sp = _lib.stream_ptr()
-        host, view = _lib.pinned_words(8 * n_rounds, sp)
-        view[:8 * n_rounds] = _lib.NO_WORD
-        samples_p = host.data_ptr()
         chal = (ctypes.c_uint64 * n_rounds)(*challenges)
         tables_p = prob.pointers()
-        with _lib.stream_lock(sp):
-            ws = _lib.workspace(_lib.workspace_bytes("sumcheck_prove_coins", size), "sumcheck_coins", sp)
-            # the folded tables live in one cached scratch buffer, a half-length slice per table (the caller's
-            # tensors are never written)
-            half_bytes = (size // 2) * 8
-            work = _lib.workspace(max(prob.n_tables * half_bytes, 256), "sumcheck_work", sp)
-            first = work.data_ptr()
-            work_p = (ctypes.c_void_p * prob.n_tables)(*range(first, first + prob.n_tables * half_bytes, half_bytes))
-            _lib.check(L.vi_sumcheck_prove_coins(tables_p, work_p, prob.n_tables, size, prob.term_off, prob.factor_idx,
-                                                 prob.coeffs, prob.n_terms, chal, samples_p, ws.data_ptr(), ws.numel(), sp))
-        # while the kernels run: what the masks add to the samples
-        added = [[_poly_eval(h, x, field_p) for x in range(deg + 1)] for h in masks]
-        _lib.check(L.vi_wait_words(samples_p, n_rounds, 8, deg + 1, sp))
-        rows = view[:8 * n_rounds].reshape(n_rounds, 8)[:, :deg + 1].tolist()
+        with _lib.polled_words(8 * n_rounds, sp) as samples:
+            samples_p = samples.host.data_ptr()
+            with _lib.stream_lock(sp):
+                ws = _lib.workspace(_lib.workspace_bytes("sumcheck_prove_coins", size), "sumcheck_coins", sp)
+                # the folded tables live in one cached scratch buffer, a half-length slice per table (the caller's
+                # tensors are never written)
+                half_bytes = (size // 2) * 8
+                work = _lib.workspace(max(prob.n_tables * half_bytes, 256), "sumcheck_work", sp)
+                first = work.data_ptr()
+                work_p = (ctypes.c_void_p * prob.n_tables)(*range(first, first + prob.n_tables * half_bytes, half_bytes))
+                _lib.check(L.vi_sumcheck_prove_coins(tables_p, work_p, prob.n_tables, size, prob.term_off, prob.factor_idx,
+                                                     prob.coeffs, prob.n_terms, chal, samples_p, ws.data_ptr(), ws.numel(), sp))
+            # while the kernels run: what the masks add to the samples
+            added = [[_poly_eval(h, x, field_p) for x in range(deg + 1)] for h in masks]
+            _lib.check(L.vi_wait_words(samples_p, n_rounds, 8, deg + 1, sp))
+            rows = samples.view[:8 * n_rounds].reshape(n_rounds, 8)[:, :deg + 1].tolist()
     # S(0) + S(1) of the first round is the sum over the cube
     claim = (rows[0][0] + rows[0][1] + mu0) % field_p
     if mask is not None:
