@@ -259,7 +259,8 @@ int vi_sumcheck_prove(const uint64_t *const *tables, uint64_t *const *work, int 
  *   challenges    host, v = log2(size) words (reduced mod p by the callee)
  *   samples       v rows of 8 words the GPU can write (device memory or pinned host memory): S_round(x) at
  *                 samples[8 * round + x], x = 0..deg, complete once the stream has reached the end of the call's work
- *   work          n_tables device buffers of size/2 words; tables are left untouched
+ *   work          n_tables device buffers of size/2 words; tables are left untouched.  work[t] == tables[t] folds in place,
+ *                 in a launch or more per round for sums under a common factor
  *   ws            vi_sumcheck_prove_coins_workspace_bytes(size) bytes of device scratch
  * At most 40 rounds. */
 size_t vi_sumcheck_prove_coins_workspace_bytes(int64_t size);

@@ -21,6 +21,7 @@
 #define __host__
 #define __forceinline__ inline
 #define __launch_bounds__(...)
+#define __align__(n) __attribute__((aligned(n)))
 #define __shared__ thread_local
 #define ext_vector_type(n) vector_size(4 * (n))                       // 32-bit elements only
 
@@ -37,7 +38,7 @@ inline dim3 threadIdx, blockIdx, blockDim, gridDim;
 namespace simt {
 
 constexpr size_t STACK = 256 << 10;
-enum State { READY, AT_WAVE, AT_GROUP, DONE };
+enum State { READY, AT_WAVE, AT_LANES, AT_VOTE, AT_GROUP, DONE };
 struct Fiber {
     ucontext_t ctx;
     State state;
@@ -72,6 +73,19 @@ inline bool release(unsigned lo, unsigned hi, State s) {
     return any;
 }
 
+// what the lanes of a branch do together (a vote, a shuffle) while the others wait behind it: releases the fibers at `s` when every
+// one that is not done waits somewhere
+inline bool release_some(unsigned lo, unsigned hi, State s) {
+    bool any = false;
+    for (unsigned i = lo; i < hi; ++i) {
+        if (fibers[i].state == READY) return false;
+        any |= fibers[i].state == s;
+    }
+    for (unsigned i = lo; any && i < hi; ++i)
+        if (fibers[i].state == s) fibers[i].state = READY;
+    return any;
+}
+
 inline void run_group(unsigned n) {
     static char *stacks = (char *)mmap(nullptr, 1024 * STACK, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);
     fibers.resize(1024);
@@ -95,7 +109,11 @@ inline void run_group(unsigned n) {
             left |= fibers[i].state != DONE;
         }
         if (!left) return;
-        for (unsigned w = 0; w < n; w += 64) ran |= release(w, w + 64 < n ? w + 64 : n, AT_WAVE);
+        for (unsigned w = 0; w < n; w += 64) {
+            const unsigned end = w + 64 < n ? w + 64 : n;
+            // votes stand in branches, so their lanes go before those that wait at a shuffle behind the branch
+            ran |= release(w, end, AT_WAVE) || release_some(w, end, AT_VOTE) || release_some(w, end, AT_LANES);
+        }
         ran |= release(0, n, AT_GROUP);
         if (!ran) {
             fprintf(stderr, "a barrier that not every thread reaches\n");
@@ -128,6 +146,7 @@ inline void launch(dim3 grid, dim3 block, const std::function<void()> &f) {
 }
 
 inline int any_true, wave_any[16];
+inline uint64_t wave_v[16][64];                                       // of shuffles, by wavefront and lane
 inline int32_t wave_a[16][64][4], wave_b[16][64][4];                  // operands of a matrix instruction, by wavefront and lane
 
 }  // namespace simt
@@ -147,13 +166,26 @@ inline int __syncthreads_or(int v) {
 inline int __any(int v) {                                             // over the threads of a wavefront that are still there
     int &any = simt::wave_any[threadIdx.x >> 6];
     any = 0;
-    simt::wait_at(simt::AT_WAVE);
+    simt::wait_at(simt::AT_VOTE);
     any |= v != 0;
-    simt::wait_at(simt::AT_WAVE);
+    simt::wait_at(simt::AT_VOTE);
     const int r = any;
-    simt::wait_at(simt::AT_WAVE);
+    simt::wait_at(simt::AT_VOTE);
     return r;
 }
+// the value of lane `from` of the wavefront, the own one where there is no such lane
+inline uint64_t simt_lane(uint64_t v, int from) {
+    uint64_t *lanes = simt::wave_v[threadIdx.x >> 6];
+    lanes[threadIdx.x & 63] = v;
+    simt::wait_at(simt::AT_LANES);
+    const uint64_t r = from >= 0 && from < 64 ? lanes[from] : v;
+    simt::wait_at(simt::AT_LANES);
+    return r;
+}
+inline uint64_t __shfl(uint64_t v, int lane, int) { return simt_lane(v, lane); }
+inline uint64_t __shfl_xor(uint64_t v, int mask, int) { return simt_lane(v, (int)(threadIdx.x & 63) ^ mask); }
+inline uint64_t __shfl_up(uint64_t v, unsigned d, int) { return simt_lane(v, (int)(threadIdx.x & 63) - (int)d); }
+inline uint64_t __shfl_down(uint64_t v, unsigned d, int) { return simt_lane(v, (int)(threadIdx.x & 63) + (int)d); }
 inline void __threadfence_system() {}
 #define __builtin_amdgcn_fence(...) ((void)0)
 #define __builtin_amdgcn_wave_barrier() simt::wait_at(simt::AT_WAVE)
@@ -181,6 +213,8 @@ inline uint32_t __umul24(uint32_t a, uint32_t b) { return (a & 0xFFFFFF) * (b & 
 inline uint32_t __umulhi(uint32_t a, uint32_t b) { return (uint32_t)(((uint64_t)a * b) >> 32); }
 inline uint32_t __float_as_uint(float f) { uint32_t u; memcpy(&u, &f, 4); return u; }
 inline uint32_t min(uint32_t a, uint32_t b) { return a < b ? a : b; }
+inline uint32_t max(uint32_t a, uint32_t b) { return a > b ? a : b; }
+inline int min(int a, int b) { return a < b ? a : b; }
 
 // sum of the products of four signed bytes, plus c
 inline int __builtin_amdgcn_sdot4(int a, int b, int c, bool) {
@@ -229,6 +263,14 @@ enum hipStreamCaptureStatus { hipStreamCaptureStatusNone = 0 };
 inline hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus *s) { *s = hipStreamCaptureStatusNone; return hipSuccess; }
 inline hipError_t hipGetDevice(int *d) { *d = 0; return hipSuccess; }
 inline hipError_t hipFuncSetAttribute(const void *, int, int) { return hipSuccess; }
+#define HIP_SYMBOL(s) s
+template <class T>
+hipError_t hipGetSymbolAddress(void **p, T &symbol) { *p = (void *)&symbol; return hipSuccess; }
+enum hipDeviceAttribute_t { hipDeviceAttributeMultiprocessorCount };
+inline hipError_t hipDeviceGetAttribute(int *v, hipDeviceAttribute_t, int) { *v = 256; return hipSuccess; }
+template <class K>
+hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int *n, K, int, size_t) { *n = 4; return hipSuccess; }
+inline hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 inline hipError_t hipSetDevice(int) { return hipSuccess; }
 inline hipError_t hipMalloc(void **p, size_t n) { *p = malloc(n); return hipSuccess; }
 inline hipError_t hipFree(void *p) { free(p); return hipSuccess; }

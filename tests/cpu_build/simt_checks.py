@@ -265,6 +265,72 @@ def tables(so):
     print("tables", flush=True)
 
 
+# Sums that take every route of vi_sumcheck_prove_coins: products with kernels of their own, the hadamard gate, sums under a common
+# factor (table 0) in all their forms, other sums in registers, in memory and beyond one descriptor.
+SUMS = {
+    "one": [(5, [0])],
+    "two": [(7, [0, 1])],
+    "three": [(1, [0, 1, 2])],
+    "four": [(3, [0, 1, 2, 3])],
+    "gate": [(3, [0, 1, 2]), (P - 3, [0, 3])],
+    "products": [(3, [0, 1, 2]), (5, [0, 3, 4])],
+    "singles": [(3, [0, 1]), (P - 7, [2, 0]), (11, [0, 3])],
+    "constant": [(3, [0, 1]), (P - 2, [0])],
+    "only a constant beside products": [(3, [0, 1, 2]), (9, [0])],
+    "mixed": [(3, [0, 1, 2]), (P - 3, [0, 3]), (9, [4, 0]), (6, [0, 5, 5]), (P - 6, [0, 5]), (4, [0])],
+    "shared": [(3, [0, 1, 2]), (5, [1, 0, 3]), (7, [2, 3, 0]), (8, [0, 1]), (0, [0, 1, 3])],
+    "common twice": [(3, [0, 0, 1]), (5, [0, 0]), (2, [1, 2, 0])],
+    "many": [(k + 1, [0, k % 37 + 1]) for k in range(50)] + [(k + 2, [0, k + 1, k + 18]) for k in range(20)],
+    "registers": [(3, [0, 1]), (4, [2, 3])],
+    "memory": [(k + 3, [k, k + 1, 10 - k]) for k in range(10)],
+    "degree four": [(2, [0, 1, 2, 3]), (3, [0, 4])],
+    "rewritten": [(2, [0, 1, 2])] + [(k + 2, [0, 3 + k]) for k in range(130)],
+}
+
+
+def sumcheck(so):
+    """Proofs with work buffers and scratch of exactly the stated sizes, tables apart from them and folded in place."""
+    L = ctypes.CDLL(so)
+    L.vi_sumcheck_prove_coins_workspace_bytes.restype, L.vi_sumcheck_prove_coins_workspace_bytes.argtypes = SZ, [I64]
+    L.vi_sumcheck_prove_coins.argtypes = [VP, VP, ctypes.c_int, I64, VP, VP, VP, ctypes.c_int, VP, VP, VP, SZ, VP]
+    L.simt_error.restype = ctypes.c_char_p
+    NO_WORD = np.uint64((1 << 64) - 1)
+
+    def check(form, v, buffers):
+        terms, size = SUMS[form], 1 << v
+        n = 1 + max(max(fs) for _, fs in terms)
+        print("sumcheck", form, v, buffers, flush=True)
+        tabs = [field(size, 100 * v + t) for t in range(n)]
+        raw = [t.copy() for t in tabs]
+        raw[0][0], raw[-1][-1] = NO_WORD, np.uint64(P)         # caller words at and above p
+        tabs[0][0], tabs[-1][-1] = int(NO_WORD) % P, 0
+        coins = field(v, v)
+        src = [t.copy() for t in raw]
+        work = src if buffers == "in place" else [np.full(max(size // 2, 1), 0xA5A5A5A5, dtype=np.uint64) for _ in range(n)]
+        off = np.cumsum([0] + [len(fs) for _, fs in terms]).astype(np.int32)
+        idx = np.array([f for _, fs in terms for f in fs], dtype=np.int32)
+        coeffs = np.array([c for c, _ in terms], dtype=np.uint64)
+        samples = np.full(8 * v, NO_WORD, dtype=np.uint64)
+        ws = scratch(L.vi_sumcheck_prove_coins_workspace_bytes(size))
+        rc = L.vi_sumcheck_prove_coins((VP * n)(*[t.ctypes.data for t in src]), (VP * n)(*[t.ctypes.data for t in work]), n, size, ptr(off), ptr(idx),
+                                       ptr(coeffs), len(terms), ptr(coins), ptr(samples), ptr(ws), len(ws), None)
+        assert rc == 0, L.simt_error()
+        _, want, _ = O.sumcheck_prove(tabs, terms, [int(c) for c in coins])
+        deg = max(len(fs) for _, fs in terms)
+        assert samples.reshape(v, 8)[:, :deg + 1].tolist() == want, (form, v, buffers)
+        if buffers == "apart":
+            assert all(np.array_equal(a, b) for a, b in zip(src, raw)), "caller's table was modified"
+
+    # lengths below the lanes of a wavefront, one to eight entries a lane, one pass of three rounds and two, each with every remainder
+    for form, terms in SUMS.items():
+        common = sum(len(fs) <= 3 and 0 in fs for _, fs in terms) == len(terms) > 1
+        for v in ((1, 6, 8, 9, 10, 11, 12) if common and len(terms) < 20 else (1, 6, 10) if len(terms) > 20 else (2, 5, 9, 11)):
+            check(form, v, "apart")
+        for v in (2, 10 if len(terms) < 20 else 7):
+            check(form, v, "in place")
+    print("sumcheck", flush=True)
+
+
 if __name__ == "__main__":
     globals()[sys.argv[1]](sys.argv[2])
     print("OK")

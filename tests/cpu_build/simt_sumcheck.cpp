@@ -1,0 +1,5 @@
+// Sumcheck proofs (verinf_amd/csrc/sumcheck.hip) on the CPU, launches and all.
+#include <hip/hip_runtime.h>
+#include "../../verinf_amd/csrc/sumcheck.hip"
+extern "C" const char *simt_error() { return vi::err_buf(); }
+extern "C" long simt_launches() { return simt::launches; }

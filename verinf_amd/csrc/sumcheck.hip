@@ -1587,8 +1587,8 @@ int prove_coins_impl(const char *who, const uint64_t *const *tables, uint64_t *c
     C.deg = deg;
 
     // products of two tables and single tables under a common factor: three rounds per pass (the hadamard gate batch of four tables
-    // has kernels of its own).  Not the rewritten problem of prove_coins_reduced, which has more single tables than a descriptor and whose
-    // tables are the work buffers: a row of workgroups would write over entries of the common factor that others still have to read
+    // has kernels of its own).  Not where the tables are the work buffers, as in the rewritten problem of prove_coins_reduced: a row of
+    // workgroups would write over entries of the common factor that others still have to read
     if (may_reduce) {
         SumShape S;
         if (sum_shape(n_tables, term_off, factor_idx, coeffs, n_terms, S) &&
@@ -1769,6 +1769,23 @@ int prove_coins_impl(const char *who, const uint64_t *const *tables, uint64_t *c
     return VI_OK;
 }
 
+// whether a work buffer lies over any of the tables (each is looked at by itself only where the room around all buffers has a table in it)
+bool work_over_tables(const uint64_t *const *tables, uint64_t *const *work, int n_tables, i64 size) {
+    auto over = [&](int t, const uint64_t *lo, const uint64_t *hi) {
+        return (uintptr_t)tables[t] < (uintptr_t)hi && (uintptr_t)lo < (uintptr_t)(tables[t] + size);
+    };
+    const uint64_t *lo = work[0], *hi = work[0];
+    for (int t = 1; t < n_tables; ++t) {
+        if ((uintptr_t)work[t] < (uintptr_t)lo) lo = work[t];
+        if ((uintptr_t)work[t] > (uintptr_t)hi) hi = work[t];
+    }
+    for (int t = 0; t < n_tables; ++t)
+        if (over(t, lo, hi + size / 2))
+            for (int u = 0; u < n_tables; ++u)
+                if (over(t, work[u], work[u] + size / 2)) return true;
+    return false;
+}
+
 }  // namespace
 
 int vi_sumcheck_prove_coins(const uint64_t *const *tables, uint64_t *const *work, int n_tables, int64_t size,
@@ -1786,8 +1803,9 @@ int vi_sumcheck_prove_coins(const uint64_t *const *tables, uint64_t *const *work
     if (rc) return rc;
     for (int t = 0; t < n_tables; ++t)
         if (!work[t]) return vi::fail(VI_EINVAL, "%s: null work buffer %d", who, t);
+    // tables that are folded in place take the launches in which a thread reads every entry that it writes
     return prove_coins_impl(who, tables, work, n_tables, size, term_off, factor_idx, coeffs, n_terms, deg, challenges, samples,
-                            (u64 *)ws, (hipStream_t)stream, true);
+                            (u64 *)ws, (hipStream_t)stream, !work_over_tables(tables, work, n_tables, size));
 }
 
 }  // extern "C"
