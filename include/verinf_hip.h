@@ -258,7 +258,8 @@ int vi_sumcheck_prove(const uint64_t *const *tables, uint64_t *const *work, int 
  * other sums keep one launch per round.
  *   challenges    host, v = log2(size) words (reduced mod p by the callee)
  *   samples       v rows of 8 words the GPU can write (device memory or pinned host memory): S_round(x) at
- *                 samples[8 * round + x], x = 0..deg, complete once the stream has reached the end of the call's work
+ *                 samples[8 * round + x], x = 0..deg, complete once the stream has reached the end of the call's work.  Each
+ *                 is stored once and past the caches, so that the host may poll them in pinned memory (vi_wait_words)
  *   work          n_tables device buffers of size/2 words; tables are left untouched.  work[t] == tables[t] folds in place,
  *                 in a launch or more per round for sums under a common factor
  *   ws            vi_sumcheck_prove_coins_workspace_bytes(size) bytes of device scratch
@@ -328,7 +329,8 @@ int vi_pad_rows(const uint8_t *seed, int64_t row_offset, const uint64_t *message
  * order of mle_eval and of the sumcheck folds.
  * vi_mle_eval replaces mle_eval (layergkr/sumcheck.py:40-48) for device tables: out[t] = the
  * multilinear extension of row t of `tables` (n_tables rows of 2^n_vars words, pitch row_stride)
- * at z (z_0 on the most significant bit), one pass per table; out is a device array of n_tables words.
+ * at z (z_0 on the most significant bit), one pass per table; out is n_tables words that the GPU
+ * can write, device memory or pinned host memory that the host may poll (vi_wait_words).
  * Workspace: vi_mle_eval_workspace_bytes(n_tables) = 8 KiB per table. */
 int vi_eq_vector(const uint64_t *z, int n_vars, int msb_first, uint64_t *out, void *stream);
 size_t vi_mle_eval_workspace_bytes(int64_t n_tables);

@@ -14,6 +14,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <functional>
+#include <map>
 #include <vector>
 
 #define __global__
@@ -145,6 +146,7 @@ inline void launch(dim3 grid, dim3 block, const std::function<void()> &f) {
         }
 }
 
+inline std::map<const void *, int> system_stores;                     // how often a word was stored for the host to see at once
 inline int any_true, wave_any[16];
 inline uint64_t wave_v[16][64];                                       // of shuffles, by wavefront and lane
 inline int32_t wave_a[16][64][4], wave_b[16][64][4];                  // operands of a matrix instruction, by wavefront and lane
@@ -191,7 +193,13 @@ inline void __threadfence_system() {}
 #define __builtin_amdgcn_wave_barrier() simt::wait_at(simt::AT_WAVE)
 #define __builtin_nontemporal_load(p) (*(p))
 #define __hip_atomic_load(p, order, scope) (*(p))
-#define __hip_atomic_store(p, v, order, scope) (*(p) = (v))
+enum { __HIP_MEMORY_SCOPE_AGENT = 4, __HIP_MEMORY_SCOPE_SYSTEM = 5 };
+template <class T, class V>
+void simt_store(T *p, V v, int scope) {
+    *p = (T)v;
+    if (scope == __HIP_MEMORY_SCOPE_SYSTEM) ++simt::system_stores[p];
+}
+#define __hip_atomic_store(p, v, order, scope) simt_store(p, v, scope)
 #define __builtin_nontemporal_store(v, p) (*(p) = (v))
 
 template <class T, class V>

@@ -294,6 +294,7 @@ def sumcheck(so):
     L.vi_sumcheck_prove_coins_workspace_bytes.restype, L.vi_sumcheck_prove_coins_workspace_bytes.argtypes = SZ, [I64]
     L.vi_sumcheck_prove_coins.argtypes = [VP, VP, ctypes.c_int, I64, VP, VP, VP, ctypes.c_int, VP, VP, VP, SZ, VP]
     L.simt_error.restype = ctypes.c_char_p
+    L.simt_system_stores.argtypes = [VP]
     NO_WORD = np.uint64((1 << 64) - 1)
 
     def check(form, v, buffers):
@@ -311,6 +312,7 @@ def sumcheck(so):
         idx = np.array([f for _, fs in terms for f in fs], dtype=np.int32)
         coeffs = np.array([c for c, _ in terms], dtype=np.uint64)
         samples = np.full(8 * v, NO_WORD, dtype=np.uint64)
+        stores = [L.simt_system_stores(samples.ctypes.data + 8 * x) for x in range(8 * v)]
         ws = scratch(L.vi_sumcheck_prove_coins_workspace_bytes(size))
         rc = L.vi_sumcheck_prove_coins((VP * n)(*[t.ctypes.data for t in src]), (VP * n)(*[t.ctypes.data for t in work]), n, size, ptr(off), ptr(idx),
                                        ptr(coeffs), len(terms), ptr(coins), ptr(samples), ptr(ws), len(ws), None)
@@ -318,6 +320,10 @@ def sumcheck(so):
         _, want, _ = O.sumcheck_prove(tabs, terms, [int(c) for c in coins])
         deg = max(len(fs) for _, fs in terms)
         assert samples.reshape(v, 8)[:, :deg + 1].tolist() == want, (form, v, buffers)
+        # the host may poll the samples: each is stored once, and past the caches
+        for x in range(8 * v):
+            at = samples.ctypes.data + 8 * x
+            assert L.simt_system_stores(at) - stores[x] == (x % 8 <= deg), (form, v, x)
         if buffers == "apart":
             assert all(np.array_equal(a, b) for a, b in zip(src, raw)), "caller's table was modified"
 

@@ -84,6 +84,9 @@ __device__ __forceinline__ u64 wave_sum(u64 v) {
     return v;
 }
 
+// A finished sample, straight through to memory: it may lie in host memory that is being polled.
+__device__ __forceinline__ void put_sample(u64 *out, u64 v) { __hip_atomic_store(out, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); }
+
 // MODE 0: evaluate pairs (src[i], src[half+i]), i < half
 // MODE 1: fold by r into dst (i < half), no evaluation
 // MODE 2: fold by r and evaluate the next round: i < half/2
@@ -298,7 +301,7 @@ __global__ __launch_bounds__(BLOCK) void k_round(const Desc D, i64 half, u64 r, 
                 if (scale != 1) v = gl::mul(v, scale);
             }
             if (x == 0) s0 = v;
-            out[x] = v;
+            put_sample(out + x, v);
         }
         if (flag) {
             __threadfence_system();
@@ -587,7 +590,7 @@ __global__ __launch_bounds__(BLOCK) void k_final(const u64 *partial, int nb, int
     u64 s0 = 0;
     for (int x = 0; x <= deg; ++x) {
         if (skip1 && x == 1) {
-            if (threadIdx.x == 0) out[1] = gl::sub(claim, s0);
+            if (threadIdx.x == 0) put_sample(out + 1, gl::sub(claim, s0));
             continue;
         }
         u64 acc = 0;
@@ -599,7 +602,7 @@ __global__ __launch_bounds__(BLOCK) void k_final(const u64 *partial, int nb, int
             u64 v = red[0];
             for (int i = 1; i < BLOCK / 64; ++i) v = gl::add(v, red[i]);
             v = scale == 1 ? v : gl::mul(v, scale);
-            out[x] = v;
+            put_sample(out + x, v);
             if (x == 0) s0 = v;
         }
         __syncthreads();

@@ -195,8 +195,7 @@ __device__ __forceinline__ void finish_samples(const ChainDesc &C, FinishShared 
             if (x <= C.deg) {
                 u64 v = y[x];
                 if (inf && x == C.deg) v = gl::addc(gl::mul(top_a, claim), top_b);
-                // straight through to memory: `out` may be host memory that is being polled
-                __hip_atomic_store(&out[(i64)k * NSAMP + x], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                put_sample(out + (i64)k * NSAMP + x, v);
             }
         }
     }
