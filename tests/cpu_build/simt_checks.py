@@ -83,7 +83,7 @@ def lookup(so):
 
     # one and several groups, copies per entry, both sides of the small table, slices, one atomic per look-up
     for n_x, n_t in ((0, 5), (1, 1), (9000, 3), (500, 1024), (9001, 1025), (300, 4096), (9001, 4096), (9001, 4097), (700, 8191), (900, 8192),
-                     (131073, 8192), (9001, 32771), (140001, 32772), (140001, 65539)):
+                     (131073, 8192), (140001, 8193), (131073, 16384), (140001, 16385), (9001, 32771), (140001, 32772), (140001, 65539)):
         rng = np.random.default_rng(n_x + n_t)
         span = np.arange(n_t, dtype=np.uint64)
         x = rng.integers(0, n_t + n_t // 8 + 1, n_x).astype(np.uint64)

@@ -168,3 +168,19 @@ def test_counters_of_16_bits(n_x, n_table, kind):
     x = table[at]
     got = to_np(cp.lookup_multiplicities(to_dev(x), to_dev(table)))
     assert np.array_equal(got, np.bincount(at, minlength=n_table).astype(np.uint64))
+
+
+@pytest.mark.parametrize("n_table", [8192, 8193, 16384, 16385, 32768])
+@pytest.mark.parametrize("n_x", [131073, 1500001, 256 * 65535])
+def test_few_entries_of_16_bit_counters(n_x, n_table):
+    """Four, two and one copy per entry, whose sums are what a counter holds at most."""
+    from verinf_amd.prover import cuda_primitives as cp
+    rng = np.random.default_rng(n_x + n_table)
+    few = np.array([0, 1, 2, n_table // 2, n_table - 2, n_table - 1], dtype=np.uint64)
+    print(n_x, n_table, flush=True)
+    for hot in (few, few[-1:]):
+        x = hot[rng.integers(0, len(hot), n_x)]
+        want = np.bincount(x.astype(np.int64), minlength=n_table).astype(np.uint64)
+        for table in (np.arange(n_table, dtype=np.uint64), rng.permutation(n_table).astype(np.uint64)):
+            got = to_np(cp.lookup_multiplicities(to_dev(x), to_dev(table)))
+            assert np.array_equal(got, want[table.astype(np.int64)])

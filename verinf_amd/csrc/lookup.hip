@@ -137,7 +137,7 @@ __device__ __forceinline__ u64 index_of(u64 x, const Finder &F, bool diagonal, b
 }
 
 // counts of the entries base .. base + mine - 1 among x[lo .. hi - 1], each at(value) an index of the table; `copies` (a power
-// of two) interleaved counters per entry.  HALF: counters of 16 bits, two to a word, one copy.
+// of two) interleaved counters per entry, so that look-ups of one entry do not queue up.  HALF: counters of 16 bits, two to a word.
 template <bool HALF, class F>
 __device__ __forceinline__ void count(const u64 *__restrict__ x, i64 lo, i64 hi, u64 base, int mine, int copies, u32 *counts, F at) {
     const int copy = threadIdx.x & (copies - 1);
@@ -150,8 +150,8 @@ __device__ __forceinline__ void count(const u64 *__restrict__ x, i64 lo, i64 hi,
 #pragma unroll
         for (int u = 0; u < UN; ++u) times[u] = i0 + u * COUNT_THREADS < hi ? 1 : 0;
         if (HALF) {
-            // without copies a value that many look-ups share would queue up: those of the thread that equal its first go as one
-            // (1.5 M look-ups of one entry of 2^16: 34.5 us without this, 17.1 with it, 27.1 with 32-bit counters)
+            // with few copies or none, look-ups of a thread that equal its first go as one (1.5 M look-ups of one entry of 2^16: 34.5 us
+            // without this, 17.1 with it, 27.1 with 32-bit counters)
 #pragma unroll
             for (int u = 1; u < UN; ++u) {
                 const bool same = v[u] == v[0];
@@ -164,7 +164,7 @@ __device__ __forceinline__ void count(const u64 *__restrict__ x, i64 lo, i64 hi,
             if (times[u]) {
                 const u64 j = at(v[u]) - base;
                 if (j >= (u64)mine) continue;
-                if (HALF) atomicAdd(&counts[(int)j >> 1], times[u] << (16 * ((int)j & 1)));
+                if (HALF) atomicAdd(&counts[((int)j >> 1) * copies + copy], times[u] << (16 * ((int)j & 1)));
                 else atomicAdd(&counts[(int)j * copies + copy], 1u);
             }
         }
@@ -177,12 +177,25 @@ __device__ __forceinline__ void put(u64 *mult, u64 c, int accumulate) {
     else if (c) atomicAdd((unsigned long long *)mult, (unsigned long long)c);
 }
 
-// a workgroup's counts to its row, or straight to the result where there are no rows
+// a workgroup's counts to its row, or straight to the result where there are no rows.  Two or four copies are one LDS read (1.5 M look-ups
+// in a range of 2^13 12.0 us a copy at a time, 11.0 this way).
 __device__ __forceinline__ void put_counts(const u32 *counts, int mine, int copies, u32 *row, bool aligned, u64 *mult, int accumulate) {
     const int tid = threadIdx.x;
     if (row && copies == 1 && aligned && (mine & 3) == 0) {
         uint4 *to = reinterpret_cast<uint4 *>(row);
         for (int i = tid; i < mine / 4; i += COUNT_THREADS) to[i] = reinterpret_cast<const uint4 *>(counts)[i];
+        return;
+    }
+    if (row && (copies == 2 || copies == 4)) {
+        for (int i = tid; i < mine; i += COUNT_THREADS) {
+            if (copies == 4) {
+                const uint4 c = reinterpret_cast<const uint4 *>(counts)[i];
+                row[i] = c.x + c.y + c.z + c.w;
+            } else {
+                const uint2 c = reinterpret_cast<const uint2 *>(counts)[i];
+                row[i] = c.x + c.y;
+            }
+        }
         return;
     }
     for (int i = tid; i < mine; i += COUNT_THREADS) {
@@ -204,10 +217,10 @@ __global__ __launch_bounds__(COUNT_THREADS) void k_count(const u64 *__restrict__
     u32 *counts = reinterpret_cast<u32 *>(lds_counts);
     constexpr int MOST = HALF ? 2 * SLICE : SLICE;
     const i64 base = (i64)blockIdx.x * MOST, group = blockIdx.y;
-    const int mine = F.n_table - base < MOST ? (int)(F.n_table - base) : MOST, words = HALF ? (mine + 1) / 2 : mine * copies;
+    const int mine = F.n_table - base < MOST ? (int)(F.n_table - base) : MOST, words = HALF ? (mine + 1) / 2 : mine;
     const u32 part = found_part(F);
     // the launch's LDS is a whole number of 16-byte words
-    for (int i = threadIdx.x; i < (words + 3) / 4; i += COUNT_THREADS) lds_counts[i] = make_uint4(0, 0, 0, 0);
+    for (int i = threadIdx.x; i < (words * copies + 3) / 4; i += COUNT_THREADS) lds_counts[i] = make_uint4(0, 0, 0, 0);
     const bool range = !found_any(part, OFF);  // a barrier as well
     if (HALF && range) {
         if (group >= range_groups) return;
@@ -222,10 +235,10 @@ __global__ __launch_bounds__(COUNT_THREADS) void k_count(const u64 *__restrict__
     __syncthreads();
     if (HALF) {
         const i64 row_words = (F.n_table + 1) / 2;
-        put_counts(counts, words, 1, rows + group * row_words + base / 2, (row_words & 3) == 0, nullptr, 0);
+        put_counts(counts, words, copies, rows + group * row_words + base / 2, (row_words & 3) == 0, nullptr, 0);
         return;
     }
-    put_counts(counts, mine, copies, rows ? rows + group * F.n_table + base : nullptr, (F.n_table & 3) == 0, mult + base, accumulate);
+    put_counts(counts, words, copies, rows ? rows + group * F.n_table + base : nullptr, (F.n_table & 3) == 0, mult + base, accumulate);
 }
 
 // The same for a table of up to SMALL_TABLE entries that nothing is known of: every workgroup takes it into its LDS, sees
@@ -409,7 +422,11 @@ Plan make_plan(i64 n_x, i64 n_table, bool promised) {
             L.slices = slices;
             L.groups = groups;
             L.range_groups = range_groups;
+            // as many copies as 32-bit counters would have: 4 of 8192 entries (1.5 M look-ups of eight entries 16.7 us with one, 11.2; 16 M 38.8
+            // and 28.5; 14.3 and 29.0 with 32-bit counters, 1.5 M of any entry 13.8, 10.7 and 11.0), 2 of 16384 (17.5, 14.1; 39.3,
+            // 29.8).  From 32768 on there is one: 1.5 M look-ups of eight entries of 2^16 take 21.6, of 32-bit counters in twice the groups 18.5.
             L.copies = 1;
+            while (n_table * L.copies * 2 <= SLICE) L.copies *= 2;
             L.row_bytes = (size_t)groups * ((n_table + 1) / 2) * sizeof(u32);
             return L;
         }
