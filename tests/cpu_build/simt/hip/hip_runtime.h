@@ -31,6 +31,7 @@ struct dim3 {
     dim3(unsigned x_ = 1, unsigned y_ = 1, unsigned z_ = 1) : x(x_), y(y_), z(z_) {}
 };
 struct alignas(16) ulonglong2 { unsigned long long x, y; };
+inline uint64_t __umul64hi(uint64_t a, uint64_t b) { return (uint64_t)((unsigned __int128)a * b >> 64); }
 struct alignas(8) uint2 { uint32_t x, y; };
 struct alignas(16) uint4 { uint32_t x, y, z, w; };
 inline uint4 make_uint4(uint32_t x, uint32_t y, uint32_t z, uint32_t w) { return uint4{x, y, z, w}; }

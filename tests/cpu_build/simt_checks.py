@@ -224,8 +224,10 @@ def matmul(so):
     L.simt_tile_workspace.restype, L.simt_tile_workspace.argtypes = SZ, [I64, ctypes.c_int]
     L.simt_tile.restype, L.simt_tile.argtypes = None, [VP, VP, VP, I64, I64, I64, ctypes.c_int, VP]
     for m, k, n, fill in ((1, 1, 1, None), (3, 17, 70, "any"), (64, 64, 64, "top"), (65, 100, 65, "half"), (130, 33, 130, None), (5, 8193, 3, "top"),
-                          (120, 70, 250, 4), (128, 64, 256, 4), (128, 130, 128, 2), (67, 5, 100, 2),
-                          (3, 17, 70, "i16"), (64, 64, 128, "i16 top"), (65, 129, 130, "i16"), (5, 1030, 3, "i16 low"), (70, 65, 40, "over a"), (40, 130, 300, "over b")):
+                          (120, 70, 250, 4), (128, 64, 256, 4), (128, 130, 128, 2), (67, 5, 100, 2), (65, 4001, 66, 2),
+                          (3, 17, 70, "i16"), (64, 64, 128, "i16 top"), (65, 129, 130, "i16"), (5, 1030, 3, "i16 low"), (70, 65, 40, "over a"), (40, 130, 300, "over b"),
+                          # residues by one workgroup per slab; more items than workgroups cut up
+                          (3, 8190, 2, "any"), (2, 32768, 3, "i16")):
         print("matmul", m, k, n, fill, flush=True)
         A, B = field((m, k), m), field((k, n), n)
         if fill == "top":

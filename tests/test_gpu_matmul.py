@@ -89,3 +89,25 @@ def test_few_rows(m, k, n):
     got = to_np(cp.gl_matmul(to_dev(A), to_dev(B)))
     cols = np.unique(np.linspace(0, n - 1, min(n, 3_000_000 // (m * k) + 2)).astype(int))
     assert np.array_equal(got[:, cols], (A.astype(object).dot(B[:, cols].astype(object)) % P).astype(np.uint64))
+
+
+# residues by three workgroups a slab and by one (340 slabs and more), of one block and of the first of several; words that the first
+# launch's sample sees and does not see
+@pytest.mark.parametrize("m,k,n", [(256, 1088, 1024), (256, 1089, 1025), (64, 760, 1070), (300, 9000, 500), (100, 16400, 300), (70, 40, 120001)])
+@pytest.mark.parametrize("kind", ["field", "mixed", "few"])
+def test_matmul_of_arbitrary_words(m, k, n, kind):
+    from verinf_amd.prover import cuda_primitives as cp
+    rng = np.random.default_rng(m + k)
+    A = rand_field((m, k), 1) if kind == "field" else rng.integers(0, 1 << 15, (m, k)).astype(np.uint64)
+    B = rng.integers(0, 1 << 15, (k, n)).astype(np.uint64) if kind == "few" else rand_field((k, n), 2)
+    if kind == "few":                                           # a word of A, and a column of B
+        A[m // 2, k // 3] = P - 12345678901
+        B[:, n - 1] = rand_field((k,), 3)
+    print(m, k, n, kind, flush=True)
+    got = to_np(cp.gl_matmul(to_dev(A), to_dev(B)))
+    rows = sorted({0, m // 2, m - 1})
+    cols = np.unique(np.concatenate([[n - 1], np.linspace(0, n - 1, 1 + 1_000_000 // k).astype(int)]))
+    want = (A[rows].astype(object).dot(B[:, cols].astype(object)) % P).astype(np.uint64)
+    assert np.array_equal(got[np.ix_(rows, cols)], want)
+    one = to_np(cp.gl_matmul(to_dev(A), to_dev(np.ones((k, 300), dtype=np.uint64))))[:, 299]              # every row
+    assert np.array_equal(one, (A.astype(object).sum(axis=1) % P).astype(np.uint64))

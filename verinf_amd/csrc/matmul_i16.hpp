@@ -35,8 +35,9 @@ constexpr int BLOCK = 256;
 constexpr int MAX_K = 32768;
 constexpr int UNIT = 16;                       // inner indices of a unit
 constexpr int STEP = 4;                        // units of a step of the product, and of a sum of k_cut
-constexpr int MAX_CUT_BLOCKS = 1020;           // workgroups of k_cut, what is resident at once; each leaves a word that says what it saw
-constexpr size_t GATE_BYTES = 16 + 4 * MAX_CUT_BLOCKS;
+constexpr int MAX_CUT_BLOCKS = 1020;           // workgroups that cut words into bytes, what is resident at once; each leaves a word that says what it saw
+constexpr size_t GATE_BYTES = 16 + 4 * MAX_CUT_BLOCKS;   // whole lines: planes across lines cost their readers and writers 8 %
+static_assert(GATE_BYTES % 128 == 0, "");
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));

@@ -30,6 +30,7 @@
 // operand reads are all contiguous 16-byte accesses in this order, and B is transposed on the way without a pass.
 #include "matmul_rns.hpp"
 
+#include <algorithm>
 #include <utility>
 
 #include "common.hpp"
@@ -44,6 +45,7 @@ constexpr int MODS[NMOD] = {256, 255, 253, 251, 247, 241, 239, 233, 229, 227, 22
 constexpr int MAX_K = 8192;                    // inner indices of one slice
 constexpr int UNIT = 16;                       // inner indices of a unit
 constexpr unsigned RESIDUE_BLOCKS = 768;       // workgroups of k_product where it makes residues: what is resident at once
+constexpr unsigned FEW_SLABS = 340;            // up to so many slabs k_cut takes three workgroups each for the residues
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
@@ -123,10 +125,18 @@ __device__ __forceinline__ void store_residues(const int (&lo)[UNIT], const int 
                                residue<I, CRT>(lo[4 * g + 2], hi[4 * g + 2]), residue<I, CRT>(lo[4 * g + 3], hi[4 * g + 3]));
     planes[I * plane + at] = v;
 }
-template <bool CRT, int... I>
-__device__ __forceinline__ void store_all(const int (&lo)[UNIT], const int (&hi)[UNIT], v4i *planes, i64 plane, i64 at,
-                                          std::integer_sequence<int, I...>) {
-    (store_residues<I, CRT>(lo, hi, planes, plane, at), ...);
+template <bool CRT, int FIRST, int... I>
+__device__ __forceinline__ void store_some(const int (&lo)[UNIT], const int (&hi)[UNIT], v4i *planes, i64 plane, i64 at,
+                                           std::integer_sequence<int, I...>) {
+    (store_residues<FIRST + I, CRT>(lo, hi, planes, plane, at), ...);
+}
+// share `share` of `shares` = 1 or 3 of the moduli
+template <bool CRT>
+__device__ __forceinline__ void store_share(const int (&lo)[UNIT], const int (&hi)[UNIT], v4i *planes, i64 plane, i64 at, unsigned share, unsigned shares) {
+    constexpr auto third = std::make_integer_sequence<int, NMOD / 3>();
+    if (shares == 1 || share == 0) store_some<CRT, 0>(lo, hi, planes, plane, at, third);
+    if (shares == 1 || share == 1) store_some<CRT, NMOD / 3>(lo, hi, planes, plane, at, third);
+    if (shares == 1 || share == 2) store_some<CRT, 2 * NMOD / 3>(lo, hi, planes, plane, at, third);
 }
 
 // ---- cutting up the operands --------------------------------------------------------------------------------------
@@ -134,6 +144,8 @@ __device__ __forceinline__ void store_all(const int (&lo)[UNIT], const int (&hi)
 // columns, so that the sixteen words that a lane reads of B and all stores are contiguous over the wavefront.  A is read along the
 // inner dimension into LDS for that and picked up with the lanes along the rows (an odd pitch in words: no bank conflicts); read by
 // each lane from its own row, 1000 x 4096 words took 37 us, 15 this way.  Inner indices from k to the padded length count as zeros.
+// Residues are made in slabs: the items of A and, for longer runs of memory, one unit of 256 columns of B (in items of B, 128 x 4096 x
+// 4096 94 us, 90 in slabs).
 // The residues of A carry the factor of the remainder theorem, so that the sums of the products come out as its y_i.
 constexpr int ITEM_UNITS = 4, LINES = 64, TILE_PITCH = ITEM_UNITS * UNIT + 1;
 
@@ -148,6 +160,7 @@ struct Cut {
     i64 k;                                     // inner indices of the slice
     int units;
     unsigned b_items, items;                   // items of B (first), of both
+    unsigned wide, b_slabs, slabs;             // slabs of B along its columns, of B (first), of both
 };
 
 // the sixteen words that a thread holds of an item: of its own column of B, or of A in the order of memory
@@ -178,77 +191,88 @@ __device__ __forceinline__ void turn_item(u64 (&w)[UNIT], u64 *tile) {
 #pragma unroll
     for (int u = 0; u < UNIT; ++u) w[u] = tile[lane * TILE_PITCH + wave * UNIT + u];
 }
-__device__ __forceinline__ void store_residues_of(const Cut &D, unsigned it, const u64 (&w)[UNIT]) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const bool is_b = it < D.b_items;
+// residues of a slab, a share of the moduli
+__device__ __forceinline__ void residues(const Cut &D, unsigned slab, u64 *tile, unsigned share, unsigned shares) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const bool is_b = slab < D.b_slabs;
     const Operand &S = is_b ? D.B : D.A;
-    const unsigned id = is_b ? it : it - D.b_items;
-    const i64 unit = (i64)(id / S.groups) * ITEM_UNITS + wave, at = (i64)(id % S.groups) * LINES + lane;
+    u64 w[UNIT];
+    i64 unit, at;
+    if (is_b) {
+        unit = slab / D.wide;
+        at = (i64)(slab - (unsigned)unit * D.wide) * BLOCK + tid;
+        const u64 *src = S.src + unit * UNIT * S.ld + at;
+#pragma unroll
+        for (int u = 0; u < UNIT; ++u) w[u] = at < S.count && unit * UNIT + u < D.k ? __builtin_nontemporal_load(&src[u * S.ld]) : 0;
+    } else {
+        const unsigned id = slab - D.b_slabs;
+        load_item(D, D.b_items + id, w);
+        turn_item(w, tile);
+        unit = (i64)(id / S.groups) * ITEM_UNITS + wave;
+        at = (i64)(id % S.groups) * LINES + lane;
+    }
     if (at >= S.count) return;
     int lo[UNIT], hi[UNIT];
 #pragma unroll
     for (int u = 0; u < UNIT; ++u) balanced_digits(w[u], lo[u], hi[u]);
-    constexpr auto all = std::make_integer_sequence<int, NMOD>();
-    if (is_b) store_all<false>(lo, hi, S.planes, (i64)D.units * S.pitch, unit * S.pitch + at, all);
-    else store_all<true>(lo, hi, S.planes, (i64)D.units * S.pitch, unit * S.pitch + at, all);
-}
-
-// residues of all items of a block, by a launch of any size
-__device__ __forceinline__ void residues(const Cut &D, u64 *tile) {
-    for (unsigned it = blockIdx.x; it < D.items; it += gridDim.x) {
-        u64 w[UNIT];
-        load_item(D, it, w);
-        if (it >= D.b_items) turn_item(w, tile);
-        store_residues_of(D, it, w);
-    }
+    if (is_b) store_share<false>(lo, hi, S.planes, (i64)D.units * S.pitch, unit * S.pitch + at, share, shares);
+    else store_share<true>(lo, hi, S.planes, (i64)D.units * S.pitch, unit * S.pitch + at, share, shares);
 }
 // done: whether matmul_i16.hpp has finished the product (NULL: it was not tried)
 __global__ __launch_bounds__(BLOCK) void k_residues(const Cut D, const u32 *done) {
     __shared__ u64 tile[LINES * TILE_PITCH];
     if (done && *done) return;
-    residues(D, tile);
+    residues(D, blockIdx.x, tile, 0, 1);
 }
 
-// The first launch of a product that matmul_i16.hpp may be able to do, as many workgroups as are resident at once: 31 us for the bytes of
-// 128 x 4096 x 4096 (a workgroup per item 39), 94 for its residues (84).  Products of arbitrary words pay that and k_product, which
-// then finds nothing to do: 128 x 4096 x 4096 167 -> 183 us, 100 x 760 x 1070 29 -> 33; from some 500 rows on the faster products outweigh it
-// (1000 x 4096 x 4096 470 -> 435).  256 words of either operand, the same for every workgroup,
-// decide whether to try (all words of 1000 x 4096 x 4096 read and cut up for nothing would be 37 us); the first item's words are on
-// their way behind them, and the next item's while this one's are cut up.  flags: 0 where all words of a workgroup's items fitted, 1
-// where one did not (the workgroup leaves), 2 if the sample says residues, which the launch then makes.
-// one_block: the product is one block of one slice, so that the items are those of the residues too; otherwise the sample's answer
-// is 1, and the next launch makes the residues of the first block.
-enum { FITS = 0, TOO_LARGE = 1, CUT_TO_RESIDUES = 2 };
+// The first launch of a product that matmul_i16.hpp may be able to do.  Sixteen runs of sixteen words of either operand, the same for every
+// workgroup, decide whether to try (all words of 1000 x 4096 x 4096 read and cut up for nothing would be 37 us; 256 words of either in as
+// many lines cost 2 us more for bytes and 4 for residues, as every workgroup reads them).
+//
+// Bytes: n_flags workgroups, what is resident at once, go over the items, the next item's words on their way while this one's are cut up
+// (128 x 4096 x 4096 32 us, a workgroup per item 39).  flags: FITS where all words of a workgroup's items fitted, TOO_LARGE where one
+// did not (the workgroup leaves).
+//
+// Residues, of the first block: a workgroup per slab (1020 workgroups for all of them 104 us for 128 x 4096 x 4096, 93 this way), of few slabs
+// three that share the moduli (512 x 512 x 512 16 -> 12).  Only flags[0] is written.
+//
+// Products of arbitrary words pay for the look and for k_product, which then finds nothing to do, 3 to 5 us; us with neither, and now:
+// 128 x 4096 x 4096 170 and 175, 64 x 4096 x 4096 156 and 161, 100 x 760 x 1070 28 and 31, 512 x 512 x 512 26.5 and 27.5, 300 x 9000 x 500 117
+// and 124; with the products' loads straight into LDS 500 x 2048 x 2048 89 and 87, 1000 x 4096 x 4096 467 and 423.  Where only
+// few words are too large and the sample misses them, the bytes have been cut for nothing as well: 128 x 4096 x 4096 209, 512 x 512 x 512 33.5,
+// 1000 x 4096 x 4096 457.
+constexpr int SAMPLE_RUN = 16;
+enum { FITS = 0, TOO_LARGE = 1, CUT_TO_RESIDUES = 2 };                // CUT_TO_RESIDUES: by the sample, in flags[0]
 
-__global__ __launch_bounds__(BLOCK, 4) void k_cut(const Cut D, const i16::Job J, int one_block) {
+__global__ __launch_bounds__(BLOCK, 4) void k_cut(const Cut D, const Cut first_block, const i16::Job J, unsigned shares) {
     __shared__ u64 tile[LINES * TILE_PITCH];
     __shared__ int part[BLOCK];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    u64 w[UNIT];
     u32 beyond = 0;
     {
         const i64 na = D.A.count * D.k, nb = D.k * D.B.count;
-        const i64 ea = tid * (na / BLOCK) + (na < BLOCK ? tid : 0), eb = tid * (nb / BLOCK) + (nb < BLOCK ? tid : 0);
+        const u64 run = (u64)(tid / SAMPLE_RUN + 1) * 0x9E3779B97F4A7C15ull;
+        const i64 ea = (i64)__umul64hi(run, (u64)na) + tid % SAMPLE_RUN, eb = (i64)__umul64hi(run, (u64)nb) + tid % SAMPLE_RUN;
         const u64 wa = ea < na ? D.A.src[ea] : 0, wb = eb < nb ? D.B.src[eb] : 0;
-        load_item(D, blockIdx.x, w);
         i16::signed_low(wa, beyond);
         i16::signed_low(wb, beyond);
     }
-    const bool small = !__syncthreads_or((int)beyond);
-    if (!small && !one_block) {
-        if (tid == 0) J.flags[blockIdx.x] = TOO_LARGE;
+    if (__syncthreads_or((int)beyond)) {
+        if (tid == 0 && blockIdx.x == 0) J.flags[0] = CUT_TO_RESIDUES;
+        const unsigned share = blockIdx.x / first_block.slabs;
+        if (share < shares) residues(first_block, blockIdx.x - share * first_block.slabs, tile, share, shares);
         return;
     }
-    for (unsigned it = blockIdx.x; it < D.items; it += gridDim.x) {
+    const unsigned step = (unsigned)J.n_flags;
+    if (blockIdx.x >= step) return;
+    u64 w[UNIT];
+    load_item(D, blockIdx.x, w);
+    for (unsigned it = blockIdx.x; it < D.items; it += step) {
         if (it >= D.b_items) turn_item(w, tile);
         u64 now[UNIT];
 #pragma unroll
         for (int u = 0; u < UNIT; ++u) now[u] = w[u];
-        if (it + gridDim.x < D.items) load_item(D, it + gridDim.x, w);
-        if (!small) {
-            store_residues_of(D, it, now);
-            continue;
-        }
+        if (it + step < D.items) load_item(D, it + step, w);
         const bool is_b = it < D.b_items;
         const i16::Side &S = is_b ? J.B : J.A;
         const unsigned id = is_b ? it : it - D.b_items, groups = is_b ? D.B.groups : D.A.groups;
@@ -261,7 +285,7 @@ __global__ __launch_bounds__(BLOCK, 4) void k_cut(const Cut D, const i16::Job J,
         if (tid < LINES) S.sums[chunk * S.pitch + at] = part[tid] + part[tid + 64] + part[tid + 128] + part[tid + 192];
         __syncthreads();
     }
-    if (tid == 0) J.flags[blockIdx.x] = small ? FITS : CUT_TO_RESIDUES;
+    if (tid == 0) J.flags[blockIdx.x] = FITS;
 }
 
 // The launch behind k_cut: the product of 16-bit numbers; or the residues of the first block, where a word has turned out not to fit
@@ -272,12 +296,15 @@ __global__ __launch_bounds__(BLOCK, 3) void k_product(const Cut D, const i16::Jo
         i16::Lds<MT, NT> product;
         u64 tile[LINES * TILE_PITCH];
     } lds;
-    u32 seen = FITS;
-    for (int i = threadIdx.x; i < J.n_flags; i += BLOCK) seen |= J.flags[i];
-    const bool fits = !__syncthreads_or((int)seen), cut = __syncthreads_or((int)(seen & CUT_TO_RESIDUES));
+    u32 seen = J.flags[0];
+    const bool cut = seen == CUT_TO_RESIDUES;
+    if (!cut)
+        for (int i = threadIdx.x; i < J.n_flags; i += BLOCK) seen |= J.flags[i];
+    const bool fits = !cut && !__syncthreads_or((int)seen);
     if (blockIdx.x == 0 && threadIdx.x == 0) *J.done = fits;
+    if (cut) return;
     if (!fits) {
-        if (!cut) residues(D, lds.tile);
+        for (unsigned it = blockIdx.x; it < D.slabs; it += gridDim.x) residues(D, it, lds.tile, 0, 1);
     } else if (blockIdx.x < (unsigned)(J.tiles * J.slices)) {
         i16::product<MT, NT>(J, lds.product);
     }
@@ -290,13 +317,18 @@ struct ModConst {
 };
 
 // One 64 WM x 64 WN tile of one plane per workgroup: four wavefronts in a 2 x 2 square, each WM x WN MFMA tiles of
-// 32 x 32.  BKU units of the inner dimension per step through two LDS buffers, the next step's loads going straight into the one
-// while the other is multiplied (through registers: 346 us at 1000 x 4096 x 4096, 334 this way; three buffers 375).
-template <int WM, int WN, int BKU, int OCC>
+// 32 x 32.  BKU units of the inner dimension per step through two LDS buffers.  The next step's loads are in registers while the
+// current one is multiplied, or, STRAIGHT, go straight into the other buffer, which leaves room for another workgroup on a CU.  With 128 x
+// 256 tiles straight is faster at all sizes (1000 x 4096 x 4096 369 us through registers, 308; three buffers 375), with the smaller ones at
+// inner dimensions below some 4000 (us a call: 500 x 2048 x 2048 98 and 91, 777 x 1234 x 2345 136 and 126, 256 x 4096 x 3000 167 and 163; 256 x
+// 4096 x 4096 236 and 242, 128 x 8000 x 4096 396 and 412), 64 x 64 only where there are several rounds of workgroups (64 x 1000 x 12000
+// 114 and 112, 64 x 4096 x 4096 165 and 169; the launch of 512 x 512 x 512 10.2 and 12.0).
+template <int WM, int WN, int BKU, int OCC, bool STRAIGHT>
 __global__ __launch_bounds__(BLOCK, OCC) void k_residue_gemm(const v4i *__restrict__ Ap, const v4i *__restrict__ Bp, u32 *__restrict__ Cp,
                                                              int units, i64 mpad, i64 npad, int mt, int nt, ModConst K, const u32 *done) {
     constexpr int TM = 64 * WM, TN = 64 * WN;
-    constexpr int LOADS = BKU * (TM + TN) / BLOCK;                     // loads of 64 16-byte words of a step per wavefront
+    constexpr int LA = BKU * TM / BLOCK, LB = BKU * TN / BLOCK;
+    constexpr int LOADS = LA + LB;                                     // loads of 64 16-byte words of a step per wavefront
     __shared__ v4i As[2][BKU * TM];
     __shared__ v4i Bs[2][BKU * TN];
     if (done && *done) return;
@@ -310,8 +342,28 @@ __global__ __launch_bounds__(BLOCK, OCC) void k_residue_gemm(const v4i *__restri
     const v4i *a_src = Ap + (i64)mod * units * mpad + (i64)tm * TM;
     const v4i *b_src = Bp + (i64)mod * units * npad + (i64)tn * TN;
 
-    // load j of the wavefront is chunk wave LOADS + j of a step: [A or B][unit][64 rows]
-    auto fetch = [&](int u0, int buf) {
+    // through registers
+    v4i ra[LA], rb[LB];
+    auto fetch = [&](int u0) {
+#pragma unroll
+        for (int i = 0; i < LA; ++i) {
+            const int c = tid + i * BLOCK;
+            ra[i] = a_src[(i64)(u0 + c / TM) * mpad + c % TM];
+        }
+#pragma unroll
+        for (int i = 0; i < LB; ++i) {
+            const int c = tid + i * BLOCK;
+            rb[i] = b_src[(i64)(u0 + c / TN) * npad + c % TN];
+        }
+    };
+    auto put = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < LA; ++i) As[buf][tid + i * BLOCK] = ra[i];
+#pragma unroll
+        for (int i = 0; i < LB; ++i) Bs[buf][tid + i * BLOCK] = rb[i];
+    };
+    // straight: load j of the wavefront is chunk wave LOADS + j of a step: [A or B][unit][64 rows]
+    auto fetch_straight = [&](int u0, int buf) {
 #pragma unroll
         for (int j = 0; j < LOADS; ++j) {
             const int c = wave * LOADS + j, ca = BKU * TM / 64, cb = c - ca;
@@ -329,11 +381,22 @@ __global__ __launch_bounds__(BLOCK, OCC) void k_residue_gemm(const v4i *__restri
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
     const int row0 = (wave >> 1) * (32 * WM) + (lane & 31), col0 = (wave & 1) * (32 * WN) + (lane & 31), half = lane >> 5;
 
-    fetch(0, 0);
+    if constexpr (STRAIGHT) {
+        fetch_straight(0, 0);
+    } else {
+        fetch(0);
+        put(0);
+        __syncthreads();
+    }
     int buf = 0;
     for (int u0 = 0; u0 < units; u0 += BKU, buf ^= 1) {
-        i16::wait_and_meet();
-        if (u0 + BKU < units) fetch(u0 + BKU, buf ^ 1);
+        const bool more = u0 + BKU < units;
+        if constexpr (STRAIGHT) {
+            i16::wait_and_meet();
+            if (more) fetch_straight(u0 + BKU, buf ^ 1);
+        } else {
+            if (more) fetch(u0 + BKU);
+        }
 #pragma unroll
         for (int s = 0; s < BKU / 2; ++s) {
             v4i a[WM], b[WN];
@@ -345,6 +408,10 @@ __global__ __launch_bounds__(BLOCK, OCC) void k_residue_gemm(const v4i *__restri
             for (int i = 0; i < WM; ++i)
 #pragma unroll
                 for (int j = 0; j < WN; ++j) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[i], b[j], acc[i][j], 0, 0, 0);
+        }
+        if constexpr (!STRAIGHT) {
+            if (more) put(buf ^ 1);
+            __syncthreads();
         }
     }
 
@@ -458,10 +525,10 @@ Plan make_plan(i64 m, i64 k, i64 n) {
     return L;
 }
 
-template <int WM, int WN, int OCC>
+template <int WM, int WN, int OCC, bool STRAIGHT>
 void launch_gemm(const v4i *A, const v4i *B, u32 *C, int units, i64 mpad, i64 npad, const ModConst &K, const u32 *done, hipStream_t s) {
     const int mt = (int)(mpad / (64 * WM)), nt = (int)(npad / (64 * WN));
-    hipLaunchKernelGGL((k_residue_gemm<WM, WN, STEP_UNITS, OCC>), dim3((unsigned)(mt * nt * NMOD)), dim3(BLOCK), 0, s, A, B, C, units, mpad, npad, mt, nt, K, done);
+    hipLaunchKernelGGL((k_residue_gemm<WM, WN, STEP_UNITS, OCC, STRAIGHT>), dim3((unsigned)(mt * nt * NMOD)), dim3(BLOCK), 0, s, A, B, C, units, mpad, npad, mt, nt, K, done);
 }
 
 }  // namespace
@@ -504,15 +571,19 @@ int rns_matmul(const uint64_t *A, const uint64_t *B, uint64_t *C, int64_t m, int
         const unsigned chunks = (unsigned)(D.units / ITEM_UNITS);
         D.b_items = D.B.groups * chunks;
         D.items = D.b_items + (with_a ? D.A.groups * chunks : 0);
+        D.wide = (unsigned)((nb + BLOCK - 1) / BLOCK);
+        D.b_slabs = D.wide * (unsigned)D.units;
+        D.slabs = D.b_slabs + D.items - D.b_items;
         return D;
     };
     i16::Job J = {};
     const bool small = i16::takes(m, k, n);
     if (small) {
         J = i16::make_job(C, m, k, n, ws);
-        const Cut D = cut(0, m, 0, k, 0, n, true);
-        J.n_flags = (int)(D.items < i16::MAX_CUT_BLOCKS ? D.items : i16::MAX_CUT_BLOCKS);
-        hipLaunchKernelGGL(k_cut, dim3((unsigned)J.n_flags), dim3(BLOCK), 0, s, D, J, m == L.mb && k <= L.kc && n == L.nb ? 1 : 0);
+        const Cut D = cut(0, m, 0, k, 0, n, true), first = cut(0, L.mb, 0, k < L.kc ? k : L.kc, 0, L.nb, true);
+        J.n_flags = (int)std::min(D.items, (unsigned)i16::MAX_CUT_BLOCKS);
+        const unsigned shares = first.slabs <= FEW_SLABS ? 3 : 1;
+        hipLaunchKernelGGL(k_cut, dim3(std::max((unsigned)J.n_flags, first.slabs * shares)), dim3(BLOCK), 0, s, D, first, J, shares);
         VI_LAUNCH_CHECK("k_cut");
     }
     for (i64 l0 = 0; l0 < k; l0 += L.kc) {
@@ -523,18 +594,21 @@ int rns_matmul(const uint64_t *A, const uint64_t *B, uint64_t *C, int64_t m, int
                 const i64 nb = n - j0 < L.nb ? n - j0 : L.nb, npad = round_up(nb, 64 * L.wn);
                 const Cut D = cut(i0, mb, l0, kc, j0, nb, j0 == 0);
                 if (small && l0 == 0 && i0 == 0 && j0 == 0) {
-                    const unsigned tiles = (unsigned)(J.tiles * J.slices), most = D.items < RESIDUE_BLOCKS ? D.items : RESIDUE_BLOCKS;
+                    const unsigned tiles = (unsigned)(J.tiles * J.slices), most = std::min(D.slabs, RESIDUE_BLOCKS);
                     const dim3 grid(tiles > most ? tiles : most);
                     if (m <= 64) hipLaunchKernelGGL((k_product<1, 2>), grid, dim3(BLOCK), 0, s, D, J);
                     else hipLaunchKernelGGL((k_product<2, 1>), grid, dim3(BLOCK), 0, s, D, J);
                     VI_LAUNCH_CHECK("k_product");
                 } else {
-                    hipLaunchKernelGGL(k_residues, dim3(D.items), dim3(BLOCK), 0, s, D, (const u32 *)J.done);
+                    hipLaunchKernelGGL(k_residues, dim3(D.slabs), dim3(BLOCK), 0, s, D, (const u32 *)J.done);
                     VI_LAUNCH_CHECK("k_residues");
                 }
-                if (L.wn == 4) launch_gemm<2, 4, 2>(Ap, Bp, Cp, D.units, mpad, npad, K, J.done, s);
-                else if (L.wn == 2) launch_gemm<2, 2, 3>(Ap, Bp, Cp, D.units, mpad, npad, K, J.done, s);
-                else launch_gemm<1, 1, 4>(Ap, Bp, Cp, D.units, mpad, npad, K, J.done, s);
+                const bool straight = kc < 4000 && (L.wm == 2 || mpad / 64 * (npad / 64) * NMOD > 2048);
+                if (L.wn == 4) launch_gemm<2, 4, 2, true>(Ap, Bp, Cp, D.units, mpad, npad, K, J.done, s);
+                else if (L.wn == 2 && straight) launch_gemm<2, 2, 3, true>(Ap, Bp, Cp, D.units, mpad, npad, K, J.done, s);
+                else if (L.wn == 2) launch_gemm<2, 2, 3, false>(Ap, Bp, Cp, D.units, mpad, npad, K, J.done, s);
+                else if (straight) launch_gemm<1, 1, 4, true>(Ap, Bp, Cp, D.units, mpad, npad, K, J.done, s);
+                else launch_gemm<1, 1, 4, false>(Ap, Bp, Cp, D.units, mpad, npad, K, J.done, s);
                 VI_LAUNCH_CHECK("k_residue_gemm");
                 hipLaunchKernelGGL(k_from_residues, dim3((unsigned)((nb + BLOCK - 1) / BLOCK), (unsigned)((mb + 3) / 4)), dim3(BLOCK), 0, s, (const u32 *)Cp,
                                    mpad / 4 * npad, npad, C + i0 * n + j0, (i64)n, mb, nb, l0 > 0 ? 1 : 0, J);
