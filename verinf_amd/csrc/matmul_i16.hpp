@@ -81,12 +81,15 @@ __device__ __forceinline__ int store_digits(const u64 (&w)[UNIT], v4i *at, i64 p
 // ---- the products -----------------------------------------------------------------------------------------------
 // 64 lanes' 16 bytes at base + 16 lane into 1 KiB of LDS, without a register in between; base and dst are the same for the wavefront.
 // As an instruction of its own the compiler does not wait for it before the next LDS read, as it does for its builtin: the waits are
-// wait_and_meet's.  (M0, which it takes its LDS address from, is not used by anything else here.)
+// wait_and_meet's.  M0, which it takes its LDS address from, has its value back afterwards: the compiler does not accept it in a list
+// of clobbered registers.
 __device__ __forceinline__ void fetch_to_lds(const v4i *base, v4i *dst, int lane) {
 #ifdef __HIP_DEVICE_COMPILE__
     const u32 at = __builtin_amdgcn_readfirstlane((u32)(uintptr_t)(__attribute__((address_space(3))) v4i *)dst);
     const u32 off = (u32)lane * 16;
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(at), "v"(off), "s"(base) : "memory");
+    u32 m0;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3\n\ts_mov_b32 m0, %0"
+                 : "=&s"(m0) : "s"(at), "v"(off), "s"(base) : "memory");
 #else
     dst[lane] = base[lane];
 #endif
