@@ -19,6 +19,7 @@
 
 #define __global__
 #define __device__
+#define __constant__ static
 #define __host__
 #define __forceinline__ inline
 #define __launch_bounds__(...)
@@ -115,7 +116,7 @@ inline void run_group(unsigned n) {
         for (unsigned w = 0; w < n; w += 64) {
             const unsigned end = w + 64 < n ? w + 64 : n;
             // votes stand in branches, so their lanes go before those that wait at a shuffle behind the branch
-            ran |= release(w, end, AT_WAVE) || release_some(w, end, AT_VOTE) || release_some(w, end, AT_LANES);
+            ran |= release(w, end, AT_WAVE) || release_some(w, end, AT_VOTE) || release_some(w, end, AT_LANES) || release_some(w, end, AT_WAVE);
         }
         ran |= release(0, n, AT_GROUP);
         if (!ran) {
@@ -190,6 +191,12 @@ inline uint64_t __shfl(uint64_t v, int lane, int) { return simt_lane(v, lane); }
 inline uint64_t __shfl_xor(uint64_t v, int mask, int) { return simt_lane(v, (int)(threadIdx.x & 63) ^ mask); }
 inline uint64_t __shfl_up(uint64_t v, unsigned d, int) { return simt_lane(v, (int)(threadIdx.x & 63) - (int)d); }
 inline uint64_t __shfl_down(uint64_t v, unsigned d, int) { return simt_lane(v, (int)(threadIdx.x & 63) + (int)d); }
+// the lanes of four, permuted: ctrl has two bits per lane (the row and bank masks leave no lane out)
+inline int __builtin_amdgcn_mov_dpp(int v, int ctrl, int, int, bool) {
+    const int lane = threadIdx.x & 63;
+    return (int)simt_lane((uint32_t)v, (lane & ~3) | ((ctrl >> (2 * (lane & 3))) & 3));
+}
+inline uint32_t __builtin_amdgcn_alignbit(uint32_t hi, uint32_t lo, uint32_t n) { return (uint32_t)(((uint64_t)hi << 32 | lo) >> (n & 31)); }
 inline void __threadfence_system() {}
 #define __builtin_amdgcn_fence(...) ((void)0)
 #define __builtin_amdgcn_wave_barrier() simt::wait_at(simt::AT_WAVE)
@@ -265,7 +272,7 @@ void simt_mfma_i32_32x32x32_i8(const A &a, const A &b, C &c) {
 
 typedef void *hipStream_t;
 typedef int hipError_t;
-enum { hipSuccess = 0, hipErrorNotReady = 1, hipFuncAttributeMaxDynamicSharedMemorySize = 0, hipMemcpyHostToDevice = 1 };
+enum { hipSuccess = 0, hipErrorNotReady = 1, hipFuncAttributeMaxDynamicSharedMemorySize = 0, hipMemcpyHostToDevice = 1, hipMemcpyDeviceToDevice = 3 };
 inline hipError_t hipGetLastError() { return hipSuccess; }
 inline const char *hipGetErrorString(hipError_t) { return ""; }
 inline hipError_t hipStreamQuery(hipStream_t) { return hipSuccess; }
@@ -285,3 +292,4 @@ inline hipError_t hipSetDevice(int) { return hipSuccess; }
 inline hipError_t hipMalloc(void **p, size_t n) { *p = malloc(n); return hipSuccess; }
 inline hipError_t hipFree(void *p) { free(p); return hipSuccess; }
 inline hipError_t hipMemcpy(void *to, const void *from, size_t n, int) { memcpy(to, from, n); return hipSuccess; }
+inline hipError_t hipMemcpyAsync(void *to, const void *from, size_t n, int, hipStream_t) { memcpy(to, from, n); return hipSuccess; }

@@ -339,6 +339,64 @@ def sumcheck(so):
     print("sumcheck", flush=True)
 
 
+def mle(so):
+    """eq vectors and evaluations, one table and several, full groups of four tables and remainders, on both sides of sixteen entries to
+    a thread; rows apart, results and scratch of exactly the stated sizes."""
+    L = ctypes.CDLL(so)
+    L.vi_mle_eval_workspace_bytes.restype, L.vi_mle_eval_workspace_bytes.argtypes = SZ, [I64]
+    L.vi_mle_eval.argtypes = [VP, I64, I64, VP, ctypes.c_int, VP, VP, SZ, VP]
+    L.vi_eq_vector.argtypes = [VP, ctypes.c_int, ctypes.c_int, VP, VP]
+    for n, k in ((0, 1), (1, 2), (2, 5), (3, 4), (4, 3), (7, 9), (12, 5), (17, 5), (18, 1), (18, 5)):
+        print("mle", n, k, flush=True)
+        size, pitch = 1 << n, (1 << n) + (3 if n < 10 else 0)
+        point = field(max(n, 1), n + 1)[:n]
+        tabs = field(k * pitch, n + k)[:(k - 1) * pitch + size]
+        for t in range(k):                                     # words at and above p in every table
+            tabs[t * pitch + (7 * t) % size] = np.uint64((1 << 64) - 1 - t)
+            tabs[t * pitch + (7 * t + 3) % size] = np.uint64(P)
+        out, ws = np.empty(k, dtype=np.uint64), scratch(L.vi_mle_eval_workspace_bytes(k))
+        assert L.vi_mle_eval(ptr(tabs), k, pitch, ptr(point), n, ptr(out), ptr(ws), len(ws), None) == 0
+        rows = [tabs[t * pitch:t * pitch + size] for t in range(k)]
+        assert out.tolist() == [O.mle_eval(r % np.uint64(P), [int(z) for z in point]) for r in rows], (n, k)
+        if n < 13:
+            eq = np.empty(size, dtype=np.uint64)
+            assert L.vi_eq_vector(ptr(point), n, 0, ptr(eq), None) == 0 and np.array_equal(eq, O.eq_vector([int(z) for z in point]))
+
+
+def blake3(so):
+    """Pads of one, four and eight words to a thread, rows that share a workgroup and rows over several; digests and trees, four lanes to a
+    compression and one."""
+    L = ctypes.CDLL(so)
+    L.vi_pad_rows.argtypes = [VP, I64, VP, I64, I64, I64, I64, VP, VP]
+    L.vi_hash_columns_workspace_bytes.restype, L.vi_hash_columns_workspace_bytes.argtypes = SZ, [I64, I64]
+    L.vi_hash_columns.argtypes = [VP, I64, I64, I64, VP, VP, SZ, VP]
+    L.vi_merkle_tree_nodes.restype, L.vi_merkle_tree_nodes.argtypes = I64, [I64]
+    L.vi_merkle_tree.argtypes = [VP, I64, VP, VP]
+    seed = np.arange(32, dtype=np.uint8) * np.uint8(7)
+    for rows, ell, width in ((1, 0, 1), (3, 5, 5), (7, 2, 19), (5, 100, 257), (300, 11, 17), (2, 8100, 9000),
+                             (1030, 500, 512), (3, 180000, 180001), (8, 65530, 65537), (8200, 1020, 1024)):
+        print("pad", rows, ell, width, flush=True)
+        pitch = ell + 1
+        msgs = field(rows * pitch, rows)[:(rows - 1) * pitch + ell]
+        out = np.empty((rows, width), dtype=np.uint64)
+        assert L.vi_pad_rows(ptr(seed), (1 << 32) - 2, ptr(msgs) if ell else None, rows, ell, pitch, width, ptr(out), None) == 0
+        for r in range(rows):
+            assert np.array_equal(out[r, :ell], msgs[r * pitch:r * pitch + ell]), (rows, ell, width, r)
+        if width > ell:
+            numbers = (np.arange(rows, dtype=np.uint64) + np.uint64((1 << 32) - 2)) % np.uint64(1 << 32)
+            want = O.row_prg(seed.tobytes(), 0, rows, width - ell, numbers)
+            assert np.array_equal(out[:, ell:], want), (rows, ell, width)
+    for m, n in ((0, 3), (1, 5), (12, 256), (128, 70), (129, 70), (300, 65), (700, 33)):
+        print("hash", m, n, flush=True)
+        mat, digests = field((max(m, 1), n), m), np.empty((n, 32), dtype=np.uint8)
+        ws = scratch(L.vi_hash_columns_workspace_bytes(m, n))
+        assert L.vi_hash_columns(ptr(mat), m, n, n, ptr(digests), ptr(ws), len(ws), None) == 0
+        assert np.array_equal(digests, O.hash_columns(mat[:m])), (m, n)
+        nodes = np.empty((L.vi_merkle_tree_nodes(n), 32), dtype=np.uint8)
+        assert L.vi_merkle_tree(ptr(digests), n, ptr(nodes), None) == 0
+        assert np.array_equal(nodes, np.concatenate(O.merkle_levels(digests)[1:])), n
+
+
 if __name__ == "__main__":
     globals()[sys.argv[1]](sys.argv[2])
     print("OK")

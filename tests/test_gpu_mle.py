@@ -61,6 +61,17 @@ def test_mle_eval_matches_oracle(gpu, n, k):
         assert gpu.mle_eval_t(to_dev(tabs[k - 1]), [(i >> (n - 1 - j)) & 1 for j in range(n)]) == int(tabs[k - 1, i]) % P
 
 
+@pytest.mark.parametrize("n,k", [(17, 4), (17, 5), (18, 2), (18, 4), (18, 5), (18, 39), (19, 3)])
+def test_mle_eval_of_several_long_tables(gpu, n, k):
+    """Eight and sixteen entries to a thread, groups of four tables and what is left of them, words at and above p in every table."""
+    rng = random.Random(n + k)
+    pt = [rng.randrange(P) for _ in range(n)]
+    tabs = rand_field((k, 1 << n), 60 + n)
+    for t in range(k):
+        tabs[t, t], tabs[t, -1 - t] = np.uint64((1 << 64) - 1 - t), np.uint64(P)
+    assert gpu.mle_eval_t(to_dev(tabs), pt) == [O.mle_eval(t % np.uint64(P), pt) for t in tabs]
+
+
 def test_mle_eval_is_what_the_folds_leave(gpu):
     n = 10
     rng = random.Random(5)
