@@ -234,6 +234,20 @@ def test_lde_of_rows_in_one_launch(cp, logK, log_rho):
         assert torch.equal(again, out[:, :N]) and torch.equal(own, co[:, :K])
 
 
+@pytest.mark.parametrize("logK,log_rho,least", [(10, 1, 2560), (10, 2, 257), (10, 3, 128), (11, 1, 1024), (11, 2, 128), (11, 3, 64), (12, 1, 256), (12, 2, 128)])
+def test_every_row_of_ragged_batches(cp, logK, log_rho, least):
+    """Rows are dealt to the XCDs by eights as far as there are eight: batches with each remainder, every row, and a row less than where
+    this launch begins, against small batches, which take other launches."""
+    K, N = 1 << logK, 1 << (logK + log_rho)
+    d = rand_field_dev((least + 24, K), logK + log_rho)
+    want = torch.cat([cp.coset_lde(d[r:r + 40].contiguous(), K, N, 7) for r in range(0, len(d), 40)])
+    for m in [least - 1] + [least + i for i in (0, 1, 2, 3, 5, 7, 8, 11, 14, 16, 23, 24)]:
+        assert torch.equal(cp.coset_lde(d[:m].contiguous(), K, N, 7), want[:m]), m
+    rows = [0, least // 2, least, least + 23]
+    host, got = (np.ascontiguousarray(np.stack([to_np(t[r]) for r in rows])) for t in (d, want))
+    assert np.array_equal(got, O.coset_lde_rows(host, K, N, 7))
+
+
 @pytest.mark.parametrize("logK,log_rho", [(12, 1), (12, 2), (12, 3), (14, 2), (14, 4), (16, 3)])
 def test_lde_with_cosets_dealt_to_several_workgroups(cp, logK, log_rho):
     """Tiles around the counts where the share of the cosets that a workgroup takes changes, and around full rounds of workgroups;

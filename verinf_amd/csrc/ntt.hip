@@ -171,7 +171,9 @@ __global__ __launch_bounds__(NTHREADS, 4) void k_ntt_row(const PassArgs P0, cons
 // passes write and read all cosets once more.  Bound by VALU issue: 130 instructions a word at K = 2^10, four cosets, 272 us for
 // 2^26 words of a floor of 255 (and 68 for the coefficients); whole extensions of 2^26 words, before and after: 2^10 -> 2^12 494 and 340 us, 2^11 -> 2^13
 // 562 and 355, 2^12 -> 2^14 485 and 424.  A workgroup has all cosets of a row where they fit its tile; else their workgroups
-// follow each other on one XCD, whose L2 puts the lines together (written 1.13 times at 2^12 -> 2^14).
+// follow each other on one XCD, whose L2 puts the lines together (written 1.13 times at 2^12 -> 2^14), as far as there are eight rows
+// for the eight of them (only where the whole grid was, batches of other sizes took up to half as long again: 1050 rows of 2^12 -> 2^14 179 us, 127
+// this way; 1050 of 2^11 -> 2^14 154 and 106).
 template <int A0, int LR>
 __global__ __launch_bounds__(NTHREADS, 4) void k_lde_row(const LdeRow A) {
     using S = LdeRowShape<A0, LR>;
@@ -179,7 +181,7 @@ __global__ __launch_bounds__(NTHREADS, 4) void k_lde_row(const LdeRow A) {
     __shared__ u64 twi[256];
     const int tid = threadIdx.x;
     u32 group = blockIdx.x / S::PARTS, part = blockIdx.x % S::PARTS;
-    if (S::PARTS > 1 && (gridDim.x & (8 * S::PARTS - 1)) == 0) {
+    if (S::PARTS > 1 && blockIdx.x < (gridDim.x & ~(8 * S::PARTS - 1))) {
         // the tiles of a row, whose words alternate in the codeword, one after the other on one XCD
         const u32 xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
         part = slot % S::PARTS;
