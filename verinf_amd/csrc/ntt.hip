@@ -654,7 +654,8 @@ bool small_ntt_passes_pay(i64 m, int logn, const Split &sp) {
 //
 // k_ntt_fast: 7.8 us a launch, one wavefront's chain, and 2.95 per million.  With K = L L the middle two are one launch whose
 // workgroups go through the cosets of their part one after the other: 21 + 7 per coset of a part for all three, and 1.84 per million
-// (memory hides behind the chain), 3.0 where tiles are dealt out in parts.
+// (memory hides behind the chain); 27 and 2.4 where tiles are dealt out in parts (5 rows of 2^16 -> 2^18 43.6 in these, 40.8 in those of
+// k_small_pass; 8 45 and 53; 40 of 2^14 -> 2^16 48.7 and 47.4, 48 48.9 and 51.9).
 //
 // Fitted to a sweep over K, 1 to 32 cosets and batches of 1 .. 2^24 points written (k_small_pass, k_ntt_fast: 2^14 -> 2^16 one row
 // 18, 40; 32 rows 44, 48; 64 rows 66, 59; 256 rows 209, 141).
@@ -667,7 +668,7 @@ double small_passes_us(const Split &sp, double million) {
 double fast_passes_us(const Split &sp, int log_rho, double tiles, double million) {
     if (sp.p == 2 && sp.a[0] == sp.a[1] && sp.a[0] >= 6) {
         const int log_parts = tiles < MID_RESIDENT ? mid_log_parts((u32)tiles, log_rho) : 0;
-        return 21 + 7.0 * (double)((1 << log_rho) >> log_parts) + 2 * (log_parts ? 3.0 : 1.84) * million;
+        return (log_parts ? 27 : 21) + 7.0 * (double)((1 << log_rho) >> log_parts) + 2 * (log_parts ? 2.4 : 1.84) * million;
     }
     return sp.p * (2 * 7.8 + 2.95 * million);
 }
@@ -679,13 +680,15 @@ bool small_lde_passes_pay(i64 m, int logK, int logN, const Split &sp) {
 }
 
 // Extensions of K = 2^10 .. 2^12 by two, four or eight as one launch to the coefficients (k_ntt_row) and one to the codewords
-// (k_lde_row), from 2^20 .. 2^22 points written, where the shorter chains of ntt_small.hpp meet it.  us, the better of the other
-// routes and this one: 2^20 points 2^10 -> 2^12 22 and 23, -> 2^13 26 and 23, -> 2^11 18 and 24; 2^21 27 and 27, 37 and 27, 27 and 29;
-// 2^12 -> 2^14 28 and 29, with 2^21 40 and 33; 2^24 points 2^10 -> 2^12 137 and 88, 2^11 -> 2^13 153 and 99, 2^12 -> 2^14 136 and 118.
+// (k_lde_row), from 2^20 .. 5 2^20 points written, where the shorter chains of ntt_small.hpp meet it.  us, the better of the other
+// routes and this one: 2^20 points 2^10 -> 2^12 21 and 22 (a row more 25 and 24), -> 2^13 25 and 23, 2^11 -> 2^13 27 and 25; 2^21 points 2^12 ->
+// 2^14 41 and 32; 2^22 points 2^10 -> 2^11 43 and 44, 5 2^20 51 and 45, 2^11 -> 2^12 50 and 45; 2^24 points 2^10 -> 2^12 135 and 88, 2^11 -> 2^13
+// 154 and 98, 2^12 -> 2^14 133 and 118.
 bool row_lde_pays(i64 m, int logK, int logN) {
     if (!row_launch_on() || !coset_rows_ok(logK, logN)) return false;
-    const int log_least = logK == TILE_LOG ? 21 : (logN - logK >= 2 ? 20 : 22);
-    return m >= (((i64)1 << log_least) >> logN);
+    const int log_rho = logN - logK;
+    const i64 least = logK == TILE_LOG ? (i64)2 << 20 : log_rho >= 2 ? (i64)1 << 20 : logK == 10 ? (i64)5 << 20 : (i64)4 << 20;
+    return m >= (least >> logN) + (logK == 10 && log_rho == 2 ? 1 : 0);
 }
 
 // Which launches an extension takes
