@@ -723,6 +723,26 @@ def test_single_tables_around_what_a_descriptor_holds(mods, singles, v):
     _check(gpu, [rand_field(1 << v, 5000 + t) for t in range(5 + singles)], terms, 90 + v, True)
 
 
+@pytest.mark.parametrize("products,singles,v", [(0, 6, 19), (0, 7, 19), (1, 63, 19), (1, 64, 19), (0, 7, 9), (0, 8, 9), (0, 7, 10), (0, 8, 10), (0, 20, 12),
+                                                (0, 21, 12), (0, 8, 13)])
+@pytest.mark.parametrize("constant", [False, True])
+def test_single_tables_in_passes_and_rewritten(mods, products, singles, v, constant):
+    """Both sides of the lines between passes over all tables and a first round that leaves one table of the single ones, and a constant,
+    which moves them."""
+    gpu, _ = mods
+    n = 1 + 2 * products + singles
+    terms = [(k + 2, [0, 1 + 2 * k, 2 + 2 * k]) for k in range(products)] + [(P - 3 - k, [1 + 2 * products + k, 0]) for k in range(singles)]
+    if constant:
+        terms.append((5, [0]))
+    tabs = [rand_field(1 << v, 7000 + t) for t in range(n)]
+    coins = _coins(v, 71)[0]
+    dev = [to_dev(t) for t in tabs]
+    print(products, singles, v, constant, flush=True)
+    claim, polys, _, _ = gpu.prove_terms_gpu([(c, [dev[i] for i in fs]) for c, fs in terms], lambda i: coins[i], P)
+    want_claim, want_samples, _ = O.sumcheck_prove(tabs, terms, coins)
+    assert claim == want_claim and [[y for _, y in s] for s in polys] == want_samples
+
+
 @pytest.mark.parametrize("coins", [[0, 5], [2, 7], [9, 2, 3], [9, 8, 0], [1, 1, 1], [P - 1, P - 2, 1], [3, 4, 5, 0, 2, 1, 0]])
 @pytest.mark.parametrize("terms,v", [([(5, [0])], 14), ([(1, [0, 1])], 13), ([(7, [0, 1])], 16), ([(1, [0, 1, 2])], 13), ([(1, [0, 1, 2])], 16),
                                      ([(3, [0, 1, 2, 3])], 13), ([(3, [0, 1, 2]), (P - 3, [0, 3])], 13), ([(3, [0, 1]), (4, [0, 2])], 10),

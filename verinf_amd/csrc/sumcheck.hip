@@ -1564,6 +1564,24 @@ int prove_coins_reduced(const char *who, const uint64_t *const *tables, uint64_t
                             (int)R.coeffs.size(), deg, challenges + 1, samples + NSAMP, part, s, false);
 }
 
+// Whether a sum under a common factor is faster rewritten than in passes of three rounds (prove_sum).  Rewritten, round 0 reads the single
+// tables once, as two streams each (5.9 TB/s), and leaves one; up to one product beside them has kernels of its own, others
+// take a launch or two per round.  Passes read eight streams a table (4.4 TB/s) and the common factor in every row of workgroups, in fewer launches:
+// the longer the tables and the more of them are single ones, the later they pay.  dropped: tables that the rewriting drops; kept: that it
+// keeps.  us in passes and rewritten: no product, 30 single tables of 2^19 86 and 76, of 2^22 305 and 276, 128 of 2^20 304 and 253, 9 of
+// 2^24 488 and 403 (8: 380 and 374); one product, 40 of 2^20 172 and 180, 64 212 and 194, 100 of 2^22 917 and 783; two products, 64 of 2^23
+// 1230 and 1280, 128 of 2^23 2082 and 1864; twenty products of eight tables, 100 of 2^22 1600 and 1530.  In between the line is within 5 %.
+// Short tables without a product, for which the last rounds are k_tail: 512 entries, 3 single tables 26.4 and 23.4 (9 26.8 and 28.0), 4096 entries,
+// 9 37.5 and 35.2, 20 37.6 and 36.6 (5 36.3 and 36.5, 24 37.6 and 40.2).
+bool rewriting_pays(int dropped, int kept, int products, i64 size) {
+    if (products == 0 && size <= 4096) return size == SUM_TAIL ? dropped <= 7 : size > SUM_TAIL && dropped >= 8 && dropped <= 20;
+    if (size < FUSE_MIN_PAIRS * 2 || products > 20) return false;                     // round 0 is more than one launch; too many to come
+    const i64 words = dropped * size;
+    if (products == 0) return size == FUSE_MIN_PAIRS * 2 ? dropped >= 7 : dropped >= 9 && words >= (i64)28 << 20;
+    if (products == 1) return dropped >= 9 && words >= (size == FUSE_MIN_PAIRS * 2 ? (i64)32 << 20 : (i64)64 << 20);
+    return dropped >= 64 && words >= (products > kept ? (i64)400 << 20 : (i64)640 << 20);
+}
+
 // all rounds of the sum over tables of `size` words; samples: log2(size) rows of NSAMP words
 int prove_coins_impl(const char *who, const uint64_t *const *tables, uint64_t *const *work, int n_tables, int64_t size,
                      const int *term_off, const int *factor_idx, const uint64_t *coeffs, int n_terms, int deg,
@@ -1589,20 +1607,20 @@ int prove_coins_impl(const char *who, const uint64_t *const *tables, uint64_t *c
     C.n_prior = v;
     C.deg = deg;
 
-    // products of two tables and single tables under a common factor: three rounds per pass (the hadamard gate batch of four tables
-    // has kernels of its own).  Not where the tables are the work buffers, as in the rewritten problem of prove_coins_reduced: a row of
-    // workgroups would write over entries of the common factor that others still have to read
     if (may_reduce) {
+        // many terms that are a single table under the common factor: from round 1 on they are one table (needs a round
+        // to fold into, so at least two rounds)
+        LinearReduction R;
+        const bool rewritable = v >= 2 && reduce_linear_terms(n_tables, term_off, factor_idx, coeffs, n_terms, deg, R);
+        // products of two tables and single tables under a common factor: three rounds per pass (the hadamard gate batch of four tables
+        // has kernels of its own).  Not where the tables are the work buffers, as in the rewritten problem of prove_coins_reduced: a row
+        // of workgroups would write over entries of the common factor that others still have to read
         SumShape S;
         if (sum_shape(n_tables, term_off, factor_idx, coeffs, n_terms, S) &&
-            !(n_tables == 4 && S.products.size() == 1 && S.singles.size() == 1 && S.c0 == 0))
+            !(n_tables == 4 && S.products.size() == 1 && S.singles.size() == 1 && S.c0 == 0) &&
+            !(rewritable && rewriting_pays(n_tables - (int)R.keep.size(), (int)R.keep.size(), (int)S.products.size() + (S.c0 ? 2 : 0), size)))
             return prove_sum(S, tables, work, size, C, part, samples, s);
-    }
-    // many terms that are a single table under the common factor: from round 1 on they are one table (needs a round
-    // to fold into, so at least two rounds)
-    if (may_reduce && v >= 2) {
-        LinearReduction R;
-        if (reduce_linear_terms(n_tables, term_off, factor_idx, coeffs, n_terms, deg, R))
+        if (rewritable)
             return prove_coins_reduced(who, tables, work, n_tables, size, term_off, factor_idx, coeffs, n_terms, deg, challenges,
                                        samples, part, s, R);
     }
