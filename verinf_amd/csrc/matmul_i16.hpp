@@ -8,9 +8,10 @@
 //              did not fit
 //   product()  all four byte products of a tile at once, put together as 64-bit integers and taken mod p
 //
-// 1000 x 4096 x 4096: 465 us through residues, 118 here: k_cut 37 (0.21 GB read and written, the rate of a copy), the product 71, two
-// launches that find nothing left to do 4.5 each.  The product runs at 1.9 POP/s, 2.3 without its first loads and last stores; a loop
-// of nothing but these matrix instructions on random bytes holds 2.9 to 3.5 POP/s on this card (power), of a nominal 5.  Deeper prefetch (3
+// 1000 x 4096 x 4096: 423 us through residues, 111 to 114 here: k_cut 37 (0.21 GB read and written, the rate of a copy), the product 71,
+// two launches that find nothing left to do 4.5 each.  The product runs at 1.9 POP/s, 2.3 without its first loads and last stores, with the
+// matrix cores busy 44 % of the cycles, the LDS 17 %; a loop of nothing but these matrix instructions on random bytes holds 2.9 to 3.5
+// POP/s on this card (power), of a nominal 5.  Deeper prefetch (3
 // or 4 buffers), wavefronts of 64 x 64 (half the LDS reads) and operands read a quarter step ahead made no difference.  Other sizes,
 // before -> after: 2048 x 4096 x 2048 450 -> 108 us, 64 x 4096 x 4096 152 -> 58, 300 x 9000 x 500 117 -> 56, 100 x 760 x 1070 28.5 -> 25.5.
 //
@@ -116,7 +117,7 @@ struct Job {
 // A tile of 64 MT x 64 NT of C by four wavefronts in a square, MT x NT matrix instructions each: the inner dimension is cut into slices where a product has few tiles.  A step is four units (64 inner indices) of both digits of
 // both operands, loaded straight into the one LDS buffer while the other is multiplied.  Three workgroups to a CU cover each other's
 // barriers, first loads and last stores (128 x 128 with eight wavefronts and one workgroup to a CU: 2048 x 700 x 11000 108 us, 90 this
-// way).
+// way).  As k_product<1, 2> (matmul_rns.hip) 10 of its 168 registers go to scratch.
 template <int MT, int NT>
 struct Lds {
     v4i buf[2][2 * STEP * 64 * (MT + NT)];

@@ -7,15 +7,15 @@
 // is a signed byte, so each residue is ONE int8 matrix product on v_mfma_i32_32x32x32_i8: 18 byte multiply-adds per
 // field multiply-add, where splitting both operands into bytes would take 64.
 //
-// What bounds it at 1000 x 4096 x 4096 (8240 us on the VALU, 440 here): the int8 products 334 us, 1.8 POP/s of the 2.9 to 3.5 that a
-// loop of nothing else holds on random bytes -- the matrix cores are busy 43 % of the cycles and the LDS a third, neither at its limit: with
-// two wavefronts to a SIMD (registers) the barrier and the operand reads of a step are not covered by the other one's products; the
-// residues 104 us, 0.44 GB at the rate of a copy; the reconstruction 21 us.
+// What bounds it at 1000 x 4096 x 4096 (8240 us on the VALU, 423 here): the int8 products 308 us, 2.0 POP/s of the 2.9 to 3.5 that a
+// loop of nothing else holds on random bytes -- the matrix cores are busy 53 % of the cycles and the LDS 20 %, neither at its limit: with
+// 2.5 wavefronts to a SIMD (registers) the barrier and the operand reads of a step are not all covered by the others' products; the
+// residues 113 us, 0.54 GB read and written and 77 % of the VALU issue rate; the reconstruction 23 us.
 //
 // Operands that are 16-bit signed numbers take fewer byte products (matmul_i16.hpp): k_cut looks at them, k_product does their
 // product, and the kernels behind it leave at once when it is done.
 //
-//   k_cut, k_residues words -> 18 planes of signed bytes
+//   k_cut, k_product, k_residues words -> 18 planes of signed bytes
 //   k_residue_gemm    per plane an int8 product; the 32-bit sums are reduced mod m_i to one byte
 //   k_from_residues   18 bytes -> the integer mod p
 //
