@@ -43,8 +43,13 @@ constexpr u64 EPS = 0xFFFFFFFFull;   // 2^32 - 1 = 2^64 mod p
 #if defined(__HIP_DEVICE_COMPILE__)
 // Hand-scheduled gfx950 sequences.  Written from 64-bit C++ the compiler spends a 64-bit compare (two issue
 // slots) and two selects on every carry test and builds register pairs with moves: 29 VALU instructions (42
-// issue slots) for a product, 7 (11) for a modular sum.  On 32-bit halves with explicit carries the same
-// functions are 19 (24), 6 and 5.  On this chip a VALU instruction that reads a carry or mask needs two
+// issue slots) for a product, 7 (11) for a modular sum.  Here a product is 15, a sum 5, a difference 4 and a butterfly 9.
+// Corrections by 2^32 - 1 are multiply-adds, which take the same 4.2 cycles as any instruction with a carry: + (2^32 - 1) with its
+// carry is 1 * (2^32 - 1) + x, and - (2^32 - 1) behind a borrow is 3 * (-0x55555555) + x with a factor of 3 or 0.  With 32-bit
+// additions and masks in their places (18, 6, 5 and 11 instructions; cycles per operation and SIMD at eight wavefronts) a product took 74,
+// now 66; a butterfly 44.5, now 36; a 16-point transform 2049, now 1782.  1024 rows 2^16 -> 2^18 2124 -> 2040 us (the clock gives
+// some of it back: 2.0 to 2.1 GHz under these loads), proofs over three tables of 2^26 567 -> 559.
+// On this chip a VALU instruction that reads a carry or mask needs two
 // wait states after the VALU instruction that wrote it; inside an asm block the assembler does not add
 // them, so every such pair below is separated by two instructions or an s_nop.  s_or_b64 also writes SCC, which the
 // compiler may be holding a loop condition in: the blocks that use it say so in their clobber lists.  A carry that leaves a
@@ -54,41 +59,52 @@ namespace dev {
 
 __device__ __forceinline__ u64 pack(u32 lo, u32 hi) { return ((u64)hi << 32) | lo; }
 
+// mask ? a : b.  The long encoding, with the mask in a pair of scalar registers: with the mask in VCC a select is the short one,
+// which takes 2.8 cycles where an instruction with a carry stands before it but was seen at 23 behind a multiply-add
+__device__ __forceinline__ u64 select(u64 mask, u64 a, u64 b) {
+    u32 r0 = (u32)a, r1 = (u32)(a >> 32);
+    asm("v_cndmask_b32_e64 %[r0], %[b0], %[r0], %[m]\n\t"
+        "v_cndmask_b32_e64 %[r1], %[b1], %[r1], %[m]"
+        : [r0] "+v"(r0), [r1] "+v"(r1)
+        : [b0] "v"((u32)b), [b1] "v"((u32)(b >> 32)), [m] "s"(mask));
+    return pack(r0, r1);
+}
+
+// d - (2^32 - 1) where a block before has put 3 in m, d itself where it has put 0: 2^32 - 1 = 3 * 0x55555555, so that both
+// factors are signed 32-bit words and the first one is an inline constant of a select on the borrow
+constexpr int BORROWED = 3;
+__device__ __forceinline__ u64 minus_eps(u64 d, u32 m) {
+    u64 r;
+    asm("v_mad_i64_i32 %[r], vcc, %[m], %[k], %[d]" : [r] "=v"(r) : [m] "v"(m), [k] "s"(-0x55555555), [d] "v"(d) : "vcc");
+    return r;
+}
+
 // w, plus 2^64 when the carry `cin` is set, lies in [0, 2p): subtract p when it is >= p.
 // r = w + (2^32 - 1) mod 2^64 is that difference, and it is the answer exactly when one of the two additions wrapped.
-__device__ __forceinline__ u64 canon_tail(u32 w0, u32 w1, u64 cin) {
-    u32 r0, r1;
-    asm("v_add_co_u32 %[r0], vcc, -1, %[w0]\n\t"
-        "s_nop 1\n\t"
-        "v_addc_co_u32 %[r1], vcc, 0, %[w1], vcc\n\t"
-        "s_or_b64 vcc, vcc, %[cin]\n\t"
-        "v_cndmask_b32 %[r0], %[w0], %[r0], vcc\n\t"
-        "v_cndmask_b32 %[r1], %[w1], %[r1], vcc"
-        : [r0] "=&v"(r0), [r1] "=&v"(r1)
-        : [w0] "v"(w0), [w1] "v"(w1), [cin] "s"(cin)
-        : "vcc", "scc");
-    return pack(r0, r1);
+__device__ __forceinline__ u64 canon_tail(u64 w, u64 cin) {
+    u64 st, r;
+    asm("v_mad_u64_u32 %[r], %[st], 1, -1, %[w]\n\t"
+        "s_or_b64 %[st], %[st], %[cin]"
+        : [r] "=v"(r), [st] "=&s"(st)
+        : [w] "v"(w), [cin] "s"(cin)
+        : "scc");
+    return select(st, r, w);
 }
 
 __device__ __forceinline__ u64 addc(u64 a, u64 b) {
     u32 a0 = (u32)a, a1 = (u32)(a >> 32), b0 = (u32)b, b1 = (u32)(b >> 32);
-    u32 s0, s1, r0, r1;
+    u32 s0, s1;
     u64 st;
     asm("v_add_co_u32 %[s0], vcc, %[a0], %[b0]\n\t"
-        "v_add_co_u32 %[r0], %[st], -1, %[s0]\n\t"
-        "s_nop 0\n\t"
-        "v_addc_co_u32 %[s1], vcc, %[a1], %[b1], vcc\n\t"
-        "v_addc_co_u32 %[r1], %[st], 0, %[s1], %[st]\n\t"
-        "s_or_b64 vcc, vcc, %[st]\n\t"
-        "v_cndmask_b32 %[r0], %[s0], %[r0], vcc\n\t"
-        "v_cndmask_b32 %[r1], %[s1], %[r1], vcc"
-        : [s0] "=&v"(s0), [s1] "=&v"(s1), [r0] "=&v"(r0), [r1] "=&v"(r1), [st] "=&s"(st)
+        "s_nop 1\n\t"
+        "v_addc_co_u32 %[s1], %[st], %[a1], %[b1], vcc"
+        : [s0] "=&v"(s0), [s1] "=v"(s1), [st] "=s"(st)
         : [a0] "v"(a0), [a1] "v"(a1), [b0] "v"(b0), [b1] "v"(b1)
-        : "vcc", "scc");
-    return pack(r0, r1);
+        : "vcc");
+    return canon_tail(pack(s0, s1), st);
 }
 
-// a - b, minus 2^32 - 1 more when it borrowed (the mask -borrow is that constant)
+// a - b, minus 2^32 - 1 more when it borrowed
 __device__ __forceinline__ u64 sub(u64 a, u64 b) {
     u32 a0 = (u32)a, a1 = (u32)(a >> 32), b0 = (u32)b, b1 = (u32)(b >> 32);
     u32 d0, d1, m;
@@ -96,76 +112,72 @@ __device__ __forceinline__ u64 sub(u64 a, u64 b) {
         "s_nop 1\n\t"
         "v_subb_co_u32 %[d1], vcc, %[a1], %[b1], vcc\n\t"
         "s_nop 1\n\t"
-        "v_subb_co_u32 %[m], vcc, %[d0], %[d0], vcc\n\t"
-        "v_sub_co_u32 %[d0], vcc, %[d0], %[m]\n\t"
-        "s_nop 1\n\t"
-        "v_subbrev_co_u32 %[d1], vcc, 0, %[d1], vcc"
-        : [d0] "=&v"(d0), [d1] "=&v"(d1), [m] "=&v"(m)
-        : [a0] "v"(a0), [a1] "v"(a1), [b0] "v"(b0), [b1] "v"(b1)
+        "v_cndmask_b32_e64 %[m], 0, %[k], vcc"
+        : [d0] "=&v"(d0), [d1] "=&v"(d1), [m] "=v"(m)
+        : [a0] "v"(a0), [a1] "v"(a1), [b0] "v"(b0), [b1] "v"(b1), [k] "n"(BORROWED)
         : "vcc");
-    return pack(d0, d1);
+    return minus_eps(pack(d0, d1), m);
 }
 
-// (u + v, u - v) of canonical u, v in one block: the two carry chains are interleaved so that each carry is read
-// three instructions after it was written and no wait has to be inserted
+// (u + v, u - v) of canonical u, v: the two carry chains are interleaved, and the first select waits behind the sum's
+// correction, so that no wait has to be inserted but one
 __device__ __forceinline__ void bfly(u64 u, u64 v, u64 &sum, u64 &dif) {
     u32 u0 = (u32)u, u1 = (u32)(u >> 32), v0 = (u32)v, v1 = (u32)(v >> 32);
-    u32 s0, s1, r0, r1, d0, d1, m;
-    u64 st, sb;
+    u32 s0, s1, d0, d1, m;
+    u64 st, sb, r, d;
     asm("v_add_co_u32 %[s0], vcc, %[u0], %[v0]\n\t"
         "v_sub_co_u32 %[d0], %[sb], %[u0], %[v0]\n\t"
-        "v_add_co_u32 %[r0], %[st], -1, %[s0]\n\t"
-        "v_addc_co_u32 %[s1], vcc, %[u1], %[v1], vcc\n\t"
-        "v_subb_co_u32 %[d1], %[sb], %[u1], %[v1], %[sb]\n\t"
-        "v_addc_co_u32 %[r1], %[st], 0, %[s1], %[st]\n\t"
-        "s_or_b64 vcc, vcc, %[st]\n\t"
-        "v_subb_co_u32 %[m], %[sb], %[d0], %[d0], %[sb]\n\t"
-        "v_sub_co_u32 %[d0], %[sb], %[d0], %[m]\n\t"
-        "v_cndmask_b32 %[r0], %[s0], %[r0], vcc\n\t"
-        "v_cndmask_b32 %[r1], %[s1], %[r1], vcc\n\t"
-        "v_subbrev_co_u32 %[d1], %[sb], 0, %[d1], %[sb]"
-        : [s0] "=&v"(s0), [s1] "=&v"(s1), [r0] "=&v"(r0), [r1] "=&v"(r1), [d0] "=&v"(d0), [d1] "=&v"(d1), [m] "=&v"(m),
-          [st] "=&s"(st), [sb] "=&s"(sb)
+        "s_nop 0\n\t"
+        "v_addc_co_u32 %[s1], %[st], %[u1], %[v1], vcc\n\t"
+        "v_subb_co_u32 %[d1], %[sb], %[u1], %[v1], %[sb]"
+        : [s0] "=&v"(s0), [s1] "=&v"(s1), [d0] "=&v"(d0), [d1] "=&v"(d1), [st] "=&s"(st), [sb] "=&s"(sb)
         : [u0] "v"(u0), [u1] "v"(u1), [v0] "v"(v0), [v1] "v"(v1)
+        : "vcc");
+    asm("v_mad_u64_u32 %[r], vcc, 1, -1, %[s]\n\t"
+        "s_or_b64 %[st], %[st], vcc\n\t"
+        "v_cndmask_b32_e64 %[m], 0, %[n], %[sb]\n\t"
+        "v_mad_i64_i32 %[d], vcc, %[m], %[k], %[dd]"
+        : [r] "=&v"(r), [m] "=&v"(m), [st] "+s"(st), [d] "=v"(d)
+        : [s] "v"(pack(s0, s1)), [dd] "v"(pack(d0, d1)), [sb] "s"(sb), [n] "n"(BORROWED), [k] "s"(-0x55555555)
         : "vcc", "scc");
-    sum = pack(r0, r1);
-    dif = pack(d0, d1);
+    sum = select(st, r, pack(s0, s1));
+    dif = d;
 }
 
 __device__ __forceinline__ u64 canon(u64 x) {
-    u32 x0 = (u32)x, x1 = (u32)(x >> 32), r0, r1;
-    asm("v_add_co_u32 %[r0], vcc, -1, %[x0]\n\t"
-        "s_nop 1\n\t"
-        "v_addc_co_u32 %[r1], vcc, 0, %[x1], vcc\n\t"
-        "s_nop 1\n\t"
-        "v_cndmask_b32 %[r0], %[x0], %[r0], vcc\n\t"
-        "v_cndmask_b32 %[r1], %[x1], %[r1], vcc"
-        : [r0] "=&v"(r0), [r1] "=&v"(r1)
-        : [x0] "v"(x0), [x1] "v"(x1)
-        : "vcc");
-    return pack(r0, r1);
+    u64 st, r;
+    asm("v_mad_u64_u32 %[r], %[st], 1, -1, %[x]\n\t"
+        "s_nop 1"
+        : [r] "=v"(r), [st] "=s"(st)
+        : [x] "v"(x));
+    return select(st, r, x);
 }
 
-// (hi:lo) given as four words l0 l1 hl hh, minus the borrow-in `bin` -> [0, p):  lo - hh - bin + hl (2^32 - 1).
-// hh + bin must be below 2^32.
-__device__ __forceinline__ u64 reduce_words(u32 l0, u32 l1, u32 hl, u32 hh, u64 bin) {
+// (hi:lo) given as four words l0 l1 hl hh, minus the borrow-in `bin`: lo - hh - bin + hl (2^32 - 1) as a word w and a carry st of
+// 2^64, together in [0, 2p).  hh + bin must be below 2^32.
+__device__ __forceinline__ u64 reduce_words_open(u32 l0, u32 l1, u32 hl, u32 hh, u64 bin, u64 *st) {
     u32 x0, x1, m;
     asm("v_subb_co_u32 %[x0], vcc, %[l0], %[hh], %[bin]\n\t"
         "s_nop 1\n\t"
         "v_subbrev_co_u32 %[x1], vcc, 0, %[l1], vcc\n\t"
         "s_nop 1\n\t"
-        "v_subb_co_u32 %[m], vcc, %[x0], %[x0], vcc\n\t"
-        "v_sub_co_u32 %[x0], vcc, %[x0], %[m]\n\t"
-        "s_nop 1\n\t"
-        "v_subbrev_co_u32 %[x1], vcc, 0, %[x1], vcc"
-        : [x0] "=&v"(x0), [x1] "=&v"(x1), [m] "=&v"(m)
-        : [l0] "v"(l0), [l1] "v"(l1), [hh] "v"(hh), [bin] "s"(bin)
+        "v_cndmask_b32_e64 %[m], 0, %[k], vcc"
+        : [x0] "=&v"(x0), [x1] "=&v"(x1), [m] "=v"(m)
+        : [l0] "v"(l0), [l1] "v"(l1), [hh] "v"(hh), [bin] "s"(bin), [k] "n"(BORROWED)
         : "vcc");
-    u64 w, st;
+    u64 w;
+    const u64 x = minus_eps(pack(x0, x1), m);
     asm("v_mad_u64_u32 %[w], %[st], %[hl], -1, %[x]"
-        : [w] "=&v"(w), [st] "=&s"(st)
-        : [hl] "v"(hl), [x] "v"(pack(x0, x1)));
-    return canon_tail((u32)w, (u32)(w >> 32), st);
+        : [w] "=v"(w), [st] "=&s"(*st)
+        : [hl] "v"(hl), [x] "v"(x));
+    return w;
+}
+
+// the same -> [0, p)
+__device__ __forceinline__ u64 reduce_words(u32 l0, u32 l1, u32 hl, u32 hh, u64 bin) {
+    u64 st;
+    const u64 w = reduce_words_open(l0, l1, hl, hh, bin, &st);
+    return canon_tail(w, st);
 }
 
 __device__ __forceinline__ u64 mul(u64 a, u64 b) {
@@ -193,35 +205,19 @@ __device__ __forceinline__ u64 mul(u64 a, u64 b) {
 }
 
 // the reduction of reduce_words() without its last step: a 64-bit word congruent to the value, not necessarily
-// below p (three instructions instead of six after the multiply-add); good as an operand of a further product
+// below p (two instructions instead of three after the multiply-add); good as an operand of a further product
 __device__ __forceinline__ u64 reduce_words_lazy(u32 l0, u32 l1, u32 hl, u32 hh, u64 bin) {
-    u32 x0, x1, m;
-    asm("v_subb_co_u32 %[x0], vcc, %[l0], %[hh], %[bin]\n\t"
-        "s_nop 1\n\t"
-        "v_subbrev_co_u32 %[x1], vcc, 0, %[l1], vcc\n\t"
-        "s_nop 1\n\t"
-        "v_subb_co_u32 %[m], vcc, %[x0], %[x0], vcc\n\t"
-        "v_sub_co_u32 %[x0], vcc, %[x0], %[m]\n\t"
-        "s_nop 1\n\t"
-        "v_subbrev_co_u32 %[x1], vcc, 0, %[x1], vcc"
-        : [x0] "=&v"(x0), [x1] "=&v"(x1), [m] "=&v"(m)
-        : [l0] "v"(l0), [l1] "v"(l1), [hh] "v"(hh), [bin] "s"(bin)
-        : "vcc");
-    u64 w, st;
-    asm("v_mad_u64_u32 %[w], %[st], %[hl], -1, %[x]"
-        : [w] "=&v"(w), [st] "=&s"(st)
-        : [hl] "v"(hl), [x] "v"(pack(x0, x1)));
+    u64 st, r;
+    const u64 w = reduce_words_open(l0, l1, hl, hh, bin, &st);
     // the sum wrapped past 2^64 (st): add 2^64 mod p = 2^32 - 1; it cannot wrap again (w <= 2^64 - 2^33 then)
-    u32 w0 = (u32)w, w1 = (u32)(w >> 32), e;
+    u32 e;
     asm("s_nop 1\n\t"
-        "v_cndmask_b32 %[e], 0, -1, %[st]\n\t"
-        "v_add_co_u32 %[w0], vcc, %[w0], %[e]\n\t"
-        "s_nop 1\n\t"
-        "v_addc_co_u32 %[w1], vcc, 0, %[w1], vcc"
-        : [e] "=&v"(e), [w0] "+v"(w0), [w1] "+v"(w1)
-        : [st] "s"(st)
+        "v_cndmask_b32_e64 %[e], 0, 1, %[st]\n\t"
+        "v_mad_u64_u32 %[r], vcc, %[e], -1, %[w]"
+        : [e] "=&v"(e), [r] "=&v"(r)
+        : [w] "v"(w), [st] "s"(st)
         : "vcc");
-    return pack(w0, w1);
+    return r;
 }
 
 // the four partial products of a * b (+ c, a 64-bit addend of the lowest one) as the words l0 l1 hl hh of the
@@ -271,7 +267,7 @@ __device__ __forceinline__ void mul_words(u64 a, u64 b, u64 c, u32 &l0, u32 &l1,
     l1 = w1;
 }
 
-// a * b + c -> [0, p): the addend rides on the first partial product (20 instructions against 24 for mul + add)
+// a * b + c -> [0, p): the addend rides on the first partial product (17 instructions against 20 for mul + add)
 __device__ __forceinline__ u64 mul_add(u64 a, u64 b, u64 c) {
     u32 l0, l1, hl, hh;
     u64 st;
@@ -296,7 +292,7 @@ __device__ __forceinline__ u64 mul_lazy(u64 a, u64 b) {
 }
 
 // five words w[0..4] (an integer below 2^160) += a * b, the full 128-bit product, nothing reduced: 13 instructions
-// against the 24 of a product reduced to [0, p) followed by a modular addition.  The two carry chains (the words
+// against the 20 of a product reduced to [0, p) followed by a modular addition.  The two carry chains (the words
 // of the product, the words of the sum) are interleaved so that each carry is read two slots after it was written.
 __device__ __forceinline__ void mul_acc(u32 (&w)[5], u64 a, u64 b) {
     u32 a0 = (u32)a, a1 = (u32)(a >> 32), b0 = (u32)b, b1 = (u32)(b >> 32);
@@ -344,6 +340,34 @@ __device__ __forceinline__ u64 mul_pow2(u64 v) {
     if (E == 0) return NEG ? sub(0, v) : v;
     constexpr int q = E >> 5, r = E & 31;
     const u32 v0 = (u32)v, v1 = (u32)(v >> 32);
+    if constexpr (q == 1 && r != 0 && !NEG) {
+        // v phi 2^r = v0 2^r phi + v1 2^r (phi - 1) = Q phi - R with R = v1 2^r and Q = v0 2^r + R < 2^(33 + r), two
+        // multiply-adds in the place of three shifts; Q phi - R = (Q0 + Q1) phi - (Q1 + R).  The carry of Q0 + Q1 and the borrow
+        // of the difference cancel where both are set; a borrow alone takes 2^32 - 1 off, a carry alone adds it
+        u64 R, Q, T, c, bo, st;
+        u32 S, d0, d1, m;
+        asm("v_mad_u64_u32 %[R], vcc, %[v1], %[c], 0\n\t"
+            "v_mad_u64_u32 %[Q], vcc, %[v0], %[c], %[R]"
+            : [R] "=&v"(R), [Q] "=v"(Q)
+            : [v0] "v"(v0), [v1] "v"(v1), [c] "s"(1u << r)
+            : "vcc");
+        const u32 q0 = (u32)Q, q1 = (u32)(Q >> 32);
+        asm("v_mad_u64_u32 %[T], vcc, %[q1], 1, %[R]\n\t"
+            "v_add_co_u32 %[S], %[c], %[q0], %[q1]"
+            : [T] "=&v"(T), [S] "=v"(S), [c] "=&s"(c)
+            : [q0] "v"(q0), [q1] "v"(q1), [R] "v"(R)
+            : "vcc");
+        asm("v_sub_co_u32 %[d0], vcc, 0, %[t0]\n\t"
+            "s_nop 1\n\t"
+            "v_subb_co_u32 %[d1], vcc, %[S], %[t1], vcc\n\t"
+            "s_andn2_b64 %[bo], vcc, %[c]\n\t"
+            "s_andn2_b64 %[st], %[c], vcc\n\t"
+            "v_cndmask_b32_e64 %[m], 0, %[k], %[bo]"
+            : [d0] "=&v"(d0), [d1] "=&v"(d1), [m] "=v"(m), [bo] "=&s"(bo), [st] "=&s"(st)
+            : [t0] "v"((u32)T), [t1] "v"((u32)(T >> 32)), [S] "v"(S), [c] "s"(c), [k] "n"(BORROWED)
+            : "vcc", "scc");
+        return canon_tail(minus_eps(pack(d0, d1), m), st);
+    }
     u32 m0, m1, m2;
     if constexpr (PIN && r != 0) {
         asm("v_lshlrev_b32 %[m0], %[r], %[v0]\n\t"
@@ -362,7 +386,7 @@ __device__ __forceinline__ u64 mul_pow2(u64 v) {
         asm("v_mad_u64_u32 %[w], %[st], %[m2], -1, %[x]"
             : [w] "=&v"(w), [st] "=&s"(st)
             : [m2] "v"(m2), [x] "v"(pack(m0, m1)));
-        const u64 x = canon_tail((u32)w, (u32)(w >> 32), st);
+        const u64 x = canon_tail(w, st);
         return NEG ? sub(0, x) : x;
     } else if (q == 1) {
         // m0 phi + m1 phi^2 + m2 phi^3 = (m0:0) + m1 (2^32 - 1) - m2
@@ -370,19 +394,14 @@ __device__ __forceinline__ u64 mul_pow2(u64 v) {
         asm("v_mad_u64_u32 %[w], %[st], %[m1], -1, %[x]"
             : [w] "=&v"(w), [st] "=&s"(st)
             : [m1] "v"(m1), [x] "v"(pack(0u, m0)));
-        const u64 x = canon_tail((u32)w, (u32)(w >> 32), st);
+        const u64 x = canon_tail(w, st);
         if (NEG) return sub((u64)m2, x);                   // m2 = 0 when r = 0
         return r ? sub(x, (u64)m2) : x;
     } else {
         // m0 phi^2 + m1 phi^3 + m2 phi^4 = m0 (2^32 - 1) - (m2:m1); both operands are below p
-        u32 e0, e1;
-        asm("v_sub_co_u32 %[e0], vcc, 0, %[m0]\n\t"
-            "s_nop 1\n\t"
-            "v_subbrev_co_u32 %[e1], vcc, 0, %[m0], vcc"
-            : [e0] "=&v"(e0), [e1] "=&v"(e1)
-            : [m0] "v"(m0)
-            : "vcc");
-        return NEG ? sub(pack(m1, m2), pack(e0, e1)) : sub(pack(e0, e1), pack(m1, m2));
+        u64 e;
+        asm("v_mad_u64_u32 %[e], vcc, %[m0], -1, 0" : [e] "=v"(e) : [m0] "v"(m0) : "vcc");
+        return NEG ? sub(pack(m1, m2), e) : sub(e, pack(m1, m2));
     }
 }
 
