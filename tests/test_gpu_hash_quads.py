@@ -27,6 +27,20 @@ def test_column_digests_around_the_switch(m, n):
     assert np.array_equal(got[cols], O.hash_columns(np.ascontiguousarray(a[:, cols])))
 
 
+@pytest.mark.parametrize("m,n", [(9, 131072), (9, 131073), (129, 65536), (129, 65537), (129, 131073), (300, 43520), (300, 43777)])
+def test_column_digests_around_two_wavefronts_per_simd(m, n):
+    """Chunks and merges on both sides of the launch size from which sums and exclusive ors have the long encoding."""
+    from verinf_amd.prover import cuda_primitives as cp
+    a = rand_field((m, n), m)
+    got = to_np(cp.hash_columns_streamed(to_dev(a)))
+    cols = [0, 1, n // 2, n - 2, n - 1]
+    assert np.array_equal(got[cols], O.hash_columns(np.ascontiguousarray(a[:, cols])))
+    rows = 9 if n > 100000 else 1                          # pads: a word a thread, both sides as well
+    seed = torch.arange(32, dtype=torch.uint8, device="cuda")
+    pads = to_np(cp.row_prg(seed, 5, rows, n // 8))
+    assert np.array_equal(pads[-1], O.row_prg(bytes(range(32)), 4 + rows, 1, n // 8)[0])
+
+
 def test_trees_of_every_small_size():
     from verinf_amd.prover import cuda_primitives as cp
     rng = np.random.default_rng(1)

@@ -41,9 +41,41 @@ __host__ __device__ constexpr int sched(int r, int i) {
 
 __device__ __forceinline__ u32 rotr(u32 x, int n) { return __builtin_amdgcn_alignbit(x, x, n); }
 
-// a + b + m in one instruction, out of the optimiser's reach
+// a ^ b and a + b, LONG: in the 64-bit encoding.  Among three-operand instructions, which are what else a G consists of and have no other
+// encoding, the short one of these takes as long as they do (half a G 24.7 cycles per SIMD at eight wavefronts), the long one a
+// good half of that (21.5): digests of 4096 x 2^16 words 705 -> 622 us, k_pad_rows of 333 x 16384 62 -> 52 together with the sums of
+// zero words.  A chain that a wavefront runs alone, or with one other, is 10 % slower with it: digests of 128 x 2^15 words 26.7 and 29.2 us,
+// x 2^16 30.8 and 33.1, x 2^17 47.1 and 47.0, x 2^18 87.0 and 82.4; the tree over 256 leaves 9.1 and 10.0.  So a launch has the long form
+// where it is more than two wavefronts per SIMD (wide_launch).
+template <bool LONG>
+__device__ __forceinline__ u32 xor2(u32 a, u32 b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    if constexpr (LONG) {
+        u32 r;
+        asm("v_xor_b32_e64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+        return r;
+    }
+#endif
+    return a ^ b;
+}
+template <bool LONG>
+__device__ __forceinline__ u32 add2(u32 a, u32 b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    if constexpr (LONG) {
+        u32 r;
+        asm("v_add_u32_e64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+        return r;
+    }
+#endif
+    return a + b;
+}
+
+// a + b + m in one instruction, out of the optimiser's reach; a word of the message that is known to be zero (most of a pad word's
+// message) leaves a cheaper sum
+template <bool LONG>
 __device__ __forceinline__ u32 add3(u32 a, u32 b, u32 m) {
 #if defined(__HIP_DEVICE_COMPILE__)
+    if (__builtin_constant_p(m) && m == 0) return add2<LONG>(a, b);
     u32 r;
     asm("v_add3_u32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(m));
     return r;
@@ -52,13 +84,13 @@ __device__ __forceinline__ u32 add3(u32 a, u32 b, u32 m) {
 #endif
 }
 
-#define B3_G(a, b, c, d, mx, my)            \
-    a = add3(a, b, mx); d = rotr(d ^ a, 16);  \
-    c = c + d;        b = rotr(b ^ c, 12);  \
-    a = add3(a, b, my); d = rotr(d ^ a, 8);   \
-    c = c + d;        b = rotr(b ^ c, 7);
+#define B3_G(a, b, c, d, mx, my)                                  \
+    a = add3<LONG>(a, b, mx);  d = rotr(xor2<LONG>(d, a), 16);        \
+    c = add2<LONG>(c, d);      b = rotr(xor2<LONG>(b, c), 12);        \
+    a = add3<LONG>(a, b, my);  d = rotr(xor2<LONG>(d, a), 8);         \
+    c = add2<LONG>(c, d);      b = rotr(xor2<LONG>(b, c), 7);
 
-template <int R>
+template <int R, bool LONG>
 __device__ __forceinline__ void b3_round(u32 (&s)[16], const u32 (&m)[16]) {
     B3_G(s[0], s[4], s[8], s[12], m[sched(R, 0)], m[sched(R, 1)])
     B3_G(s[1], s[5], s[9], s[13], m[sched(R, 2)], m[sched(R, 3)])
@@ -71,6 +103,7 @@ __device__ __forceinline__ void b3_round(u32 (&s)[16], const u32 (&m)[16]) {
 }
 
 // cv <- first eight words of compress(cv, m, counter, block_len, flags)
+template <bool LONG>
 __device__ __forceinline__ void compress(u32 (&cv)[8], const u32 (&m)[16], u64 counter, u32 block_len, u32 flags) {
     u32 s[16];
 #pragma unroll
@@ -81,8 +114,8 @@ __device__ __forceinline__ void compress(u32 (&cv)[8], const u32 (&m)[16], u64 c
     s[13] = (u32)(counter >> 32);
     s[14] = block_len;
     s[15] = flags;
-    b3_round<0>(s, m); b3_round<1>(s, m); b3_round<2>(s, m); b3_round<3>(s, m);
-    b3_round<4>(s, m); b3_round<5>(s, m); b3_round<6>(s, m);
+    b3_round<0, LONG>(s, m); b3_round<1, LONG>(s, m); b3_round<2, LONG>(s, m); b3_round<3, LONG>(s, m);
+    b3_round<4, LONG>(s, m); b3_round<5, LONG>(s, m); b3_round<6, LONG>(s, m);
 #pragma unroll
     for (int i = 0; i < 8; ++i) cv[i] = s[i] ^ s[i + 8];
 }
@@ -117,6 +150,7 @@ __device__ __forceinline__ u32 quad_turn(u32 v) {
 // lo, hi: words q and 4 + q of the chaining value, in and out.  msg: the sixteen message words of the quad in LDS.  All four
 // lanes of a quad take part.
 __device__ __forceinline__ void quad_compress(u32 &lo, u32 &hi, const u32 *msg, const QuadSchedule &S, int q, u64 counter, u32 block_len, u32 flags) {
+    constexpr bool LONG = false;
     u32 m[7][4];
 #pragma unroll
     for (int r = 0; r < 7; ++r)
@@ -199,6 +233,7 @@ __global__ __launch_bounds__(BLOCK) void k_chunk_cvs_quad(const u64 *__restrict_
 //   rows          first row of the slab (row pitch `stride` words), slab_rows rows in it
 //   single_root   the whole message is this one chunk: its last block carries ROOT
 // cvs[(chunk0 + c) * n + col] receives 8 words.
+template <bool LONG>
 __global__ __launch_bounds__(BLOCK) void k_chunk_cvs(const u64 *__restrict__ rows, i64 slab_rows, i64 n, i64 stride, i64 chunk0,
                                                      int single_root, u32 *__restrict__ cvs) {
     const i64 col = (i64)blockIdx.x * BLOCK + threadIdx.x;
@@ -224,7 +259,7 @@ __global__ __launch_bounds__(BLOCK) void k_chunk_cvs(const u64 *__restrict__ row
         u32 flags = 0;
         if (b == 0) flags |= CHUNK_START;
         if (b == n_blocks - 1) flags |= CHUNK_END | (single_root ? ROOT : 0u);
-        compress(cv, m, (u64)(chunk0 + c), (u32)(here * 8), flags);
+        compress<LONG>(cv, m, (u64)(chunk0 + c), (u32)(here * 8), flags);
     }
     u32 *o = cvs + ((chunk0 + c) * n + col) * 8;
 #pragma unroll
@@ -236,7 +271,7 @@ __global__ __launch_bounds__(BLOCK) void k_chunk_cvs(const u64 *__restrict__ row
 // level LV above the input level from the up to 2^LV input nodes under it (2^LV - 1 compressions, the lower ones
 // first), so the levels in between are never written.  cnt[j] = nodes of level j (cnt[0] = count of the input
 // level); the merge of the last two nodes of a level is the root.
-template <int LV>
+template <int LV, bool LONG>
 __device__ __forceinline__ void merge_node(const u32 *__restrict__ in, i64 n, i64 col, i64 idx, const i64 (&cnt)[4], u32 (&o)[8]) {
     if constexpr (LV == 0) {
         const u32 *p = in + (idx * n + col) * 8;
@@ -244,19 +279,19 @@ __device__ __forceinline__ void merge_node(const u32 *__restrict__ in, i64 n, i6
         for (int k = 0; k < 8; ++k) o[k] = p[k];
     } else {
         if (2 * idx + 1 >= cnt[LV - 1]) {
-            merge_node<LV - 1>(in, n, col, 2 * idx, cnt, o);
+            merge_node<LV - 1, LONG>(in, n, col, 2 * idx, cnt, o);
             return;
         }
         u32 l[8], r[8], m[16];
-        merge_node<LV - 1>(in, n, col, 2 * idx, cnt, l);
-        merge_node<LV - 1>(in, n, col, 2 * idx + 1, cnt, r);
+        merge_node<LV - 1, LONG>(in, n, col, 2 * idx, cnt, l);
+        merge_node<LV - 1, LONG>(in, n, col, 2 * idx + 1, cnt, r);
 #pragma unroll
         for (int k = 0; k < 8; ++k) { m[k] = l[k]; m[8 + k] = r[k]; o[k] = IV[k]; }
-        compress(o, m, 0, 64, PARENT | (cnt[LV - 1] == 2 ? ROOT : 0u));
+        compress<LONG>(o, m, 0, 64, PARENT | (cnt[LV - 1] == 2 ? ROOT : 0u));
     }
 }
 
-template <int LV>
+template <int LV, bool LONG>
 __global__ __launch_bounds__(BLOCK) void k_merge_levels(const u32 *__restrict__ in, i64 count, i64 n, i64 idx0, u32 *__restrict__ out) {
     const i64 col = (i64)blockIdx.x * BLOCK + threadIdx.x;
     if (col >= n) return;
@@ -266,7 +301,7 @@ __global__ __launch_bounds__(BLOCK) void k_merge_levels(const u32 *__restrict__ 
     for (int j = 1; j < 4; ++j) cnt[j] = (cnt[j - 1] + 1) / 2;
     const i64 i = idx0 + blockIdx.y;
     u32 o[8];
-    merge_node<LV>(in, n, col, i, cnt, o);
+    merge_node<LV, LONG>(in, n, col, i, cnt, o);
     u32 *dst = out + (i * n + col) * 8;
 #pragma unroll
     for (int k = 0; k < 8; ++k) dst[k] = o[k];
@@ -283,7 +318,7 @@ __global__ __launch_bounds__(BLOCK) void k_merkle_level(const u32 *__restrict__ 
     u32 m[16], cv[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) { m[k] = l[k]; m[8 + k] = r[k]; cv[k] = IV[k]; }
-    compress(cv, m, 0, 64, CHUNK_START | CHUNK_END | ROOT);
+    compress<false>(cv, m, 0, 64, CHUNK_START | CHUNK_END | ROOT);
 #pragma unroll
     for (int k = 0; k < 8; ++k) out[i * 8 + k] = cv[k];
 }
@@ -340,7 +375,7 @@ __global__ __launch_bounds__(BLOCK) void k_merkle_subtree(const u32 *__restrict_
             }
 #pragma unroll
             for (int k = 0; k < 8; ++k) cv[k] = IV[k];
-            compress(cv, m, 0, 64, CHUNK_START | CHUNK_END | ROOT);
+            compress<false>(cv, m, 0, 64, CHUNK_START | CHUNK_END | ROOT);
             u32 *o = out + off + i * 8;
             u32 *keep = buf[(j + 1) & 1] + threadIdx.x * 8;
 #pragma unroll
@@ -367,6 +402,7 @@ struct PrgRow {
 };
 
 __device__ __forceinline__ PrgRow prg_row(const u32 *__restrict__ seed, u64 row) {
+    constexpr bool LONG = false;               // some of it is the wavefront's, on the scalar unit
     PrgRow R;
 #pragma unroll
     for (int i = 0; i < 8; ++i) { R.m[i] = seed[i]; R.s[i] = IV[i]; }
@@ -387,30 +423,33 @@ __device__ __forceinline__ PrgRow prg_row(const u32 *__restrict__ seed, u64 row)
     return R;
 }
 
+template <bool LONG>
 __device__ __forceinline__ u64 prg_word(const PrgRow &R, i64 k) {
     u32 m[16], s[16];
 #pragma unroll
     for (int i = 0; i < 16; ++i) { m[i] = R.m[i]; s[i] = R.s[i]; }
     m[10] = (u32)k; m[11] = (u32)((u64)k >> 32);
     B3_G(s[1], s[6], s[11], s[12], m[10], m[11])
-    b3_round<1>(s, m); b3_round<2>(s, m); b3_round<3>(s, m);
-    b3_round<4>(s, m); b3_round<5>(s, m); b3_round<6>(s, m);
+    b3_round<1, LONG>(s, m); b3_round<2, LONG>(s, m); b3_round<3, LONG>(s, m);
+    b3_round<4, LONG>(s, m); b3_round<5, LONG>(s, m); b3_round<6, LONG>(s, m);
     const u64 raw = ((u64)(s[1] ^ s[9]) << 32) | (s[0] ^ s[8]);
     return raw >= 0xFFFFFFFF00000001ull ? raw - 0xFFFFFFFF00000001ull : raw;
 }
 
+template <bool LONG>
 __global__ __launch_bounds__(BLOCK) void k_row_prg(const u32 *__restrict__ seed, const u64 *__restrict__ row_indices, u32 row_offset,
                                                    i64 n_rows, i64 slack, u64 *__restrict__ out, i64 out_stride) {
     const i64 g = (i64)blockIdx.x * BLOCK + threadIdx.x;
     if (g >= n_rows * slack) return;
     const i64 r = g / slack, k = g - r * slack;
-    out[r * out_stride + k] = prg_word(prg_row(seed, row_indices ? row_indices[r] : (u64)(u32)(row_offset + (u32)r)), k);
+    out[r * out_stride + k] = prg_word<LONG>(prg_row(seed, row_indices ? row_indices[r] : (u64)(u32)(row_offset + (u32)r)), k);
 }
 
 // Message and pad of a padded row in one launch: out[r][k] = messages[r][k] for k < ell, and the value of k_row_prg at
 // k - ell behind it.  The hashing is bound by VALU issue (600 instructions a value), so the copy rides along (333 rows of
 // 8192 + 8192: 9 us as a launch of its own).  2^log_lanes threads of a workgroup take words first, first + step, ... of a row,
 // spread over the whole row so that every workgroup copies and hashes its share; the values of a thread have one PrgRow.
+template <bool LONG>
 __global__ __launch_bounds__(BLOCK) void k_pad_rows(const u32 *__restrict__ seed, u32 row_offset, const u64 *__restrict__ messages, i64 in_stride,
                                                     i64 ell, i64 n_rows, u32 segments, int log_lanes, i64 width, u64 *__restrict__ out) {
     const u32 group = blockIdx.x / segments;
@@ -422,7 +461,7 @@ __global__ __launch_bounds__(BLOCK) void k_pad_rows(const u32 *__restrict__ seed
     for (; k < ell; k += step) to[k] = from[k];
     if (k >= width) return;
     const PrgRow R = prg_row(seed, (u64)(u32)(row_offset + (u32)r));
-    for (; k < width; k += step) to[k] = prg_word(R, k - ell);
+    for (; k < width; k += step) to[k] = prg_word<LONG>(R, k - ell);
 }
 
 // The test-combiner challenge of the protocol (prover/protocol.py:127-135, device twin
@@ -456,7 +495,7 @@ __device__ __forceinline__ u64 challenge(const ChallengeKey &k, u64 cid) {
     m[8] = (u32)lo;  m[9] = (u32)(lo >> 32);
     m[10] = (u32)hi; m[11] = (u32)(hi >> 32);
     m[12] = m[13] = m[14] = m[15] = 0;
-    compress(cv, m, 0, (u32)(40 + k.label_len), CHUNK_START | CHUNK_END | ROOT);
+    compress<false>(cv, m, 0, (u32)(40 + k.label_len), CHUNK_START | CHUNK_END | ROOT);
     return gl::reduce128(((u64)cv[1] << 32) | cv[0], ((u64)cv[3] << 32) | cv[2]);
 }
 
@@ -498,6 +537,9 @@ __global__ __launch_bounds__(BLOCK) void k_spmv(const u64 *__restrict__ values, 
     }
 }
 
+// more than two wavefronts per SIMD: the long encoding of xor2 and add2
+inline bool wide_launch(const dim3 &grid) { return (i64)grid.x * grid.y * BLOCK > (i64)1 << 17; }
+
 inline i64 chunks_of(i64 m) { return m <= 0 ? 1 : (m + ROWS_PER_CHUNK - 1) / ROWS_PER_CHUNK; }
 
 }  // namespace
@@ -513,7 +555,7 @@ int launch_chunks(const u64 *rows, i64 slab_rows, i64 n, i64 row_stride, i64 chu
         hipLaunchKernelGGL(k_chunk_cvs_quad, grid, dim3(BLOCK), 0, s, rows, slab_rows, n, row_stride, chunk0, single_root ? 1 : 0, cvs);
     } else {
         dim3 grid((unsigned)((n + BLOCK - 1) / BLOCK), (unsigned)slab_chunks);
-        hipLaunchKernelGGL(k_chunk_cvs, grid, dim3(BLOCK), 0, s, rows, slab_rows, n, row_stride, chunk0, single_root ? 1 : 0, cvs);
+        hipLaunchKernelGGL(wide_launch(grid) ? k_chunk_cvs<true> : k_chunk_cvs<false>, grid, dim3(BLOCK), 0, s, rows, slab_rows, n, row_stride, chunk0, single_root ? 1 : 0, cvs);
     }
     VI_LAUNCH_CHECK("k_chunk_cvs");
     return VI_OK;
@@ -569,8 +611,9 @@ int vi_hash_columns_finalize(int64_t n, int64_t n_chunks_total, void *ws, size_t
         for (i64 lo = 0; lo < top; lo += 65535) {                 // grid.y limit
             const i64 cnt = top - lo < 65535 ? top - lo : 65535;
             dim3 grid((unsigned)((n + BLOCK - 1) / BLOCK), (unsigned)cnt);
-            if (lv == 1) hipLaunchKernelGGL(k_merge_levels<1>, grid, dim3(BLOCK), 0, s, (const u32 *)a, count, (i64)n, lo, dst);
-            else hipLaunchKernelGGL(k_merge_levels<2>, grid, dim3(BLOCK), 0, s, (const u32 *)a, count, (i64)n, lo, dst);
+            const auto kernel = wide_launch(grid) ? (lv == 1 ? k_merge_levels<1, true> : k_merge_levels<2, true>)
+                                                  : (lv == 1 ? k_merge_levels<1, false> : k_merge_levels<2, false>);
+            hipLaunchKernelGGL(kernel, grid, dim3(BLOCK), 0, s, (const u32 *)a, count, (i64)n, lo, dst);
             VI_LAUNCH_CHECK("k_merge_levels");
         }
         u32 *t = a; a = b; b = t;
@@ -646,7 +689,7 @@ int vi_row_prg(const uint8_t *seed, const uint64_t *row_indices, int64_t row_off
     const i64 total = n_rows * slack;
     const i64 blocks = (total + BLOCK - 1) / BLOCK;
     if (blocks > 0x7FFFFFFF) return vi::fail(VI_EINVAL, "vi_row_prg: %lld values exceed one launch", (long long)total);
-    hipLaunchKernelGGL(k_row_prg, dim3((unsigned)blocks), dim3(BLOCK), 0, (hipStream_t)stream, (const u32 *)seed, row_indices,
+    hipLaunchKernelGGL(wide_launch(dim3((unsigned)blocks)) ? k_row_prg<true> : k_row_prg<false>, dim3((unsigned)blocks), dim3(BLOCK), 0, (hipStream_t)stream, (const u32 *)seed, row_indices,
                        (u32)row_offset, (i64)n_rows, (i64)slack, out, (i64)out_stride);
     VI_LAUNCH_CHECK("k_row_prg");
     return VI_OK;
@@ -670,7 +713,8 @@ int vi_pad_rows(const uint8_t *seed, int64_t row_offset, const uint64_t *message
     const i64 units = (width + ((i64)1 << log_lanes) - 1) >> log_lanes, segments = log_lanes < 8 ? 1 : (units + (1 << log_per) - 1) >> log_per;
     const i64 groups = (n_rows + (BLOCK >> log_lanes) - 1) / (BLOCK >> log_lanes);
     if (groups > 0x7FFFFFFF / segments) return vi::fail(VI_EINVAL, "vi_pad_rows: %lld words exceed one launch", (long long)(n_rows * width));
-    hipLaunchKernelGGL(k_pad_rows, dim3((unsigned)(groups * segments)), dim3(BLOCK), 0, (hipStream_t)stream, (const u32 *)seed, (u32)row_offset, messages,
+    const dim3 grid((unsigned)(groups * segments));
+    hipLaunchKernelGGL(wide_launch(grid) ? k_pad_rows<true> : k_pad_rows<false>, grid, dim3(BLOCK), 0, (hipStream_t)stream, (const u32 *)seed, (u32)row_offset, messages,
                        (i64)in_stride, (i64)ell, (i64)n_rows, (u32)segments, log_lanes, (i64)width, out);
     VI_LAUNCH_CHECK("k_pad_rows");
     return VI_OK;
