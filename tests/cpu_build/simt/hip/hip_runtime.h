@@ -284,7 +284,12 @@ inline hipError_t hipFuncSetAttribute(const void *, int, int) { return hipSucces
 template <class T>
 hipError_t hipGetSymbolAddress(void **p, T &symbol) { *p = (void *)&symbol; return hipSuccess; }
 enum hipDeviceAttribute_t { hipDeviceAttributeMultiprocessorCount };
-inline hipError_t hipDeviceGetAttribute(int *v, hipDeviceAttribute_t, int) { *v = 256; return hipSuccess; }
+// SIMT_CUS: a smaller chip, on which launches of the resident grid go round several times at small sizes
+inline hipError_t hipDeviceGetAttribute(int *v, hipDeviceAttribute_t, int) {
+    const char *cus = getenv("SIMT_CUS");
+    *v = cus ? atoi(cus) : 256;
+    return hipSuccess;
+}
 template <class K>
 hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int *n, K, int, size_t) { *n = 4; return hipSuccess; }
 inline hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }

@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 torch = pytest.importorskip("torch")
 from oracle import oracle as O  # noqa: E402
-from tests.gpu_util import P, rand_field, to_dev, to_np, unhex  # noqa: E402
+from tests.gpu_util import P, rand_field, rand_field_dev, to_dev, to_np, unhex  # noqa: E402
 
 
 @pytest.fixture(scope="module")
@@ -758,6 +758,22 @@ def test_first_sample_at_one_from_a_later_round(mods, terms, v, coins):
     claim, polys, _, _ = gpu.prove_terms_gpu([(c, [dev[i] for i in fs]) for c, fs in terms], lambda i: coins[i], P)
     want_claim, want_samples, _ = O.sumcheck_prove(tabs, terms, coins)
     assert claim == want_claim and [[y for _, y in s] for s in polys] == want_samples
+
+
+@pytest.mark.parametrize("v", [20, 21, 22, 24])
+@pytest.mark.parametrize("terms", [[(5, [0])], [(7, [0, 1])], [(1, [0, 1, 2])], [(3, [0, 1, 2, 3])], [(3, [0, 1, 2]), (P - 3, [0, 3])]])
+def test_first_passes_around_what_the_chip_holds(mods, terms, v):
+    """One launch whose threads have a column each, and pieces of columns taken from a counter beyond; tables that start on 8 bytes
+    only, words at and above p among them."""
+    gpu, _ = mods
+    n = 1 + max(max(fs) for _, fs in terms)
+    tabs = [rand_field_dev(((1 << v) + 1,), 31 * v + t)[1:] for t in range(n)]
+    for t in tabs:
+        t.view(torch.int64)[::(1 << 13) + 5] = -1                      # 2^64 - 1
+    coins = _coins(v, v)[0]
+    claim, polys, _, _ = gpu.prove_terms_gpu([(c, [tabs[i] for i in fs]) for c, fs in terms], lambda i: coins[i], P)
+    want_claim, want, _ = O.sumcheck_prove([to_np(t) % np.uint64(P) for t in tabs], terms, coins)
+    assert claim == want_claim and [[y for _, y in s] for s in polys] == want
 
 
 @pytest.mark.parametrize("v", range(1, 16))

@@ -300,6 +300,17 @@ __device__ __forceinline__ void canon_all(u64 (&v)[N]) {
     }
 }
 
+template <int N>
+__device__ __forceinline__ void canon_pairs(u64 (&lo)[N], u64 (&hi)[N]) {
+    u32 top = 0;
+#pragma unroll
+    for (int i = 0; i < N; ++i) top = max(max(top, (u32)(lo[i] >> 32)), (u32)(hi[i] >> 32));
+    if (__any(top == 0xFFFFFFFFu)) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) { lo[i] = gl::canon(lo[i]); hi[i] = gl::canon(hi[i]); }
+    }
+}
+
 template <int NT, int SHAPE, bool FIRST>
 __device__ __forceinline__ u64 fast_load(const FastDesc &D, int t, i64 idx) {
     u64 v = D.src[t][idx];
@@ -310,18 +321,18 @@ __device__ __forceinline__ u64 fast_load(const FastDesc &D, int t, i64 idx) {
     return v;
 }
 
-// sum over the rows of NSAMP words at `rows` -> out[0..ns), by one workgroup of BLOCK threads
-template <int NS>
+// sum over the rows of NSAMP words at `rows` -> out[0..ns), by one workgroup of THREADS threads
+template <int NS, int THREADS = BLOCK>
 __device__ __forceinline__ void block_sum_rows(const u64 *rows, int n_rows, u64 *out, u64 (*red)[NSAMP]) {
     u64 v[NS];
 #pragma unroll
     for (int x = 0; x < NS; ++x) v[x] = 0;
-    for (int b0 = threadIdx.x; b0 < n_rows; b0 += 2 * BLOCK) {         // two rows per thread in flight
+    for (int b0 = threadIdx.x; b0 < n_rows; b0 += 2 * THREADS) {         // two rows per thread in flight
         u64 t[2][NS];
 #pragma unroll
         for (int u = 0; u < 2; ++u)
 #pragma unroll
-            for (int x = 0; x < NS; ++x) t[u][x] = (b0 + u * BLOCK < n_rows) ? rows[(i64)(b0 + u * BLOCK) * NSAMP + x] : 0;
+            for (int x = 0; x < NS; ++x) t[u][x] = (b0 + u * THREADS < n_rows) ? rows[(i64)(b0 + u * THREADS) * NSAMP + x] : 0;
 #pragma unroll
         for (int u = 0; u < 2; ++u)
 #pragma unroll
@@ -336,14 +347,14 @@ __device__ __forceinline__ void block_sum_rows(const u64 *rows, int n_rows, u64 
     __syncthreads();
     if (threadIdx.x < NS) {
         u64 sum = red[0][threadIdx.x];
-        for (int i = 1; i < BLOCK / 64; ++i) sum = gl::addc(sum, red[i][threadIdx.x]);
+        for (int i = 1; i < THREADS / 64; ++i) sum = gl::addc(sum, red[i][threadIdx.x]);
         out[threadIdx.x] = sum;
     }
     __syncthreads();
 }
 
 // a pass's sums of its three rounds over the workgroup, times scale -> row at `row`, region_words apart
-template <int NS>
+template <int NS, int WAVES = BLOCK / 64>
 __device__ __forceinline__ void pass_sums(const SampleAcc<true> (&acc0)[NS], const SampleAcc<true> (&acc1)[NS], const SampleAcc<true> (&acc2)[NS],
                                           u64 (*red)[3 * NS], u64 *row, i64 region_words, u64 scale) {
     u64 v[3 * NS];
@@ -360,29 +371,29 @@ __device__ __forceinline__ void pass_sums(const SampleAcc<true> (&acc0)[NS], con
     if (threadIdx.x < 3 * NS) {
         u64 s = red[0][threadIdx.x];
 #pragma unroll
-        for (int w = 1; w < BLOCK / 64; ++w) s = gl::addc(s, red[w][threadIdx.x]);
+        for (int w = 1; w < WAVES; ++w) s = gl::addc(s, red[w][threadIdx.x]);
         if (scale != 1) s = gl::mul(s, scale);
         row[threadIdx.x / NS * region_words + threadIdx.x % NS] = s;
     }
 }
 
-// Three rounds on eight entries of every table, v[t][c] = entry i + c cols (canonical): the samples of the seven pairs into the rounds'
-// accumulators, the entry folded three times into `folded`.  ONE: the first round sums S(1) too.
-template <int NT, int SHAPE, bool ONE>
-__device__ __forceinline__ void three_rounds(u64 (&v)[NT][8], u64 r0, u64 r1, u64 r2, SampleAcc<true> (&acc0)[FastShape<NT, SHAPE>::NS],
-                                             SampleAcc<true> (&acc1)[FastShape<NT, SHAPE>::NS], SampleAcc<true> (&acc2)[FastShape<NT, SHAPE>::NS],
-                                             u64 (&folded)[NT]) {
+// Three rounds on eight entries of every table: load(c, lo, hi), called for c = 0 .. 3 in turn, gives entries i + c cols and i + (c + 4) cols
+// (canonical).  The samples of the seven pairs go into the rounds' accumulators, the entry folded three times into `folded`.  ONE: the
+// first round sums S(1) too.
+template <int NT, int SHAPE, bool ONE, class Load>
+__device__ __forceinline__ void three_rounds_from(Load load, u64 r0, u64 r1, u64 r2, SampleAcc<true> (&acc0)[FastShape<NT, SHAPE>::NS],
+                                                  SampleAcc<true> (&acc1)[FastShape<NT, SHAPE>::NS], SampleAcc<true> (&acc2)[FastShape<NT, SHAPE>::NS],
+                                                  u64 (&folded)[NT]) {
     // the scheduler is kept from interleaving the pairs: each one's temporaries die before the next starts
-    u64 lo[NT], hi[NT], dif[NT];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
+    u64 lo[NT], hi[NT], dif[NT], v[NT][4];
+    static_for<0, 4>([&](auto c_) {
+        constexpr int c = decltype(c_)::value;
         VI_SCHED_FENCE();
-#pragma unroll
-        for (int t = 0; t < NT; ++t) { lo[t] = v[t][c]; hi[t] = v[t][c + 4]; }
+        load(c_, lo, hi);
         eval_pair<NT, SHAPE, !ONE, true>(lo, hi, dif, acc0);
 #pragma unroll
         for (int t = 0; t < NT; ++t) v[t][c] = gl::mul_add(r0, dif[t], lo[t]);
-    }
+    });
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
         VI_SCHED_FENCE();
@@ -398,6 +409,47 @@ __device__ __forceinline__ void three_rounds(u64 (&v)[NT][8], u64 r0, u64 r1, u6
     eval_pair<NT, SHAPE, true, true>(lo, hi, dif, acc2);
 #pragma unroll
     for (int t = 0; t < NT; ++t) folded[t] = gl::mul_add(r2, dif[t], lo[t]);
+}
+
+// the same of entries in registers, v[t][c] = entry i + c cols
+template <int NT, int SHAPE, bool ONE>
+__device__ __forceinline__ void three_rounds(const u64 (&v)[NT][8], u64 r0, u64 r1, u64 r2, SampleAcc<true> (&acc0)[FastShape<NT, SHAPE>::NS],
+                                             SampleAcc<true> (&acc1)[FastShape<NT, SHAPE>::NS], SampleAcc<true> (&acc2)[FastShape<NT, SHAPE>::NS],
+                                             u64 (&folded)[NT]) {
+    auto load = [&](auto c_, u64 (&lo)[NT], u64 (&hi)[NT]) {
+        constexpr int c = decltype(c_)::value;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) { lo[t] = v[t][c]; hi[t] = v[t][c + 4]; }
+    };
+    three_rounds_from<NT, SHAPE, ONE>(load, r0, r1, r2, acc0, acc1, acc2, folded);
+}
+
+// 64 words at src into LDS, by one wavefront and without a register in between; src and dst are the same for all its lanes.  Two
+// loads of four bytes a lane, which ask for no more than the alignment of a word.  The compiler does not wait for them: loads_arrived()
+// does.  M0 has its value back afterwards (the compiler does not accept it in a list of clobbered registers).
+__device__ __forceinline__ void words_to_lds(const u64 *src, u64 *dst, int lane) {
+#ifdef __HIP_DEVICE_COMPILE__
+    const u32 at = __builtin_amdgcn_readfirstlane((u32)(uintptr_t)(__attribute__((address_space(3))) u64 *)dst);
+    u32 m0;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %3, %5\n\t"
+                 "s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %4, %5\n\ts_mov_b32 m0, %0"
+                 : "=&s"(m0) : "s"(at), "s"(at + 256), "v"((u32)lane * 4), "v"((u32)lane * 4 + 256), "s"(src) : "memory");
+#else
+    dst[lane] = src[lane];
+#endif
+}
+// all but the LATER youngest of the wavefront's loads and stores are complete
+template <int LATER>
+__device__ __forceinline__ void loads_arrived() {
+#ifdef __HIP_DEVICE_COMPILE__
+    asm volatile("s_waitcnt vmcnt(%0)" : : "n"(LATER) : "memory");
+#endif
+}
+// the wavefront's LDS reads are complete
+__device__ __forceinline__ void lds_reads_done() {
+#ifdef __HIP_DEVICE_COMPILE__
+    asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+#endif
 }
 
 // Three rounds in one pass.  cols = n / 8 for tables of n words; thread i < cols owns entries i + c cols.
@@ -444,6 +496,88 @@ __global__ __launch_bounds__(BLOCK) void k_pass3(const FastDesc D, i64 cols, u64
         for (int t = 0; t < NT; ++t) D.dst[t][i] = folded[t];
     }
     pass_sums<NS>(acc0, acc1, acc2, red, part + (i64)blockIdx.x * NSAMP, (i64)gridDim.x * NSAMP, 1);
+}
+
+// The same for more columns than fit the chip at once.  Two things keep the plain loop from either of its bounds there: a SIMD
+// serves its oldest wavefront first, so of four workgroups of a CU with the same share the first was done after 250 us and the last
+// after 450 (three tables of 2^26), alone by then; and a wavefront's loads wait for its arithmetic.  So a workgroup has all the wavefronts
+// of a CU, which take pieces of 64 columns from a counter in LDS, and a piece's entries are on their way into LDS while
+// the piece before it is worked on (18 of 24 words a lane for three tables; the last pair's go to registers, as they have three pairs' time).
+// First pass over three tables of 2^26 424 -> 384 us (resident grid with equal shares and this staging: 436); its proof 559 -> 512.
+template <int NT>
+struct LongPass {
+    static constexpr int THREADS = NT <= 3 ? 1024 : 768;               // 128 and 168 registers
+};
+
+template <int NT, int SHAPE, bool FIRST, bool ONE>
+__global__ __launch_bounds__(LongPass<NT>::THREADS) void k_pass3_long(const FastDesc D, i64 cols, u64 r0, u64 r1, u64 r2, u64 *part,
+                                                 const u64 *prev_part, int prev_rows, u64 *prev_sums) {
+    constexpr int NS = FastShape<NT, SHAPE>::NS;
+    constexpr int WAVES = LongPass<NT>::THREADS / 64;
+    __shared__ u64 red[WAVES][3 * NS];
+    __shared__ u64 red_prev[WAVES][NSAMP];
+    __shared__ u64 stage[WAVES][6 * NT][64];
+    __shared__ int next;
+    if (threadIdx.x == 0) next = WAVES;
+    __syncthreads();
+    if (prev_rows > 0 && blockIdx.x < 3)
+        block_sum_rows<NS, 64 * WAVES>(prev_part + (i64)blockIdx.x * prev_rows * NSAMP, prev_rows, prev_sums + blockIdx.x * NSAMP, red_prev);
+    SampleAcc<true> acc0[NS], acc1[NS], acc2[NS];
+#pragma unroll
+    for (int x = 0; x < NS; ++x) { acc0[x].zero(); acc1[x].zero(); acc2[x].zero(); }
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    u64 (&mine)[6 * NT][64] = stage[wave];
+    // entries c and c + 4 of table t are rows 2 (3 t + c) and 2 (3 t + c) + 1 of the wavefront's stage; c = 3 goes to registers
+    auto fetch = [&](i64 first) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                words_to_lds(D.src[t] + first + c * cols, mine[2 * (3 * t + c)], lane);
+                words_to_lds(D.src[t] + first + (c + 4) * cols, mine[2 * (3 * t + c) + 1], lane);
+            }
+    };
+    // piece j of the workgroup: sixteen in a row, then its next sixteen
+    auto piece = [&](int j) { return ((i64)(j >> 4) * gridDim.x + blockIdx.x) * 1024 + (j & 15) * 64; };
+    i64 first = piece(wave), following = 0;
+    if (first < cols) fetch(first);
+    for (; first < cols; first = following) {
+        const i64 i = first + lane;
+        u64 last[NT][2];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            last[t][0] = D.src[t][i + 3 * cols];
+            last[t][1] = D.src[t][i + 7 * cols];
+        }
+        loads_arrived<2 * NT>();
+        auto load = [&](auto c_, u64 (&lo)[NT], u64 (&hi)[NT]) {
+            constexpr int c = decltype(c_)::value;
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                lo[t] = c < 3 ? mine[2 * (3 * t + c % 3)][lane] : last[t][0];
+                hi[t] = c < 3 ? mine[2 * (3 * t + c % 3) + 1][lane] : last[t][1];
+            }
+            if constexpr (c == 2) {
+                int j = 0;
+                if (lane == 0) j = atomicAdd(&next, 1);
+                following = piece((int)__builtin_amdgcn_readfirstlane((u32)__shfl((u64)j, 0, 64)));
+                lds_reads_done();
+                if (following < cols) fetch(following);
+            }
+            if (FIRST) {
+                canon_pairs(lo, hi);
+                if (SHAPE == 2) {
+                    lo[NT - 1] = gl::mul(lo[NT - 1], D.lin_coeff);
+                    hi[NT - 1] = gl::mul(hi[NT - 1], D.lin_coeff);
+                }
+            }
+        };
+        u64 folded[NT];
+        three_rounds_from<NT, SHAPE, ONE>(load, r0, r1, r2, acc0, acc1, acc2, folded);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) D.dst[t][i] = folded[t];
+    }
+    pass_sums<NS, WAVES>(acc0, acc1, acc2, red, part + (i64)blockIdx.x * NSAMP, (i64)gridDim.x * NSAMP, 1);
 }
 
 // pairs per table a tail workgroup holds after its first fold
@@ -584,17 +718,25 @@ template <int NT, int SHAPE, bool FIRST, bool ONE>
 int launch_pass3(const FastDesc &F, i64 cols, const u64 *r, u64 *part, const u64 *prev_part, int prev_rows,
                  u64 *prev_sums, hipStream_t s) {
     static std::mutex mu;
-    static int caps[64] = {0};
+    static int caps[64] = {0}, cus[64] = {0};
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
-    int cap;
+    int cap, n_cus;
     {
         std::lock_guard<std::mutex> lock(mu);
-        if (!caps[dev]) caps[dev] = resident_blocks(k_pass3<NT, SHAPE, FIRST, ONE>, 64);
+        if (!caps[dev]) {
+            caps[dev] = resident_blocks(k_pass3<NT, SHAPE, FIRST, ONE>, 64);
+            cus[dev] = resident_blocks(k_pass3<NT, SHAPE, FIRST, ONE>, 1);
+        }
         cap = caps[dev];
+        n_cus = cus[dev];
     }
     int nb = blocks_for(cols);
-    if (nb > cap) nb = cap;
+    if (nb > cap) {
+        hipLaunchKernelGGL((k_pass3_long<NT, SHAPE, FIRST, ONE>), dim3(n_cus), dim3(LongPass<NT>::THREADS), 0, s, F, cols, r[0], r[1], r[2], part,
+                           prev_part, prev_rows, prev_sums);
+        return n_cus;
+    }
     if (nb < 3 && prev_rows > 0) nb = 3;     // the first three workgroups add up the previous pass's sums
     hipLaunchKernelGGL((k_pass3<NT, SHAPE, FIRST, ONE>), dim3(nb), dim3(BLOCK), 0, s, F, cols, r[0], r[1], r[2], part,
                        prev_part, prev_rows, prev_sums);
