@@ -115,6 +115,26 @@ __global__ __launch_bounds__(BLOCK) void k_probe(int op, const u64 *a, const u64
             }
             r = gl::wide_reduce(A);
         }
+        else if (op >= 20 && op < 32) {
+            // two at once: the first result, and the second (of other operands)
+            u64 p, q;
+            const u64 e = ((x << 17) | (x >> 47)) ^ y;
+            if (op < 22) gl::sub2(x, y, p, y, x, q);
+            else if (op < 24) gl::addc2(x, y, p, y, y, q);
+            else if (op < 26) gl::mul2(x, y, p, y, y, q);
+            else if (op < 28) gl::mul_lazy2(x, y, p, y, y, q);
+            else if (op < 30) gl::mul_add2(x, y, e, p, y, y, x, q);
+            else {
+                gl::Wide A, B;
+                gl::wide_zero(A);
+                gl::wide_zero(B);
+                for (int k = 0; k < 40; ++k) gl::wide_mul_acc2(A, x, y, B, ~0ull, ~y);
+                p = gl::wide_reduce(A);
+                q = gl::wide_reduce(B);
+            }
+            r = op & 1 ? q : p;
+            if (op == 26 || op == 27) r = gl::canon(r);
+        }
         else if (op >= 300) r = shift_pinned_by<0>(x, op - 300);
         else r = shift_by<0>(x, op - 100);
         out[i] = r;
@@ -386,7 +406,7 @@ int vi_gl_axpy(uint64_t *y, uint64_t alpha, const uint64_t *x, int64_t n, void *
 
 int vi_gl_probe(int op, const uint64_t *a, const uint64_t *b, uint64_t *out, int64_t n, void *stream) {
     const bool shift = (op >= 100 && op < 196) || (op >= 300 && op < 492);
-    if (!shift && (op < 0 || op > 11)) return vi::fail(VI_EINVAL, "vi_gl_probe: op = %d", op);
+    if (!shift && (op < 0 || (op > 11 && op < 20) || op > 31)) return vi::fail(VI_EINVAL, "vi_gl_probe: op = %d", op);
     if (n < 0) return vi::fail(VI_EINVAL, "vi_gl_probe: n = %lld", (long long)n);
     if (n == 0) return VI_OK;
     const bool needs_b = !shift && op != 4;

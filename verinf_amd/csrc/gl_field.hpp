@@ -405,6 +405,186 @@ __device__ __forceinline__ u64 mul_pow2(u64 v) {
     }
 }
 
+// ---- two at once ------------------------------------------------------------------------------------------------
+// The same operations on two independent sets of operands, their instructions interleaved: where a SIMD has four wavefronts, a
+// product takes 77 cycles alone and 66 beside another (66 and 64 with eight wavefronts), as its carries are waited for otherwise.
+
+__device__ __forceinline__ void sub2(u64 a, u64 b, u64 &x, u64 c, u64 d, u64 &y) {
+    u32 x0, x1, y0, y1, m, n;
+    u64 t;
+    asm("v_sub_co_u32 %[x0], vcc, %[a0], %[b0]\n\t"
+        "v_sub_co_u32 %[y0], %[t], %[c0], %[d0]\n\t"
+        "s_nop 0\n\t"
+        "v_subb_co_u32 %[x1], vcc, %[a1], %[b1], vcc\n\t"
+        "v_subb_co_u32 %[y1], %[t], %[c1], %[d1], %[t]\n\t"
+        "s_nop 0\n\t"
+        "v_cndmask_b32_e64 %[m], 0, %[k], vcc\n\t"
+        "v_cndmask_b32_e64 %[n], 0, %[k], %[t]"
+        : [x0] "=&v"(x0), [x1] "=&v"(x1), [y0] "=&v"(y0), [y1] "=&v"(y1), [m] "=&v"(m), [n] "=v"(n), [t] "=&s"(t)
+        : [a0] "v"((u32)a), [a1] "v"((u32)(a >> 32)), [b0] "v"((u32)b), [b1] "v"((u32)(b >> 32)), [c0] "v"((u32)c), [c1] "v"((u32)(c >> 32)),
+          [d0] "v"((u32)d), [d1] "v"((u32)(d >> 32)), [k] "n"(BORROWED)
+        : "vcc");
+    x = minus_eps(pack(x0, x1), m);
+    y = minus_eps(pack(y0, y1), n);
+}
+
+// two words with their carries, as canon_tail
+__device__ __forceinline__ void canon_tail2(u64 w, u64 st, u64 &x, u64 v, u64 tt, u64 &y) {
+    u64 r, z;
+    asm("v_mad_u64_u32 %[r], vcc, 1, -1, %[w]\n\t"
+        "s_or_b64 %[st], %[st], vcc\n\t"
+        "v_mad_u64_u32 %[z], vcc, 1, -1, %[v]\n\t"
+        "s_or_b64 %[tt], %[tt], vcc"
+        : [r] "=&v"(r), [z] "=v"(z), [st] "+s"(st), [tt] "+s"(tt)
+        : [w] "v"(w), [v] "v"(v)
+        : "vcc", "scc");
+    x = select(st, r, w);
+    y = select(tt, z, v);
+}
+
+__device__ __forceinline__ void addc2(u64 a, u64 b, u64 &x, u64 c, u64 d, u64 &y) {
+    u32 s0, s1, t0, t1;
+    u64 st, tt;
+    asm("v_add_co_u32 %[s0], vcc, %[a0], %[b0]\n\t"
+        "v_add_co_u32 %[t0], %[tt], %[c0], %[d0]\n\t"
+        "s_nop 0\n\t"
+        "v_addc_co_u32 %[s1], %[st], %[a1], %[b1], vcc\n\t"
+        "v_addc_co_u32 %[t1], %[tt], %[c1], %[d1], %[tt]"
+        : [s0] "=&v"(s0), [s1] "=&v"(s1), [t0] "=&v"(t0), [t1] "=&v"(t1), [st] "=&s"(st), [tt] "=&s"(tt)
+        : [a0] "v"((u32)a), [a1] "v"((u32)(a >> 32)), [b0] "v"((u32)b), [b1] "v"((u32)(b >> 32)), [c0] "v"((u32)c), [c1] "v"((u32)(c >> 32)),
+          [d0] "v"((u32)d), [d1] "v"((u32)(d >> 32))
+        : "vcc");
+    canon_tail2(pack(s0, s1), st, x, pack(t0, t1), tt, y);
+}
+
+// partial products of a b and c d as in mul_words, ADD: with the addends e and f
+template <bool ADD>
+__device__ __forceinline__ void partial_products2(u64 a, u64 b, u64 e, u64 c, u64 d, u64 f, u64 &p00, u64 &mm, u64 &p11, u64 &st, u64 &cy, u64 &q00, u64 &nn,
+                                                  u64 &q11, u64 &tt, u64 &cz) {
+    const u32 a0 = (u32)a, a1 = (u32)(a >> 32), b0 = (u32)b, b1 = (u32)(b >> 32), c0 = (u32)c, c1 = (u32)(c >> 32), d0 = (u32)d, d1 = (u32)(d >> 32);
+    if (ADD) {
+        asm("v_mad_u64_u32 %[mm], vcc, %[a1], %[b0], 0\n\t"
+            "v_mad_u64_u32 %[nn], vcc, %[c1], %[d0], 0\n\t"
+            "v_mad_u64_u32 %[p00], %[cy], %[a0], %[b0], %[e]\n\t"
+            "v_mad_u64_u32 %[q00], %[cz], %[c0], %[d0], %[f]\n\t"
+            "v_mad_u64_u32 %[mm], %[st], %[a0], %[b1], %[mm]\n\t"
+            "v_mad_u64_u32 %[nn], %[tt], %[c0], %[d1], %[nn]\n\t"
+            "v_mad_u64_u32 %[p11], vcc, %[a1], %[b1], 0\n\t"
+            "v_mad_u64_u32 %[q11], vcc, %[c1], %[d1], 0"
+            : [p00] "=&v"(p00), [mm] "=&v"(mm), [p11] "=&v"(p11), [st] "=&s"(st), [cy] "=&s"(cy), [q00] "=&v"(q00), [nn] "=&v"(nn), [q11] "=&v"(q11),
+              [tt] "=&s"(tt), [cz] "=&s"(cz)
+            : [a0] "v"(a0), [a1] "v"(a1), [b0] "v"(b0), [b1] "v"(b1), [c0] "v"(c0), [c1] "v"(c1), [d0] "v"(d0), [d1] "v"(d1), [e] "v"(e), [f] "v"(f)
+            : "vcc");
+    } else {
+        asm("v_mad_u64_u32 %[mm], vcc, %[a1], %[b0], 0\n\t"
+            "v_mad_u64_u32 %[nn], vcc, %[c1], %[d0], 0\n\t"
+            "v_mad_u64_u32 %[p00], vcc, %[a0], %[b0], 0\n\t"
+            "v_mad_u64_u32 %[q00], vcc, %[c0], %[d0], 0\n\t"
+            "v_mad_u64_u32 %[mm], %[st], %[a0], %[b1], %[mm]\n\t"
+            "v_mad_u64_u32 %[nn], %[tt], %[c0], %[d1], %[nn]\n\t"
+            "v_mad_u64_u32 %[p11], vcc, %[a1], %[b1], 0\n\t"
+            "v_mad_u64_u32 %[q11], vcc, %[c1], %[d1], 0"
+            : [p00] "=&v"(p00), [mm] "=&v"(mm), [p11] "=&v"(p11), [st] "=&s"(st), [q00] "=&v"(q00), [nn] "=&v"(nn), [q11] "=&v"(q11), [tt] "=&s"(tt)
+            : [a0] "v"(a0), [a1] "v"(a1), [b0] "v"(b0), [b1] "v"(b1), [c0] "v"(c0), [c1] "v"(c1), [d0] "v"(d0), [d1] "v"(d1)
+            : "vcc");
+    }
+}
+
+// x = a b (+ e), y = c d (+ f).  LAZY: words congruent to them, not necessarily below p
+template <bool ADD, bool LAZY>
+__device__ __forceinline__ void mul2(u64 a, u64 b, u64 e, u64 &x, u64 c, u64 d, u64 f, u64 &y) {
+    u64 p00, mm, p11, st, cy, q00, nn, q11, tt, cz;
+    partial_products2<ADD>(a, b, e, c, d, f, p00, mm, p11, st, cy, q00, nn, q11, tt, cz);
+    u32 g0 = (u32)p11, g1 = (u32)(p11 >> 32), h0 = (u32)q11, h1 = (u32)(q11 >> 32);
+    if (ADD) {
+        asm("v_addc_co_u32 %[g0], vcc, 0, %[g0], %[cy]\n\t"
+            "v_addc_co_u32 %[h0], %[cz], 0, %[h0], %[cz]\n\t"
+            "s_nop 0\n\t"
+            "v_addc_co_u32 %[g1], vcc, 0, %[g1], vcc\n\t"
+            "v_addc_co_u32 %[h1], vcc, 0, %[h1], %[cz]"
+            : [g0] "+&v"(g0), [g1] "+&v"(g1), [h0] "+&v"(h0), [h1] "+&v"(h1), [cz] "+&s"(cz)
+            : [cy] "s"(cy)
+            : "vcc");
+    }
+    u32 w1 = (u32)(p00 >> 32), v1 = (u32)(q00 >> 32), hl, hh, kl, kh, x0, x1, y0, y1, m, n;
+    u64 t;
+    asm("v_add_co_u32 %[w1], vcc, %[w1], %[m0]\n\t"
+        "v_add_co_u32 %[v1], %[t], %[v1], %[n0]\n\t"
+        "s_nop 0\n\t"
+        "v_addc_co_u32 %[hl], vcc, %[g0], %[m1], vcc\n\t"
+        "v_addc_co_u32 %[kl], %[t], %[h0], %[n1], %[t]\n\t"
+        "s_nop 0\n\t"
+        "v_addc_co_u32 %[hh], vcc, 0, %[g1], vcc\n\t"
+        "v_subb_co_u32 %[x0], vcc, %[l0], %[hh], %[st]\n\t"
+        "v_addc_co_u32 %[kh], %[t], 0, %[h1], %[t]\n\t"
+        "v_subb_co_u32 %[y0], %[t], %[k0], %[kh], %[tt]\n\t"
+        "v_subbrev_co_u32 %[x1], vcc, 0, %[w1], vcc\n\t"
+        "s_nop 0\n\t"
+        "v_subbrev_co_u32 %[y1], %[t], 0, %[v1], %[t]\n\t"
+        "v_cndmask_b32_e64 %[m], 0, %[k3], vcc\n\t"
+        "s_nop 0\n\t"
+        "v_cndmask_b32_e64 %[n], 0, %[k3], %[t]"
+        : [w1] "+&v"(w1), [v1] "+&v"(v1), [hl] "=&v"(hl), [hh] "=&v"(hh), [kl] "=&v"(kl), [kh] "=&v"(kh), [x0] "=&v"(x0), [x1] "=&v"(x1),
+          [y0] "=&v"(y0), [y1] "=&v"(y1), [m] "=&v"(m), [n] "=&v"(n), [t] "=&s"(t)
+        : [l0] "v"((u32)p00), [m0] "v"((u32)mm), [m1] "v"((u32)(mm >> 32)), [g0] "v"(g0), [g1] "v"(g1), [st] "s"(st),
+          [k0] "v"((u32)q00), [n0] "v"((u32)nn), [n1] "v"((u32)(nn >> 32)), [h0] "v"(h0), [h1] "v"(h1), [tt] "s"(tt), [k3] "n"(BORROWED)
+        : "vcc");
+    u64 X, Y, w, v;
+    asm("v_mad_i64_i32 %[X], vcc, %[m], %[k], %[x]\n\t"
+        "v_mad_i64_i32 %[Y], vcc, %[n], %[k], %[y]\n\t"
+        "v_mad_u64_u32 %[w], %[st], %[hl], -1, %[X]\n\t"
+        "v_mad_u64_u32 %[v], %[tt], %[kl], -1, %[Y]"
+        : [X] "=&v"(X), [Y] "=&v"(Y), [w] "=&v"(w), [v] "=&v"(v), [st] "=&s"(st), [tt] "=&s"(tt)
+        : [m] "v"(m), [n] "v"(n), [hl] "v"(hl), [kl] "v"(kl), [x] "v"(pack(x0, x1)), [y] "v"(pack(y0, y1)), [k] "s"(-0x55555555)
+        : "vcc");
+    if (LAZY) {
+        u32 i, j;
+        asm("s_nop 0\n\t"
+            "v_cndmask_b32_e64 %[i], 0, 1, %[st]\n\t"
+            "v_cndmask_b32_e64 %[j], 0, 1, %[tt]\n\t"
+            "v_mad_u64_u32 %[x], vcc, %[i], -1, %[w]\n\t"
+            "v_mad_u64_u32 %[y], vcc, %[j], -1, %[v]"
+            : [i] "=&v"(i), [j] "=&v"(j), [x] "=&v"(x), [y] "=v"(y)
+            : [w] "v"(w), [v] "v"(v), [st] "s"(st), [tt] "s"(tt)
+            : "vcc");
+    } else {
+        canon_tail2(w, st, x, v, tt, y);
+    }
+}
+
+// A += a b, B += c d as in mul_acc
+__device__ __forceinline__ void mul_acc2(u32 (&A)[5], u64 a, u64 b, u32 (&B)[5], u64 c, u64 d) {
+    u64 p00, mm, p11, st, cy, q00, nn, q11, tt, cz;
+    partial_products2<false>(a, b, 0, c, d, 0, p00, mm, p11, st, cy, q00, nn, q11, tt, cz);
+    u32 w1 = (u32)(p00 >> 32), v1 = (u32)(q00 >> 32), hl, hh, kl, kh;
+    u64 ca, cb, t;
+    asm("v_add_co_u32 %[w1], vcc, %[w1], %[m0]\n\t"
+        "v_add_co_u32 %[v1], %[t], %[v1], %[n0]\n\t"
+        "v_add_co_u32 %[A0], %[ca], %[A0], %[l0]\n\t"
+        "v_add_co_u32 %[B0], %[cb], %[B0], %[k0]\n\t"
+        "v_addc_co_u32 %[hl], vcc, %[g0], %[m1], vcc\n\t"
+        "v_addc_co_u32 %[kl], %[t], %[h0], %[n1], %[t]\n\t"
+        "v_addc_co_u32 %[A1], %[ca], %[A1], %[w1], %[ca]\n\t"
+        "v_addc_co_u32 %[B1], %[cb], %[B1], %[v1], %[cb]\n\t"
+        "v_addc_co_u32 %[hh], vcc, 0, %[g1], vcc\n\t"
+        "v_addc_co_u32 %[kh], %[t], 0, %[h1], %[t]\n\t"
+        "v_addc_co_u32 %[A2], %[ca], %[A2], %[hl], %[ca]\n\t"
+        "v_addc_co_u32 %[B2], %[cb], %[B2], %[kl], %[cb]\n\t"
+        "v_addc_co_u32 %[hh], vcc, 0, %[hh], %[st]\n\t"
+        "v_addc_co_u32 %[kh], vcc, 0, %[kh], %[tt]\n\t"
+        "v_addc_co_u32 %[A3], %[ca], %[A3], %[hh], %[ca]\n\t"
+        "v_addc_co_u32 %[B3], %[cb], %[B3], %[kh], %[cb]\n\t"
+        "s_nop 0\n\t"
+        "v_addc_co_u32 %[A4], vcc, 0, %[A4], %[ca]\n\t"
+        "v_addc_co_u32 %[B4], vcc, 0, %[B4], %[cb]"
+        : [w1] "+&v"(w1), [v1] "+&v"(v1), [hl] "=&v"(hl), [hh] "=&v"(hh), [kl] "=&v"(kl), [kh] "=&v"(kh), [t] "=&s"(t), [ca] "=&s"(ca), [cb] "=&s"(cb),
+          [A0] "+&v"(A[0]), [A1] "+&v"(A[1]), [A2] "+&v"(A[2]), [A3] "+&v"(A[3]), [A4] "+&v"(A[4]),
+          [B0] "+&v"(B[0]), [B1] "+&v"(B[1]), [B2] "+&v"(B[2]), [B3] "+&v"(B[3]), [B4] "+&v"(B[4])
+        : [l0] "v"((u32)p00), [m0] "v"((u32)mm), [m1] "v"((u32)(mm >> 32)), [g0] "v"((u32)p11), [g1] "v"((u32)(p11 >> 32)), [st] "s"(st),
+          [k0] "v"((u32)q00), [n0] "v"((u32)nn), [n1] "v"((u32)(nn >> 32)), [h0] "v"((u32)q11), [h1] "v"((u32)(q11 >> 32)), [tt] "s"(tt)
+        : "vcc");
+}
+
 }  // namespace dev
 #endif
 
@@ -531,6 +711,53 @@ VI_HD u64 mul_lazy(u64 a, u64 b) {
     return reduce128_lazy(lo, hi);
 }
 
+// two at once (dev::mul2 and its neighbours): x from the first operands, y from the second
+VI_HD void sub2(u64 a, u64 b, u64 &x, u64 c, u64 d, u64 &y) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    dev::sub2(a, b, x, c, d, y);
+#else
+    const u64 first = sub(a, b);
+    y = sub(c, d);
+    x = first;
+#endif
+}
+VI_HD void addc2(u64 a, u64 b, u64 &x, u64 c, u64 d, u64 &y) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    dev::addc2(a, b, x, c, d, y);
+#else
+    const u64 first = addc(a, b);
+    y = addc(c, d);
+    x = first;
+#endif
+}
+VI_HD void mul2(u64 a, u64 b, u64 &x, u64 c, u64 d, u64 &y) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    dev::mul2<false, false>(a, b, 0, x, c, d, 0, y);
+#else
+    const u64 first = mul(a, b);
+    y = mul(c, d);
+    x = first;
+#endif
+}
+VI_HD void mul_lazy2(u64 a, u64 b, u64 &x, u64 c, u64 d, u64 &y) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    dev::mul2<false, true>(a, b, 0, x, c, d, 0, y);
+#else
+    const u64 first = mul_lazy(a, b);
+    y = mul_lazy(c, d);
+    x = first;
+#endif
+}
+VI_HD void mul_add2(u64 a, u64 b, u64 e, u64 &x, u64 c, u64 d, u64 f, u64 &y) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    dev::mul2<true, false>(a, b, e, x, c, d, f, y);
+#else
+    const u64 first = mul_add(a, b, e);
+    y = mul_add(c, d, f);
+    x = first;
+#endif
+}
+
 // Sums of products kept as plain integers: five 32-bit words, reduced once at the end.
 struct Wide {
     u32 w[5];
@@ -552,6 +779,15 @@ VI_HD void wide_mul_acc(Wide &A, u64 a, u64 b) {
         A.w[i] = (u32)t;
         carry = t >> 32;
     }
+#endif
+}
+// A += a * b and B += c * d
+VI_HD void wide_mul_acc2(Wide &A, u64 a, u64 b, Wide &B, u64 c, u64 d) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    dev::mul_acc2(A.w, a, b, B.w, c, d);
+#else
+    wide_mul_acc(A, a, b);
+    wide_mul_acc(B, c, d);
 #endif
 }
 // the integer mod p: words 0..3 as a 128-bit value, word 4 weighs 2^128 = -2^32

@@ -237,6 +237,8 @@ struct SampleAcc<true> {
     __device__ __forceinline__ void zero() { gl::wide_zero(v); }
     __device__ __forceinline__ void add_product(u64 a, u64 b) { gl::wide_mul_acc(v, a, b); }
     __device__ __forceinline__ u64 value() const { return gl::wide_reduce(v); }
+    // x += a b and y += c d
+    static __device__ __forceinline__ void add_two(SampleAcc &x, u64 a, u64 b, SampleAcc &y, u64 c, u64 d) { gl::wide_mul_acc2(x.v, a, b, y.v, c, d); }
 };
 template <>
 struct SampleAcc<false> {
@@ -244,7 +246,33 @@ struct SampleAcc<false> {
     __device__ __forceinline__ void zero() { v = 0; }
     __device__ __forceinline__ void add_product(u64 a, u64 b) { v = gl::addc(v, gl::mul(a, b)); }
     __device__ __forceinline__ u64 value() const { return v; }
+    static __device__ __forceinline__ void add_two(SampleAcc &x, u64 a, u64 b, SampleAcc &y, u64 c, u64 d) {
+        u64 p, q;
+        gl::mul2(a, b, p, c, d, q);
+        gl::addc2(x.v, p, x.v, y.v, q, y.v);
+    }
 };
+
+// the same operation on N independent pairs, two at once (gl::mul2 and its neighbours)
+template <int N>
+__device__ __forceinline__ void differences(const u64 (&hi)[N], const u64 (&lo)[N], u64 (&dif)[N]) {
+#pragma unroll
+    for (int t = 0; t + 1 < N; t += 2) gl::sub2(hi[t], lo[t], dif[t], hi[t + 1], lo[t + 1], dif[t + 1]);
+    if constexpr (N & 1) dif[N - 1] = gl::sub(hi[N - 1], lo[N - 1]);
+}
+template <int N>
+__device__ __forceinline__ void sums(const u64 (&a)[N], const u64 (&b)[N], u64 (&out)[N]) {
+#pragma unroll
+    for (int t = 0; t + 1 < N; t += 2) gl::addc2(a[t], b[t], out[t], a[t + 1], b[t + 1], out[t + 1]);
+    if constexpr (N & 1) out[N - 1] = gl::addc(a[N - 1], b[N - 1]);
+}
+// lo + r (hi - lo)
+template <int N>
+__device__ __forceinline__ void folds(u64 r, const u64 (&dif)[N], const u64 (&lo)[N], u64 (&out)[N]) {
+#pragma unroll
+    for (int t = 0; t + 1 < N; t += 2) gl::mul_add2(r, dif[t], lo[t], out[t], r, dif[t + 1], lo[t + 1], out[t + 1]);
+    if constexpr (N & 1) out[N - 1] = gl::mul_add(r, dif[N - 1], lo[N - 1]);
+}
 
 // One pair (lo, hi) of every table: adds S(x) of the pair to acc[x] for x = 0..deg-1 (x = 1 left out when SKIP1)
 // and the pair's leading coefficient to acc[deg] (or S(deg) when the degree is 1), and returns the differences
@@ -255,11 +283,33 @@ __device__ __forceinline__ void eval_pair(const u64 (&lo)[NT], const u64 (&hi)[N
     constexpr int NS = FastShape<NT, SHAPE>::NS;
     constexpr bool INF = FastShape<NT, SHAPE>::INF;
     u64 cur[NT];
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-        cur[t] = lo[t];
-        dif[t] = gl::sub(hi[t], lo[t]);
+    differences(hi, lo, dif);
+    if constexpr (NT == 2) {
+        // samples two at once as well
+        constexpr int second = SHAPE == 3 ? 2 : NS - 1;
+        if (SHAPE == 3) sums(hi, dif, cur);
+        const u64 (&other)[NT] = SHAPE == 3 ? cur : dif;
+        SampleAcc<WIDE>::add_two(acc[0], lo[0], lo[1], acc[second], other[0], other[1]);
+        if (!SKIP1) acc[1].add_product(hi[0], hi[1]);
+        return;
     }
+    if constexpr (NT == 3) {
+        u64 v, w;
+        sums(hi, dif, cur);                                // S(2)
+        if (SKIP1) {
+            gl::mul_lazy2(lo[0], lo[1], v, dif[0], dif[1], w);
+            SampleAcc<WIDE>::add_two(acc[0], v, lo[2], acc[3], w, dif[2]);
+            acc[2].add_product(gl::mul_lazy(cur[0], cur[1]), cur[2]);
+        } else {
+            gl::mul_lazy2(lo[0], lo[1], v, hi[0], hi[1], w);
+            SampleAcc<WIDE>::add_two(acc[0], v, lo[2], acc[1], w, hi[2]);
+            gl::mul_lazy2(cur[0], cur[1], v, dif[0], dif[1], w);
+            SampleAcc<WIDE>::add_two(acc[2], v, cur[2], acc[3], w, dif[2]);
+        }
+        return;
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t) cur[t] = lo[t];
 #pragma unroll
     for (int x = 0; x < NS; ++x) {
         const bool at_inf = INF && x == NS - 1;
@@ -268,8 +318,6 @@ __device__ __forceinline__ void eval_pair(const u64 (&lo)[NT], const u64 (&hi)[N
                 // eq (a b + c): the c term has degree 2 and does not reach the leading coefficient
                 if (at_inf) acc[x].add_product(gl::mul_lazy(dif[1], dif[2]), dif[0]);
                 else acc[x].add_product(gl::mul_add_lazy(cur[1], cur[2], cur[3]), cur[0]);
-            } else if constexpr (SHAPE == 3) {
-                if (!at_inf) acc[x].add_product(cur[0], cur[1]);
             } else if constexpr (NT == 1) {
                 acc[x].add_product(cur[0], 1);
             } else {
@@ -385,30 +433,25 @@ __device__ __forceinline__ void three_rounds_from(Load load, u64 r0, u64 r1, u64
                                                   SampleAcc<true> (&acc1)[FastShape<NT, SHAPE>::NS], SampleAcc<true> (&acc2)[FastShape<NT, SHAPE>::NS],
                                                   u64 (&folded)[NT]) {
     // the scheduler is kept from interleaving the pairs: each one's temporaries die before the next starts
-    u64 lo[NT], hi[NT], dif[NT], v[NT][4];
+    u64 lo[NT], hi[NT], dif[NT], v[4][NT];
     static_for<0, 4>([&](auto c_) {
         constexpr int c = decltype(c_)::value;
         VI_SCHED_FENCE();
         load(c_, lo, hi);
         eval_pair<NT, SHAPE, !ONE, true>(lo, hi, dif, acc0);
-#pragma unroll
-        for (int t = 0; t < NT; ++t) v[t][c] = gl::mul_add(r0, dif[t], lo[t]);
+        folds(r0, dif, lo, v[c]);
     });
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
         VI_SCHED_FENCE();
 #pragma unroll
-        for (int t = 0; t < NT; ++t) { lo[t] = v[t][c]; hi[t] = v[t][c + 2]; }
+        for (int t = 0; t < NT; ++t) { lo[t] = v[c][t]; hi[t] = v[c + 2][t]; }
         eval_pair<NT, SHAPE, true, true>(lo, hi, dif, acc1);
-#pragma unroll
-        for (int t = 0; t < NT; ++t) v[t][c] = gl::mul_add(r1, dif[t], lo[t]);
+        folds(r1, dif, lo, v[c]);
     }
     VI_SCHED_FENCE();
-#pragma unroll
-    for (int t = 0; t < NT; ++t) { lo[t] = v[t][0]; hi[t] = v[t][1]; }
-    eval_pair<NT, SHAPE, true, true>(lo, hi, dif, acc2);
-#pragma unroll
-    for (int t = 0; t < NT; ++t) folded[t] = gl::mul_add(r2, dif[t], lo[t]);
+    eval_pair<NT, SHAPE, true, true>(v[0], v[1], dif, acc2);
+    folds(r2, dif, v[0], folded);
 }
 
 // the same of entries in registers, v[t][c] = entry i + c cols
@@ -638,8 +681,9 @@ __global__ __launch_bounds__(TAIL_THREADS) void k_tail(const FastDesc D, i64 siz
             }
             eval_pair<NT, SHAPE, !ONE, false>(lo, hi, dif, acc);
             if (h > 1) {
+                folds(r, dif, lo, lo);
 #pragma unroll
-                for (int t = 0; t < NT; ++t) tab[t][i] = gl::mul_add(r, dif[t], lo[t]);
+                for (int t = 0; t < NT; ++t) tab[t][i] = lo[t];
             }
         }
         leave_sums();
@@ -654,8 +698,9 @@ __global__ __launch_bounds__(TAIL_THREADS) void k_tail(const FastDesc D, i64 siz
 #pragma unroll
             for (int t = 0; t < NT; ++t) { lo[t] = tab[t][i]; hi[t] = tab[t][h + i]; }
             eval_pair<NT, SHAPE, true, false>(lo, hi, dif, acc);
+            folds(r, dif, lo, lo);
 #pragma unroll
-            for (int t = 0; t < NT; ++t) tab[t][i] = gl::mul_add(r, dif[t], lo[t]);
+            for (int t = 0; t < NT; ++t) tab[t][i] = lo[t];
         }
         leave_sums();
     }
@@ -667,12 +712,14 @@ __global__ __launch_bounds__(TAIL_THREADS) void k_tail(const FastDesc D, i64 siz
         for (int t = 0; t < NT; ++t) val[t] = (lane < 2 * h) ? tab[t][lane] : 0;
         for (; h >= 1; h >>= 1) {
             const u64 r = C.r[++k];
+            u64 up[NT];
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
                 if (lane < 2 * h) small[t][2 * h + lane] = val[t];
-                const u64 up = __shfl_down(val[t], (unsigned)h, 64);       // lanes past the pairs compute on what they get and drop it
-                val[t] = gl::mul_add(r, gl::sub(up, val[t]), val[t]);
+                up[t] = __shfl_down(val[t], (unsigned)h, 64);              // lanes past the pairs compute on what they get and drop it
             }
+            differences(up, val, up);
+            folds(r, up, val, val);
         }
     }
     __syncthreads();

@@ -137,8 +137,9 @@ __device__ __forceinline__ void lane_round(u64 (&v)[3][8], u64 r, u64 (&total)[4
 #pragma unroll
         for (int t = 0; t < 3; ++t) { lo[t] = v[t][c]; hi[t] = v[t][c + P]; }
         eval_pair<3, 1, !ONE, false>(lo, hi, dif, acc);
+        folds(r, dif, lo, lo);
 #pragma unroll
-        for (int t = 0; t < 3; ++t) v[t][c] = gl::mul_add(r, dif[t], lo[t]);
+        for (int t = 0; t < 3; ++t) v[t][c] = lo[t];
     }
 #pragma unroll
     for (int x = 0; x < 4; ++x) total[x] = acc[x].v;
@@ -198,8 +199,9 @@ __global__ __launch_bounds__(BLOCK) void k_sum_tail(const SumDesc D, int size, c
                 hi[t] = __shfl_down(v[t][0], (unsigned)h, 64);         // lanes past the pairs compute on what they get and drop it
             }
             eval_pair<3, 1, !ONE, false>(lo, hi, dif, acc);
+            folds(C.r[level], dif, lo, lo);
 #pragma unroll
-            for (int t = 0; t < 3; ++t) v[t][0] = gl::mul_add(C.r[level], dif[t], lo[t]);
+            for (int t = 0; t < 3; ++t) v[t][0] = lo[t];
 #pragma unroll
             for (int x = 0; x < 4; ++x) total[8 - level][x] = lane < h ? acc[x].v : 0;
         }
