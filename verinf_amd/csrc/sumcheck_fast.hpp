@@ -470,13 +470,20 @@ __device__ __forceinline__ void three_rounds(const u64 (&v)[NT][8], u64 r0, u64 
 // 64 words at src into LDS, by one wavefront and without a register in between; src and dst are the same for all its lanes.  Two
 // loads of four bytes a lane, which ask for no more than the alignment of a word.  The compiler does not wait for them: loads_arrived()
 // does.  M0 has its value back afterwards (the compiler does not accept it in a list of clobbered registers).
+// ONCE: words that nothing reads again, with the streaming hint.
+template <bool ONCE>
 __device__ __forceinline__ void words_to_lds(const u64 *src, u64 *dst, int lane) {
 #ifdef __HIP_DEVICE_COMPILE__
     const u32 at = __builtin_amdgcn_readfirstlane((u32)(uintptr_t)(__attribute__((address_space(3))) u64 *)dst);
     u32 m0;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %3, %5\n\t"
-                 "s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %4, %5\n\ts_mov_b32 m0, %0"
-                 : "=&s"(m0) : "s"(at), "s"(at + 256), "v"((u32)lane * 4), "v"((u32)lane * 4 + 256), "s"(src) : "memory");
+    if (ONCE)
+        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %3, %5 nt\n\t"
+                     "s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %4, %5 nt\n\ts_mov_b32 m0, %0"
+                     : "=&s"(m0) : "s"(at), "s"(at + 256), "v"((u32)lane * 4), "v"((u32)lane * 4 + 256), "s"(src) : "memory");
+    else
+        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %3, %5\n\t"
+                     "s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %4, %5\n\ts_mov_b32 m0, %0"
+                     : "=&s"(m0) : "s"(at), "s"(at + 256), "v"((u32)lane * 4), "v"((u32)lane * 4 + 256), "s"(src) : "memory");
 #else
     dst[lane] = src[lane];
 #endif
@@ -546,7 +553,10 @@ __global__ __launch_bounds__(BLOCK) void k_pass3(const FastDesc D, i64 cols, u64
 // after 450 (three tables of 2^26), alone by then; and a wavefront's loads wait for its arithmetic.  So a workgroup has all the wavefronts
 // of a CU, which take pieces of 64 columns from a counter in LDS, and a piece's entries are on their way into LDS while
 // the piece before it is worked on (18 of 24 words a lane for three tables; the last pair's go to registers, as they have three pairs' time).
-// First pass over three tables of 2^26 424 -> 384 us (resident grid with equal shares and this staging: 436); its proof 559 -> 512.
+// Where the pieces lie decides the rate of memory: 24 streams of three tables of 2^26 and an eighth as much written take 384 us with
+// sixteen pieces of a workgroup in a row, 346 with the workgroups' pieces beside each other, 315 with the streaming hint on the loads
+// besides (without the writes 290, 256 and 224: 7.2 TB/s; one stream 5.9).  The proof over them 559 -> 475 us; with equal shares of the
+// columns and this staging 543, with pieces in rows of sixteen 510.
 template <int NT>
 struct LongPass {
     static constexpr int THREADS = NT <= 3 ? 1024 : 768;               // 128 and 168 registers
@@ -576,12 +586,12 @@ __global__ __launch_bounds__(LongPass<NT>::THREADS) void k_pass3_long(const Fast
         for (int t = 0; t < NT; ++t)
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
-                words_to_lds(D.src[t] + first + c * cols, mine[2 * (3 * t + c)], lane);
-                words_to_lds(D.src[t] + first + (c + 4) * cols, mine[2 * (3 * t + c) + 1], lane);
+                words_to_lds<FIRST>(D.src[t] + first + c * cols, mine[2 * (3 * t + c)], lane);
+                words_to_lds<FIRST>(D.src[t] + first + (c + 4) * cols, mine[2 * (3 * t + c) + 1], lane);
             }
     };
-    // piece j of the workgroup: sixteen in a row, then its next sixteen
-    auto piece = [&](int j) { return ((i64)(j >> 4) * gridDim.x + blockIdx.x) * 1024 + (j & 15) * 64; };
+    // piece j of the workgroup, the workgroups' pieces beside each other
+    auto piece = [&](int j) { return ((i64)j * gridDim.x + blockIdx.x) * 64; };
     i64 first = piece(wave), following = 0;
     if (first < cols) fetch(first);
     for (; first < cols; first = following) {
@@ -589,8 +599,9 @@ __global__ __launch_bounds__(LongPass<NT>::THREADS) void k_pass3_long(const Fast
         u64 last[NT][2];
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
-            last[t][0] = D.src[t][i + 3 * cols];
-            last[t][1] = D.src[t][i + 7 * cols];
+            const u64 *p = D.src[t] + i + 3 * cols, *q = D.src[t] + i + 7 * cols;
+            last[t][0] = FIRST ? __builtin_nontemporal_load(p) : *p;
+            last[t][1] = FIRST ? __builtin_nontemporal_load(q) : *q;
         }
         loads_arrived<2 * NT>();
         auto load = [&](auto c_, u64 (&lo)[NT], u64 (&hi)[NT]) {
