@@ -144,8 +144,12 @@ __device__ __forceinline__ void count(const u64 *__restrict__ x, i64 lo, i64 hi,
     constexpr int UN = HALF ? 8 : 4;           // look-ups of a thread in flight
     for (i64 i0 = lo + threadIdx.x; i0 < hi; i0 += UN * COUNT_THREADS) {
         u64 v[UN];
+        // requested together: as loads behind a test each they were waited for one by one.  In the place of those past the end the first.
+        // 2^24 look-ups in 2^20 entries 337 -> 295 us, 1.5 M in 2^20 51.7 -> 48.  (Those of the next trip as well: 253 and 44.7, but in tables of
+        // one slice 3 % more, 1.5 M in 2^16 17.9 and 18.5.)
 #pragma unroll
-        for (int u = 0; u < UN; ++u) v[u] = i0 + u * COUNT_THREADS < hi ? x[i0 + u * COUNT_THREADS] : 0;
+        for (int u = 0; u < UN; ++u) v[u] = x[i0 + u * COUNT_THREADS < hi ? i0 + u * COUNT_THREADS : lo];
+        VI_SCHED_FENCE();
         u32 times[UN];
 #pragma unroll
         for (int u = 0; u < UN; ++u) times[u] = i0 + u * COUNT_THREADS < hi ? 1 : 0;
