@@ -150,7 +150,13 @@ __global__ __launch_bounds__(BLOCK) void k_probe(int op, const u64 *a, const u64
 // inverts (1.5 M elements 13.6 -> 12.4 us, 16 M 89 -> 71).  Zeros are taken out of the product and map to zero, so every output
 // equals the Fermat power a^(p-2) of the reference kernel (prover/cuda_primitives.py:289-303).
 //
-// Elements of a thread: four while the chip has SIMDs to spare, then eight, then twelve, which share an inversion (us with 4, 8 and 12:
+// A call lasts as long as a thread's chain of products, up to a few million elements; beyond that VALU issue.  The thread's
+// elements run as two halves side by side and what feeds another product is only reduced to a congruent word: us per call in a
+// queue, one half and canonical words -> now: 200000 elements 8.0 -> 6.8, 700001 9.4 -> 8.3, 1.5 M 12.0 -> 10.5, 6 M 30.0 -> 26.6,
+// 16 M 71.0 -> 62.3 (one inversion to an element, lazily reduced words alone: 100000 7.5 -> 6.6).
+//
+// Elements of a thread: four while the chip has SIMDs to spare, then eight, then twelve, which share an inversion (us with 4, 8 and 12,
+// measured with one half:
 // 300000 8.7, 9.7, 10.7; 700001 9.6, 10.9, 11.3; 1.5 M 13.3, 12.4, 13.3; 3 M 21.8, 22.0, 17.5; 6 M 33.6, 32.4, 29.4; 16 M 78.6, 70.8, 68.0).
 constexpr int INV_THREADS = 256;
 
@@ -182,35 +188,45 @@ __global__ __launch_bounds__(INV_THREADS) void k_inv_batched(const u64 *a, u64 *
         if (v == 0) { zero |= 1u << j; v = 1; }
         x[j] = v;
     }
+    // two halves of the elements with interleaved products (gl::mul2)
+    constexpr int H = INV_E / 2;
     pre[0] = x[0];
+    pre[H] = x[H];
 #pragma unroll
-    for (int j = 1; j < INV_E; ++j) pre[j] = gl::mul(pre[j - 1], x[j]);
-    prod[tid] = pre[INV_E - 1];
+    for (int j = 1; j < H; ++j) gl::mul_lazy2(pre[j - 1], x[j], pre[j], pre[H + j - 1], x[H + j], pre[H + j]);
+    prod[tid] = gl::mul_lazy(pre[H - 1], pre[INV_E - 1]);
     __syncthreads();
     if (tid < 64) {
-        constexpr int PER = INV_THREADS / 64;
-        u64 y[PER], before[PER];
+        static_assert(INV_THREADS == 256, "four products to a lane");
+        u64 y[4], low, high, r[4];
 #pragma unroll
-        for (int j = 0; j < PER; ++j) y[j] = prod[tid + 64 * j];
-        before[0] = y[0];
+        for (int j = 0; j < 4; ++j) y[j] = prod[tid + 64 * j];
+        gl::mul_lazy2(y[0], y[1], low, y[2], y[3], high);
+        const u64 all = gl::inv(gl::mul_lazy(low, high));
+        u64 a01, a23;                          // 1 / (y0 y1), 1 / (y2 y3)
+        gl::mul_lazy2(all, high, a01, all, low, a23);
+        gl::mul_lazy2(a01, y[1], r[0], a01, y[0], r[1]);
+        gl::mul_lazy2(a23, y[3], r[2], a23, y[2], r[3]);
 #pragma unroll
-        for (int j = 1; j < PER; ++j) before[j] = gl::mul(before[j - 1], y[j]);
-        u64 acc = gl::inv(before[PER - 1]);
-#pragma unroll
-        for (int j = PER - 1; j >= 0; --j) {
-            prod[tid + 64 * j] = j ? gl::mul(acc, before[j - 1]) : acc;
-            if (j) acc = gl::mul(acc, y[j]);
-        }
+        for (int j = 0; j < 4; ++j) prod[tid + 64 * j] = r[j];
     }
     __syncthreads();
-    u64 acc = prod[tid];
-#pragma unroll
-    for (int j = INV_E - 1; j >= 0; --j) {
-        const u64 r = j ? gl::mul(acc, pre[j - 1]) : acc;
-        if (j) acc = gl::mul(acc, x[j]);
+    u64 low = prod[tid], high;
+    gl::mul_lazy2(low, pre[INV_E - 1], low, low, pre[H - 1], high);            // 1 / (x0 .. x(H-1)) and 1 / (xH ..)
+    auto put = [&](int j, u64 r) {
         const i64 i = (i64)j * groups + g;
         if (g < groups && i < n) out[i] = (zero >> j) & 1 ? 0 : r;
+    };
+#pragma unroll
+    for (int j = H - 1; j >= 1; --j) {
+        u64 r, q;
+        gl::mul2(low, pre[j - 1], r, high, pre[H + j - 1], q);
+        gl::mul_lazy2(low, x[j], low, high, x[H + j], high);
+        put(j, r);
+        put(H + j, q);
     }
+    put(0, gl::canon(low));
+    put(H, gl::canon(high));
 }
 
 __global__ __launch_bounds__(BLOCK) void k_axpy(u64 *y, u64 alpha, const u64 *x, i64 n) {

@@ -205,19 +205,27 @@ __device__ __forceinline__ u64 mul(u64 a, u64 b) {
 }
 
 // the reduction of reduce_words() without its last step: a 64-bit word congruent to the value, not necessarily
-// below p (two instructions instead of three after the multiply-add); good as an operand of a further product
+// below p; good as an operand of a further product.  The borrow of lo - hh and the carry of + hl (2^32 - 1) weigh -2^64 and 2^64: where one
+// of them is set, 2^32 - 1 comes off or on at the end (one correction where reduce_words() has two, and a shorter chain).  The word cannot
+// wrap by that: with the carry alone it is at most 2^64 - 2^33, with the borrow alone at least 2^64 - 2^32.
 __device__ __forceinline__ u64 reduce_words_lazy(u32 l0, u32 l1, u32 hl, u32 hh, u64 bin) {
-    u64 st, r;
-    const u64 w = reduce_words_open(l0, l1, hl, hh, bin, &st);
-    // the sum wrapped past 2^64 (st): add 2^64 mod p = 2^32 - 1; it cannot wrap again (w <= 2^64 - 2^33 then)
-    u32 e;
-    asm("s_nop 1\n\t"
-        "v_cndmask_b32_e64 %[e], 0, 1, %[st]\n\t"
-        "v_mad_u64_u32 %[r], vcc, %[e], -1, %[w]"
-        : [e] "=&v"(e), [r] "=&v"(r)
-        : [w] "v"(w), [st] "s"(st)
+    u32 x0, x1, m;
+    u64 bo, st, w;
+    asm("v_subb_co_u32 %[x0], vcc, %[l0], %[hh], %[bin]\n\t"
+        "s_nop 1\n\t"
+        "v_subbrev_co_u32 %[x1], %[bo], 0, %[l1], vcc"
+        : [x0] "=&v"(x0), [x1] "=v"(x1), [bo] "=s"(bo)
+        : [l0] "v"(l0), [l1] "v"(l1), [hh] "v"(hh), [bin] "s"(bin)
         : "vcc");
-    return r;
+    asm("v_mad_u64_u32 %[w], %[st], %[hl], -1, %[x]\n\t"
+        "s_xor_b64 vcc, %[bo], %[st]\n\t"
+        "s_nop 0\n\t"
+        "v_cndmask_b32_e64 %[m], %[k3], -%[k3], %[st]\n\t"
+        "v_cndmask_b32_e64 %[m], 0, %[m], vcc"
+        : [w] "=&v"(w), [m] "=&v"(m), [st] "=&s"(st)
+        : [hl] "v"(hl), [x] "v"(pack(x0, x1)), [bo] "s"(bo), [k3] "n"(BORROWED)
+        : "vcc", "scc");
+    return minus_eps(w, m);
 }
 
 // the four partial products of a * b (+ c, a 64-bit addend of the lowest one) as the words l0 l1 hl hh of the
@@ -507,7 +515,7 @@ __device__ __forceinline__ void mul2(u64 a, u64 b, u64 e, u64 &x, u64 c, u64 d, 
             : "vcc");
     }
     u32 w1 = (u32)(p00 >> 32), v1 = (u32)(q00 >> 32), hl, hh, kl, kh, x0, x1, y0, y1, m, n;
-    u64 t;
+    u64 t, bo;
     asm("v_add_co_u32 %[w1], vcc, %[w1], %[m0]\n\t"
         "v_add_co_u32 %[v1], %[t], %[v1], %[n0]\n\t"
         "s_nop 0\n\t"
@@ -518,36 +526,41 @@ __device__ __forceinline__ void mul2(u64 a, u64 b, u64 e, u64 &x, u64 c, u64 d, 
         "v_subb_co_u32 %[x0], vcc, %[l0], %[hh], %[st]\n\t"
         "v_addc_co_u32 %[kh], %[t], 0, %[h1], %[t]\n\t"
         "v_subb_co_u32 %[y0], %[t], %[k0], %[kh], %[tt]\n\t"
-        "v_subbrev_co_u32 %[x1], vcc, 0, %[w1], vcc\n\t"
+        "v_subbrev_co_u32 %[x1], %[bo], 0, %[w1], vcc\n\t"
         "s_nop 0\n\t"
-        "v_subbrev_co_u32 %[y1], %[t], 0, %[v1], %[t]\n\t"
-        "v_cndmask_b32_e64 %[m], 0, %[k3], vcc\n\t"
-        "s_nop 0\n\t"
-        "v_cndmask_b32_e64 %[n], 0, %[k3], %[t]"
+        "v_subbrev_co_u32 %[y1], %[t], 0, %[v1], %[t]"
         : [w1] "+&v"(w1), [v1] "+&v"(v1), [hl] "=&v"(hl), [hh] "=&v"(hh), [kl] "=&v"(kl), [kh] "=&v"(kh), [x0] "=&v"(x0), [x1] "=&v"(x1),
-          [y0] "=&v"(y0), [y1] "=&v"(y1), [m] "=&v"(m), [n] "=&v"(n), [t] "=&s"(t)
+          [y0] "=&v"(y0), [y1] "=&v"(y1), [t] "=&s"(t), [bo] "=&s"(bo)
         : [l0] "v"((u32)p00), [m0] "v"((u32)mm), [m1] "v"((u32)(mm >> 32)), [g0] "v"(g0), [g1] "v"(g1), [st] "s"(st),
-          [k0] "v"((u32)q00), [n0] "v"((u32)nn), [n1] "v"((u32)(nn >> 32)), [h0] "v"(h0), [h1] "v"(h1), [tt] "s"(tt), [k3] "n"(BORROWED)
+          [k0] "v"((u32)q00), [n0] "v"((u32)nn), [n1] "v"((u32)(nn >> 32)), [h0] "v"(h0), [h1] "v"(h1), [tt] "s"(tt)
         : "vcc");
-    u64 X, Y, w, v;
-    asm("v_mad_i64_i32 %[X], vcc, %[m], %[k], %[x]\n\t"
-        "v_mad_i64_i32 %[Y], vcc, %[n], %[k], %[y]\n\t"
-        "v_mad_u64_u32 %[w], %[st], %[hl], -1, %[X]\n\t"
-        "v_mad_u64_u32 %[v], %[tt], %[kl], -1, %[Y]"
-        : [X] "=&v"(X), [Y] "=&v"(Y), [w] "=&v"(w), [v] "=&v"(v), [st] "=&s"(st), [tt] "=&s"(tt)
-        : [m] "v"(m), [n] "v"(n), [hl] "v"(hl), [kl] "v"(kl), [x] "v"(pack(x0, x1)), [y] "v"(pack(y0, y1)), [k] "s"(-0x55555555)
-        : "vcc");
+    u64 w, v;
     if (LAZY) {
-        u32 i, j;
-        asm("s_nop 0\n\t"
-            "v_cndmask_b32_e64 %[i], 0, 1, %[st]\n\t"
-            "v_cndmask_b32_e64 %[j], 0, 1, %[tt]\n\t"
-            "v_mad_u64_u32 %[x], vcc, %[i], -1, %[w]\n\t"
-            "v_mad_u64_u32 %[y], vcc, %[j], -1, %[v]"
-            : [i] "=&v"(i), [j] "=&v"(j), [x] "=&v"(x), [y] "=v"(y)
-            : [w] "v"(w), [v] "v"(v), [st] "s"(st), [tt] "s"(tt)
-            : "vcc");
+        asm("v_mad_u64_u32 %[w], %[st], %[hl], -1, %[x]\n\t"
+            "v_mad_u64_u32 %[v], %[tt], %[kl], -1, %[y]\n\t"
+            "s_xor_b64 %[bo], %[bo], %[st]\n\t"
+            "s_xor_b64 %[t], %[t], %[tt]\n\t"
+            "v_cndmask_b32_e64 %[m], %[k3], -%[k3], %[st]\n\t"
+            "v_cndmask_b32_e64 %[n], %[k3], -%[k3], %[tt]\n\t"
+            "v_cndmask_b32_e64 %[m], 0, %[m], %[bo]\n\t"
+            "v_cndmask_b32_e64 %[n], 0, %[n], %[t]"
+            : [w] "=&v"(w), [v] "=&v"(v), [m] "=&v"(m), [n] "=&v"(n), [st] "=&s"(st), [tt] "=&s"(tt), [bo] "+&s"(bo), [t] "+&s"(t)
+            : [hl] "v"(hl), [kl] "v"(kl), [x] "v"(pack(x0, x1)), [y] "v"(pack(y0, y1)), [k3] "n"(BORROWED)
+            : "scc");
+        x = minus_eps(w, m);
+        y = minus_eps(v, n);
     } else {
+        u64 X, Y;
+        asm("s_nop 0\n\t"
+            "v_cndmask_b32_e64 %[m], 0, %[k3], %[bo]\n\t"
+            "v_cndmask_b32_e64 %[n], 0, %[k3], %[t]\n\t"
+            "v_mad_i64_i32 %[X], vcc, %[m], %[k], %[x]\n\t"
+            "v_mad_i64_i32 %[Y], vcc, %[n], %[k], %[y]\n\t"
+            "v_mad_u64_u32 %[w], %[st], %[hl], -1, %[X]\n\t"
+            "v_mad_u64_u32 %[v], %[tt], %[kl], -1, %[Y]"
+            : [X] "=&v"(X), [Y] "=&v"(Y), [w] "=&v"(w), [v] "=&v"(v), [m] "=&v"(m), [n] "=&v"(n), [st] "=&s"(st), [tt] "=&s"(tt)
+            : [bo] "s"(bo), [t] "s"(t), [hl] "v"(hl), [kl] "v"(kl), [x] "v"(pack(x0, x1)), [y] "v"(pack(y0, y1)), [k3] "n"(BORROWED), [k] "s"(-0x55555555)
+            : "vcc");
         canon_tail2(w, st, x, v, tt, y);
     }
 }
