@@ -70,9 +70,10 @@ template <int A2, bool INV>
 void run_fast(const PassArgs &A_in) {
     PassArgs A = A_in;
     A.uniform = (g_allow_uniform && pass_uniform(A, &A.n1_valid)) ? 1 : 0;
-    if (A.uniform && A.is_final && A.ndig == 0) {          // the launcher's choice of the whole-tile form
-        ++g_single_uniform_runs;
-        run_fast_u<A2, INV, true, false, true>(A);
+    if (rows_single_pass(A)) {                             // the launcher's choice of the form for rows
+        g_single_uniform_runs += A.uniform;
+        if (A.uniform) run_fast_u<A2, INV, true, false, true>(A);
+        else run_fast_u<A2, INV, false, false, true>(A);
         return;
     }
     if (INV && A.uniform && g_allow_half && upper_half_zero(A)) { ++g_half_runs; run_fast_u<A2, INV, true, true>(A); }
@@ -141,10 +142,10 @@ void run_row(const PassArgs &P0, const PassArgs &P1_in) {
 // runs passes[q] (and passes[q + 1] with it when the two fuse); returns how many passes it consumed
 int run_passes_at(const std::vector<PassArgs> &passes, size_t q);
 
-template <bool INV, bool UNI>
+template <bool INV, bool UNI, bool SGL = UNI>
 void run_512_u(const PassArgs &A) {
     i64 tiles = pass_tiles(A);
-    std::vector<u64> lds(UNI ? SglLds<5>::WORDS : fast_lds_words(A.a));
+    std::vector<u64> lds(SGL ? SglLds<5>::WORDS : fast_lds_words(A.a));
     std::vector<u64> regs((size_t)NTHREADS * 16);
     std::vector<u32> oks(NTHREADS);
     for (i64 tile = 0; tile < tiles; ++tile) {
@@ -153,10 +154,10 @@ void run_512_u(const PassArgs &A) {
         for (int tid = 0; tid < NTHREADS; ++tid) {
             u64 pw[16] = {};
             if (A.pre) fast_pre_load<5, false>(A, tile, tid, 0, pw);
-            fast_stage1<5, INV, false, false, UNI>(A, tile, tid, 0, oks[tid], *reinterpret_cast<const u64(*)[16]>(&regs[(size_t)tid * 16]), pw,
+            fast_stage1<5, INV, false, false, SGL>(A, tile, tid, 0, oks[tid], *reinterpret_cast<const u64(*)[16]>(&regs[(size_t)tid * 16]), pw,
                                                    A.twi, lds.data());
         }
-        for (int tid = 0; tid < NTHREADS; ++tid) fast_stage2_512<INV, UNI>(A, tile, tid, lds.data());
+        for (int tid = 0; tid < NTHREADS; ++tid) fast_stage2_512<INV, UNI, SGL>(A, tile, tid, lds.data());
     }
 }
 
@@ -168,6 +169,7 @@ void run_512(const PassArgs &A_in) {
     A.uniform = (g_allow_uniform && pass_uniform(A, &A.n1_valid)) ? 1 : 0;
     if (A.uniform) ++g_single_uniform_runs;
     if (A.uniform) run_512_u<INV, true>(A);
+    else if (rows_single_pass(A)) run_512_u<INV, false, true>(A);
     else run_512_u<INV, false>(A);
 }
 

@@ -145,7 +145,7 @@ def test_short_rows_in_one_launch(emu, logn, m):
 def test_single_pass_rows_in_whole_tiles(emu, logn, m, whole):
     """A transform of at most 512 points is one pass over tiles of 4096 / n rows.  When the batch is a whole number of
     tiles (and the rows are contiguous) the tiles are addressed through scalar bases; a batch that is not keeps the
-    per-element path.  Both against the oracle, forward and inverse, with words at and above p in the input."""
+    per-element addressing.  Both against the oracle, forward and inverse, with words at and above p in the input."""
     a = _rand((m, 1 << logn), 1300 + 17 * logn + m)
     raw = a.copy()
     raw[m - 1, -3:] = np.array([P, P + 7, (1 << 64) - 1], dtype=np.uint64)

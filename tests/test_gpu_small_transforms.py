@@ -86,6 +86,38 @@ def test_larger_batches(cp, logk, log_rho, m):
     assert np.array_equal(to_np(code), got)
 
 
+@pytest.mark.parametrize("logk", range(5, 10))
+@pytest.mark.parametrize("log_rho", range(5))
+def test_passes_over_short_rows_in_parts_of_tiles(cp, logk, log_rho):
+    """Batches beyond the single launch whose last tile of 4096 words holds one row or lacks one, from rows of any width and stride:
+    against the single launch over slices of the batch, and the last rows against the oracle."""
+    K, N = 1 << logk, 1 << (logk + log_rho)
+    tile = max(1, 4096 // N)
+    for m in ((5 << 20) // 2 // N // tile * tile + 1, (3 << 20) // N // tile * tile - 1):
+        for w in (K, K - 3, K // 2 + 1):
+            a = torch.randint(-(1 << 63), (1 << 63) - 1, (m, w + 5), dtype=torch.int64, device="cuda",
+                              generator=torch.Generator(device="cuda").manual_seed(m + w)).view(torch.uint64)
+            src = a[:, :w]
+            coeffs, code = cp.coset_lde_with_coeffs(src, K, N)
+            assert torch.equal(cp.coset_lde(src, K, N), code)
+            assert torch.equal(cp.coset_extend(coeffs, K, N), code)
+            step = (1 << 18) // N
+            for i in range(0, m, step):
+                some, want = cp.coset_lde_with_coeffs(src[i:i + step], K, N)
+                assert torch.equal(coeffs[i:i + step], some) and torch.equal(code[i:i + step], want), (m, w, i)
+            words = to_np(src[m - 2:].contiguous()) % np.uint64(P)
+            assert np.array_equal(to_np(code[m - 2:]), O.coset_lde_rows(np.ascontiguousarray(words), K, N, 7))
+        rows = torch.randint(-(1 << 63), (1 << 63) - 1, (m << log_rho, K), dtype=torch.int64, device="cuda").view(torch.uint64)[:-1]
+        for transform in (cp.ntt_forward_batched, cp.ntt_inverse_batched):
+            whole = rows.clone()
+            transform(whole)
+            step = (1 << 18) // K
+            for i in range(0, rows.shape[0], step):
+                some = rows[i:i + step].clone()
+                transform(some)
+                assert torch.equal(whole[i:i + step], some), (m, i)
+
+
 @pytest.mark.parametrize("logn", range(12, 21))
 def test_transforms_of_longer_rows(cp, logn):
     """Few rows (two or three launches of four points per thread) against the oracle and against a batch beyond them."""

@@ -52,12 +52,12 @@ __global__ __launch_bounds__(NTHREADS) void k_ntt_pass(const PassArgs A) {
 // UNI: compiled for passes whose tiles are all addressed by scalar bases plus 32-bit thread offsets (pass_uniform).
 // HALF: the first pass over source rows at most half as wide as the transform (upper_half_zero): eight of a thread's
 // sixteen inputs are zero, so they are not loaded and the first butterfly level of stage 1 is skipped.
-// SGL: a single-pass transform over whole tiles of contiguous rows (pass_uniform): stage 2 stores along output rows.
+// SGL: a single-pass transform of rows (rows_single_pass): stage 2 stores along output rows.
 template <int A2, bool INV, bool FIN, bool UNI, bool HALF = false, bool SGL = false>
 __global__ __launch_bounds__(NTHREADS, 4) void k_ntt_fast(const PassArgs A_in) {
     PassArgs A = A_in;
     if (FIN) A.is_final = 1;
-    static_assert(!SGL || (FIN && UNI && !HALF), "whole-tile single-pass transforms are uniform final passes");
+    static_assert(!SGL || (FIN && !HALF), "single-pass transforms are final passes");
     __shared__ u64 lds[SGL ? SglLds<A2>::WORDS : TILE + (16 << A2)];
     __shared__ u64 twi[16 << A2];
     const int tid = threadIdx.x;
@@ -119,12 +119,12 @@ __global__ __launch_bounds__(NTHREADS, 4) void k_ntt_fast(const PassArgs A_in) {
 
 
 // 512-point rows: one pass, 16 x 32 (fast_stage2_512); eight rows (or row-coset pairs) per workgroup
-template <bool INV, bool UNI>
+template <bool INV, bool UNI, bool SGL = UNI>
 __global__ __launch_bounds__(NTHREADS, 4) void k_ntt_512(const PassArgs A_in) {
     PassArgs A = A_in;
     A.is_final = 1;
     constexpr int A2 = 5;
-    __shared__ u64 lds[UNI ? SglLds<A2>::WORDS : TILE + (16 << A2)];
+    __shared__ u64 lds[SGL ? SglLds<A2>::WORDS : TILE + (16 << A2)];
     __shared__ u64 twi[16 << A2];
     const int tid = threadIdx.x;
     const i64 tile = blockIdx.x;
@@ -138,9 +138,9 @@ __global__ __launch_bounds__(NTHREADS, 4) void k_ntt_512(const PassArgs A_in) {
 #pragma unroll
     for (int i = 0; i < 2; ++i) twi[twi_slot<A2, true>((tid + i * NTHREADS) >> 4, (tid + i * NTHREADS) & 15)] = tw_mine[i];
     __syncthreads();
-    fast_stage1<A2, INV, false, true, UNI>(A, tile, tid, 0, ok, reg, pw, twi, lds);
+    fast_stage1<A2, INV, false, true, SGL>(A, tile, tid, 0, ok, reg, pw, twi, lds);
     __syncthreads();
-    fast_stage2_512<INV, UNI>(A, tile, tid, lds);
+    fast_stage2_512<INV, UNI, SGL>(A, tile, tid, lds);
 }
 
 // Rows of 2^10 .. 2^12 points: the whole transform in one launch (row_stage0), 16 >> A0 rows per workgroup.  The
@@ -433,9 +433,13 @@ void launch_fast_a(const PassArgs &A_in, dim3 grid, dim3 block, hipStream_t s) {
     A.uniform = pass_uniform(A, &A.n1_valid) ? 1 : 0;
     if (A.uniform && A.inverse && upper_half_zero(A))
         hipLaunchKernelGGL((k_ntt_fast<A2, true, false, true, true>), grid, block, 0, s, A);
-    else if (A.uniform && A.is_final && A.ndig == 0) {     // single-pass transform over whole tiles
-        if (A.inverse) hipLaunchKernelGGL((k_ntt_fast<A2, true, true, true, false, true>), grid, block, 0, s, A);
-        else hipLaunchKernelGGL((k_ntt_fast<A2, false, true, true, false, true>), grid, block, 0, s, A);
+    else if (rows_single_pass(A)) {
+        switch ((A.inverse ? 2 : 0) + A.uniform) {
+            case 0: hipLaunchKernelGGL((k_ntt_fast<A2, false, true, false, false, true>), grid, block, 0, s, A); break;
+            case 1: hipLaunchKernelGGL((k_ntt_fast<A2, false, true, true, false, true>), grid, block, 0, s, A); break;
+            case 2: hipLaunchKernelGGL((k_ntt_fast<A2, true, true, false, false, true>), grid, block, 0, s, A); break;
+            default: hipLaunchKernelGGL((k_ntt_fast<A2, true, true, true, false, true>), grid, block, 0, s, A); break;
+        }
     } else if (A.uniform) launch_fast_u<A2, true>(A, grid, block, s);
     else launch_fast_u<A2, false>(A, grid, block, s);
 }
@@ -510,10 +514,12 @@ int launch_passes(const std::vector<PassArgs> &passes, hipStream_t s) {
             PassArgs U = A;
             U.is_final = 1;
             U.uniform = pass_uniform(U, &U.n1_valid) ? 1 : 0;
-            switch ((U.inverse ? 2 : 0) + U.uniform) {
+            switch ((U.inverse ? 4 : 0) + (rows_single_pass(U) ? 2 : 0) + U.uniform) {     // a uniform one is one of rows
                 case 0: hipLaunchKernelGGL((k_ntt_512<false, false>), grid, block, 0, s, U); break;
-                case 1: hipLaunchKernelGGL((k_ntt_512<false, true>), grid, block, 0, s, U); break;
-                case 2: hipLaunchKernelGGL((k_ntt_512<true, false>), grid, block, 0, s, U); break;
+                case 2: hipLaunchKernelGGL((k_ntt_512<false, false, true>), grid, block, 0, s, U); break;
+                case 3: hipLaunchKernelGGL((k_ntt_512<false, true>), grid, block, 0, s, U); break;
+                case 4: hipLaunchKernelGGL((k_ntt_512<true, false>), grid, block, 0, s, U); break;
+                case 6: hipLaunchKernelGGL((k_ntt_512<true, false, true>), grid, block, 0, s, U); break;
                 default: hipLaunchKernelGGL((k_ntt_512<true, true>), grid, block, 0, s, U); break;
             }
         } else {

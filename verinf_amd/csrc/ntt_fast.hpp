@@ -143,6 +143,18 @@ struct TileU {
     int shcd;         // log2 of the output stride between columns (0 except in a single-pass transform, whose columns are rows)
 };
 
+// A single-pass transform of rows, whatever their width, strides and number, or of rows by up to eight cosets that it interleaves: its second
+// stage stores along the output (SGL, see lds_slot), 128 bytes of it or more with one instruction of a wavefront.  With the columns along the lanes,
+// as other passes store, that instruction touches a piece of 8 to 64 bytes of a line of each of up to 64 rows.  Whole tiles of contiguous
+// rows (pass_uniform) had this form first.  us for 2^26 points in an odd number of rows of 2^5, 2^6, 2^7, 2^8, 2^9: 623, 577, 364, 268, 263 ->
+// 195, 198, 196, 207, 232.  Extensions of 2^K points by four, 2^27 words written, K = 5 to 9: 761, 614, 599, 574, 625 -> 478, 486, 505,
+// 534, 594; from rows of three quarters of the width (the inverse transform's rows are not contiguous) 1990, 1753, 900, 630, 640 -> 473, 485,
+// 508, 534, 605; by eight, K = 6 to 9: 526, 501, 512, 550 -> 424, 441, 478, 533.  Sixteen cosets would take all lanes above k1, more do not fit.
+inline bool rows_single_pass(const PassArgs &A) { return A.is_final && A.ndig == 0 && A.log_rho <= 3; }
+
+// its column of a trip over sixteen of them: the coset in the lowest bits of the thread's number, k1 in the next four, the row above
+VI_HD int rows_column(int tid, int log_rho) { return ((tid >> (4 + log_rho)) << log_rho) + (tid & ((1 << log_rho) - 1)); }
+
 // does the pass qualify?  On success *n1_valid = how many of a thread's sixteen stage-1 inputs exist (the first
 // n1_valid; 16 unless the source rows are narrower than the transform).
 inline bool pass_uniform(const PassArgs &A, int *n1_valid) {
@@ -361,8 +373,8 @@ template <int A2, bool TWT>
 VI_HD constexpr int twi_slot(int n2, int k1) { return TWT ? (k1 << A2) + n2 : n2 * 16 + k1; }
 
 // Where (k1, n2, column c) sits in LDS between the two stages: [k1][n2][c] with one word of padding per (k1, n2) row.
-// SGL (a single-pass transform over whole tiles, pass_uniform): stage 2 runs k1 along the lanes there, so that a
-// wavefront's stores are 128-byte runs of output rows (with the columns along the lanes, as in the other passes,
+// SGL (a single-pass transform, rows_single_pass): stage 2 runs the cosets and then k1 along the lanes there, so that a
+// wavefront's stores are runs of 128 bytes and more of output rows (with the columns along the lanes, as in the other passes,
 // consecutive lanes would store whole rows apart: the columns of such a tile ARE its rows); the k1 pitch is then
 // padded to 4 mod 8 words, which puts the sixteen k1 of a wavefront on different banks.
 // The 512-point kernel has no LDS to spare (with any padding of the k1 pitch a fourth workgroup no longer fits a CU):
@@ -445,27 +457,37 @@ VI_HD void fast_stage2(const PassArgs &A, i64 tile, int tid, int t_loop, const u
     const int st = (1 << lt) + 1;
     const int c = tid & ((1 << lt) - 1);
     if constexpr (SGL) {
-        // whole tiles of a single-pass transform: thread (k1 = low four bits, sixteen columns per trip), outputs
-        // k1 + 16 k2 of row c at word (c << a) + k1 + 16 k2 of the tile
-        static_assert(UNI, "whole tiles are addressed through scalar bases");
-        const TileU U = tile_uniform<A2>(A, tile);
-        const URun dst = urun(A.dst + U.dst_u);
-        const int k1 = tid & 15;
+        // a single-pass transform: thread (k1 = four bits of its number, sixteen columns per trip), outputs k1 + 16 k2 of row c
+        // at word (c << a) + k1 + 16 k2 of the tile (UNI: a whole tile of contiguous rows), or the interleaved outputs of a row's
+        // cosets, the coset in the lowest bits of the thread's number
+        const int lr = UNI ? 0 : A.log_rho;
+        const int k1 = (tid >> lr) & 15;
+        URun dst;
+        int shcd = 0;
+        if constexpr (UNI) {
+            const TileU U = tile_uniform<A2>(A, tile);
+            dst = urun(A.dst + U.dst_u);
+            shcd = U.shcd;
+        }
 #pragma unroll
         for (int i = 0; i < 16 / E2; ++i) {
-            const int cc = (tid >> 4) + 16 * i;
-            const u32 off = ((u32)cc << U.shcd) + (u32)k1;
+            const int cc = UNI ? (tid >> 4) + 16 * i : rows_column(tid, lr) + 16 * i;
+            const u32 off = ((u32)cc << shcd) + (u32)k1;
             u64 x[E2];
 #pragma unroll
             for (int n2 = 0; n2 < E2; ++n2) x[n2] = lds[lds_slot<A2, true>(st, k1, n2, cc)];
             VI_SCHED_FENCE();
             dft_reg<A2, INV>(x);
             VI_SCHED_FENCE();
+            const i64 g = (tile << lt) + cc, row = g >> lr;
+            if (!UNI && row >= A.n_rows) continue;
+            u64 *out = A.dst + row * A.dst_row_stride + (g & ((1 << lr) - 1)) + (k1 << lr);
 #pragma unroll
             for (int k2 = 0; k2 < E2; ++k2) {
                 u64 v = x[k2];
                 if (A.scale != 1) v = gl::mul(v, A.scale);
-                ustore_stream(dst, (u32)k2 << 4, off, v);
+                if constexpr (UNI) ustore_stream(dst, (u32)k2 << 4, off, v);
+                else VI_STREAM_STORE(&out[(i64)k2 << (4 + lr)], v);
                 if ((k2 & 3) == 3) VI_SCHED_FENCE();
             }
         }
@@ -540,20 +562,21 @@ VI_HD void fast_stage2(const PassArgs &A, i64 tile, int tid, int t_loop, const u
 // x[j] + x[j + 16] and gets the even outputs from a 16-point transform, thread h = 1 forms the differences times
 // w_32^j (shifts) and gets the odd outputs -- no exchange between the two.  h is the top bit of the thread id, so a
 // wavefront is all sums or all differences.  Per-element addressing (a single pass is never a uniform pass).
-template <bool INV, bool UNI = false>
+template <bool INV, bool UNI = false, bool SGL = UNI>
 VI_HD void fast_stage2_512(const PassArgs &A, i64 tile, int tid, const u64 *lds) {
     constexpr int A2 = 5;
     const int lt = logT(A);                                // 3: eight columns per tile
     const int st = (1 << lt) + 1;
-    // UNI (whole tiles of contiguous rows): k1 along the lanes, see lds_slot
-    const int c = UNI ? (tid >> 4) & ((1 << lt) - 1) : tid & ((1 << lt) - 1);
-    const int k1 = UNI ? tid & 15 : (tid >> lt) & 15, h = tid >> (lt + 4);
+    // SGL: k1 along the lanes, see lds_slot
+    const int lr = UNI ? 0 : A.log_rho;
+    const int c = SGL ? (UNI ? (tid >> 4) & ((1 << lt) - 1) : rows_column(tid & 127, lr)) : tid & ((1 << lt) - 1);
+    const int k1 = SGL ? (tid >> lr) & 15 : (tid >> lt) & 15, h = tid >> (lt + 4);
     ColRef R{};
     if (!UNI) R = col_ref(A, tile, c);
     const int lc = A.B + A.log_rho;
     u64 x[32], y[16];
 #pragma unroll
-    for (int n2 = 0; n2 < 32; ++n2) x[n2] = lds[lds_slot<A2, UNI>(st, k1, n2, c)];
+    for (int n2 = 0; n2 < 32; ++n2) x[n2] = lds[lds_slot<A2, SGL>(st, k1, n2, c)];
     if (h == 0) {
 #pragma unroll
         for (int j = 0; j < 16; ++j) y[j] = gl::addc(x[j], x[j + 16]);
