@@ -118,6 +118,25 @@ def test_passes_over_short_rows_in_parts_of_tiles(cp, logk, log_rho):
                 assert torch.equal(whole[i:i + step], some), (m, i)
 
 
+@pytest.mark.parametrize("logk,log_rho", [(7, 0), (7, 1), (5, 2), (9, 1)])
+def test_a_small_workspace_takes_the_same_extension(cp, logk, log_rho):
+    """Rows enough for the passes, with a workspace for all of them (two launches), for a third, and for one row (one launch)."""
+    from verinf_amd import _lib
+    L = _lib.lib()
+    K, N = 1 << logk, 1 << (logk + log_rho)
+    m = (5 << 20) // N + 1
+    src = to_dev(rand_field((m, K), logk + log_rho))
+    one = L.vi_coset_lde_min_workspace_bytes(K, N)
+    want = cp.coset_lde(src, K, N)
+    for rows, launches in ((m, 2), (m // 3, None), (1, 1)):
+        assert launches is None or L.vi_coset_lde_launches(m, K, N, one * rows) == launches
+        ws = torch.empty(one * rows, dtype=torch.uint8, device="cuda")
+        out = torch.zeros_like(want)
+        rc = L.vi_coset_lde(src.data_ptr(), m, K, K, K, N, 7, out.data_ptr(), N, ws.data_ptr(), ws.numel(), None)
+        torch.cuda.synchronize()
+        assert rc == 0 and torch.equal(out, want), rows
+
+
 @pytest.mark.parametrize("logn", range(12, 21))
 def test_transforms_of_longer_rows(cp, logn):
     """Few rows (two or three launches of four points per thread) against the oracle and against a batch beyond them."""

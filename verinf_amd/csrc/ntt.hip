@@ -604,27 +604,31 @@ bool small_ntt_pays(i64 m, int logn) {
     return logn <= 4 || (m << logn) <= ((i64)1 << 20);
 }
 
-// Extensions of K < 2^12 in one launch, by log2 of the points written.  While a batch leaves SIMDs idle the single launch is the
+// Extensions of K < 2^12 in one launch, by the points written.  While a batch leaves SIMDs idle the single launch is the
 // shorter chain (2^16 points 16 to 36 against 5 to 16): up to 2^21, or 2^19 from eight cosets on (2^22 at K <= 2^4), as its
 // stores are single words rho apart.  Beyond that it stays ahead where the passes are slow themselves (us for 2^26 points):
-// below 32 points they have no register kernel (K = 2^3, two cosets 709 against 266); short rows they store a column at a time,
-// rho words in a piece (one or two cosets up to K = 2^7: 1356 and 289 at 2^5, 506 and 409 at 2^7; four at 2^6: 312 and 471);
-// and at K = 2^10 they go twice through memory in each direction (four cosets 580 and 513).  At K = 2^11, and at 2^5 with four
-// cosets, the two meet at 2^24 points.
+// below 32 points they have no register kernel (K = 2^3, two cosets 709 against 266); at one or two cosets up to K = 2^6 its four or eight
+// points a thread save the way through memory (2^5: 412 and 295 against 354 and 264; two cosets of 2^6 meet at 2^25 points, 303 and 306; of
+// 2^7, 2^22 points 33.6 and 32.7, 2^23 49.0 and 54.8, 2^26 316 and 400; four of 2^5, 2^21 points 21.3 and 15.0, 2^22 27.5 and 30.7, 2^23 41 and 54);
+// and at K = 2^10 they go twice through memory in each direction (four cosets 580 and 513).  At K = 2^11 the two meet at 2^24 points.
+// m: the rows that the workspace takes at once, so that a small one does not cut a batch into many launches.
 bool small_lde_pays(i64 m, int logK, int logN, bool in_place) {
     if (logK < SMALL_MIN_LOG || logK >= SMALL_MAX_LOG) return false;
     const int log_rho = logN - logK;
     if (log_rho > 8) return false;
-    int log_most;
+    i64 most;
     if (log_rho <= 2) {
-        const int short_rows = log_rho <= 1 ? 7 : 4;
-        log_most = logK <= short_rows || logK == 10 ? 62 : (logK == 11 || logK == 5 ? 24 : 21);
+        const int short_rows = log_rho <= 1 ? 6 : 4;
+        if (logK <= short_rows || logK == 10) most = (i64)1 << 62;
+        else if (logK == 5) most = (i64)7 << 19;
+        else if (logK == 7 && log_rho == 1) most = (i64)5 << 20;
+        else most = (i64)1 << (logK == 11 ? 24 : 21);
     } else {
         // in place one workgroup has to run through the cosets of its rows: eight or more of them are the longer chain
         if (in_place && logK > 4) return false;
-        log_most = logK <= 4 ? 22 : 19;
+        most = (i64)1 << (logK <= 4 ? 22 : 19);
     }
-    return m <= (((i64)1 << log_most) >> logN);
+    return m <= most >> logN;
 }
 
 // A row of 2^12 fills a CU, so the single launch takes 23 us per round of 256 workgroups (34 with two cosets in each): ahead of
@@ -699,9 +703,9 @@ bool row_lde_pays(i64 m, int logK, int logN) {
 
 // Which launches an extension takes
 enum LdeRoute { LDE_PASSES, LDE_SINGLE, LDE_SMALL_PASSES, LDE_ROWS };
-LdeRoute lde_route(i64 m, int logK, int logN, bool in_place, const Split &sp) {
+LdeRoute lde_route(i64 m, i64 chunk, int logK, int logN, bool in_place, const Split &sp) {
     if (row_lde_pays(m, logK, logN)) return LDE_ROWS;
-    if (small_lde_pays(m, logK, logN, in_place)) return LDE_SINGLE;
+    if (small_lde_pays(chunk, logK, logN, in_place)) return LDE_SINGLE;
     if (logK == SMALL_MAX_LOG && single_round_of_rows(m, logN - logK, in_place)) return LDE_SINGLE;
     return small_lde_passes_pay(m, logK, logN, sp) ? LDE_SMALL_PASSES : LDE_PASSES;
 }
@@ -814,12 +818,12 @@ int64_t vi_coset_lde_launches(int64_t m, int64_t K, int64_t N, size_t ws_bytes) 
     size_t one = vi_coset_lde_min_workspace_bytes(K, N);
     if (!one || m <= 0 || ws_bytes < one) return 0;
     i64 chunk = (i64)(ws_bytes / one);
-    const LdeRoute route = lde_route(m, vi::ilog2(K), vi::ilog2(N), false, split_digits(vi::ilog2(K)));
-    if (route == LDE_SINGLE) return 1;
     if (chunk > m) chunk = m;
     if (chunk > max_lde_chunk(vi::ilog2(K), vi::ilog2(N))) chunk = max_lde_chunk(vi::ilog2(K), vi::ilog2(N));
     const i64 n_chunks = (m + chunk - 1) / chunk;         // balancing keeps the chunk count
     chunk = (m + n_chunks - 1) / n_chunks;
+    const LdeRoute route = lde_route(m, chunk, vi::ilog2(K), vi::ilog2(N), false, split_digits(vi::ilog2(K)));
+    if (route == LDE_SINGLE) return 1;
     if (route == LDE_ROWS) return 2 * n_chunks;
     // the pass list of one chunk, planned with placeholder addresses (only their being null or not matters)
     const int logK = vi::ilog2(K), logN = vi::ilog2(N);
@@ -920,7 +924,7 @@ int coset_lde_impl(const char *who, const uint64_t *in, int64_t m, int64_t width
     if (!rc) rc = get_tables(logK, 0, &Tf);
     if (!rc) rc = get_pre(logK, logN, shift, &pre, pin);
     if (rc) return rc;
-    const LdeRoute route = lde_route(m, logK, logN, coeffs == in, Ti->sp);
+    const LdeRoute route = lde_route(m, chunk, logK, logN, coeffs == in, Ti->sp);
     const Tables *TiRow = nullptr, *TfRow = nullptr;
     if (coset_rows_ok(logK, logN)) {                       // whatever the batch: one of another size may be captured
         rc = get_tables(logK, 1, &TiRow, true);
