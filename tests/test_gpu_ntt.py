@@ -248,6 +248,32 @@ def test_every_row_of_ragged_batches(cp, logK, log_rho, least):
     assert np.array_equal(got, O.coset_lde_rows(host, K, N, 7))
 
 
+@pytest.mark.parametrize("logK,least", [(10, 1536), (11, 513), (12, 257)])
+def test_extension_to_as_many_points_by_rows(cp, logK, least):
+    """One coset, around the row where the two launches by rows begin: rows that fill no tile, ragged and strided sources, coefficients
+    over their messages, codewords from them, and a workspace of few rows, which leaves the batch to other launches."""
+    from verinf_amd import _lib
+    L = _lib.lib()
+    K = 1 << logK
+    big = rand_field_dev((least + 5, K + 3), logK)
+    for m, width in [(least - 1, K), (least, K), (least + 1, K - 77), (least + 2, 300), (least + 5, 1)]:
+        src = big[:m, :width]
+        want = O.coset_lde_rows(np.ascontiguousarray(to_np(src)), K, K, 11)
+        assert np.array_equal(to_np(cp.coset_lde(src, K, K, 11)), want), (m, width)
+        own = torch.zeros((m, K), dtype=torch.uint64, device="cuda")
+        own[:, :width] = src
+        coeffs, code = cp.coset_lde_with_coeffs(own, K, K, 11, in_place=True)
+        assert np.array_equal(to_np(code), want), (m, width)
+        ws = torch.empty(3 * L.vi_coset_lde_min_workspace_bytes(K, K), dtype=torch.uint8, device="cuda")
+        again = torch.empty((m, K), dtype=torch.uint64, device="cuda")
+        _lib.check(L.vi_coset_lde(src.data_ptr(), m, width, K + 3, K, K, 11, again.data_ptr(), K, ws.data_ptr(), ws.numel(), _lib.stream_ptr()))
+        assert torch.equal(again, code), (m, width)
+        again.zero_()
+        ws = torch.empty(L.vi_coset_lde_workspace_bytes(m, K, K), dtype=torch.uint8, device="cuda")
+        _lib.check(L.vi_coset_extend(coeffs.data_ptr(), m, K, K, K, K, 11, again.data_ptr(), K, ws.data_ptr(), ws.numel(), _lib.stream_ptr()))
+        assert torch.equal(again, code), (m, width)
+
+
 @pytest.mark.parametrize("logK,log_rho", [(12, 1), (12, 2), (12, 3), (14, 2), (14, 4), (16, 3)])
 def test_lde_with_cosets_dealt_to_several_workgroups(cp, logK, log_rho):
     """Tiles around the counts where the share of the cosets that a workgroup takes changes, and around full rounds of workgroups;

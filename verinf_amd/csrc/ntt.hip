@@ -568,6 +568,7 @@ void launch_lde_row(const LdeRow &A, int log_rho, hipStream_t s) {
     constexpr int per = 16 >> A0;
     const dim3 grid((unsigned)((pairs + per - 1) / per)), block(NTHREADS);
     switch (log_rho) {
+        case 0: hipLaunchKernelGGL((k_lde_row<A0, 0>), grid, block, 0, s, A); break;
         case 1: hipLaunchKernelGGL((k_lde_row<A0, 1>), grid, block, 0, s, A); break;
         case 2: hipLaunchKernelGGL((k_lde_row<A0, 2>), grid, block, 0, s, A); break;
         default:
@@ -689,14 +690,17 @@ bool small_lde_passes_pay(i64 m, int logK, int logN, const Split &sp) {
     return small_passes_us(sp, million) < fast_passes_us(sp, log_rho, (double)m * (double)((i64)1 << logK) / TILE, million);
 }
 
-// Extensions of K = 2^10 .. 2^12 by two, four or eight as one launch to the coefficients (k_ntt_row) and one to the codewords
+// Extensions of K = 2^10 .. 2^12 to as many points, by two, four or eight as one launch to the coefficients (k_ntt_row) and one to the codewords
 // (k_lde_row), from 2^20 .. 5 2^20 points written, where the shorter chains of ntt_small.hpp meet it.  us, the better of the other
 // routes and this one: 2^20 points 2^10 -> 2^12 21 and 22 (a row more 25 and 24), -> 2^13 25 and 23, 2^11 -> 2^13 27 and 25; 2^21 points 2^12 ->
 // 2^14 41 and 32; 2^22 points 2^10 -> 2^11 43 and 44, 5 2^20 51 and 45, 2^11 -> 2^12 50 and 45; 2^24 points 2^10 -> 2^12 135 and 88, 2^11 -> 2^13
-// 154 and 98, 2^12 -> 2^14 133 and 118.
+// 154 and 98, 2^12 -> 2^14 133 and 118.  To as many points: 2^10 2^20 points 19 and 22, 2^20.3 22 and 26, 2^20.6 28 and 27, 2^22 55 and 45, 2^26
+// 857 and 512; 2^11 and 2^12, whose single launches are one round of workgroups at 2^20 points, 21 and 24 and 23 and 25 there, 2^20.3 28.4 and 27.7
+// and 38 and 30, 2^22 65 and 47 and 58 and 50, 2^26 871 and 545 and 735 and 580.
 bool row_lde_pays(i64 m, int logK, int logN) {
     if (!row_launch_on() || !coset_rows_ok(logK, logN)) return false;
     const int log_rho = logN - logK;
+    if (log_rho == 0) return logK == 10 ? m >= ((i64)3 << 19) >> logN : m > ((i64)1 << 20) >> logN;
     const i64 least = logK == TILE_LOG ? (i64)2 << 20 : log_rho >= 2 ? (i64)1 << 20 : logK == 10 ? (i64)5 << 20 : (i64)4 << 20;
     return m >= (least >> logN) + (logK == 10 && log_rho == 2 ? 1 : 0);
 }
@@ -704,7 +708,8 @@ bool row_lde_pays(i64 m, int logK, int logN) {
 // Which launches an extension takes
 enum LdeRoute { LDE_PASSES, LDE_SINGLE, LDE_SMALL_PASSES, LDE_ROWS };
 LdeRoute lde_route(i64 m, i64 chunk, int logK, int logN, bool in_place, const Split &sp) {
-    if (row_lde_pays(m, logK, logN)) return LDE_ROWS;
+    // to as many points a single launch takes what a small workspace would cut into many pairs
+    if (row_lde_pays(logK == logN ? chunk : m, logK, logN)) return LDE_ROWS;
     if (small_lde_pays(chunk, logK, logN, in_place)) return LDE_SINGLE;
     if (logK == SMALL_MAX_LOG && single_round_of_rows(m, logN - logK, in_place)) return LDE_SINGLE;
     return small_lde_passes_pay(m, logK, logN, sp) ? LDE_SMALL_PASSES : LDE_PASSES;

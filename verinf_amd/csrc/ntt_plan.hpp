@@ -168,7 +168,7 @@ inline void append_coset_merged(int logK, int logN, std::vector<u64> &t) {
 // factor w_N^(256 t n1) a power of two when K rho / 256 <= 64.  Appended: w_K^(k r) w_N^(t r) at [t][k][r] (N words).
 inline bool coset_rows_ok(int logK, int logN) {
     const int log_rho = logN - logK;
-    return row_single_ok(logK) && log_rho >= 1 && log_rho <= 3 && logN <= 14;
+    return row_single_ok(logK) && log_rho >= 0 && log_rho <= 3 && logN <= 14;
 }
 inline void append_coset_rows(int logK, int logN, std::vector<u64> &t) {
     const Split rs = row_split(logK);
