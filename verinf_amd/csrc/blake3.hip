@@ -555,7 +555,8 @@ int launch_chunks(const u64 *rows, i64 slab_rows, i64 n, i64 row_stride, i64 chu
         hipLaunchKernelGGL(k_chunk_cvs_quad, grid, dim3(BLOCK), 0, s, rows, slab_rows, n, row_stride, chunk0, single_root ? 1 : 0, cvs);
     } else {
         dim3 grid((unsigned)((n + BLOCK - 1) / BLOCK), (unsigned)slab_chunks);
-        hipLaunchKernelGGL(wide_launch(grid) ? k_chunk_cvs<true> : k_chunk_cvs<false>, grid, dim3(BLOCK), 0, s, rows, slab_rows, n, row_stride, chunk0, single_root ? 1 : 0, cvs);
+        const auto kernel = wide_launch(grid) ? k_chunk_cvs<true> : k_chunk_cvs<false>;
+        hipLaunchKernelGGL(kernel, grid, dim3(BLOCK), 0, s, rows, slab_rows, n, row_stride, chunk0, single_root ? 1 : 0, cvs);
     }
     VI_LAUNCH_CHECK("k_chunk_cvs");
     return VI_OK;
@@ -689,7 +690,9 @@ int vi_row_prg(const uint8_t *seed, const uint64_t *row_indices, int64_t row_off
     const i64 total = n_rows * slack;
     const i64 blocks = (total + BLOCK - 1) / BLOCK;
     if (blocks > 0x7FFFFFFF) return vi::fail(VI_EINVAL, "vi_row_prg: %lld values exceed one launch", (long long)total);
-    hipLaunchKernelGGL(wide_launch(dim3((unsigned)blocks)) ? k_row_prg<true> : k_row_prg<false>, dim3((unsigned)blocks), dim3(BLOCK), 0, (hipStream_t)stream, (const u32 *)seed, row_indices,
+    const dim3 grid((unsigned)blocks);
+    const auto kernel = wide_launch(grid) ? k_row_prg<true> : k_row_prg<false>;
+    hipLaunchKernelGGL(kernel, grid, dim3(BLOCK), 0, (hipStream_t)stream, (const u32 *)seed, row_indices,
                        (u32)row_offset, (i64)n_rows, (i64)slack, out, (i64)out_stride);
     VI_LAUNCH_CHECK("k_row_prg");
     return VI_OK;
@@ -714,7 +717,8 @@ int vi_pad_rows(const uint8_t *seed, int64_t row_offset, const uint64_t *message
     const i64 groups = (n_rows + (BLOCK >> log_lanes) - 1) / (BLOCK >> log_lanes);
     if (groups > 0x7FFFFFFF / segments) return vi::fail(VI_EINVAL, "vi_pad_rows: %lld words exceed one launch", (long long)(n_rows * width));
     const dim3 grid((unsigned)(groups * segments));
-    hipLaunchKernelGGL(wide_launch(grid) ? k_pad_rows<true> : k_pad_rows<false>, grid, dim3(BLOCK), 0, (hipStream_t)stream, (const u32 *)seed, (u32)row_offset, messages,
+    const auto kernel = wide_launch(grid) ? k_pad_rows<true> : k_pad_rows<false>;
+    hipLaunchKernelGGL(kernel, grid, dim3(BLOCK), 0, (hipStream_t)stream, (const u32 *)seed, (u32)row_offset, messages,
                        (i64)in_stride, (i64)ell, (i64)n_rows, (u32)segments, log_lanes, (i64)width, out);
     VI_LAUNCH_CHECK("k_pad_rows");
     return VI_OK;
