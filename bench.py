@@ -35,8 +35,8 @@ HBM_PEAK_GBS = 8000.0           # MI355X HBM3E, published
 # (profiles/k_lde_mid_k_ntt_fast__coset_lde_1024x2p16_to_2p18.md).  roofline.traffic is this figure divided by the
 # launches of a step, like roofline.achieved.
 LDE_TRAFFIC_BYTES_PER_STEP = 8.06e9
-# VALU wave-instructions one LDE step issues (rocprofv3 --pmc SQ_INSTS_VALU, same profile: per 512-row chunk 58.7 M in
-# the strided inverse launch, 290.1 M in k_lde_mid and 188.1 M in the final forward launch) and the rate at which
+# VALU wave-instructions one LDE step issues (rocprofv3 --pmc SQ_INSTS_VALU, same profile: per 512-row chunk 51.2 M in
+# the strided inverse launch, 253.6 M in k_lde_mid and 162.1 M in the final forward launch) and the rate at which
 # 1024 SIMDs issue the instruction classes these kernels consist of (carry, multiply, three-operand and shift
 # instructions: one per 4.16 cycles per SIMD, measured by `bench.py --valu-probe`,
 # profiles/valu_issue_rates__probe.md) at the 2.4 GHz peak clock
