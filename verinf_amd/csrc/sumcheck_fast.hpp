@@ -790,12 +790,14 @@ int launch_pass3(const FastDesc &F, i64 cols, const u64 *r, u64 *part, const u64
         n_cus = cus[dev];
     }
     int nb = blocks_for(cols);
+    const int least = prev_rows > 0 ? 3 : 1; // the first three workgroups add up the previous pass's sums
     if (nb > cap) {
-        hipLaunchKernelGGL((k_pass3_long<NT, SHAPE, FIRST, ONE>), dim3(n_cus), dim3(LongPass<NT>::THREADS), 0, s, F, cols, r[0], r[1], r[2], part,
+        nb = std::max(n_cus, least);
+        hipLaunchKernelGGL((k_pass3_long<NT, SHAPE, FIRST, ONE>), dim3(nb), dim3(LongPass<NT>::THREADS), 0, s, F, cols, r[0], r[1], r[2], part,
                            prev_part, prev_rows, prev_sums);
-        return n_cus;
+        return nb;
     }
-    if (nb < 3 && prev_rows > 0) nb = 3;     // the first three workgroups add up the previous pass's sums
+    nb = std::max(nb, least);
     hipLaunchKernelGGL((k_pass3<NT, SHAPE, FIRST, ONE>), dim3(nb), dim3(BLOCK), 0, s, F, cols, r[0], r[1], r[2], part,
                        prev_part, prev_rows, prev_sums);
     return nb;
