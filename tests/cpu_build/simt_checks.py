@@ -337,7 +337,13 @@ def sumcheck(so):
             if cus == 1:
                 check(form, 14, "apart")
                 check(form, 16, "in place")
-            check(form, 16 + cus, "apart")
+            # a second pass of 32 pieces for three workgroups' 48 wavefronts (36 for four tables), and of 64 and 128
+            if cus < 3:
+                check(form, 16 + cus, "apart")
+            else:
+                check(form, 18, "in place")
+                if form in ("three", "gate"):
+                    check(form, 19, "apart")
         print("sumcheck", flush=True)
         return
     # lengths below the lanes of a wavefront, one to eight entries a lane, one pass of three rounds and two, each with every remainder

@@ -27,7 +27,7 @@ def built(tmp_path_factory):
 
 @pytest.mark.parametrize("unit,what,switches", [("lookup", "lookup", {}), ("ntt", "ntt", {}), ("ntt", "ntt", {"VI_NTT_ROW": "0"}), ("ntt", "lde", {}), ("ntt", "tables", {}),
                                                 ("matmul", "matmul", {}), ("sumcheck", "sumcheck", {}), ("sumcheck", "sumcheck", {"SIMT_CUS": "1"}),
-                                                ("sumcheck", "sumcheck", {"SIMT_CUS": "2"}), ("mle", "mle", {}), ("blake3", "blake3", {})])
+                                                ("sumcheck", "sumcheck", {"SIMT_CUS": "2"}), ("sumcheck", "sumcheck", {"SIMT_CUS": "3"}), ("mle", "mle", {}), ("blake3", "blake3", {})])
 def test_kernels_on_the_cpu(built, unit, what, switches):
     asan = subprocess.check_output(["g++", "-print-file-name=libasan.so"], text=True).strip()
     env = dict(os.environ, LD_PRELOAD=asan, ASAN_OPTIONS="detect_leaks=0,verify_asan_link_order=0", OPENBLAS_NUM_THREADS="1", **switches)

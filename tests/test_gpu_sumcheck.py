@@ -776,6 +776,18 @@ def test_first_passes_around_what_the_chip_holds(mods, terms, v):
     assert claim == want_claim and [[y for _, y in s] for s in polys] == want
 
 
+@pytest.mark.parametrize("terms,v", [([(7, [0, 1])], 25), ([(5, [0])], 26)])
+def test_second_passes_beyond_what_the_chip_holds(mods, terms, v):
+    """The second pass in place by pieces from a counter, which two tables reach at 2^25 (three and four at 2^24, above), and several columns to
+    a thread in it: one table's threads take so few registers that its passes have the largest grid, and go round."""
+    gpu, _ = mods
+    tabs = [rand_field_dev((1 << v,), 17 * v + t) for t in range(len(terms[0][1]))]
+    coins = _coins(v, v)[0]
+    claim, polys, _, _ = gpu.prove_terms_gpu([(c, [tabs[i] for i in fs]) for c, fs in terms], lambda i: coins[i], P)
+    want_claim, want, _ = O.sumcheck_prove([to_np(t) for t in tabs], terms, coins)
+    assert claim == want_claim and [[y for _, y in s] for s in polys] == want
+
+
 @pytest.mark.parametrize("v", range(1, 16))
 @pytest.mark.parametrize("terms", [[(5, [0])], [(7, [0, 1])], [(1, [0, 1, 2])], [(3, [0, 1, 2, 3])], [(3, [0, 1, 2]), (P - 3, [0, 3])]])
 def test_every_length_of_the_last_launch(mods, terms, v):
