@@ -25,21 +25,20 @@ struct Point {
 };
 
 // e[j], j < 2^JB: eq entries of the indices (j << (n - JB)) | g.
-// Constant indices into pt.z only, so that the by-value argument stays in the kernarg segment.
+// Indices into pt.z are the same for all threads, so that the by-value argument stays in the kernarg segment.
 template <int JB>
 __device__ __forceinline__ void eq_entries(const Point &pt, int n, i64 g, u64 (&e)[1 << JB]) {
     // two running products, whose chains are interleaved (gl::mul_lazy2), as are the products of the split: one table of 2^26 evaluated in
-    // 211 -> 178 us, eq_vector of 2^24 34 -> 32
+    // 211 -> 178 us, eq_vector of 2^24 34 -> 32.  A loop, as a small call waits for its instructions: unrolled for all MAX_VARS variables, those that
+    // are not there stepped over, k_mle_partial<3> was 39 KB and is 20: an evaluation over 2^3 entries 7.8 -> 5.3 us, 2^10 7.9 -> 6.1, 39 tables of 2^14
+    // 12.4 -> 10.6 (one running product, unrolled: 6.7, 7.5 and 12.2)
     u64 even = 1, odd = 1;
     auto factor = [&](int zi) {
         const u64 z = pt.z[zi], other = z <= 1 ? 1 - z : gl::P + 1 - z;        // the same for all threads
         return (g >> (n - 1 - zi)) & 1 ? z : other;
     };
-#pragma unroll
-    for (int zi = JB; zi < MAX_VARS; zi += 2) {
-        if (zi + 1 < n) gl::mul_lazy2(even, factor(zi), even, odd, factor(zi + 1 < MAX_VARS ? zi + 1 : zi), odd);
-        else if (zi < n) even = gl::mul_lazy(even, factor(zi));
-    }
+#pragma unroll 1
+    for (int zi = JB; zi < n; zi += 2) gl::mul_lazy2(even, factor(zi), even, odd, zi + 1 < n ? factor(zi + 1) : 1, odd);
     e[0] = gl::mul(even, odd);
 #pragma unroll
     for (int zi = JB - 1; zi >= 0; --zi) {
