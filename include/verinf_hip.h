@@ -76,8 +76,9 @@ int vi_gl_unop(int op, const uint64_t *a, uint64_t arg, uint64_t *out, int64_t n
  * 7: the lazily reduced product, made canonical;  8 / 9: a * b + c with c = rotl(a, 17) ^ b, canonical / lazily
  * reduced then made canonical;  10: the five-word sum a b + b b + a a + ~a ~b + (2^64 - 1)^2 reduced;
  * 11: forty times a b summed in five words, reduced;
- * 20 .. 31: two operations at once, the even number for the first result and the odd one for the second, whose operands are other
- * ones: 20 differences, 22 sums, 24 products, 26 lazily reduced products, 28 products with an addend, 30 sums of forty products;
+ * 20 .. 35: two operations at once, the even number for the first result and the odd one for the second, whose operands are other
+ * ones: 20 differences, 22 sums, 24 products, 26 lazily reduced products, 28 products with an addend, 30 sums of forty products,
+ * 32 sums and 34 differences of butterflies;
  * 100 + e, 0 <= e < 96: canonical a times 2^e (the compile-time shift twiddle);
  * 300 + e, 0 <= e < 192: the same for any exponent (2^96 = -1), in the form the coset loop of the fused LDE launch uses. */
 int vi_gl_probe(int op, const uint64_t *a, const uint64_t *b, uint64_t *out, int64_t n, void *stream);

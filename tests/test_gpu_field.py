@@ -184,6 +184,8 @@ def test_device_field_primitives_one_by_one():
     for op in (24, 26):
         assert run(op, xa, ya) == [x * y % P for x, y in zip(xa, ya)] and run(op + 1, xa, ya) == [y * y % P for y in ya]
     assert run(28, xa, ya) == [(x * y + c) % P for x, y, c in zip(xa, ya, cs)] and run(29, xa, ya) == [(y * y + x) % P for x, y in zip(xa, ya)]
+    assert run(32, xs, ys) == run(33, xs, ys) == [(x + y) % P for x, y in zip(xs, ys)]
+    assert run(34, xs, ys) == [(x - y) % P for x, y in zip(xs, ys)] and run(35, xs, ys) == [(y - x) % P for x, y in zip(xs, ys)]
     assert run(30, xa, ya) == [40 * x * y % P for x, y in zip(xa, ya)] and run(31, xa, ya) == [40 * M * (M - y) % P for y in ya]
     for e in range(96):
         assert run(100 + e, canon, canon) == [(x << e) % P for x in canon], e

@@ -115,7 +115,7 @@ __global__ __launch_bounds__(BLOCK) void k_probe(int op, const u64 *a, const u64
             }
             r = gl::wide_reduce(A);
         }
-        else if (op >= 20 && op < 32) {
+        else if (op >= 20 && op < 36) {
             // two at once: the first result, and the second (of other operands)
             u64 p, q;
             const u64 e = ((x << 17) | (x >> 47)) ^ y;
@@ -124,6 +124,12 @@ __global__ __launch_bounds__(BLOCK) void k_probe(int op, const u64 *a, const u64
             else if (op < 26) gl::mul2(x, y, p, y, y, q);
             else if (op < 28) gl::mul_lazy2(x, y, p, y, y, q);
             else if (op < 30) gl::mul_add2(x, y, e, p, y, y, x, q);
+            else if (op >= 32) {
+                u64 s, d, t, v;
+                gl::bfly2(x, y, s, d, y, x, t, v);
+                p = op < 34 ? s : d;
+                q = op < 34 ? t : v;
+            }
             else {
                 gl::Wide A, B;
                 gl::wide_zero(A);
@@ -422,7 +428,7 @@ int vi_gl_axpy(uint64_t *y, uint64_t alpha, const uint64_t *x, int64_t n, void *
 
 int vi_gl_probe(int op, const uint64_t *a, const uint64_t *b, uint64_t *out, int64_t n, void *stream) {
     const bool shift = (op >= 100 && op < 196) || (op >= 300 && op < 492);
-    if (!shift && (op < 0 || (op > 11 && op < 20) || op > 31)) return vi::fail(VI_EINVAL, "vi_gl_probe: op = %d", op);
+    if (!shift && (op < 0 || (op > 11 && op < 20) || op > 35)) return vi::fail(VI_EINVAL, "vi_gl_probe: op = %d", op);
     if (n < 0) return vi::fail(VI_EINVAL, "vi_gl_probe: n = %lld", (long long)n);
     if (n == 0) return VI_OK;
     const bool needs_b = !shift && op != 4;

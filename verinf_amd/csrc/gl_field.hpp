@@ -436,6 +436,41 @@ __device__ __forceinline__ void sub2(u64 a, u64 b, u64 &x, u64 c, u64 d, u64 &y)
     y = minus_eps(pack(y0, y1), n);
 }
 
+// as bfly: the first carries are read three slots after they were written, the masks of the corrections later still
+__device__ __forceinline__ void bfly2(u64 u, u64 v, u64 &sum, u64 &dif, u64 x, u64 y, u64 &sum2, u64 &dif2) {
+    u32 s0, s1, d0, d1, t0, t1, e0, e1, m, n;
+    u64 st, sb, tt, tb, r, d, z, e;
+    asm("v_add_co_u32 %[s0], vcc, %[u0], %[v0]\n\t"
+        "v_sub_co_u32 %[d0], %[sb], %[u0], %[v0]\n\t"
+        "v_add_co_u32 %[t0], %[tt], %[x0], %[y0]\n\t"
+        "v_sub_co_u32 %[e0], %[tb], %[x0], %[y0]\n\t"
+        "v_addc_co_u32 %[s1], %[st], %[u1], %[v1], vcc\n\t"
+        "v_subb_co_u32 %[d1], %[sb], %[u1], %[v1], %[sb]\n\t"
+        "v_addc_co_u32 %[t1], %[tt], %[x1], %[y1], %[tt]\n\t"
+        "v_subb_co_u32 %[e1], %[tb], %[x1], %[y1], %[tb]"
+        : [s0] "=&v"(s0), [s1] "=&v"(s1), [d0] "=&v"(d0), [d1] "=&v"(d1), [t0] "=&v"(t0), [t1] "=&v"(t1), [e0] "=&v"(e0), [e1] "=&v"(e1),
+          [st] "=&s"(st), [sb] "=&s"(sb), [tt] "=&s"(tt), [tb] "=&s"(tb)
+        : [u0] "v"((u32)u), [u1] "v"((u32)(u >> 32)), [v0] "v"((u32)v), [v1] "v"((u32)(v >> 32)), [x0] "v"((u32)x), [x1] "v"((u32)(x >> 32)),
+          [y0] "v"((u32)y), [y1] "v"((u32)(y >> 32))
+        : "vcc");
+    asm("v_mad_u64_u32 %[r], vcc, 1, -1, %[s]\n\t"
+        "s_or_b64 %[st], %[st], vcc\n\t"
+        "v_mad_u64_u32 %[z], vcc, 1, -1, %[t]\n\t"
+        "s_or_b64 %[tt], %[tt], vcc\n\t"
+        "v_cndmask_b32_e64 %[m], 0, %[k3], %[sb]\n\t"
+        "v_cndmask_b32_e64 %[n], 0, %[k3], %[tb]\n\t"
+        "v_mad_i64_i32 %[d], vcc, %[m], %[k], %[dd]\n\t"
+        "v_mad_i64_i32 %[e], vcc, %[n], %[k], %[ee]"
+        : [r] "=&v"(r), [z] "=&v"(z), [m] "=&v"(m), [n] "=&v"(n), [st] "+&s"(st), [tt] "+&s"(tt), [d] "=&v"(d), [e] "=v"(e)
+        : [s] "v"(pack(s0, s1)), [dd] "v"(pack(d0, d1)), [t] "v"(pack(t0, t1)), [ee] "v"(pack(e0, e1)), [sb] "s"(sb), [tb] "s"(tb), [k3] "n"(BORROWED),
+          [k] "s"(-0x55555555)
+        : "vcc", "scc");
+    sum = select(st, r, pack(s0, s1));
+    sum2 = select(tt, z, pack(t0, t1));
+    dif = d;
+    dif2 = e;
+}
+
 // two words with their carries, as canon_tail
 __device__ __forceinline__ void canon_tail2(u64 w, u64 st, u64 &x, u64 v, u64 tt, u64 &y) {
     u64 r, z;
@@ -741,6 +776,16 @@ VI_HD void addc2(u64 a, u64 b, u64 &x, u64 c, u64 d, u64 &y) {
     const u64 first = addc(a, b);
     y = addc(c, d);
     x = first;
+#endif
+}
+VI_HD void bfly2(u64 u, u64 v, u64 &sum, u64 &dif, u64 x, u64 y, u64 &sum2, u64 &dif2) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    dev::bfly2(u, v, sum, dif, x, y, sum2, dif2);
+#else
+    const u64 s = addc(u, v), d = sub(u, v);
+    bfly(x, y, sum2, dif2);
+    sum = s;
+    dif = d;
 #endif
 }
 VI_HD void mul2(u64 a, u64 b, u64 &x, u64 c, u64 d, u64 &y) {

@@ -8,6 +8,12 @@
 // between the inverse and the forward transform: decimation in frequency leaves a thread the four consecutive slots
 // (bit-reversed coefficients) that decimation in time starts from, so there is no reordering in between.
 //
+// A SIMD has one or two wavefronts here, so a chain's length is what counts, and a thread's butterflies and products go two at once
+// (gl::bfly2, gl::mul2).  One at a time the corrections by multiply-adds were the longer chains: extensions of 2^7 points by two, 2^20 points, 11.6 us
+// with corrections by additions and 12.1, by four 14.8 and 15.4.  us, calls in a queue, additions one at a time -> multiply-adds two at
+// once: 2^7 by two, 2^20 points, 11.2 -> 10.9, by four 14.4 -> 13.1, 2^8 by four 15.7 -> 13.1, 2^10 by two 16.7 -> 15.6; 12 rows of 2^7 by two 6.2 -> 5.9;
+// a first pass over sixteen rows of 2^12 4.67 -> 4.37, the last the same; 2^18 points as passes 13.2 -> 12.7.
+//
 // Rows of more points take the passes of ntt_plan.hpp, digit by digit, with the same four points per thread (k_small_pass): a
 // launch takes 4.3 us where one of k_ntt_fast takes 8, and the cosets of an extension run side by side.  One row of 2^16
 // extended to 2^18: 57 -> 21 us; 16 rows of 2^12 transformed, calls in a queue: 11.6 -> 8.6 us (two launches where k_ntt_row is
@@ -85,26 +91,22 @@ __device__ __forceinline__ void small_dif(u64 (&x)[4], const SmallTwiddles<LOGN>
         if constexpr ((LOGN & 1) && l == 0) {
             // (x0, x2) and (x1, x3) with w^t and w^(t + N/4) = w_4 w^t
             u64 s0, d0, s1, d1;
-            gl::bfly(x[0], x[2], s0, d0);
-            gl::bfly(x[1], x[3], s1, d1);
+            gl::bfly2(x[0], x[2], s0, d0, x[1], x[3], s1, d1);
             if constexpr (INV) d1 = gl::neg(d1);
             x[0] = s0;
             x[1] = s1;
-            x[2] = gl::mul(d0, W.w[l][0]);
-            x[3] = gl::mul(small_i(d1), W.w[l][0]);
+            gl::mul2(d0, W.w[l][0], x[2], small_i(d1), W.w[l][0], x[3]);
         } else {
             u64 s0, d0, s1, d1;
-            gl::bfly(x[0], x[2], s0, d0);
-            gl::bfly(x[1], x[3], s1, d1);
+            gl::bfly2(x[0], x[2], s0, d0, x[1], x[3], s1, d1);
             d1 = small_i(d1);
             u64 y1, y3;
-            gl::bfly(s0, s1, x[0], x[1]);                              // outputs 0 and 2 mod 4 of the span
-            gl::bfly(d0, d1, INV ? y3 : y1, INV ? y1 : y3);
+            // outputs 0 and 2 mod 4 of the span, and 1 and 3
+            gl::bfly2(s0, s1, x[0], x[1], d0, d1, INV ? y3 : y1, INV ? y1 : y3);
             x[2] = y1;
             x[3] = y3;
             if constexpr (L > 4) {
-                x[1] = gl::mul(x[1], W.w[l][1]);
-                x[2] = gl::mul(x[2], W.w[l][0]);
+                gl::mul2(x[1], W.w[l][1], x[1], x[2], W.w[l][0], x[2]);
                 x[3] = gl::mul(x[3], W.w[l][2]);
             }
         }
@@ -127,10 +129,9 @@ __device__ __forceinline__ void small_dit(u64 (&x)[4], const SmallTwiddles<LOGN>
     static_for<0, LEVELS>([&](auto b_) {
         constexpr int l = LEVELS - 1 - decltype(b_)::value, L = small_span<LOGN>(l);
         if constexpr ((LOGN & 1) && l == 0) {
-            const u64 o0 = gl::mul(x[2], W.w[l][0]), o1 = small_i(gl::mul(x[3], W.w[l][0]));
-            u64 s0, d0, s1, d1;
-            gl::bfly(x[0], o0, s0, d0);
-            gl::bfly(x[1], o1, s1, d1);
+            u64 o0, o1, s0, d0, s1, d1;
+            gl::mul2(x[2], W.w[l][0], o0, x[3], W.w[l][0], o1);
+            gl::bfly2(x[0], o0, s0, d0, x[1], small_i(o1), s1, d1);
             x[0] = s0;
             x[1] = s1;
             x[2] = d0;
@@ -139,16 +140,12 @@ __device__ __forceinline__ void small_dit(u64 (&x)[4], const SmallTwiddles<LOGN>
             // the quarters of a span hold the points 0, 2, 1, 3 mod 4
             u64 t2 = x[1], t1 = x[2], t3 = x[3];
             if constexpr (L > 4) {
+                gl::mul2(t1, W.w[l][0], t1, t3, W.w[l][2], t3);
                 t2 = gl::mul(t2, W.w[l][1]);
-                t1 = gl::mul(t1, W.w[l][0]);
-                t3 = gl::mul(t3, W.w[l][2]);
             }
             u64 s0, d0, s1, d1;
-            gl::bfly(x[0], t2, s0, d0);
-            gl::bfly(t1, t3, s1, d1);
-            d1 = small_i(d1);
-            gl::bfly(s0, s1, x[0], x[2]);
-            gl::bfly(d0, d1, x[1], x[3]);
+            gl::bfly2(x[0], t2, s0, d0, t1, t3, s1, d1);
+            gl::bfly2(s0, s1, x[0], x[2], d0, small_i(d1), x[1], x[3]);
         }
         if constexpr (l > 0) {
             constexpr int LW = L, LR = (LOGN & 1) && l == 1 ? N : small_span<LOGN>(l - 1);
@@ -186,12 +183,14 @@ __global__ __launch_bounds__(SmallShape<LOGN>::WG) void k_small_ntt(u64 *rows, i
     for (int c = 0; c < 4; ++c) mine[small_pad(4 * t + c)] = x[c];
     small_sync<LOGN>();
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        const int k = t + c * S::TR;
-        u64 v = mine[small_pad(small_brev(k, LOGN))];
-        if constexpr (INV) v = gl::mul(v, scale);
-        if (there) p[k] = v;
+    for (int c = 0; c < 4; ++c) x[c] = mine[small_pad(small_brev(t + c * S::TR, LOGN))];
+    if constexpr (INV) {
+#pragma unroll
+        for (int c = 0; c < 4; c += 2) gl::mul2(x[c], scale, x[c], x[c + 1], scale, x[c + 1]);
     }
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+        if (there) p[t + c * S::TR] = x[c];
 }
 
 struct SmallLde {
@@ -234,7 +233,7 @@ __global__ __launch_bounds__(SmallShape<LOGN>::WG) void k_small_lde(const SmallL
         for (int c = 0; c < 4; ++c) coef[c] = gl::canon(coef[c]);
         small_dif<LOGN, true>(coef, W, t, mine);
 #pragma unroll
-        for (int c = 0; c < 4; ++c) coef[c] = gl::mul(coef[c], A.scale);
+        for (int c = 0; c < 4; c += 2) gl::mul2(coef[c], A.scale, coef[c], coef[c + 1], A.scale, coef[c + 1]);
         if (A.coeffs && first == 0 && there) {
 #pragma unroll
             for (int c = 0; c < 4; ++c) A.coeffs[row * A.coeffs_stride + small_brev(4 * t + c, LOGN)] = coef[c];
@@ -247,7 +246,10 @@ __global__ __launch_bounds__(SmallShape<LOGN>::WG) void k_small_lde(const SmallL
     for (int k = first; k < first + A.cosets; ++k) {
         u64 x[4];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) x[c] = gl::mul(coef[c], A.pre[((i64)k << LOGN) + small_brev(4 * t + c, LOGN)]);
+        for (int c = 0; c < 4; c += 2) {
+            const u64 *pre = A.pre + ((i64)k << LOGN);
+            gl::mul2(coef[c], pre[small_brev(4 * t + c, LOGN)], x[c], coef[c + 1], pre[small_brev(4 * t + c + 1, LOGN)], x[c + 1]);
+        }
         small_sync<LOGN>();                                            // the transform before this one has read the row
         small_dit<LOGN>(x, F, t, mine);
         if (there) {
@@ -311,7 +313,7 @@ __global__ __launch_bounds__(256) void k_small_pass(const PassArgs P, const u64 
     }
     if (!FINAL && P.pre) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) x[i] = gl::mul(x[i], f[i]);
+        for (int i = 0; i < 4; i += 2) gl::mul2(x[i], f[i], x[i], x[i + 1], f[i + 1], x[i + 1]);
     }
     small_dif<A, INV, !FINAL>(x, W, t, mine);
 #pragma unroll
@@ -322,12 +324,13 @@ __global__ __launch_bounds__(256) void k_small_pass(const PassArgs P, const u64 
     if (!FINAL) o += coset * P.dst_coset_stride + ((ocol >> P.logR) << (A + P.logR)) + r;
     else o += ocol;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int k = k0 + i * S::TR;
-        u64 v = lds[oc * S::PITCH + small_pad(small_brev(k, A))];
-        if (!FINAL || P.scale != 1) v = gl::mul(v, w[i]);
-        o[(i64)k << (FINAL ? lc : P.logR)] = v;
+    for (int i = 0; i < 4; ++i) x[i] = lds[oc * S::PITCH + small_pad(small_brev(k0 + i * S::TR, A))];
+    if (!FINAL || P.scale != 1) {
+#pragma unroll
+        for (int i = 0; i < 4; i += 2) gl::mul2(x[i], w[i], x[i], x[i + 1], w[i + 1], x[i + 1]);
     }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[(i64)(k0 + i * S::TR) << (FINAL ? lc : P.logR)] = x[i];
 }
 
 template <int A>
