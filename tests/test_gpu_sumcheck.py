@@ -778,8 +778,8 @@ def test_first_passes_around_what_the_chip_holds(mods, terms, v):
 
 @pytest.mark.parametrize("terms,v", [([(7, [0, 1])], 25), ([(5, [0])], 26)])
 def test_second_passes_beyond_what_the_chip_holds(mods, terms, v):
-    """The second pass in place by pieces from a counter, which two tables reach at 2^25 (three and four at 2^24, above), and several columns to
-    a thread in it: one table's threads take so few registers that its passes have the largest grid, and go round."""
+    """The second pass in place by pieces from a counter, which two tables reach at 2^25 (three and four at 2^24, above) and one, whose threads
+    take so few registers that the largest grid is resident, at 2^26."""
     gpu, _ = mods
     tabs = [rand_field_dev((1 << v,), 17 * v + t) for t in range(len(terms[0][1]))]
     coins = _coins(v, v)[0]

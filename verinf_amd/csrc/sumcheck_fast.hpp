@@ -529,8 +529,7 @@ __global__ __launch_bounds__(BLOCK) void k_pass3(const FastDesc D, i64 cols, u64
     SampleAcc<true> acc0[NS], acc1[NS], acc2[NS];
 #pragma unroll
     for (int x = 0; x < NS; ++x) { acc0[x].zero(); acc1[x].zero(); acc2[x].zero(); }
-    const i64 stride = (i64)gridDim.x * BLOCK;
-    for (i64 i = (i64)blockIdx.x * BLOCK + threadIdx.x; i < cols; i += stride) {
+    if (const i64 i = (i64)blockIdx.x * BLOCK + threadIdx.x; i < cols) {
         u64 v[NT][8];
 #pragma unroll
         for (int t = 0; t < NT; ++t)
@@ -786,6 +785,13 @@ __global__ __launch_bounds__(TAIL_THREADS) void k_tail(const FastDesc D, i64 siz
     finish_samples(C, sh, out);
 }
 
+// k_pass3 has a column a thread where all of them are resident at once, k_pass3_long what is more, and first passes over three and four
+// tables from four workgroups a CU on.  us of a pass and of the one behind it, which has fewer rows to add up, long and with a workgroup for 256
+// columns: one table of 2^23 19.0 + 5.5 and 21.0 + 7.9, 2^26 103 + 18 and 122 + 21; two of 2^22 21.4 + 7.2 and 22.0 + 9.6, 2^26 219 + 31 and 246 + 36 (2^24 61 +
+// 12 and 53 + 13 where they stay in the last-level cache from proof to proof); three of 2^21 23.5 + 10.4 and 21.1 + 12.1, the proofs 63.7 and 64.6; 2^22
+// 33.9 + 10.4 and 35.1 + 13.4; four of 2^21 proofs 90.1 and 94.2, gates of 2^21 72.3 and 75.0 on one box, 79.0 and 77.0 on another; 2^22 42.7 + 11.8 and
+// 41.2 + 15.1, 2^26 459 + 65 and 527 + 83.  Second passes of four workgroups a CU: 2^24, three tables 21.2 + 9.8 and 18.4 + 10.7, gates 23.6 + 11.4 and
+// 21.5 + 12.3.
 template <int NT, int SHAPE, bool FIRST, bool ONE>
 int launch_pass3(const FastDesc &F, i64 cols, const u64 *r, u64 *part, const u64 *prev_part, int prev_rows,
                  u64 *prev_sums, hipStream_t s) {
@@ -797,21 +803,20 @@ int launch_pass3(const FastDesc &F, i64 cols, const u64 *r, u64 *part, const u64
     {
         std::lock_guard<std::mutex> lock(mu);
         if (!caps[dev]) {
-            caps[dev] = resident_blocks(k_pass3<NT, SHAPE, FIRST, ONE>, 64);
+            caps[dev] = resident_blocks(k_pass3<NT, SHAPE, FIRST, ONE>, FIRST && NT >= 3 ? 3 : 64);
             cus[dev] = resident_blocks(k_pass3<NT, SHAPE, FIRST, ONE>, 1);
         }
         cap = caps[dev];
         n_cus = cus[dev];
     }
-    int nb = blocks_for(cols);
     const int least = prev_rows > 0 ? 3 : 1; // the first three workgroups add up the previous pass's sums
-    if (nb > cap) {
-        nb = std::max(n_cus, least);
+    if (cols > (i64)cap * BLOCK) {
+        const int nb = std::max(n_cus, least);
         hipLaunchKernelGGL((k_pass3_long<NT, SHAPE, FIRST, ONE>), dim3(nb), dim3(LongPass<NT>::THREADS), 0, s, F, cols, r[0], r[1], r[2], part,
                            prev_part, prev_rows, prev_sums);
         return nb;
     }
-    nb = std::max(nb, least);
+    const int nb = std::max(blocks_for(cols), least);
     hipLaunchKernelGGL((k_pass3<NT, SHAPE, FIRST, ONE>), dim3(nb), dim3(BLOCK), 0, s, F, cols, r[0], r[1], r[2], part,
                        prev_part, prev_rows, prev_sums);
     return nb;
